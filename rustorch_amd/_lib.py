@@ -6,6 +6,8 @@ of the package fails with it.  There is no CPU fallback.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -130,6 +132,30 @@ def lib():
     L.rt_set_strict_non_finite_v.restype = C.c_int
     _lib = L
     return L
+
+
+NATIVE_PATH = os.path.join(_HERE, "lib", "_rt_native.so")
+
+
+class _Native:
+    """The CPython binding of the device entries (csrc/pynative.cpp), loaded on first use: `native.rt_x(...)` takes
+    rt_x's arguments without the error detail -- device buffers, tensors, streams and shapes as they are -- and returns
+    None, or what `errors.check` makes an exception of."""
+
+    def __getattr__(self, name):
+        lib()
+        if not os.path.exists(NATIVE_PATH):
+            raise LibraryMissing(f"{NATIVE_PATH} is missing: build it with `make -C rustorch_amd/csrc`.")
+        loader = importlib.machinery.ExtensionFileLoader("_rt_native", NATIVE_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_rt_native", loader))
+        loader.exec_module(module)
+        self.__dict__.update({n: getattr(module, n) for n in dir(module) if n.startswith("rt_")})
+        if name not in self.__dict__:
+            raise AttributeError(name)
+        return self.__dict__[name]
+
+
+native = _Native()
 
 
 def hip_runtime():

@@ -12,8 +12,7 @@ from dataclasses import dataclass
 import numpy as np
 
 from . import _lib as L
-from .device import dev_ptr
-from .errors import raise_for
+from .errors import check, raise_for
 
 
 @dataclass
@@ -123,75 +122,47 @@ def flash_backward_workspace_bytes(shape: AttentionShape) -> int:
 
 def flash_backward_f32_dev(shape, q, k, v, d_out, dq, dk, dv, workspace, workspace_bytes, stream=None):
     """flash_backward on device-resident f32 [B,H,N,D] tensors; enqueues on `stream` and returns."""
-    err = L.RtErr()
-    s = shape._c()
-    rc = L.lib().rt_flash_backward_f32_dev(stream, C.byref(s), dev_ptr(q), dev_ptr(k), dev_ptr(v), dev_ptr(d_out),
-                                           dev_ptr(dq), dev_ptr(dk), dev_ptr(dv), dev_ptr(workspace),
-                                           workspace_bytes, C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_flash_backward_f32_dev(stream, shape, q, k, v, d_out, dq, dk, dv, workspace, workspace_bytes))
 
 
 def flash_forward_stats_f32_dev(shape, q, k, v, out, lse, stream=None):
     """Unmasked f32 forward that also writes lse[b,h,i] = m_i + ln(l_i): what flash_backward_saved_f32_dev takes back."""
-    err = L.RtErr()
-    s = shape._c()
-    rc = L.lib().rt_flash_forward_stats_f32_dev(stream, C.byref(s), dev_ptr(q), dev_ptr(k), dev_ptr(v), dev_ptr(out),
-                                                dev_ptr(lse), C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_flash_forward_stats_f32_dev(stream, shape, q, k, v, out, lse))
 
 
 def flash_backward_saved_f32_dev(shape, q, k, v, out, lse, d_out, dq, dk, dv, workspace, workspace_bytes, stream=None):
     """The backward from a saved forward (cpu_backward.rs:3-4, :29-35); workspace: batch*heads*seq floats."""
-    err = L.RtErr()
-    s = shape._c()
-    rc = L.lib().rt_flash_backward_saved_f32_dev(stream, C.byref(s), dev_ptr(q), dev_ptr(k), dev_ptr(v), dev_ptr(out),
-                                                 dev_ptr(lse), dev_ptr(d_out), dev_ptr(dq), dev_ptr(dk), dev_ptr(dv),
-                                                 dev_ptr(workspace), workspace_bytes, C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_flash_backward_saved_f32_dev(stream, shape, q, k, v, out, lse, d_out, dq, dk, dv, workspace,
+                                                   workspace_bytes))
 
 
 # ---- device-resident tensors (torch GPU tensors, HipStorage, or raw addresses) ---------------------------
 
 
 def flash_forward_f32_dev(shape, q, k, v, out, mask: Mask = None, keep_dev=None, n_kv_heads=0, stream=None):
-    mask = mask or Mask.none()
-    err = L.RtErr()
-    s = shape._c()
-    rc = L.lib().rt_flash_forward_f32_dev(stream, C.byref(s), n_kv_heads, dev_ptr(q), dev_ptr(k), dev_ptr(v),
-                                          mask.kind, dev_ptr(keep_dev), dev_ptr(out), C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_flash_forward_f32_dev(stream, shape, n_kv_heads, q, k, v, mask.kind if mask else L.RT_MASK_NONE,
+                                            keep_dev, out))
 
 
 def flash_forward_bf16_dev(shape, q, k, v, out, mask: Mask = None, keep_dev=None, n_kv_heads=0, stream=None):
     """bf16 [B,H,N,D] device tensors; enqueues on `stream` and returns."""
-    mask = mask or Mask.none()
-    err = L.RtErr()
-    s = shape._c()
-    rc = L.lib().rt_flash_forward_bf16_dev(stream, C.byref(s), n_kv_heads, dev_ptr(q), dev_ptr(k), dev_ptr(v),
-                                           mask.kind, dev_ptr(keep_dev), dev_ptr(out), C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_flash_forward_bf16_dev(stream, shape, n_kv_heads, q, k, v, mask.kind if mask else L.RT_MASK_NONE,
+                                             keep_dev, out))
 
 
 def flash_forward_window_bf16_dev(shape, q, k, v, out, window: int, n_kv_heads=0, bnhd=False, stream=None):
     """Causal attention with a sliding window (position i sees keys j <= i with i - j < window: the mask of
     rustorch_nn::masks::sliding_window_mask, crates/rustorch-nn/src/masks.rs:41-60, never materialised) on bf16 device
     tensors [B,H,N,D], or [B,N,H,D] with `bnhd`.  Enqueues on `stream` and returns."""
-    err = L.RtErr()
-    s = shape._c()
-    fn = L.lib().rt_flash_forward_window_bnhd_bf16_dev if bnhd else L.lib().rt_flash_forward_window_bf16_dev
-    raise_for(fn(stream, C.byref(s), n_kv_heads, dev_ptr(q), dev_ptr(k), dev_ptr(v), int(window), dev_ptr(out),
-                 C.byref(err)), err)
+    fn = L.native.rt_flash_forward_window_bnhd_bf16_dev if bnhd else L.native.rt_flash_forward_window_bf16_dev
+    check(fn(stream, shape, n_kv_heads, q, k, v, int(window), out))
 
 
 def flash_forward_varlen_bf16_dev(shape, q, k, v, seq_lens_dev, out, zero_padded_rows=True, n_kv_heads=0,
                                   stream=None):
     """Padded-batch causal prefill: per-sequence valid lengths (device int32[batch])."""
-    err = L.RtErr()
-    s = shape._c()
-    rc = L.lib().rt_flash_forward_varlen_bf16_dev(stream, C.byref(s), n_kv_heads, dev_ptr(q), dev_ptr(k),
-                                                  dev_ptr(v), dev_ptr(seq_lens_dev), int(bool(zero_padded_rows)),
-                                                  dev_ptr(out), C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_flash_forward_varlen_bf16_dev(stream, shape, n_kv_heads, q, k, v, seq_lens_dev,
+                                                    int(bool(zero_padded_rows)), out))
 
 
 # ---- [batch, seq, heads, dim] tensors: the layout MultiHeadAttention keeps its projections in --------------
@@ -240,22 +211,16 @@ def mha_forward_masked_f32_dev(q, k, v, out, batch: int, t_q: int, t_kv: int, he
                                mask_len: int = 0, stream=None):
     """`mha_forward_masked_f32` on device-resident f32 tensors ([B,t,H*hd]); `attn_mask` is a device buffer of
     `mask_len` elements (t_q*t_kv or B*H*t_q*t_kv) or None.  Enqueues on `stream` and returns."""
-    err = L.RtErr()
-    rc = L.lib().rt_mha_forward_masked_f32_dev(stream, dev_ptr(q), dev_ptr(k), dev_ptr(v), dev_ptr(attn_mask),
-                                               mask_len if attn_mask is not None else 0, dev_ptr(out), batch, t_q, t_kv,
-                                               heads, head_dim, C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_mha_forward_masked_f32_dev(stream, q, k, v, attn_mask, mask_len if attn_mask is not None else 0, out,
+                                                 batch, t_q, t_kv, heads, head_dim))
 
 
 def mha_forward_masked_bf16_dev(q, k, v, out, batch: int, t_q: int, t_kv: int, heads: int, head_dim: int, attn_mask=None,
                                 mask_len: int = 0, stream=None):
     """The same composed path on bf16 device tensors ([B,t,H*hd] bit patterns) with an f32 device mask of `mask_len`
     elements (t_q*t_kv or B*H*t_q*t_kv) or None; bf16 out.  Enqueues on `stream` and returns."""
-    err = L.RtErr()
-    rc = L.lib().rt_mha_forward_masked_bf16_dev(stream, dev_ptr(q), dev_ptr(k), dev_ptr(v), dev_ptr(attn_mask),
-                                                mask_len if attn_mask is not None else 0, dev_ptr(out), batch, t_q, t_kv,
-                                                heads, head_dim, C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_mha_forward_masked_bf16_dev(stream, q, k, v, attn_mask, mask_len if attn_mask is not None else 0, out,
+                                                 batch, t_q, t_kv, heads, head_dim))
 
 
 def mha_attention_route(t_q: int, t_kv: int, has_mask: bool) -> str:
@@ -286,19 +251,11 @@ def mha_attention_f32(q, k, v, batch: int, t_q: int, t_kv: int, heads: int, head
 
 def flash_forward_bnhd_f32_dev(shape, q, k, v, out, mask: Mask = None, keep_dev=None, n_kv_heads=0, stream=None):
     """f32 [B,N,H,D] device tensors (k, v: [B,N,Hkv,D]); `shape` is still (batch, heads, seq, dim)."""
-    mask = mask or Mask.none()
-    err = L.RtErr()
-    s = shape._c()
-    rc = L.lib().rt_flash_forward_bnhd_f32_dev(stream, C.byref(s), n_kv_heads, dev_ptr(q), dev_ptr(k), dev_ptr(v),
-                                               mask.kind, dev_ptr(keep_dev), dev_ptr(out), C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_flash_forward_bnhd_f32_dev(stream, shape, n_kv_heads, q, k, v, mask.kind if mask else L.RT_MASK_NONE,
+                                                 keep_dev, out))
 
 
 def flash_forward_bnhd_bf16_dev(shape, q, k, v, out, mask: Mask = None, keep_dev=None, n_kv_heads=0, stream=None):
     """bf16 [B,N,H,D] device tensors (k, v: [B,N,Hkv,D]); `shape` is still (batch, heads, seq, dim)."""
-    mask = mask or Mask.none()
-    err = L.RtErr()
-    s = shape._c()
-    rc = L.lib().rt_flash_forward_bnhd_bf16_dev(stream, C.byref(s), n_kv_heads, dev_ptr(q), dev_ptr(k), dev_ptr(v),
-                                                mask.kind, dev_ptr(keep_dev), dev_ptr(out), C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_flash_forward_bnhd_bf16_dev(stream, shape, n_kv_heads, q, k, v, mask.kind if mask else L.RT_MASK_NONE,
+                                                  keep_dev, out))

@@ -61,11 +61,12 @@ int fail_hip(rt_err_detail* e, hipError_t code, const char* where) {
 int g_num_cus = 0;
 int g_decode_waves = 0;  // one-wave workgroups one launch of the decode kernel keeps resident
 std::mutex g_init_mutex;
-int g_init_status = -1;  // -1: not tried
+std::atomic<int> g_init_status{-1};  // -1: not tried
 char g_init_msg[160];
 
 // Finds a gfx950 device once per process.  Never falls back to anything else.
 int ensure_device(rt_err_detail* err, int device = -1) {
+    if (device < 0 && g_init_status.load(std::memory_order_acquire) == RT_OK) return RT_OK;  // every call but the first
     std::lock_guard<std::mutex> lock(g_init_mutex);
     if (g_init_status == RT_OK && device < 0) return RT_OK;
     int count = 0;

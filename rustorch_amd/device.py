@@ -8,7 +8,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib as L
-from .errors import raise_for
+from .errors import check, raise_for
 
 
 class HipStorage:
@@ -114,8 +114,7 @@ def shutdown():
 def i32_add_dev(buf, n: int, delta: int, stream=None):
     """Adds `delta` to the `n` int32 values of a device buffer, asynchronously on `stream` (positions and context
     lengths of a decode loop that lives in a HIP graph)."""
-    err = L.RtErr()
-    raise_for(L.lib().rt_i32_add_dev(stream, dev_ptr(buf), n, delta, C.byref(err)), err)
+    check(L.native.rt_i32_add_dev(stream, buf, n, delta))
 
 
 def debug_force_bf16_prefill_kernel(name: str = "auto"):
@@ -129,17 +128,3 @@ def set_strict_non_finite_v(on: bool) -> bool:
     """Causal prefill entries follow the reference for non-finite V at hidden keys (every row NaN in that column,
     cpu_forward.rs:268-425) at the cost of one more pass over V.  Returns the previous setting."""
     return bool(L.lib().rt_set_strict_non_finite_v(1 if on else 0))
-
-
-def dev_ptr(x) -> int:
-    """Raw device address of a HipStorage, a torch tensor on the GPU, or an int."""
-    if x is None:
-        return None
-    if isinstance(x, HipStorage):
-        return x.ptr
-    if isinstance(x, (int, np.integer)):
-        return int(x)
-    if hasattr(x, "data_ptr"):
-        assert x.is_cuda and x.is_contiguous(), "device entry points take contiguous GPU tensors"
-        return x.data_ptr()
-    raise TypeError(type(x))

@@ -151,3 +151,9 @@ def raise_for(status: int, err: "L.RtErr"):
     if status == L.RT_ERR_ROPE_POSITION_OVERFLOW:
         raise PositionOverflow(err.expected, err.got)
     raise DeviceError(status, err.message.decode(errors="replace"), err.hip_error, err.expected, err.got)
+
+
+def check(result):
+    """The outcome of an entry of `_lib.native`: None, or (status, which, expected, got, got2, hip_error, message)."""
+    if result is not None:
+        raise_for(result[0], L.RtErr(*result[1:]))

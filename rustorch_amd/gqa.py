@@ -6,7 +6,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib as L
-from .errors import raise_for
+from .errors import check, raise_for
 
 
 def gqa_forward_f32(q, k, v, out, batch, n_heads, n_kv_heads, seq_q, seq_kv, head_dim):
@@ -29,9 +29,4 @@ def gqa_forward_f32(q, k, v, out, batch, n_heads, n_kv_heads, seq_q, seq_kv, hea
 
 def gqa_forward_f32_dev(q, k, v, out, batch, n_heads, n_kv_heads, seq_q, seq_kv, head_dim, stream=None):
     """The same on device-resident f32 tensors; enqueues on `stream` and returns."""
-    from .device import dev_ptr
-
-    err = L.RtErr()
-    rc = L.lib().rt_gqa_forward_f32_dev(stream, dev_ptr(q), dev_ptr(k), dev_ptr(v), dev_ptr(out), batch, n_heads,
-                                        n_kv_heads, seq_q, seq_kv, head_dim, C.byref(err))
-    raise_for(rc, err)
+    check(L.native.rt_gqa_forward_f32_dev(stream, q, k, v, out, batch, n_heads, n_kv_heads, seq_q, seq_kv, head_dim))

@@ -8,11 +8,9 @@ is trimmed or copied out before attention.
 """
 from __future__ import annotations
 
-import ctypes as C
-
 from . import _lib as L
-from .device import HipStorage, dev_ptr
-from .errors import LayerOutOfRange, Overflow, raise_for
+from .device import HipStorage
+from .errors import LayerOutOfRange, Overflow, check
 
 _ELEM = {"bf16": 2, "f32": 4}
 
@@ -51,11 +49,9 @@ class KVCache:
             raise LayerOutOfRange(layer_idx, len(self._layers))
         batch, n_heads, max_seq, head_dim = self._dims
         k, v = self._layers[layer_idx]
-        err = L.RtErr()
-        raise_for(L.lib().rt_kv_cache_append_dev(stream, dev_ptr(k), dev_ptr(v), dev_ptr(new_k),
-                                                 new_k.byte_len // self.elem_bytes, dev_ptr(new_v),
-                                                 new_v.byte_len // self.elem_bytes, batch, n_heads, max_seq, head_dim,
-                                                 self._current_len, seq_added, self.elem_bytes, C.byref(err)), err)
+        check(L.native.rt_kv_cache_append_dev(stream, k, v, new_k, new_k.byte_len // self.elem_bytes, new_v,
+                                              new_v.byte_len // self.elem_bytes, batch, n_heads, max_seq, head_dim,
+                                              self._current_len, seq_added, self.elem_bytes))
 
     def advance(self, seq_added: int) -> None:
         """kv_cache.rs:194-204."""
