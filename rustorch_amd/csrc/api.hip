@@ -1674,7 +1674,13 @@ RT_API void* rt_buf_alloc(size_t bytes, rt_err_detail* err) {
 RT_API int rt_buf_free(void* ptr, rt_err_detail* err) {
     clear_err(err);
     if (!ptr) return RT_OK;
-    HIP_TRY(hipFree(ptr), "hipFree");
+    // a buffer may go at any time -- a garbage collector's -- and so while some stream of the process is being captured,
+    // where a free would end the capture with an error unless this thread says that it knows what it does
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
+    const hipError_t freed = hipFree(ptr);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    HIP_TRY(freed, "hipFree");
     return RT_OK;
 }
 
