@@ -21,9 +21,13 @@ namespace {
 
 constexpr int kPrepMaxD = 512;
 
-// grid (n_heads + n_kv, seq, batch), one wave per head row
+// grid (n_heads + n_kv, seq, batch), one wave per head row; lane l holds the pairs (k, k + D/2), k = l + 64 j.  What
+// bounds a decode step's launch is its chain of waits, so everything it reads is requested at once (the row, gamma, the
+// table row, V) and the one serial part, the sum of squares in index order, adds squares that the lanes have formed in
+// parallel, four per LDS read: 3.4 -> 2.9 us for 32 + 8 heads of 128.
+constexpr int kPrepPairs = kPrepMaxD / 2 / kWave;
 __global__ __launch_bounds__(64) void decode_prepare_kernel(DecodePrepareParams p) {
-    __shared__ float row[kPrepMaxD];
+    __shared__ __attribute__((aligned(16))) float squares[kPrepMaxD];
     const int lane = threadIdx.x;
     const int h = blockIdx.x, sq = blockIdx.y, b = blockIdx.z;
     const int D = p.head_dim, half = D / 2, S = p.seq;
@@ -36,39 +40,72 @@ __global__ __launch_bounds__(64) void decode_prepare_kernel(DecodePrepareParams 
     const int kvh = h - p.n_heads;
     const size_t q_row = (((size_t)b * p.n_heads + h) * S + sq) * D;
     const size_t kv_row = (((size_t)b * p.n_kv + kvh) * S + sq) * D;
+    const size_t cache_row = (((size_t)b * p.n_kv + kvh) * (size_t)p.max_seq + (size_t)pos) * D;
     const uint16_t* src = is_q ? p.q + q_row : p.k_in + kv_row;
     const float* gamma = is_q ? p.q_gamma : p.k_gamma;
-
-    for (int i = lane; i < D; i += kWave) row[i] = bf16_bits_to_f32(src[i]);
-    __syncthreads();
-    if (gamma) {
-        // rms_norm_inplace (model.rs:862-885): sq accumulates in index order; every lane walks the whole row
-        // (broadcast reads), which keeps the reference's summation order without a serial section
-        float sq = 0.0f;
-        for (int i = 0; i < D; i++) {
-            const float v = row[i];
-            sq = sq + v * v;
-        }
-        const float inv_d = 1.0f / (float)D;
-        const float inv_rms = 1.0f / sqrtf(sq * inv_d + p.eps);
-        __syncthreads();
-        for (int i = lane; i < D; i += kWave) row[i] = row[i] * inv_rms * gamma[i];
-        __syncthreads();
-    }
     const float* cs = p.cos_table + (size_t)pos * half;
     const float* sn = p.sin_table + (size_t)pos * half;
-    uint16_t* dst = is_q ? p.q + q_row
-                         : p.k_cache + (((size_t)b * p.n_kv + kvh) * (size_t)p.max_seq + (size_t)pos) * D;
-    for (int k = lane; k < half; k += kWave) {
-        const float c = cs[k], si = sn[k];
-        const float x0 = row[k], x1 = row[k + half];
-        dst[k] = f32_to_bf16_bits(x0 * c - x1 * si);
-        dst[k + half] = f32_to_bf16_bits(x1 * c + x0 * si);
+
+    float x0[kPrepPairs], x1[kPrepPairs], c[kPrepPairs], si[kPrepPairs], g0[kPrepPairs], g1[kPrepPairs];
+    uint16_t v0[kPrepPairs], v1[kPrepPairs];
+#pragma unroll
+    for (int j = 0; j < kPrepPairs; j++) {
+        const int k = lane + kWave * j;
+        if (k >= half) break;
+        x0[j] = bf16_bits_to_f32(src[k]);
+        x1[j] = bf16_bits_to_f32(src[k + half]);
+        if (gamma) {
+            g0[j] = gamma[k];
+            g1[j] = gamma[k + half];
+        }
+        c[j] = cs[k];
+        si[j] = sn[k];
+        if (!is_q) {
+            v0[j] = p.v_in[kv_row + k];
+            v1[j] = p.v_in[kv_row + k + half];
+        }
     }
-    if (!is_q) {
-        const uint16_t* vs = p.v_in + kv_row;
-        uint16_t* vd = p.v_cache + (((size_t)b * p.n_kv + kvh) * (size_t)p.max_seq + (size_t)pos) * D;
-        for (int i = lane; i < D; i += kWave) vd[i] = vs[i];
+    if (gamma) {
+        // rms_norm_inplace (model.rs:862-885): sq accumulates in index order; every lane walks the whole row (broadcast
+        // reads), which keeps the reference's summation order without a serial section
+#pragma unroll
+        for (int j = 0; j < kPrepPairs; j++) {
+            const int k = lane + kWave * j;
+            if (k >= half) break;
+            squares[k] = x0[j] * x0[j];
+            squares[k + half] = x1[j] * x1[j];
+        }
+        __syncthreads();
+        float sum = 0.0f;
+        int i = 0;
+        for (; i + 32 <= D; i += 32) {
+            f32x4_t t[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) t[e] = *(const f32x4_t*)(squares + i + 4 * e);
+#pragma unroll
+            for (int e = 0; e < 32; e++) sum = sum + t[e / 4][e % 4];
+        }
+        for (; i < D; i++) sum = sum + squares[i];
+        const float inv_d = 1.0f / (float)D;
+        const float inv_rms = 1.0f / sqrtf(sum * inv_d + p.eps);
+#pragma unroll
+        for (int j = 0; j < kPrepPairs; j++) {
+            if (lane + kWave * j >= half) break;
+            x0[j] = x0[j] * inv_rms * g0[j];
+            x1[j] = x1[j] * inv_rms * g1[j];
+        }
+    }
+    uint16_t* dst = is_q ? p.q + q_row : p.k_cache + cache_row;
+#pragma unroll
+    for (int j = 0; j < kPrepPairs; j++) {
+        const int k = lane + kWave * j;
+        if (k >= half) break;
+        dst[k] = f32_to_bf16_bits(x0[j] * c[j] - x1[j] * si[j]);
+        dst[k + half] = f32_to_bf16_bits(x1[j] * c[j] + x0[j] * si[j]);
+        if (!is_q) {
+            p.v_cache[cache_row + k] = v0[j];
+            p.v_cache[cache_row + k + half] = v1[j];
+        }
     }
 }
 
