@@ -291,37 +291,68 @@ struct SlotTable {
 };
 std::map<int, SlotTable> g_slots;  // per device; guarded by g_ws_mutex
 
-// The slot of `stream` on the current device (taking a free one if it has none yet): its scratch and size, or
-// *ptr = nullptr when no slot is free.
+// The slot of `stream` on the current device (taking a free one if it has none yet), -1 when no slot is free.
+int stream_slot(hipStream_t stream, int* slot, rt_err_detail* err) {
+    *slot = -1;
+    int dev = 0;
+    HIP_TRY(hipGetDevice(&dev), "hipGetDevice");
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    SlotTable& t = g_slots[dev];
+    for (int i = 0; i < rt::kStreamSlots && *slot < 0; i++)
+        if (t.used[i] && t.owner[i] == stream) *slot = i;
+    for (int i = 0; i < rt::kStreamSlots && *slot < 0; i++)
+        if (!t.used[i]) {
+            t.used[i] = true;
+            t.owner[i] = stream;
+            *slot = i;
+        }
+    return RT_OK;
+}
+
+// A slot's scratch and its size, or *ptr = nullptr when no slot is free.
 int stream_slot_scratch(hipStream_t stream, float** ptr, size_t* bytes, rt_err_detail* err) {
     *ptr = nullptr;
     *bytes = 0;
-    int dev = 0;
-    HIP_TRY(hipGetDevice(&dev), "hipGetDevice");
     int slot = -1;
-    {
-        std::lock_guard<std::mutex> lock(g_ws_mutex);
-        SlotTable& t = g_slots[dev];
-        for (int i = 0; i < rt::kStreamSlots && slot < 0; i++)
-            if (t.used[i] && t.owner[i] == stream) slot = i;
-        for (int i = 0; i < rt::kStreamSlots && slot < 0; i++)
-            if (!t.used[i]) {
-                t.used[i] = true;
-                t.owner[i] = stream;
-                slot = i;
-            }
-    }
-    if (slot < 0) return RT_OK;
+    int rc = stream_slot(stream, &slot, err);
+    if (rc || slot < 0) return rc;
     HIP_TRY(rt::stream_static_scratch(slot, ptr, bytes), "hipGetSymbolAddress(stream scratch)");
     return RT_OK;
 }
 
-// the caller holds g_ws_mutex
+// How the decode kernels run a call: in the latency form (one launch, partials folded inside it) where that is the faster
+// one, the stream has a slot (the slot's counters belong to it alone) and is not being captured.  A graph may be
+// replayed on any stream, beside other work of the stream it was captured from, so what is captured keeps no state
+// between launches: split and merge kernel, whose two launches cost little inside a graph.  max_len: the longest context
+// there can be.
+int plan_decode(hipStream_t stream, rt::DecodeSplitParams& p, int max_len, rt_err_detail* err) {
+    const int n_splits = rt::decode_latency_splits(p.batch, p.heads, p.kv_heads, p.dim, p.max_seq, max_len, g_num_cus);
+    if (n_splits == 0 || ((uintptr_t)p.out & 7) != 0) return RT_OK;
+    if (n_splits > 1) {  // (one split: no partials, no state)
+        if ((long long)p.batch * p.kv_heads > rt::kDecodeCounters) return RT_OK;
+        if (stream) {
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            HIP_TRY(hipStreamIsCapturing(stream, &cap), "hipStreamIsCapturing");
+            if (cap != hipStreamCaptureStatusNone) return RT_OK;
+        }
+        int slot = -1;
+        int rc = stream_slot(stream, &slot, err);
+        if (rc || slot < 0) return rc;
+        HIP_TRY(rt::decode_counters(slot, &p.counters), "hipGetSymbolAddress(decode counters)");
+    }
+    p.n_splits = n_splits;
+    return RT_OK;
+}
+
+// the caller holds g_ws_mutex.  The slot's next owner must find its counters at rest: the stream is waited for.
 void release_stream_slot(int dev, hipStream_t stream) {
     auto it = g_slots.find(dev);
     if (it == g_slots.end()) return;
     for (int i = 0; i < rt::kStreamSlots; i++)
-        if (it->second.used[i] && it->second.owner[i] == stream) it->second.used[i] = false;
+        if (it->second.used[i] && it->second.owner[i] == stream) {
+            (void)hipStreamSynchronize(stream);
+            it->second.used[i] = false;
+        }
 }
 
 struct DevPtr {  // a device address inside a Stage's block
@@ -468,6 +499,8 @@ RT_API int rt_init(int device, rt_err_detail* err) {
     size_t scratch_bytes = 0;
     HIP_TRY(rt::decode_static_scratch(&scratch, &scratch_bytes), "hipGetSymbolAddress(static scratch)");
     HIP_TRY(rt::stream_static_scratch(0, &scratch, &scratch_bytes), "hipGetSymbolAddress(stream scratch)");
+    uint32_t* counters = nullptr;
+    HIP_TRY(rt::decode_counters(0, &counters), "hipGetSymbolAddress(decode counters)");
     return RT_OK;
 }
 
@@ -1433,6 +1466,8 @@ RT_API int rt_gqa_decode_online_bf16(void* stream, const void* q, const void* k_
         sp.max_seq = max_seq;
         sp.n_part = rt::decode_split_parts(1, max_seq);
         sp.scale_log2e = (1.0f / sqrtf((float)head_dim)) * rt::kLog2eHost;
+        rc = plan_decode((hipStream_t)stream, sp, kv_len, err);
+        if (rc) return rc;
         HIP_TRY(rt::launch_decode_split((hipStream_t)stream, sp), "decode_split launch");
         return RT_OK;
     }
@@ -1586,6 +1621,8 @@ RT_API int rt_gqa_decode_batched_bf16(void* stream, const void* q, const void* k
         p.span_min = rt::decode_split_span_min(batch);
         p.n_waves = g_decode_waves;
         p.scale_log2e = (1.0f / sqrtf((float)head_dim)) * rt::kLog2eHost;
+        rc = plan_decode((hipStream_t)stream, p, max_seq, err);
+        if (rc) return rc;
         HIP_TRY(rt::launch_decode_split((hipStream_t)stream, p), "decode_split launch");
         return RT_OK;
     }
@@ -1653,6 +1690,8 @@ RT_API int rt_gqa_decode_batched_bf16_noalloc(void* stream, const void* q, const
     p.n_waves = g_decode_waves;
     p.scale_log2e = (1.0f / sqrtf((float)head_dim)) * rt::kLog2eHost;
     p.compact = 1;
+    rc = plan_decode((hipStream_t)stream, p, max_seq, err);
+    if (rc) return rc;
     HIP_TRY(rt::launch_decode_split((hipStream_t)stream, p), "decode_split launch");
     return RT_OK;
 }

@@ -9,6 +9,7 @@
 //                         and leaves an (o, m, l) partial; the merge kernel folds the partials with the
 //                         online-softmax monoid (crates/rustorch-attention/src/online_softmax.rs:105-131,
 //                         extended with o).
+//   decode_latency_kernel the same decode in one launch, for batches and contexts small enough that latency counts.
 //   kv_append_kernel      llm_kernels.rs:353-372.
 //   kv_block_append_kernel  KVLayerCache::append, crates/rustorch-nn/src/kv_cache.rs:77-112 (seq_added rows per head).
 #include <algorithm>
@@ -190,6 +191,7 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(AttnRowsParams p) {
 // Lane l holds column h = l % 16 and the 8 keys 16*rt + 4*(l/16) + i of the step, which as they
 // stand are the 8 contraction slots of its B operand for the second product; the V operand is
 // fetched with the same slot -> key map.
+constexpr uint32_t kBufferFlags = 0x00020000u;  // dword 3 of a raw buffer descriptor: 32-bit data format, no swizzle
 constexpr int kDecRows = 32;     // key rows per step
 constexpr int kDecSpanMin = 8;   // a wave takes at least this many steps (bounds the partials per segment); batches
 constexpr int kDecSpanMinOne = 2;  // the same for a single sequence, where the latency of one call is what counts
@@ -239,21 +241,189 @@ __device__ __forceinline__ int dec_seq_start(const DecodeSplitParams& p, int lan
     return t;
 }
 
+// Geometry of a wave's private LDS tile, and the step both decode kernels run on it.
+template <int HD>
+struct DecTile {
+    static constexpr int LDK = HD + 8;    // +16 B: 16 rows x 16 B tile all 64 banks
+    static constexpr int LDV = HD + 16;   // +32 B: 8 rows x 32 B tile all 64 banks (transposing reads)
+    static constexpr int KS = HD / 32;    // contraction steps of the score product
+    static constexpr int DT = HD / 16;    // 16-row tiles of O^T
+    static constexpr int CH = HD / 8;     // 16-byte chunks per row
+    static constexpr int RPI = 64 / CH;   // rows covered by one wave load instruction
+    static constexpr int NLD = kDecRows / RPI;  // load instructions per tile
+    static constexpr int HALFS = kDecRows * (LDK + LDV);  // bf16 elements of one tile (K, then V)
+};
+
+// The running state of one wave: column h = lane % 16 of O^T, and its (m, l); l is this lane's share of the row sum.
+template <int HD>
+struct DecState {
+    f32x4_t o[DecTile<HD>::DT];
+    float m, l;
+    __device__ __forceinline__ void reset() {
+#pragma unroll
+        for (int t = 0; t < DecTile<HD>::DT; t++) o[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        m = neg_inf();
+        l = 0.0f;
+    }
+    // the row sum over the four 16-lane groups
+    __device__ __forceinline__ float l_total() const {
+        auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+        const float x = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
+        auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        return __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
+    }
+};
+
+// Rows 32 st .. of one (sequence, kv head) segment into registers, fully coalesced; rows past the end re-read the last
+// row (masked by dec_step).  Every cache row is read exactly once per launch: streaming (non-temporal) loads keep the
+// rows from displacing each other and the partials in L2, worth 12 % of the step on a 1.3 GB cache.
+template <int HD>
+__device__ __forceinline__ void dec_load(const DecodeSplitParams& p, int b, int kvh, int st, int len, int lane,
+                                         u32x4_t (&kreg)[DecTile<HD>::NLD], u32x4_t (&vreg)[DecTile<HD>::NLD]) {
+    using T = DecTile<HD>;
+    const size_t base = ((size_t)b * p.kv_heads + kvh) * (size_t)p.max_seq * HD;
+    const uint16_t* K = p.k_cache + base;
+    const uint16_t* V = p.v_cache + base;
+    const int ld_row = lane / T::CH, ld_c = lane % T::CH;
+#pragma unroll
+    for (int i = 0; i < T::NLD; i++) {
+        const int r = min(st * kDecRows + T::RPI * i + ld_row, len - 1);
+        kreg[i] = __builtin_nontemporal_load((const u32x4_t*)(K + (size_t)r * HD + 8 * ld_c));
+        vreg[i] = __builtin_nontemporal_load((const u32x4_t*)(V + (size_t)r * HD + 8 * ld_c));
+    }
+}
+template <int HD>
+__device__ __forceinline__ void dec_park(uint16_t* Kw, uint16_t* Vw, int lane, const u32x4_t (&kreg)[DecTile<HD>::NLD],
+                                         const u32x4_t (&vreg)[DecTile<HD>::NLD]) {
+    using T = DecTile<HD>;
+    const int ld_row = lane / T::CH, ld_c = lane % T::CH;
+#pragma unroll
+    for (int i = 0; i < T::NLD; i++) {
+        *(u32x4_t*)(Kw + (T::RPI * i + ld_row) * T::LDK + 8 * ld_c) = kreg[i];
+        *(u32x4_t*)(Vw + (T::RPI * i + ld_row) * T::LDV + 8 * ld_c) = vreg[i];
+    }
+}
+// Q as B operand: column h = lane % 16 (zero beyond the group), contraction slots 8*(lane/16)..+8
+template <int HD>
+__device__ __forceinline__ void dec_load_q(const DecodeSplitParams& p, int b, int kvh, int lane, bf16x8_t (&q)[DecTile<HD>::KS]) {
+    const int G = p.heads / p.kv_heads, hcol = lane & 15, g4 = lane >> 4;
+#pragma unroll
+    for (int ks = 0; ks < DecTile<HD>::KS; ks++) {
+        u32x4_t z = {0u, 0u, 0u, 0u};
+        if (hcol < G) z = *(const u32x4_t*)(p.q + ((size_t)b * p.heads + (size_t)kvh * G + hcol) * HD + 32 * ks + 8 * g4);
+        q[ks] = __builtin_bit_cast(bf16x8_t, z);
+    }
+}
+
+// One step of 32 keys: `left` of them exist (32 except on the ragged last step of a segment); `lazy`: 8 / c.
+template <int HD>
+__device__ __forceinline__ void dec_step(const uint16_t* Kw, const uint16_t* Vw, int lane, int left, float c, float lazy,
+                                         const bf16x8_t (&q)[DecTile<HD>::KS], DecState<HD>& st) {
+    using T = DecTile<HD>;
+    const int hcol = lane & 15, g4 = lane >> 4;
+    const int k_off = hcol * T::LDK + 8 * g4;
+    const int tr_off = (4 * g4 + (hcol >> 2)) * T::LDV + 4 * (hcol & 3);
+    // ---- S^T = K . Q^T, two 16-key row tiles
+    f32x4_t s[2];
+#pragma unroll
+    for (int rt = 0; rt < 2; rt++) {
+        s[rt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ks = 0; ks < T::KS; ks++) {
+            bf16x8_t a = *(const bf16x8_t*)(Kw + 16 * rt * T::LDK + k_off + 32 * ks);
+            s[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, q[ks], s[rt], 0, 0, 0);
+        }
+    }
+    if (left < kDecRows) {
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (16 * rt + 4 * g4 + i >= left) s[rt][i] = neg_inf();
+    }
+    // ---- column max over the 32 keys: in-lane, then across the four 16-lane groups
+    float m_step = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
+                         fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+    {
+        auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(m_step), __float_as_uint(m_step), false, false);
+        m_step = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
+        auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m_step), __float_as_uint(m_step), false, false);
+        m_step = fmaxf(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
+    }
+    if (__any(m_step > st.m + lazy)) {  // raise the running max only when it pays (wave-uniform)
+        float m_new = fmaxf(st.m, m_step);
+        float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
+        float alpha = __builtin_amdgcn_exp2f((st.m - m_use) * c);
+        st.m = m_new;
+        st.l *= alpha;
+#pragma unroll
+        for (int tt = 0; tt < T::DT; tt++) st.o[tt] *= alpha;
+    }
+    const float mc = ((st.m == neg_inf()) ? 0.0f : st.m) * c;
+    float pe[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) pe[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i >> 2][i & 3], c, -mc));
+    st.l += ((pe[0] + pe[1]) + (pe[2] + pe[3])) + ((pe[4] + pe[5]) + (pe[6] + pe[7]));
+    u32x4_t pb;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        f32x2v x = {pe[2 * e], pe[2 * e + 1]};
+        pb[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2v));
+    }
+    const bf16x8_t pB = __builtin_bit_cast(bf16x8_t, pb);
+    // ---- O^T += V^T . P^T: slots 0-3 of a lane are keys 4g..4g+3, slots 4-7 keys 16+4g..16+4g+3
+#pragma unroll
+    for (int dt = 0; dt < T::DT; dt++) {
+        const uint16_t* vp = Vw + tr_off + 16 * dt;
+        u32x2_t lo = lds_read_tr16_b64(vp);
+        u32x2_t hi = lds_read_tr16_b64(vp + 16 * T::LDV);
+        u32x4_t av = {lo[0], lo[1], hi[0], hi[1]};
+        st.o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av), pB, st.o[dt], 0, 0, 0);
+    }
+}
+
+// ---- partials that another workgroup of the same launch reads -------------------------------------------------
+// The workgroup that finishes a segment last folds its partials, inside the same launch.  A release fence before the
+// counter would write the XCD's whole L2 back (twice the time of the launch on a 1.3 GB cache); instead every partial
+// is stored at device scope (sc1: through the L2 to memory), the stores are waited for, and the counter is a
+// device-scope atomic behind that wait.  The reader's loads are device-scope as well and do not hit stale lines of its
+// own L2.  Which workgroup folds depends on the timing, the order of the fold does not.  The partials are addressed
+// through a buffer descriptor: that is how a 16-byte access with a scope can be written (each at most 8 MiB or what the
+// caller's workspace holds: 32-bit offsets).
+constexpr int kScopeDevice = 16;  // sc1
+__device__ __forceinline__ void put4(__amdgpu_buffer_rsrc_t rs, uint32_t byte, f32x4_t v) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), rs, byte, 0, kScopeDevice);
+}
+__device__ __forceinline__ void put2(__amdgpu_buffer_rsrc_t rs, uint32_t byte, float a, float b) {
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{__float_as_uint(a), __float_as_uint(b)}, rs, byte, 0, kScopeDevice);
+}
+__device__ __forceinline__ f32x4_t get4(__amdgpu_buffer_rsrc_t rs, uint32_t byte) {
+    return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, byte, 0, kScopeDevice));
+}
+__device__ __forceinline__ f32x2v get2(__amdgpu_buffer_rsrc_t rs, uint32_t byte) {
+    return __builtin_bit_cast(f32x2v, __builtin_amdgcn_raw_buffer_load_b64(rs, byte, 0, kScopeDevice));
+}
+__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// Counts one finished partial of `n`; true for the one that completes the set, which also puts the counter back to 0
+// for the next launch.
+__device__ __forceinline__ bool count_partial(uint32_t* counter, int n) {
+    const uint32_t old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (old + 1u != (uint32_t)n) return false;
+    __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
 struct DecCursor {  // position in the flat step list
     int b, kvh, st, steps_b, len_b;
 };
 
 template <int HD>
 __global__ __launch_bounds__(64) void decode_split_kernel(DecodeSplitParams p) {
-    constexpr int LDK = HD + 8;    // +16 B: 16 rows x 16 B tile all 64 banks
-    constexpr int LDV = HD + 16;   // +32 B: 8 rows x 32 B tile all 64 banks (transposing reads)
-    constexpr int KS = HD / 32;    // contraction steps of the score product
-    constexpr int DT = HD / 16;    // 16-row tiles of O^T
-    constexpr int CH = HD / 8;     // 16-byte chunks per row
-    constexpr int RPI = 64 / CH;   // rows covered by one wave load instruction
-    constexpr int NLD = kDecRows / RPI;  // load instructions per tile
-    __shared__ __attribute__((aligned(16))) uint16_t Kw[kDecRows * LDK];
-    __shared__ __attribute__((aligned(16))) uint16_t Vw[kDecRows * LDV];
+    using T = DecTile<HD>;
+    constexpr int KS = T::KS, DT = T::DT, NLD = T::NLD;
+    __shared__ __attribute__((aligned(16))) uint16_t tile[T::HALFS];
+    uint16_t* const Kw = tile;
+    uint16_t* const Vw = tile + kDecRows * T::LDK;
 
     const int lane = threadIdx.x;
     const int hcol = lane & 15, g4 = lane >> 4;
@@ -306,134 +476,31 @@ __global__ __launch_bounds__(64) void decode_split_kernel(DecodeSplitParams p) {
         }
     };
 
-    const float c = p.scale_log2e;
-    const float lazy_raw = 8.0f / c;
-    const int ld_row = lane / CH, ld_c = lane % CH;
-    const int k_off = hcol * LDK + 8 * g4;
-    const int tr_off = (4 * g4 + (hcol >> 2)) * LDV + 4 * (hcol & 3);
-
+    const float c = p.scale_log2e, lazy = 8.0f / c;
     u32x4_t kreg[NLD], vreg[NLD];
-    auto issue_loads = [&](const DecCursor& cc) {
-        const size_t base = ((size_t)cc.b * Hkv + cc.kvh) * (size_t)p.max_seq * HD;
-        const uint16_t* K = p.k_cache + base;
-        const uint16_t* V = p.v_cache + base;
-#pragma unroll
-        for (int i = 0; i < NLD; i++) {
-            int r = min(cc.st * kDecRows + RPI * i + ld_row, cc.len_b - 1);  // rows past the end re-read the last row; masked below
-            // every cache row is read exactly once per launch: streaming (non-temporal) loads keep the rows from
-            // displacing each other and the partials in L2, worth 12 % of the step on a 1.3 GB cache
-            kreg[i] = __builtin_nontemporal_load((const u32x4_t*)(K + (size_t)r * HD + 8 * ld_c));
-            vreg[i] = __builtin_nontemporal_load((const u32x4_t*)(V + (size_t)r * HD + 8 * ld_c));
-        }
-    };
-    // Q as B operand: column h = lane % 16 (zero beyond the group), contraction slots 8*(lane/16)..+8
     bf16x8_t qreg[KS], qnext[KS];
-    auto load_q = [&](const DecCursor& cc, bf16x8_t (&q)[KS]) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            u32x4_t z = {0u, 0u, 0u, 0u};
-            if (hcol < G) z = *(const u32x4_t*)(p.q + ((size_t)cc.b * p.heads + (size_t)cc.kvh * G + hcol) * HD + 32 * ks + 8 * g4);
-            q[ks] = __builtin_bit_cast(bf16x8_t, z);
-        }
-    };
-
-    f32x4_t acc_o[DT];
-    float m_run, l_run;
-    auto reset_state = [&]() {
-#pragma unroll
-        for (int t = 0; t < DT; t++) acc_o[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        m_run = neg_inf();
-        l_run = 0.0f;
-    };
-    reset_state();
+    DecState<HD> state;
+    state.reset();
 
     DecCursor nxt = cur;  // the prefetch cursor runs one step ahead of `cur`
-    load_q(cur, qreg);
-    issue_loads(nxt);
+    dec_load_q<HD>(p, cur.b, cur.kvh, lane, qreg);
+    dec_load<HD>(p, nxt.b, nxt.kvh, nxt.st, nxt.len_b, lane, kreg, vreg);
     advance(nxt);
 
     for (int t = first; t < last; t++) {
         // registers -> the wave's LDS tile (the previous step's reads have been consumed by its MFMAs)
-#pragma unroll
-        for (int i = 0; i < NLD; i++) {
-            *(u32x4_t*)(Kw + (RPI * i + ld_row) * LDK + 8 * ld_c) = kreg[i];
-            *(u32x4_t*)(Vw + (RPI * i + ld_row) * LDV + 8 * ld_c) = vreg[i];
-        }
+        dec_park<HD>(Kw, Vw, lane, kreg, vreg);
         const bool more = t + 1 < last;
         if (more) {  // next step's rows (and, on a segment change, its queries) fly while this one computes
-            issue_loads(nxt);
-            if (nxt.st == 0) load_q(nxt, qnext);
+            dec_load<HD>(p, nxt.b, nxt.kvh, nxt.st, nxt.len_b, lane, kreg, vreg);
+            if (nxt.st == 0) dec_load_q<HD>(p, nxt.b, nxt.kvh, lane, qnext);
         }
-
-        // ---- S^T = K . Q^T, two 16-key row tiles
-        f32x4_t s[2];
-#pragma unroll
-        for (int rt = 0; rt < 2; rt++) {
-            s[rt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                bf16x8_t a = *(const bf16x8_t*)(Kw + 16 * rt * LDK + k_off + 32 * ks);
-                s[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qreg[ks], s[rt], 0, 0, 0);
-            }
-        }
-        const int r0 = cur.st * kDecRows;
-        if (r0 + kDecRows > cur.len_b) {  // ragged last step of a segment
-#pragma unroll
-            for (int rt = 0; rt < 2; rt++)
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (r0 + 16 * rt + 4 * g4 + i >= cur.len_b) s[rt][i] = neg_inf();
-        }
-        // ---- column max over the 32 keys: in-lane, then across the four 16-lane groups
-        float m_step = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
-                             fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
-        {
-            auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(m_step), __float_as_uint(m_step), false, false);
-            m_step = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
-            auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m_step), __float_as_uint(m_step), false, false);
-            m_step = fmaxf(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
-        }
-        if (__any(m_step > m_run + lazy_raw)) {  // raise the running max only when it pays (wave-uniform)
-            float m_new = fmaxf(m_run, m_step);
-            float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
-            float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * c);
-            m_run = m_new;
-            l_run *= alpha;
-#pragma unroll
-            for (int tt = 0; tt < DT; tt++) acc_o[tt] *= alpha;
-        }
-        const float mc = ((m_run == neg_inf()) ? 0.0f : m_run) * c;
-        float pe[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) pe[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i >> 2][i & 3], c, -mc));
-        l_run += ((pe[0] + pe[1]) + (pe[2] + pe[3])) + ((pe[4] + pe[5]) + (pe[6] + pe[7]));
-        u32x4_t pb;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            f32x2v x = {pe[2 * e], pe[2 * e + 1]};
-            pb[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2v));
-        }
-        const bf16x8_t pB = __builtin_bit_cast(bf16x8_t, pb);
-        // ---- O^T += V^T . P^T: slots 0-3 of a lane are keys 4g..4g+3, slots 4-7 keys 16+4g..16+4g+3
-#pragma unroll
-        for (int dt = 0; dt < DT; dt++) {
-            const uint16_t* vp = Vw + tr_off + 16 * dt;
-            u32x2_t lo = lds_read_tr16_b64(vp);
-            u32x2_t hi = lds_read_tr16_b64(vp + 16 * LDV);
-            u32x4_t av = {lo[0], lo[1], hi[0], hi[1]};
-            acc_o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av), pB, acc_o[dt], 0, 0, 0);
-        }
+        dec_step<HD>(Kw, Vw, lane, cur.len_b - cur.st * kDecRows, c, lazy, qreg, state);
 
         // ---- end of a segment (or of this wave's span): leave the partial and start afresh
         const bool seg_end = (cur.st == cur.steps_b - 1);
         if (seg_end || !more) {
-            float l_all = l_run;
-            {
-                auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(l_all), __float_as_uint(l_all), false, false);
-                l_all = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
-                auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_all), __float_as_uint(l_all), false, false);
-                l_all = __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
-            }
+            const float l_all = state.l_total();
             const int seg_first = t - cur.st;  // flat index of the segment's first step
             const int part = w - seg_first / span;
             if (hcol < G) {
@@ -441,15 +508,15 @@ __global__ __launch_bounds__(64) void decode_split_kernel(DecodeSplitParams p) {
                 float* ws_ml = p.ws + dec_slots(p) * HD;
                 const size_t slot = p.compact ? ((size_t)w + (size_t)cur.b * Hkv + cur.kvh) * G + hcol
                                               : ((size_t)cur.b * p.heads + (size_t)cur.kvh * G + hcol) * p.n_part + part;
-                // acc_o[dt][i] = O^T[d = 16dt + 4g + i][h]
+                // state.o[dt][i] = O^T[d = 16dt + 4g + i][h]
 #pragma unroll
-                for (int dt = 0; dt < DT; dt++) *(f32x4_t*)(ws_o + slot * HD + 16 * dt + 4 * g4) = acc_o[dt];
+                for (int dt = 0; dt < DT; dt++) *(f32x4_t*)(ws_o + slot * HD + 16 * dt + 4 * g4) = state.o[dt];
                 if (g4 == 0) {
-                    ws_ml[slot * 2] = m_run * c;  // the merge works in the exp2 domain
+                    ws_ml[slot * 2] = state.m * c;  // the merge works in the exp2 domain
                     ws_ml[slot * 2 + 1] = l_all;
                 }
             }
-            reset_state();
+            state.reset();
             if (seg_end && more) {
 #pragma unroll
                 for (int ks = 0; ks < KS; ks++) qreg[ks] = qnext[ks];
@@ -457,6 +524,156 @@ __global__ __launch_bounds__(64) void decode_split_kernel(DecodeSplitParams p) {
         }
         cur = nxt;
         if (more) advance(nxt);
+    }
+}
+
+// The same decode where latency counts and not bandwidth: few steps in all.  One launch; grid (splits, kv heads,
+// batch), a workgroup of four waves per (segment, split).  A split is at least four steps, one per wave, whatever the
+// segment's length, so a short context is folded inside one workgroup; a longer one is cut into p.n_splits splits,
+// whose partials the workgroup that finishes last folds.  Bound by its chain of waits: 4.2 us for one split (arguments,
+// rows, products, fold of the waves), 3 us more for a fold across workgroups (stores out, counter, loads back).  32 / 8
+// heads of 128, us per call, before (split + merge kernel) and now: 4 sequences of 64-512 16.7 / 8.1, 128 of 32-256
+// 26.7 / 17.9, one of 2048 9.3 / 8.5.
+constexpr int kLatWaves = 4;
+constexpr int kLatMaxSplits = 24;
+
+template <int HD>
+__global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSplitParams p) {
+    using T = DecTile<HD>;
+    constexpr int DT = T::DT, NT = 64 * kLatWaves;
+    constexpr int LDO = HD + 4;  // floats per row of the workgroup's folded output: 16 rows tile the banks
+    constexpr int TILE_B = kLatWaves * T::HALFS * 2, RED_B = kLatWaves * 16 * LDO * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[TILE_B > RED_B ? TILE_B : RED_B];
+    __shared__ float red_m[kLatWaves][16], red_l[kLatWaves][16];
+    __shared__ float wgt[kLatMaxSplits][16], inv_l[16];
+    __shared__ int is_last;
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int hcol = lane & 15, g4 = lane >> 4;
+    const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+    const int G = p.heads / p.kv_heads;
+    const int seg = b * p.kv_heads + kvh;
+    const int len = dec_len(p, b), steps = dec_steps(len);
+    const int per = max((steps + p.n_splits - 1) / p.n_splits, kLatWaves);
+    const int n_act = (steps + per - 1) / per;  // splits that hold keys
+    uint16_t* const out = p.out + (size_t)seg * G * HD;
+    if (split >= n_act) {
+        if (steps == 0 && split == 0)  // no key: rows of zeros (gqa.rs:261; llm_kernels.rs:456)
+            for (int i = tid; i < G * HD / 4; i += NT) *(u32x2_t*)(out + 4 * i) = u32x2_t{0u, 0u};
+        return;
+    }
+    const int t1 = min(steps, (split + 1) * per);
+    uint16_t* const Kw = (uint16_t*)lds + wave * T::HALFS;
+    uint16_t* const Vw = Kw + kDecRows * T::LDK;
+    const float c = p.scale_log2e, lazy = 8.0f / c;
+
+    DecState<HD> state;
+    state.reset();
+    int t = split * per + wave;
+    if (t < t1) {
+        u32x4_t kreg[T::NLD], vreg[T::NLD];
+        bf16x8_t qreg[T::KS];
+        dec_load<HD>(p, b, kvh, t, len, lane, kreg, vreg);
+        dec_load_q<HD>(p, b, kvh, lane, qreg);
+        for (; t < t1; t += kLatWaves) {
+            dec_park<HD>(Kw, Vw, lane, kreg, vreg);
+            if (t + kLatWaves < t1) dec_load<HD>(p, b, kvh, t + kLatWaves, len, lane, kreg, vreg);
+            dec_step<HD>(Kw, Vw, lane, len - t * kDecRows, c, lazy, qreg, state);
+        }
+    }
+
+    // ---- fold the four waves
+    const float l_wave = state.l_total(), m_wave = state.m * c;  // exp2 domain from here on
+    if (g4 == 0) {
+        red_m[wave][hcol] = m_wave;
+        red_l[wave][hcol] = l_wave;
+    }
+    __syncthreads();  // also: every wave is done with its tile
+    float m_wg = neg_inf(), l_wg = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kLatWaves; w++) m_wg = fmaxf(m_wg, red_m[w][hcol]);
+    const float m_use = (m_wg == neg_inf()) ? 0.0f : m_wg;
+#pragma unroll
+    for (int w = 0; w < kLatWaves; w++) l_wg += red_l[w][hcol] * __builtin_amdgcn_exp2f(red_m[w][hcol] - m_use);
+    float* const red = (float*)lds;
+    if (hcol < G) {
+        const float f = __builtin_amdgcn_exp2f(m_wave - m_use);
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) *(f32x4_t*)(red + (wave * 16 + hcol) * LDO + 16 * dt + 4 * g4) = state.o[dt] * f;
+    }
+    if (wave == 0 && g4 == 0) inv_l[hcol] = 1.0f / l_wg;
+    __syncthreads();
+    const uint32_t n_slots = (uint32_t)p.batch * p.heads * p.n_splits, ml_byte = n_slots * HD * 4;
+    const uint32_t slot0 = (uint32_t)seg * p.n_splits * G;  // partial k of head h: slot0 + k * G + h
+    const __amdgpu_buffer_rsrc_t ws_rs = __builtin_amdgcn_make_buffer_rsrc((void*)p.ws, 0, n_slots * (HD + 2) * 4, kBufferFlags);
+    for (int x = tid; x < G * HD / 4; x += NT) {
+        const int h = x / (HD / 4), d = 4 * (x - h * (HD / 4));
+        f32x4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < kLatWaves; w++) o += *(const f32x4_t*)(red + (w * 16 + h) * LDO + d);
+        if (n_act == 1) {
+            o *= inv_l[h];
+            *(u32x2_t*)(out + h * HD + d) = u32x2_t{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+        } else {
+            put4(ws_rs, ((slot0 + split * G + h) * HD + d) * 4, o);
+        }
+    }
+    if (n_act == 1) return;
+    if (tid < G) put2(ws_rs, ml_byte + (slot0 + split * G + tid) * 8, m_wg, l_wg);  // (tid < 16: hcol == tid)
+    stores_done();
+    __syncthreads();
+    if (tid == 0) is_last = count_partial(p.counters + seg, n_act) ? 1 : 0;
+    __syncthreads();
+    if (!is_last) return;
+
+    // ---- the last workgroup of the segment: the weighted sum of its partials.  SUB groups of threads take every SUB-th
+    // split of four elements, eight loads of a thread in flight at a time; the first loads are requested ahead of the
+    // (m, l) pairs the weights are made of.
+    const int n_x = G * HD / 4;
+    const int sub_n = n_x >= NT ? 1 : NT / n_x;
+    const int xt = sub_n == 1 ? tid : tid % n_x, sub = sub_n == 1 ? 0 : tid / n_x;
+    constexpr int kGroup = 8;
+    f32x4_t a[kGroup];
+    auto load_group = [&](int x, int k0) {
+        const uint32_t at = (slot0 * HD + 4u * (uint32_t)min(x, n_x - 1)) * 4u;
+#pragma unroll
+        for (int j = 0; j < kGroup; j++) a[j] = get4(ws_rs, at + (uint32_t)min(k0 + j * sub_n, n_act - 1) * (uint32_t)(G * HD * 4));
+    };
+    load_group(xt, sub);
+    for (int h = wave; h < G; h += kLatWaves) {  // one lane per split
+        const f32x2v ml = lane < n_act ? get2(ws_rs, ml_byte + (slot0 + lane * G + h) * 8) : f32x2v{neg_inf(), 0.0f};
+        float m = ml[0];
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+        const float f = __builtin_amdgcn_exp2f(ml[0] - ((m == neg_inf()) ? 0.0f : m));
+        const float l = wave_sum(ml[1] * f);
+        wgt[lane][h] = f;  // 0 past the last split
+        if (lane == 0) inv_l[h] = 1.0f / l;
+    }
+    __syncthreads();
+    for (int x0 = 0; x0 < n_x; x0 += NT) {
+        const int x = x0 + xt;
+        const bool on = x < n_x && sub < sub_n;
+        const int h = on ? x / (HD / 4) : 0;
+        f32x4_t part = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int k0 = sub; k0 < n_act; k0 += kGroup * sub_n) {
+            if (x0 + k0 != sub) load_group(x, k0);
+#pragma unroll
+            for (int j = 0; j < kGroup; j++) {
+                const int k = k0 + j * sub_n;
+                part += a[j] * (k < n_act ? wgt[k][h] : 0.0f);
+            }
+        }
+        if (sub_n > 1) {  // (n_x < NT: one round)
+            if (on) *(f32x4_t*)(red + 4 * (sub * n_x + x)) = part;
+            __syncthreads();
+            if (on && sub == 0)
+                for (int j = 1; j < sub_n; j++) part += *(const f32x4_t*)(red + 4 * (j * n_x + x));
+        }
+        if (on && sub == 0) {
+            const f32x4_t o = part * inv_l[h];
+            *(u32x2_t*)(out + 4 * x) = u32x2_t{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+        }
     }
 }
 
@@ -573,6 +790,10 @@ __global__ __launch_bounds__(256) void kv_block_append_kernel(T* __restrict__ k_
 
 template <int HD>
 hipError_t launch_split_hd(hipStream_t stream, const DecodeSplitParams& p) {
+    if (p.n_splits > 0) {
+        hipLaunchKernelGGL(decode_latency_kernel<HD>, dim3(p.n_splits, p.kv_heads, p.batch), dim3(64 * kLatWaves), 0, stream, p);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(decode_split_kernel<HD>, dim3(p.n_waves), dim3(64), 0, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -667,6 +888,55 @@ hipError_t stream_static_scratch(int slot, float** ptr, size_t* bytes) {
     *ptr = (float*)((unsigned char*)g_stream_scratch_ptr[dev] + (size_t)slot * kStreamSlotBytes);
     *bytes = kStreamSlotBytes;
     return hipSuccess;
+}
+
+// One counter per (sequence, kv head) and stream slot, for the launches that fold their own partials: zero when the code
+// object is loaded, and back to zero at the end of every launch.
+static __device__ uint32_t decode_counter_block[(size_t)kStreamSlots * kDecodeCounters];
+
+namespace {
+void* g_decode_counter_ptr[kMaxDevices] = {};
+}  // namespace
+
+hipError_t decode_counters(int slot, uint32_t** ptr) {
+    if (slot < 0 || slot >= kStreamSlots) return hipErrorInvalidValue;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
+    std::lock_guard<std::mutex> lock(g_scratch_mutex);
+    if (!g_decode_counter_ptr[dev]) {
+        void* addr = nullptr;
+        e = hipGetSymbolAddress(&addr, HIP_SYMBOL(decode_counter_block));
+        if (e != hipSuccess) return e;
+        if (!addr) return hipErrorInvalidSymbol;
+        g_decode_counter_ptr[dev] = addr;
+    }
+    *ptr = (uint32_t*)g_decode_counter_ptr[dev] + (size_t)slot * kDecodeCounters;
+    return hipSuccess;
+}
+
+// Where the lines lie, from us per call at 32 / 8 heads of 128 unless said (latency form against split + merge):
+//   contexts up to 1056 whatever the batch, 64 sequences of 128-1024: 29.9 / 32.1, 128 of 62-500: 27.5 / 36.1; and up to
+//   10000 steps in all, 16 of 256-2048: 19.6 / 20.7.  Beyond both the streaming kernel's equal spans win: 20 of 500-4000
+//   with 40 heads 40.9 / 36.6, 64 of 256-2048: 56.3 / 53.9, 16 of 1024-8192: 57.6 / 52.3.
+//   At head dim 256 one workgroup's LDS fills a CU, and a fold moves twice the bytes: not with more segments than CUs (30
+//   sequences of 97-777 with 12 heads: 40.0 / 36.0), nor for one long sequence (16 / 2 heads, 8000: 19.5 / 17.0).
+//   Splitting costs a fold of about 3 us: not below 12 steps (384 keys: 9.8 against 10.3), and not beyond a workgroup per
+//   CU (30 sequences of 75-600, 8 heads of 64: 7.8 with one workgroup per segment, 10.0 with two).  More than 24 splits
+//   make the fold longer than they make the walk shorter (one sequence of 8192: 16.5, with 32: 17.0, with 64: 21.2).
+int decode_latency_splits(int batch, int heads, int kv_heads, int dim, int max_seq, int max_len, int n_cus) {
+    const long long segs = (long long)batch * kv_heads, steps = (max_len + kDecRows - 1) / kDecRows;
+    if (steps > 33 && segs * steps > 10000) return 0;
+    if (dim == 256 && (batch == 1 ? steps > 40 : segs > n_cus)) return 0;
+    if (steps <= 3 * kLatWaves) return 1;
+    long long n = std::min<long long>((steps + kLatWaves - 1) / kLatWaves, kLatMaxSplits);
+    n = std::min<long long>(n, n_cus / segs);
+    // what the room for partials allows in every entry (the caller's workspace and the library's slots alike, so that
+    // all give the same bits)
+    n = std::min<long long>(n, decode_split_parts(batch, max_seq));
+    n = std::min<long long>(n, (long long)(kStreamSlotBytes / ((size_t)batch * heads * ((size_t)dim + 2) * sizeof(float))));
+    return (int)std::max<long long>(n, 1);
 }
 
 hipError_t launch_decode_split(hipStream_t stream, const DecodeSplitParams& p) {
