@@ -12,7 +12,7 @@ from dataclasses import dataclass
 import numpy as np
 
 from . import _lib as L
-from .errors import check, raise_for
+from .errors import check
 
 
 @dataclass
@@ -68,28 +68,29 @@ class Mask:
         return False
 
 
+_F32 = np.dtype(np.float32)
+
+
 def _f32(a):
-    a = np.ascontiguousarray(np.ravel(a), dtype=np.float32)
-    return a, a.ctypes.data_as(C.POINTER(C.c_float))
+    """`a` as a C-contiguous f32 array (itself where it is one)."""
+    if type(a) is np.ndarray and a.dtype == _F32 and a.flags.c_contiguous:
+        return a
+    return np.ascontiguousarray(np.ravel(a), dtype=np.float32)
+
+
+def _out(out, n):
+    if out is None:
+        return np.empty(n, dtype=np.float32)
+    assert out.dtype == _F32 and out.flags.c_contiguous
+    return out
 
 
 def flash_forward_masked(shape: AttentionShape, q, k, v, mask: Mask, out=None):
     """cpu_forward.rs:193-242.  q, k, v: flat f32 [B,H,N,D]; returns (and fills) flat f32 `out`."""
-    q, qp = _f32(q)
-    k, kp = _f32(k)
-    v, vp = _f32(v)
-    if out is None:
-        out = np.zeros(shape.buffer_len(), dtype=np.float32)
-    assert out.dtype == np.float32 and out.flags.c_contiguous
-    keep_p, keep_n = None, 0
-    if mask.kind == L.RT_MASK_PADDING:
-        keep_p, keep_n = mask.keep.ctypes.data_as(C.POINTER(C.c_uint8)), mask.keep.size
-    err = L.RtErr()
-    s = shape._c()
-    rc = L.lib().rt_flash_forward_masked_f32(C.byref(s), qp, q.size, kp, k.size, vp, v.size, mask.kind, keep_p,
-                                             keep_n, out.ctypes.data_as(C.POINTER(C.c_float)), out.size,
-                                             C.byref(err))
-    raise_for(rc, err)
+    q, k, v, out = _f32(q), _f32(k), _f32(v), _out(out, shape.buffer_len())
+    keep = mask.keep if mask.kind == L.RT_MASK_PADDING else None
+    check(L.native.rt_flash_forward_masked_f32(shape, q, q.size, k, k.size, v, v.size, mask.kind, keep,
+                                               0 if keep is None else keep.size, out, out.size))
     return out
 
 
@@ -101,18 +102,11 @@ def flash_forward(shape: AttentionShape, q, k, v, out=None):
 def flash_backward(shape: AttentionShape, q, k, v, d_out, dq=None, dk=None, dv=None):
     """rustorch_attention::flash_backward (crates/rustorch-attention/src/cpu_backward.rs:46-185): gradients of
     unmasked attention.  q, k, v, d_out: flat f32 [B,H,N,D]; fills (overwrites) and returns flat f32 (dq, dk, dv)."""
-    ins = [_f32(a) for a in (q, k, v, d_out)]
-    outs = [np.zeros(shape.buffer_len(), dtype=np.float32) if o is None else o for o in (dq, dk, dv)]
-    args = []
-    for a, ptr in ins:
-        args += [ptr, a.size]
-    for o in outs:
-        assert o.dtype == np.float32 and o.flags.c_contiguous
-        args += [o.ctypes.data_as(C.POINTER(C.c_float)), o.size]
-    err = L.RtErr()
-    s = shape._c()
-    raise_for(L.lib().rt_flash_backward_f32(C.byref(s), *args, C.byref(err)), err)
-    return tuple(outs)
+    q, k, v, d_out = _f32(q), _f32(k), _f32(v), _f32(d_out)
+    dq, dk, dv = (_out(o, shape.buffer_len()) for o in (dq, dk, dv))
+    check(L.native.rt_flash_backward_f32(shape, q, q.size, k, k.size, v, v.size, d_out, d_out.size, dq, dq.size, dk, dk.size,
+                                         dv, dv.size))
+    return dq, dk, dv
 
 
 def flash_backward_workspace_bytes(shape: AttentionShape) -> int:
@@ -171,17 +165,8 @@ def flash_forward_varlen_bf16_dev(shape, q, k, v, seq_lens_dev, out, zero_padded
 def mha_flash_forward_f32(q, k, v, batch: int, seq: int, heads: int, head_dim: int, out=None):
     """rustorch_nn::attention::mha_flash_forward_f32 (crates/rustorch-nn/src/attention.rs:452-495): q, k, v flat
     f32 [B,T,H,hd]; returns flat f32 [B,T,H*hd].  Unmasked attention per (batch, head); no transposed copies."""
-    q, qp = _f32(q)
-    k, kp = _f32(k)
-    v, vp = _f32(v)
-    if out is None:
-        out = np.zeros(batch * seq * heads * head_dim, dtype=np.float32)
-    assert out.dtype == np.float32 and out.flags.c_contiguous
-    err = L.RtErr()
-    rc = L.lib().rt_mha_flash_forward_f32(qp, q.size, kp, k.size, vp, v.size,
-                                          out.ctypes.data_as(C.POINTER(C.c_float)), out.size, batch, seq, heads,
-                                          head_dim, C.byref(err))
-    raise_for(rc, err)
+    q, k, v, out = _f32(q), _f32(k), _f32(v), _out(out, batch * seq * heads * head_dim)
+    check(L.native.rt_mha_flash_forward_f32(q, q.size, k, k.size, v, v.size, out, out.size, batch, seq, heads, head_dim))
     return out
 
 
@@ -192,18 +177,10 @@ def mha_forward_masked_f32(q, k, v, batch: int, t_q: int, t_kv: int, heads: int,
     [B,t_kv,H*hd] (flat f32; t_q != t_kv is cross-attention).  `attn_mask` is an additive f32 bias with t_q*t_kv
     ([T,T] / [1,T,T]) or B*H*t_q*t_kv ([B*H,T,T]) elements, e.g. from `masks.causal_mask`, or None.  Returns flat
     f32 [B,t_q,H*hd]."""
-    q, qp = _f32(q)
-    k, kp = _f32(k)
-    v, vp = _f32(v)
-    m, mp = (None, None) if attn_mask is None else _f32(np.ravel(attn_mask))
-    if out is None:
-        out = np.zeros(batch * t_q * heads * head_dim, dtype=np.float32)
-    assert out.dtype == np.float32 and out.flags.c_contiguous
-    err = L.RtErr()
-    rc = L.lib().rt_mha_forward_masked_f32(qp, q.size, kp, k.size, vp, v.size, mp, 0 if m is None else m.size,
-                                           out.ctypes.data_as(C.POINTER(C.c_float)), out.size, batch, t_q, t_kv, heads,
-                                           head_dim, C.byref(err))
-    raise_for(rc, err)
+    q, k, v, out = _f32(q), _f32(k), _f32(v), _out(out, batch * t_q * heads * head_dim)
+    m = None if attn_mask is None else _f32(attn_mask)
+    check(L.native.rt_mha_forward_masked_f32(q, q.size, k, k.size, v, v.size, m, 0 if m is None else m.size, out, out.size,
+                                             batch, t_q, t_kv, heads, head_dim))
     return out
 
 
@@ -240,10 +217,10 @@ def mha_attention_f32(q, k, v, batch: int, t_q: int, t_kv: int, heads: int, head
     (attention.rs:325-399): projected q [B,t_q,H*hd], k, v [B,t_kv,H*hd] -> context [B,t_q,H*hd], flat f32."""
     route = mha_attention_route(t_q, t_kv, attn_mask is not None)
     if route == "identity":
-        v, _ = _f32(v)
+        v = _f32(v)
         if v.size != batch * heads * head_dim:
             raise ValueError(f"v has {v.size} elements, expected {batch * heads * head_dim}")
-        return v.copy()
+        return v.ravel().copy()
     if route == "flash":
         return mha_flash_forward_f32(q, k, v, batch, t_q, heads, head_dim)
     return mha_forward_masked_f32(q, k, v, batch, t_q, t_kv, heads, head_dim, attn_mask)

@@ -10,8 +10,11 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "../../include/rt_attn.h"
@@ -359,99 +362,338 @@ struct DevPtr {  // a device address inside a Stage's block
     void* p = nullptr;
 };
 
-struct DevBuf {
-    void* p = nullptr;
-    ~DevBuf() {
-        if (p) (void)hipFree(p);
+// 16 bytes per thread and round: uploads out of pinned memory, downloads into it
+__global__ __launch_bounds__(256) void stage_copy_kernel(uint4* dst, const uint4* src, size_t n16) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += (size_t)gridDim.x * blockDim.x) dst[i] = src[i];
+}
+hipError_t stage_copy(void* dst, const void* src, size_t bytes) {
+    hipLaunchKernelGGL(stage_copy_kernel, dim3(64), dim3(256), 0, nullptr, (uint4*)dst, (const uint4*)src, (bytes + 15) / 16);
+    return hipGetLastError();
+}
+
+// Two threads that help a host-slice call copy: the caller's tensors are as a rule not in its core's cache, and one core
+// moves them at about 30 GB/s where the bus takes 55.  A job is a list of copies taken in order by whoever is free, the
+// caller included; copy i may start when `ready` > i.  The threads sleep between jobs and end with rt_shutdown.
+class CopyCrew {
+public:
+    struct Piece {
+        char* dst;
+        const char* src;
+        size_t bytes;
+    };
+    struct Job {
+        std::vector<Piece> pieces;
+        std::unique_ptr<std::atomic<bool>[]> done;
+        std::atomic<size_t> next{0}, ready{0};
+        explicit Job(std::vector<Piece> p) : pieces(std::move(p)), done(new std::atomic<bool>[pieces.size()]) {
+            for (size_t i = 0; i < pieces.size(); i++) done[i].store(false, std::memory_order_relaxed);
+        }
+        // takes the next copy if it may start; false: nothing to take
+        bool copy_one() {
+            size_t i = next.load(std::memory_order_relaxed);
+            do {
+                if (i >= pieces.size() || ready.load(std::memory_order_acquire) <= i) return false;
+            } while (!next.compare_exchange_weak(i, i + 1, std::memory_order_relaxed));
+            memcpy(pieces[i].dst, pieces[i].src, pieces[i].bytes);
+            done[i].store(true, std::memory_order_release);
+            return true;
+        }
+        void wait(size_t i) {  // for copy i, helping meanwhile
+            while (!done[i].load(std::memory_order_acquire))
+                if (!copy_one()) __builtin_ia32_pause();
+        }
+        // copies that have not been taken are not taken any more; returns when those that have been are done
+        void close() {
+            const size_t taken = next.exchange(pieces.size(), std::memory_order_relaxed);
+            for (size_t i = 0; i < std::min(taken, pieces.size()); i++)
+                while (!done[i].load(std::memory_order_acquire)) __builtin_ia32_pause();
+        }
+        bool finished() const { return next.load(std::memory_order_relaxed) >= pieces.size(); }
+    };
+
+    // Hands a job to the helpers (one at a time: the caller holds the staging pool, and closes the job when it is through)
+    void start(const std::shared_ptr<Job>& job) {
+        {
+            std::lock_guard<std::mutex> lock(mutex_);
+            job_ = job;
+            while (threads_.size() < kHelpers) threads_.emplace_back([this] { help(); });
+        }
+        wake_.notify_all();
+    }
+    void stop() {
+        {
+            std::lock_guard<std::mutex> lock(mutex_);
+            stop_ = true;
+        }
+        wake_.notify_all();
+        for (auto& t : threads_) t.join();
+        threads_.clear();
+        stop_ = false;
+        job_.reset();
+    }
+
+private:
+    static constexpr size_t kHelpers = 2;
+    void help() {
+        std::shared_ptr<Job> last;
+        for (;;) {
+            std::shared_ptr<Job> job;
+            {
+                std::unique_lock<std::mutex> lock(mutex_);
+                wake_.wait(lock, [&] { return stop_ || (job_ && job_ != last); });
+                if (stop_) return;
+                job = last = job_;
+            }
+            while (!job->finished())
+                if (!job->copy_one()) __builtin_ia32_pause();
+        }
+    }
+    std::mutex mutex_;
+    std::condition_variable wake_;
+    std::vector<std::thread> threads_;
+    std::shared_ptr<Job> job_;
+    bool stop_ = false;
+};
+CopyCrew& crew() {
+    static CopyCrew* c = new CopyCrew;  // never destroyed: its threads may sleep in it when the process ends
+    return *c;
+}
+
+// What the host-slice entries keep between calls: pinned memory (a ring for uploads, a region for results) and, up to
+// kStageKeepBytes, the device block of the last call (hipMalloc + hipFree: 23 us per call).  One call at a time holds it.
+// Freed by rt_shutdown.
+constexpr size_t kStageInBytes = (size_t)16 << 20, kStageOutBytes = (size_t)8 << 20, kStageKeepBytes = (size_t)64 << 20;
+constexpr size_t kStageChunk = (size_t)768 << 10;
+constexpr size_t kStageDirectBytes = (size_t)512 << 10;  // results up to this size are stored into pinned memory
+constexpr size_t kStageCrewBytes = (size_t)8 << 20;  // calls that move this much share their copies with the helpers (16 MiB:
+                                                     // 640 -> 550 us; 4 MiB: 171 -> 179, their waking costs more)
+constexpr int kStageSlots = 8;
+struct StagePool {
+    std::mutex mutex;
+    char* in = nullptr;
+    char* out = nullptr;
+    hipEvent_t landed[kStageSlots] = {};
+    void* block = nullptr;
+    size_t block_bytes = 0;
+    int block_dev = -1;
+
+    bool ready() {  // false: no pinned memory to be had
+        if (in) return true;
+        bool ok = hipHostMalloc((void**)&in, kStageInBytes, hipHostMallocDefault) == hipSuccess &&
+                  hipHostMalloc((void**)&out, kStageOutBytes, hipHostMallocDefault) == hipSuccess;
+        for (auto& e : landed) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+        if (!ok) release();
+        return ok;
+    }
+    void release() {
+        if (in) (void)hipHostFree(in);
+        if (out) (void)hipHostFree(out);
+        for (auto& e : landed) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+        if (block) (void)hipFree(block);
+        in = out = nullptr;
+        block = nullptr;
+        block_bytes = 0;
+        (void)hipGetLastError();
     }
 };
+StagePool g_stage;
 
 // Staging of one host-slice call: every input, output and scratch buffer of the call sits in ONE device block.
-// Small calls (inputs + outputs within kPinnedBytes) travel through a pinned host buffer the library keeps, as one
-// host-to-device and one device-to-host transfer: a pageable hipMemcpy costs about 60 us whatever its size below
-// a megabyte, and a call has four of them.  One call at a time can hold the pinned buffer; a call that finds it
-// taken (another thread is inside a host-slice entry) or that is larger copies buffer by buffer instead.
-constexpr size_t kPinnedBytes = (size_t)4 << 20;
-std::mutex g_pinned_mutex;
-void* g_pinned = nullptr;
-
+//
+// A pageable hipMemcpy costs 60-150 us below a megabyte, and a call has four of them.  Here the inputs go through the
+// pinned ring, kStageChunk at a time, each chunk with a copy kernel behind it on the stream, so that the host copies
+// one chunk while the GPU fetches the one before (3 MiB: 93 us, against 120 in one piece and 105-125 with DMA copies,
+// which cost 10 us each; chunks of 256 KiB 112).  Results come back the same way, the host copying one chunk while the
+// next arrives; small ones are written into pinned memory by the attention kernels themselves (larger ones slow the
+// kernel down by more than the copy takes: 1 MiB of results 29 -> 47 us).  A call that finds the pool taken (another
+// thread is inside a host-slice entry) copies buffer by buffer instead.
 class Stage {
 public:
-    void in(const void* host, size_t bytes, void** dev) { items_.push_back({host, nullptr, bytes, dev, 0, 0}); }
-    void out(void* host, size_t bytes, void** dev) { items_.push_back({nullptr, host, bytes, dev, 0, 1}); }
-    void scratch(size_t bytes, void** dev) { items_.push_back({nullptr, nullptr, bytes, dev, 0, 2}); }
+    void in(const void* host, size_t bytes, void** dev) { items_.push_back({host, nullptr, bytes, dev, 0, kIn}); }
+    // whole_lines: the kernels that write this output store 16 bytes per lane, whole rows
+    void out(void* host, size_t bytes, void** dev, bool whole_lines) {
+        items_.push_back({nullptr, host, bytes, dev, 0, kOut});
+        direct_ = direct_ && whole_lines;
+    }
+    void scratch(size_t bytes, void** dev) { items_.push_back({nullptr, nullptr, bytes, dev, 0, kScratch}); }
 
-    // Allocates the block, hands out the device pointers and uploads the inputs (register inputs, then outputs,
-    // then scratch).
+    // Hands out the device pointers and enqueues the uploads (register inputs, then outputs, then scratch).
     int commit(rt_err_detail* err) {
-        size_t off = 0;
+        lock_ = std::unique_lock<std::mutex>(g_stage.mutex, std::try_to_lock);
+        if (lock_.owns_lock() && !g_stage.ready()) lock_.unlock();
+        size_t in_bytes = 0, out_bytes = 0, total = 0;
         for (auto& it : items_) {
-            it.off = off;
-            off += (it.bytes + 255) & ~(size_t)255;
-            if (it.kind == 0) in_end_ = off;
-            if (it.kind == 1) io_end_ = off;
+            if (it.kind == kIn) in_bytes += padded(it.bytes);
+            if (it.kind == kOut) out_bytes += padded(it.bytes);
         }
-        if (io_end_ < in_end_) io_end_ = in_end_;
-        HIP_TRY(hipMalloc(&block_.p, off ? off : 256), "hipMalloc staging block");
-        for (auto& it : items_) *it.dev = (char*)block_.p + it.off;
-        if (io_end_ <= kPinnedBytes) {
-            lock_ = std::unique_lock<std::mutex>(g_pinned_mutex, std::try_to_lock);
-            if (lock_.owns_lock() && !g_pinned && hipHostMalloc(&g_pinned, kPinnedBytes, hipHostMallocDefault) != hipSuccess) {
-                (void)hipGetLastError();
-                g_pinned = nullptr;
-                lock_.unlock();
+        crewed_ = in_bytes + out_bytes >= kStageCrewBytes;
+        direct_ = direct_ && lock_.owns_lock() && out_bytes <= kStageDirectBytes;
+        size_t out_off = 0;
+        for (auto& it : items_) {
+            size_t& off = (it.kind == kOut && direct_) ? out_off : total;
+            it.off = off;
+            off += padded(it.bytes);
+        }
+        int rc = get_block(total ? total : 256, err);
+        if (rc) return rc;
+        for (auto& it : items_) *it.dev = ((it.kind == kOut && direct_) ? g_stage.out : block_) + it.off;
+        if (!lock_.owns_lock()) {
+            for (auto& it : items_)
+                if (it.kind == kIn && it.bytes) HIP_TRY(hipMemcpy(*it.dev, it.host_in, it.bytes, hipMemcpyHostToDevice), "copy input");
+            return RT_OK;
+        }
+        // The inputs lie at the head of the block, one behind the other: a copy kernel moves kStageChunk of that range
+        // whatever inputs it spans.
+        std::vector<CopyCrew::Piece> pieces;
+        std::vector<Range> ranges;
+        size_t at = 0;  // position in the ring
+        for (auto& it : items_) {
+            if (it.kind != kIn) continue;
+            for (size_t done = 0; done < it.bytes;) {
+                if (ranges.empty() || ranges.back().bytes >= kStageChunk) {
+                    if (at + kStageChunk + 256 > kStageInBytes) {  // the ring is full: what is in it has to have left
+                        rc = upload(pieces, ranges, err);
+                        if (rc) return rc;
+                        HIP_TRY(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+                        pieces.clear();
+                        ranges.clear();
+                        at = 0;
+                    }
+                    ranges.push_back({it.off + done, at, 0, 0});
+                }
+                Range& r = ranges.back();
+                const size_t n = std::min(kStageChunk - r.bytes, it.bytes - done);
+                pieces.push_back({g_stage.in + at, (const char*)it.host_in + done, n});
+                done += n;
+                const size_t step = done == it.bytes ? padded(it.off + done) - (it.off + done - n) : n;  // to where the next input begins
+                at += step;
+                r.bytes += step;
+                r.end_piece = pieces.size();
             }
         }
-        if (lock_.owns_lock()) {
-            for (auto& it : items_)
-                if (it.kind == 0 && it.bytes) memcpy((char*)g_pinned + it.off, it.host_in, it.bytes);
-            if (in_end_) HIP_TRY(hipMemcpyAsync(block_.p, g_pinned, in_end_, hipMemcpyHostToDevice, nullptr), "upload");
-        } else {
-            for (auto& it : items_)
-                if (it.kind == 0 && it.bytes)
-                    HIP_TRY(hipMemcpy((char*)block_.p + it.off, it.host_in, it.bytes, hipMemcpyHostToDevice), "copy input");
-        }
-        return RT_OK;
+        return upload(pieces, ranges, err);
     }
 
     // Brings the outputs back; returns after they are in the caller's buffers.
     int fetch(rt_err_detail* err) {
-        fetched_ = true;  // every path below ends with the stream idle (or reports the failure of the attempt)
-        if (lock_.owns_lock()) {
-            if (io_end_ > in_end_)
-                HIP_TRY(hipMemcpyAsync((char*)g_pinned + in_end_, (char*)block_.p + in_end_, io_end_ - in_end_,
-                                       hipMemcpyDeviceToHost, nullptr),
-                        "download");
+        if (lock_.owns_lock() && !direct_) {
+            // chunk k travels through slot k % kStageSlots
+            constexpr size_t kSlotBytes = kStageOutBytes / kStageSlots;
+            static_assert(kStageChunk <= kSlotBytes, "a chunk fits its slot");
+            std::vector<CopyCrew::Piece> pieces;
+            std::vector<const char*> from;
+            for (auto& it : items_)
+                if (it.kind == kOut)
+                    for (size_t done = 0; done < it.bytes; done += kStageChunk) {
+                        pieces.push_back({(char*)it.host_out + done, g_stage.out + (pieces.size() % kStageSlots) * kSlotBytes,
+                                          std::min(kStageChunk, it.bytes - done)});
+                        from.push_back((const char*)*it.dev + done);
+                    }
+            const size_t n = pieces.size();
+            std::unique_ptr<Running> run;
+            if (crewed_) run.reset(new Running(pieces));
+            for (size_t sent = 0, got = 0; got < n; got++) {
+                for (; sent < n && sent < got + kStageSlots; sent++) {
+                    if (run && sent >= kStageSlots) run->job->wait(sent - kStageSlots);
+                    HIP_TRY(stage_copy((void*)pieces[sent].src, from[sent], pieces[sent].bytes), "download");
+                    HIP_TRY(hipEventRecord(g_stage.landed[sent % kStageSlots], nullptr), "hipEventRecord");
+                }
+                HIP_TRY(hipEventSynchronize(g_stage.landed[got % kStageSlots]), "hipEventSynchronize");
+                if (run) run->job->ready.store(got + 1, std::memory_order_release);
+                else memcpy(pieces[got].dst, pieces[got].src, pieces[got].bytes);
+            }
+            for (size_t i = 0; run && i < n; i++) run->job->wait(i);
+        } else if (lock_.owns_lock()) {
             HIP_TRY(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
             for (auto& it : items_)
-                if (it.kind == 1 && it.bytes) memcpy(it.host_out, (char*)g_pinned + it.off, it.bytes);
+                if (it.kind == kOut && it.bytes) memcpy(it.host_out, *it.dev, it.bytes);
         } else {
             for (auto& it : items_)
-                if (it.kind == 1 && it.bytes)
-                    HIP_TRY(hipMemcpy(it.host_out, (char*)block_.p + it.off, it.bytes, hipMemcpyDeviceToHost), "copy output");
+                if (it.kind == kOut && it.bytes)
+                    HIP_TRY(hipMemcpy(it.host_out, *it.dev, it.bytes, hipMemcpyDeviceToHost), "copy output");
         }
+        fetched_ = true;  // the stream has passed everything this call enqueued
         return RT_OK;
     }
 
     ~Stage() {
-        // an early return (a failed launch) may leave work in flight that still reads the block or the pinned buffer
-        if (block_.p && !fetched_) (void)hipStreamSynchronize(nullptr);
+        // an early return (a failed launch) may leave work in flight that still uses the block or the pinned memory
+        if (block_ && !fetched_) (void)hipStreamSynchronize(nullptr);
+        if (own_block_) (void)hipFree(own_block_);
     }
 
 private:
+    enum Kind { kIn, kOut, kScratch };
     struct Item {
         const void* host_in;
         void* host_out;
         size_t bytes;
         void** dev;
         size_t off;
-        int kind;  // 0 input, 1 output, 2 scratch
+        Kind kind;
     };
+    static size_t padded(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+
+    // A list of copies under way, with the helpers where the call is large enough; closed on every way out.
+    struct Running {
+        std::shared_ptr<CopyCrew::Job> job;
+        Running(std::vector<CopyCrew::Piece> pieces) : job(std::make_shared<CopyCrew::Job>(std::move(pieces))) { crew().start(job); }
+        ~Running() { job->close(); }
+    };
+
+    struct Range {  // of the block and of the ring, with the pieces [.., end_piece) that fill it
+        size_t block_off, ring_off, bytes, end_piece;
+    };
+
+    // The pieces into the ring, a copy kernel behind each range of it.
+    int upload(const std::vector<CopyCrew::Piece>& pieces, const std::vector<Range>& ranges, rt_err_detail* err) {
+        std::unique_ptr<Running> run;
+        if (crewed_) {
+            run.reset(new Running(pieces));
+            run->job->ready.store(pieces.size(), std::memory_order_release);
+        }
+        size_t i = 0;
+        for (const Range& r : ranges) {
+            for (; i < r.end_piece; i++) {
+                if (run) run->job->wait(i);
+                else memcpy(pieces[i].dst, pieces[i].src, pieces[i].bytes);
+            }
+            HIP_TRY(stage_copy(block_ + r.block_off, g_stage.in + r.ring_off, r.bytes), "upload");
+        }
+        return RT_OK;
+    }
+
+    int get_block(size_t bytes, rt_err_detail* err) {
+        int dev = 0;
+        HIP_TRY(hipGetDevice(&dev), "hipGetDevice");
+        if (lock_.owns_lock() && bytes <= kStageKeepBytes) {
+            if (g_stage.block_bytes < bytes || g_stage.block_dev != dev) {
+                if (g_stage.block) (void)hipFree(g_stage.block);
+                g_stage.block = nullptr;
+                g_stage.block_bytes = 0;
+                const size_t want = std::min(kStageKeepBytes, std::max(bytes + bytes / 2, (size_t)1 << 20));
+                HIP_TRY(hipMalloc(&g_stage.block, want), "hipMalloc staging block");
+                g_stage.block_bytes = want;
+                g_stage.block_dev = dev;
+            }
+            block_ = (char*)g_stage.block;
+        } else {
+            HIP_TRY(hipMalloc(&own_block_, bytes), "hipMalloc staging block");
+            block_ = (char*)own_block_;
+        }
+        return RT_OK;
+    }
+
     std::vector<Item> items_;
-    size_t in_end_ = 0, io_end_ = 0;
+    char* block_ = nullptr;
+    void* own_block_ = nullptr;  // freed with the call; null where the pool's block serves it
+    bool direct_ = true;         // results go to pinned memory straight from the kernels
+    bool crewed_ = false;        // copies are shared with the helpers
     bool fetched_ = false;
-    std::unique_lock<std::mutex> lock_;  // declared before block_: the block is freed first, then the pinned buffer released
-    DevBuf block_;
+    std::unique_lock<std::mutex> lock_;
 };
 
 }  // namespace
@@ -504,6 +746,9 @@ RT_API int rt_init(int device, rt_err_detail* err) {
     return RT_OK;
 }
 
+// The f32 kernels that store 16 bytes per lane (the others store single elements, which pinned memory does not take well).
+static bool whole_lines_f32(uint64_t dim) { return dim % 4 == 0 && dim <= 128; }
+
 // ---- prefill, host slices -------------------------------------------------------------------------
 
 RT_API int rt_flash_forward_masked_f32(const rt_attention_shape* shape, const float* q, size_t q_len, const float* k,
@@ -527,11 +772,12 @@ RT_API int rt_flash_forward_masked_f32(const rt_attention_shape* shape, const fl
     Stage st;
     void *dq, *dk, *dv, *dout, *dkeep = nullptr;
     size_t bytes = n * sizeof(float);
+    const bool lines = whole_lines_f32(shape->dim);
     st.in(q, bytes, &dq);
     st.in(k, bytes, &dk);
     st.in(v, bytes, &dv);
     if (mask_kind == RT_MASK_PADDING) st.in(keep, keep_len, &dkeep);
-    st.out(out, bytes, &dout);
+    st.out(out, bytes, &dout, lines);
     rc = st.commit(err);
     if (rc) return rc;
     rc = flash_f32_device(nullptr, shape, shape->heads, (const float*)dq, (const float*)dk, (const float*)dv, mask_kind,
@@ -618,7 +864,7 @@ RT_API int rt_gqa_forward_f32(const float* q, size_t q_len, const float* k, size
     st.in(q, q_expected * 4, &dq.p);
     st.in(k, kv_expected * 4, &dk.p);
     st.in(v, kv_expected * 4, &dv.p);
-    st.out(out, q_expected * 4, &dout.p);
+    st.out(out, q_expected * 4, &dout.p, whole_lines_f32(head_dim));
     rc = st.commit(err);
     if (rc) return rc;
     rc = gqa_device(nullptr, (const float*)dq.p, (const float*)dk.p, (const float*)dv.p, (float*)dout.p, batch, n_heads,
@@ -729,7 +975,7 @@ RT_API int rt_flash_backward_f32(const rt_attention_shape* shape, const float* q
     const float* host_in[4] = {q, k, v, d_out};
     float* host_out[3] = {dq, dk, dv};
     for (int i = 0; i < 4; i++) st.in(host_in[i], bytes, &in[i].p);
-    for (int i = 0; i < 3; i++) st.out(host_out[i], bytes, &out[i].p);
+    for (int i = 0; i < 3; i++) st.out(host_out[i], bytes, &out[i].p, whole_lines_f32(shape->dim));
     st.scratch(rt_flash_backward_workspace_bytes(shape), &ws.p);
     rc = st.commit(err);
     if (rc) return rc;
@@ -1041,7 +1287,7 @@ RT_API int rt_mha_flash_forward_f32(const float* q, size_t q_len, const float* k
     st.in(q, bytes, &dq.p);
     st.in(k, bytes, &dk.p);
     st.in(v, bytes, &dv.p);
-    st.out(out, bytes, &dout.p);
+    st.out(out, bytes, &dout.p, whole_lines_f32(head_dim));
     rc = st.commit(err);
     if (rc) return rc;
     rc = flash_f32_device(nullptr, &shape, heads, (const float*)dq.p, (const float*)dk.p, (const float*)dv.p,
@@ -1124,7 +1370,7 @@ RT_API int rt_mha_forward_masked_f32(const float* q, size_t q_len, const float* 
     st.in(k, kv_expected * 4, &dk.p);
     st.in(v, kv_expected * 4, &dv.p);
     st.in(mask, mask_len * 4, &dm.p);
-    st.out(out, q_expected * 4, &dout.p);
+    st.out(out, q_expected * 4, &dout.p, whole_lines_f32(head_dim));
     rc = st.commit(err);
     if (rc) return rc;
     rc = mha_masked_device(nullptr, (const float*)dq.p, (const float*)dk.p, (const float*)dv.p,
@@ -1827,8 +2073,8 @@ RT_API int rt_stream_destroy(void* stream, rt_err_detail* err) {
 
 RT_API int rt_shutdown(rt_err_detail* err) {
     clear_err(err);
-    // what the library keeps between calls: the per-stream scratch of rt_gqa_decode_online_bf16 and the pinned staging
-    // buffer of the host-slice entries.  The caller makes sure no call is in flight.
+    // what the library keeps between calls: the per-stream scratch of rt_gqa_decode_online_bf16 and the staging memory
+    // of the host-slice entries.  The caller makes sure no call is in flight.
     {
         std::lock_guard<std::mutex> lock(g_ws_mutex);
         for (auto& kv : g_ws) {
@@ -1839,9 +2085,9 @@ RT_API int rt_shutdown(rt_err_detail* err) {
         g_slots.clear();
     }
     {
-        std::lock_guard<std::mutex> lock(g_pinned_mutex);
-        if (g_pinned) (void)hipHostFree(g_pinned);
-        g_pinned = nullptr;
+        std::lock_guard<std::mutex> lock(g_stage.mutex);
+        crew().stop();
+        g_stage.release();
     }
     (void)hipGetLastError();
     return RT_OK;

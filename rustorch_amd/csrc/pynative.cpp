@@ -1,8 +1,8 @@
-// CPython binding of the device entries of librt_attn_hip.so: what a program calls once per layer and token, where the
-// host side of a call is what its time consists of.  A ctypes call of such an entry (a structure for the error detail,
-// a structure for the shape, one Python-level conversion per pointer, then ctypes' own conversion of every argument)
-// costs 2.9 us on top of the 2.4 us the HIP runtime takes to launch a kernel; the same call through this module costs
-// 0.9 us (4 tensors, AttentionShape, measured with torch tensors on the box's EPYC host).
+// CPython binding of the compute entries of librt_attn_hip.so: what a program calls once per layer and token, where the
+// host side of a call is what its time consists of.  Through ctypes (a structure for the error detail, a structure for
+// the shape, one Python-level conversion per pointer, then ctypes' own conversion of every argument) a call took 5.6 us
+// of host time, of which the HIP runtime needs 2.4 to launch a kernel; through this module it takes 3.7 (four torch
+// tensors and an AttentionShape).
 //
 // bind<F> turns an entry of include/rt_attn.h into a Python function by its C signature: the arguments in the entry's
 // own order without the trailing rt_err_detail*, converted by type.  It returns None for RT_OK, otherwise the tuple
@@ -92,12 +92,23 @@ bool shape_field(PyObject* o, PyObject* name, uint64_t* out) {
     return ok;
 }
 
-// One converted argument of C type T.
-template <typename T>
+// One converted argument of C type T.  Host: pointers are contiguous host buffers (numpy arrays), held for the call.
+template <typename T, bool Host>
 struct Arg {
     T v;
+    Py_buffer buf{};
+    ~Arg() {
+        if (Host && buf.obj) PyBuffer_Release(&buf);
+    }
     bool set(PyObject* o) {
-        if constexpr (std::is_pointer_v<T>) {
+        if constexpr (std::is_pointer_v<T> && Host) {
+            v = nullptr;
+            if (o == Py_None) return true;
+            constexpr bool writes = !std::is_const_v<std::remove_pointer_t<T>>;
+            if (PyObject_GetBuffer(o, &buf, PyBUF_C_CONTIGUOUS | (writes ? PyBUF_WRITABLE : 0)) != 0) return false;
+            v = (T)buf.buf;
+            return true;
+        } else if constexpr (std::is_pointer_v<T>) {
             void* p = nullptr;
             if (!as_address(o, &p)) return false;
             v = (T)p;
@@ -114,8 +125,8 @@ struct Arg {
     }
     T get() { return v; }
 };
-template <>
-struct Arg<const rt_attention_shape*> {  // an AttentionShape
+template <bool Host>
+struct Arg<const rt_attention_shape*, Host> {  // an AttentionShape
     rt_attention_shape s;
     bool set(PyObject* o) {
         return shape_field(o, s_batch, &s.batch) && shape_field(o, s_heads, &s.heads) && shape_field(o, s_seq, &s.seq) &&
@@ -124,14 +135,14 @@ struct Arg<const rt_attention_shape*> {  // an AttentionShape
     const rt_attention_shape* get() { return &s; }
 };
 
-template <auto F>
+template <auto F, bool Host>
 struct Bind;
-template <typename... A, int (*F)(A...)>
-struct Bind<F> {
+template <typename... A, int (*F)(A...), bool Host>
+struct Bind<F, Host> {
     static constexpr size_t N = sizeof...(A) - 1;  // without the error detail
     template <size_t... I>
     static PyObject* go(PyObject* const* args, std::index_sequence<I...>) {
-        std::tuple<Arg<std::tuple_element_t<I, std::tuple<A...>>>...> c;
+        std::tuple<Arg<std::tuple_element_t<I, std::tuple<A...>>, Host>...> c;
         if (!(std::get<I>(c).set(args[I]) && ...)) return nullptr;
         rt_err_detail err;
         int rc;
@@ -151,7 +162,8 @@ struct Bind<F> {
     }
 };
 
-#define RT_BIND(name) {#name, (PyCFunction)(void (*)(void)) & Bind<&name>::call, METH_FASTCALL, nullptr}
+#define RT_BIND(name) {#name, (PyCFunction)(void (*)(void)) & Bind<&name, false>::call, METH_FASTCALL, nullptr}
+#define RT_BIND_HOST(name) {#name, (PyCFunction)(void (*)(void)) & Bind<&name, true>::call, METH_FASTCALL, nullptr}
 
 PyMethodDef methods[] = {
     RT_BIND(rt_flash_forward_f32_dev),
@@ -176,6 +188,11 @@ PyMethodDef methods[] = {
     RT_BIND(rt_gqa_decode_batched_bf16_noalloc),
     RT_BIND(rt_gqa_decode_chunk_bf16),
     RT_BIND(rt_i32_add_dev),
+    RT_BIND_HOST(rt_flash_forward_masked_f32),
+    RT_BIND_HOST(rt_flash_backward_f32),
+    RT_BIND_HOST(rt_gqa_forward_f32),
+    RT_BIND_HOST(rt_mha_flash_forward_f32),
+    RT_BIND_HOST(rt_mha_forward_masked_f32),
     {nullptr, nullptr, 0, nullptr},
 };
 
