@@ -1059,9 +1059,8 @@ RT_API int rt_flash_forward_f32_dev(void* stream, const rt_attention_shape* shap
 }
 
 // Which bf16 prefill kernel serves a call.  RT_ATTN_BF16_PREFILL=tile|persistent|wide in the environment forces one
-// where it applies (for measurements and tests); otherwise the persistent 8-wave kernel takes head dim 128 (and head
-// dim 64 under a key-padding mask) on unpadded batches with at least 512 rows per sequence and a job for every CU,
-// and the 4-wave tile kernel everything else.
+// where it applies (for measurements and tests); otherwise flash_bf16_common weighs the persistent 8-wave kernel
+// against the 4-wave tile kernel.
 enum class PrefillKernel { kAuto, kTile, kPersistent, kWide };
 // A debug switch for measurements and tests, not part of the reference's surface: rt_debug_force_bf16_prefill_kernel
 // sets it; until that is called, the value is what RT_ATTN_BF16_PREFILL=tile|persistent held when the library made its
@@ -1144,23 +1143,40 @@ static int flash_bf16_common(void* stream, const rt_attention_shape* shape, uint
         HIP_TRY(rt::launch_attn_rows_bf16((hipStream_t)stream, r), "attn_rows_bf16 launch");
         return strict_pass((hipStream_t)stream, shape, n_kv_heads, v, out, seq_lens, mask, bnhd, true, err);
     }
-    // the persistent kernel needs a job (256 query rows of one head) for every CU and gains on the tile kernel as the
-    // rows get longer; a padded batch is a set of jobs of very different lengths, which the tile kernel's
-    // dispatcher-balanced workgroups handle better
-    const bool persistent_dim = shape->dim == 64 || shape->dim == 128;
+    // The persistent kernel needs a job (256 query rows of one head) for every CU and long rows; it multiplies faster than
+    // the tile kernel, which balances better: 128-row workgroups that the dispatcher hands out, against whole jobs dealt
+    // beforehand.  Head dim 64 is the tile kernel's on every shape tried (N = 700 .. 32768, 3-26 %), and so is a padded
+    // batch, a set of jobs of very different lengths.  At head dim 128 the two are weighed by what their busiest worker
+    // has to do: a persistent step (256 rows x 128 keys) takes 3.15 us, four tile steps (128 rows x 64 keys) 3.85 us, and
+    // either kernel two and a half steps around every job.  (us, persistent / tile, causal, 32 / 8 heads: 2 sequences of
+    // 1100 32.6 / 31.1, 1501 45.5 / 46.8, 2048 70.5 / 74.9, 2500 112.8 / 109.9; 1 of 2048 48.4 / 43.8, 4096 124 / 136.)
+    // Under a key-padding mask the tile kernel takes another fifth longer and the persistent one stays ahead.
+    rt::FlashBf16Params p{};
+    p.batch = (int)shape->batch;
+    p.heads = (int)shape->heads;
+    p.kv_heads = (int)n_kv_heads;
+    p.group = (int)(shape->heads / n_kv_heads);
+    p.seq = (int)shape->seq;
+    p.dim = (int)shape->dim;
+    p.mask = mask;
+    p.n_workers = g_num_cus;
     const uint64_t jobs256 = (shape->seq + 255) / 256 * shape->batch * shape->heads;
-    bool persistent = persistent_dim && shape->seq >= 512 && jobs256 >= (uint64_t)g_num_cus && mask != rt::kMaskVarlenCausal;
+    bool persistent = shape->dim == 128 && shape->seq >= 512 && jobs256 >= (uint64_t)g_num_cus && mask != rt::kMaskVarlenCausal;
     const PrefillKernel forced = prefill_kernel_override();
     if (forced == PrefillKernel::kTile || forced == PrefillKernel::kWide) persistent = false;
-    // head dim 64 exactly, no mask or the causal one: the tile kernel (whose K/V tiles go straight from memory to LDS
-    // at this head dim) measured ahead of the persistent kernel on every shape tried (N = 1024 .. 32768, 4-9 %) and
-    // level with the kernel of 64 query rows per wave, which therefore runs only when it is asked for
-    if (forced == PrefillKernel::kAuto && shape->dim == 64 && (mask == rt::kMaskNone || mask == rt::kMaskCausal)) persistent = false;
-    if (forced == PrefillKernel::kPersistent && persistent_dim) persistent = true;
+    if (forced == PrefillKernel::kPersistent && (shape->dim == 64 || shape->dim == 128)) persistent = true;
     if (mask == rt::kMaskPadding && shape->seq > (uint64_t)rt::kFlashBf16MaxPaddingKeys) persistent = false;
     if (persistent) {  // that kernel addresses the rows of one (batch, head) slab with 32-bit byte offsets
         const uint64_t pitch_b = (bnhd ? shape->heads : 1) * shape->dim * 2;
         if (shape->seq * pitch_b >= (1ull << 32)) persistent = false;
+    }
+    if (persistent) {
+        const float busiest = rt::plan_flash_bf16(p);
+        if (forced == PrefillKernel::kAuto && mask != rt::kMaskPadding) {
+            const float tiles = (float)((shape->seq + 127) / 128);  // of 128 rows, each 64 keys a step
+            const float steps = tiles * ((mask == rt::kMaskCausal ? tiles + 1.0f : 2.0f * tiles) + 2.5f) * (float)(shape->batch * shape->heads);
+            if (3.85f * steps / (4.0f * (float)g_num_cus) + 2.0f < 3.15f * busiest) persistent = false;
+        }
     }
     const int dim = (int)shape->dim;
     rt::TensorLayout lq, lkv;
@@ -1204,24 +1220,15 @@ static int flash_bf16_common(void* stream, const rt_attention_shape* shape, uint
         HIP_TRY(rt::launch_flash_tile_bf16((hipStream_t)stream, t), "flash_tile_bf16 launch");
         return strict_pass((hipStream_t)stream, shape, n_kv_heads, v, out, seq_lens, mask, bnhd, true, err);
     }
-    rt::FlashBf16Params p;
     p.q = (const uint16_t*)q;
     p.k = (const uint16_t*)k;
     p.v = (const uint16_t*)v;
     p.out = (uint16_t*)out;
     p.keep = keep;
     p.seq_lens = seq_lens;
-    p.batch = (int)shape->batch;
-    p.heads = (int)shape->heads;
-    p.kv_heads = (int)n_kv_heads;
-    p.group = (int)(shape->heads / n_kv_heads);
-    p.seq = (int)shape->seq;
-    p.dim = dim;
-    p.mask = mask;
     p.ref_bc = ref_bc;
     p.zero_padded_rows = zero_padded_rows;
     p.scale_log2e = scale * rt::kLog2eHost;
-    p.n_workers = g_num_cus;
     p.lq = p.lo = lq;
     p.lkv = lkv;
     HIP_TRY(rt::launch_flash_bf16((hipStream_t)stream, p), "flash_fwd_bf16 launch");

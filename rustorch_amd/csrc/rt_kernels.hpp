@@ -88,10 +88,13 @@ struct FlashBf16Params {
     int zero_padded_rows;
     float scale_log2e;  // (1/sqrt(dim)) * log2(e)
     int n_workers;      // persistent workgroups to launch: the number of CUs
+    int rank_major;     // the order in which an XCD's jobs are dealt (plan_flash_bf16)
     TensorLayout lq, lkv, lo;  // layouts of q, of k and v, of out; seq * row_pitch * 2 bytes must stay below 2^32
 };
 // dim in {64, 128}; a padding mask (kMaskPadding) of at most kFlashBf16MaxPaddingKeys keys.
 constexpr int kFlashBf16MaxPaddingKeys = 65536;
+// Chooses the order the jobs are dealt in; returns the load of the busiest worker, in steps of 128 keys for 256 rows.
+float plan_flash_bf16(FlashBf16Params& p);
 hipError_t launch_flash_bf16(hipStream_t stream, const FlashBf16Params& p);
 
 // The general bf16 forward (flash_bf16_tile.hip): any dim <= 256 that is a multiple of 8, own key count, per-sequence
