@@ -189,10 +189,14 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
     // one XCD and share K and V through its L2.
     const int G = PACKED ? p.pack : 1;  // heads per packed row block (1: rows are positions of one head)
     const int rows_total = p.seq_q * G;
-    const int hx = blockIdx.x, b = blockIdx.y;
-    const int zz = (int)gridDim.z - 1 - (int)blockIdx.z;
-    // kv head: hx itself when rows are packed, else hx / group (group_magic = 2^32 / group + 1, exact below 2^16 heads)
-    const int kvh = (PACKED || p.group_magic == 0) ? hx : (int)__umulhi((uint32_t)hx, p.group_magic);
+    // The heads of a GQA group follow one another at a distance of kv_heads in the grid, so that a group lands on one XCD
+    // (or on those its kv heads leave it) and shares its keys through that L2: grid position x is head x / kv_heads of
+    // group x % kv_heads (kv_magic = 2^32 / kv_heads + 1, exact below 2^16 heads; 0 where every head has its own keys).
+    const int b = blockIdx.y;
+    const int gx = PACKED ? 0 : (int)__umulhi(blockIdx.x, p.kv_magic);
+    const int kvh = (int)blockIdx.x - gx * p.kv_heads;
+    const int hx = PACKED ? kvh : kvh * p.group + gx;
+    const int zz = p.n_qtiles - 1 - (int)blockIdx.z;
     const int h0 = PACKED ? hx * G : hx;  // head of a row with g = 0
     const int D = p.dim;
 
@@ -270,6 +274,12 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
             }
         }
     }
+
+    // The rest of the arguments, requested together: left to itself the compiler loads a field where it is first used
+    // and waits for a line at a time.
+    asm volatile("" ::"s"(p.q), "s"(p.out), "s"(p.q_lens), "s"(p.kv_lens), "s"(p.seq_q), "s"(p.zero_padded_rows), "s"(p.scale_log2e),
+                 "s"(p.lq.batch_stride), "s"(p.lq.head_stride), "s"(p.lq.row_pitch), "s"(p.lo.batch_stride),
+                 "s"(p.lo.head_stride), "s"(p.lo.row_pitch));
 
     // (DIRECT reads the lengths through the constant address space -- nothing writes them during the launch: behind
     // the assembly statements of the tile requests, which count as writers of memory, the compiler would otherwise
@@ -1136,8 +1146,9 @@ __global__ __launch_bounds__(256, 2) void flash_wide_bf16_kernel(FlashTileParams
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hh = lane >> 5;
     const int rows_total = p.seq_q;
-    const int hx = blockIdx.x, b = blockIdx.y;
-    const int kvh = p.group_magic == 0 ? hx : (int)__umulhi((uint32_t)hx, p.group_magic);
+    const int b = blockIdx.y;
+    const int gx = (int)__umulhi(blockIdx.x, p.kv_magic);  // (as in the tile kernel)
+    const int kvh = (int)blockIdx.x - gx * p.kv_heads, hx = kvh * p.group + gx;
     const uint16_t* const Kg = p.k + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
     const uint16_t* const Vg = p.v + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
 
@@ -1169,7 +1180,7 @@ __global__ __launch_bounds__(256, 2) void flash_wide_bf16_kernel(FlashTileParams
     const int n_q = p.q_lens ? min(max(p.q_lens[b], 0), p.seq_q) : p.seq_q;          // valid query positions
     const int n_keys = p.kv_lens ? min(max(p.kv_lens[b], 0), p.seq_kv) : p.seq_kv;  // keys that exist
     // rank of the query tile: the last one first; in a padded batch counted from the sequence's own last valid tile
-    int qtile = (int)gridDim.z - 1 - (int)blockIdx.z;
+    int qtile = p.n_qtiles - 1 - (int)blockIdx.z;
     if (p.q_lens) {
         const int n_qt = (n_q + WROWS - 1) / WROWS;
         const int rank = (int)blockIdx.z;
@@ -1614,6 +1625,20 @@ bool flash_tile_bf16_addressable(long long seq_kv, long long row_pitch) {
     return seq_kv >= 0 && row_pitch > 0 && (unsigned long long)(seq_kv + 512) * (unsigned long long)row_pitch * 2ull < (1ull << 32);
 }
 
+// What the kernels take grid positions for heads by.
+static void set_grid_order(FlashTileParams& p, long long z) {
+    p.n_qtiles = (int)z;
+    p.kv_magic = 0;
+    if (p.pack > 1 || p.decode_rows || p.group == 1) return;
+    if (p.kv_heads == 1) {  // (2^32 / 1 does not fit the multiplier) every head with keys of its own, at the same address
+        p.kv_heads = p.heads;
+        p.group = 1;
+        p.lkv.head_stride = 0;
+        return;
+    }
+    p.kv_magic = (uint32_t)(0x100000000ull / (unsigned long long)p.kv_heads) + 1u;
+}
+
 // 64 rows per wave: head dim 64 exactly, rows of one head, masks none / causal (with or without per-sequence lengths)
 bool flash_wide_bf16_supported(const FlashTileParams& p) {
     return p.dim == 64 && p.pack <= 1 && !p.bias && p.n_splits <= 1 && (p.mask == kMaskNone || p.mask == kMaskCausal) &&
@@ -1627,7 +1652,7 @@ hipError_t launch_flash_wide_bf16(hipStream_t stream, const FlashTileParams& par
     const long long n_qtiles = ((long long)p.seq_q + WROWS - 1) / WROWS;
     if (p.batch > 65535 || n_qtiles > 65535 || p.heads > 65535) return hipErrorInvalidValue;  // grid limits
     p.pack = 1;
-    p.group_magic = p.group > 1 ? (uint32_t)(0x100000000ull / (unsigned long long)p.group) + 1u : 0u;
+    set_grid_order(p, n_qtiles);
     dim3 grid((unsigned)p.heads, (unsigned)p.batch, (unsigned)n_qtiles);
     if (p.mask == kMaskCausal) hipLaunchKernelGGL(flash_wide_bf16_kernel<kMaskCausal>, grid, dim3(256), 0, stream, p);
     else hipLaunchKernelGGL(flash_wide_bf16_kernel<kMaskNone>, grid, dim3(256), 0, stream, p);
@@ -1649,7 +1674,7 @@ hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& par
     if (p.n_splits > 1 && (p.pack != p.group || p.bias || p.mask != kMaskCausal || !p.part_o || !p.part_ml))
         return hipErrorInvalidValue;  // the chunked decode only
     if (p.batch > 65535 || n_qtiles * p.n_splits > 65535 || heads_u > 65535 || p.group < 1) return hipErrorInvalidValue;  // grid limits
-    p.group_magic = p.group > 1 ? (uint32_t)(0x100000000ull / (unsigned long long)p.group) + 1u : 0u;
+    set_grid_order(p, n_qtiles * p.n_splits);
     dim3 grid((unsigned)heads_u, (unsigned)p.batch, (unsigned)(n_qtiles * p.n_splits));
     if (p.dim <= 32) return launch_dp<32>(stream, p, grid);
     if (p.dim <= 64) return launch_dp<64>(stream, p, grid);

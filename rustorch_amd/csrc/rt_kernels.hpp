@@ -1,6 +1,7 @@
 // Kernel parameter blocks and launchers shared between the kernel files and the C ABI.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace rt {
@@ -99,33 +100,32 @@ hipError_t launch_flash_bf16(hipStream_t stream, const FlashBf16Params& p);
 
 // The general bf16 forward (flash_bf16_tile.hip): any dim <= 256 that is a multiple of 8, own key count, per-sequence
 // query / key counts, causal mask aligned to the last key, key-padding vector, additive f32 bias, packed GQA rows.
+// The order of the fields is that of their use in the kernel: the launch's arguments are read from memory 64 bytes at a
+// time, and the first line holds all that the first requests for keys need.
 struct FlashTileParams {
-    const uint16_t* q;
     const uint16_t* k;
     const uint16_t* v;
+    TensorLayout lkv;
+    int seq_kv, dim;
+    int kv_heads, group;
+    uint32_t kv_magic;        // set by the launcher: 2^32 / kv_heads + 1, for a division by a multiply (0 when group is 1)
+    int n_qtiles;             // set by the launcher: the grid's z
+    // ---- second line
+    const uint16_t* q;
     uint16_t* out;
-    const uint8_t* keep;      // kMaskPadding: device, seq_kv bytes
+    TensorLayout lq, lo;
+    // ---- third line
     const int32_t* q_lens;    // optional device int32[batch]: valid query positions (rows past them are padding)
     const int32_t* kv_lens;   // optional device int32[batch]: keys that exist
-    const float* bias;        // optional additive score bias, f32 rows of seq_kv per query position, added after scaling
-    long long bias_bh_stride; // elements between the biases of consecutive (batch, head) pairs; 0 = one for all
-    int bias_vec4;            // bias rows may be read 16 bytes at a time (base and seq_kv * 4 bytes both 16-byte aligned)
-    int batch, heads, kv_heads, group;
-    uint32_t group_magic;     // set by the launcher: 2^32 / group + 1 (0 when group is 1), for head / group by a multiply
+    int seq_q;
+    float scale_log2e;        // (1/sqrt(dim)) * log2(e)
+    int zero_padded_rows;     // rows past q_lens[b]: +0.0 (else NaN)
     // 1: a tile's rows are positions of one head.  group: rows run over (position, head of the GQA group), row
     // r = position * group + head-in-group, so that all heads of a kv head share one pass over its keys.
     int pack;
-    // rows are positions of a chunked decode over a cache: a position that sees no key is a row of zeros (the
-    // reference's decode kernels leave it so), not the NaN row of flash_forward.  Implied by pack > 1; a group of one
-    // head sets it.
-    int decode_rows;
-    int seq_q, seq_kv, dim;
-    int mask;   // kMaskNone, kMaskCausal (key j visible to position i iff j <= i + (keys - valid queries)), kMaskPadding
-    int ref_bc;
-    int zero_padded_rows;  // rows past q_lens[b]: +0.0 (else NaN)
-    float scale_log2e;     // (1/sqrt(dim)) * log2(e)
-    float scale;           // 1/sqrt(dim)
-    TensorLayout lq, lkv, lo;
+    // Sliding window (causal mask only, unpacked rows, no bias; 0 = none): position i sees the `window` keys that end
+    // with key i + (keys - valid queries), as sliding_window_mask builds it (crates/rustorch-nn/src/masks.rs:41-60).
+    int window;
     // Split over the keys (packed rows only; zero-initialise to leave it off): n_splits > 1 cuts every (sequence, kv
     // head)'s walk into that many spans of whole tiles; each leaves a partial per packed row in part_o
     // ([batch, kv_heads, seq_q * pack, n_splits, dim] f32) and part_ml (the same index, (m, l) pairs), and a second
@@ -133,10 +133,21 @@ struct FlashTileParams {
     int n_splits;
     float* part_o;
     float* part_ml;
-    // Sliding window (causal mask only, unpacked rows, no bias; 0 = none): position i sees the `window` keys that end
-    // with key i + (keys - valid queries), as sliding_window_mask builds it (crates/rustorch-nn/src/masks.rs:41-60).
-    int window;
+    // ---- what only some forms read
+    const uint8_t* keep;      // kMaskPadding: device, seq_kv bytes
+    const float* bias;        // optional additive score bias, f32 rows of seq_kv per query position, added after scaling
+    long long bias_bh_stride; // elements between the biases of consecutive (batch, head) pairs; 0 = one for all
+    int bias_vec4;            // bias rows may be read 16 bytes at a time (base and seq_kv * 4 bytes both 16-byte aligned)
+    float scale;              // 1/sqrt(dim)
+    int ref_bc;
+    int batch, heads;
+    int mask;   // kMaskNone, kMaskCausal (key j visible to position i iff j <= i + (keys - valid queries)), kMaskPadding
+    // rows are positions of a chunked decode over a cache: a position that sees no key is a row of zeros (the
+    // reference's decode kernels leave it so), not the NaN row of flash_forward.  Implied by pack > 1; a group of one
+    // head sets it.
+    int decode_rows;
 };
+static_assert(offsetof(FlashTileParams, q) == 64 && offsetof(FlashTileParams, q_lens) == 128, "lines of the arguments");
 bool flash_tile_bf16_supported(int dim);
 // keys per LDS tile of the tile kernel at head dim `dim` (the unit the split over the keys is cut in)
 int flash_tile_bf16_key_tile(int dim);
