@@ -266,7 +266,12 @@ int stream_workspace(hipStream_t stream, size_t bytes, float** out, rt_err_detai
         // grow geometrically, so that a context that lengthens token by token retires a handful of blocks at most
         size_t want = std::max<size_t>(std::max<size_t>(bytes, (size_t)1 << 20), 2 * w.bytes);
         void* fresh = nullptr;
-        HIP_TRY(hipMalloc(&fresh, want), "hipMalloc workspace");
+        // (another thread may be capturing its own stream, which an allocation would end with an error)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
+        const hipError_t got = hipMalloc(&fresh, want);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        HIP_TRY(got, "hipMalloc workspace");
         if (w.ptr) w.retired.push_back(w.ptr);
         w.ptr = fresh;
         w.bytes = want;
@@ -1749,6 +1754,36 @@ RT_API int rt_gqa_decode_naive_bf16(void* stream, const void* q, const void* k_c
     return rt_gqa_decode_online_bf16(stream, q, k_cache, v_cache, out, n_heads, n_kv, kv_len, head_dim, max_seq, err);
 }
 
+namespace {
+// Into how many spans the keys of a chunk's units are cut: the cheapest of a workgroup's tile steps (1.15 us at head dim
+// 128 with a CU to itself, half as much again for every workgroup that shares it) plus, when there are spans, the merge
+// launch (4 us) and the partials' way to memory and back (4.5 TB/s).  Over 30 shapes (2 to 512 positions, 700 to 8192
+// keys, head dims 64 to 256) its choice is within 3 % of the best count measured, 6 % at one of them.  One sequence, 32
+// heads over 8, 8192 keys: 16 positions 119 -> 15.3 us (32 spans), 128 positions 123 -> 29.3 us (8), 512 positions 122
+// -> 74 us (4).
+// Units that fill the chip by themselves are not cut, and no span is shorter than two key tiles.
+long long chunk_splits(long long slabs, long long rows, int head_dim, long long keys) {
+    const long long key_tile = rt::flash_tile_bf16_key_tile(head_dim), tiles = (keys + key_tile - 1) / key_tile;
+    const long long units = slabs * ((rows + 127) / 128);
+    if (units >= g_num_cus || tiles < 4) return 1;
+    const long long occ = rt::flash_tile_bf16_workgroups(head_dim);
+    const float step_us = 1.15f * (float)key_tile * (float)head_dim / (64.0f * 128.0f);
+    const float partial_us = (float)(slabs * rows) * (float)(head_dim + 2) * (2 * sizeof(float)) / 4.5e6f;
+    long long best = 1;
+    float best_us = 0.0f;
+    for (long long n = 1; n <= std::min<long long>(tiles / 2, 64) && (n - 1) * units < occ * g_num_cus; n++) {
+        const long long per_cu = (units * n + g_num_cus - 1) / g_num_cus, rounds = per_cu / occ, rest = per_cu % occ;
+        const float load = 0.5f * (float)(rounds * (occ + 1) + (rest ? rest + 1 : 0));
+        const float us = (float)((tiles + n - 1) / n) * step_us * load + (n > 1 ? 4.0f + (float)n * partial_us : 0.0f);
+        if (n == 1 || us < best_us) {
+            best = n;
+            best_us = us;
+        }
+    }
+    return best;
+}
+}  // namespace
+
 // Several new positions per sequence against the cache, causally masked: the bf16 form of gqa_decode_batched_f32
 // (crates/rustorch-metal/src/kernels.rs:14432-14516), batched over sequences with their own context lengths.
 RT_API int rt_gqa_decode_chunk_bf16(void* stream, const void* q, const void* k_cache, const void* v_cache, void* out,
@@ -1798,32 +1833,36 @@ RT_API int rt_gqa_decode_chunk_bf16(void* stream, const void* q, const void* k_c
     t.scale_log2e = t.scale * rt::kLog2eHost;
     t.lq = t.lo = rt::layout_bnhd((long long)n_heads, (long long)seq_new, head_dim);
     t.lkv = rt::layout_bhnd((long long)n_kv, (long long)max_seq, head_dim);
-    // Few (sequence, kv head, query tile) units and a long cache -- the reference's own call shape, one sequence:
-    // cut the keys into spans so that every CU has a workgroup (two per CU measured 20 % slower at four new positions,
-    // the same at sixteen), each span at least two key tiles long.  The
-    // partials go to this stream's slot of the library's fixed scratch block (nothing is allocated); with no slot free,
-    // to the buffer the library allocates per stream.
-    const long long units = (long long)batch * n_kv * (((long long)seq_new * group + 127) / 128);
-    const int key_tile = rt::flash_tile_bf16_key_tile(head_dim);
-    const long long tiles_max = ((long long)t.seq_kv + key_tile - 1) / key_tile;
-    long long n_splits = 1;
-    if (units < g_num_cus && tiles_max >= 4)
-        n_splits = std::min<long long>(std::min<long long>((g_num_cus + units - 1) / units, tiles_max / 2), 64);
+    // Few (sequence, kv head, query tile) units and a long cache -- the reference's own call shape, one sequence: cut the
+    // keys into spans (chunk_splits).  The partials go to this stream's slot of the library's fixed scratch block where
+    // it holds them, else to the buffer the library keeps per stream; under capture, where that one cannot be allocated,
+    // to as many spans as the slot holds.
+    const long long rows = (long long)seq_new * group;
+    long long n_splits = chunk_splits((long long)batch * n_kv, rows, head_dim, t.seq_kv);
+    float* ws = nullptr;
+    const size_t part_rows = (size_t)batch * n_kv * (size_t)((rows + 31) / 32 * 32);
+    const size_t per_split = part_rows * ((size_t)head_dim + 2) * sizeof(float);
     if (n_splits > 1) {
-        const size_t per_split = (size_t)batch * n_kv * (size_t)seq_new * group * ((size_t)head_dim + 2) * sizeof(float);
-        float* ws = nullptr;
         size_t slot_bytes = 0;
         rc = stream_slot_scratch((hipStream_t)stream, &ws, &slot_bytes, err);
         if (rc) return rc;
-        if (ws && slot_bytes / per_split >= 2) {
-            n_splits = std::min<long long>(n_splits, (long long)(slot_bytes / per_split));
-        } else {
-            rc = stream_workspace((hipStream_t)stream, per_split * (size_t)n_splits, &ws, err);
-            if (rc) return rc;
+        if (!ws || slot_bytes < per_split * (size_t)n_splits) {
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (ws && stream) HIP_TRY(hipStreamIsCapturing((hipStream_t)stream, &cap), "hipStreamIsCapturing");
+            float* kept = nullptr;
+            if (cap == hipStreamCaptureStatusNone) {
+                rc = stream_workspace((hipStream_t)stream, per_split * (size_t)n_splits, &kept, err);
+                if (rc && !ws) return rc;
+                clear_err(err);
+            }
+            if (kept) ws = kept;
+            else n_splits = (long long)(slot_bytes / per_split);  // (below two: the call runs without partials)
         }
+    }
+    if (n_splits > 1) {
         t.n_splits = (int)n_splits;
         t.part_o = ws;
-        t.part_ml = ws + (size_t)batch * n_kv * (size_t)seq_new * group * (size_t)n_splits * (size_t)head_dim;
+        t.part_ml = ws + part_rows * (size_t)n_splits * (size_t)head_dim;
     }
     HIP_TRY(rt::launch_flash_tile_bf16((hipStream_t)stream, t), "flash_tile_bf16 launch");
     return RT_OK;

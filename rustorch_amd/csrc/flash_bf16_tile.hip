@@ -961,24 +961,21 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
     // 16 bytes per lane.
     const float l = t_sum_with_other_half(l_run);
     if constexpr (SPLIT) {
-        // the partial of this span: O as accumulated (relative to the running max as it stands), that max in the exp2
+        // The partial of this span: O as accumulated (relative to the running max as it stands), that max in the exp2
         // domain, the row sum.  A workgroup without tiles, or a row that saw no key of the span, leaves (0, -inf, 0).
+        // Stored as it stands in the registers, 32 rows to a block: eight columns of the 32 rows are 1 KB in one piece
+        // (row by row, 16 bytes here and there, the stores took 1-2 us of a short span).
         const int r = q0 + 32 * wq + col;
         if (r < rows_total) {
-            const size_t slot = (((size_t)b * p.kv_heads + kvh) * (size_t)rows_total + (size_t)r) * (size_t)p.n_splits + (size_t)split;
-            float* const po = p.part_o + slot * (size_t)D;
+            const size_t block = (((size_t)b * p.kv_heads + kvh) * (size_t)((rows_total + 31) / 32) + (size_t)(q0 / 32 + wq)) * (size_t)p.n_splits + (size_t)split;
+            float* const po = p.part_o + block * (size_t)(32 * D) + 4 * lane;
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int d0 = 32 * dt + 8 * j + 4 * hh;
-                    if (d0 < D)
-                        *(f32x4_t*)(po + d0) = f32x4_t{acc_o[dt][4 * j], acc_o[dt][4 * j + 1], acc_o[dt][4 * j + 2], acc_o[dt][4 * j + 3]};
-                }
-            if (hh == 0) {
-                p.part_ml[2 * slot] = m_run * cc;
-                p.part_ml[2 * slot + 1] = l;
-            }
+                for (int j = 0; j < 4; j++)
+                    if (32 * dt + 8 * j < D)
+                        *(f32x4_t*)(po + 256 * (4 * dt + j)) = f32x4_t{acc_o[dt][4 * j], acc_o[dt][4 * j + 1], acc_o[dt][4 * j + 2], acc_o[dt][4 * j + 3]};
+            p.part_ml[64 * block + lane] = hh == 0 ? m_run * cc : l;
         }
         return;
     }
@@ -1063,59 +1060,108 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
     }
 }
 
-// Folds the partials the SPLIT kernel leaves: thread (row, d) walks the row's n_splits partials (o[d], m, l), weighs each
-// by 2^(m - max m) and writes o / l as bf16 where the unsplit kernel would have written the row.  No partial with a
-// key (every m is -inf): the position sees no key at all, a row of zeros.
+// Folds the partials the SPLIT kernel leaves: each is weighed by 2^(m - max m), o / l goes out as bf16 where the unsplit
+// kernel would have written the row.  No partial with a key (every m is -inf): the position sees no key at all, a row
+// of zeros.  A wave takes eight columns of 32 rows, as the partials hold them: 1 KB a load, and a lane's weights are its
+// own row's.  With many partials the four waves of a workgroup share them out (PARTS) and meet in LDS: a wave has eight
+// loads of each kind in flight, and a latency for every eight is what the kernel takes.
+template <bool PARTS>
 __global__ __launch_bounds__(256) void flash_split_merge_kernel(FlashTileParams p) {
-    const int D = p.dim, G = p.pack;
-    const size_t rows_total = (size_t)p.seq_q * G;
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t row_all = idx / (size_t)D;
-    const int d = (int)(idx - row_all * (size_t)D);
-    if (row_all >= (size_t)p.batch * p.kv_heads * rows_total) return;
-    const size_t r = row_all % rows_total, bk = row_all / rows_total;
-    const int kvh = (int)(bk % (size_t)p.kv_heads), b = (int)(bk / (size_t)p.kv_heads);
-    const float* ml = p.part_ml + 2 * row_all * (size_t)p.n_splits;
-    const float* po = p.part_o + row_all * (size_t)p.n_splits * (size_t)D + d;
-    // One pass, eight partials at a time: the loads of a group are independent of each other (a dependent load per
-    // partial would cost a memory latency each), and the running (m, acc, l) is rescaled once per group.
     constexpr int kGroup = 8;
-    float m_all = neg_inf(), acc = 0.0f, l_all = 0.0f;
+    __shared__ float fold[PARTS ? 3 : 1][6][64];
+    const int D = p.dim, G = p.pack, n = p.n_splits, lane = threadIdx.x % 64;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint32_t rows_total = (uint32_t)p.seq_q * (uint32_t)G, blocks = (rows_total + 31) / 32, pieces = (uint32_t)D / 8;
+    const uint32_t item = PARTS ? blockIdx.x : 4 * blockIdx.x + wave;
+    if (item >= (uint32_t)p.batch * (uint32_t)p.kv_heads * blocks * pieces) return;  // (PARTS: one item per workgroup, all there)
+    const uint32_t block = item / pieces, piece = item - block * pieces, bk = block / blocks;
+    const uint32_t r = (block - bk * blocks) * 32 + (lane & 31);
+    const uint32_t b = bk / (uint32_t)p.kv_heads, kvh = bk - b * (uint32_t)p.kv_heads;
+    const bool row_in = r < rows_total;
+    const float* const ml = p.part_ml + (size_t)block * n * 64 + (lane & 31);
+    const float* const po = p.part_o + (size_t)block * n * (32 * D) + 256 * piece + 4 * lane;
+
+    constexpr int STEP = PARTS ? 4 : 1;
+    float m_all = neg_inf(), l_all = 0.0f;
+    f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
     bool nan_m = false;
-    for (int k0 = 0; k0 < p.n_splits; k0 += kGroup) {
-        float mv[kGroup], lv[kGroup], ov[kGroup];
+    if (row_in) {
+        for (int k0 = PARTS ? (int)wave : 0; k0 < n; k0 += kGroup * STEP) {
+            float mv[kGroup], lv[kGroup];
+            f32x4_t ov[kGroup];
 #pragma unroll
-        for (int j = 0; j < kGroup; j++) {
-            const int k = min(k0 + j, p.n_splits - 1);  // repeats of the last partial get weight 0 below
-            mv[j] = ml[2 * k];
-            lv[j] = ml[2 * k + 1];
-            ov[j] = po[(size_t)k * D];
+            for (int j = 0; j < kGroup; j++) {
+                const int k = k0 + STEP * j;
+                mv[j] = neg_inf();
+                lv[j] = 0.0f;
+                ov[j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                if (k < n) {
+                    mv[j] = ml[64 * k];
+                    lv[j] = ml[64 * k + 32];
+                    ov[j] = *(const f32x4_t*)(po + (size_t)k * (32 * D));
+                }
+            }
+            float m_new = m_all;
+#pragma unroll
+            for (int j = 0; j < kGroup; j++) {
+                m_new = fmaxf(m_new, mv[j]);
+                nan_m |= mv[j] != mv[j];
+            }
+            const float m_use = m_new == neg_inf() ? 0.0f : m_new;
+            const float rescale = m_all == neg_inf() ? 0.0f : __builtin_amdgcn_exp2f(m_all - m_use);
+            l_all *= rescale;
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[e] *= rescale;
+#pragma unroll
+            for (int j = 0; j < kGroup; j++) {
+                // an empty partial (m = -inf) is the identity
+                const float w = mv[j] == neg_inf() ? 0.0f : __builtin_amdgcn_exp2f(mv[j] - m_use);
+                l_all += lv[j] * w;
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[e] += ov[j][e] * w;
+            }
+            m_all = m_new;
         }
+    }
+    if constexpr (PARTS) {
+        if (wave > 0) {
+            fold[wave - 1][0][lane] = nan_m ? __builtin_nanf("") : m_all;
+            fold[wave - 1][1][lane] = l_all;
+#pragma unroll
+            for (int e = 0; e < 4; e++) fold[wave - 1][2 + e][lane] = acc[e];
+        }
+        __syncthreads();
+        if (wave > 0) return;
         float m_new = m_all;
 #pragma unroll
-        for (int j = 0; j < kGroup; j++) {
-            m_new = fmaxf(m_new, mv[j]);
-            nan_m |= (mv[j] != mv[j]);
+        for (int j = 0; j < 3; j++) {
+            m_new = fmaxf(m_new, fold[j][0][lane]);
+            nan_m |= fold[j][0][lane] != fold[j][0][lane];
         }
-        const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
-        const float rescale = (m_all == neg_inf()) ? 0.0f : __builtin_amdgcn_exp2f(m_all - m_use);
-        acc *= rescale;
+        const float m_use = m_new == neg_inf() ? 0.0f : m_new;
+        const float rescale = m_all == neg_inf() ? 0.0f : __builtin_amdgcn_exp2f(m_all - m_use);
         l_all *= rescale;
 #pragma unroll
-        for (int j = 0; j < kGroup; j++) {
-            // an empty partial (m = -inf) is the identity
-            const float w = (k0 + j < p.n_splits && mv[j] != neg_inf()) ? __builtin_amdgcn_exp2f(mv[j] - m_use) : 0.0f;
-            acc += ov[j] * w;
-            l_all += lv[j] * w;
+        for (int e = 0; e < 4; e++) acc[e] *= rescale;
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const float mj = fold[j][0][lane], w = mj == neg_inf() ? 0.0f : __builtin_amdgcn_exp2f(mj - m_use);
+            l_all += fold[j][1][lane] * w;
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[e] += fold[j][2 + e][lane] * w;
         }
         m_all = m_new;
     }
-    float x = acc / l_all;
-    if (m_all == neg_inf() && !nan_m) x = 0.0f;
-    const size_t s_pos = r / (size_t)G;
-    const int g = (int)(r - s_pos * (size_t)G);
-    p.out[(size_t)b * p.lo.batch_stride + (size_t)(kvh * G + g) * p.lo.head_stride + s_pos * (size_t)p.lo.row_pitch + d] =
-        f32_to_bf16_bits(x);
+    if (!row_in) return;
+    const uint32_t s_pos = r / (uint32_t)G, g = r - s_pos * (uint32_t)G;
+    uint16_t* const dst = p.out + (size_t)b * p.lo.batch_stride + (size_t)(kvh * G + g) * p.lo.head_stride +
+                          (size_t)s_pos * p.lo.row_pitch + 8 * piece + 4 * (lane >> 5);
+    uint2 x = make_uint2(0u, 0u);
+    if (m_all != neg_inf() || nan_m) {
+        x.x = (uint32_t)f32_to_bf16_bits(acc[0] / l_all) | (uint32_t)f32_to_bf16_bits(acc[1] / l_all) << 16;
+        x.y = (uint32_t)f32_to_bf16_bits(acc[2] / l_all) | (uint32_t)f32_to_bf16_bits(acc[3] / l_all) << 16;
+    }
+    *(uint2*)dst = x;
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1596,8 +1642,9 @@ hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
         hipError_t e = direct ? launch_one<DP, kMaskCausal, false, true, true, false, kDirect>(stream, p, grid)
                               : launch_one<DP, kMaskCausal, false, true, true>(stream, p, grid);
         if (e != hipSuccess) return e;
-        const size_t total = (size_t)p.batch * p.kv_heads * (size_t)p.seq_q * p.pack * (size_t)p.dim;
-        hipLaunchKernelGGL(flash_split_merge_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, p);
+        const size_t items = (size_t)p.batch * p.kv_heads * (((size_t)p.seq_q * p.pack + 31) / 32) * (size_t)(p.dim / 8);
+        if (p.n_splits > 8) hipLaunchKernelGGL(flash_split_merge_kernel<true>, dim3((unsigned)items), dim3(256), 0, stream, p);
+        else hipLaunchKernelGGL(flash_split_merge_kernel<false>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, stream, p);
         return hipGetLastError();
     }
     if (p.pack > 1 || p.decode_rows) return direct ? launch_one<DP, kMaskCausal, false, true, false, false, kDirect>(stream, p, grid)
@@ -1619,6 +1666,7 @@ hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
 
 bool flash_tile_bf16_supported(int dim) { return dim > 0 && dim <= 256 && dim % 8 == 0; }
 int flash_tile_bf16_key_tile(int dim) { return dim <= 128 ? 64 : 32; }
+int flash_tile_bf16_workgroups(int dim) { return dim <= 64 ? 3 : (dim <= 128 ? 2 : 1); }
 // The kernel addresses the keys of one (batch, kv head) with 32-bit byte offsets (tile offset + lane offset, the
 // requests that run a few tiles past the last one included).
 bool flash_tile_bf16_addressable(long long seq_kv, long long row_pitch) {

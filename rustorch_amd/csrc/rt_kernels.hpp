@@ -127,9 +127,9 @@ struct FlashTileParams {
     // with key i + (keys - valid queries), as sliding_window_mask builds it (crates/rustorch-nn/src/masks.rs:41-60).
     int window;
     // Split over the keys (packed rows only; zero-initialise to leave it off): n_splits > 1 cuts every (sequence, kv
-    // head)'s walk into that many spans of whole tiles; each leaves a partial per packed row in part_o
-    // ([batch, kv_heads, seq_q * pack, n_splits, dim] f32) and part_ml (the same index, (m, l) pairs), and a second
-    // kernel folds them into `out`.
+    // head)'s walk into that many spans of whole tiles; each leaves a partial per block of 32 packed rows in part_o
+    // ([batch, kv_heads, blocks, n_splits, dim / 8, 2, 32, 4] f32: columns 8 i + 4 j + e of row k at [i, j, k, e]) and
+    // part_ml (the same block, [2, 32]: m, l), and a second kernel folds them into `out`.
     int n_splits;
     float* part_o;
     float* part_ml;
@@ -151,6 +151,7 @@ static_assert(offsetof(FlashTileParams, q) == 64 && offsetof(FlashTileParams, q_
 bool flash_tile_bf16_supported(int dim);
 // keys per LDS tile of the tile kernel at head dim `dim` (the unit the split over the keys is cut in)
 int flash_tile_bf16_key_tile(int dim);
+int flash_tile_bf16_workgroups(int dim);  // that share a CU
 hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& p);
 bool flash_tile_bf16_addressable(long long seq_kv, long long row_pitch);  // K/V slabs below 4 GiB (32-bit offsets)
 // the same walk with 64 query rows per wave: head dim 64, masks none / causal, rows of one head
