@@ -48,6 +48,8 @@ struct FlashF32Params {
 };
 // dim <= 256 (the tiled four-wave kernel up to 128).  Returns hipErrorInvalidValue for an unsupported dim.
 hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p);
+// The form on the bf16 matrix cores: dim <= 128 and a multiple of 4, 16-byte aligned rows, mask none or causal, no bias.
+hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p);
 
 // Backward of unmasked f32 attention; every tensor is [batch, heads, seq, dim] row-major and contiguous.
 struct FlashBwdF32Params {

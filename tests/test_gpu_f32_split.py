@@ -1,0 +1,102 @@
+"""f32 attention on the bf16 matrix cores, operands as three bf16 terms: sizes whose launches take that kernel (many rows),
+at the edges of its 128-row workgroups and 32-key tiles, and values the split does not carry.
+
+The bound against 64 bits is 1e-6 of the result's 2-norm: an f32 product of these sizes rounds each of up to 384 / 32 tile sums
+and each weight once, about 2^-24 sqrt(20) = 2.7e-7; the f32 kernel it stands in for shows up to 4e-7 here."""
+import numpy as np
+import pytest
+
+import rustorch_amd as ra
+from _gpu import dev
+from _util import seeded_normal
+
+pytestmark = pytest.mark.gpu
+
+
+def run(q, k, v, causal):
+    b, h, n, d = q.shape
+    out = ra.HipStorage(q.size * 4)
+    out.upload(np.full(q.size, 7.0, dtype=np.float32))
+    mask = ra.Mask.causal() if causal else ra.Mask.none()
+    ra.flash_forward_f32_dev(ra.AttentionShape.new(b, h, n, d), dev(q.ravel()), dev(k.ravel()), dev(v.ravel()), out, mask)
+    ra.synchronize()
+    return out.download(np.float32).reshape(q.shape)
+
+
+def attention64(q, k, v, causal):
+    q, k, v = (x.astype(np.float64) for x in (q, k, v))
+    with np.errstate(all="ignore"):
+        s = q @ np.swapaxes(k, -1, -2) / np.sqrt(q.shape[-1])
+        if causal:
+            n = q.shape[2]
+            s = np.where(np.tril(np.ones((n, n), dtype=bool)), s, -np.inf)
+        p = np.exp(s - s.max(axis=-1, keepdims=True))
+        return (p / p.sum(axis=-1, keepdims=True)) @ v
+
+
+def inputs(b, h, n, d):
+    return [seeded_normal((b, h, n, d), i).reshape(b, h, n, d) for i in (1, 2, 3)]
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("b,h,n,d", [
+    (8, 16, 256, 64),   # whole tiles
+    (8, 16, 225, 60),   # 31 keys of the last tile missing, head dim padded
+    (13, 20, 161, 36),  # one row in a workgroup's second wave, head pairs not a multiple of eight
+    (8, 32, 384, 32),   # head dim 32: half the threads split
+    (16, 16, 130, 64),  # two rows in the last workgroup
+])
+def test_against_64_bits(b, h, n, d, causal):
+    q, k, v = inputs(b, h, n, d)
+    got = run(q, k, v, causal)
+    want = attention64(q, k, v, causal)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+    assert np.abs(got - want).max() <= 5e-6
+
+
+@pytest.mark.parametrize("what", ["key inf", "value inf", "query nan", "value nan", "large"])
+def test_values_the_split_does_not_carry(what):
+    """Rows they reach are what f32 arithmetic makes of them; the rest are as they were."""
+    b, h, n, d = 8, 16, 256, 64
+    q, k, v = inputs(b, h, n, d)
+    want = attention64(q, k, v, True)
+    at = (3, 5)
+    if what == "key inf":
+        q[at][:, 9] = -np.abs(q[at][:, 9]) - 0.1  # every query's score of key 40 is -inf: its weight is zero
+        k[at][40, 9] = np.inf
+    elif what == "value inf":
+        v[at][200, 1] = np.inf
+    elif what == "query nan":
+        q[at][17, 3] = np.nan
+    elif what == "value nan":
+        v[at][255, 63] = np.nan
+    else:
+        q[at][100] = 1e25
+        k[at][100] = 1e25  # row 100 sees its own key only; the products pass the f32 range
+        k[at][100, 1::2] = -1e10
+    got = run(q, k, v, True)
+    other = np.ones((b, h), dtype=bool)
+    other[at] = False
+    assert np.abs(got[other] - want[other]).max() <= 5e-6
+    with np.errstate(all="ignore"):
+        slab = got[at]
+        if what == "key inf":
+            ref = attention64(q[3:4, 5:6], k[3:4, 5:6], v[3:4, 5:6], True)[0, 0]
+            assert np.abs(slab - ref).max() <= 5e-6
+        elif what == "value inf":
+            assert np.isposinf(slab[200:, 1]).all() and np.isfinite(slab[:, 2:]).all()
+        elif what == "query nan":
+            assert np.isnan(slab[17]).all() and np.isfinite(np.delete(slab, 17, axis=0)).all()
+        elif what == "value nan":
+            assert np.isnan(slab[255, 63]) and np.isfinite(slab[:255, :63]).all()
+        else:
+            assert np.isfinite(slab[:100]).all() and np.abs(slab[:100] - want[at][:100]).max() <= 5e-6
+
+
+def test_small_values():
+    """V rows of 2^-120: the last of three bf16 terms would be lost."""
+    q, k, v = inputs(8, 16, 256, 64)
+    v[2, 7] *= np.float32(2.0 ** -120)
+    got, want = run(q, k, v, False), attention64(q, k, v, False)
+    assert np.linalg.norm(got[2, 7].astype(np.float64) - want[2, 7]) <= 1e-6 * np.linalg.norm(want[2, 7])
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
