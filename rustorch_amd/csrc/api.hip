@@ -918,6 +918,7 @@ int flash_bwd_device(hipStream_t stream, const rt_attention_shape* s, const floa
     p.seq = (int)s->seq;
     p.dim = (int)s->dim;
     p.scale = 1.0f / sqrtf((float)s->dim);
+    p.n_cus = g_num_cus;
     if (saved_out) {
         HIP_TRY(rt::launch_flash_bwd_f32_saved(stream, p, saved_out, saved_lse, workspace), "flash_bwd_f32 launch");
     } else if (s->dim > 256) {
@@ -930,7 +931,7 @@ int flash_bwd_device(hipStream_t stream, const rt_attention_shape* s, const floa
         if (rc) return rc;
         HIP_TRY(rt::launch_flash_bwd_f32_saved(stream, p, o, lse_ws, lse_ws + rows), "flash_bwd_f32 launch");
     } else {
-        HIP_TRY(rt::launch_flash_bwd_f32(stream, p, workspace, g_num_cus), "flash_bwd_f32 launch");
+        HIP_TRY(rt::launch_flash_bwd_f32(stream, p, workspace), "flash_bwd_f32 launch");
     }
     return RT_OK;
 }

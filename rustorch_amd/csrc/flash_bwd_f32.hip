@@ -528,7 +528,7 @@ size_t flash_bwd_f32_workspace_floats(int batch, int heads, int seq, int dim) {
     return (size_t)batch * heads * seq * ((size_t)dim + 2);
 }
 
-hipError_t launch_flash_bwd_f32(hipStream_t stream, const FlashBwdF32Params& p_in, float* workspace, int n_cus) {
+hipError_t launch_flash_bwd_f32(hipStream_t stream, const FlashBwdF32Params& p_in, float* workspace) {
     if (p_in.batch == 0 || p_in.heads == 0 || p_in.seq == 0 || p_in.dim == 0) return hipSuccess;
     if (p_in.dim > 256) return hipErrorInvalidValue;  // (the tiled forward stops there; the caller brings O and the statistic)
     const size_t rows = (size_t)p_in.batch * p_in.heads * p_in.seq;
@@ -551,7 +551,7 @@ hipError_t launch_flash_bwd_f32(hipStream_t stream, const FlashBwdF32Params& p_i
     f.mask = kMaskNone;
     f.ref_bc = 64;
     f.scale = p_in.scale;
-    f.n_cus = n_cus;
+    f.n_cus = p_in.n_cus;
     f.lq = f.lkv = f.lo = layout_bhnd(p_in.heads, p_in.seq, p_in.dim);
     hipError_t e = launch_flash_f32(stream, f);
     if (e != hipSuccess) return e;
@@ -576,6 +576,16 @@ hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Param
     auto aligned = [](const void* ptr) { return (uintptr_t)ptr % 16 == 0; };
     p.vec = (p.dim % 4 == 0) && aligned(p.q) && aligned(p.k) && aligned(p.v) && aligned(p.d_out) && aligned(p.dq) &&
             aligned(p.dk) && aligned(p.dv);
+    if (p.vec && p.dim <= 64 && aligned(p.o)) {  // many rows: the bf16 matrix cores, by the rule of the forward
+        FlashF32Params f{};
+        f.batch = p.batch;
+        f.heads = p.heads;
+        f.seq = p.seq;
+        f.dim = p.dim;
+        f.mask = kMaskNone;
+        f.n_cus = p.n_cus;
+        if (flash_f32_split_pays(f)) return launch_flash_bwd_f32_split(stream, p);
+    }
     dim3 grid((p.seq + kRows - 1) / kRows, p.heads, p.batch), block(256);
     const int dt = (p.dim + 31) / 32;
     switch (dt) {

@@ -488,13 +488,18 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
     }
 }
 
+}  // namespace
+
 // Which of the two kernels has less to do on its busiest SIMD, in tile steps of this file's kernel.  This one spreads
 // 32-row workgroups whose waves share the keys, so it is near the mean of the chip; the split kernel owns 128 rows a
 // workgroup and walks all their keys, at 0.58 of the time per step at head dim 64 (1.6 against 2.83 us per tile of 32 x 32
-// and SIMD) and 0.68 at 32 (1.08 against 1.6); half a step more of fixed cost here.  Both sides of the line, head dim 64,
-// us here / there: one sequence of 8 heads, 2048 keys 99 / 100, causal 55 / 99; 4096 keys 331 / 200, causal 175 / 193;
-// 2 x 12 heads, 999 keys 76 / 55, causal 50 / 53; 8 x 16 heads, 256 keys 32 / 22, causal 31 / 22.
-bool f32_split_pays(const FlashF32Params& p) {
+// and SIMD) and 0.68 at 32 (1.08 against 1.6); half a step more of fixed cost here.  Without a mask the gradients follow
+// the same rule, so that they form the scores in the order in which the row statistic was formed: their kernels take 0.73
+// and 0.79 of a step, and the line lies where forward and gradients together break even (0.69 and 0.76).  Both sides of it
+// at head dim 64, us here / there: one sequence of 8 heads, 2048 keys 99 / 99 (gradients 250 / 336), causal 55 / 99; 4096
+// keys 331 / 197, causal 175 / 193; 2 x 12 heads, 999 keys 76 / 55 (gradients 200 / 178), causal 50 / 53; 8 x 16 heads,
+// 256 keys 32 / 22 (gradients 89 / 66), causal 31 / 22.
+bool flash_f32_split_pays(const FlashF32Params& p) {
     const double n_cus = p.n_cus > 0 ? p.n_cus : 256;
     const long long keys = p.seq_kv ? p.seq_kv : p.seq;
     const double tiles = (double)((keys + 31) / 32), blocks = (p.seq + 127) / 128, n_bh = (double)p.heads * p.batch;
@@ -503,10 +508,9 @@ bool f32_split_pays(const FlashF32Params& p) {
     const double per_cu = n_bh * blocks / n_cus;
     double there = __builtin_ceil(per_cu) * tiles;
     if (causal) there = __builtin_fmax(tiles, 1.1 * per_cu * (tiles + 4) / 2);
-    return there * (p.dim > 32 ? 0.58 : 0.68) < here + 0.5;
+    const double step = p.dim > 32 ? (causal ? 0.58 : 0.69) : (causal ? 0.68 : 0.76);
+    return there * step < here + 0.5;
 }
-
-}  // namespace
 
 hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p) {
     if (p.batch == 0 || p.heads == 0 || p.seq == 0) return hipSuccess;
@@ -524,7 +528,7 @@ hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p) {
         pz.zigzag = (p.mask == kMaskCausal) && ((long long)grid.x * grid.y * grid.z <= resident) ? 1 : 0;
         const bool exact = (p.dim % 32 == 0), pad = (p.mask == kMaskPadding);
         if (p.bias && p.mask != kMaskNone) return hipErrorInvalidValue;  // a bias comes without a mask kind
-        if (!p.bias && !pad && dt <= 2 && f32_split_pays(p)) return launch_flash_f32_split(stream, p);
+        if (!p.bias && !pad && dt <= 2 && flash_f32_split_pays(p)) return launch_flash_f32_split(stream, p);
         const int mode = pad ? 2 : (p.mask == kMaskCausal ? 1 : (p.bias ? 3 : 0));
         auto launch = [&](auto dt_c, auto exact_c) {
             constexpr int kDT = decltype(dt_c)::value;

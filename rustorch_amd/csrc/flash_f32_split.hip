@@ -160,15 +160,19 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
             }
         }
     };
-    // Splitting: pair x of this thread's 8 NI (K and V of item x / 8, four pairs each), then the writes.
+    // Splitting: 24 NI steps, three for each pair of this thread's 8 NI (K and V of an item, four pairs each), then the writes.
     struct Parts {
         u32x4_t w[2 * NI][3];
     };
-    auto split_pair = [&](Parts& o, int x) {
-        const int n = x / 8, e = x % 4;
+    SplitPair pair;
+    auto split_step = [&](Parts& o, int y) {  // term y % 3 of pair y / 3
+        const int x = y / 3, u = y % 3, n = x / 8, e = x % 4;
         const bool is_v = (x % 8) >= 4;
         const float x0 = is_v ? vreg[n][2 * e] : kreg[n][e >> 1][2 * (e & 1)];
         const float x1 = is_v ? vreg[n][2 * e + 1] : kreg[n][e >> 1][2 * (e & 1) + 1];
+        if (u == 0) pair.r = split_f32x2_t{x0, x1};
+        o.w[2 * n + (is_v ? 1 : 0)][u][e] = pair.step(u);
+        if (u < 2) return;
         chk = __builtin_fmaf(x0, x0, chk);
         chk = __builtin_fmaf(x1, x1, chk);
         if (is_v) {  // scores of small keys are small whatever is lost of them; small values are the result's size
@@ -176,10 +180,6 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
             v_max = __builtin_fmaxf(__builtin_fmaxf(v_max, __builtin_fabsf(x0)), __builtin_fabsf(x1));
             if (e == 3) chk = split_too_small(v_max) ? kSplitMost : chk;
         }
-        uint32_t w[3];
-        split2(x0, x1, w);
-#pragma unroll
-        for (int u = 0; u < 3; u++) o.w[2 * n + (is_v ? 1 : 0)][u][e] = w[u];
     };
     auto write_tile = [&](const Parts& o, __bf16* kbuf, __bf16* vbuf) {
 #pragma unroll
@@ -198,7 +198,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
     auto store_tile = [&](__bf16* kbuf, __bf16* vbuf) {
         Parts o;
 #pragma unroll
-        for (int x = 0; x < 8 * NI; x++) split_pair(o, x);
+        for (int x = 0; x < 24 * NI; x++) split_step(o, x);
         write_tile(o, kbuf, vbuf);
     };
 
@@ -297,21 +297,29 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
         rescale();
         u32x4_t pw[2][3];
         float part[2] = {0.0f, 0.0f};
+        SplitPair sp;
+        auto weight_step = [&](int x) {  // 16 steps, two a pair
+            const int g = x / 2;
+            if (x % 2 == 0) {
 #pragma unroll
-        for (int g = 0; g < 8; g++) {
-            __builtin_amdgcn_sched_barrier(0);
+                for (int u = 0; u < 2; u++) {
+                    const float e = __builtin_amdgcn_exp2f((s[2 * g + u] - m_use) * kLog2e);
+                    part[u] += e;
+                    sp.r[u] = e;
+                }
+            } else {
 #pragma unroll
-            for (int n = 2 * KS + g * KS / 2; n < 2 * KS + (g + 1) * KS / 2; n++) score_step(kn, s_next, n);
-            const float e0 = __builtin_amdgcn_exp2f((s[2 * g] - m_use) * kLog2e);
-            const float e1 = __builtin_amdgcn_exp2f((s[2 * g + 1] - m_use) * kLog2e);
-            part[0] += e0;
-            part[1] += e1;
-            uint32_t w[3];
-            split2(e0, e1, w);
+                for (int u = 0; u < 3; u++) pw[g >> 2][u][g & 3] = sp.step(u);
+            }
+        };
+        RT_ORDER();
 #pragma unroll
-            for (int u = 0; u < 3; u++) pw[g >> 2][u][g & 3] = w[u];
+        for (int n = 0; n < 4 * KS; n++) {
+            score_step(kn, s_next, 2 * KS + n);
+#pragma unroll
+            for (int x = n * 16 / (4 * KS); x < (n + 1) * 16 / (4 * KS); x++) weight_step(x);
+            RT_ORDER();
         }
-        __builtin_amdgcn_sched_barrier(0);
         add_sum(part[0] + part[1]);
         // A tile's product in registers of its own, smallest terms first, then one addition to the sum: in the sum
         // itself each of the twelve instructions would round at its size, and the error against 64 bits grew above
@@ -329,13 +337,14 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
 #pragma unroll
             for (int term = 0; term < 6; term++) {
 #pragma unroll
-                for (int j = 0; j < 2; j++)
+                for (int j = 0; j < 2; j++) {
                     o = mfma_h(v[kPlaneA[term]][j], __builtin_bit_cast(bf16x8_t, pw[j][kPlaneC[term]]), o);
-                // this term's share of the pairs of the tile that is split: 8 NI pairs over 6 DT places
+                    // its share of the next tile's split: 24 NI steps behind 12 DT instructions
+                    const int n = (6 * t + term) * 2 + j;
 #pragma unroll
-                for (int x = (6 * t + term) * 8 * NI / (6 * DT); x < (6 * t + term + 1) * 8 * NI / (6 * DT); x++)
-                    split_pair(kv_parts, x);
-                __builtin_amdgcn_sched_barrier(0);
+                    for (int x = n * 24 * NI / (12 * DT); x < (n + 1) * 24 * NI / (12 * DT); x++) split_step(kv_parts, x);
+                    RT_ORDER();
+                }
             }
 #pragma unroll
             for (int i = 0; i < 16; i++) acc_o[t][i] += o[i];
@@ -359,7 +368,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
 #pragma unroll
             for (int i = 0; i < 16; i++) s[i] = 0.0f;
             for (int ks = 0; ks < DPAD / 2; ks++) {
-                const int d = 2 * ks + hh;
+                const int d = 8 * (ks >> 2) + 4 * hh + (ks & 3);  // the f32 kernel's order
                 const float a = (kv0 + col < N && d < D) ? Kg[(size_t)(kv0 + col) * kv_pitch + d] : 0.0f;
                 const float bq = (q_row < Nq && d < D) ? Qg[(size_t)q_row * q_pitch + d] : 0.0f;
                 s = __builtin_amdgcn_mfma_f32_32x32x2f32(a, bq, s, 0, 0, 0);

@@ -50,6 +50,7 @@ struct FlashF32Params {
 hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p);
 // The form on the bf16 matrix cores: dim <= 128 and a multiple of 4, 16-byte aligned rows, mask none or causal, no bias.
 hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p);
+bool flash_f32_split_pays(const FlashF32Params& p);
 
 // Backward of unmasked f32 attention; every tensor is [batch, heads, seq, dim] row-major and contiguous.
 struct FlashBwdF32Params {
@@ -62,6 +63,7 @@ struct FlashBwdF32Params {
     float* dv;
     int batch, heads, seq, dim;
     float scale;
+    int n_cus;  // CUs of the device (0: unknown)
     // filled by the launcher
     const float* o;
     const float* lse;
@@ -71,11 +73,13 @@ struct FlashBwdF32Params {
 // Floats of scratch launch_flash_bwd_f32 needs (O, the row statistic and delta).
 size_t flash_bwd_f32_workspace_floats(int batch, int heads, int seq, int dim);
 // dim <= 128.  Runs the forward kernel, then dQ (which also leaves delta) and dK/dV on `stream`.
-hipError_t launch_flash_bwd_f32(hipStream_t stream, const FlashBwdF32Params& p, float* workspace, int n_cus);
+hipError_t launch_flash_bwd_f32(hipStream_t stream, const FlashBwdF32Params& p, float* workspace);
 // The same from a saved forward: `o` [B,H,N,D] and `lse` [B,H,N] as launch_flash_f32 leaves them (FlashF32Params::lse);
 // `delta` is B*H*N floats of scratch.  Runs dQ (which also leaves delta), then dK/dV.
 hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Params& p, const float* o, const float* lse,
                                       float* delta);
+// Its form on the bf16 matrix cores: p.o, p.lse and p.delta set, dim <= 64 and a multiple of 4, all tensors 16-byte aligned.
+hipError_t launch_flash_bwd_f32_split(hipStream_t stream, const FlashBwdF32Params& p);
 
 struct FlashBf16Params {
     const uint16_t* q;

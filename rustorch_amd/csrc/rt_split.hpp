@@ -22,16 +22,24 @@ struct Split8 {
     bf16x8_t p[3];  // h, m, l
 };
 
-__device__ __forceinline__ void split2(float x0, float x1, uint32_t (&w)[3]) {
-    split_f32x2_t r = {x0, x1};
-#pragma unroll
-    for (int n = 0; n < 3; n++) {
-        w[n] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, split_bf16x2_t));
+// Two values on their way through the split: step n = 0, 1, 2 gives the packed h, m and l.  Five vector instructions a
+// step fit between two matrix instructions of one wave.
+struct SplitPair {
+    split_f32x2_t r;
+    __device__ __forceinline__ uint32_t step(int n) {
+        const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, split_bf16x2_t));
         if (n < 2) {
-            r[0] -= bf16_lo(w[n]);
-            r[1] -= bf16_hi(w[n]);
+            r[0] -= bf16_lo(w);
+            r[1] -= bf16_hi(w);
         }
+        return w;
     }
+};
+
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t (&w)[3]) {
+    SplitPair s{{x0, x1}};
+#pragma unroll
+    for (int n = 0; n < 3; n++) w[n] = s.step(n);
 }
 
 __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
@@ -48,6 +56,9 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
     for (int n = 0; n < 3; n++) s.p[n] = __builtin_bit_cast(bf16x8_t, w[n]);
     return s;
 }
+
+// A fixed place in the instruction order: what is written before it stays before it.
+#define RT_ORDER() __builtin_amdgcn_sched_barrier(0)
 
 __device__ __forceinline__ f32x16_t mfma_h(bf16x8_t a, bf16x8_t b, f32x16_t acc) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);

@@ -1,4 +1,4 @@
-"""f32 attention on the bf16 matrix cores, operands as three bf16 terms: sizes whose launches take that kernel (many rows),
+"""f32 attention and its gradients on the bf16 matrix cores, operands as three bf16 terms: sizes whose launches take that kernel (many rows),
 at the edges of its 128-row workgroups and 32-key tiles, and values the split does not carry.
 
 The bound against 64 bits is 1e-6 of the result's 2-norm: an f32 product of these sizes rounds each of up to 384 / 32 tile sums
@@ -100,3 +100,73 @@ def test_small_values():
     got, want = run(q, k, v, False), attention64(q, k, v, False)
     assert np.linalg.norm(got[2, 7].astype(np.float64) - want[2, 7]) <= 1e-6 * np.linalg.norm(want[2, 7])
     assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
+def run_backward(q, k, v, d_out):
+    b, h, n, d = q.shape
+    shape = ra.AttentionShape.new(b, h, n, d)
+    dq_, dk_, dv_, dd = (dev(x.ravel()) for x in (q, k, v, d_out))
+    out, lse, ws = ra.HipStorage(q.size * 4), ra.HipStorage(b * h * n * 4), ra.HipStorage(b * h * n * 4)
+    grads = [ra.HipStorage(q.size * 4) for _ in range(3)]
+    for g in grads:
+        g.upload(np.full(q.size, 7.0, dtype=np.float32))
+    ra.flash_forward_stats_f32_dev(shape, dq_, dk_, dv_, out, lse)
+    ra.flash_backward_saved_f32_dev(shape, dq_, dk_, dv_, out, lse, dd, *grads, ws, b * h * n * 4)
+    ra.synchronize()
+    return [g.download(np.float32).reshape(q.shape) for g in grads]
+
+
+def gradients64(q, k, v, d_out):
+    q, k, v, d_out = (x.astype(np.float64) for x in (q, k, v, d_out))
+    scale = 1 / np.sqrt(q.shape[-1])
+    with np.errstate(all="ignore"):
+        s = q @ np.swapaxes(k, -1, -2) * scale
+        p = np.exp(s - s.max(axis=-1, keepdims=True))
+        p /= p.sum(axis=-1, keepdims=True)
+        dp = d_out @ np.swapaxes(v, -1, -2)
+        ds = p * (dp - (p * dp).sum(axis=-1, keepdims=True)) * scale
+        return ds @ k, np.swapaxes(ds, -1, -2) @ q, np.swapaxes(p, -1, -2) @ d_out
+
+
+@pytest.mark.parametrize("b,h,n,d", [
+    (8, 16, 256, 64),
+    (8, 16, 225, 60),
+    (8, 32, 353, 32),   # one row in the last tile, head dim 32
+    (8, 28, 481, 36),   # head pairs not a multiple of the XCDs' share, padded head dim
+    (16, 16, 130, 64),
+])
+def test_gradients_against_64_bits(b, h, n, d):
+    """The bound is the forward's times two: dS carries the errors of P and of dP - delta."""
+    x = inputs(b, h, n, d) + [seeded_normal((b, h, n, d), 4).reshape(b, h, n, d)]
+    for name, got, want in zip(("dq", "dk", "dv"), run_backward(*x), gradients64(*x)):
+        assert np.linalg.norm(got - want) <= 2e-6 * np.linalg.norm(want), name
+
+
+@pytest.mark.parametrize("what", ["key inf", "d_out nan", "query nan", "small"])
+def test_gradients_of_values_the_split_does_not_carry(what):
+    """Only the head that holds them changes: by the rules of f32 arithmetic, or, for small ones, not in precision."""
+    b, h, n, d = 8, 16, 256, 64
+    x = inputs(b, h, n, d) + [seeded_normal((b, h, n, d), 4).reshape(b, h, n, d)]
+    q, k, v, d_out = x
+    at = (3, 5)
+    if what == "key inf":
+        q[at][:, 9] = -np.abs(q[at][:, 9]) - 0.1
+        k[at][40, 9] = np.inf
+    elif what == "d_out nan":
+        d_out[at][17, 3] = np.nan
+    elif what == "query nan":
+        q[at][17, 3] = np.nan
+    else:
+        d_out[at] *= np.float32(2.0 ** -115)
+    got, want = run_backward(*x), gradients64(*x)
+    other = np.ones((b, h), dtype=bool)
+    other[at] = False
+    for name, g, w in zip(("dq", "dk", "dv"), got, want):
+        assert np.linalg.norm(g[other] - w[other]) <= 2e-6 * np.linalg.norm(w[other]), name
+        gs, ws = g[at].astype(np.float64), w[at]
+        if what == "small":
+            assert np.linalg.norm(gs - ws) <= 2e-6 * np.linalg.norm(ws), name
+        else:
+            fin = np.isfinite(ws)
+            assert np.array_equal(np.isnan(gs), np.isnan(ws)), name
+            assert not fin.any() or np.linalg.norm((gs - ws)[fin]) <= 2e-6 * np.linalg.norm(ws[fin]), name
