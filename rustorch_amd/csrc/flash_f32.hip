@@ -498,7 +498,8 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
 // and 0.79 of a step, and the line lies where forward and gradients together break even (0.69 and 0.76).  Both sides of it
 // at head dim 64, us here / there: one sequence of 8 heads, 2048 keys 99 / 99 (gradients 250 / 336), causal 55 / 99; 4096
 // keys 331 / 197, causal 175 / 193; 2 x 12 heads, 999 keys 76 / 55 (gradients 200 / 178), causal 50 / 53; 8 x 16 heads,
-// 256 keys 32 / 22 (gradients 89 / 66), causal 31 / 22.
+// 256 keys 32 / 22 (gradients 89 / 66), causal 31 / 22.  Head dim 128: 8 heads, 2048 keys 191 / 192, 16 heads, 1500 keys
+// 219 / 146, causal 135 / 144; 4 x 16 heads, 1024 keys 405 / 218, causal 249 / 133.
 bool flash_f32_split_pays(const FlashF32Params& p) {
     const double n_cus = p.n_cus > 0 ? p.n_cus : 256;
     const long long keys = p.seq_kv ? p.seq_kv : p.seq;
@@ -507,7 +508,11 @@ bool flash_f32_split_pays(const FlashF32Params& p) {
     const double here = n_bh * ((p.seq + 31) / 32) * (causal ? (tiles + 1) / 2 : tiles) / (4 * n_cus);
     const double per_cu = n_bh * blocks / n_cus;
     double there = __builtin_ceil(per_cu) * tiles;
-    if (causal) there = __builtin_fmax(tiles, 1.1 * per_cu * (tiles + 4) / 2);
+    if (causal) {
+        if (p.dim <= 64) there = __builtin_fmax(tiles, 1.1 * per_cu * (tiles + 4) / 2);
+        else there = per_cu > 1 ? __builtin_ceil(per_cu / 2) * (tiles + 4) : tiles;  // two blocks a workgroup
+    }
+    if (p.dim > 64) return there * 0.55 < here + 0.5;
     const double step = p.dim > 32 ? (causal ? 0.58 : 0.69) : (causal ? 0.68 : 0.76);
     return there * step < here + 0.5;
 }
@@ -528,7 +533,8 @@ hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p) {
         pz.zigzag = (p.mask == kMaskCausal) && ((long long)grid.x * grid.y * grid.z <= resident) ? 1 : 0;
         const bool exact = (p.dim % 32 == 0), pad = (p.mask == kMaskPadding);
         if (p.bias && p.mask != kMaskNone) return hipErrorInvalidValue;  // a bias comes without a mask kind
-        if (!p.bias && !pad && dt <= 2 && flash_f32_split_pays(p)) return launch_flash_f32_split(stream, p);
+        // (above head dim 64 the gradients have no such form, and a row statistic they read is formed as they form the scores)
+        if (!p.bias && !pad && (dt <= 2 || !p.lse) && flash_f32_split_pays(p)) return launch_flash_f32_split(stream, p);
         const int mode = pad ? 2 : (p.mask == kMaskCausal ? 1 : (p.bias ? 3 : 0));
         auto launch = [&](auto dt_c, auto exact_c) {
             constexpr int kDT = decltype(dt_c)::value;

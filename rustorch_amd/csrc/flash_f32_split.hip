@@ -10,7 +10,7 @@
 // or two (1.56 and 1.58 us a tile); 64 matrix instructions of 64 clocks in the f32 kernel.  B=4 H=16 N=1024 D=64: 181 ->
 // 102 us, causal 120 -> 69; B=2 N=2048 336 -> 189, causal 187 -> 119.  Relative error against 64 bits at those sizes
 // 4.2e-7 -> 1.7e-7 and 5.1e-7 -> 2.2e-7 (four instructions round a score at its size instead of 32, one addition a tile
-// the output instead of 16).
+// the output instead of 16).  Above head dim 64 LDS holds one workgroup a CU: D=128 405 -> 218 us, causal 249 -> 133.
 #include <type_traits>
 
 #include "rt_common.hpp"
@@ -21,10 +21,12 @@ namespace rt {
 
 namespace {
 
+#define RT_INLINE __attribute__((always_inline))  // lambdas over the wave's registers: a call would put them in memory
+
 constexpr int kTile = 32;  // keys per step, query rows per wave
 
 template <int DT, bool kExactD, bool kCausal>
-__global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Params p) {
+__global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kernel(FlashF32Params p) {
     constexpr int DPAD = 32 * DT;
     constexpr int KS = DPAD / 16;          // contraction chunks of the score product
     constexpr int LDK = DPAD + 8;          // bf16 elements: 16-byte reads of 8 rows tile all banks
@@ -40,21 +42,22 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
     const int col = lane & 31, hh = lane >> 5;
     const int Nq = p.seq, N = p.seq_kv ? p.seq_kv : p.seq;
     const int D = kExactD ? DPAD : p.dim;
-    const int nq = (int)gridDim.x, n_bh = (int)(gridDim.y * gridDim.z);
+    // p.zigzag 2 (head dims above 64): a workgroup takes two blocks of a head, a long and a short one, in turn
+    const int nq = (int)gridDim.x, n_bh = (int)(gridDim.y * gridDim.z), n_blk = (Nq + 4 * kTile - 1) / (4 * kTile);
     int h = blockIdx.y, b = blockIdx.z;
-    int qblk = nq - 1 - (int)blockIdx.x;  // longest causal rows first
+    int x = (int)blockIdx.x;
+    bool short_first = false;
     if ((n_bh & 7) == 0) {                // a head's workgroups on one XCD: its K and V come into one L2
         const int lin = (int)blockIdx.x + nq * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z);
         const int xcd = lin & 7, r = lin >> 3, half = (nq * (n_bh >> 3)) >> 1;
         const int bh = (r / nq) * 8 + xcd;
-        qblk = nq - 1 - r % nq;
+        x = r % nq;
         // all resident at once: list positions r and r + half share a CU, a long one and a short one of them
-        if (p.zigzag && r >= half && half % nq == 0) qblk = (r - half) % nq;
+        short_first = p.zigzag == 1 && r >= half && half % nq == 0;
         h = bh % (int)gridDim.y;
         b = bh / (int)gridDim.y;
     }
-    const int q0 = qblk * 4 * kTile, q0w = q0 + wave * kTile;
-    const int q_row = q0w + col;
+    int qblk = short_first ? x : n_blk - 1 - x;  // longest causal rows first
     const int kvh = h / p.group;
     const float* __restrict__ Qg = p.q + (size_t)b * p.lq.batch_stride + (size_t)h * p.lq.head_stride;
     const float* __restrict__ Kg = p.k + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
@@ -62,6 +65,9 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
     float* __restrict__ Og = p.out + (size_t)b * p.lo.batch_stride + (size_t)h * p.lo.head_stride;
     const size_t q_pitch = p.lq.row_pitch, kv_pitch = p.lkv.row_pitch, o_pitch = p.lo.row_pitch;
 
+    for (;;) {
+    const int q0 = qblk * 4 * kTile, q0w = q0 + wave * kTile;
+    const int q_row = q0w + col;
     float chk = 0.0f;  // sum of squares of everything this thread splits
     float v_max = 0.0f;
 
@@ -115,7 +121,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
         const int g = idx / DPAD;
         v_off[n] = 4u * ((uint32_t)(16 * (g >> 1) + 4 * (g & 1)) * (uint32_t)kv_pitch + (uint32_t)(idx % DPAD));
     }
-    auto load_tile = [&](int tile) {
+    auto load_tile = [&](int tile) RT_INLINE {
         if (tile * kTile + kTile <= N) {  // wave-uniform
             const char* kb = (const char*)(Kg + (size_t)tile * kTile * kv_pitch);
             const char* vb = (const char*)(Vg + (size_t)tile * kTile * kv_pitch);
@@ -165,7 +171,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
         u32x4_t w[2 * NI][3];
     };
     SplitPair pair;
-    auto split_step = [&](Parts& o, int y) {  // term y % 3 of pair y / 3
+    auto split_step = [&](Parts& o, int y) RT_INLINE {  // term y % 3 of pair y / 3
         const int x = y / 3, u = y % 3, n = x / 8, e = x % 4;
         const bool is_v = (x % 8) >= 4;
         const float x0 = is_v ? vreg[n][2 * e] : kreg[n][e >> 1][2 * (e & 1)];
@@ -181,7 +187,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
             if (e == 3) chk = split_too_small(v_max) ? kSplitMost : chk;
         }
     };
-    auto write_tile = [&](const Parts& o, __bf16* kbuf, __bf16* vbuf) {
+    auto write_tile = [&](const Parts& o, __bf16* kbuf, __bf16* vbuf) RT_INLINE {
 #pragma unroll
         for (int n = 0; n < NI; n++) {
             const int idx = 256 * n + tid;
@@ -195,7 +201,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
             }
         }
     };
-    auto store_tile = [&](__bf16* kbuf, __bf16* vbuf) {
+    auto store_tile = [&](__bf16* kbuf, __bf16* vbuf) RT_INLINE {
         Parts o;
 #pragma unroll
         for (int x = 0; x < 24 * NI; x++) split_step(o, x);
@@ -204,7 +210,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
 
     // A score tile (register i: key 8 (i/4) + 4 hh + i%4, query `col`): scaled and masked, then turned into weights.
     // weights() returns the factor the sums so far have to be multiplied by.
-    auto scale_mask = [&](f32x16_t& s, int kv0) {
+    auto scale_mask = [&](f32x16_t& s, int kv0) RT_INLINE {
 #pragma unroll
         for (int i = 0; i < 16; i++) s[i] *= p.scale;
         if ((kv0 + kTile > N) || (kCausal && kv0 + kTile - 1 > q0w)) {
@@ -216,7 +222,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
             }
         }
     };
-    auto row_max = [&](const f32x16_t& s) {
+    auto row_max = [&](const f32x16_t& s) RT_INLINE {
         float m_tile = neg_inf();  // NaN never wins, as in the reference's `if x > m`
 #pragma unroll
         for (int i = 0; i < 16; i++) m_tile = __builtin_fmaxf(m_tile, s[i]);
@@ -225,19 +231,19 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
     };
     // the maximum goes to m_run; returns what is subtracted from the scores
     float alpha = 0.0f;
-    auto take_max = [&](float m_tile) {
+    auto take_max = [&](float m_tile) RT_INLINE {
         const float m_new = __builtin_fmaxf(m_tile, m_run);
         const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
         alpha = (m_run == neg_inf()) ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_use) * kLog2e);
         m_run = m_new;
         return m_use;
     };
-    auto add_sum = [&](float tile_l) {
+    auto add_sum = [&](float tile_l) RT_INLINE {
         const float add = tile_l - l_low * alpha, before = l_run * alpha;
         l_run = before + add;
         l_low = (l_run - before) - add;
     };
-    auto rescale = [&]() {
+    auto rescale = [&]() RT_INLINE {
         if (__any(alpha != 1.0f)) {
 #pragma unroll
             for (int t = 0; t < DT; t++)
@@ -249,17 +255,17 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
     // read from LDS one plane ahead of its use.
     constexpr int kPlaneA[6] = {2, 1, 1, 0, 0, 0}, kPlaneC[6] = {0, 1, 0, 2, 1, 0};
     bf16x8_t kf[2][KS];
-    auto read_plane = [&](const __bf16* kbuf, int a) {
+    auto read_plane = [&](const __bf16* kbuf, int a) RT_INLINE {
 #pragma unroll
         for (int j = 0; j < KS; j++) kf[a & 1][j] = *(const bf16x8_t*)(kbuf + a * KPL + col * LDK + 8 * hh + 16 * j);
     };
-    auto score_step = [&](const __bf16* kbuf, f32x16_t& s, int n) {  // n: 0 .. 6 KS - 1, a constant
+    auto score_step = [&](const __bf16* kbuf, f32x16_t& s, int n) RT_INLINE {  // n: 0 .. 6 KS - 1, a constant
         const int term = n / KS, j = n % KS;
         if (n == 0) read_plane(kbuf, 1);
         if (n == KS) read_plane(kbuf, 0);  // plane 2 has been used
         s = mfma_h(kf[kPlaneA[term] & 1][j], qf[j].p[kPlaneC[term]], s);
     };
-    auto zero16 = [](f32x16_t& x) {
+    auto zero16 = [](f32x16_t& x) RT_INLINE {
 #pragma unroll
         for (int i = 0; i < 16; i++) x[i] = 0.0f;
     };
@@ -298,7 +304,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
         u32x4_t pw[2][3];
         float part[2] = {0.0f, 0.0f};
         SplitPair sp;
-        auto weight_step = [&](int x) {  // 16 steps, two a pair
+        auto weight_step = [&](int x) RT_INLINE {  // 16 steps, two a pair
             const int g = x / 2;
             if (x % 2 == 0) {
 #pragma unroll
@@ -399,7 +405,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
     const float l = l_run + other_half(l_run);
     const bool good = (l > 0.0f) && (fabsf(l) != __uint_as_float(0x7f800000u)) && (l == l);
     const float inv_l = 1.0f / l;
-    if (q_row >= Nq) return;
+    if (q_row < Nq) {
     if (p.lse && hh == 0) p.lse[((size_t)b * p.heads + h) * (size_t)Nq + q_row] = m_run + logf(l);
     float* o_row = Og + (size_t)q_row * o_pitch;
 #pragma unroll
@@ -412,6 +418,11 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
             for (int i = 0; i < 4; i++) o[i] = good ? acc_o[t][4 * g + i] * inv_l : quiet_nan();
             if (kExactD || d < D) *(f32x4_t*)(o_row + d) = o;
         }
+    }
+    // (every wave is behind the barrier of the test above: the tiles of the next block may come into LDS)
+    if (DT <= 2 || !kCausal || p.zigzag != 2 || qblk == x || n_blk - 1 - x == x) return;
+    qblk = x;
+    }
 }
 
 }  // namespace
@@ -419,7 +430,16 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_kernel(FlashF32Par
 hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p_in) {
     FlashF32Params p = p_in;
     dim3 grid((p.seq + 4 * kTile - 1) / (4 * kTile), p.heads, p.batch), block(256);
-    p.zigzag = p.mask == kMaskCausal && (long long)grid.x * grid.y * grid.z <= 2ll * p.n_cus;
+    // Causal rows are of unequal length.  Up to head dim 64 two workgroups share a CU: where all are resident at once the
+    // pairs are made by place.  Above, one fills a CU (LDS), and left to the order of the launch the long blocks of a later
+    // head met the long ones before them: two blocks a workgroup (B=4 H=16 N=1024 D=128 203 -> 133 us).
+    const long long n = (long long)grid.x * grid.y * grid.z;
+    p.zigzag = 0;
+    if (p.mask == kMaskCausal && p.dim <= 64 && n <= 2ll * p.n_cus) p.zigzag = 1;
+    if (p.mask == kMaskCausal && p.dim > 64 && n > p.n_cus) {
+        p.zigzag = 2;
+        grid.x = (grid.x + 1) / 2;
+    }
     auto launch = [&](auto dt_c, auto exact_c) {
         constexpr int kDT = decltype(dt_c)::value;
         constexpr bool kEx = decltype(exact_c)::value;
@@ -433,6 +453,8 @@ hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p_in
     switch ((p.dim + 31) / 32) {
         case 1: launch_dt(std::integral_constant<int, 1>{}); break;
         case 2: launch_dt(std::integral_constant<int, 2>{}); break;
+        case 3: launch_dt(std::integral_constant<int, 3>{}); break;
+        case 4: launch_dt(std::integral_constant<int, 4>{}); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

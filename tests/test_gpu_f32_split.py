@@ -45,6 +45,10 @@ def inputs(b, h, n, d):
     (13, 20, 161, 36),  # one row in a workgroup's second wave, head pairs not a multiple of eight
     (8, 32, 384, 32),   # head dim 32: half the threads split
     (16, 16, 130, 64),  # two rows in the last workgroup
+    (8, 16, 256, 128),
+    (8, 32, 353, 96),   # three blocks of rows, two a workgroup where causal
+    (9, 16, 225, 80),
+    (8, 32, 353, 68),
 ])
 def test_against_64_bits(b, h, n, d, causal):
     q, k, v = inputs(b, h, n, d)
