@@ -277,6 +277,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
 
     // The rest of the arguments, requested together: left to itself the compiler loads a field where it is first used
     // and waits for a line at a time.
+    if constexpr (MODE == kMaskPadding) asm volatile("" ::"s"(p.keep), "s"(p.ref_bc));
     asm volatile("" ::"s"(p.q), "s"(p.out), "s"(p.q_lens), "s"(p.kv_lens), "s"(p.seq_q), "s"(p.zero_padded_rows), "s"(p.scale_log2e),
                  "s"(p.lq.batch_stride), "s"(p.lq.head_stride), "s"(p.lq.row_pitch), "s"(p.lo.batch_stride),
                  "s"(p.lo.head_stride), "s"(p.lo.row_pitch));
