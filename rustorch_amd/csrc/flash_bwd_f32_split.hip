@@ -7,9 +7,10 @@
 // the rows of a column in the order the weights sit in the accumulators).  Every output row has one owner: no atomics, the
 // same bits on every launch.
 //
-// What bounds them: matrix and vector instructions together, as in the forward kernel; at head dim 64 a tile is 72 (dQ) and
-// 96 (dK/dV) matrix instructions of 32 clocks and about 440 and 550 vector ones of 4 per wave, LDS holds two tiles of both
-// streams for one workgroup a CU, and a wave takes the register file of its SIMD.  Between two matrix instructions stands a
+// What bounds them: matrix and vector instructions together, as in the forward kernel (counted: 38 % and 43 % of the clocks of
+// either kernel); at head dim 64 a tile is 72 (dQ) and 96 (dK/dV) matrix instructions of 32 clocks and about 580 and 745
+// vector ones of 4 per wave.  LDS holds two tiles of both streams for one workgroup a CU, and a wave takes the register
+// file of its SIMD; the moves that makes necessary are a tenth of the vector instructions.  Between two matrix instructions stands a
 // step of the next tile's split or of the weights (two matrix instructions behind each other hold the wave until the first
 // is done: 382 -> 370 us; without any order 418).  B=4 H=16 N=1024 D=64, dQ and dK/dV: 506 -> 370 us, B=2 N=2048 973 ->
 // 704, head dim 32 273 -> 216; relative error against 64 bits 5.9e-7 -> 4.5e-7, 7.3e-7 -> 5.9e-7, 5.5e-7 -> 4.4e-7.

@@ -6,8 +6,8 @@
 // into registers, the weights where they are formed.
 //
 // What bounds it: matrix and vector instructions together.  A tile of 32 keys is 48 matrix instructions of 32 clocks and
-// about 380 vector instructions of 4 per wave, and the two add up to nine tenths of the time, whether a SIMD holds one wave
-// or two (1.56 and 1.58 us a tile); 64 matrix instructions of 64 clocks in the f32 kernel.  B=4 H=16 N=1024 D=64: 181 ->
+// about 400 vector instructions of 4 per wave, and the two add up to the whole of the time (46 % and 55 % of the clocks),
+// whether a SIMD holds one wave or two (1.56 and 1.58 us a tile); 64 matrix instructions of 64 clocks in the f32 kernel.  B=4 H=16 N=1024 D=64: 181 ->
 // 102 us, causal 120 -> 69; B=2 N=2048 336 -> 189, causal 187 -> 119.  Relative error against 64 bits at those sizes
 // 4.2e-7 -> 1.7e-7 and 5.1e-7 -> 2.2e-7 (four instructions round a score at its size instead of 32, one addition a tile
 // the output instead of 16).  Above head dim 64 LDS holds one workgroup a CU: D=128 405 -> 218 us, causal 249 -> 133.
