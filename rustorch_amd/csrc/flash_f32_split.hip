@@ -66,362 +66,362 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
     const size_t q_pitch = p.lq.row_pitch, kv_pitch = p.lkv.row_pitch, o_pitch = p.lo.row_pitch;
 
     for (;;) {
-    const int q0 = qblk * 4 * kTile, q0w = q0 + wave * kTile;
-    const int q_row = q0w + col;
-    float chk = 0.0f;  // sum of squares of everything this thread splits
-    float v_max = 0.0f;
+        const int q0 = qblk * 4 * kTile, q0w = q0 + wave * kTile;
+        const int q_row = q0w + col;
+        float chk = 0.0f;  // sum of squares of everything this thread splits
+        float v_max = 0.0f;
 
-    // Q as B operand: chunk j, this lane's 8 elements d = 16j + 8hh ..
-    Split8 qf[KS];
+        // Q as B operand: chunk j, this lane's 8 elements d = 16j + 8hh ..
+        Split8 qf[KS];
 #pragma unroll
-    for (int j = 0; j < KS; j++) {
-        float x[8];
+        for (int j = 0; j < KS; j++) {
+            float x[8];
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-            const int d = 16 * j + 8 * hh + 4 * u;
-            if (q_row < Nq && d < D) z = *(const f32x4_t*)(Qg + (size_t)q_row * q_pitch + d);
+            for (int u = 0; u < 2; u++) {
+                f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+                const int d = 16 * j + 8 * hh + 4 * u;
+                if (q_row < Nq && d < D) z = *(const f32x4_t*)(Qg + (size_t)q_row * q_pitch + d);
 #pragma unroll
-            for (int i = 0; i < 4; i++) x[4 * u + i] = z[i];
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i++) chk = __builtin_fmaf(x[i], x[i], chk);
-        qf[j] = split8(x);
-    }
-
-    f32x16_t acc_o[DT];
-#pragma unroll
-    for (int t = 0; t < DT; t++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) acc_o[t][i] = 0.0f;
-    float m_run = neg_inf(), l_run = 0.0f, l_low = 0.0f;  // l_low: what the additions to l_run rounded off
-
-    const int kv_end = kCausal ? min(N, q0 + 4 * kTile) : N;
-    const int n_tiles = (kv_end + kTile - 1) / kTile;
-    const int wave_end = q0w >= Nq ? 0 : (kCausal ? min(N, q0w + kTile) : N);
-    const int n_wave = (wave_end + kTile - 1) / kTile;  // tiles this wave has scores in
-
-    // A tile's way into LDS: 8 elements of a K row per item, and 8 keys of a V column, in the order the weights sit in
-    // the score accumulators (slot 8g + e is key 16 (g/2) + 4 (g%2) + 8 (e/4) + e%4).  Rows behind the last key repeat
-    // it: their weights are exact zeros, and a zero times a finite value adds nothing.
-    f32x4_t kreg[NI][2];
-    float vreg[NI][8];
-#pragma unroll
-    for (int n = 0; n < NI; n++) {  // threads without an item split zeros
-        kreg[n][0] = kreg[n][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int e = 0; e < 8; e++) vreg[n][e] = 0.0f;
-    }
-    // byte offsets of this thread's items from a tile's first row; the rows of a V item follow at uniform steps
-    uint32_t k_off[NI], v_off[NI];
-#pragma unroll
-    for (int n = 0; n < NI; n++) {
-        const int idx = 256 * n + tid;
-        k_off[n] = 4u * ((uint32_t)(idx / (DPAD / 8)) * (uint32_t)kv_pitch + 8u * (uint32_t)(idx % (DPAD / 8)));
-        const int g = idx / DPAD;
-        v_off[n] = 4u * ((uint32_t)(16 * (g >> 1) + 4 * (g & 1)) * (uint32_t)kv_pitch + (uint32_t)(idx % DPAD));
-    }
-    auto load_tile = [&](int tile) RT_INLINE {
-        if (tile * kTile + kTile <= N) {  // wave-uniform
-            const char* kb = (const char*)(Kg + (size_t)tile * kTile * kv_pitch);
-            const char* vb = (const char*)(Vg + (size_t)tile * kTile * kv_pitch);
-#pragma unroll
-            for (int n = 0; n < NI; n++) {
-                const int idx = 256 * n + tid;
-                if (ITEMS % 256 == 0 || idx < ITEMS) {
-#pragma unroll
-                    for (int u = 0; u < 2; u++) {
-                        f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-                        if (kExactD || 8 * (idx % (DPAD / 8)) + 4 * u < D) z = *(const f32x4_t*)(kb + k_off[n] + 16 * u);
-                        kreg[n][u] = z;
-                    }
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const char* row = vb + (size_t)(8 * (e >> 2) + (e & 3)) * kv_pitch * 4;
-                        vreg[n][e] = (kExactD || idx % DPAD < D) ? *(const float*)(row + v_off[n]) : 0.0f;
-                    }
-                }
-            }
-            return;
-        }
-#pragma unroll
-        for (int n = 0; n < NI; n++) {
-            const int idx = 256 * n + tid;
-            if (ITEMS % 256 == 0 || idx < ITEMS) {
-                const int r = idx / (DPAD / 8), c = idx % (DPAD / 8);
-                const float* kr = Kg + (size_t)min(tile * kTile + r, N - 1) * kv_pitch + 8 * c;
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-                    if (kExactD || 8 * c + 4 * u < D) z = *(const f32x4_t*)(kr + 4 * u);
-                    kreg[n][u] = z;
-                }
-                const int d = idx % DPAD, g = idx / DPAD;
-                const int key0 = tile * kTile + 16 * (g >> 1) + 4 * (g & 1);
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int key = min(key0 + 8 * (e >> 2) + (e & 3), N - 1);
-                    vreg[n][e] = (kExactD || d < D) ? Vg[(size_t)key * kv_pitch + d] : 0.0f;
-                }
-            }
-        }
-    };
-    // Splitting: 24 NI steps, three for each pair of this thread's 8 NI (K and V of an item, four pairs each), then the writes.
-    struct Parts {
-        u32x4_t w[2 * NI][3];
-    };
-    SplitPair pair;
-    auto split_step = [&](Parts& o, int y) RT_INLINE {  // term y % 3 of pair y / 3
-        const int x = y / 3, u = y % 3, n = x / 8, e = x % 4;
-        const bool is_v = (x % 8) >= 4;
-        const float x0 = is_v ? vreg[n][2 * e] : kreg[n][e >> 1][2 * (e & 1)];
-        const float x1 = is_v ? vreg[n][2 * e + 1] : kreg[n][e >> 1][2 * (e & 1) + 1];
-        if (u == 0) pair.r = split_f32x2_t{x0, x1};
-        o.w[2 * n + (is_v ? 1 : 0)][u][e] = pair.step(u);
-        if (u < 2) return;
-        chk = __builtin_fmaf(x0, x0, chk);
-        chk = __builtin_fmaf(x1, x1, chk);
-        if (is_v) {  // scores of small keys are small whatever is lost of them; small values are the result's size
-            if (e == 0) v_max = 0.0f;
-            v_max = __builtin_fmaxf(__builtin_fmaxf(v_max, __builtin_fabsf(x0)), __builtin_fabsf(x1));
-            if (e == 3) chk = split_too_small(v_max) ? kSplitMost : chk;
-        }
-    };
-    auto write_tile = [&](const Parts& o, __bf16* kbuf, __bf16* vbuf) RT_INLINE {
-#pragma unroll
-        for (int n = 0; n < NI; n++) {
-            const int idx = 256 * n + tid;
-            if (ITEMS % 256 == 0 || idx < ITEMS) {
-                const int r = idx / (DPAD / 8), c = idx % (DPAD / 8), d = idx % DPAD, g = idx / DPAD;
-#pragma unroll
-                for (int u = 0; u < 3; u++) {
-                    *(u32x4_t*)(kbuf + u * KPL + r * LDK + 8 * c) = o.w[2 * n][u];
-                    *(u32x4_t*)(vbuf + u * VPL + d * LDV + 8 * g) = o.w[2 * n + 1][u];
-                }
-            }
-        }
-    };
-    auto store_tile = [&](__bf16* kbuf, __bf16* vbuf) RT_INLINE {
-        Parts o;
-#pragma unroll
-        for (int x = 0; x < 24 * NI; x++) split_step(o, x);
-        write_tile(o, kbuf, vbuf);
-    };
-
-    // A score tile (register i: key 8 (i/4) + 4 hh + i%4, query `col`): scaled and masked, then turned into weights.
-    // weights() returns the factor the sums so far have to be multiplied by.
-    auto scale_mask = [&](f32x16_t& s, int kv0) RT_INLINE {
-#pragma unroll
-        for (int i = 0; i < 16; i++) s[i] *= p.scale;
-        if ((kv0 + kTile > N) || (kCausal && kv0 + kTile - 1 > q0w)) {
-            asm volatile("");  // a branch: the selects cost more than the jump
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int kr = kv0 + 8 * (i >> 2) + 4 * hh + (i & 3);
-                if (kr >= N || (kCausal && kr > q_row)) s[i] = neg_inf();
-            }
-        }
-    };
-    auto row_max = [&](const f32x16_t& s) RT_INLINE {
-        float m_tile = neg_inf();  // NaN never wins, as in the reference's `if x > m`
-#pragma unroll
-        for (int i = 0; i < 16; i++) m_tile = __builtin_fmaxf(m_tile, s[i]);
-        auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(m_tile), __float_as_uint(m_tile), false, false);
-        return __builtin_fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    };
-    // the maximum goes to m_run; returns what is subtracted from the scores
-    float alpha = 0.0f;
-    auto take_max = [&](float m_tile) RT_INLINE {
-        const float m_new = __builtin_fmaxf(m_tile, m_run);
-        const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
-        alpha = (m_run == neg_inf()) ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_use) * kLog2e);
-        m_run = m_new;
-        return m_use;
-    };
-    auto add_sum = [&](float tile_l) RT_INLINE {
-        const float add = tile_l - l_low * alpha, before = l_run * alpha;
-        l_run = before + add;
-        l_low = (l_run - before) - add;
-    };
-    auto rescale = [&]() RT_INLINE {
-        if (__any(alpha != 1.0f)) {
-#pragma unroll
-            for (int t = 0; t < DT; t++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) acc_o[t][i] *= alpha;
-        }
-    };
-    // The 6 KS instructions of a score product: planes (a, c) of the six terms, the small ones first.  A plane of K is
-    // read from LDS one plane ahead of its use.
-    constexpr int kPlaneA[6] = {2, 1, 1, 0, 0, 0}, kPlaneC[6] = {0, 1, 0, 2, 1, 0};
-    bf16x8_t kf[2][KS];
-    auto read_plane = [&](const __bf16* kbuf, int a) RT_INLINE {
-#pragma unroll
-        for (int j = 0; j < KS; j++) kf[a & 1][j] = *(const bf16x8_t*)(kbuf + a * KPL + col * LDK + 8 * hh + 16 * j);
-    };
-    auto score_step = [&](const __bf16* kbuf, f32x16_t& s, int n) RT_INLINE {  // n: 0 .. 6 KS - 1, a constant
-        const int term = n / KS, j = n % KS;
-        if (n == 0) read_plane(kbuf, 1);
-        if (n == KS) read_plane(kbuf, 0);  // plane 2 has been used
-        s = mfma_h(kf[kPlaneA[term] & 1][j], qf[j].p[kPlaneC[term]], s);
-    };
-    auto zero16 = [](f32x16_t& x) RT_INLINE {
-#pragma unroll
-        for (int i = 0; i < 16; i++) x[i] = 0.0f;
-    };
-
-    __bf16* const v_lds = lds + 2 * KBUF;
-    load_tile(0);
-    store_tile(lds, v_lds);
-    if (n_tiles > 1) {
-        load_tile(1);
-        store_tile(lds + KBUF, v_lds + VBUF);
-    }
-    __syncthreads();
-    f32x16_t s_next;
-    zero16(s_next);
-    read_plane(lds, 2);
-#pragma unroll
-    for (int n = 0; n < 6 * KS; n++) score_step(lds, s_next, n);
-    int v_now = 0;  // tile % 3
-    // A step multiplies the next tile's scores while this tile's weights are formed, and this tile's weights with V while
-    // the tile after the next is split: the matrix instructions have vector work between them in the same wave.  The
-    // scheduling barriers keep that order; left to itself the compiler puts the one kind behind the other.
-    for (int tile = 0; tile < n_tiles; tile++) {
-        const __bf16* kn = lds + ((tile + 1) & 1) * KBUF;  // behind the last tile: scores of no tile, not used
-        const __bf16* vb = v_lds + v_now * VBUF + col * LDV + 8 * hh;
-        const int v_put = v_now == 0 ? 2 : v_now - 1;  // (tile + 2) % 3
-        if (tile + 2 < n_tiles) load_tile(tile + 2);
-        f32x16_t s = s_next;
-        scale_mask(s, tile * kTile);
-        read_plane(kn, 2);
-        zero16(s_next);
-        // a third of the score product beside the row maximum, the rest beside the weights, two at a time
-#pragma unroll
-        for (int n = 0; n < 2 * KS; n++) score_step(kn, s_next, n);
-        const float m_use = take_max(row_max(s));
-        rescale();
-        u32x4_t pw[2][3];
-        float part[2] = {0.0f, 0.0f};
-        SplitPair sp;
-        auto weight_step = [&](int x) RT_INLINE {  // 16 steps, two a pair
-            const int g = x / 2;
-            if (x % 2 == 0) {
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const float e = __builtin_amdgcn_exp2f((s[2 * g + u] - m_use) * kLog2e);
-                    part[u] += e;
-                    sp.r[u] = e;
-                }
-            } else {
-#pragma unroll
-                for (int u = 0; u < 3; u++) pw[g >> 2][u][g & 3] = sp.step(u);
-            }
-        };
-        RT_ORDER();
-#pragma unroll
-        for (int n = 0; n < 4 * KS; n++) {
-            score_step(kn, s_next, 2 * KS + n);
-#pragma unroll
-            for (int x = n * 16 / (4 * KS); x < (n + 1) * 16 / (4 * KS); x++) weight_step(x);
-            RT_ORDER();
-        }
-        add_sum(part[0] + part[1]);
-        // A tile's product in registers of its own, smallest terms first, then one addition to the sum: in the sum
-        // itself each of the twelve instructions would round at its size, and the error against 64 bits grew above
-        // that of the f32 kernel.
-        Parts kv_parts;
-#pragma unroll
-        for (int t = 0; t < DT; t++) {
-            f32x16_t o;
-            zero16(o);
-            bf16x8_t v[3][2];
-#pragma unroll
-            for (int a = 2; a >= 0; a--)
-#pragma unroll
-                for (int j = 0; j < 2; j++) v[a][j] = *(const bf16x8_t*)(vb + a * VPL + t * 32 * LDV + 16 * j);
-#pragma unroll
-            for (int term = 0; term < 6; term++) {
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    o = mfma_h(v[kPlaneA[term]][j], __builtin_bit_cast(bf16x8_t, pw[j][kPlaneC[term]]), o);
-                    // its share of the next tile's split: 24 NI steps behind 12 DT instructions
-                    const int n = (6 * t + term) * 2 + j;
-#pragma unroll
-                    for (int x = n * 24 * NI / (12 * DT); x < (n + 1) * 24 * NI / (12 * DT); x++) split_step(kv_parts, x);
-                    RT_ORDER();
-                }
+                for (int i = 0; i < 4; i++) x[4 * u + i] = z[i];
             }
 #pragma unroll
-            for (int i = 0; i < 16; i++) acc_o[t][i] += o[i];
+            for (int i = 0; i < 8; i++) chk = __builtin_fmaf(x[i], x[i], chk);
+            qf[j] = split8(x);
         }
-        write_tile(kv_parts, lds + (tile & 1) * KBUF, v_lds + v_put * VBUF);
-        v_now = v_now == 2 ? 0 : v_now + 1;
-        __syncthreads();
-    }
 
-    if (__syncthreads_or(!(chk < kSplitMost))) {
-        // something here the split does not carry: the wave's rows once more in f32, straight from memory
+        f32x16_t acc_o[DT];
 #pragma unroll
         for (int t = 0; t < DT; t++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc_o[t][i] = 0.0f;
-        m_run = neg_inf();
-        l_run = l_low = 0.0f;
-        for (int tile = 0; tile < n_wave; tile++) {
-            const int kv0 = tile * kTile;
-            f32x16_t s;
+        float m_run = neg_inf(), l_run = 0.0f, l_low = 0.0f;  // l_low: what the additions to l_run rounded off
+
+        const int kv_end = kCausal ? min(N, q0 + 4 * kTile) : N;
+        const int n_tiles = (kv_end + kTile - 1) / kTile;
+        const int wave_end = q0w >= Nq ? 0 : (kCausal ? min(N, q0w + kTile) : N);
+        const int n_wave = (wave_end + kTile - 1) / kTile;  // tiles this wave has scores in
+
+        // A tile's way into LDS: 8 elements of a K row per item, and 8 keys of a V column, in the order the weights sit in
+        // the score accumulators (slot 8g + e is key 16 (g/2) + 4 (g%2) + 8 (e/4) + e%4).  Rows behind the last key repeat
+        // it: their weights are exact zeros, and a zero times a finite value adds nothing.
+        f32x4_t kreg[NI][2];
+        float vreg[NI][8];
 #pragma unroll
-            for (int i = 0; i < 16; i++) s[i] = 0.0f;
-            for (int ks = 0; ks < DPAD / 2; ks++) {
-                const int d = 8 * (ks >> 2) + 4 * hh + (ks & 3);  // the f32 kernel's order
-                const float a = (kv0 + col < N && d < D) ? Kg[(size_t)(kv0 + col) * kv_pitch + d] : 0.0f;
-                const float bq = (q_row < Nq && d < D) ? Qg[(size_t)q_row * q_pitch + d] : 0.0f;
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(a, bq, s, 0, 0, 0);
+        for (int n = 0; n < NI; n++) {  // threads without an item split zeros
+            kreg[n][0] = kreg[n][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int e = 0; e < 8; e++) vreg[n][e] = 0.0f;
+        }
+        // byte offsets of this thread's items from a tile's first row; the rows of a V item follow at uniform steps
+        uint32_t k_off[NI], v_off[NI];
+#pragma unroll
+        for (int n = 0; n < NI; n++) {
+            const int idx = 256 * n + tid;
+            k_off[n] = 4u * ((uint32_t)(idx / (DPAD / 8)) * (uint32_t)kv_pitch + 8u * (uint32_t)(idx % (DPAD / 8)));
+            const int g = idx / DPAD;
+            v_off[n] = 4u * ((uint32_t)(16 * (g >> 1) + 4 * (g & 1)) * (uint32_t)kv_pitch + (uint32_t)(idx % DPAD));
+        }
+        auto load_tile = [&](int tile) RT_INLINE {
+            if (tile * kTile + kTile <= N) {  // wave-uniform
+                const char* kb = (const char*)(Kg + (size_t)tile * kTile * kv_pitch);
+                const char* vb = (const char*)(Vg + (size_t)tile * kTile * kv_pitch);
+#pragma unroll
+                for (int n = 0; n < NI; n++) {
+                    const int idx = 256 * n + tid;
+                    if (ITEMS % 256 == 0 || idx < ITEMS) {
+#pragma unroll
+                        for (int u = 0; u < 2; u++) {
+                            f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+                            if (kExactD || 8 * (idx % (DPAD / 8)) + 4 * u < D) z = *(const f32x4_t*)(kb + k_off[n] + 16 * u);
+                            kreg[n][u] = z;
+                        }
+#pragma unroll
+                        for (int e = 0; e < 8; e++) {
+                            const char* row = vb + (size_t)(8 * (e >> 2) + (e & 3)) * kv_pitch * 4;
+                            vreg[n][e] = (kExactD || idx % DPAD < D) ? *(const float*)(row + v_off[n]) : 0.0f;
+                        }
+                    }
+                }
+                return;
             }
-            scale_mask(s, kv0);
+#pragma unroll
+            for (int n = 0; n < NI; n++) {
+                const int idx = 256 * n + tid;
+                if (ITEMS % 256 == 0 || idx < ITEMS) {
+                    const int r = idx / (DPAD / 8), c = idx % (DPAD / 8);
+                    const float* kr = Kg + (size_t)min(tile * kTile + r, N - 1) * kv_pitch + 8 * c;
+#pragma unroll
+                    for (int u = 0; u < 2; u++) {
+                        f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+                        if (kExactD || 8 * c + 4 * u < D) z = *(const f32x4_t*)(kr + 4 * u);
+                        kreg[n][u] = z;
+                    }
+                    const int d = idx % DPAD, g = idx / DPAD;
+                    const int key0 = tile * kTile + 16 * (g >> 1) + 4 * (g & 1);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const int key = min(key0 + 8 * (e >> 2) + (e & 3), N - 1);
+                        vreg[n][e] = (kExactD || d < D) ? Vg[(size_t)key * kv_pitch + d] : 0.0f;
+                    }
+                }
+            }
+        };
+        // Splitting: 24 NI steps, three for each pair of this thread's 8 NI (K and V of an item, four pairs each), then the writes.
+        struct Parts {
+            u32x4_t w[2 * NI][3];
+        };
+        SplitPair pair;
+        auto split_step = [&](Parts& o, int y) RT_INLINE {  // term y % 3 of pair y / 3
+            const int x = y / 3, u = y % 3, n = x / 8, e = x % 4;
+            const bool is_v = (x % 8) >= 4;
+            const float x0 = is_v ? vreg[n][2 * e] : kreg[n][e >> 1][2 * (e & 1)];
+            const float x1 = is_v ? vreg[n][2 * e + 1] : kreg[n][e >> 1][2 * (e & 1) + 1];
+            if (u == 0) pair.r = split_f32x2_t{x0, x1};
+            o.w[2 * n + (is_v ? 1 : 0)][u][e] = pair.step(u);
+            if (u < 2) return;
+            chk = __builtin_fmaf(x0, x0, chk);
+            chk = __builtin_fmaf(x1, x1, chk);
+            if (is_v) {  // scores of small keys are small whatever is lost of them; small values are the result's size
+                if (e == 0) v_max = 0.0f;
+                v_max = __builtin_fmaxf(__builtin_fmaxf(v_max, __builtin_fabsf(x0)), __builtin_fabsf(x1));
+                if (e == 3) chk = split_too_small(v_max) ? kSplitMost : chk;
+            }
+        };
+        auto write_tile = [&](const Parts& o, __bf16* kbuf, __bf16* vbuf) RT_INLINE {
+#pragma unroll
+            for (int n = 0; n < NI; n++) {
+                const int idx = 256 * n + tid;
+                if (ITEMS % 256 == 0 || idx < ITEMS) {
+                    const int r = idx / (DPAD / 8), c = idx % (DPAD / 8), d = idx % DPAD, g = idx / DPAD;
+#pragma unroll
+                    for (int u = 0; u < 3; u++) {
+                        *(u32x4_t*)(kbuf + u * KPL + r * LDK + 8 * c) = o.w[2 * n][u];
+                        *(u32x4_t*)(vbuf + u * VPL + d * LDV + 8 * g) = o.w[2 * n + 1][u];
+                    }
+                }
+            }
+        };
+        auto store_tile = [&](__bf16* kbuf, __bf16* vbuf) RT_INLINE {
+            Parts o;
+#pragma unroll
+            for (int x = 0; x < 24 * NI; x++) split_step(o, x);
+            write_tile(o, kbuf, vbuf);
+        };
+
+        // A score tile (register i: key 8 (i/4) + 4 hh + i%4, query `col`): scaled and masked, then turned into weights.
+        // weights() returns the factor the sums so far have to be multiplied by.
+        auto scale_mask = [&](f32x16_t& s, int kv0) RT_INLINE {
+#pragma unroll
+            for (int i = 0; i < 16; i++) s[i] *= p.scale;
+            if ((kv0 + kTile > N) || (kCausal && kv0 + kTile - 1 > q0w)) {
+                asm volatile("");  // a branch: the selects cost more than the jump
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int kr = kv0 + 8 * (i >> 2) + 4 * hh + (i & 3);
+                    if (kr >= N || (kCausal && kr > q_row)) s[i] = neg_inf();
+                }
+            }
+        };
+        auto row_max = [&](const f32x16_t& s) RT_INLINE {
+            float m_tile = neg_inf();  // NaN never wins, as in the reference's `if x > m`
+#pragma unroll
+            for (int i = 0; i < 16; i++) m_tile = __builtin_fmaxf(m_tile, s[i]);
+            auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(m_tile), __float_as_uint(m_tile), false, false);
+            return __builtin_fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+        };
+        // the maximum goes to m_run; returns what is subtracted from the scores
+        float alpha = 0.0f;
+        auto take_max = [&](float m_tile) RT_INLINE {
+            const float m_new = __builtin_fmaxf(m_tile, m_run);
+            const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
+            alpha = (m_run == neg_inf()) ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_use) * kLog2e);
+            m_run = m_new;
+            return m_use;
+        };
+        auto add_sum = [&](float tile_l) RT_INLINE {
+            const float add = tile_l - l_low * alpha, before = l_run * alpha;
+            l_run = before + add;
+            l_low = (l_run - before) - add;
+        };
+        auto rescale = [&]() RT_INLINE {
+            if (__any(alpha != 1.0f)) {
+#pragma unroll
+                for (int t = 0; t < DT; t++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc_o[t][i] *= alpha;
+            }
+        };
+        // The 6 KS instructions of a score product: planes (a, c) of the six terms, the small ones first.  A plane of K is
+        // read from LDS one plane ahead of its use.
+        constexpr int kPlaneA[6] = {2, 1, 1, 0, 0, 0}, kPlaneC[6] = {0, 1, 0, 2, 1, 0};
+        bf16x8_t kf[2][KS];
+        auto read_plane = [&](const __bf16* kbuf, int a) RT_INLINE {
+#pragma unroll
+            for (int j = 0; j < KS; j++) kf[a & 1][j] = *(const bf16x8_t*)(kbuf + a * KPL + col * LDK + 8 * hh + 16 * j);
+        };
+        auto score_step = [&](const __bf16* kbuf, f32x16_t& s, int n) RT_INLINE {  // n: 0 .. 6 KS - 1, a constant
+            const int term = n / KS, j = n % KS;
+            if (n == 0) read_plane(kbuf, 1);
+            if (n == KS) read_plane(kbuf, 0);  // plane 2 has been used
+            s = mfma_h(kf[kPlaneA[term] & 1][j], qf[j].p[kPlaneC[term]], s);
+        };
+        auto zero16 = [](f32x16_t& x) RT_INLINE {
+#pragma unroll
+            for (int i = 0; i < 16; i++) x[i] = 0.0f;
+        };
+
+        __bf16* const v_lds = lds + 2 * KBUF;
+        load_tile(0);
+        store_tile(lds, v_lds);
+        if (n_tiles > 1) {
+            load_tile(1);
+            store_tile(lds + KBUF, v_lds + VBUF);
+        }
+        __syncthreads();
+        f32x16_t s_next;
+        zero16(s_next);
+        read_plane(lds, 2);
+#pragma unroll
+        for (int n = 0; n < 6 * KS; n++) score_step(lds, s_next, n);
+        int v_now = 0;  // tile % 3
+        // A step multiplies the next tile's scores while this tile's weights are formed, and this tile's weights with V while
+        // the tile after the next is split: the matrix instructions have vector work between them in the same wave.  The
+        // scheduling barriers keep that order; left to itself the compiler puts the one kind behind the other.
+        for (int tile = 0; tile < n_tiles; tile++) {
+            const __bf16* kn = lds + ((tile + 1) & 1) * KBUF;  // behind the last tile: scores of no tile, not used
+            const __bf16* vb = v_lds + v_now * VBUF + col * LDV + 8 * hh;
+            const int v_put = v_now == 0 ? 2 : v_now - 1;  // (tile + 2) % 3
+            if (tile + 2 < n_tiles) load_tile(tile + 2);
+            f32x16_t s = s_next;
+            scale_mask(s, tile * kTile);
+            read_plane(kn, 2);
+            zero16(s_next);
+            // a third of the score product beside the row maximum, the rest beside the weights, two at a time
+#pragma unroll
+            for (int n = 0; n < 2 * KS; n++) score_step(kn, s_next, n);
             const float m_use = take_max(row_max(s));
-            float tile_l = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                s[i] = __builtin_amdgcn_exp2f((s[i] - m_use) * kLog2e);
-                tile_l += s[i];
-            }
-            add_sum(tile_l);
             rescale();
+            u32x4_t pw[2][3];
+            float part[2] = {0.0f, 0.0f};
+            SplitPair sp;
+            auto weight_step = [&](int x) RT_INLINE {  // 16 steps, two a pair
+                const int g = x / 2;
+                if (x % 2 == 0) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int kr = kv0 + 8 * (i >> 2) + 4 * hh + (i & 3);
+                    for (int u = 0; u < 2; u++) {
+                        const float e = __builtin_amdgcn_exp2f((s[2 * g + u] - m_use) * kLog2e);
+                        part[u] += e;
+                        sp.r[u] = e;
+                    }
+                } else {
 #pragma unroll
-                for (int t = 0; t < DT; t++) {
-                    const int d = 32 * t + col;
-                    const float a = (kr < N && d < D) ? Vg[(size_t)kr * kv_pitch + d] : 0.0f;
-                    acc_o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, s[i], acc_o[t], 0, 0, 0);
+                    for (int u = 0; u < 3; u++) pw[g >> 2][u][g & 3] = sp.step(u);
+                }
+            };
+            RT_ORDER();
+#pragma unroll
+            for (int n = 0; n < 4 * KS; n++) {
+                score_step(kn, s_next, 2 * KS + n);
+#pragma unroll
+                for (int x = n * 16 / (4 * KS); x < (n + 1) * 16 / (4 * KS); x++) weight_step(x);
+                RT_ORDER();
+            }
+            add_sum(part[0] + part[1]);
+            // A tile's product in registers of its own, smallest terms first, then one addition to the sum: in the sum
+            // itself each of the twelve instructions would round at its size, and the error against 64 bits grew above
+            // that of the f32 kernel.
+            Parts kv_parts;
+#pragma unroll
+            for (int t = 0; t < DT; t++) {
+                f32x16_t o;
+                zero16(o);
+                bf16x8_t v[3][2];
+#pragma unroll
+                for (int a = 2; a >= 0; a--)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) v[a][j] = *(const bf16x8_t*)(vb + a * VPL + t * 32 * LDV + 16 * j);
+#pragma unroll
+                for (int term = 0; term < 6; term++) {
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        o = mfma_h(v[kPlaneA[term]][j], __builtin_bit_cast(bf16x8_t, pw[j][kPlaneC[term]]), o);
+                        // its share of the next tile's split: 24 NI steps behind 12 DT instructions
+                        const int n = (6 * t + term) * 2 + j;
+#pragma unroll
+                        for (int x = n * 24 * NI / (12 * DT); x < (n + 1) * 24 * NI / (12 * DT); x++) split_step(kv_parts, x);
+                        RT_ORDER();
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc_o[t][i] += o[i];
+            }
+            write_tile(kv_parts, lds + (tile & 1) * KBUF, v_lds + v_put * VBUF);
+            v_now = v_now == 2 ? 0 : v_now + 1;
+            __syncthreads();
+        }
+
+        if (__syncthreads_or(!(chk < kSplitMost))) {
+            // something here the split does not carry: the wave's rows once more in f32, straight from memory
+#pragma unroll
+            for (int t = 0; t < DT; t++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc_o[t][i] = 0.0f;
+            m_run = neg_inf();
+            l_run = l_low = 0.0f;
+            for (int tile = 0; tile < n_wave; tile++) {
+                const int kv0 = tile * kTile;
+                f32x16_t s;
+#pragma unroll
+                for (int i = 0; i < 16; i++) s[i] = 0.0f;
+                for (int ks = 0; ks < DPAD / 2; ks++) {
+                    const int d = 8 * (ks >> 2) + 4 * hh + (ks & 3);  // the f32 kernel's order
+                    const float a = (kv0 + col < N && d < D) ? Kg[(size_t)(kv0 + col) * kv_pitch + d] : 0.0f;
+                    const float bq = (q_row < Nq && d < D) ? Qg[(size_t)q_row * q_pitch + d] : 0.0f;
+                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(a, bq, s, 0, 0, 0);
+                }
+                scale_mask(s, kv0);
+                const float m_use = take_max(row_max(s));
+                float tile_l = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    s[i] = __builtin_amdgcn_exp2f((s[i] - m_use) * kLog2e);
+                    tile_l += s[i];
+                }
+                add_sum(tile_l);
+                rescale();
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int kr = kv0 + 8 * (i >> 2) + 4 * hh + (i & 3);
+#pragma unroll
+                    for (int t = 0; t < DT; t++) {
+                        const int d = 32 * t + col;
+                        const float a = (kr < N && d < D) ? Vg[(size_t)kr * kv_pitch + d] : 0.0f;
+                        acc_o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, s[i], acc_o[t], 0, 0, 0);
+                    }
                 }
             }
         }
-    }
 
-    const float l = l_run + other_half(l_run);
-    const bool good = (l > 0.0f) && (fabsf(l) != __uint_as_float(0x7f800000u)) && (l == l);
-    const float inv_l = 1.0f / l;
-    if (q_row < Nq) {
-    if (p.lse && hh == 0) p.lse[((size_t)b * p.heads + h) * (size_t)Nq + q_row] = m_run + logf(l);
-    float* o_row = Og + (size_t)q_row * o_pitch;
+        const float l = l_run + other_half(l_run);
+        const bool good = (l > 0.0f) && (fabsf(l) != __uint_as_float(0x7f800000u)) && (l == l);
+        const float inv_l = 1.0f / l;
+        if (q_row < Nq) {
+        if (p.lse && hh == 0) p.lse[((size_t)b * p.heads + h) * (size_t)Nq + q_row] = m_run + logf(l);
+        float* o_row = Og + (size_t)q_row * o_pitch;
 #pragma unroll
-    for (int t = 0; t < DT; t++)
+        for (int t = 0; t < DT; t++)
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int d = 32 * t + 8 * g + 4 * hh;
-            f32x4_t o;
+            for (int g = 0; g < 4; g++) {
+                const int d = 32 * t + 8 * g + 4 * hh;
+                f32x4_t o;
 #pragma unroll
-            for (int i = 0; i < 4; i++) o[i] = good ? acc_o[t][4 * g + i] * inv_l : quiet_nan();
-            if (kExactD || d < D) *(f32x4_t*)(o_row + d) = o;
+                for (int i = 0; i < 4; i++) o[i] = good ? acc_o[t][4 * g + i] * inv_l : quiet_nan();
+                if (kExactD || d < D) *(f32x4_t*)(o_row + d) = o;
+            }
         }
-    }
-    // (every wave is behind the barrier of the test above: the tiles of the next block may come into LDS)
-    if (DT <= 2 || !kCausal || p.zigzag != 2 || qblk == x || n_blk - 1 - x == x) return;
-    qblk = x;
+        // (every wave is behind the barrier of the test above: the tiles of the next block may come into LDS)
+        if (DT <= 2 || !kCausal || p.zigzag != 2 || qblk == x || n_blk - 1 - x == x) return;
+        qblk = x;
     }
 }
 
