@@ -536,6 +536,7 @@ __global__ __launch_bounds__(64) void decode_split_kernel(DecodeSplitParams p) {
 // 26.7 / 17.9, one of 2048 9.3 / 8.5.
 constexpr int kLatWaves = 4;
 constexpr int kLatMaxSplits = 24;
+static_assert(kLatMaxSplits <= 64, "the fold gives every split a lane");
 
 template <int HD>
 __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSplitParams p) {
@@ -647,7 +648,7 @@ __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSp
         for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
         const float f = __builtin_amdgcn_exp2f(ml[0] - ((m == neg_inf()) ? 0.0f : m));
         const float l = wave_sum(ml[1] * f);
-        wgt[lane][h] = f;  // 0 past the last split
+        if (lane < kLatMaxSplits) wgt[lane][h] = f;  // (lanes past the last split hold 0)
         if (lane == 0) inv_l[h] = 1.0f / l;
     }
     __syncthreads();

@@ -38,3 +38,24 @@ def test_contexts_at_the_edges(oracle, b, hq, hkv, d, max_seq, lens):
         if b == 1:
             break
     stream.destroy()
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (2, 2, 64), (16, 1, 64), (16, 1, 256)])
+def test_every_count_of_splits_folds_whole(oracle, hq, hkv, d):
+    """Contexts whose splits number 1, 2, 3, ... to the most there are: every head's weights and sum stand, whichever
+    waves of the folding workgroup come late (V is one everywhere, so a missing weight, sum or partial moves a row away
+    from one; a weight is rounded to bf16, 2^-9, the sum of weights is not)."""
+    max_seq = 3200 if d < 256 else 1280
+    qb, _ = bf16_round(seeded_normal((1, hq, d), 1))
+    kb, _ = bf16_round(seeded_normal((1, hkv, max_seq, d), 2))
+    dq, dk = dev(qb), dev(kb)
+    dv = dev(np.full(hkv * max_seq * d, 0x3F80, dtype=np.uint16))
+    outs, lens = [], list(range(97, max_seq, 128))
+    for n in lens:
+        outs.append(ra.HipStorage(hq * d * 2))
+        outs[-1].upload(np.full(hq * d, 0x7B7B, dtype=np.uint16))
+        K.gqa_decode_online_bf16(None, dq, dk, dv, outs[-1], hq, hkv, n, d, max_seq)
+    ra.synchronize()
+    for n, o in zip(lens, outs):
+        got = oracle.bf16_to_f32(o.download(np.uint16))
+        assert np.abs(got - 1).max() <= 2 ** -7, n
