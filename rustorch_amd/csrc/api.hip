@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <map>
 #include <memory>
@@ -328,31 +329,92 @@ int stream_slot_scratch(hipStream_t stream, float** ptr, size_t* bytes, rt_err_d
     return RT_OK;
 }
 
+int is_capturing(hipStream_t stream, bool* yes, rt_err_detail* err) {
+    *yes = false;
+    if (!stream) return RT_OK;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(stream, &cap), "hipStreamIsCapturing");
+    *yes = cap != hipStreamCaptureStatusNone;
+    return RT_OK;
+}
+
+// A number no other launch of the process has, its low 8 bits zero.  It starts at no particular place, so that what earlier
+// processes left in memory holds no number of this one.
+uint64_t next_launch_id() {
+    static std::atomic<uint64_t> next{(uint64_t)std::chrono::steady_clock::now().time_since_epoch().count() * 0x9e3779b97f4a7c15ull};
+    return next.fetch_add(1, std::memory_order_relaxed) << 8;
+}
+
 // How the decode kernels run a call: in the latency form (one launch, partials folded inside it) where that is the faster
-// one, the stream has a slot (the slot's counters belong to it alone) and is not being captured.  A graph may be
-// replayed on any stream, beside other work of the stream it was captured from, so what is captured keeps no state
-// between launches: split and merge kernel, whose two launches cost little inside a graph.  max_len: the longest context
+// one and the stream is not being captured: a captured launch would bring its id along on every replay, so with more than
+// one split a graph gets split and merge kernel, whose two launches cost little inside it.  max_len: the longest context
 // there can be.
 int plan_decode(hipStream_t stream, rt::DecodeSplitParams& p, int max_len, rt_err_detail* err) {
     const int n_splits = rt::decode_latency_splits(p.batch, p.heads, p.kv_heads, p.dim, p.max_seq, max_len, g_num_cus);
     if (n_splits == 0 || ((uintptr_t)p.out & 7) != 0) return RT_OK;
-    if (n_splits > 1) {  // (one split: no partials, no state)
-        if ((long long)p.batch * p.kv_heads > rt::kDecodeCounters) return RT_OK;
-        if (stream) {
-            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-            HIP_TRY(hipStreamIsCapturing(stream, &cap), "hipStreamIsCapturing");
-            if (cap != hipStreamCaptureStatusNone) return RT_OK;
-        }
-        int slot = -1;
-        int rc = stream_slot(stream, &slot, err);
-        if (rc || slot < 0) return rc;
-        HIP_TRY(rt::decode_counters(slot, &p.counters), "hipGetSymbolAddress(decode counters)");
+    if (n_splits > 1) {  // (one split: no partials)
+        bool captured = false;
+        int rc = is_capturing(stream, &captured, err);
+        if (rc || captured) return rc;
+        p.launch_id = next_launch_id();
     }
     p.n_splits = n_splits;
     return RT_OK;
 }
 
-// the caller holds g_ws_mutex.  The slot's next owner must find its counters at rest: the stream is waited for.
+// hipStreamPerThread is one handle for a stream of every thread, so calls on it share a slot (or block) that nothing
+// orders.  They take turns: a call's launch waits, on the GPU, for the event behind the launch of the call before it.
+// Under capture, where a wait for work outside it is an error, the call has to do without scratch.
+class ScratchTurn {
+public:
+    int enter(hipStream_t stream, bool* scratch, rt_err_detail* err) {
+        *scratch = true;
+        if (stream != hipStreamPerThread) return RT_OK;
+        bool captured = false;
+        int rc = is_capturing(stream, &captured, err);
+        if (rc) return rc;
+        if (captured) {
+            *scratch = false;
+            return RT_OK;
+        }
+        int dev = 0;
+        HIP_TRY(hipGetDevice(&dev), "hipGetDevice");
+        lock_ = std::unique_lock<std::mutex>(mutex());
+        hipEvent_t& e = events()[dev];
+        if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+        HIP_TRY(hipStreamWaitEvent(stream, e, 0), "hipStreamWaitEvent");
+        event_ = e;
+        return RT_OK;
+    }
+    // behind the launch
+    int leave(hipStream_t stream, rt_err_detail* err) {
+        if (!event_) return RT_OK;
+        const hipError_t e = hipEventRecord(event_, stream);
+        if (e != hipSuccess) (void)hipStreamSynchronize(stream);
+        HIP_TRY(e, "hipEventRecord");
+        return RT_OK;
+    }
+    static void release() {
+        std::lock_guard<std::mutex> lock(mutex());
+        for (auto& e : events())
+            if (e.second) (void)hipEventDestroy(e.second);
+        events().clear();
+    }
+
+private:
+    static std::mutex& mutex() {
+        static std::mutex m;
+        return m;
+    }
+    static std::map<int, hipEvent_t>& events() {  // by device
+        static std::map<int, hipEvent_t> m;
+        return m;
+    }
+    std::unique_lock<std::mutex> lock_;
+    hipEvent_t event_ = nullptr;
+};
+
+// the caller holds g_ws_mutex.  Launches of the stream may still use the slot: it is waited for.
 void release_stream_slot(int dev, hipStream_t stream) {
     auto it = g_slots.find(dev);
     if (it == g_slots.end()) return;
@@ -746,8 +808,6 @@ RT_API int rt_init(int device, rt_err_detail* err) {
     size_t scratch_bytes = 0;
     HIP_TRY(rt::decode_static_scratch(&scratch, &scratch_bytes), "hipGetSymbolAddress(static scratch)");
     HIP_TRY(rt::stream_static_scratch(0, &scratch, &scratch_bytes), "hipGetSymbolAddress(stream scratch)");
-    uint32_t* counters = nullptr;
-    HIP_TRY(rt::decode_counters(0, &counters), "hipGetSymbolAddress(decode counters)");
     return RT_OK;
 }
 
@@ -1665,6 +1725,24 @@ static int check_decode_dims(int32_t batch, int32_t n_heads, int32_t n_kv, int32
     return RT_OK;
 }
 
+// Scratch of a single-sequence decode (p.ws, p.n_waves, p.compact).
+static int online_scratch(hipStream_t stream, rt::DecodeSplitParams& p, rt_err_detail* err) {
+    size_t slot_bytes = 0;
+    int rc = stream_slot_scratch(stream, &p.ws, &slot_bytes, err);
+    if (rc) return rc;
+    if (p.ws) {
+        // compact numbering: (waves + kv heads) * group partials of dim + 2 floats
+        const size_t per_wave = (size_t)(p.heads / p.kv_heads) * ((size_t)p.dim + 2) * sizeof(float);
+        const long long fit = (long long)(slot_bytes / per_wave) - p.kv_heads;
+        if (fit >= std::min<long long>(p.n_waves, 256)) {
+            p.n_waves = (int)std::min<long long>(p.n_waves, fit);
+            p.compact = 1;
+            return RT_OK;
+        }
+    }
+    return stream_workspace(stream, rt::decode_split_workspace_bytes(1, p.heads, p.dim, p.max_seq), &p.ws, err);
+}
+
 RT_API int rt_gqa_decode_online_bf16(void* stream, const void* q, const void* k_cache, const void* v_cache,
                                      void* out, int32_t n_heads, int32_t n_kv, int32_t kv_len, int32_t head_dim,
                                      int32_t max_seq, rt_err_detail* err) {
@@ -1682,42 +1760,19 @@ RT_API int rt_gqa_decode_online_bf16(void* stream, const void* q, const void* k_
     // element-wise kernel below
     const bool aligned = ((((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0);
     if (aligned && rt::decode_split_supported(n_heads, n_kv, head_dim)) {
-        // the split-K kernels of the batched entry, on a batch of one.  The reference's signature has no workspace
-        // argument: the partials go to this stream's slot of the library's fixed scratch block (nothing is allocated,
-        // so the call can be captured into a graph), in the compact slot numbering; only when no slot is free, or the
-        // slot cannot hold a useful number of partials, to a buffer the library allocates per stream
+        // the split-K kernels of the batched entry, on a batch of one
         rt::DecodeSplitParams sp{};
         sp.span_min = rt::decode_split_span_min(1);
         // no more one-wave workgroups than there are spans of the minimum length (short contexts)
         const long long steps = (long long)n_kv * ((kv_len + 31) / 32);
         const long long spans = (steps + sp.span_min - 1) / sp.span_min;
         sp.n_waves = (int)std::min<long long>(g_decode_waves, std::max<long long>(spans, 1));
-        float* ws = nullptr;
-        size_t slot_bytes = 0;
-        rc = stream_slot_scratch((hipStream_t)stream, &ws, &slot_bytes, err);
-        if (rc) return rc;
-        if (ws) {
-            // compact numbering: (waves + n_kv) * group partials of head_dim + 2 floats
-            const size_t per_wave = (size_t)(n_heads / n_kv) * ((size_t)head_dim + 2) * sizeof(float);
-            const long long fit = (long long)(slot_bytes / per_wave) - n_kv;
-            if (fit >= std::min<long long>(sp.n_waves, 256)) {
-                sp.n_waves = (int)std::min<long long>(sp.n_waves, fit);
-                sp.compact = 1;
-            } else {
-                ws = nullptr;
-            }
-        }
-        if (!ws) {
-            rc = stream_workspace((hipStream_t)stream, rt::decode_split_workspace_bytes(1, n_heads, head_dim, max_seq), &ws, err);
-            if (rc) return rc;
-        }
         sp.q = (const uint16_t*)q;
         sp.k_cache = (const uint16_t*)k_cache;
         sp.v_cache = (const uint16_t*)v_cache;
         sp.out = (uint16_t*)out;
         sp.kv_lens = nullptr;
         sp.kv_len = kv_len;
-        sp.ws = ws;
         sp.batch = 1;
         sp.heads = n_heads;
         sp.kv_heads = n_kv;
@@ -1727,8 +1782,26 @@ RT_API int rt_gqa_decode_online_bf16(void* stream, const void* q, const void* k_
         sp.scale_log2e = (1.0f / sqrtf((float)head_dim)) * rt::kLog2eHost;
         rc = plan_decode((hipStream_t)stream, sp, kv_len, err);
         if (rc) return rc;
-        HIP_TRY(rt::launch_decode_split((hipStream_t)stream, sp), "decode_split launch");
-        return RT_OK;
+        // The reference's signature has no workspace argument: the partials go to this stream's slot of the library's fixed
+        // scratch block (nothing is allocated, so the call can be captured into a graph), in the compact slot numbering;
+        // only when no slot is free, or the slot cannot hold a useful number of partials, to a buffer the library
+        // allocates per stream.  Where neither may be used: one split, which leaves no partials, if the output is aligned for it.
+        ScratchTurn turn;
+        if (sp.n_splits != 1) {
+            bool scratch = false;
+            rc = turn.enter((hipStream_t)stream, &scratch, err);
+            if (rc) return rc;
+            if (scratch) {
+                rc = online_scratch((hipStream_t)stream, sp, err);
+                if (rc) return rc;
+            } else if (((uintptr_t)out & 7) == 0) {
+                sp.n_splits = 1;
+            }
+        }
+        if (sp.ws || sp.n_splits == 1) {
+            HIP_TRY(rt::launch_decode_split((hipStream_t)stream, sp), "decode_split launch");
+            return turn.leave((hipStream_t)stream, err);
+        }
     }
     rt::AttnRowsParams p{};
     p.q = q;
@@ -1843,15 +1916,23 @@ RT_API int rt_gqa_decode_chunk_bf16(void* stream, const void* q, const void* k_c
     float* ws = nullptr;
     const size_t part_rows = (size_t)batch * n_kv * (size_t)((rows + 31) / 32 * 32);
     const size_t per_split = part_rows * ((size_t)head_dim + 2) * sizeof(float);
+    ScratchTurn turn;
+    if (n_splits > 1) {
+        bool scratch = false;
+        rc = turn.enter((hipStream_t)stream, &scratch, err);
+        if (rc) return rc;
+        if (!scratch) n_splits = 1;
+    }
     if (n_splits > 1) {
         size_t slot_bytes = 0;
         rc = stream_slot_scratch((hipStream_t)stream, &ws, &slot_bytes, err);
         if (rc) return rc;
         if (!ws || slot_bytes < per_split * (size_t)n_splits) {
-            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-            if (ws && stream) HIP_TRY(hipStreamIsCapturing((hipStream_t)stream, &cap), "hipStreamIsCapturing");
+            bool captured = false;
+            if (ws) rc = is_capturing((hipStream_t)stream, &captured, err);
+            if (rc) return rc;
             float* kept = nullptr;
-            if (cap == hipStreamCaptureStatusNone) {
+            if (!captured) {
                 rc = stream_workspace((hipStream_t)stream, per_split * (size_t)n_splits, &kept, err);
                 if (rc && !ws) return rc;
                 clear_err(err);
@@ -1866,7 +1947,7 @@ RT_API int rt_gqa_decode_chunk_bf16(void* stream, const void* q, const void* k_c
         t.part_ml = ws + part_rows * (size_t)n_splits * (size_t)head_dim;
     }
     HIP_TRY(rt::launch_flash_tile_bf16((hipStream_t)stream, t), "flash_tile_bf16 launch");
-    return RT_OK;
+    return turn.leave((hipStream_t)stream, err);
 }
 
 RT_API size_t rt_gqa_decode_workspace_bytes(int32_t batch, int32_t n_heads, int32_t n_kv, int32_t head_dim,
@@ -2131,6 +2212,7 @@ RT_API int rt_shutdown(rt_err_detail* err) {
         g_ws.clear();
         g_slots.clear();
     }
+    ScratchTurn::release();
     {
         std::lock_guard<std::mutex> lock(g_stage.mutex);
         crew().stop();

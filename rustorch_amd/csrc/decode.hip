@@ -404,14 +404,41 @@ __device__ __forceinline__ f32x2v get2(__amdgpu_buffer_rsrc_t rs, uint32_t byte)
     return __builtin_bit_cast(f32x2v, __builtin_amdgcn_raw_buffer_load_b64(rs, byte, 0, kScopeDevice));
 }
 __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// Counts one finished partial of `n`; true for the one that completes the set, which also puts the counter back to 0
-// for the next launch.
-__device__ __forceinline__ bool count_partial(uint32_t* counter, int n) {
-    const uint32_t old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (old + 1u != (uint32_t)n) return false;
-    __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return true;
-}
+// A segment's word, (launch id | count): the memory it lies in holds anything at first, another launch's word included,
+// so every workgroup makes sure, ahead of its own count, that the word carries this launch's id: it replaces what it has
+// seen there unless that has the id.  A replacement fails only if another workgroup of the launch was first.  `seen` is
+// requested ahead of everything else and the replacement sent when the first rows are there, so that neither is waited for
+// by itself (sent behind the walk: 0.4 us more a call).  The token of a context of 2048, 32 / 8 heads of 128, with its
+// preparation: 11.2 us with counters of 4 bytes side by side that the library kept at zero, 11.5 with words side by side,
+// 10.7 with a line for each.
+typedef unsigned long long word_t;
+constexpr int kWordPitch = 128;  // bytes from one segment's word to the next: atomics on one line wait for each other
+struct SegWord {
+    word_t* at;
+    word_t id, seen, got;
+    __device__ __forceinline__ bool ours(word_t x) const { return ((x ^ id) >> 8) == 0; }
+    __device__ __forceinline__ void replace() {
+        got = seen;
+        __hip_atomic_compare_exchange_strong(at, &got, ours(seen) ? seen : id, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void request(word_t* word, word_t launch_id) {
+        at = word;
+        id = launch_id;
+        seen = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void settle() {
+        while (got != seen && !ours(got)) {
+            seen = got;
+            replace();
+        }
+    }
+    // counts one finished partial of `n`; true for the one that completes the set
+    __device__ __forceinline__ bool count(int n) {
+        const word_t old = __hip_atomic_fetch_add(at, (word_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return (int)(old & 255u) + 1 == n;
+    }
+};
 
 struct DecCursor {  // position in the flat step list
     int b, kvh, st, steps_b, len_b;
@@ -536,7 +563,7 @@ __global__ __launch_bounds__(64) void decode_split_kernel(DecodeSplitParams p) {
 // 26.7 / 17.9, one of 2048 9.3 / 8.5.
 constexpr int kLatWaves = 4;
 constexpr int kLatMaxSplits = 24;
-static_assert(kLatMaxSplits <= 64, "the fold gives every split a lane");
+static_assert(kLatMaxSplits <= 64, "the fold gives every split a lane, a segment's word eight bits of count");
 
 template <int HD>
 __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSplitParams p) {
@@ -554,6 +581,10 @@ __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSp
     const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
     const int G = p.heads / p.kv_heads;
     const int seg = b * p.kv_heads + kvh;
+    const uint32_t n_slots = (uint32_t)p.batch * p.heads * p.n_splits, ml_byte = n_slots * HD * 4;
+    SegWord word;
+    if (tid == 0 && p.n_splits > 1)
+        word.request((word_t*)((unsigned char*)p.ws + (size_t)n_slots * (HD + 2) * 4 + (size_t)seg * kWordPitch), p.launch_id);
     const int len = dec_len(p, b), steps = dec_steps(len);
     const int per = max((steps + p.n_splits - 1) / p.n_splits, kLatWaves);
     const int n_act = (steps + per - 1) / per;  // splits that hold keys
@@ -563,6 +594,7 @@ __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSp
             for (int i = tid; i < G * HD / 4; i += NT) *(u32x2_t*)(out + 4 * i) = u32x2_t{0u, 0u};
         return;
     }
+    const bool counts = tid == 0 && n_act > 1;
     const int t1 = min(steps, (split + 1) * per);
     uint16_t* const Kw = (uint16_t*)lds + wave * T::HALFS;
     uint16_t* const Vw = Kw + kDecRows * T::LDK;
@@ -571,13 +603,14 @@ __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSp
     DecState<HD> state;
     state.reset();
     int t = split * per + wave;
-    if (t < t1) {
+    if (t < t1) {  // (so it is for wave 0)
         u32x4_t kreg[T::NLD], vreg[T::NLD];
         bf16x8_t qreg[T::KS];
         dec_load<HD>(p, b, kvh, t, len, lane, kreg, vreg);
         dec_load_q<HD>(p, b, kvh, lane, qreg);
         for (; t < t1; t += kLatWaves) {
             dec_park<HD>(Kw, Vw, lane, kreg, vreg);
+            if (counts && t == split * per) word.replace();
             if (t + kLatWaves < t1) dec_load<HD>(p, b, kvh, t + kLatWaves, len, lane, kreg, vreg);
             dec_step<HD>(Kw, Vw, lane, len - t * kDecRows, c, lazy, qreg, state);
         }
@@ -604,7 +637,6 @@ __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSp
     }
     if (wave == 0 && g4 == 0) inv_l[hcol] = 1.0f / l_wg;
     __syncthreads();
-    const uint32_t n_slots = (uint32_t)p.batch * p.heads * p.n_splits, ml_byte = n_slots * HD * 4;
     const uint32_t slot0 = (uint32_t)seg * p.n_splits * G;  // partial k of head h: slot0 + k * G + h
     const __amdgpu_buffer_rsrc_t ws_rs = __builtin_amdgcn_make_buffer_rsrc((void*)p.ws, 0, n_slots * (HD + 2) * 4, kBufferFlags);
     for (int x = tid; x < G * HD / 4; x += NT) {
@@ -621,9 +653,10 @@ __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSp
     }
     if (n_act == 1) return;
     if (tid < G) put2(ws_rs, ml_byte + (slot0 + split * G + tid) * 8, m_wg, l_wg);  // (tid < 16: hcol == tid)
+    if (counts) word.settle();
     stores_done();
     __syncthreads();
-    if (tid == 0) is_last = count_partial(p.counters + seg, n_act) ? 1 : 0;
+    if (tid == 0) is_last = word.count(n_act) ? 1 : 0;
     __syncthreads();
     if (!is_last) return;
 
@@ -891,32 +924,6 @@ hipError_t stream_static_scratch(int slot, float** ptr, size_t* bytes) {
     return hipSuccess;
 }
 
-// One counter per (sequence, kv head) and stream slot, for the launches that fold their own partials: zero when the code
-// object is loaded, and back to zero at the end of every launch.
-static __device__ uint32_t decode_counter_block[(size_t)kStreamSlots * kDecodeCounters];
-
-namespace {
-void* g_decode_counter_ptr[kMaxDevices] = {};
-}  // namespace
-
-hipError_t decode_counters(int slot, uint32_t** ptr) {
-    if (slot < 0 || slot >= kStreamSlots) return hipErrorInvalidValue;
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-    std::lock_guard<std::mutex> lock(g_scratch_mutex);
-    if (!g_decode_counter_ptr[dev]) {
-        void* addr = nullptr;
-        e = hipGetSymbolAddress(&addr, HIP_SYMBOL(decode_counter_block));
-        if (e != hipSuccess) return e;
-        if (!addr) return hipErrorInvalidSymbol;
-        g_decode_counter_ptr[dev] = addr;
-    }
-    *ptr = (uint32_t*)g_decode_counter_ptr[dev] + (size_t)slot * kDecodeCounters;
-    return hipSuccess;
-}
-
 // Where the lines lie, from us per call at 32 / 8 heads of 128 unless said (latency form against split + merge):
 //   contexts up to 1056 whatever the batch, 64 sequences of 128-1024: 29.9 / 32.1, 128 of 62-500: 27.5 / 36.1; and up to
 //   10000 steps in all, 16 of 256-2048: 19.6 / 20.7.  Beyond both the streaming kernel's equal spans win: 20 of 500-4000
@@ -933,10 +940,12 @@ int decode_latency_splits(int batch, int heads, int kv_heads, int dim, int max_s
     if (steps <= 3 * kLatWaves) return 1;
     long long n = std::min<long long>((steps + kLatWaves - 1) / kLatWaves, kLatMaxSplits);
     n = std::min<long long>(n, n_cus / segs);
-    // what the room for partials allows in every entry (the caller's workspace and the library's slots alike, so that
-    // all give the same bits)
-    n = std::min<long long>(n, decode_split_parts(batch, max_seq));
-    n = std::min<long long>(n, (long long)(kStreamSlotBytes / ((size_t)batch * heads * ((size_t)dim + 2) * sizeof(float))));
+    // what the room for partials and words allows in every entry (the caller's workspace and the library's blocks alike, so
+    // that all give the same bits)
+    static_assert(kStaticScratchBytes >= kStreamSlotBytes, "room in every entry");
+    const size_t room = std::min(decode_split_workspace_bytes(batch, heads, dim, max_seq), kStreamSlotBytes);
+    const size_t words = (size_t)segs * kWordPitch, one = (size_t)batch * heads * ((size_t)dim + 2) * sizeof(float);
+    n = std::min<long long>(n, room > words ? (long long)((room - words) / one) : 1);
     return (int)std::max<long long>(n, 1);
 }
 

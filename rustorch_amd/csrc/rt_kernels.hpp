@@ -225,11 +225,13 @@ struct DecodeSplitParams {
     // group): along the flat step list every partial advances the wave, the segment or both, so the sum numbers
     // them without collisions, and (n_waves + batch * kv_heads) * group slots hold any batch whatever its lengths.
     int compact;
-    // > 0: the latency form, one launch with that many splits per segment (decode_latency_splits).  `counters`: a zeroed
-    // counter per (sequence, kv head), through which the workgroup that finishes a segment last learns to fold its
-    // partials; `out` 8-byte aligned.  0: the split kernel followed by the merge kernel.
+    // > 0: the latency form, one launch with that many splits per segment (decode_latency_splits), `out` 8-byte aligned.
+    // Above one split, batch * heads * n_splits partials lie at the head of `ws` and behind them a line with a word for each
+    // (sequence, kv head), through which the workgroup that finishes a segment last learns to fold its partials.  Whatever
+    // `ws` held before, the launch sets its words up itself, by `launch_id`: no other launch's, its low 8 bits zero.
+    // 0: the split kernel followed by the merge kernel.
     int n_splits;
-    uint32_t* counters;
+    uint64_t launch_id;
 };
 bool decode_split_supported(int heads, int kv_heads, int dim);
 int decode_split_span_min(int batch);
@@ -247,9 +249,6 @@ hipError_t decode_static_scratch(float** ptr, size_t* bytes);
 constexpr int kStreamSlots = 8;
 constexpr size_t kStreamSlotBytes = (size_t)8 << 20;
 hipError_t stream_static_scratch(int slot, float** ptr, size_t* bytes);
-// The counters that belong to a slot: kDecodeCounters of them, zero outside a launch.
-constexpr int kDecodeCounters = 16384;
-hipError_t decode_counters(int slot, uint32_t** ptr);
 // Splits per (sequence, kv head) of the latency form, or 0 where the step list is long enough for the streaming one;
 // `max_len`: the longest context there can be.
 int decode_latency_splits(int batch, int heads, int kv_heads, int dim, int max_seq, int max_len, int n_cus);

@@ -1,0 +1,163 @@
+// Tests of the library's host code (csrc/api.hip) without a GPU: its object, a HIP runtime that only keeps books
+// (fake_hip.hpp), and launchers that remember what they were given.
+//   api_host_test NAME   runs one test, "ok" at its end
+#include "fake_hip.hpp"
+
+#include <atomic>
+#include <cstdint>
+#include <cstdio>
+#include <functional>
+
+#include "../../include/rt_attn.h"
+#include "../../rustorch_amd/csrc/rt_kernels.hpp"
+
+static int g_failed = 0;
+#define CHECK(cond)                                                     \
+    do {                                                                \
+        if (!(cond)) {                                                  \
+            std::printf("FAIL %s:%d: %s\n", __FILE__, __LINE__, #cond); \
+            ++g_failed;                                                 \
+        }                                                               \
+    } while (0)
+
+// ---- the launchers ---------------------------------------------------------------------------------------------
+static std::mutex g_mutex;
+static std::vector<rt::DecodeSplitParams> g_decode;
+static std::vector<rt::FlashTileParams> g_tile;
+static int g_rows = 0;
+alignas(256) static unsigned char g_slots[rt::kStreamSlots][4096];
+
+namespace rt {
+hipError_t launch_flash_f32(hipStream_t s, const FlashF32Params& p) {
+    fake::log("flash_f32", s);
+    const size_t n = (size_t)p.batch * p.heads * p.seq * p.dim;
+    for (size_t i = 0; i < n; i++) p.out[i] = p.q[i] + 2.0f * p.k[i] + 4.0f * p.v[i];
+    return hipSuccess;
+}
+hipError_t launch_decode_split(hipStream_t s, const DecodeSplitParams& p) {
+    fake::log("decode", s);
+    std::lock_guard<std::mutex> lock(g_mutex);
+    g_decode.push_back(p);
+    return hipSuccess;
+}
+hipError_t launch_flash_tile_bf16(hipStream_t s, const FlashTileParams& p) {
+    fake::log("tile", s);
+    std::lock_guard<std::mutex> lock(g_mutex);
+    g_tile.push_back(p);
+    return hipSuccess;
+}
+hipError_t launch_attn_rows_bf16(hipStream_t, const AttnRowsParams&) { return g_rows++, hipSuccess; }
+hipError_t launch_attn_rows_f32(hipStream_t, const AttnRowsParams&) { return hipSuccess; }
+size_t flash_bwd_f32_workspace_floats(int, int, int, int) { return 64; }
+hipError_t launch_flash_bwd_f32(hipStream_t, const FlashBwdF32Params&, float*) { return hipSuccess; }
+hipError_t launch_flash_bwd_f32_saved(hipStream_t, const FlashBwdF32Params&, const float*, const float*, float*) { return hipSuccess; }
+float plan_flash_bf16(FlashBf16Params&) { return 0.0f; }
+hipError_t launch_flash_bf16(hipStream_t, const FlashBf16Params&) { return hipSuccess; }
+bool flash_tile_bf16_supported(int dim) { return dim <= 256 && dim % 8 == 0; }
+int flash_tile_bf16_key_tile(int) { return 64; }
+int flash_tile_bf16_workgroups(int) { return 2; }
+bool flash_tile_bf16_addressable(long long, long long) { return true; }
+bool flash_wide_bf16_supported(const FlashTileParams&) { return false; }
+hipError_t launch_flash_wide_bf16(hipStream_t, const FlashTileParams&) { return hipSuccess; }
+hipError_t launch_strict_hidden_v(hipStream_t, const StrictVParams&, bool) { return hipSuccess; }
+bool decode_split_supported(int, int, int) { return true; }
+int decode_split_span_min(int) { return 2; }
+int decode_split_parts(int, int max_seq) { return max_seq / 64 + 1; }
+size_t decode_split_workspace_bytes(int b, int h, int d, int m) { return (size_t)b * h * (d + 2) * 4 * (m / 64 + 1); }
+size_t decode_split_compact_bytes(int, int, int, int, int) { return 1024; }
+hipError_t decode_static_scratch(float** p, size_t* n) { return *p = (float*)g_slots[0], *n = 8 << 20, hipSuccess; }
+hipError_t stream_static_scratch(int slot, float** p, size_t* n) { return *p = (float*)g_slots[slot], *n = kStreamSlotBytes, hipSuccess; }
+int decode_latency_splits(int, int, int, int, int, int max_len, int) { return max_len > 4096 ? 0 : (max_len > 384 ? 8 : 1); }
+hipError_t launch_kv_block_append(hipStream_t, void*, void*, const void*, const void*, size_t, size_t, size_t, size_t, size_t, size_t) { return hipSuccess; }
+hipError_t launch_decode_prepare(hipStream_t, const DecodePrepareParams&) { return hipSuccess; }
+hipError_t launch_kv_append_bf16(hipStream_t, uint16_t*, uint16_t*, const uint16_t*, const uint16_t*, int, int, int, int) { return hipSuccess; }
+}  // namespace rt
+
+alignas(256) static char g_buf[1 << 16];  // an address for whatever is not looked into
+
+static int online(hipStream_t s, int kv_len, void* out = g_buf) {
+    return rt_gqa_decode_online_bf16(s, g_buf, g_buf, g_buf, out, 8, 2, kv_len, 64, 8192, nullptr);
+}
+static int chunk(hipStream_t s) { return rt_gqa_decode_chunk_bf16(s, g_buf, g_buf, g_buf, g_buf, nullptr, 4096, 1, 16, 8, 2, 64, 8192, nullptr); }
+
+// ---- tests -----------------------------------------------------------------------------------------------------
+
+// The launches of a batched call work in the caller's workspace alone, under whatever handle: none shares memory, or the
+// id it goes by, with another.
+static void batched_calls_share_nothing() {
+    const size_t need = rt_gqa_decode_workspace_bytes(2, 8, 2, 64, 1024);
+    std::vector<std::vector<char>> ws(4, std::vector<char>(need + 16));
+    int32_t lens[2] = {1024, 500};
+    auto call = [&](int i, hipStream_t s) {
+        void* w = (void*)(((uintptr_t)ws[(size_t)i].data() + 15) & ~(uintptr_t)15);
+        CHECK(rt_gqa_decode_batched_bf16(s, g_buf, g_buf, g_buf, g_buf, lens, 2, 8, 2, 64, 1024, w, need, nullptr) == RT_OK);
+    };
+    std::thread a(call, 0, hipStreamPerThread), b(call, 1, hipStreamPerThread);
+    a.join();
+    b.join();
+    call(2, nullptr);
+    call(3, nullptr);
+    CHECK(g_decode.size() == 4);
+    for (size_t i = 0; i < g_decode.size(); i++) {
+        CHECK(g_decode[i].n_splits > 1 && (g_decode[i].launch_id & 255) == 0);
+        for (size_t j = 0; j < i; j++) CHECK(g_decode[i].launch_id != g_decode[j].launch_id && g_decode[i].ws != g_decode[j].ws);
+    }
+    hipStream_t s;
+    (void)hipStreamCreate(&s);
+    ((fake::Stream*)s)->capturing = true;  // a replay would bring the same id
+    call(0, s);
+    CHECK(g_decode.back().n_splits == 0);
+}
+
+// hipStreamPerThread is a stream of every thread: what calls on it do in shared scratch has an order.
+static void calls_on_the_per_thread_stream_take_turns() {
+    CHECK(rt_init(0, nullptr) == RT_OK);
+    std::vector<std::thread> threads;
+    for (int i = 0; i < 4; i++)
+        threads.emplace_back([i] {
+            for (int n = 0; n < 50; n++) CHECK((i % 2 ? online(hipStreamPerThread, n % 2 ? 2000 : 8000) : chunk(hipStreamPerThread)) == RT_OK);
+        });
+    for (auto& t : threads) t.join();
+    const auto& ops = fake::state().ops;
+    void* event = nullptr;
+    size_t launches = 0;
+    for (size_t i = 0; i < ops.size(); i++) {
+        if (ops[i].what != "decode" && ops[i].what != "tile") continue;
+        launches++;
+        CHECK(i > 0 && i + 1 < ops.size());
+        const auto &before = ops[i - 1], &after = ops[i + 1];
+        CHECK(before.what == "wait" && before.thread == ops[i].thread && before.stream == ops[i].stream);
+        CHECK(after.what == "record" && after.thread == ops[i].thread && after.stream == ops[i].stream);
+        CHECK(before.event == after.event && (!event || event == before.event));
+        event = before.event;
+    }
+    CHECK(launches == 200);
+    // what needs no scratch waits for nobody, nor does an ordinary stream
+    fake::state().ops.clear();
+    CHECK(online(hipStreamPerThread, 300) == RT_OK);
+    CHECK(online(nullptr, 2000) == RT_OK && chunk(nullptr) == RT_OK);
+    for (auto& o : fake::state().ops) CHECK(o.what == "decode" || o.what == "tile");
+    // under capture there is nothing to wait for: no scratch, and so no splits
+    fake::state().per_thread_capturing = true;
+    CHECK(online(hipStreamPerThread, 8000) == RT_OK && g_decode.back().n_splits == 1);
+    CHECK(online(hipStreamPerThread, 8000, g_buf + 2) == RT_OK && g_rows == 1);
+    CHECK(chunk(hipStreamPerThread) == RT_OK && g_tile.back().n_splits <= 1);
+    fake::state().per_thread_capturing = false;
+    CHECK(rt_shutdown(nullptr) == RT_OK);
+    CHECK(online(hipStreamPerThread, 2000) == RT_OK);
+    CHECK(fake::state().errors == 0);
+}
+
+int main(int argc, char** argv) {
+    const std::map<std::string, std::function<void()>> tests = {
+        {"batched_calls_share_nothing", batched_calls_share_nothing},
+        {"calls_on_the_per_thread_stream_take_turns", calls_on_the_per_thread_stream_take_turns},
+    };
+    if (argc == 2 && tests.count(argv[1])) tests.at(argv[1])();
+    else {
+        for (auto& t : tests) std::printf("%s\n", t.first.c_str());
+        return argc == 1 ? 0 : 2;
+    }
+    if (!g_failed) std::printf("ok\n");
+    return g_failed ? 1 : 0;
+}

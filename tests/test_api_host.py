@@ -1,0 +1,19 @@
+"""The library's host code on the CPU (tests/cpp/api_host_test.cpp): what its entries hand to the launchers, whom they
+share memory with, and what they do when the machine refuses something."""
+import os
+import subprocess
+
+import pytest
+
+CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
+
+
+@pytest.mark.parametrize("name", [
+    "batched_calls_share_nothing",
+    "calls_on_the_per_thread_stream_take_turns",
+])
+def test_host_code(name):
+    subprocess.check_call(["make", "-s", "-C", CPP, "api_host_test"])
+    r = subprocess.run([os.path.join(CPP, "api_host_test"), name], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.strip().endswith("ok")
