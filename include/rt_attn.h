@@ -117,7 +117,7 @@ int rt_flash_forward_f32(const rt_attention_shape *shape, const float *q, size_t
  * q, k, v lengths, out length, padding length; seq == 0 returns RT_OK without touching `out`.
  * A row with no visible key is NaN (cpu_forward.rs:411-420); with RT_MASK_PADDING, when none of
  * keep[0 .. min(bc, seq)) is set every row is NaN, as the reference's tiled recurrence gives.
- * dim <= 256 (RT_ERR_UNSUPPORTED beyond). */
+ * dim <= 512 (RT_ERR_UNSUPPORTED beyond). */
 int rt_flash_forward_masked_f32(const rt_attention_shape *shape, const float *q, size_t q_len, const float *k,
                                 size_t k_len, const float *v, size_t v_len, int mask_kind, const uint8_t *keep,
                                 size_t keep_len, float *out, size_t out_len, rt_err_detail *err);
@@ -148,7 +148,7 @@ int rt_mha_flash_forward_f32(const float *q, size_t q_len, const float *k, size_
  * unmasked attention from q, k, v and the upstream gradient d_out, all [batch,heads,seq,dim] host slices.
  * Check order: q, k, v, d_out lengths (RT_ERR_BUFFER_SHAPE_MISMATCH, which = q/k/v/do), then the three outputs
  * (RT_ERR_OUTPUT_SHAPE_MISMATCH, got = the longest of them); seq == 0 returns RT_OK without touching the outputs.
- * The outputs are overwritten, not accumulated into.  dim <= 128. */
+ * The outputs are overwritten, not accumulated into.  dim <= 512 (tuned up to 128). */
 int rt_flash_backward_f32(const rt_attention_shape *shape, const float *q, size_t q_len, const float *k,
                           size_t k_len, const float *v, size_t v_len, const float *d_out, size_t d_out_len, float *dq,
                           size_t dq_len, float *dk, size_t dk_len, float *dv, size_t dv_len, rt_err_detail *err);
@@ -168,7 +168,7 @@ int rt_flash_backward_f32_dev(void *stream, const rt_attention_shape *shape, con
  * gradient dO)"; the reference's CPU function recomputes instead).  rt_flash_forward_stats_f32_dev is the unmasked
  * forward that also writes the row statistic lse[b,h,i] = m_i + ln(l_i) ([batch,heads,seq] f32);
  * rt_flash_backward_saved_f32_dev takes that `out` and `lse` back and skips the recomputation.  `workspace`:
- * batch*heads*seq floats (RT_ERR_WORKSPACE_TOO_SMALL otherwise).  dim <= 128 for the backward. */
+ * batch*heads*seq floats (RT_ERR_WORKSPACE_TOO_SMALL otherwise).  dim <= 512 (tuned up to 128). */
 int rt_flash_forward_stats_f32_dev(void *stream, const rt_attention_shape *shape, const float *q, const float *k,
                                    const float *v, float *out, float *lse, rt_err_detail *err);
 int rt_flash_backward_saved_f32_dev(void *stream, const rt_attention_shape *shape, const float *q, const float *k,
@@ -332,9 +332,15 @@ int rt_qk_norm_rope_kv_append_bf16(void *stream, void *q, const void *k_in, cons
  * a batch of one (head_dim 64, 128 or 256, at most 16 query heads per kv head; other shapes take a one-workgroup-per-head
  * kernel).  The reference's signature has no workspace and its launcher allocates nothing (llm_kernels.rs:915-958):
  * the partials go to a slot of a fixed 64 MiB block of device memory inside the library (8 slots of 8 MiB; a
- * (device, stream) pair takes a free slot on its first call and keeps it until rt_stream_destroy / rt_shutdown, so
- * calls on different streams never share scratch), and the call allocates nothing: it may be the first call on a
- * stream and may be recorded into a HIP graph.  Only a ninth concurrent stream, or a shape whose partials do not fit a
+ * (device, stream) pair takes a free slot on its first call that leaves partials and keeps it until rt_stream_destroy /
+ * rt_shutdown, so calls on different streams never share scratch), and the call allocates nothing: it may be the first
+ * call on a stream and may be recorded into a HIP graph.  A stream is known by its handle: one that was used here is
+ * destroyed through rt_stream_destroy, or idle when its owner destroys it, so that the handle's next stream does not
+ * meet its work.  hipStreamPerThread, one handle for a stream of every thread, has one slot, and calls on it wait on the
+ * GPU for each other (recorded into a graph, they run without partials: longer on a long context).  A graph keeps the
+ * slot of the stream it was recorded on: it is replayed on that stream, or while nothing else uses the slot.  A recorded
+ * call folds its partials in a launch of its own, and its results may differ from an eager call's in the last bit of the
+ * accumulation's order (the bounds are the same).  Only a ninth concurrent stream, or a shape whose partials do not fit a
  * slot (more than ~500 kv heads at 16 query heads each and head_dim 256), falls back to a buffer the library allocates
  * per (device, stream) on that stream's first call (then not under capture; a grown buffer replaces the old one,
  * which is kept until rt_stream_destroy / rt_shutdown).  q and the caches should be
@@ -354,9 +360,11 @@ int rt_gqa_decode_naive_bf16(void *stream, const void *q, const void *k_cache, c
 
 /* The batched, ragged form of the same call: q/out [batch,n_heads,head_dim], caches
  * [batch,n_kv,max_seq,head_dim], kv_lens device int32[batch] (sequence b reads [..kv_lens[b]]).
- * Split-K over the context with a second-pass (m, l, o) merge; `workspace` (device, at least
- * rt_gqa_decode_workspace_bytes(...) bytes, 16-byte aligned or the call fails with RT_ERR_WORKSPACE_TOO_SMALL)
- * holds the partial results.  q and the caches should be 16-byte aligned too (tensors that are not take the
+ * Split-K over the context with an (m, l, o) merge, in one launch where latency counts (short contexts, small batches)
+ * and by a second kernel elsewhere and under capture; `workspace` (device, at least rt_gqa_decode_workspace_bytes(...)
+ * bytes, 16-byte aligned or the call fails with RT_ERR_WORKSPACE_TOO_SMALL) holds the partial results.  The call works in
+ * it alone, whatever it held before, and keeps nothing from one call for the next: calls with workspaces of their own may
+ * overlap on any streams.  q and the caches should be 16-byte aligned too (tensors that are not take the
  * one-workgroup-per-head kernel: same results, slower, no workspace).  The split-K kernels cover
  * head_dim 64, 128 and 256 with at most 16 query heads per kv head; other shapes take a one-workgroup-per-head kernel
  * (head_dim <= 512) that needs no workspace (rt_gqa_decode_workspace_bytes returns 0 for them).
@@ -389,7 +397,8 @@ int rt_gqa_decode_chunk_bf16(void *stream, const void *q, const void *k_cache, c
 
 /* No counterpart in the reference.  rt_gqa_decode_batched_bf16 for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): same arguments without
- * the workspace, same kernels, same results bit for bit.  The split-K partials go to a fixed 8 MiB block of device
+ * the workspace, same kernels, same results bit for bit (an eager call's those of an eager call, a recorded call's those
+ * of a recorded one: see rt_gqa_decode_online_bf16).  The split-K partials go to a fixed 8 MiB block of device
  * memory inside the library (one per GPU, there from the moment the library's code is loaded on that GPU until the
  * process ends); the call allocates and frees nothing.  rt_init(device) looks the block's address up; without it
  * the first call on a device does.
