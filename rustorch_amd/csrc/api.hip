@@ -9,6 +9,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
@@ -539,26 +540,32 @@ struct StagePool {
     std::mutex mutex;
     char* in = nullptr;
     char* out = nullptr;
-    hipEvent_t landed[kStageSlots] = {};
+    // "the chunk in this slot has landed", by device: an event is recorded in streams of its own device only
+    std::map<int, std::array<hipEvent_t, kStageSlots>> landed;
     void* block = nullptr;
     size_t block_bytes = 0;
     int block_dev = -1;
 
-    bool ready() {  // false: no pinned memory to be had
-        if (in) return true;
-        bool ok = hipHostMalloc((void**)&in, kStageInBytes, hipHostMallocDefault) == hipSuccess &&
-                  hipHostMalloc((void**)&out, kStageOutBytes, hipHostMallocDefault) == hipSuccess;
-        for (auto& e : landed) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    bool ready(int dev) {  // false: no pinned memory, or no events, to be had
+        bool ok = true;
+        if (!in)
+            ok = hipHostMalloc((void**)&in, kStageInBytes, hipHostMallocPortable) == hipSuccess &&
+                 hipHostMalloc((void**)&out, kStageOutBytes, hipHostMallocPortable) == hipSuccess;
+        if (ok && !landed.count(dev)) {
+            auto& events = landed[dev];
+            events.fill(nullptr);
+            for (auto& e : events) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+        }
         if (!ok) release();
         return ok;
     }
     void release() {
         if (in) (void)hipHostFree(in);
         if (out) (void)hipHostFree(out);
-        for (auto& e : landed) {
-            if (e) (void)hipEventDestroy(e);
-            e = nullptr;
-        }
+        for (auto& events : landed)
+            for (auto& e : events.second)
+                if (e) (void)hipEventDestroy(e);
+        landed.clear();
         if (block) (void)hipFree(block);
         in = out = nullptr;
         block = nullptr;
@@ -590,7 +597,8 @@ public:
     // Hands out the device pointers and enqueues the uploads (register inputs, then outputs, then scratch).
     int commit(rt_err_detail* err) {
         lock_ = std::unique_lock<std::mutex>(g_stage.mutex, std::try_to_lock);
-        if (lock_.owns_lock() && !g_stage.ready()) lock_.unlock();
+        HIP_TRY(hipGetDevice(&dev_), "hipGetDevice");
+        if (lock_.owns_lock() && !g_stage.ready(dev_)) lock_.unlock();
         size_t in_bytes = 0, out_bytes = 0, total = 0;
         for (auto& it : items_) {
             if (it.kind == kIn) in_bytes += padded(it.bytes);
@@ -660,15 +668,16 @@ public:
                         from.push_back((const char*)*it.dev + done);
                     }
             const size_t n = pieces.size();
+            auto& landed = g_stage.landed[dev_];
             std::unique_ptr<Running> run;
             if (crewed_) run.reset(new Running(pieces));
             for (size_t sent = 0, got = 0; got < n; got++) {
                 for (; sent < n && sent < got + kStageSlots; sent++) {
                     if (run && sent >= kStageSlots) run->job->wait(sent - kStageSlots);
                     HIP_TRY(stage_copy((void*)pieces[sent].src, from[sent], pieces[sent].bytes), "download");
-                    HIP_TRY(hipEventRecord(g_stage.landed[sent % kStageSlots], nullptr), "hipEventRecord");
+                    HIP_TRY(hipEventRecord(landed[sent % kStageSlots], nullptr), "hipEventRecord");
                 }
-                HIP_TRY(hipEventSynchronize(g_stage.landed[got % kStageSlots]), "hipEventSynchronize");
+                HIP_TRY(hipEventSynchronize(landed[got % kStageSlots]), "hipEventSynchronize");
                 if (run) run->job->ready.store(got + 1, std::memory_order_release);
                 else memcpy(pieces[got].dst, pieces[got].src, pieces[got].bytes);
             }
@@ -734,17 +743,15 @@ private:
     }
 
     int get_block(size_t bytes, rt_err_detail* err) {
-        int dev = 0;
-        HIP_TRY(hipGetDevice(&dev), "hipGetDevice");
         if (lock_.owns_lock() && bytes <= kStageKeepBytes) {
-            if (g_stage.block_bytes < bytes || g_stage.block_dev != dev) {
+            if (g_stage.block_bytes < bytes || g_stage.block_dev != dev_) {
                 if (g_stage.block) (void)hipFree(g_stage.block);
                 g_stage.block = nullptr;
                 g_stage.block_bytes = 0;
                 const size_t want = std::min(kStageKeepBytes, std::max(bytes + bytes / 2, (size_t)1 << 20));
                 HIP_TRY(hipMalloc(&g_stage.block, want), "hipMalloc staging block");
                 g_stage.block_bytes = want;
-                g_stage.block_dev = dev;
+                g_stage.block_dev = dev_;
             }
             block_ = (char*)g_stage.block;
         } else {
@@ -755,6 +762,7 @@ private:
     }
 
     std::vector<Item> items_;
+    int dev_ = 0;
     char* block_ = nullptr;
     void* own_block_ = nullptr;  // freed with the call; null where the pool's block serves it
     bool direct_ = true;         // results go to pinned memory straight from the kernels

@@ -148,10 +148,36 @@ static void calls_on_the_per_thread_stream_take_turns() {
     CHECK(fake::state().errors == 0);
 }
 
+// A host-slice call whose results come by chunks, checked.
+static int host_call(uint64_t seq, uint64_t heads = 4) {
+    rt_attention_shape shape = {1, heads, seq, 64, 64, 64};
+    const size_t n = heads * seq * 64;
+    std::vector<float> q(n), k(n), v(n), out(n, -1.0f);
+    for (size_t i = 0; i < n; i++) q[i] = (float)(i % 1000), k[i] = (float)(i % 777), v[i] = (float)(i % 501);
+    const int rc = rt_flash_forward_f32(&shape, q.data(), n, k.data(), n, v.data(), n, out.data(), n, nullptr);
+    size_t wrong = 0;
+    for (size_t i = 0; i < n; i++) wrong += out[i] != q[i] + 2.0f * k[i] + 4.0f * v[i];
+    CHECK(rc != RT_OK || wrong == 0);
+    return rc;
+}
+
+static void host_slices_follow_the_current_device() {
+    for (int dev : {0, 1, 0, 1}) {
+        (void)hipSetDevice(dev);
+        CHECK(host_call(1024) == RT_OK);   // kept block
+        CHECK(host_call(20000) == RT_OK);  // ring more than once, block of its own, copies shared with the helpers
+    }
+    CHECK(rt_shutdown(nullptr) == RT_OK);
+    CHECK(fake::state().memory.empty());
+    CHECK(host_call(1024) == RT_OK);
+    CHECK(fake::state().errors == 0);
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> tests = {
         {"batched_calls_share_nothing", batched_calls_share_nothing},
         {"calls_on_the_per_thread_stream_take_turns", calls_on_the_per_thread_stream_take_turns},
+        {"host_slices_follow_the_current_device", host_slices_follow_the_current_device},
     };
     if (argc == 2 && tests.count(argv[1])) tests.at(argv[1])();
     else {

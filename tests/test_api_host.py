@@ -11,6 +11,7 @@ CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
 @pytest.mark.parametrize("name", [
     "batched_calls_share_nothing",
     "calls_on_the_per_thread_stream_take_turns",
+    "host_slices_follow_the_current_device",
 ])
 def test_host_code(name):
     subprocess.check_call(["make", "-s", "-C", CPP, "api_host_test"])
