@@ -145,7 +145,7 @@ class _Native:
     def __getattr__(self, name):
         lib()
         if not os.path.exists(NATIVE_PATH):
-            raise LibraryMissing(f"{NATIVE_PATH} is missing: build it with `make -C rustorch_amd/csrc`.")
+            raise LibraryMissing(f"{NATIVE_PATH} is missing: build it with `make -C rustorch_amd/csrc native`.")
         loader = importlib.machinery.ExtensionFileLoader("_rt_native", NATIVE_PATH)
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_rt_native", loader))
         loader.exec_module(module)
