@@ -13,6 +13,7 @@
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
+#include <exception>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -62,6 +63,12 @@ int fail_hip(rt_err_detail* e, hipError_t code, const char* where) {
         hipError_t _e = (expr);                               \
         if (_e != hipSuccess) return fail_hip(err, _e, where); \
     } while (0)
+
+// Behind the body of an entry that may allocate on the host: no exception passes a C entry.
+#define RT_NO_THROW                                               \
+    catch (const std::exception& e) {                             \
+        return fail_hip(err, hipErrorOutOfMemory, e.what());      \
+    }
 
 int g_num_cus = 0;
 int g_decode_waves = 0;  // one-wave workgroups one launch of the decode kernel keeps resident
@@ -267,6 +274,7 @@ int stream_workspace(hipStream_t stream, size_t bytes, float** out, rt_err_detai
     if (w.bytes < bytes) {
         // grow geometrically, so that a context that lengthens token by token retires a handful of blocks at most
         size_t want = std::max<size_t>(std::max<size_t>(bytes, (size_t)1 << 20), 2 * w.bytes);
+        w.retired.reserve(w.retired.size() + 1);
         void* fresh = nullptr;
         // (another thread may be capturing its own stream, which an allocation would end with an error)
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
@@ -484,7 +492,10 @@ public:
         {
             std::lock_guard<std::mutex> lock(mutex_);
             job_ = job;
-            while (threads_.size() < kHelpers) threads_.emplace_back([this] { help(); });
+            try {
+                while (threads_.size() < kHelpers) threads_.emplace_back([this] { help(); });
+            } catch (const std::exception&) {  // no thread to be had: the caller copies by itself
+            }
         }
         wake_.notify_all();
     }
@@ -827,7 +838,7 @@ static bool whole_lines_f32(uint64_t dim) { return dim % 4 == 0 && dim <= 128; }
 RT_API int rt_flash_forward_masked_f32(const rt_attention_shape* shape, const float* q, size_t q_len, const float* k,
                                        size_t k_len, const float* v, size_t v_len, int mask_kind,
                                        const uint8_t* keep, size_t keep_len, float* out, size_t out_len,
-                                       rt_err_detail* err) {
+                                       rt_err_detail* err) try {
     clear_err(err);
     if (!shape) return fail(err, RT_ERR_NULL_POINTER, -1, 0, 0, "shape is NULL");
     int rc = validate_flash(shape, q_len, k_len, v_len, out_len, mask_kind, keep_len, err);
@@ -857,7 +868,7 @@ RT_API int rt_flash_forward_masked_f32(const rt_attention_shape* shape, const fl
                           (const uint8_t*)dkeep, (float*)dout, err);
     if (rc) return rc;
     return st.fetch(err);
-}
+} RT_NO_THROW
 
 RT_API int rt_flash_forward_f32(const rt_attention_shape* shape, const float* q, size_t q_len, const float* k,
                                 size_t k_len, const float* v, size_t v_len, float* out, size_t out_len,
@@ -910,7 +921,7 @@ int gqa_device(hipStream_t stream, const float* q, const float* k, const float* 
 
 RT_API int rt_gqa_forward_f32(const float* q, size_t q_len, const float* k, size_t k_len, const float* v,
                               size_t v_len, float* out, size_t out_len, size_t batch, size_t n_heads,
-                              size_t n_kv_heads, size_t seq_q, size_t seq_kv, size_t head_dim, rt_err_detail* err) {
+                              size_t n_kv_heads, size_t seq_q, size_t seq_kv, size_t head_dim, rt_err_detail* err) try {
     clear_err(err);
     // gqa.rs:106-141
     if (n_kv_heads == 0 || n_heads % n_kv_heads != 0)
@@ -944,7 +955,7 @@ RT_API int rt_gqa_forward_f32(const float* q, size_t q_len, const float* k, size
                     n_kv_heads, seq_q, seq_kv, head_dim, err);
     if (rc) return rc;
     return st.fetch(err);
-}
+} RT_NO_THROW
 
 RT_API int rt_gqa_forward_f32_dev(void* stream, const float* q, const float* k, const float* v, float* out, size_t batch,
                                   size_t n_heads, size_t n_kv_heads, size_t seq_q, size_t seq_kv, size_t head_dim,
@@ -1016,7 +1027,7 @@ RT_API size_t rt_flash_backward_workspace_bytes(const rt_attention_shape* shape)
 RT_API int rt_flash_backward_f32(const rt_attention_shape* shape, const float* q, size_t q_len, const float* k,
                                  size_t k_len, const float* v, size_t v_len, const float* d_out, size_t d_out_len,
                                  float* dq, size_t dq_len, float* dk, size_t dk_len, float* dv, size_t dv_len,
-                                 rt_err_detail* err) {
+                                 rt_err_detail* err) try {
     clear_err(err);
     if (!shape) return fail(err, RT_ERR_NULL_POINTER, -1, 0, 0, "shape is NULL");
     // cpu_backward.rs:59-74: no ZeroDim check here, unlike the forward
@@ -1057,7 +1068,7 @@ RT_API int rt_flash_backward_f32(const rt_attention_shape* shape, const float* q
                           (const float*)in[3].p, (float*)out[0].p, (float*)out[1].p, (float*)out[2].p, (float*)ws.p, err);
     if (rc) return rc;
     return st.fetch(err);
-}
+} RT_NO_THROW
 
 RT_API int rt_flash_backward_f32_dev(void* stream, const rt_attention_shape* shape, const float* q, const float* k,
                                      const float* v, const float* d_out, float* dq, float* dk, float* dv,
@@ -1350,7 +1361,7 @@ RT_API int rt_flash_forward_bnhd_f32_dev(void* stream, const rt_attention_shape*
 
 RT_API int rt_mha_flash_forward_f32(const float* q, size_t q_len, const float* k, size_t k_len, const float* v,
                                     size_t v_len, float* out, size_t out_len, size_t batch, size_t seq, size_t heads,
-                                    size_t head_dim, rt_err_detail* err) {
+                                    size_t head_dim, rt_err_detail* err) try {
     clear_err(err);
     // the reference transposes to [B,H,T,hd] and calls flash_forward (attention.rs:474-483): same checks, same order
     rt_attention_shape shape = {batch, heads, seq, head_dim, 64, 64};
@@ -1375,7 +1386,7 @@ RT_API int rt_mha_flash_forward_f32(const float* q, size_t q_len, const float* k
                           RT_MASK_NONE, nullptr, (float*)dout.p, err, true);
     if (rc) return rc;
     return st.fetch(err);
-}
+} RT_NO_THROW
 
 namespace {
 
@@ -1425,7 +1436,7 @@ int mha_masked_device(hipStream_t stream, const float* q, const float* k, const 
 RT_API int rt_mha_forward_masked_f32(const float* q, size_t q_len, const float* k, size_t k_len, const float* v,
                                      size_t v_len, const float* mask, size_t mask_len, float* out, size_t out_len,
                                      size_t batch, size_t t_q, size_t t_kv, size_t heads, size_t head_dim,
-                                     rt_err_detail* err) {
+                                     rt_err_detail* err) try {
     clear_err(err);
     if (head_dim == 0) return fail(err, RT_ERR_ZERO_DIM, -1, 0, 0, "dim must be > 0");
     const size_t embed = heads * head_dim;
@@ -1459,7 +1470,7 @@ RT_API int rt_mha_forward_masked_f32(const float* q, size_t q_len, const float* 
                            head_dim, err);
     if (rc) return rc;
     return st.fetch(err);
-}
+} RT_NO_THROW
 
 RT_API int rt_mha_forward_masked_f32_dev(void* stream, const float* q, const float* k, const float* v, const float* mask,
                                          size_t mask_len, float* out, size_t batch, size_t t_q, size_t t_kv,
@@ -1753,7 +1764,7 @@ static int online_scratch(hipStream_t stream, rt::DecodeSplitParams& p, rt_err_d
 
 RT_API int rt_gqa_decode_online_bf16(void* stream, const void* q, const void* k_cache, const void* v_cache,
                                      void* out, int32_t n_heads, int32_t n_kv, int32_t kv_len, int32_t head_dim,
-                                     int32_t max_seq, rt_err_detail* err) {
+                                     int32_t max_seq, rt_err_detail* err) try {
     clear_err(err);
     int rc = check_decode_dims(1, n_heads, n_kv, head_dim, max_seq, err);
     if (rc) return rc;
@@ -1828,7 +1839,7 @@ RT_API int rt_gqa_decode_online_bf16(void* stream, const void* q, const void* k_
     p.scale = 1.0f / sqrtf((float)head_dim);
     HIP_TRY(rt::launch_attn_rows_bf16((hipStream_t)stream, p), "attn_rows_bf16 launch");
     return RT_OK;
-}
+} RT_NO_THROW
 
 RT_API int rt_gqa_decode_naive_bf16(void* stream, const void* q, const void* k_cache, const void* v_cache, void* out,
                                     int32_t n_heads, int32_t n_kv, int32_t kv_len, int32_t head_dim, int32_t max_seq,
@@ -1871,7 +1882,7 @@ long long chunk_splits(long long slabs, long long rows, int head_dim, long long 
 RT_API int rt_gqa_decode_chunk_bf16(void* stream, const void* q, const void* k_cache, const void* v_cache, void* out,
                                     const int32_t* kv_lens, int32_t kv_len, int32_t batch, int32_t seq_new,
                                     int32_t n_heads, int32_t n_kv, int32_t head_dim, int32_t max_seq,
-                                    rt_err_detail* err) {
+                                    rt_err_detail* err) try {
     clear_err(err);
     int rc = check_decode_dims(batch, n_heads, n_kv, head_dim, max_seq, err);
     if (rc) return rc;
@@ -1956,7 +1967,7 @@ RT_API int rt_gqa_decode_chunk_bf16(void* stream, const void* q, const void* k_c
     }
     HIP_TRY(rt::launch_flash_tile_bf16((hipStream_t)stream, t), "flash_tile_bf16 launch");
     return turn.leave((hipStream_t)stream, err);
-}
+} RT_NO_THROW
 
 RT_API size_t rt_gqa_decode_workspace_bytes(int32_t batch, int32_t n_heads, int32_t n_kv, int32_t head_dim,
                                             int32_t max_seq) {

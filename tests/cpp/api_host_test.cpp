@@ -36,12 +36,14 @@ hipError_t launch_flash_f32(hipStream_t s, const FlashF32Params& p) {
 }
 hipError_t launch_decode_split(hipStream_t s, const DecodeSplitParams& p) {
     fake::log("decode", s);
+    fake::Inside here;
     std::lock_guard<std::mutex> lock(g_mutex);
     g_decode.push_back(p);
     return hipSuccess;
 }
 hipError_t launch_flash_tile_bf16(hipStream_t s, const FlashTileParams& p) {
     fake::log("tile", s);
+    fake::Inside here;
     std::lock_guard<std::mutex> lock(g_mutex);
     g_tile.push_back(p);
     return hipSuccess;
@@ -72,6 +74,24 @@ hipError_t launch_kv_block_append(hipStream_t, void*, void*, const void*, const 
 hipError_t launch_decode_prepare(hipStream_t, const DecodePrepareParams&) { return hipSuccess; }
 hipError_t launch_kv_append_bf16(hipStream_t, uint16_t*, uint16_t*, const uint16_t*, const uint16_t*, int, int, int, int) { return hipSuccess; }
 }  // namespace rt
+
+// ---- a machine that refuses -------------------------------------------------------------------------------------
+static std::atomic<long> g_news_left{-1};  // this many allocations of the host are granted to the calling thread; -1: all
+static thread_local bool g_counted = false;
+void* operator new(size_t n) {
+    if (g_counted && !fake::inside && g_news_left.load() >= 0 && g_news_left.fetch_sub(1) == 0) throw std::bad_alloc();
+    return malloc(n ? n : 1);
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
+
+static std::atomic<bool> g_refuse_threads{false};
+#include <dlfcn.h>
+extern "C" int pthread_create(pthread_t* t, const pthread_attr_t* a, void* (*f)(void*), void* arg) noexcept {
+    if (g_refuse_threads) return EAGAIN;
+    static auto real = (int (*)(pthread_t*, const pthread_attr_t*, void* (*)(void*), void*))dlsym(RTLD_NEXT, "pthread_create");
+    return real(t, a, f, arg);
+}
 
 alignas(256) static char g_buf[1 << 16];  // an address for whatever is not looked into
 
@@ -173,11 +193,63 @@ static void host_slices_follow_the_current_device() {
     CHECK(fake::state().errors == 0);
 }
 
+static void a_host_without_threads_copies_by_itself() {
+    g_refuse_threads = true;
+    CHECK(host_call(20000) == RT_OK);
+    g_refuse_threads = false;
+    CHECK(host_call(20000) == RT_OK);
+}
+
+// Whichever allocation fails: the entry returns an error, and the next call is as if nothing had been.
+static void a_host_without_memory_is_an_error() {
+    static float q[3 * 5 * 64], out[3 * 5 * 64];
+    static std::vector<float> big(4 * 20000 * 64, 1.0f), big_out(big.size());
+    rt_attention_shape small_shape = {1, 3, 5, 64, 64, 64}, big_shape = {1, 4, 20000, 64, 64, 64};
+    const size_t n = 3 * 5 * 64;
+    rt_err_detail err;
+    hipStream_t s = nullptr;
+    const std::vector<std::function<int()>> calls = {
+        [&] { return rt_flash_forward_masked_f32(&small_shape, q, n, q, n, q, n, RT_MASK_NONE, nullptr, 0, out, n, &err); },
+        [&] { return rt_flash_forward_masked_f32(&big_shape, big.data(), big.size(), big.data(), big.size(), big.data(), big.size(),
+                                                 RT_MASK_NONE, nullptr, 0, big_out.data(), big.size(), &err); },
+        [&] { return rt_gqa_forward_f32(q, n, q, n, q, n, out, n, 1, 3, 3, 5, 5, 64, &err); },
+        [&] { return rt_flash_backward_f32(&small_shape, q, n, q, n, q, n, q, n, out, n, out, n, out, n, &err); },
+        [&] { return rt_mha_flash_forward_f32(q, n, q, n, q, n, out, n, 1, 5, 3, 64, &err); },
+        [&] { return rt_mha_forward_masked_f32(q, n, q, n, q, n, nullptr, 0, out, n, 1, 5, 5, 3, 64, &err); },
+        [&] { return rt_gqa_decode_online_bf16(s, g_buf, g_buf, g_buf, g_buf, 8, 2, 2000, 64, 8192, &err); },
+        [&] { return rt_gqa_decode_chunk_bf16(s, g_buf, g_buf, g_buf, g_buf, nullptr, 4096, 1, 16, 8, 2, 64, 8192, &err); },
+    };
+    CHECK(rt_init(0, nullptr) == RT_OK);
+    for (size_t i = 0; i < calls.size(); i++) {
+        int failures = 0;
+        for (long k = 0; k < 1000; k++) {
+            (void)rt_shutdown(nullptr);
+            (void)hipStreamCreate(&s);  // (nothing is kept for it yet)
+            g_news_left = k;
+            g_counted = true;
+            const int rc = calls[i]();
+            g_counted = false;
+            const bool all_granted = g_news_left > 0;
+            g_news_left = -1;
+            CHECK(rc == RT_OK || (rc == RT_ERR_HIP && err.hip_error == hipErrorOutOfMemory));
+            CHECK(calls[i]() == RT_OK);
+            failures += rc != RT_OK;
+            if (rc == RT_OK && all_granted) break;
+        }
+        CHECK(failures > 0);
+    }
+    CHECK(host_call(20000) == RT_OK);
+    (void)rt_shutdown(nullptr);
+    CHECK(fake::state().memory.empty());
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> tests = {
         {"batched_calls_share_nothing", batched_calls_share_nothing},
         {"calls_on_the_per_thread_stream_take_turns", calls_on_the_per_thread_stream_take_turns},
         {"host_slices_follow_the_current_device", host_slices_follow_the_current_device},
+        {"a_host_without_threads_copies_by_itself", a_host_without_threads_copies_by_itself},
+        {"a_host_without_memory_is_an_error", a_host_without_memory_is_an_error},
     };
     if (argc == 2 && tests.count(argv[1])) tests.at(argv[1])();
     else {

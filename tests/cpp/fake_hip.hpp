@@ -41,8 +41,14 @@ inline State& state() {
 }
 inline thread_local int current_device = 0;
 inline thread_local dim3 push_grid, push_block;
+inline thread_local int inside = 0;  // the runtime's own allocations are none of the library's
+struct Inside {
+    Inside() { inside++; }
+    ~Inside() { inside--; }
+};
 
 inline void log(const char* what, hipStream_t stream, void* event = nullptr) {
+    Inside here;
     std::lock_guard<std::mutex> lock(state().mutex);
     state().ops.push_back({what, stream, std::this_thread::get_id(), event});
 }
@@ -70,12 +76,14 @@ hipError_t hipGetLastError(void) { return hipSuccess; }
 
 hipError_t hipMalloc(void** p, size_t n) {
     *p = aligned_alloc(256, (n + 255) / 256 * 256);
+    fake::Inside here;
     std::lock_guard<std::mutex> lock(fake::state().mutex);
     fake::state().memory[*p] = fake::current_device;
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
     *p = aligned_alloc(256, (n + 255) / 256 * 256);
+    fake::Inside here;
     std::lock_guard<std::mutex> lock(fake::state().mutex);
     fake::state().memory[*p] = -1;
     return hipSuccess;
@@ -92,7 +100,7 @@ hipError_t hipHostFree(void* p) { return hipFree(p); }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { return memcpy(d, s, n), hipSuccess; }
 
-hipError_t hipStreamCreate(hipStream_t* s) { return *s = (hipStream_t) new fake::Stream{fake::current_device}, hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t* s) { fake::Inside here; return *s = (hipStream_t) new fake::Stream{fake::current_device}, hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { return delete (fake::Stream*)s, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { return fake::log("synchronize", s), hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* c) {
@@ -101,7 +109,7 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* c) {
 }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hipSuccess; }
 
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return *e = (hipEvent_t) new fake::Event{fake::current_device}, hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { fake::Inside here; return *e = (hipEvent_t) new fake::Event{fake::current_device}, hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { return delete (fake::Event*)e, hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     if (((fake::Event*)e)->device != fake::device_of(s)) return fake::refuse(hipErrorInvalidHandle);
@@ -141,6 +149,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* n, hipStream_t* s
     return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void* host, dim3, dim3, void** args, size_t, hipStream_t s) {
+    fake::Inside here;
     const std::string& name = fake::state().kernels[host];
     fake::log("kernel", s);
     if (name.find("stage_copy") != std::string::npos)

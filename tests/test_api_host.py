@@ -12,6 +12,8 @@ CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
     "batched_calls_share_nothing",
     "calls_on_the_per_thread_stream_take_turns",
     "host_slices_follow_the_current_device",
+    "a_host_without_threads_copies_by_itself",
+    "a_host_without_memory_is_an_error",
 ])
 def test_host_code(name):
     subprocess.check_call(["make", "-s", "-C", CPP, "api_host_test"])
