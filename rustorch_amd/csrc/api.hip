@@ -681,7 +681,6 @@ public:
             const size_t n = pieces.size();
             auto& landed = g_stage.landed[dev_];
             std::unique_ptr<Running> run;
-            if (crewed_) run.reset(new Running(pieces));
             for (size_t sent = 0, got = 0; got < n; got++) {
                 for (; sent < n && sent < got + kStageSlots; sent++) {
                     if (run && sent >= kStageSlots) run->job->wait(sent - kStageSlots);
@@ -689,6 +688,8 @@ public:
                     HIP_TRY(hipEventRecord(landed[sent % kStageSlots], nullptr), "hipEventRecord");
                 }
                 HIP_TRY(hipEventSynchronize(landed[got % kStageSlots]), "hipEventSynchronize");
+                // the helpers are called when there is something to copy: until then they would spin through the kernel
+                if (crewed_ && !run) run.reset(new Running(pieces));
                 if (run) run->job->ready.store(got + 1, std::memory_order_release);
                 else memcpy(pieces[got].dst, pieces[got].src, pieces[got].bytes);
             }

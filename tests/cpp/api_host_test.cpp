@@ -6,6 +6,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstdio>
+#include <ctime>
 #include <functional>
 
 #include "../../include/rt_attn.h"
@@ -193,6 +194,23 @@ static void host_slices_follow_the_current_device() {
     CHECK(fake::state().errors == 0);
 }
 
+// A call whose copies are shared waits for its kernel as any other: no core is busy meanwhile.
+static void no_thread_spins_through_the_kernel() {
+    rt_attention_shape shape = {1, 4, 20000, 64, 64, 64};
+    std::vector<float> x(4 * 20000 * 64, 1.0f), out(x.size());
+    auto call = [&] { return rt_flash_forward_f32(&shape, x.data(), x.size(), x.data(), x.size(), x.data(), x.size(), out.data(), x.size(), nullptr); };
+    auto cpu_ms = [&] {
+        const clock_t before = clock();  // of all threads
+        CHECK(call() == RT_OK);
+        return (double)(clock() - before) * 1e3 / CLOCKS_PER_SEC;
+    };
+    (void)cpu_ms();
+    const double idle = cpu_ms();
+    fake::state().busy_ms = 500;
+    CHECK(cpu_ms() < idle + 250.0);
+    CHECK(fake::state().busy_ms == 0);
+}
+
 static void a_host_without_threads_copies_by_itself() {
     g_refuse_threads = true;
     CHECK(host_call(20000) == RT_OK);
@@ -248,6 +266,7 @@ int main(int argc, char** argv) {
         {"batched_calls_share_nothing", batched_calls_share_nothing},
         {"calls_on_the_per_thread_stream_take_turns", calls_on_the_per_thread_stream_take_turns},
         {"host_slices_follow_the_current_device", host_slices_follow_the_current_device},
+        {"no_thread_spins_through_the_kernel", no_thread_spins_through_the_kernel},
         {"a_host_without_threads_copies_by_itself", a_host_without_threads_copies_by_itself},
         {"a_host_without_memory_is_an_error", a_host_without_memory_is_an_error},
     };

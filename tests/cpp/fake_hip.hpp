@@ -4,12 +4,14 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
 #include <thread>
+#include <utility>
 #include <vector>
 
 namespace fake {
@@ -33,6 +35,7 @@ struct State {
     std::map<const void*, std::string> kernels;  // host handle -> device name
     std::map<void*, int> memory;                 // allocation -> device, -1: pinned
     bool per_thread_capturing = false;
+    unsigned busy_ms = 0;  // how long the GPU works before the next event is reached
     int errors = 0;  // calls a real runtime would have refused
 };
 inline State& state() {
@@ -115,7 +118,10 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     if (((fake::Event*)e)->device != fake::device_of(s)) return fake::refuse(hipErrorInvalidHandle);
     return fake::log("record", s, e), hipSuccess;
 }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) {
+    std::this_thread::sleep_for(std::chrono::milliseconds(std::exchange(fake::state().busy_ms, 0u)));
+    return hipSuccess;
+}
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
     hipStreamCaptureStatus c;
     (void)hipStreamIsCapturing(s, &c);
