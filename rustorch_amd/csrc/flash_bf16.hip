@@ -45,7 +45,6 @@
 // needed anyway, bounds every P of the lane.  Only when a share passes 2^16, or is not a number, or the row
 // has no max yet, does the wave compute the item max, rescale O and l and redo P from the scores.
 #include <algorithm>
-#include <vector>
 
 #include "rt_common.hpp"
 #include "rt_kernels.hpp"
@@ -735,7 +734,10 @@ hipError_t launch_hd(hipStream_t stream, const FlashBf16Params& p, dim3 grid, di
 // query tiles leave two long jobs with one worker and two short ones with another, and dealing by rank (every head's
 // longest job first) is then the shorter of the two: 2 sequences of 1501 rows, 32 heads: 58.8 -> 45.5 us, 1 of 3000:
 // 116 -> 79.
+// This runs on every call that the persistent kernel may serve: 0.1 to 0.75 us of the host (loads of runs of equal jobs;
+// job by job with a division each it was up to 12 us, 7 x 12 heads of 8192 rows).
 constexpr float kBoundarySteps = 2.5f;  // what lies between two jobs of a worker
+constexpr int kMostWorkers = 512;       // whose loads are added up one by one
 float plan_flash_bf16(FlashBf16Params& p) {
     const int n_qtiles = (p.seq + BR - 1) / BR, n_bh = p.batch * p.heads;
     const long long n_jobs = (long long)n_qtiles * n_bh;
@@ -749,18 +751,35 @@ float plan_flash_bf16(FlashBf16Params& p) {
     const bool by_xcd = (n_bh & 7) == 0 && (W & 7) == 0;
     const int C = by_xcd ? W >> 3 : W, heads = by_xcd ? n_bh >> 3 : n_bh;
     const long long n = (long long)n_qtiles * heads;
-    if (n > 16ll * C) {  // many jobs a worker: any order is balanced
+    if (n > 16ll * C || C > kMostWorkers) {  // many jobs a worker: any order is balanced
         float total = 0.0f;
         for (int r = 0; r < n_qtiles; r++) total += length(r);
         return total * (float)heads / (float)C;
     }
     auto makespan = [&](bool rank_major) {
-        std::vector<float> load((size_t)C, 0.0f);
-        for (int q = 0; q < (int)n; q++) {
-            const int i = q / C, at = q - i * C;
-            load[(size_t)((i & 1) ? C - 1 - at : at)] += length(rank_major ? q / heads : q % n_qtiles);
+        float load[kMostWorkers];
+        std::fill(load, load + C, 0.0f);
+        // runs of jobs of one rank: `each` of them, the next rank behind them, the first behind the last
+        const int each = rank_major ? heads : 1;
+        int rank = 0, left = each, todo = (int)n;
+        float len = length(0);
+        for (int i = 0; todo > 0; i++) {
+            const int round = std::min(C, todo);
+            for (int at = 0; at < round;) {
+                const int run = std::min(left, round - at);
+                float* to = load + ((i & 1) ? C - at - run : at);
+                for (int x = 0; x < run; x++) to[x] += len;
+                at += run;
+                left -= run;
+                if (left == 0) {
+                    rank = rank + 1 == n_qtiles ? 0 : rank + 1;
+                    left = each;
+                    len = length(rank);
+                }
+            }
+            todo -= round;
         }
-        return *std::max_element(load.begin(), load.end());
+        return *std::max_element(load, load + C);
     };
     if (!by_xcd) return makespan(true);
     const float by_head = makespan(false), by_rank = makespan(true);

@@ -3,6 +3,7 @@
 //   api_host_test NAME   runs one test, "ok" at its end
 #include "fake_hip.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <cstdint>
 #include <cstdio>
@@ -54,8 +55,6 @@ hipError_t launch_attn_rows_f32(hipStream_t, const AttnRowsParams&) { return hip
 size_t flash_bwd_f32_workspace_floats(int, int, int, int) { return 64; }
 hipError_t launch_flash_bwd_f32(hipStream_t, const FlashBwdF32Params&, float*) { return hipSuccess; }
 hipError_t launch_flash_bwd_f32_saved(hipStream_t, const FlashBwdF32Params&, const float*, const float*, float*) { return hipSuccess; }
-float plan_flash_bf16(FlashBf16Params&) { return 0.0f; }
-hipError_t launch_flash_bf16(hipStream_t, const FlashBf16Params&) { return hipSuccess; }
 bool flash_tile_bf16_supported(int dim) { return dim <= 256 && dim % 8 == 0; }
 int flash_tile_bf16_key_tile(int) { return 64; }
 int flash_tile_bf16_workgroups(int) { return 2; }
@@ -77,9 +76,11 @@ hipError_t launch_kv_append_bf16(hipStream_t, uint16_t*, uint16_t*, const uint16
 }  // namespace rt
 
 // ---- a machine that refuses -------------------------------------------------------------------------------------
+static std::atomic<long> g_news{0};
 static std::atomic<long> g_news_left{-1};  // this many allocations of the host are granted to the calling thread; -1: all
 static thread_local bool g_counted = false;
 void* operator new(size_t n) {
+    if (g_counted) g_news++;
     if (g_counted && !fake::inside && g_news_left.load() >= 0 && g_news_left.fetch_sub(1) == 0) throw std::bad_alloc();
     return malloc(n ? n : 1);
 }
@@ -261,11 +262,57 @@ static void a_host_without_memory_is_an_error() {
     CHECK(fake::state().memory.empty());
 }
 
+// The prefill plan is what dealing the jobs one by one gives (jobs of 256 rows, rounds back and forth over the workers of
+// an XCD, or over all), and it costs a call no allocation.
+static void the_prefill_plan_deals_as_the_kernel_does() {
+    auto by_hand = [](const rt::FlashBf16Params& p, bool rank_major, int workers, int heads, int n_qtiles) {
+        std::vector<float> load((size_t)workers, 0.0f);
+        for (int q = 0; q < n_qtiles * heads; q++) {
+            const int round = q / workers, at = q % workers, rank = rank_major ? q / heads : q % n_qtiles;
+            const int keys = p.mask == rt::kMaskCausal ? std::min(p.seq, (n_qtiles - rank) * 256) : p.seq;
+            load[(size_t)(round % 2 ? workers - 1 - at : at)] += (float)((keys + 127) / 128) + 2.5f;
+        }
+        float most = 0.0f;
+        for (float x : load) most = std::max(most, x);
+        return most;
+    };
+    int ranked = 0;
+    for (int cus : {256, 304, 64, 12})
+        for (int batch : {1, 2, 3, 8})
+            for (int heads : {1, 5, 8, 12, 28, 32, 40})
+                for (int seq : {512, 777, 1024, 1501, 2048, 3000, 4096, 9000})
+                    for (int mask : {rt::kMaskNone, rt::kMaskCausal}) {
+                        rt::FlashBf16Params p{};
+                        p.batch = batch;
+                        p.heads = p.kv_heads = heads;
+                        p.group = 1;
+                        p.seq = seq;
+                        p.dim = 128;
+                        p.mask = mask;
+                        p.n_workers = cus;
+                        g_news = 0;
+                        g_counted = true;
+                        const float got = rt::plan_flash_bf16(p);
+                        g_counted = false;
+                        CHECK(g_news == 0);
+                        const int n_qtiles = (seq + 255) / 256, n_bh = batch * heads, w = std::min(cus, n_qtiles * n_bh);
+                        const bool by_xcd = n_bh % 8 == 0 && w % 8 == 0;
+                        const int workers = by_xcd ? w / 8 : w, list = by_xcd ? n_bh / 8 : n_bh;
+                        if (n_qtiles * list > 16 * workers) continue;  // the mean stands for it
+                        const float rank = by_hand(p, true, workers, list, n_qtiles), head = by_hand(p, false, workers, list, n_qtiles);
+                        CHECK(got == (by_xcd ? std::min(rank, head) : rank));
+                        CHECK(p.rank_major == (by_xcd && rank < head));
+                        ranked += p.rank_major;
+                    }
+    CHECK(ranked > 0);
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> tests = {
         {"batched_calls_share_nothing", batched_calls_share_nothing},
         {"calls_on_the_per_thread_stream_take_turns", calls_on_the_per_thread_stream_take_turns},
         {"host_slices_follow_the_current_device", host_slices_follow_the_current_device},
+        {"the_prefill_plan_deals_as_the_kernel_does", the_prefill_plan_deals_as_the_kernel_does},
         {"no_thread_spins_through_the_kernel", no_thread_spins_through_the_kernel},
         {"a_host_without_threads_copies_by_itself", a_host_without_threads_copies_by_itself},
         {"a_host_without_memory_is_an_error", a_host_without_memory_is_an_error},
