@@ -30,15 +30,12 @@ __device__ __forceinline__ void zero16(f32x16_t& x) {
     for (int i = 0; i < 16; i++) x[i] = 0.0f;
 }
 
-// what the split does not carry raises the sum to kSplitMost (rt_split.hpp)
+// what the split does not carry raises the largest magnitude to kSplitMost (rt_split.hpp)
 __device__ __forceinline__ void check8(const float (&x)[8], float& chk) {
     float m = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        chk = __builtin_fmaf(x[i], x[i], chk);
-        m = __builtin_fmaxf(m, __builtin_fabsf(x[i]));
-    }
-    chk = split_too_small(m) ? kSplitMost : chk;
+    for (int i = 0; i < 8; i++) m = split_max(m, x[i]);
+    chk = split_too_small(m) ? kSplitMost : __builtin_fmaxf(chk, m);
 }
 
 // One streamed matrix [N, D]: a tile's rows and columns on their way from memory into LDS.  Rows behind the last repeat it;
@@ -92,10 +89,8 @@ struct Stream {
         if (!kCol && n == 2) {  // the columns hold the same values
             const float x0 = r[e >> 1][2 * (e & 1)], x1 = r[e >> 1][2 * (e & 1) + 1];
             if (e == 0) m = 0.0f;
-            chk = __builtin_fmaf(x0, x0, chk);
-            chk = __builtin_fmaf(x1, x1, chk);
-            m = __builtin_fmaxf(__builtin_fmaxf(m, __builtin_fabsf(x0)), __builtin_fabsf(x1));
-            if (e == 3) chk = split_too_small(m) ? kSplitMost : chk;
+            m = split_max(split_max(m, x0), x1);
+            if (e == 3) chk = split_too_small(m) ? kSplitMost : __builtin_fmaxf(chk, m);
         }
         if (x == 11 && (ITEMS % 256 == 0 || tid < ITEMS)) {
             __bf16* at = kCol ? buf + COLS + (tid % DPAD) * LDV + 8 * (tid / DPAD)
@@ -215,7 +210,7 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
         if (tid < 64) {
             const int row = row0 + (tid & 31);
             st = row < N ? (tid < 32 ? lse : delta)[row] : 0.0f;
-            chk = __builtin_fmaf(st, st, chk);
+            chk = split_max(chk, st);
             if (row >= N && tid < 32) st = -neg_inf();
         }
     };
@@ -233,12 +228,12 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
     const int n_tiles = (N + kTile - 1) / kTile;
     load(0);
     store(0);
+    const bool uncarried = __syncthreads_or(!(chk < kSplitMost));  // seen already: no step of the loop below
     if (n_tiles > 1) load(kTile);
-    __syncthreads();
     // In a step the next tile (in registers since the step before) is split between the instructions of the score-shaped
     // products, and the second half of the weights is formed between those of the first half's gradient products: with one
     // wave a SIMD nothing else would keep both units busy.  The scheduling barriers keep that order.
-    for (int tile = 0; tile < n_tiles; tile++) {
+    for (int tile = 0; tile < (uncarried ? 0 : n_tiles); tile++) {
         const __bf16* qb = lds + (tile & 1) * BUF;
         const __bf16* ob = qb + St::SIZE;
         __bf16* nb = lds + ((tile + 1) & 1) * BUF;  // behind the last tile: a repeat that nobody reads
@@ -351,51 +346,60 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
         acc_dv[t] += low_dv[t];
         acc_dk[t] += low_dk[t];
     }
-    if (__syncthreads_or(!(chk < kSplitMost))) {
-        // something here the split does not carry: the wave's rows once more in f32, straight from memory
+    if (uncarried || __syncthreads_or(!(chk < kSplitMost))) {
+        // something here the split does not carry: the rows once more in f32, the tiles through LDS two at a time.  For a
+        // launch of both kernels (B=4 H=16 N=1024 D=64) 551 us where the first tiles show it, 684 where only the last does;
+        // straight from memory 2880; the f32 kernels alone 506.
+        using Tile = F32Tile<DT>;
+        static_assert(4 * Tile::SIZE * sizeof(float) <= sizeof(lds), "two tiles of Q and dO");
+        float* const f32_lds = (float*)lds;
 #pragma unroll
         for (int t = 0; t < DT; t++) {
             zero16(acc_dv[t]);
             zero16(acc_dk[t]);
         }
+        float k[16 * DT], v[16 * DT];
+        f32_row<DT>(k, Kg + (size_t)key * D, key < N, D, hh);
+        f32_row<DT>(v, Vg + (size_t)key * D, key < N, D, hh);
+        Tile qt, ot;
+        float st_f = 0.0f;
+        auto load_f = [&](int q0) {
+            qt.load(Qg, (size_t)D, q0, N, D, tid);
+            ot.load(dOg, (size_t)D, q0, N, D, tid);
+            if (tid < 64) {
+                const int row = q0 + (tid & 31);
+                st_f = row < N ? (tid < 32 ? lse : delta)[row] : (tid < 32 ? -neg_inf() : 0.0f);
+            }
+        };
+        auto store_f = [&](int b2) {
+            qt.store(f32_lds + b2 * 2 * Tile::SIZE, tid);
+            ot.store(f32_lds + b2 * 2 * Tile::SIZE + Tile::SIZE, tid);
+            if (tid < 64) stat[b2][tid >> 5][tid & 31] = st_f;
+        };
+        load_f(0);
+        store_f(0);
+        __syncthreads();
         for (int tile = 0; tile < n_tiles; tile++) {
-            const int q0 = tile * kTile;
+            const float* qb = f32_lds + (tile & 1) * 2 * Tile::SIZE;
+            const float* ob = qb + Tile::SIZE;
+            if (tile + 1 < n_tiles) load_f((tile + 1) * kTile);
             f32x16_t s, dp;
             zero16(s);
             zero16(dp);
-            for (int ks = 0; ks < DPAD / 2; ks++) {
-                const int d = 8 * (ks >> 2) + 4 * hh + (ks & 3);  // the f32 kernels' order
-                const bool qok = q0 + col < N && d < D, kok = key < N && d < D;
-                const size_t qi = (size_t)(q0 + col) * D + d, ki = (size_t)key * D + d;
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(qok ? Qg[qi] : 0.0f, kok ? Kg[ki] : 0.0f, s, 0, 0, 0);
-                dp = __builtin_amdgcn_mfma_f32_32x32x2f32(qok ? dOg[qi] : 0.0f, kok ? Vg[ki] : 0.0f, dp, 0, 0, 0);
-            }
-            __syncthreads();
-            if (tid < 64) {
-                const int row = q0 + (tid & 31);
-                stat[0][tid >> 5][tid & 31] = row < N ? (tid < 32 ? lse : delta)[row] : (tid < 32 ? -neg_inf() : 0.0f);
-            }
-            __syncthreads();
+            f32_rows<DT>(s, qb, k, col, hh);
+            f32_rows<DT>(dp, ob, v, col, hh);
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int r = 8 * (i >> 2) + 4 * hh + (i & 3);
                 float pv, ds;
-                weight(s[i], dp[i], stat[0][0][r], stat[0][1][r], pv, ds);
+                weight(s[i], dp[i], stat[tile & 1][0][r], stat[tile & 1][1][r], pv, ds);
                 s[i] = pv;
                 dp[i] = ds;
             }
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int row = q0 + 8 * (i >> 2) + 4 * hh + (i & 3);
-#pragma unroll
-                for (int t = 0; t < DT; t++) {
-                    const int d = 32 * t + col;
-                    const bool ok = row < N && d < D;
-                    const size_t at = (size_t)row * D + d;
-                    acc_dv[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(ok ? dOg[at] : 0.0f, s[i], acc_dv[t], 0, 0, 0);
-                    acc_dk[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(ok ? Qg[at] : 0.0f, dp[i], acc_dk[t], 0, 0, 0);
-                }
-            }
+            f32_cols<DT>(acc_dv, ob, s, col, hh);
+            f32_cols<DT>(acc_dk, qb, dp, col, hh);
+            if (tile + 1 < n_tiles) store_f((tile + 1) & 1);
+            __syncthreads();
         }
     }
     store_rows<DT>(p.dv + base, acc_dv, key, hh, N, D);
@@ -443,8 +447,7 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_k
     delta_q += other_half(delta_q);
     if (hh == 0 && q_ok) p.delta[(size_t)bh * N + q_row] = delta_q;
     float lse_q = q_ok ? p.lse[(size_t)bh * N + q_row] : 0.0f;
-    chk = __builtin_fmaf(lse_q, lse_q, chk);
-    chk = __builtin_fmaf(delta_q, delta_q, chk);
+    chk = split_max(split_max(chk, lse_q), delta_q);
     if (!q_ok) lse_q = -neg_inf();  // weights of zero
 
     f32x16_t acc[DT], low[DT];  // as in the kernel above
@@ -481,9 +484,9 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_k
     const int n_tiles = (N + kTile - 1) / kTile;
     load(0);
     store(0);
+    const bool uncarried = __syncthreads_or(!(chk < kSplitMost));  // seen already: no step of the loop below
     if (n_tiles > 1) load(kTile);
-    __syncthreads();
-    for (int tile = 0; tile < n_tiles; tile++) {  // a step as in the kernel above
+    for (int tile = 0; tile < (uncarried ? 0 : n_tiles); tile++) {  // a step as in the kernel above
         const __bf16* kb = lds + (tile & 1) * BUF;
         const __bf16* vb = kb + StK::SIZE;
         __bf16* nb = lds + ((tile + 1) & 1) * BUF;
@@ -563,33 +566,41 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_k
 
 #pragma unroll
     for (int t = 0; t < DT; t++) acc[t] += low[t];
-    if (__syncthreads_or(!(chk < kSplitMost))) {  // as in the kernel above
+    if (uncarried || __syncthreads_or(!(chk < kSplitMost))) {  // as in the kernel above
+        using Tile = F32Tile<DT>;
+        static_assert(4 * Tile::SIZE * sizeof(float) <= sizeof(lds), "two tiles of K and V");
+        float* const f32_lds = (float*)lds;
 #pragma unroll
         for (int t = 0; t < DT; t++) zero16(acc[t]);
+        float q[16 * DT], o[16 * DT];
+        f32_row<DT>(q, Qg + (size_t)q_row * D, q_ok, D, hh);
+        f32_row<DT>(o, dOg + (size_t)q_row * D, q_ok, D, hh);
+        Tile kt, vt;
+        auto load_f = [&](int kv0) {
+            kt.load(Kg, (size_t)D, kv0, N, D, tid);
+            vt.load(Vg, (size_t)D, kv0, N, D, tid);
+        };
+        auto store_f = [&](int b2) {
+            kt.store(f32_lds + b2 * 2 * Tile::SIZE, tid);
+            vt.store(f32_lds + b2 * 2 * Tile::SIZE + Tile::SIZE, tid);
+        };
+        load_f(0);
+        store_f(0);
+        __syncthreads();
         for (int tile = 0; tile < n_tiles; tile++) {
-            const int kv0 = tile * kTile;
+            const float* kb = f32_lds + (tile & 1) * 2 * Tile::SIZE;
+            if (tile + 1 < n_tiles) load_f((tile + 1) * kTile);
             f32x16_t s, dp;
             zero16(s);
             zero16(dp);
-            for (int ks = 0; ks < DPAD / 2; ks++) {
-                const int d = 8 * (ks >> 2) + 4 * hh + (ks & 3);  // the f32 kernels' order
-                const bool kok = kv0 + col < N && d < D, ok = q_ok && d < D;
-                const size_t ki = (size_t)(kv0 + col) * D + d, qi = (size_t)q_row * D + d;
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kok ? Kg[ki] : 0.0f, ok ? Qg[qi] : 0.0f, s, 0, 0, 0);
-                dp = __builtin_amdgcn_mfma_f32_32x32x2f32(kok ? Vg[ki] : 0.0f, ok ? dOg[qi] : 0.0f, dp, 0, 0, 0);
-            }
-            hide_edge(s, kv0);
+            f32_rows<DT>(s, kb, q, col, hh);
+            f32_rows<DT>(dp, kb + Tile::SIZE, o, col, hh);
+            hide_edge(s, tile * kTile);
 #pragma unroll
             for (int i = 0; i < 16; i++) dp[i] = weight(s[i], dp[i]);
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int row = kv0 + 8 * (i >> 2) + 4 * hh + (i & 3);
-#pragma unroll
-                for (int t = 0; t < DT; t++) {
-                    const int d = 32 * t + col;
-                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(row < N && d < D ? Kg[(size_t)row * D + d] : 0.0f, dp[i], acc[t], 0, 0, 0);
-                }
-            }
+            f32_cols<DT>(acc, kb, dp, col, hh);
+            if (tile + 1 < n_tiles) store_f((tile + 1) & 1);
+            __syncthreads();
         }
     }
     store_rows<DT>(p.dq + base, acc, q_row, hh, N, D);

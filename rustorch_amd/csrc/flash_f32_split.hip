@@ -38,8 +38,6 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
     // tiles t and t + 1 of K, t to t + 2 of V
     __shared__ __attribute__((aligned(16))) __bf16 lds[2 * KBUF + 3 * VBUF];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int col = lane & 31, hh = lane >> 5;
     const int Nq = p.seq, N = p.seq_kv ? p.seq_kv : p.seq;
     const int D = kExactD ? DPAD : p.dim;
     // p.zigzag 2 (head dims above 64): a workgroup takes two blocks of a head, a long and a short one, in turn
@@ -66,9 +64,13 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
     const size_t q_pitch = p.lq.row_pitch, kv_pitch = p.lkv.row_pitch, o_pitch = p.lo.row_pitch;
 
     for (;;) {
+        int tid = threadIdx.x;
+        if constexpr (DT > 2 && kCausal) asm volatile("" : "+v"(tid));  // formed once a block, not kept in registers between two
+        const int lane = tid & 63, wave = tid >> 6;
+        const int col = lane & 31, hh = lane >> 5;
         const int q0 = qblk * 4 * kTile, q0w = q0 + wave * kTile;
         const int q_row = q0w + col;
-        float chk = 0.0f;  // sum of squares of everything this thread splits
+        float chk = 0.0f;  // the largest magnitude of everything this thread splits
         float v_max = 0.0f;
 
         // Q as B operand: chunk j, this lane's 8 elements d = 16j + 8hh ..
@@ -85,7 +87,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
                 for (int i = 0; i < 4; i++) x[4 * u + i] = z[i];
             }
 #pragma unroll
-            for (int i = 0; i < 8; i++) chk = __builtin_fmaf(x[i], x[i], chk);
+            for (int i = 0; i < 8; i++) chk = split_max(chk, x[i]);
             qf[j] = split8(x);
         }
 
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
 
         // A tile's way into LDS: 8 elements of a K row per item, and 8 keys of a V column, in the order the weights sit in
         // the score accumulators (slot 8g + e is key 16 (g/2) + 4 (g%2) + 8 (e/4) + e%4).  Rows behind the last key repeat
-        // it: their weights are exact zeros, and a zero times a finite value adds nothing.
+        // it: their weights are exact zeros, and what a zero makes of its value the key itself has made of every row.
         f32x4_t kreg[NI][2];
         float vreg[NI][8];
 #pragma unroll
@@ -179,12 +181,12 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             if (u == 0) pair.r = split_f32x2_t{x0, x1};
             o.w[2 * n + (is_v ? 1 : 0)][u][e] = pair.step(u);
             if (u < 2) return;
-            chk = __builtin_fmaf(x0, x0, chk);
-            chk = __builtin_fmaf(x1, x1, chk);
             if (is_v) {  // scores of small keys are small whatever is lost of them; small values are the result's size
                 if (e == 0) v_max = 0.0f;
-                v_max = __builtin_fmaxf(__builtin_fmaxf(v_max, __builtin_fabsf(x0)), __builtin_fabsf(x1));
-                if (e == 3) chk = split_too_small(v_max) ? kSplitMost : chk;
+                v_max = split_max(split_max(v_max, x0), x1);
+                if (e == 3) chk = split_too_small(v_max) ? kSplitMost : __builtin_fmaxf(chk, v_max);
+            } else {
+                chk = split_max(split_max(chk, x0), x1);
             }
         };
         auto write_tile = [&](const Parts& o, __bf16* kbuf, __bf16* vbuf) RT_INLINE {
@@ -277,7 +279,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             load_tile(1);
             store_tile(lds + KBUF, v_lds + VBUF);
         }
-        __syncthreads();
+        const bool uncarried = __syncthreads_or(!(chk < kSplitMost));  // seen already: no step of the loop below
         f32x16_t s_next;
         zero16(s_next);
         read_plane(lds, 2);
@@ -287,7 +289,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
         // A step multiplies the next tile's scores while this tile's weights are formed, and this tile's weights with V while
         // the tile after the next is split: the matrix instructions have vector work between them in the same wave.  The
         // scheduling barriers keep that order; left to itself the compiler puts the one kind behind the other.
-        for (int tile = 0; tile < n_tiles; tile++) {
+        for (int tile = 0; tile < (uncarried ? 0 : n_tiles); tile++) {
             const __bf16* kn = lds + ((tile + 1) & 1) * KBUF;  // behind the last tile: scores of no tile, not used
             const __bf16* vb = v_lds + v_now * VBUF + col * LDV + 8 * hh;
             const int v_put = v_now == 0 ? 2 : v_now - 1;  // (tile + 2) % 3
@@ -360,45 +362,55 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             __syncthreads();
         }
 
-        if (__syncthreads_or(!(chk < kSplitMost))) {
-            // something here the split does not carry: the wave's rows once more in f32, straight from memory
+        if (uncarried || __syncthreads_or(!(chk < kSplitMost))) {
+            // something here the split does not carry: the rows once more in f32, the tiles through LDS two at a time.  For a
+            // launch (B=4 H=16 N=1024 D=64) 158 us where the first tiles show it, 240 where only the last does; straight from
+            // memory 770; the f32 kernel alone 181.
+            using Tile = F32Tile<DT>;
+            static_assert(4 * Tile::SIZE * sizeof(float) <= sizeof(lds), "two tiles of K and V");
+            float* const f32_lds = (float*)lds;
+            int tid_f = tid;  // what follows from it is formed here, not kept in registers through the loop above
+            asm volatile("" : "+v"(tid_f));
+            const int col_f = tid_f & 31, hh_f = (tid_f >> 5) & 1;
 #pragma unroll
-            for (int t = 0; t < DT; t++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) acc_o[t][i] = 0.0f;
+            for (int t = 0; t < DT; t++) zero16(acc_o[t]);
             m_run = neg_inf();
             l_run = l_low = 0.0f;
-            for (int tile = 0; tile < n_wave; tile++) {
-                const int kv0 = tile * kTile;
-                f32x16_t s;
+            float q[16 * DT];
+            f32_row<DT>(q, Qg + (size_t)q_row * q_pitch, q_row < Nq, D, hh_f);
+            Tile kt, vt;
+            auto load = [&](int tile) RT_INLINE {
+                kt.load(Kg, kv_pitch, tile * kTile, N, D, tid_f);
+                vt.load(Vg, kv_pitch, tile * kTile, N, D, tid_f);
+            };
+            auto store = [&](int tile) RT_INLINE {
+                kt.store(f32_lds + (tile & 1) * 2 * Tile::SIZE, tid_f);
+                vt.store(f32_lds + (tile & 1) * 2 * Tile::SIZE + Tile::SIZE, tid_f);
+            };
+            load(0);
+            store(0);
+            __syncthreads();
+            for (int tile = 0; tile < n_tiles; tile++) {
+                const float* kb = f32_lds + (tile & 1) * 2 * Tile::SIZE;
+                if (tile + 1 < n_tiles) load(tile + 1);
+                if (tile < n_wave) {
+                    f32x16_t s;
+                    zero16(s);
+                    f32_rows<DT>(s, kb, q, col_f, hh_f);
+                    scale_mask(s, tile * kTile);
+                    const float m_use = take_max(row_max(s));
+                    float tile_l = 0.0f;
 #pragma unroll
-                for (int i = 0; i < 16; i++) s[i] = 0.0f;
-                for (int ks = 0; ks < DPAD / 2; ks++) {
-                    const int d = 8 * (ks >> 2) + 4 * hh + (ks & 3);  // the f32 kernel's order
-                    const float a = (kv0 + col < N && d < D) ? Kg[(size_t)(kv0 + col) * kv_pitch + d] : 0.0f;
-                    const float bq = (q_row < Nq && d < D) ? Qg[(size_t)q_row * q_pitch + d] : 0.0f;
-                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(a, bq, s, 0, 0, 0);
-                }
-                scale_mask(s, kv0);
-                const float m_use = take_max(row_max(s));
-                float tile_l = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    s[i] = __builtin_amdgcn_exp2f((s[i] - m_use) * kLog2e);
-                    tile_l += s[i];
-                }
-                add_sum(tile_l);
-                rescale();
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int kr = kv0 + 8 * (i >> 2) + 4 * hh + (i & 3);
-#pragma unroll
-                    for (int t = 0; t < DT; t++) {
-                        const int d = 32 * t + col;
-                        const float a = (kr < N && d < D) ? Vg[(size_t)kr * kv_pitch + d] : 0.0f;
-                        acc_o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, s[i], acc_o[t], 0, 0, 0);
+                    for (int i = 0; i < 16; i++) {
+                        s[i] = __builtin_amdgcn_exp2f((s[i] - m_use) * kLog2e);
+                        tile_l += s[i];
                     }
+                    add_sum(tile_l);
+                    rescale();
+                    f32_cols<DT>(acc_o, kb + Tile::SIZE, s, col_f, hh_f);
                 }
+                if (tile + 1 < n_tiles) store(tile + 1);
+                __syncthreads();
             }
         }
 
@@ -419,7 +431,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
                 if (kExactD || d < D) *(f32x4_t*)(o_row + d) = o;
             }
         }
-        // (every wave is behind the barrier of the test above: the tiles of the next block may come into LDS)
+        // (every wave is behind a barrier behind its last tile: those of the next block may come into LDS)
         if (DT <= 2 || !kCausal || p.zigzag != 2 || qblk == x || n_blk - 1 - x == x) return;
         qblk = x;
     }

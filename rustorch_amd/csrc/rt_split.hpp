@@ -6,10 +6,10 @@
 // is below 2^-26 |x y|, less than half of an f32 rounding.  Every term is exact in the f32 accumulator of
 // v_mfma_f32_32x32x16_bf16, whose rate is 16 times that of v_mfma_f32_32x32x2_f32: six of them are 2.7 times the f32 rate.
 //
-// Infinities and NaN do not survive the split (inf - inf), and finite values whose products overflow f32 would give
-// inf - inf where one product gives inf.  The kernels sum the squares of everything they split: below 2^60 no
-// operand exceeds 2^30 and neither can happen, in a product of two nor in the gradients' products of three.  A workgroup
-// that finds the sum above it, or NaN, does its rows once more on the f32 matrix cores.
+// NaN survives the split as three NaN, and whatever f32 arithmetic makes NaN of it comes out NaN here.  Infinities do not
+// (inf - inf), and finite values whose products overflow f32 would give inf - inf where one product gives inf.  The
+// kernels keep the largest magnitude of everything they split: below 2^30 neither can happen, in a product of two nor in
+// the gradients' products of three.  A workgroup that finds one above it does its rows once more on the f32 matrix cores.
 #pragma once
 #include "rt_common.hpp"
 
@@ -64,8 +64,67 @@ __device__ __forceinline__ f32x16_t mfma_h(bf16x8_t a, bf16x8_t b, f32x16_t acc)
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
 }
 
-constexpr float kSplitMost = 0x1p60f;  // the sum of squares from which on the split products are not used
+constexpr float kSplitMost = 0x1p30f;  // the magnitude from which on the split products are not used
 // The same for values so small that the last term of the split would count (largest of a group of eight; zeros are fine).
 __device__ __forceinline__ bool split_too_small(float group_max) { return group_max < 0x1p-80f && group_max > 0.0f; }
+// The larger magnitude; a NaN is not seen.
+__device__ __forceinline__ float split_max(float m, float x) { return __builtin_fmaxf(m, __builtin_fabsf(x)); }
+
+// A tile of 32 rows in f32 on its way through the 256 threads of a workgroup into LDS, zeros beyond the last row and D: for
+// the rows that are done once more.  16-byte loads; a row's start is 4 banks behind the one before it.
+template <int DT>
+struct F32Tile {
+    static constexpr int CH = 8 * DT, LD = 32 * DT + 4, SIZE = 32 * LD;
+    f32x4_t r[DT];
+    __device__ __forceinline__ void load(const float* __restrict__ src, size_t pitch, int row0, int N, int D, int tid) {
+#pragma unroll
+        for (int n = 0; n < DT; n++) {
+            const int idx = 256 * n + tid, row = row0 + idx / CH, d = 4 * (idx % CH);
+            f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (row < N && d < D) z = *(const f32x4_t*)(src + (size_t)row * pitch + d);
+            r[n] = z;
+        }
+    }
+    __device__ __forceinline__ void store(float* dst, int tid) const {
+#pragma unroll
+        for (int n = 0; n < DT; n++) {
+            const int idx = 256 * n + tid;
+            *(f32x4_t*)(dst + (idx / CH) * LD + 4 * (idx % CH)) = r[n];
+        }
+    }
+};
+
+// acc += X . Y^T over the head dim, in the order of the f32 kernels (d = 8j + 4 hh + i): row `col` of a tile in LDS as A
+// operand, y[4j + i] in registers as B.
+template <int DT>
+__device__ __forceinline__ void f32_rows(f32x16_t& acc, const float* tile, const float (&y)[16 * DT], int col, int hh) {
+#pragma unroll
+    for (int j = 0; j < 4 * DT; j++) {
+        const f32x4_t a = *(const f32x4_t*)(tile + col * F32Tile<DT>::LD + 8 * j + 4 * hh);
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], y[4 * j + i], acc, 0, 0, 0);
+    }
+}
+// acc[t] += X^T . w over the tile's rows: column 32t + col of the tile, w as a score accumulator holds it
+template <int DT>
+__device__ __forceinline__ void f32_cols(f32x16_t (&acc)[DT], const float* tile, const f32x16_t& w, int col, int hh) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const float* row = tile + (8 * (i >> 2) + 4 * hh + (i & 3)) * F32Tile<DT>::LD + col;
+#pragma unroll
+        for (int t = 0; t < DT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(row[32 * t], w[i], acc[t], 0, 0, 0);
+    }
+}
+// The B operand of f32_rows: this lane's elements of a row, zeros beyond D and where `ok` is false.
+template <int DT>
+__device__ __forceinline__ void f32_row(float (&y)[16 * DT], const float* __restrict__ row, bool ok, int D, int hh) {
+#pragma unroll
+    for (int j = 0; j < 4 * DT; j++) {
+        f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (ok && 8 * j + 4 * hh < D) z = *(const f32x4_t*)(row + 8 * j + 4 * hh);
+#pragma unroll
+        for (int i = 0; i < 4; i++) y[4 * j + i] = z[i];
+    }
+}
 
 }  // namespace rt
