@@ -407,10 +407,10 @@ __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)
 // A segment's word, (launch id | count): the memory it lies in holds anything at first, another launch's word included,
 // so every workgroup makes sure, ahead of its own count, that the word carries this launch's id: it replaces what it has
 // seen there unless that has the id.  A replacement fails only if another workgroup of the launch was first.  `seen` is
-// requested ahead of everything else and the replacement sent when the first rows are there, so that neither is waited for
-// by itself (sent behind the walk: 0.4 us more a call).  The token of a context of 2048, 32 / 8 heads of 128, with its
-// preparation: 11.2 us with counters of 4 bytes side by side that the library kept at zero, 11.5 with words side by side,
-// 10.7 with a line for each.
+// requested ahead of everything else and the replacement sent behind the requests for the first rows, so that neither is
+// waited for by itself (sent behind the walk: 0.4 us more a call).  The token of a context of 2048, 32 / 8 heads of 128,
+// with its preparation: 11.2 us with counters of 4 bytes side by side that the library kept at zero, 11.5 with words side
+// by side, 10.6 with a line for each.
 typedef unsigned long long word_t;
 constexpr int kWordPitch = 128;  // bytes from one segment's word to the next: atomics on one line wait for each other
 struct SegWord {
@@ -608,9 +608,9 @@ __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSp
         bf16x8_t qreg[T::KS];
         dec_load<HD>(p, b, kvh, t, len, lane, kreg, vreg);
         dec_load_q<HD>(p, b, kvh, lane, qreg);
+        if (counts) word.replace();
         for (; t < t1; t += kLatWaves) {
             dec_park<HD>(Kw, Vw, lane, kreg, vreg);
-            if (counts && t == split * per) word.replace();
             if (t + kLatWaves < t1) dec_load<HD>(p, b, kvh, t + kLatWaves, len, lane, kreg, vreg);
             dec_step<HD>(Kw, Vw, lane, len - t * kDecRows, c, lazy, qreg, state);
         }
