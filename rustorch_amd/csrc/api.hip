@@ -1171,6 +1171,19 @@ RT_API int rt_debug_force_bf16_prefill_kernel(int which) {
     return RT_OK;
 }
 
+RT_API int rt_debug_f32_split_products(const rt_attention_shape* shape, uint64_t seq_kv, int mask_kind, int with_lse) {
+    if (!shape || !fits_int(shape->batch) || !fits_int(shape->heads) || !fits_int(shape->seq) || !fits_int(seq_kv) || shape->dim == 0 || shape->dim > 512) return 0;
+    rt::FlashF32Params p{};
+    p.batch = (int)shape->batch;
+    p.heads = (int)shape->heads;
+    p.seq = (int)shape->seq;
+    p.seq_kv = (int)seq_kv;
+    p.dim = (int)shape->dim;
+    p.mask = mask_kind;
+    p.n_cus = g_num_cus;
+    return rt::flash_f32_takes_split(p, with_lse != 0) ? 1 : 0;
+}
+
 RT_API int rt_set_strict_non_finite_v(int on) { return g_strict_v.exchange(on ? 1 : 0); }
 
 static int flash_bf16_common(void* stream, const rt_attention_shape* shape, uint64_t n_kv_heads, const void* q,

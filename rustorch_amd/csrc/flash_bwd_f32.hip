@@ -576,7 +576,7 @@ hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Param
     auto aligned = [](const void* ptr) { return (uintptr_t)ptr % 16 == 0; };
     p.vec = (p.dim % 4 == 0) && aligned(p.q) && aligned(p.k) && aligned(p.v) && aligned(p.d_out) && aligned(p.dq) &&
             aligned(p.dk) && aligned(p.dv);
-    if (p.vec && p.dim <= 64 && aligned(p.o)) {  // many rows: the bf16 matrix cores, by the rule of the forward
+    if (p.vec && aligned(p.o)) {  // many rows: the bf16 matrix cores, by the rule of the forward
         FlashF32Params f{};
         f.batch = p.batch;
         f.heads = p.heads;
@@ -584,7 +584,7 @@ hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Param
         f.dim = p.dim;
         f.mask = kMaskNone;
         f.n_cus = p.n_cus;
-        if (flash_f32_split_pays(f)) return launch_flash_bwd_f32_split(stream, p);
+        if (flash_f32_takes_split(f, true)) return launch_flash_bwd_f32_split(stream, p);
     }
     dim3 grid((p.seq + kRows - 1) / kRows, p.heads, p.batch), block(256);
     const int dt = (p.dim + 31) / 32;

@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
 // keys 331 / 197, causal 175 / 193; 2 x 12 heads, 999 keys 76 / 55 (gradients 200 / 178), causal 50 / 53; 8 x 16 heads,
 // 256 keys 32 / 22 (gradients 89 / 66), causal 31 / 22.  Head dim 128: 8 heads, 2048 keys 191 / 192, 16 heads, 1500 keys
 // 219 / 146, causal 135 / 144; 4 x 16 heads, 1024 keys 405 / 218, causal 249 / 133.
-bool flash_f32_split_pays(const FlashF32Params& p) {
+static bool flash_f32_split_pays(const FlashF32Params& p) {
     const double n_cus = p.n_cus > 0 ? p.n_cus : 256;
     const long long keys = p.seq_kv ? p.seq_kv : p.seq;
     const double tiles = (double)((keys + 31) / 32), blocks = (p.seq + 127) / 128, n_bh = (double)p.heads * p.batch;
@@ -515,6 +515,11 @@ bool flash_f32_split_pays(const FlashF32Params& p) {
     if (p.dim > 64) return there * 0.55 < here + 0.5;
     const double step = p.dim > 32 ? (causal ? 0.58 : 0.69) : (causal ? 0.68 : 0.76);
     return there * step < here + 0.5;
+}
+
+// (above head dim 64 the gradients have no such form, and a row statistic they read is formed as they form the scores)
+bool flash_f32_takes_split(const FlashF32Params& p, bool with_lse) {
+    return p.dim % 4 == 0 && p.dim <= (with_lse ? 64 : 128) && !p.bias && p.mask != kMaskPadding && flash_f32_split_pays(p);
 }
 
 hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p) {
@@ -533,8 +538,7 @@ hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p) {
         pz.zigzag = (p.mask == kMaskCausal) && ((long long)grid.x * grid.y * grid.z <= resident) ? 1 : 0;
         const bool exact = (p.dim % 32 == 0), pad = (p.mask == kMaskPadding);
         if (p.bias && p.mask != kMaskNone) return hipErrorInvalidValue;  // a bias comes without a mask kind
-        // (above head dim 64 the gradients have no such form, and a row statistic they read is formed as they form the scores)
-        if (!p.bias && !pad && (dt <= 2 || !p.lse) && flash_f32_split_pays(p)) return launch_flash_f32_split(stream, p);
+        if (flash_f32_takes_split(p, p.lse != nullptr)) return launch_flash_f32_split(stream, p);
         const int mode = pad ? 2 : (p.mask == kMaskCausal ? 1 : (p.bias ? 3 : 0));
         auto launch = [&](auto dt_c, auto exact_c) {
             constexpr int kDT = decltype(dt_c)::value;

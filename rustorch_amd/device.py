@@ -124,6 +124,13 @@ def debug_force_bf16_prefill_kernel(name: str = "auto"):
         raise ValueError(name)
 
 
+def debug_f32_split_products(shape, mask=None, seq_kv: int = 0, with_lse: bool = False) -> bool:
+    """Whether an f32 forward of `shape` runs on the bf16 matrix cores, operands as three bf16 terms (measurement / test
+    query); `with_lse`: the forward that keeps its row statistic, and the gradients."""
+    s = shape._c()
+    return bool(L.lib().rt_debug_f32_split_products(C.byref(s), seq_kv, mask.kind if mask else L.RT_MASK_NONE, int(with_lse)))
+
+
 def set_strict_non_finite_v(on: bool) -> bool:
     """Causal prefill entries follow the reference for non-finite V at hidden keys (every row NaN in that column,
     cpu_forward.rs:268-425) at the cost of one more pass over V.  Returns the previous setting."""

@@ -36,6 +36,7 @@ hipError_t launch_flash_f32(hipStream_t s, const FlashF32Params& p) {
     for (size_t i = 0; i < n; i++) p.out[i] = p.q[i] + 2.0f * p.k[i] + 4.0f * p.v[i];
     return hipSuccess;
 }
+bool flash_f32_takes_split(const FlashF32Params&, bool) { return false; }
 hipError_t launch_decode_split(hipStream_t s, const DecodeSplitParams& p) {
     fake::log("decode", s);
     fake::Inside here;

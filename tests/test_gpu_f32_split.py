@@ -13,6 +13,16 @@ from _util import seeded_normal
 pytestmark = pytest.mark.gpu
 
 
+# on the other side of the rule's line, some of them under one mask only: the f32 matrix cores, to the same bound
+BESIDE = [(13, 20, 161, 36), (16, 16, 130, 64), (9, 16, 225, 80)]
+
+
+def assert_split(b, h, n, d, causal=False, seq_kv=0, with_lse=False):
+    """The launch takes the kernels this file is about."""
+    assert ra.debug_f32_split_products(ra.AttentionShape.new(b, h, n, d), ra.Mask.causal() if causal else ra.Mask.none(), seq_kv,
+                                       with_lse)
+
+
 def run(q, k, v, causal):
     b, h, n, d = q.shape
     out = ra.HipStorage(q.size * 4)
@@ -42,13 +52,14 @@ def inputs(b, h, n, d):
 @pytest.mark.parametrize("b,h,n,d", [
     (8, 16, 256, 64),   # whole tiles
     (8, 16, 225, 60),   # 31 keys of the last tile missing, head dim padded
-    (13, 20, 161, 36),  # one row in a workgroup's second wave, head pairs not a multiple of eight
+    (9, 14, 417, 36),   # one row in a workgroup's second wave, head pairs not a multiple of eight
     (8, 32, 384, 32),   # head dim 32: half the threads split
-    (16, 16, 130, 64),  # two rows in the last workgroup
+    (8, 16, 386, 64),   # two rows in the last workgroup
     (8, 16, 256, 128),
     (8, 32, 353, 96),   # three blocks of rows, two a workgroup where causal
-    (9, 16, 225, 80),
+    (8, 16, 225, 80),
     (8, 32, 353, 68),
+    *BESIDE,
 ])
 def test_against_64_bits(b, h, n, d, causal):
     q, k, v = inputs(b, h, n, d)
@@ -185,6 +196,7 @@ def gradients64(q, k, v, d_out):
     (8, 16, 225, 60),
     (8, 32, 353, 32),   # one row in the last tile, head dim 32
     (8, 28, 481, 36),   # head pairs not a multiple of the XCDs' share, padded head dim
+    (8, 16, 386, 64),   # two rows in the last workgroup
     (16, 16, 130, 64),
 ])
 def test_gradients_against_64_bits(b, h, n, d):
@@ -222,3 +234,87 @@ def test_gradients_of_values_the_split_does_not_carry(what):
             fin = np.isfinite(ws)
             assert np.array_equal(np.isnan(gs), np.isnan(ws)), name
             assert not fin.any() or np.linalg.norm((gs - ws)[fin]) <= 2e-6 * np.linalg.norm(ws[fin]), name
+
+
+def shapes_of(test):
+    return next(m.args[1] for m in test.pytestmark if m.name == "parametrize" and m.args[0] == "b,h,n,d")
+
+
+def test_the_shapes_of_this_file_take_these_kernels():
+    for shape in shapes_of(test_against_64_bits):
+        if shape not in BESIDE:
+            assert_split(*shape)
+            assert_split(*shape, causal=True)
+    for shape in shapes_of(test_gradients_against_64_bits):
+        if shape not in BESIDE:
+            assert_split(*shape, with_lse=True)
+    for b, h, n, d in BESIDE:
+        assert not ra.debug_f32_split_products(ra.AttentionShape.new(b, h, n, d), ra.Mask.causal())
+
+
+def bnhd(x):
+    return np.ascontiguousarray(np.swapaxes(x, 1, 2))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("b,h,hkv,n,d", [
+    (8, 16, 16, 225, 60),
+    (8, 16, 4, 256, 64),
+    (9, 14, 7, 417, 36),   # head pairs not a multiple of eight, padded head dim
+    (8, 32, 1, 384, 32),   # one kv head for all
+    (8, 32, 8, 353, 96),   # two blocks of rows a workgroup where causal
+    (8, 16, 8, 225, 128),
+])
+def test_grouped_heads_and_rows_apart(b, h, hkv, n, d, causal):
+    """kv heads that serve groups, and [batch, seq, heads, dim] tensors, against 64 bits; both layouts give the same bits."""
+    assert_split(b, h, n, d, causal)
+    q = seeded_normal((b, h, n, d), 1).reshape(b, h, n, d)
+    k, v = (seeded_normal((b, hkv, n, d), i).reshape(b, hkv, n, d) for i in (2, 3))
+    want = attention64(q, np.repeat(k, h // hkv, axis=1), np.repeat(v, h // hkv, axis=1), causal)
+    shape, mask = ra.AttentionShape.new(b, h, n, d), ra.Mask.causal() if causal else ra.Mask.none()
+    got = []
+    for layout, call in ((np.ascontiguousarray, ra.flash_forward_f32_dev), (bnhd, ra.flash_forward_bnhd_f32_dev)):
+        out = ra.HipStorage(q.size * 4)
+        out.upload(np.full(q.size, 7.0, dtype=np.float32))
+        call(shape, dev(layout(q)), dev(layout(k)), dev(layout(v)), out, mask, n_kv_heads=hkv)
+        ra.synchronize()
+        got.append(layout(out.download(np.float32).reshape(layout(q).shape)))
+    assert np.linalg.norm(got[0] - want) <= 1e-6 * np.linalg.norm(want)
+    assert np.abs(got[0] - want).max() <= 5e-6
+    assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("b,h,hkv,t_q,t_kv,d", [
+    (8, 16, 16, 256, 300, 64),
+    (8, 16, 16, 225, 31, 60),    # one ragged tile of keys
+    (12, 21, 21, 161, 513, 36),
+    (8, 32, 32, 353, 97, 96),
+    (8, 16, 4, 225, 257, 128),   # kv heads that serve groups (the grouped entry)
+    (8, 32, 8, 384, 33, 32),
+])
+def test_keys_of_another_length(b, h, hkv, t_q, t_kv, d):
+    assert_split(b, h, t_q, d, seq_kv=t_kv)
+    q = seeded_normal((b, h, t_q, d), 1).reshape(b, h, t_q, d)
+    k, v = (seeded_normal((b, hkv, t_kv, d), i).reshape(b, hkv, t_kv, d) for i in (2, 3))
+    want = attention64(q, np.repeat(k, h // hkv, axis=1), np.repeat(v, h // hkv, axis=1), False)
+    out = ra.HipStorage(q.size * 4)
+    out.upload(np.full(q.size, 7.0, dtype=np.float32))
+    if hkv == h:
+        ra.mha_forward_masked_f32_dev(dev(bnhd(q)), dev(bnhd(k)), dev(bnhd(v)), out, b, t_q, t_kv, h, d)
+        ra.synchronize()
+        got = bnhd(out.download(np.float32).reshape(b, t_q, h, d))
+    else:
+        ra.gqa_forward_f32_dev(dev(q), dev(k), dev(v), out, b, h, hkv, t_q, t_kv, d)
+        ra.synchronize()
+        got = out.download(np.float32).reshape(q.shape)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+    assert np.abs(got - want).max() <= 5e-6
+
+
+def test_the_rule_turns_away_what_the_kernels_do_not_take():
+    """Padding masks, head dims that are no multiple of 4 or above 128 (64 with the row statistic), and few rows."""
+    big = ra.AttentionShape.new
+    assert not ra.debug_f32_split_products(big(8, 16, 256, 64), ra.Mask.padding(np.ones(256, dtype=bool)))
+    for d, with_lse in ((62, False), (132, False), (256, False), (68, True), (128, True)):
+        assert not ra.debug_f32_split_products(big(8, 16, 1024, d), with_lse=with_lse)
+    assert not ra.debug_f32_split_products(big(1, 1, 64, 64))
