@@ -27,7 +27,15 @@ static std::mutex g_mutex;
 static std::vector<rt::DecodeSplitParams> g_decode;
 static std::vector<rt::FlashTileParams> g_tile;
 static int g_rows = 0;
-alignas(256) static unsigned char g_slots[rt::kStreamSlots][4096];
+
+// the kernels of decode.hip, by their names
+static void note_launch(const std::string& name, dim3 grid, void** args, hipStream_t s) {
+    if (name.find("attn_rows") != std::string::npos) g_rows++;
+    if (name.find("decode_latency") == std::string::npos && name.find("decode_split") == std::string::npos) return;
+    fake::log("decode", s);
+    std::lock_guard<std::mutex> lock(g_mutex);
+    g_decode.push_back(*(rt::DecodeSplitParams*)args[0]);
+}
 
 namespace rt {
 hipError_t launch_flash_f32(hipStream_t s, const FlashF32Params& p) {
@@ -37,13 +45,6 @@ hipError_t launch_flash_f32(hipStream_t s, const FlashF32Params& p) {
     return hipSuccess;
 }
 bool flash_f32_takes_split(const FlashF32Params&, bool) { return false; }
-hipError_t launch_decode_split(hipStream_t s, const DecodeSplitParams& p) {
-    fake::log("decode", s);
-    fake::Inside here;
-    std::lock_guard<std::mutex> lock(g_mutex);
-    g_decode.push_back(p);
-    return hipSuccess;
-}
 hipError_t launch_flash_tile_bf16(hipStream_t s, const FlashTileParams& p) {
     fake::log("tile", s);
     fake::Inside here;
@@ -51,8 +52,6 @@ hipError_t launch_flash_tile_bf16(hipStream_t s, const FlashTileParams& p) {
     g_tile.push_back(p);
     return hipSuccess;
 }
-hipError_t launch_attn_rows_bf16(hipStream_t, const AttnRowsParams&) { return g_rows++, hipSuccess; }
-hipError_t launch_attn_rows_f32(hipStream_t, const AttnRowsParams&) { return hipSuccess; }
 size_t flash_bwd_f32_workspace_floats(int, int, int, int) { return 64; }
 hipError_t launch_flash_bwd_f32(hipStream_t, const FlashBwdF32Params&, float*) { return hipSuccess; }
 hipError_t launch_flash_bwd_f32_saved(hipStream_t, const FlashBwdF32Params&, const float*, const float*, float*) { return hipSuccess; }
@@ -62,18 +61,7 @@ int flash_tile_bf16_workgroups(int) { return 2; }
 bool flash_tile_bf16_addressable(long long, long long) { return true; }
 bool flash_wide_bf16_supported(const FlashTileParams&) { return false; }
 hipError_t launch_flash_wide_bf16(hipStream_t, const FlashTileParams&) { return hipSuccess; }
-hipError_t launch_strict_hidden_v(hipStream_t, const StrictVParams&, bool) { return hipSuccess; }
-bool decode_split_supported(int, int, int) { return true; }
-int decode_split_span_min(int) { return 2; }
-int decode_split_parts(int, int max_seq) { return max_seq / 64 + 1; }
-size_t decode_split_workspace_bytes(int b, int h, int d, int m) { return (size_t)b * h * (d + 2) * 4 * (m / 64 + 1); }
-size_t decode_split_compact_bytes(int, int, int, int, int) { return 1024; }
-hipError_t decode_static_scratch(float** p, size_t* n) { return *p = (float*)g_slots[0], *n = 8 << 20, hipSuccess; }
-hipError_t stream_static_scratch(int slot, float** p, size_t* n) { return *p = (float*)g_slots[slot], *n = kStreamSlotBytes, hipSuccess; }
-int decode_latency_splits(int, int, int, int, int, int max_len, int) { return max_len > 4096 ? 0 : (max_len > 384 ? 8 : 1); }
-hipError_t launch_kv_block_append(hipStream_t, void*, void*, const void*, const void*, size_t, size_t, size_t, size_t, size_t, size_t) { return hipSuccess; }
 hipError_t launch_decode_prepare(hipStream_t, const DecodePrepareParams&) { return hipSuccess; }
-hipError_t launch_kv_append_bf16(hipStream_t, uint16_t*, uint16_t*, const uint16_t*, const uint16_t*, int, int, int, int) { return hipSuccess; }
 }  // namespace rt
 
 // ---- a machine that refuses -------------------------------------------------------------------------------------
@@ -108,12 +96,12 @@ static int chunk(hipStream_t s) { return rt_gqa_decode_chunk_bf16(s, g_buf, g_bu
 // The launches of a batched call work in the caller's workspace alone, under whatever handle: none shares memory, or the
 // id it goes by, with another.
 static void batched_calls_share_nothing() {
-    const size_t need = rt_gqa_decode_workspace_bytes(2, 8, 2, 64, 1024);
+    const size_t need = rt_gqa_decode_workspace_bytes(2, 8, 2, 64, 3000);
     std::vector<std::vector<char>> ws(4, std::vector<char>(need + 16));
-    int32_t lens[2] = {1024, 500};
+    int32_t lens[2] = {3000, 500};
     auto call = [&](int i, hipStream_t s) {
         void* w = (void*)(((uintptr_t)ws[(size_t)i].data() + 15) & ~(uintptr_t)15);
-        CHECK(rt_gqa_decode_batched_bf16(s, g_buf, g_buf, g_buf, g_buf, lens, 2, 8, 2, 64, 1024, w, need, nullptr) == RT_OK);
+        CHECK(rt_gqa_decode_batched_bf16(s, g_buf, g_buf, g_buf, g_buf, lens, 2, 8, 2, 64, 3000, w, need, nullptr) == RT_OK);
     };
     std::thread a(call, 0, hipStreamPerThread), b(call, 1, hipStreamPerThread);
     a.join();
@@ -138,7 +126,7 @@ static void calls_on_the_per_thread_stream_take_turns() {
     std::vector<std::thread> threads;
     for (int i = 0; i < 4; i++)
         threads.emplace_back([i] {
-            for (int n = 0; n < 50; n++) CHECK((i % 2 ? online(hipStreamPerThread, n % 2 ? 2000 : 8000) : chunk(hipStreamPerThread)) == RT_OK);
+            for (int n = 0; n < 50; n++) CHECK((i % 2 ? online(hipStreamPerThread, n % 2 ? 2000 : 8192) : chunk(hipStreamPerThread)) == RT_OK);
         });
     for (auto& t : threads) t.join();
     const auto& ops = fake::state().ops;
@@ -263,6 +251,27 @@ static void a_host_without_memory_is_an_error() {
     CHECK(fake::state().memory.empty());
 }
 
+// One-launch decode: what it leaves fits the memory of every entry, and what the kernel counts on holds.
+static void partials_and_words_fit() {
+    int split = 0;
+    for (int batch : {1, 2, 3, 7, 16, 64, 200, 4000})
+        for (int kv : {1, 2, 8, 32})
+            for (int group : {1, 3, 16})
+                for (int dim : {64, 128, 256})
+                    for (int max_seq : {1, 100, 384, 385, 513, 1056, 2048, 5000, 8192, 100000})
+                        for (int cus : {64, 256, 304}) {
+                            const int heads = kv * group;
+                            const int n = rt::decode_latency_splits(batch, heads, kv, dim, max_seq, max_seq, cus);
+                            CHECK(n >= 0 && n <= 24);
+                            if (n <= 1) continue;
+                            split++;
+                            const size_t used = (size_t)batch * heads * n * (dim + 2) * 4 + (size_t)batch * kv * 128;
+                            CHECK(used <= rt::decode_split_workspace_bytes(batch, heads, dim, max_seq) && used <= rt::kStreamSlotBytes);
+                            CHECK((long long)n * batch * kv <= cus);
+                        }
+    CHECK(split > 0);
+}
+
 // The prefill plan is what dealing the jobs one by one gives (jobs of 256 rows, rounds back and forth over the workers of
 // an XCD, or over all), and it costs a call no allocation.
 static void the_prefill_plan_deals_as_the_kernel_does() {
@@ -309,7 +318,9 @@ static void the_prefill_plan_deals_as_the_kernel_does() {
 }
 
 int main(int argc, char** argv) {
+    fake::on_launch() = note_launch;
     const std::map<std::string, std::function<void()>> tests = {
+        {"partials_and_words_fit", partials_and_words_fit},
         {"batched_calls_share_nothing", batched_calls_share_nothing},
         {"calls_on_the_per_thread_stream_take_turns", calls_on_the_per_thread_stream_take_turns},
         {"host_slices_follow_the_current_device", host_slices_follow_the_current_device},

@@ -7,6 +7,7 @@
 #include <chrono>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <string>
@@ -43,6 +44,19 @@ inline State& state() {
     return s;
 }
 inline thread_local int current_device = 0;
+struct Var {
+    size_t bytes;
+    std::map<int, std::vector<char>> by_device;
+};
+inline std::map<const void*, Var>& vars() {
+    static std::map<const void*, Var> v;
+    return v;
+}
+// what a test makes of a launch (the kernel's mangled name, its arguments)
+inline std::function<void(const std::string&, dim3, void**, hipStream_t)>& on_launch() {
+    static std::function<void(const std::string&, dim3, void**, hipStream_t)> f;
+    return f;
+}
 inline thread_local dim3 push_grid, push_block;
 inline thread_local int inside = 0;  // the runtime's own allocations are none of the library's
 struct Inside {
@@ -128,7 +142,16 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
     if (c != hipStreamCaptureStatusNone) return fake::refuse(hipErrorStreamCaptureIsolation);
     return fake::log("wait", s, e), hipSuccess;
 }
-hipError_t hipGetSymbolAddress(void**, const void*) { return hipErrorInvalidSymbol; }
+hipError_t hipGetSymbolAddress(void** p, const void* symbol) {
+    fake::Inside here;
+    std::lock_guard<std::mutex> lock(fake::state().mutex);
+    auto it = fake::vars().find(symbol);
+    if (it == fake::vars().end()) return hipErrorInvalidSymbol;
+    auto& mem = it->second.by_device[fake::current_device];
+    mem.resize(it->second.bytes + 256);
+    *p = (void*)(((uintptr_t)mem.data() + 255) & ~(uintptr_t)255);
+    return hipSuccess;
+}
 
 // what a compiled kernel launch calls
 static void* fake_fatbin;
@@ -137,7 +160,7 @@ void __hipUnregisterFatBinary(void**) {}
 void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, dim3*, dim3*, int*) {
     fake::state().kernels[host] = name;
 }
-void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+void __hipRegisterVar(void**, void* var, char*, char*, int, size_t bytes, int, int) { fake::vars()[var].bytes = bytes; }
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t, hipStream_t s);
 hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* n, hipStream_t* s);
 static thread_local hipStream_t fake_push_stream;
@@ -154,10 +177,10 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* n, hipStream_t* s
     *s = fake_push_stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* host, dim3, dim3, void** args, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void* host, dim3 grid, dim3, void** args, size_t, hipStream_t s) {
     fake::Inside here;
     const std::string& name = fake::state().kernels[host];
-    fake::log("kernel", s);
+    if (fake::on_launch()) fake::on_launch()(name, grid, args, s);
     if (name.find("stage_copy") != std::string::npos)
         memcpy(*(void**)args[0], *(void**)args[1], *(size_t*)args[2] * 16);
     return hipSuccess;

@@ -9,6 +9,7 @@ CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
 
 
 @pytest.mark.parametrize("name", [
+    "partials_and_words_fit",
     "batched_calls_share_nothing",
     "calls_on_the_per_thread_stream_take_turns",
     "host_slices_follow_the_current_device",
