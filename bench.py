@@ -316,12 +316,11 @@ def main():
     d64_p = None
     if args.only in (None, "d64"):
         Bd, Hd, Nd, Dd = 4, 32, 4096, 64
-        # (the library takes the tile kernel here; RT_ATTN_BF16_PREFILL=wide|persistent in the environment forces another,
-        # which the leg then names)
+        # (the library takes the tile kernel here; RT_ATTN_BF16_PREFILL=wide in the environment forces another, which the
+        # leg then names)
         d64_kernel, d64_traffic = {
             "wide": ("flash_wide_bf16_kernel<causal>",
                      profile_traffic("flash_wide_bf16_b4_h32_n4096_d64.md", "flash_wide_bf16_kernel<causal>")),
-            "persistent": ("flash_fwd_bf16_kernel<64, causal>", None),
         }.get(os.environ.get("RT_ATTN_BF16_PREFILL", ""),
               ("flash_tile_bf16_kernel<64, causal, direct>",
                profile_traffic("flash_tile_bf16_b4_h32_n4096_d64.md", "flash_tile_bf16_kernel<64,causal,direct>")))

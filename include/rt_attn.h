@@ -220,7 +220,7 @@ int rt_flash_forward_window_bnhd_bf16_dev(void *stream, const rt_attention_shape
 
 /* No counterpart in the reference: a switch for measurements and tests.  which = 0 lets the library choose between
  * its bf16 prefill kernels (the default), 1 forces the tile kernel, 2 the persistent kernel where it applies (head
- * dim 64 / 128, no per-sequence lengths), 3 the kernel with 64 query rows per wave where it applies (head dim 64,
+ * dim 128, no per-sequence lengths; elsewhere the tile kernel), 3 the kernel with 64 query rows per wave where it applies (head dim 64,
  * mask none or causal; elsewhere the tile kernel).  Process-wide; until it is called the value is taken, once, from
  * RT_ATTN_BF16_PREFILL=tile|persistent|wide in the environment.  Returns RT_ERR_UNSUPPORTED for another value. */
 int rt_debug_force_bf16_prefill_kernel(int which);

@@ -1263,7 +1263,7 @@ static int flash_bf16_common(void* stream, const rt_attention_shape* shape, uint
     bool persistent = shape->dim == 128 && shape->seq >= 512 && jobs256 >= (uint64_t)g_num_cus && mask != rt::kMaskVarlenCausal;
     const PrefillKernel forced = prefill_kernel_override();
     if (forced == PrefillKernel::kTile || forced == PrefillKernel::kWide) persistent = false;
-    if (forced == PrefillKernel::kPersistent && (shape->dim == 64 || shape->dim == 128)) persistent = true;
+    if (forced == PrefillKernel::kPersistent && shape->dim == 128 && mask != rt::kMaskVarlenCausal) persistent = true;
     if (mask == rt::kMaskPadding && shape->seq > (uint64_t)rt::kFlashBf16MaxPaddingKeys) persistent = false;
     if (persistent) {  // that kernel addresses the rows of one (batch, head) slab with 32-bit byte offsets
         const uint64_t pitch_b = (bnhd ? shape->heads : 1) * shape->dim * 2;
@@ -1324,9 +1324,7 @@ static int flash_bf16_common(void* stream, const rt_attention_shape* shape, uint
     p.v = (const uint16_t*)v;
     p.out = (uint16_t*)out;
     p.keep = keep;
-    p.seq_lens = seq_lens;
     p.ref_bc = ref_bc;
-    p.zero_padded_rows = zero_padded_rows;
     p.scale_log2e = scale * rt::kLog2eHost;
     p.lq = p.lo = lq;
     p.lkv = lkv;

@@ -148,12 +148,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void flash_fwd_bf16_kernel(FlashBf16Pa
     constexpr int NLD = BC / RPI / NWAVES;   // load instructions per wave, per matrix, per tile
     constexpr int KS = HD / 16;              // contraction steps of the score product
     constexpr int DT = HD / 32;              // 32-row tiles of O^T
-    constexpr bool kCausal = (MODE == kMaskCausal) || (MODE == kMaskVarlenCausal);
-    // Two barriers per step (see the header) at head dim 128.  At head dim 64 a matrix cluster is half as long as a
-    // softmax cluster, the pipe is no longer what paces the waves, and the older scheme measures 2-3 % faster: a
-    // barrier behind every cluster, waves 4-7 held one cluster behind waves 0-3 by one extra barrier at either end
-    // of a job.
-    constexpr bool kLockstep = (HD == 64);
+    constexpr bool kCausal = MODE == kMaskCausal;
     static_assert(NLD >= 1 && NLD <= NITEMS && BC % (RPI * NWAVES) == 0, "tile load split");
 
     // [K stage 0][K stage 1][V stage 0][V stage 1]: with this order every operand read of the steady state
@@ -168,8 +163,8 @@ __global__ __launch_bounds__(NTHREADS, 1) void flash_fwd_bf16_kernel(FlashBf16Pa
 
     // slot swizzles (see the header): K rows are read 16 at a time at one slot (b128), V rows 4 at a
     // time over 4 adjacent slots (transposing b64 reads)
-    auto swz_k = [](int r) { return HD == 128 ? (r & 15) : ((r >> 1) & 7); };
-    auto swz_v = [](int r) { return HD == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
+    auto swz_k = [](int r) { return r & 15; };
+    auto swz_v = [](int r) { return 4 * (r & 3); };
     auto swz_o = [](int r) { return r & (SPR - 1); };
 
     // ---- jobs.  A job is one (batch*head, 256-row query tile); every workgroup walks its own list.
@@ -226,7 +221,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void flash_fwd_bf16_kernel(FlashBf16Pa
     // index also occupies, so operand ks (dt) of a lane sits at base ^ 32*ks (base ^ 64*dt): one register
     // per matrix, one XOR per read.  The stage bit is toggled into the bases once per step; item and
     // half-item offsets are immediates.
-    static_assert(HD == 128 || HD == 64, "operand address algebra below");
+    static_assert(HD == 128, "operand address algebra below");
     // K A-operand: row col of an item, slot (2ks + hh) ^ swz_k(col)
     uint32_t k_base = (uint32_t)(col * ROWB + ((hh ^ swz_k(col)) * 16));
     // V^T A-operand: lane j of a 16-group addresses row j/4 (+4hh), 4 columns; slot (4dt + low) ^ swz_v(row)
@@ -333,11 +328,9 @@ __global__ __launch_bounds__(NTHREADS, 1) void flash_fwd_bf16_kernel(FlashBf16Pa
         Kg = (const unsigned char*)(p.k + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride);
         Vg = (const unsigned char*)(p.v + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride);
         Og = p.out + (size_t)b * p.lo.batch_stride + (size_t)h * p.lo.head_stride;
-        n_keys = N;  // keys that exist for this sequence
-        if (MODE == kMaskVarlenCausal) n_keys = min(N, max(0, p.seq_lens[b]));
+        n_keys = N;
         int kv_end = n_keys;
         if (kCausal) kv_end = min(n_keys, q0 + BR);
-        if (MODE == kMaskVarlenCausal && q0 >= n_keys) kv_end = 0;  // a tile of padded query rows
         n_steps = (kv_end + BC - 1) / BC;
         // The wave's 32 query rows are one contiguous block: fetched in whole rows (load n, lane l: row
         // RPI*n + l/SPR, slot l%SPR), which costs the address unit a quarter of what row-per-lane loads
@@ -518,10 +511,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void flash_fwd_bf16_kernel(FlashBf16Pa
     // barriers the first publishes this wave's share of the next tile (vmcnt(0) before it).
     auto cluster_edge = [&](bool after_c, int i) {
         __builtin_amdgcn_sched_barrier(0);
-        if (kLockstep) {
-            if (after_c && i == 2) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's share has landed
-            __builtin_amdgcn_s_barrier();
-        } else if (i >= 2 && (grp == 1) == after_c) {
+        if (i >= 2 && (grp == 1) == after_c) {
             if (i == 2) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
             __builtin_amdgcn_s_barrier();
         }
@@ -623,12 +613,10 @@ __global__ __launch_bounds__(NTHREADS, 1) void flash_fwd_bf16_kernel(FlashBf16Pa
 
         // an item needs masking when its last key lies past the last existing key or past the wave's first row
         const int mask_from = kCausal ? min(n_keys - 1, qw) : n_keys - 1;
-        if (kLockstep && grp == 1) cluster_barrier();  // the second group runs one cluster behind the first
         if (n_steps > 0) {
 #pragma unroll
             for (int ks = 0; ks < KS; ks++) k_read_one(std::integral_constant<int, 0>{}, 0, ks);  // K(0)
         }
-        if (kLockstep) cluster_barrier();
         __builtin_amdgcn_sched_barrier(0);
         // With a causal mask the job's last key tile starts past the last row of the waves that own the upper
         // half of the query tile: for them every score of that step would be masked.  Such a wave finishes its
@@ -649,7 +637,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void flash_fwd_bf16_kernel(FlashBf16Pa
         }
         if (dead_last) {
 #pragma unroll 1
-            for (int cl = 0; cl < (kLockstep ? 2 * NITEMS : 2); cl++) cluster_barrier();
+            for (int cl = 0; cl < 2; cl++) cluster_barrier();
             k_base ^= (uint32_t)TILE_B;
             v_base ^= (uint32_t)TILE_B;
         }
@@ -658,13 +646,11 @@ __global__ __launch_bounds__(NTHREADS, 1) void flash_fwd_bf16_kernel(FlashBf16Pa
             v_base ^= (uint32_t)TILE_B;
         }
         cluster_barrier();  // every wave has read its last operands: LDS is free for the output and the next job
-        if (kLockstep && grp == 0) cluster_barrier();  // (the first group waits for the second to finish)
 
         // ---- this job's output.  Stage 1 of LDS is free (the next job's first tile goes to stage 0): each
         // wave parks its 32 normalised rows there, swizzled, and streams them out as whole rows.
         const int qw_out = qw;
         uint16_t* __restrict__ og_out = Og;
-        const bool padded_row = (MODE == kMaskVarlenCausal) && (q_row >= n_keys);
         job = job_of_round(++round);
         if (job >= 0) begin_job(job);  // its loads travel while the output is normalised and stored
 
@@ -688,9 +674,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void flash_fwd_bf16_kernel(FlashBf16Pa
                 float o[4];
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    float x = good ? acc_o[dt][4 * j + r] * inv_l : quiet_nan();
-                    if (padded_row) x = p.zero_padded_rows ? 0.0f : quiet_nan();
-                    o[r] = x;
+                    o[r] = good ? acc_o[dt][4 * j + r] * inv_l : quiet_nan();
                 }
                 u32x2_t wv = {cvt_pk_bf16(o[0], o[1]), cvt_pk_bf16(o[2], o[3])};
                 *(u32x2_t __attribute__((address_space(3)))*)(uintptr_t)(park ^ (uint32_t)(16 * (4 * dt + j))) = wv;
@@ -719,9 +703,6 @@ hipError_t launch_hd(hipStream_t stream, const FlashBf16Params& p, dim3 grid, di
         case kMaskNone: hipLaunchKernelGGL((flash_fwd_bf16_kernel<HD, kMaskNone>), grid, block, 0, stream, p); break;
         case kMaskCausal: hipLaunchKernelGGL((flash_fwd_bf16_kernel<HD, kMaskCausal>), grid, block, 0, stream, p); break;
         case kMaskPadding: hipLaunchKernelGGL((flash_fwd_bf16_kernel<HD, kMaskPadding>), grid, block, 0, stream, p); break;
-        case kMaskVarlenCausal:
-            hipLaunchKernelGGL((flash_fwd_bf16_kernel<HD, kMaskVarlenCausal>), grid, block, 0, stream, p);
-            break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -794,11 +775,7 @@ hipError_t launch_flash_bf16(hipStream_t stream, const FlashBf16Params& p) {
     size_t n_jobs = (size_t)n_qtiles * p.batch * p.heads;
     size_t workers = p.n_workers > 0 ? (size_t)p.n_workers : 256;
     dim3 grid((unsigned)(n_jobs < workers ? n_jobs : workers)), block(NTHREADS);
-    switch (p.dim) {
-        case 64: return launch_hd<64>(stream, p, grid, block);
-        case 128: return launch_hd<128>(stream, p, grid, block);
-        default: return hipErrorInvalidValue;
-    }
+    return p.dim == 128 ? launch_hd<128>(stream, p, grid, block) : hipErrorInvalidValue;
 }
 
 }  // namespace rt

@@ -87,18 +87,16 @@ struct FlashBf16Params {
     const uint16_t* v;
     uint16_t* out;
     const uint8_t* keep;      // kMaskPadding
-    const int32_t* seq_lens;  // kMaskVarlenCausal: device int32[batch]
     int batch, heads, kv_heads, group;
     int seq, dim;
     int mask;
     int ref_bc;
-    int zero_padded_rows;
     float scale_log2e;  // (1/sqrt(dim)) * log2(e)
     int n_workers;      // persistent workgroups to launch: the number of CUs
     int rank_major;     // the order in which an XCD's jobs are dealt (plan_flash_bf16)
     TensorLayout lq, lkv, lo;  // layouts of q, of k and v, of out; seq * row_pitch * 2 bytes must stay below 2^32
 };
-// dim in {64, 128}; a padding mask (kMaskPadding) of at most kFlashBf16MaxPaddingKeys keys.
+// dim 128, masks none, causal and padding; a padding mask (kMaskPadding) of at most kFlashBf16MaxPaddingKeys keys.
 constexpr int kFlashBf16MaxPaddingKeys = 65536;
 // Chooses the order the jobs are dealt in; returns the load of the busiest worker, in steps of 128 keys for 256 rows.
 float plan_flash_bf16(FlashBf16Params& p);
