@@ -519,7 +519,7 @@ def main():
                             args.steps, args.warmup, spread_steps=0)
             single[str(kv_len)] = {"us_per_call": t1.mean_ms * 1e3,
                                    "GB/s": (2 * Hkv * kv_len * Dd * 2 + 2 * Hq * Dd * 2) / (t1.mean_ms * 1e-3) / 1e9}
-        decode["single_sequence"] = dict(single, note="rt_gqa_decode_online_bf16, 32 q / 8 kv heads, D=128: two launches "
+        decode["single_sequence"] = dict(single, note="rt_gqa_decode_online_bf16, 32 q / 8 kv heads, D=128: one launch "
                                                       "per call, issued back to back from the host")
         # several new positions of ONE sequence against its long cache, each causal to itself (the reference's
         # gqa_decode_batched_f32 call shape): the keys are cut into spans, a second kernel folds the partials.  Every
