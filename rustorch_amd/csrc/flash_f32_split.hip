@@ -279,7 +279,9 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             load_tile(1);
             store_tile(lds + KBUF, v_lds + VBUF);
         }
-        const bool uncarried = __syncthreads_or(!(chk < kSplitMost));  // seen already: no step of the loop below
+        // Seen already: no step of the loop below, straight to the second pass, whose first tile may overwrite what a late
+        // wave still reads here for scores that nobody uses then.
+        const bool uncarried = __syncthreads_or(!(chk < kSplitMost));
         f32x16_t s_next;
         zero16(s_next);
         read_plane(lds, 2);
