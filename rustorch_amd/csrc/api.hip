@@ -1529,7 +1529,8 @@ RT_API int rt_mha_forward_masked_bf16_dev(void* stream, const void* q, const voi
     int rc = ensure_device(err);
     if (rc) return rc;
     if (!rt::flash_tile_bf16_supported((int)head_dim) || (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) != 0 ||
-        !rt::flash_tile_bf16_addressable((long long)t_kv, (long long)(heads * head_dim))) {
+        !rt::flash_tile_bf16_addressable((long long)t_kv, (long long)(heads * head_dim)) ||
+        (mask_len && !rt::flash_tile_bf16_bias_addressable((long long)t_kv))) {
         // head dims and alignments the matrix-core kernel does not cover: one workgroup per query row, any speed
         if (t_kv == 0) return rt_buf_zero(out, q_expected * 2, stream, err);
         rt::AttnRowsParams r{};

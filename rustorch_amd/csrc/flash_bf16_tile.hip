@@ -90,6 +90,7 @@ struct TileCfg {
     static constexpr int STAGE_BYTES = KT * DP * 2;
     static constexpr int LDS_BYTES_DIRECT = 4 * STAGE_BYTES > 4 * REGION ? 4 * STAGE_BYTES : 4 * REGION;
     static constexpr int OCC_DIRECT = DP <= 64 ? 3 : 2;
+    static constexpr int BIAS_BYTES = 32 * 32 * 4;  // a wave's bias values of an item: 32 rows of 32 keys
 };
 
 // 16 bytes per lane from a buffer straight into LDS: lane l lands at LDS byte address lds_block + 16 l (lds_block is
@@ -102,6 +103,15 @@ __device__ __forceinline__ void t_buffer_to_lds(const u32x4_t& rsrc, uint32_t la
     const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
     const uint32_t so = __builtin_amdgcn_readfirstlane(tile_off);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so)
+                 : "memory");
+}
+// the same, 4 bytes per lane: lane l lands at lds_block + 4 l
+__device__ __forceinline__ void t_buffer_to_lds_b32(const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
+    const uint32_t so = __builtin_amdgcn_readfirstlane(tile_off);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
                  :
                  : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so)
                  : "memory");
@@ -141,7 +151,7 @@ __device__ __forceinline__ u32x4_t t_make_rsrc(const void* base, uint32_t bytes)
 // moved by that many keys, as for a span of SPLIT), and an item that holds keys below some row's window is masked on
 // that side as well.
 //
-// DIRECT (head dim 64 or 128 exactly, no bias, no key-padding vector): the tiles travel from memory straight into LDS
+// DIRECT (head dim 64 or 128 exactly, no key-padding vector): the tiles travel from memory straight into LDS
 // (buffer_load_dwordx4 ... lds) instead of through registers and LDS writes.  After a tile's barrier the waves request
 // K(t+2) and V(t+1) into the stages K(t) and V(t-1) have just left and wait for their own requests ahead of the next
 // tile's barrier.  LDS rows are unpadded (a landing block of 1 KB is contiguous) and their 16-byte slots are XORed
@@ -150,10 +160,10 @@ __device__ __forceinline__ u32x4_t t_make_rsrc(const void* base, uint32_t bytes)
 // N=1024: 52.3 -> 49.3 us), 7-9 % on long ones (B=4 H=32 N=4096: 306 -> 283 us), 4-7 % at head dim 128; three stages
 // per matrix or four workgroups per CU (head dim 64) are no faster.
 template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, bool DIRECT = false>
-__global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIRECT : ((BIAS && DP == 64) ? 2 : TileCfg<DP>::OCC)) void flash_tile_bf16_kernel(FlashTileParams p) {
+__global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (DIRECT ? TileCfg<DP>::OCC_DIRECT : TileCfg<DP>::OCC)) void flash_tile_bf16_kernel(FlashTileParams p) {
     static_assert(!SPLIT || (PACKED && !BIAS && MODE == kMaskCausal), "the split over the keys serves the chunked decode");
     static_assert(!WIN || (!PACKED && !BIAS && !SPLIT && MODE == kMaskCausal), "the window is a causal mask's");
-    static_assert(!DIRECT || ((DP == 64 || DP == 128) && !BIAS && MODE != kMaskPadding), "tiles straight into LDS: head dim 64 or 128 exactly");
+    static_assert(!DIRECT || ((DP == 64 || DP == 128) && MODE != kMaskPadding), "tiles straight into LDS: head dim 64 or 128 exactly");
     using Cfg = TileCfg<DP>;
     constexpr int KT = Cfg::KT, LDK = Cfg::LDK, LDV = Cfg::LDV, NI = Cfg::NI, TTHREADS = Cfg::THREADS;
     constexpr int KS = DP / 16;        // contraction steps of the score product
@@ -168,9 +178,10 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
     // Head dims above 128 do not have the registers for two score tiles and their operands in flight (O alone is 128
     // registers), nor does head dim 128 with a bias (two items' bias values) or with a key-padding mask: there an
     // item runs its three phases one after the other, and K is parked with V.
-    constexpr bool PIPE = DP <= 128 && !((BIAS || MODE == kMaskPadding) && DP == 128);
+    constexpr bool PIPE = DP <= 128 && !((((BIAS && !DIRECT) || MODE == kMaskPadding)) && DP == 128);
 
-    __shared__ alignas(DIRECT ? 1024 : 16) unsigned char lds[DIRECT ? Cfg::LDS_BYTES_DIRECT : Cfg::LDS_BYTES];
+    constexpr int kTilesLds = DIRECT ? Cfg::LDS_BYTES_DIRECT : Cfg::LDS_BYTES;  // BIAS: the four waves' bias values behind the tiles
+    __shared__ alignas(DIRECT || BIAS ? 1024 : 16) unsigned char lds[BIAS ? (kTilesLds + 1023) / 1024 * 1024 + 4 * Cfg::BIAS_BYTES : kTilesLds];
     uint16_t* const Ks = (uint16_t*)lds;                      // [2][KT * LDK]
     uint16_t* const Vs = (uint16_t*)lds + 2 * KT * LDK;       // [2][KT * LDV]
     // DIRECT: [K stage 0][K stage 1][V stage 0][V stage 1], rows of ROWB bytes without padding
@@ -449,7 +460,6 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
         // ---- this lane's query row
         const int r = q0 + 32 * wq + col;
         const int s_pos = G > 1 ? r / G : r;
-        const int g = r - s_pos * G;
         const bool exists = r < rows_total;
         valid = exists && s_pos < n_q;
         int lim = n_keys - 1;  // last key this row sees
@@ -476,6 +486,55 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
         const int r_q = min(r, rows_total - 1);
         const int s_q = G > 1 ? r_q / G : r_q;
         const size_t q_off = (size_t)b * p.lq.batch_stride + (size_t)(h0 + (r_q - s_q * G)) * p.lq.head_stride + (size_t)s_q * p.lq.row_pitch;
+
+        // BIAS (scores = (q . k) * scale + bias, crates/rustorch-nn/src/attention.rs:378-392, kept in the natural domain so
+        // that a bias of -1e4 weighs as it does in the reference): f32 rows of seq_kv per (batch, head), or one matrix for
+        // all.  An item's 32 rows of 32 keys go from memory to the wave's own 4 KB of LDS as whole 128-byte pieces of a row
+        // (8 rows a load instruction, or 2 where the rows are not 16-byte aligned), and from there into the order the scores
+        // sit in; the 16-byte slots of a row are XORed with bits of the row, as those of a K tile of 128-byte rows.  Read
+        // from its row in memory by each lane, 16 bytes of 32 rows at a time, the bias kept the address unit busy for half
+        // of the launch and the waves waiting for 54 % of theirs: B=4 H=16 T=1024 hd=64 47.4 -> 28.3 us, 1023 keys (4-byte
+        // requests) 93.9 -> 34.9, one matrix a head at B=4 H=16 T=770 hd=96 119 -> 58.3.  Keys behind the last one read the next row, or zeros
+        // behind the tensor: those scores are masked.
+        u32x4_t bias_rsrc = {0u, 0u, 0u, 0u};
+        uint32_t bias_lane[2] = {0u, 0u}, bias_at = 0, bias_step = 0;
+        const uint32_t bias_lds = BIAS ? (uint32_t)((kTilesLds + 1023) / 1024 * 1024 + wave * Cfg::BIAS_BYTES) : 0u;
+        const bool bias_vec4 = BIAS && p.bias_vec4;
+        if constexpr (BIAS) {
+            const int r_first = q0 + 32 * wq, n_rows = max(min(32, rows_total - r_first), 0);
+            const float* const bb = p.bias + ((size_t)b * p.heads + h0) * (size_t)p.bias_bh_stride + (size_t)min(r_first, rows_total - 1) * (size_t)p.seq_kv;
+            const uint32_t pitch = (uint32_t)p.seq_kv * 4u;
+            bias_rsrc = t_make_rsrc(bb, (uint32_t)n_rows * pitch);
+            if (bias_vec4) {  // instruction n: rows 8 n + lane / 8
+                const int row = lane >> 3, slot = (lane & 7) ^ (row >> 1);
+                bias_lane[0] = (uint32_t)row * pitch + 16u * (uint32_t)slot;
+                bias_lane[1] = (uint32_t)row * pitch + 16u * (uint32_t)(slot ^ 4);
+                bias_step = 8u * pitch;
+            } else {  // instruction n: rows 2 n + lane / 32
+                bias_lane[0] = (uint32_t)(lane >> 5) * pitch;
+                bias_lane[1] = 4u * (uint32_t)(lane & 31);
+                bias_step = 2u * pitch;
+            }
+            bias_at = bias_lds + (uint32_t)(col * 128 + ((hh ^ ((col >> 1) & 7)) * 16));
+        }
+        auto bias_request = [&](int item) __attribute__((always_inline)) {
+            const uint32_t k_off = 128u * (uint32_t)item;
+            if (bias_vec4) {
+#pragma unroll
+                for (int n = 0; n < 4; n++)
+                    t_buffer_to_lds(bias_rsrc, bias_lane[n & 1], k_off + (uint32_t)n * bias_step, lds_base + bias_lds + 1024u * (uint32_t)n);
+            } else {
+#pragma unroll
+                for (int n = 0; n < 16; n++)
+                    t_buffer_to_lds_b32(bias_rsrc, bias_lane[0] + (bias_lane[1] ^ (16u * (uint32_t)(n & 7))), k_off + (uint32_t)n * bias_step,
+                                        lds_base + bias_lds + 256u * (uint32_t)n);
+            }
+        };
+        auto bias_read = [&](f32x4_t (&bv)[4]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) bv[j] = *(const f32x4_t*)(lds + (bias_at ^ (uint32_t)(32 * j)));
+        };
+        if constexpr (BIAS) bias_request(0);
 
         // Mask::Padding hiding the reference's whole first key tile: every row NaN (the tiled recurrence of
         // cpu_forward.rs:268-425 takes exp(-inf - (-inf)) on that tile and never recovers)
@@ -528,12 +587,18 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
             else return Vs + st * KT * LDV + item * 32 * LDV + v_off;
         };
 
-        // bias rows of this lane's query: f32 [seq_q, seq_kv] per (batch, head) or one for all
-        const float* bias_row = nullptr;
-        if (BIAS) bias_row = p.bias + ((size_t)b * p.heads + (h0 + g)) * (size_t)p.bias_bh_stride + (size_t)s_pos * (size_t)p.seq_kv;
 
         // K(0), V(0) -> stage 0, K(1) -> stage 1; then the register sets take K(2) .. K(1 + PF) and V(1) .. V(PF)
         // (K(j) travels in set j % PF, and so does V(j))
+        f32x4_t bv[4] = {};  // bias values of the item whose softmax step comes next
+        auto bias_first = [&]() __attribute__((always_inline)) {
+            if constexpr (BIAS) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                bias_read(bv);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                bias_request(1);
+            }
+        };
         if constexpr (DIRECT) {
             // tile 0 and K(1) have landed (and the queries); V rows of tile 0 past the last key, requested before the
             // lengths were known, are zeroed by the lane that fetched them
@@ -543,11 +608,13 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
                 for (int n = 0; n < NLD; n++)
                     if (dl_row + 4 * RPI * n >= n_keys) *(u32x4_t*)(lds + 2 * STAGE_B + (wave + 4 * n) * 1024 + 16 * lane) = u32x4_t{0u, 0u, 0u, 0u};
             }
+            bias_first();
         } else {
             park_k(kreg[0], 0);
             park_v(std::integral_constant<int, 0>{}, 0);
             keep_cur = keep_next;
             if (PIPE) park_k(k1, 1);
+            bias_first();
             {
                 auto prefetch = [&](auto i_c) __attribute__((always_inline)) {
                     constexpr int I = decltype(i_c)::value;  // 0 .. PF - 1
@@ -564,27 +631,8 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
         __syncthreads();
 
         // ---- pieces of a step
-        // bias values of an item (scores = (q . k) * scale + bias, crates/rustorch-nn/src/attention.rs:378-392, kept in
-        // the natural domain so that a bias of -1e4 weighs as it does in the reference): requested a step ahead
-        auto bias_fetch = [&](int k0, f32x4_t (&bv)[4]) __attribute__((always_inline)) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int kb = k0 + 8 * j + 4 * hh;
-                f32x4_t x = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (valid) {
-                    if (p.bias_vec4 && kb + 3 < n_keys) {
-                        x = *(const f32x4_t*)(bias_row + kb);
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            if (kb + e < n_keys) x[e] = bias_row[kb + e];
-                    }
-                }
-                bv[j] = x;
-            }
-        };
         // the bias, then the masks, on the scores of the item whose keys start at k0 (item `it` of its tile)
-        auto mask_item = [&](int it, int k0, f32x16_t& sc, const f32x4_t (&bv)[4]) __attribute__((always_inline)) {
+        auto mask_item = [&](int it, int k0, f32x16_t& sc) __attribute__((always_inline)) {
             if (BIAS) {
 #pragma unroll
                 for (int i = 0; i < 16; i++) sc[i] = __builtin_fmaf(sc[i], p.scale, bv[i >> 2][i & 3]);
@@ -642,28 +690,24 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
         f32x16_t s_a, s_b;        // S(j), made in step j - 1, and S(j + 1)
         bf16x8_t p_a[2], p_b[2];  // P(j - 1) and P(j)
         p_a[0] = p_a[1] = p_b[0] = p_b[1] = __builtin_bit_cast(bf16x8_t, u32x4_t{0u, 0u, 0u, 0u});
-        f32x4_t bv_a[4] = {}, bv_b[4] = {};  // bias values of item j and of item j + 1
 
         // S(0), before the pipeline starts
         {
 #pragma unroll
             for (int i = 0; i < 16; i++) s_a[i] = s_b[i] = 0.0f;
-            if (BIAS) bias_fetch(0, bv_a);
             if (PIPE && n_it > 0) {
 #pragma unroll
                 for (int ks = 0; ks < KS; ks++)
                     s_a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, load_op(2 * ks, k_at(0, 0), nullptr)), qreg[ks], s_a, 0, 0, 0);
                 // The running max starts at the max of item 0, taken here, so that the first step already runs the
-                // fast path (without it the step would form P twice and rescale an O that is still zero).  The masks
-                // are applied first; the step applies them again, which changes nothing.  (Not with a bias: adding it
-                // is part of the mask step and must happen once.)
-                if (!BIAS) {
-                    mask_item(0, 0, s_a, bv_a);
-                    const float m0 = t_max_with_other_half(t_max16(s_a));
-                    if (m0 > neg_inf()) {  // (false for -inf and for NaN: such a row waits for the slow path)
-                        m_run = m0;
-                        neg_mc = -m0 * cc;
-                    }
+                // fast path (without it the step would form P twice and rescale an O that is still zero).  The bias and the
+                // masks go on a copy: the step applies them to the scores.
+                f32x16_t s_0 = s_a;
+                mask_item(0, 0, s_0);
+                const float m0 = t_max_with_other_half(t_max16(s_0));
+                if (m0 > neg_inf()) {  // (false for -inf and for NaN: such a row waits for the slow path)
+                    m_run = m0;
+                    neg_mc = -m0 * cc;
                 }
             }
         }
@@ -710,15 +754,30 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
             neg_mc = (m_new == neg_inf()) ? (valid ? __uint_as_float(0x7f800000u) : 0.0f) : -mc;
             exp_plain(sc, -mc, w, part);
         };
+        // BIAS: the next item's bias values leave LDS at the end of a step, and the values of the item behind it are
+        // requested over them.  WAIT: requests made since that may still be on their way.
+        auto bias_take = [&](auto wait_c) __attribute__((always_inline)) {
+            if constexpr (BIAS) {
+                constexpr int WAIT = decltype(wait_c)::value;
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAIT) : "memory");
+                bias_read(bv);
+            }
+        };
+        auto bias_ahead = [&](int k0) __attribute__((always_inline)) {
+            if constexpr (BIAS) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                bias_request((k0 >> 5) + 2);
+            }
+        };
         // An item whose three phases run one after the other (head dims above 128): S, the softmax step, P.V
         auto step_simple = [&](int it, int k0, const uint16_t* kp, const uint16_t* vp) __attribute__((always_inline)) {
-            if (BIAS) bias_fetch(k0, bv_a);
 #pragma unroll
             for (int i = 0; i < 16; i++) s_a[i] = 0.0f;
 #pragma unroll
             for (int ks = 0; ks < KS; ks++)
                 s_a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8_t*)(kp + 16 * ks), qreg[ks], s_a, 0, 0, 0);
-            mask_item(it, k0, s_a, bv_a);
+            mask_item(it, k0, s_a);
+            bias_take(std::integral_constant<int, 0>{});
             uint32_t w[8];
             float part;
             exp_plain(s_a, neg_mc, w, part);
@@ -726,6 +785,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
             l_run += part;
             p_a[0] = __builtin_bit_cast(bf16x8_t, u32x4_t{w[0], w[1], w[2], w[3]});
             p_a[1] = __builtin_bit_cast(bf16x8_t, u32x4_t{w[4], w[5], w[6], w[7]});
+            bias_ahead(k0);
             drain(vp);
         };
 
@@ -744,10 +804,8 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
         // The fences between the groups name the vector values and the B operands of the matrix instructions on
         // either side, which is what keeps each matrix instruction inside its group.
         auto step = [&](int it, int k0, const uint16_t* kp, const uint16_t* vp, f32x16_t& s_cur, f32x16_t& s_next,
-                        bf16x8_t (&p_prev)[2], bf16x8_t (&p_new)[2], f32x4_t (&bv_cur)[4],
-                        f32x4_t (&bv_next)[4]) __attribute__((always_inline)) {
-            if (BIAS) bias_fetch(k0 + 32, bv_next);
-            mask_item(it, k0, s_cur, bv_cur);
+                        bf16x8_t (&p_prev)[2], bf16x8_t (&p_new)[2], auto wait_c) __attribute__((always_inline)) {
+            mask_item(it, k0, s_cur);
 #pragma unroll
             for (int i = 0; i < 16; i++) s_next[i] = 0.0f;
             u32x4_t ops[NM];
@@ -788,6 +846,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
 #pragma unroll
             for (int gq = 0; gq < 6; gq++) {
                 if (gq + LOOK < 6) fetch_group(gq + LOOK);
+                if (gq == 4) bias_take(wait_c);
                 multiply_group(gq);
                 const int half = gq / 3;
                 if (gq % 3 == 0) {
@@ -817,6 +876,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
                 fence_b(gq);
                 if (gq + 1 < 6) fence_b(gq + 1);
             }
+            bias_ahead(k0);
             float part = part0 + part1;
             if (__builtin_expect(__any(!(part <= kTileTrigSum)), 0)) raise_max_and_redo(s_cur, w, part);
             l_run += part;
@@ -825,14 +885,10 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
         };
         // a step whose results are moved back into the first of each pair
         auto step_a = [&](int it, int k0, const uint16_t* kp, const uint16_t* vp) __attribute__((always_inline)) {
-            step(it, k0, kp, vp, s_a, s_b, p_a, p_b, bv_a, bv_b);
+            step(it, k0, kp, vp, s_a, s_b, p_a, p_b, std::integral_constant<int, 0>{});
             s_a = s_b;
             p_a[0] = p_b[0];
             p_a[1] = p_b[1];
-            if (BIAS) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) bv_a[j] = bv_b[j];
-            }
         };
         // slot j of the walk: a step while the wave has items left, then once the P.V of its last item
         auto slot = [&](int j, int it, const uint16_t* kp, const uint16_t* vp) __attribute__((always_inline)) {
@@ -848,8 +904,10 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
             if constexpr (DIRECT) {
                 // K(t+2) over K(t), V(t+1) over V(t-1): requested now that every wave is done with those, awaited
                 // (vmcnt) ahead of the next tile's barrier
-                if (t + 2 < n_tiles) dl_tile(Kd, dl_k, (uint32_t)(t + 2) * tile_bytes_g, (uint32_t)(st * STAGE_B));
-                if (t + 1 < n_tiles) dl_tile(Vd, dl_v, (uint32_t)(t + 1) * tile_bytes_g, (uint32_t)((2 + (st ^ 1)) * STAGE_B));
+                // (BIAS: always, so that a step knows how many requests follow that for its bias values; behind the last
+                // tiles they land zeros that nobody reads)
+                if (BIAS || t + 2 < n_tiles) dl_tile(Kd, dl_k, (uint32_t)(t + 2) * tile_bytes_g, (uint32_t)(st * STAGE_B));
+                if (BIAS || t + 1 < n_tiles) dl_tile(Vd, dl_v, (uint32_t)(t + 1) * tile_bytes_g, (uint32_t)((2 + (st ^ 1)) * STAGE_B));
             } else {
                 // (behind the last tiles these park and request copies of the last tile, which nobody reads)
                 park_k(kreg[KSET], st);
@@ -859,8 +917,15 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
             }
         };
         // what a wave does ahead of a tile's barrier: DIRECT waits for its own requests of a tile ago
-        auto meet = [&]() __attribute__((always_inline)) {
-            if constexpr (DIRECT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // (BIAS: all but those for bias values, the last the wave has made when `stepped` -- a step lies between them and
+        // the tile's requests)
+        auto meet = [&](auto stepped_c) __attribute__((always_inline)) {
+            if constexpr (DIRECT && BIAS && decltype(stepped_c)::value) {
+                if (bias_vec4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+            } else if constexpr (DIRECT) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            }
             __syncthreads();
         };
         // the same for a tile of which the wave walks every item: straight-line code, the pairs swapped from step to step
@@ -872,10 +937,10 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
             constexpr bool kLater = decltype(later_c)::value;
             const int k0 = t * KT;
             if (NI > 1) {
-                step(0, k0, k_at(st, 1), (!kLater && t == 0) ? v_at(st, 0) : v_at(st ^ 1, NI - 1), s_a, s_b, p_a, p_b, bv_a, bv_b);
-                meet();
+                step(0, k0, k_at(st, 1), (!kLater && t == 0) ? v_at(st, 0) : v_at(st ^ 1, NI - 1), s_a, s_b, p_a, p_b, std::integral_constant<int, 0>{});
+                meet(std::true_type{});
                 park_next(t, kset_c, vset_c, st_c);
-                step(1, k0 + 32, k_at(st ^ 1, 0), v_at(st, 0), s_b, s_a, p_b, p_a, bv_b, bv_a);
+                step(1, k0 + 32, k_at(st ^ 1, 0), v_at(st, 0), s_b, s_a, p_b, p_a, std::integral_constant<int, DIRECT ? 2 * NLD : 0>{});
             } else {
                 step_a(0, k0, k_at(st ^ 1, 0), (!kLater && t == 0) ? v_at(st, 0) : v_at(st ^ 1, 0));
                 __syncthreads();
@@ -889,7 +954,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
             // first item: the next item is item 1 of this tile (or item 0 of the next tile when a tile is one item);
             // the previous item is the last of tile t - 1 (at t = 0 there is none: P is zero, and V(0) stands in)
             slot(t * NI, 0, NI > 1 ? k_at(st, 1) : k_at(st ^ 1, 0), t == 0 ? v_at(st, 0) : v_at(st ^ 1, NI - 1));
-            meet();
+            meet(std::false_type{});
             park_next(t, kset_c, vset_c, st);
             if (NI > 1) {
                 slot(t * NI + 1, 1, k_at(st ^ 1, 0), v_at(st, 0));
@@ -950,6 +1015,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, DIRECT ? TileCfg<DP>::OCC_DIR
         }
         // a wave that walked every item of the workgroup still owes the last P.V
         if (PIPE && n_it == n_tiles * NI && n_it > 0) drain(v_at((n_tiles - 1) & 1, NI - 1));
+        if constexpr (BIAS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (requests behind the last item and the last tile)
         __syncthreads();  // the output rows are staged over the tiles
     }
     // (a workgroup without tiles still has its early requests in flight: they land in its LDS)
@@ -1651,7 +1717,8 @@ hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
                                   : launch_one<DP, kMaskCausal, false, true>(stream, p, grid);
     if (p.window > 0) return direct ? launch_one<DP, kMaskCausal, false, false, false, true, kDirect>(stream, p, grid)
                                     : launch_one<DP, kMaskCausal, false, false, false, true>(stream, p, grid);
-    if (p.bias) return launch_one<DP, kMaskNone, true, false>(stream, p, grid);
+    if (p.bias) return direct ? launch_one<DP, kMaskNone, true, false, false, false, kDirect>(stream, p, grid)
+                              : launch_one<DP, kMaskNone, true, false>(stream, p, grid);
     if (direct && !p.bias && p.mask == kMaskNone) return launch_one<DP, kMaskNone, false, false, false, false, kDirect>(stream, p, grid);
     if (direct && !p.bias && p.mask == kMaskCausal) return launch_one<DP, kMaskCausal, false, false, false, false, kDirect>(stream, p, grid);
     switch (p.mask) {
@@ -1672,6 +1739,8 @@ int flash_tile_bf16_workgroups(int dim) { return dim <= 64 ? 3 : (dim <= 128 ? 2
 bool flash_tile_bf16_addressable(long long seq_kv, long long row_pitch) {
     return seq_kv >= 0 && row_pitch > 0 && (unsigned long long)(seq_kv + 512) * (unsigned long long)row_pitch * 2ull < (1ull << 32);
 }
+// ... and the bias values of 32 rows likewise.
+bool flash_tile_bf16_bias_addressable(long long seq_kv) { return seq_kv < (1ll << 24); }
 
 // What the kernels take grid positions for heads by.
 static void set_grid_order(FlashTileParams& p, long long z) {
@@ -1711,7 +1780,7 @@ hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& par
     FlashTileParams p = params;
     if (p.batch == 0 || p.heads == 0 || p.seq_q == 0) return hipSuccess;
     if (!flash_tile_bf16_supported(p.dim) || p.pack < 1) return hipErrorInvalidValue;
-    if (p.bias && p.mask != kMaskNone) return hipErrorInvalidValue;
+    if (p.bias && (p.mask != kMaskNone || !flash_tile_bf16_bias_addressable(p.seq_kv))) return hipErrorInvalidValue;
     if (!flash_tile_bf16_addressable(p.seq_kv, p.lkv.row_pitch)) return hipErrorInvalidValue;
     if ((p.pack > 1 || p.decode_rows) && (p.bias || p.mask != kMaskCausal)) return hipErrorInvalidValue;  // packed rows: the chunked decode only
     if (p.window < 0 || (p.window > 0 && (p.pack > 1 || p.decode_rows || p.bias || p.mask != kMaskCausal || p.n_splits > 1))) return hipErrorInvalidValue;

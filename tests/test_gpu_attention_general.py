@@ -77,6 +77,30 @@ def test_masked_rows_and_edge_cases(oracle):
     assert np.array_equal(a1, a2), f"{int((a1 != a2).sum())} of {a1.size} elements differ"
 
 
+@pytest.mark.parametrize("d", [8, 32, 64, 80, 128, 256])
+@pytest.mark.parametrize("tq,tkv", [(1, 1), (31, 32), (33, 33), (64, 63), (128, 64), (129, 65), (100, 96), (161, 132), (40, 321)])
+@pytest.mark.parametrize("lead", [0, 1])
+def test_additive_mask_at_the_edges_of_items(oracle, d, tq, tkv, lead):
+    """Rows of 16- and of 4-byte alignment (`lead` elements ahead of the mask), one matrix for all and one a head; what
+    lies around the mask in memory is NaN, which no row may take in."""
+    b, h = 2, 3
+    rng = np.random.default_rng(tq + tkv)
+    for per_head in (False, True):
+        mask = rng.standard_normal((b * h, tq, tkv) if per_head else (tq, tkv)).astype(np.float32)
+        mask[rng.random(mask.shape) < 0.3] = -1.0e4
+        held = np.full(mask.size + lead + 600, np.nan, dtype=np.float32)
+        held[4 + lead:4 + lead + mask.size] = mask.ravel()
+        buf = dev(held)
+        bits = [bf16_round(seeded_normal(b * n * h * d, i)) for i, n in enumerate((tq, tkv, tkv))]
+        dq, dk, dv = (dev(x[0]) for x in bits)
+        dout = ra.HipStorage(bits[0][0].size * 2)
+        ra.mha_forward_masked_bf16_dev(dq, dk, dv, dout, b, tq, tkv, h, d, buf.ptr + 4 * (4 + lead), mask.size)
+        ra.synchronize()
+        got = oracle.bf16_to_f32(dout.download(np.uint16))
+        want = oracle.mha_forward_masked(*(x[1] for x in bits), b, tq, tkv, h, d, mask)
+        assert_bf16_parity(got, want, d, None, f"tq={tq} tkv={tkv} d={d} lead={lead} per_head={per_head}")
+
+
 def test_masked_bf16_errors():
     z = ra.HipStorage(1 << 16)
     with pytest.raises(ra.DeviceError) as ei:  # head dim above 512
