@@ -107,6 +107,16 @@ __device__ __forceinline__ void t_buffer_to_lds(const u32x4_t& rsrc, uint32_t la
                  : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so)
                  : "memory");
 }
+// the same for the lanes of `on` alone (what the others would have brought stays as it is in LDS); no branch around it
+__device__ __forceinline__ void t_buffer_to_lds_of(uint64_t on, const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
+    const uint32_t so = __builtin_amdgcn_readfirstlane(tile_off);
+    uint64_t all;
+    asm volatile("s_mov_b32 m0, %1\n\ts_and_saveexec_b64 %0, %5\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\ts_mov_b64 exec, %0"
+                 : "=&s"(all)
+                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so), "s"(on)
+                 : "memory", "scc");
+}
 // the same, 4 bytes per lane: lane l lands at lds_block + 4 l
 __device__ __forceinline__ void t_buffer_to_lds_b32(const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
     const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
@@ -122,6 +132,9 @@ __device__ __forceinline__ u32x4_t t_make_rsrc(const void* base, uint32_t bytes)
     return u32x4_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
                    (uint32_t)__builtin_amdgcn_readfirstlane(bytes), kBufferFlags};
 }
+
+// How K/V tiles come into LDS: through registers, or straight there with rows of DP columns or with rows of fewer.
+enum TileWay : int { kTilesRegs = 0, kTilesDirect = 1, kTilesDirectPart = 2 };
 
 // MODE: kMaskNone, kMaskCausal, kMaskPadding.  BIAS: an additive f32 score bias is applied (then MODE is kMaskNone).
 // PACKED: query rows run over (position, head of the GQA group) (then MODE is kMaskCausal and there is no bias).
@@ -151,19 +164,23 @@ __device__ __forceinline__ u32x4_t t_make_rsrc(const void* base, uint32_t bytes)
 // moved by that many keys, as for a span of SPLIT), and an item that holds keys below some row's window is masked on
 // that side as well.
 //
-// DIRECT (head dim 64 or 128 exactly, no key-padding vector): the tiles travel from memory straight into LDS
+// DIRECT (head dims up to 128, no key-padding vector): the tiles travel from memory straight into LDS
 // (buffer_load_dwordx4 ... lds) instead of through registers and LDS writes.  After a tile's barrier the waves request
 // K(t+2) and V(t+1) into the stages K(t) and V(t-1) have just left and wait for their own requests ahead of the next
 // tile's barrier.  LDS rows are unpadded (a landing block of 1 KB is contiguous) and their 16-byte slots are XORed
 // with bits of the row, as in flash_bf16.hip.  Same instructions on the same operands otherwise: the same bits.
 // Measured against the register path, interleaved in one process: 3-5 % on short or padded sequences (B=16 H=16
-// N=1024: 52.3 -> 49.3 us), 7-9 % on long ones (B=4 H=32 N=4096: 306 -> 283 us), 4-7 % at head dim 128; three stages
-// per matrix or four workgroups per CU (head dim 64) are no faster.
-template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, bool DIRECT = false>
-__global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (DIRECT ? TileCfg<DP>::OCC_DIRECT : TileCfg<DP>::OCC)) void flash_tile_bf16_kernel(FlashTileParams p) {
+// N=1024: 52.3 -> 49.3 us), 7-9 % on long ones (B=4 H=32 N=4096: 306 -> 283 us), 4-7 % at head dim 128, 10-11 % at 96 and
+// 80 (B=2 H=16 N=4096: 123.5 -> 111.8 and 119.6 -> 107.7), 5 % at 32 (58.4 -> 55.8); three stages per matrix or four
+// workgroups per CU (head dim 64) are no faster.  Head dims between the tile widths have a form of their own
+// (kTilesDirectPart), whose requests leave the lanes behind the head dim out: two scalar instructions a request, which
+// cost the masked form at head dim 64 6 % where the kernel of whole rows had them too (28.3 -> 29.9 us; a branch 31.1).
+template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs>
+__global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES ? TileCfg<DP>::OCC_DIRECT : TileCfg<DP>::OCC)) void flash_tile_bf16_kernel(FlashTileParams p) {
     static_assert(!SPLIT || (PACKED && !BIAS && MODE == kMaskCausal), "the split over the keys serves the chunked decode");
     static_assert(!WIN || (!PACKED && !BIAS && !SPLIT && MODE == kMaskCausal), "the window is a causal mask's");
-    static_assert(!DIRECT || ((DP == 64 || DP == 128) && MODE != kMaskPadding), "tiles straight into LDS: head dim 64 or 128 exactly");
+    static_assert(TILES == kTilesRegs || (DP <= 128 && MODE != kMaskPadding), "tiles straight into LDS: head dims up to 128, no key-padding vector");
+    constexpr bool DIRECT = TILES != kTilesRegs, WHOLE = TILES == kTilesDirect;
     using Cfg = TileCfg<DP>;
     constexpr int KT = Cfg::KT, LDK = Cfg::LDK, LDV = Cfg::LDV, NI = Cfg::NI, TTHREADS = Cfg::THREADS;
     constexpr int KS = DP / 16;        // contraction steps of the score product
@@ -241,26 +258,60 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (DIREC
         ld_off[n] = ((uint32_t)row * kv_pitch + (ld_on[n] ? (uint32_t)(8 * ch) : 0u)) * 2u;
     }
     u32x4_t k1[NL];
-    // DIRECT: a wave's load instruction fills 1 KB of LDS (RPI = 8 rows at head dim 64, 4 at 128), lane l the 16 bytes
-    // at 16 l; instruction n of wave w fills block w + 4 n of a stage.  Bank conflicts are avoided by an XOR of the
-    // 16-byte slot index with bits of the row (K rows are read 16 at a time at one slot, V rows 4 at a time over 4
-    // adjacent slots by the transposing reads), applied on the way in: the lane fetches the slot that belongs at its
-    // LDS position.
+    // DIRECT: a wave's load instruction fills 1 KB of LDS with 64 chunks of 16 bytes, lane l the 16 bytes at 16 l;
+    // instruction n of wave w fills block w + 4 n of a stage: chunk 64 (w + 4 n) + l, which is slot chunk % SPR of row
+    // chunk / SPR.  Bank conflicts are avoided by an XOR of the slot index with bits of the row (K rows are read 16 at a
+    // time at one slot, V rows 4 at a time over 4 adjacent slots by the transposing reads; four rows of 64 or of 192 bytes
+    // start at four different quarters of the banks, which is all that V asks for), applied on the way in: the lane fetches
+    // the slot that belongs at its LDS position.  Slots behind the head dim are not requested: they are zero from the start.
     constexpr int SPR = DP / 8;                // 16-byte slots per row
-    constexpr int RPI = 64 / (SPR > 64 ? 64 : SPR);  // rows per load instruction of a wave
-    constexpr int NLD = KT / (4 * RPI);        // load instructions per wave, matrix and tile
-    auto swz_k = [](int r) __attribute__((always_inline)) { return DP == 128 ? (r & 15) : ((r >> 1) & 7); };
-    auto swz_v = [](int r) __attribute__((always_inline)) { return DP == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
-    static_assert(!DIRECT || (4 * RPI) % 16 == 0, "the row swizzles must not depend on the load index");
+    constexpr int NLD = KT * SPR / 256;        // load instructions per wave, matrix and tile
+    auto swz_k = [](int r) __attribute__((always_inline)) {
+        return DP == 128 ? (r & 15) : (DP == 64 ? ((r >> 1) & 7) : ((r >> 2) & 3));
+    };
+    auto swz_v = [](int r) __attribute__((always_inline)) { return DP == 128 ? 4 * (r & 3) : (DP == 64 ? 4 * ((r >> 1) & 1) : 0); };
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
-    const int dl_row = RPI * wave + lane / SPR;  // row of the lane's chunk in instruction 0; instruction n: + 4 RPI n (the swizzles do not see n)
-    const uint32_t dl_k = (uint32_t)dl_row * kv_pitch * 2u + (uint32_t)(((lane % SPR) ^ swz_k(dl_row)) * 16);
-    const uint32_t dl_v = (uint32_t)dl_row * kv_pitch * 2u + (uint32_t)(((lane % SPR) ^ swz_v(dl_row)) * 16);
-    // the tile whose first row lies tile_off bytes into the descriptor -> the stage at stage_off
-    auto dl_tile = [&](const u32x4_t& rs, uint32_t lane_off, uint32_t tile_off, uint32_t stage_off) __attribute__((always_inline)) {
+    int dl_row[NLD];                            // row of the lane's chunk of instruction n,
+    uint32_t dl_k[NLD], dl_v[NLD];              // its byte offsets from a tile's first row in K and in V,
+    uint64_t dl_k_on[NLD], dl_v_on[NLD];        // and the lanes whose chunk lies within the head dim
 #pragma unroll
-        for (int n = 0; n < NLD; n++)
-            t_buffer_to_lds(rs, lane_off, tile_off + (uint32_t)(4 * RPI * n) * kv_pitch * 2u, lds_base + stage_off + (uint32_t)((wave + 4 * n) * 1024));
+    for (int n = 0; n < NLD; n++) {
+        const int c = 64 * (wave + 4 * n) + lane, row = c / SPR, slot = c - row * SPR;
+        dl_row[n] = row;
+        const int sk = slot ^ swz_k(row), sv = slot ^ swz_v(row);
+        dl_k[n] = (uint32_t)row * kv_pitch * 2u + (uint32_t)(16 * sk);
+        dl_v[n] = (uint32_t)row * kv_pitch * 2u + (uint32_t)(16 * sv);
+        dl_k_on[n] = __ballot(8 * sk < D);
+        dl_v_on[n] = __ballot(8 * sv < D);
+        if (DP != 96 && n > 0) {  // (the same columns, 256 / SPR rows on: known to the compiler)
+            dl_k[n] = dl_k[0] + (uint32_t)(256 / SPR * n) * kv_pitch * 2u;
+            dl_v[n] = dl_v[0] + (uint32_t)(256 / SPR * n) * kv_pitch * 2u;
+            dl_k_on[n] = dl_k_on[0];
+            dl_v_on[n] = dl_v_on[0];
+        }
+    }
+    if constexpr (DIRECT && !WHOLE) {
+#pragma unroll
+        for (int n = 0; n < NLD; n++) {
+            unsigned char* const at = lds + (wave + 4 * n) * 1024 + 16 * lane;
+            const bool k_on = (dl_k_on[n] >> lane) & 1, v_on = (dl_v_on[n] >> lane) & 1;
+#pragma unroll
+            for (int st = 0; st < 2; st++) {
+                if (!k_on) *(u32x4_t*)(at + st * STAGE_B) = u32x4_t{0u, 0u, 0u, 0u};
+                if (!v_on) *(u32x4_t*)(at + (2 + st) * STAGE_B) = u32x4_t{0u, 0u, 0u, 0u};
+            }
+        }
+    }
+    // the tile whose first row lies tile_off bytes into the descriptor -> the stage at stage_off
+    auto dl_tile = [&](const u32x4_t& rs, const uint32_t (&lane_off)[NLD], const uint64_t (&on)[NLD], uint32_t tile_off, uint32_t stage_off) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < NLD; n++) {
+            const uint32_t block = lds_base + stage_off + (uint32_t)((wave + 4 * n) * 1024);
+            const uint32_t lane_at = DP == 96 ? lane_off[n] : lane_off[0];
+            const uint32_t off = DP == 96 ? tile_off : tile_off + (uint32_t)(256 / SPR * n) * kv_pitch * 2u;
+            if constexpr (WHOLE) t_buffer_to_lds(rs, lane_at, off, block);
+            else t_buffer_to_lds_of(on[DP == 96 ? n : 0], rs, lane_at, off, block);
+        }
     };
     // Tile 0 (K and V) and K of tile 1 are requested before the sequence lengths have arrived (a dependent load
     // away), through descriptors that end with the tensor's last row: the rows of V(0) past the last key are zeroed
@@ -271,9 +322,9 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (DIREC
         const uint32_t all_bytes = p.seq_kv > 0 ? ((uint32_t)(p.seq_kv - 1) * kv_pitch + (uint32_t)D) * 2u : 0u;
         if constexpr (DIRECT) {
             const u32x4_t Kall = t_make_rsrc(Kg, all_bytes), Vall = t_make_rsrc(Vg, all_bytes);
-            dl_tile(Kall, dl_k, 0u, 0u);
-            dl_tile(Vall, dl_v, 0u, 2u * STAGE_B);
-            dl_tile(Kall, dl_k, tile_bytes_g, STAGE_B);
+            dl_tile(Kall, dl_k, dl_k_on, 0u, 0u);
+            dl_tile(Vall, dl_v, dl_v_on, 0u, 2u * STAGE_B);
+            dl_tile(Kall, dl_k, dl_k_on, tile_bytes_g, STAGE_B);
         } else {
             const __amdgpu_buffer_rsrc_t Kall = __builtin_amdgcn_make_buffer_rsrc((void*)Kg, 0, all_bytes, kBufferFlags);
             const __amdgpu_buffer_rsrc_t Vall = __builtin_amdgcn_make_buffer_rsrc((void*)Vg, 0, all_bytes, kBufferFlags);
@@ -382,9 +433,9 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (DIREC
     const __amdgpu_buffer_rsrc_t Vbuf = __builtin_amdgcn_make_buffer_rsrc((void*)Vg, 0, slab_bytes, kBufferFlags);
     const u32x4_t Kd = t_make_rsrc(Kg, slab_bytes), Vd = t_make_rsrc(Vg, slab_bytes);  // (DIRECT: the same descriptors as scalars)
     if (DIRECT && (SPLIT || WIN)) {
-        dl_tile(Kd, dl_k, 0u, 0u);
-        dl_tile(Vd, dl_v, 0u, 2u * STAGE_B);
-        dl_tile(Kd, dl_k, tile_bytes_g, STAGE_B);
+        dl_tile(Kd, dl_k, dl_k_on, 0u, 0u);
+        dl_tile(Vd, dl_v, dl_v_on, 0u, 2u * STAGE_B);
+        dl_tile(Kd, dl_k, dl_k_on, tile_bytes_g, STAGE_B);
     } else if (SPLIT || WIN) {  // tile 0 (K and V) and K of tile 1 of the span / of the window
 #pragma unroll
         for (int n = 0; n < NL; n++) {
@@ -569,11 +620,13 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (DIREC
         const int v_off = (((lane & 15) >> 2) + 4 * hh) * LDV + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
         // DIRECT (byte offsets): the same operand rows and columns in the swizzled layout.  The swizzles only permute
         // address bits that the operand index also occupies, so operand ks sits at k_base ^ 32 ks, operand dt at
-        // v_base ^ 64 dt.
-        uint32_t k_base = 0, v_base = 0;
+        // v_base ^ 64 dt; in rows of 192 bytes, whose start has bits among those, the two operands of four slots have a base
+        // each, and four slots on is 64 bytes on.
+        uint32_t k_base = 0, k_base1 = 0, v_base = 0;
         if constexpr (DIRECT) {
             const int j = lane & 15, g16 = (lane >> 4) & 1, vrow = (j >> 2) + 4 * hh, low = 2 * g16 + ((j & 3) >> 1);
             k_base = (uint32_t)(col * ROWB + ((hh ^ swz_k(col)) * 16));
+            if constexpr (DP == 96) k_base1 = (uint32_t)(col * ROWB + (((2 + hh) ^ swz_k(col)) * 16));
             v_base = (uint32_t)(2 * STAGE_B + vrow * ROWB + ((low ^ swz_v(vrow)) * 16) + 8 * (j & 1));
         }
         // where the operands of item `item` of stage `st` start: with the lane's own offset (padded layout), or without
@@ -606,7 +659,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (DIREC
             if (n_keys < KT) {
 #pragma unroll
                 for (int n = 0; n < NLD; n++)
-                    if (dl_row + 4 * RPI * n >= n_keys) *(u32x4_t*)(lds + 2 * STAGE_B + (wave + 4 * n) * 1024 + 16 * lane) = u32x4_t{0u, 0u, 0u, 0u};
+                    if (dl_row[n] >= n_keys) *(u32x4_t*)(lds + 2 * STAGE_B + (wave + 4 * n) * 1024 + 16 * lane) = u32x4_t{0u, 0u, 0u, 0u};
             }
             bias_first();
         } else {
@@ -665,9 +718,12 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (DIREC
         // the previous item (contraction slots 0-3 of a lane are keys 16u + 4hh + 0..3, slots 4-7 keys 16u + 8 + 4hh + 0..3)
         auto load_op = [&](int m, const uint16_t* kp, const uint16_t* vp) __attribute__((always_inline)) {
             if constexpr (DIRECT) {
-                if ((m & 1) == 0) return *(const u32x4_t*)((const unsigned char*)kp + (k_base ^ (uint32_t)(32 * (m >> 1))));
                 const int i = m >> 1, u = i / DT, dt = i - u * DT;
-                const unsigned char* const vq = (const unsigned char*)vp + (v_base ^ (uint32_t)(64 * dt)) + 16 * u * ROWB;
+                if ((m & 1) == 0) {
+                    if constexpr (DP == 96) return *(const u32x4_t*)((const unsigned char*)kp + ((i & 1) ? k_base1 : k_base) + 64 * (i >> 1));
+                    return *(const u32x4_t*)((const unsigned char*)kp + (k_base ^ (uint32_t)(32 * i)));
+                }
+                const unsigned char* const vq = (const unsigned char*)vp + (DP == 96 ? v_base + (uint32_t)(64 * dt) : (v_base ^ (uint32_t)(64 * dt))) + 16 * u * ROWB;
                 const u32x2_t lo = t_lds_read_tr16((const uint16_t*)vq);
                 const u32x2_t hi = t_lds_read_tr16((const uint16_t*)(vq + 8 * ROWB));
                 return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
@@ -906,8 +962,8 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (DIREC
                 // (vmcnt) ahead of the next tile's barrier
                 // (BIAS: always, so that a step knows how many requests follow that for its bias values; behind the last
                 // tiles they land zeros that nobody reads)
-                if (BIAS || t + 2 < n_tiles) dl_tile(Kd, dl_k, (uint32_t)(t + 2) * tile_bytes_g, (uint32_t)(st * STAGE_B));
-                if (BIAS || t + 1 < n_tiles) dl_tile(Vd, dl_v, (uint32_t)(t + 1) * tile_bytes_g, (uint32_t)((2 + (st ^ 1)) * STAGE_B));
+                if (BIAS || t + 2 < n_tiles) dl_tile(Kd, dl_k, dl_k_on, (uint32_t)(t + 2) * tile_bytes_g, (uint32_t)(st * STAGE_B));
+                if (BIAS || t + 1 < n_tiles) dl_tile(Vd, dl_v, dl_v_on, (uint32_t)(t + 1) * tile_bytes_g, (uint32_t)((2 + (st ^ 1)) * STAGE_B));
             } else {
                 // (behind the last tiles these park and request copies of the last tile, which nobody reads)
                 park_k(kreg[KSET], st);
@@ -982,10 +1038,8 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (DIREC
             t0 = n_tiles;
         }
         const int t_full = PIPE ? n_it / NI : 0;
-        if constexpr (PF == 1 && (DP == 64 || (DIRECT && DP == 128)) && !BIAS && MODE != kMaskPadding) {
-            // (head dim 64 only: the wider kernels and the ones with a bias or a padding mask have no register to spare for
-            // the second copy of the tile's code)
-            // one register set: tile 0 on its own, then the tiles in pairs (odd, even) whose LDS stages are compile-time
+        if constexpr (DIRECT && !BIAS) {
+            // (the others have no register to spare for the second copy of the tile's code)  Tile 0 on its own, then the tiles in pairs (odd, even) whose LDS stages are compile-time
             // constants, then what is left of the tiles the wave walks in full
             using IC0 = std::integral_constant<int, 0>;
             using IC1 = std::integral_constant<int, 1>;
@@ -1694,39 +1748,35 @@ __global__ __launch_bounds__(256, 2) void flash_wide_bf16_kernel(FlashTileParams
     }
 }
 
-template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, bool DIRECT = false>
+template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs>
 hipError_t launch_one(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
-    hipLaunchKernelGGL((flash_tile_bf16_kernel<DP, MODE, BIAS, PACKED, SPLIT, WIN, DIRECT>), grid, dim3(TileCfg<DP>::THREADS), 0, stream, p);
+    hipLaunchKernelGGL((flash_tile_bf16_kernel<DP, MODE, BIAS, PACKED, SPLIT, WIN, TILES>), grid, dim3(TileCfg<DP>::THREADS), 0, stream, p);
     return hipGetLastError();
 }
 
-template <int DP>
-hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
-    constexpr bool kDirect = DP == 64 || DP == 128;  // head dim 64 or 128 exactly: the tiles go straight to LDS
-    const bool direct = kDirect && p.dim == DP;
+// Tiles straight to LDS wherever the kernel has that form: head dims up to 128 without a key-padding vector.
+template <int DP, int TILES>
+hipError_t launch_tiles(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
     if (p.n_splits > 1) {  // (rows packed over a group of one head are rows of that head)
-        hipError_t e = direct ? launch_one<DP, kMaskCausal, false, true, true, false, kDirect>(stream, p, grid)
-                              : launch_one<DP, kMaskCausal, false, true, true>(stream, p, grid);
+        hipError_t e = launch_one<DP, kMaskCausal, false, true, true, false, TILES>(stream, p, grid);
         if (e != hipSuccess) return e;
         const size_t items = (size_t)p.batch * p.kv_heads * (((size_t)p.seq_q * p.pack + 31) / 32) * (size_t)(p.dim / 8);
         if (p.n_splits > 8) hipLaunchKernelGGL(flash_split_merge_kernel<true>, dim3((unsigned)items), dim3(256), 0, stream, p);
         else hipLaunchKernelGGL(flash_split_merge_kernel<false>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, stream, p);
         return hipGetLastError();
     }
-    if (p.pack > 1 || p.decode_rows) return direct ? launch_one<DP, kMaskCausal, false, true, false, false, kDirect>(stream, p, grid)
-                                  : launch_one<DP, kMaskCausal, false, true>(stream, p, grid);
-    if (p.window > 0) return direct ? launch_one<DP, kMaskCausal, false, false, false, true, kDirect>(stream, p, grid)
-                                    : launch_one<DP, kMaskCausal, false, false, false, true>(stream, p, grid);
-    if (p.bias) return direct ? launch_one<DP, kMaskNone, true, false, false, false, kDirect>(stream, p, grid)
-                              : launch_one<DP, kMaskNone, true, false>(stream, p, grid);
-    if (direct && !p.bias && p.mask == kMaskNone) return launch_one<DP, kMaskNone, false, false, false, false, kDirect>(stream, p, grid);
-    if (direct && !p.bias && p.mask == kMaskCausal) return launch_one<DP, kMaskCausal, false, false, false, false, kDirect>(stream, p, grid);
-    switch (p.mask) {
-        case kMaskNone: return launch_one<DP, kMaskNone, false, false>(stream, p, grid);
-        case kMaskCausal: return launch_one<DP, kMaskCausal, false, false>(stream, p, grid);
-        case kMaskPadding: return launch_one<DP, kMaskPadding, false, false>(stream, p, grid);
-        default: return hipErrorInvalidValue;
-    }
+    if (p.pack > 1 || p.decode_rows) return launch_one<DP, kMaskCausal, false, true, false, false, TILES>(stream, p, grid);
+    if (p.window > 0) return launch_one<DP, kMaskCausal, false, false, false, true, TILES>(stream, p, grid);
+    if (p.bias) return launch_one<DP, kMaskNone, true, false, false, false, TILES>(stream, p, grid);
+    if (p.mask == kMaskNone) return launch_one<DP, kMaskNone, false, false, false, false, TILES>(stream, p, grid);
+    if (p.mask == kMaskCausal) return launch_one<DP, kMaskCausal, false, false, false, false, TILES>(stream, p, grid);
+    return hipErrorInvalidValue;
+}
+template <int DP>
+hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
+    if (p.mask == kMaskPadding) return launch_one<DP, kMaskPadding, false, false>(stream, p, grid);
+    if constexpr (DP > 128) return launch_tiles<DP, kTilesRegs>(stream, p, grid);
+    else return p.dim == DP ? launch_tiles<DP, kTilesDirect>(stream, p, grid) : launch_tiles<DP, kTilesDirectPart>(stream, p, grid);
 }
 
 }  // namespace

@@ -91,3 +91,30 @@ def test_flash_bnhd_f32_dev_matches_oracle(oracle, b, n, h, d):
     want = oracle.flash_forward_masked(oracle.AttentionShape(b, h, n, d), to_bhnd(q, b, n, h, d),
                                        to_bhnd(k, b, n, h, d), to_bhnd(v, b, n, h, d), "causal")
     assert_close_nan(got, to_bnhd(want, b, h, n, d), 1e-5, f"bnhd f32 {b},{n},{h},{d}")
+
+
+@pytest.mark.parametrize("d", [8, 24, 32, 40, 64, 72, 80, 96, 104, 128])
+@pytest.mark.parametrize("n", [1, 33, 64, 65, 129, 200])
+@pytest.mark.parametrize("mask_name", ["none", "causal", "window"])
+def test_bnhd_heads_do_not_meet(oracle, d, n, mask_name):
+    """What lies behind a head's columns in a [B,N,H,D] row is the next head's, here NaN and infinities: at head dims
+    between the tile widths it must not come into the head's own products."""
+    b, h = 2, 2
+    rng = np.random.default_rng(d + n)
+    x = [rng.standard_normal((b, n, h, d)).astype(np.float32) for _ in range(3)]
+    for t in x[1:]:
+        t[:, :, 1] = np.where(rng.random((b, n, d)) < 0.5, np.nan, np.inf)
+    bits = [bf16_round(t.ravel()) for t in x]
+    dq, dk, dv = (dev(t[0]) for t in bits)
+    out = ra.HipStorage(b * n * h * d * 2)
+    shape = ra.AttentionShape.new(b, h, n, d)
+    if mask_name == "window":
+        ra.flash_forward_window_bf16_dev(shape, dq, dk, dv, out, 40, bnhd=True)
+    else:
+        ra.flash_forward_bnhd_bf16_dev(shape, dq, dk, dv, out, ra.Mask.causal() if mask_name == "causal" else ra.Mask.none())
+    ra.synchronize()
+    got = oracle.bf16_to_f32(out.download(np.uint16)).reshape(b, n, h, d)[:, :, 0].copy().ravel()
+    q, k, v = (np.ascontiguousarray(t[1].reshape(b, n, h, d)[:, :, 0]).ravel() for t in bits)
+    mask = {"none": None, "causal": oracle.causal_mask(n), "window": oracle.sliding_window_mask(n, 40)}[mask_name]
+    want = oracle.mha_forward_masked(q, k, v, b, n, n, 1, d, mask)
+    assert_bf16_parity(got, want, d, None, f"n={n} d={d} {mask_name}")
