@@ -1789,8 +1789,6 @@ int flash_tile_bf16_workgroups(int dim) { return dim <= 64 ? 3 : (dim <= 128 ? 2
 bool flash_tile_bf16_addressable(long long seq_kv, long long row_pitch) {
     return seq_kv >= 0 && row_pitch > 0 && (unsigned long long)(seq_kv + 512) * (unsigned long long)row_pitch * 2ull < (1ull << 32);
 }
-// ... and the bias values of 32 rows likewise.
-bool flash_tile_bf16_bias_addressable(long long seq_kv) { return seq_kv < (1ll << 24); }
 
 // What the kernels take grid positions for heads by.
 static void set_grid_order(FlashTileParams& p, long long z) {

@@ -158,7 +158,7 @@ int flash_tile_bf16_key_tile(int dim);
 int flash_tile_bf16_workgroups(int dim);  // that share a CU
 hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& p);
 bool flash_tile_bf16_addressable(long long seq_kv, long long row_pitch);  // K/V slabs below 4 GiB (32-bit offsets)
-bool flash_tile_bf16_bias_addressable(long long seq_kv);  // 32 rows of an additive bias likewise
+inline bool flash_tile_bf16_bias_addressable(long long seq_kv) { return seq_kv < (1ll << 24); }  // 32 rows of an additive bias likewise
 // the same walk with 64 query rows per wave: head dim 64, masks none / causal, rows of one head
 bool flash_wide_bf16_supported(const FlashTileParams& p);
 hipError_t launch_flash_wide_bf16(hipStream_t stream, const FlashTileParams& p);
