@@ -1303,6 +1303,7 @@ static int flash_bf16_common(void* stream, const rt_attention_shape* shape, uint
         t.kv_heads = (int)n_kv_heads;
         t.group = (int)(shape->heads / n_kv_heads);
         t.pack = 1;
+        t.n_cus = g_num_cus;
         t.seq_q = t.seq_kv = (int)shape->seq;
         t.dim = dim;
         t.mask = mask == rt::kMaskVarlenCausal ? rt::kMaskCausal : mask;
@@ -1565,6 +1566,7 @@ RT_API int rt_mha_forward_masked_bf16_dev(void* stream, const void* q, const voi
     t.heads = t.kv_heads = (int)heads;
     t.group = 1;
     t.pack = 1;
+    t.n_cus = g_num_cus;
     t.seq_q = (int)t_q;
     t.seq_kv = (int)t_kv;
     t.dim = (int)head_dim;
@@ -1616,6 +1618,7 @@ static int flash_window_bf16(void* stream, const rt_attention_shape* shape, uint
     t.kv_heads = (int)n_kv_heads;
     t.group = (int)(shape->heads / n_kv_heads);
     t.pack = 1;
+    t.n_cus = g_num_cus;
     t.seq_q = t.seq_kv = (int)shape->seq;
     t.dim = dim;
     t.mask = rt::kMaskCausal;

@@ -175,10 +175,18 @@ enum TileWay : int { kTilesRegs = 0, kTilesDirect = 1, kTilesDirectPart = 2 };
 // workgroups per CU (head dim 64) are no faster.  Head dims between the tile widths have a form of their own
 // (kTilesDirectPart), whose requests leave the lanes behind the head dim out: two scalar instructions a request, which
 // cost the masked form at head dim 64 6 % where the kernel of whole rows had them too (28.3 -> 29.9 us; a branch 31.1).
-template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs>
-__global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES ? TileCfg<DP>::OCC_DIRECT : TileCfg<DP>::OCC)) void flash_tile_bf16_kernel(FlashTileParams p) {
+//
+// HALVES (DIRECT, rows of one head, no window): the workgroup is eight waves, two to a SIMD, and the tiles of its walk are
+// cut in two: waves 0-3 take the first half of them and waves 4-7 the second, each half in stages of its own and for the
+// same query rows; at the end the second half's O, max and row sum go through LDS to the first, which folds them in as
+// the split form's merge does.  For launches that leave a CU one workgroup: its waves, alone on their SIMDs, take 800
+// clocks an item at head dim 64 where three of them together take 500 each, and 2100 with a bias, whose latency one wave
+// does not hide.  (launch_halves has the figures.)
+template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs, bool HALVES = false>
+__global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : BIAS && DP == 64 ? 2 : (TILES ? TileCfg<DP>::OCC_DIRECT : TileCfg<DP>::OCC)) void flash_tile_bf16_kernel(FlashTileParams p) {
     static_assert(!SPLIT || (PACKED && !BIAS && MODE == kMaskCausal), "the split over the keys serves the chunked decode");
     static_assert(!WIN || (!PACKED && !BIAS && !SPLIT && MODE == kMaskCausal), "the window is a causal mask's");
+    static_assert(!HALVES || (TILES != kTilesRegs && !PACKED && !SPLIT && !WIN), "halves of the walk: tiles straight to LDS, rows of one head");
     static_assert(TILES == kTilesRegs || (DP <= 128 && MODE != kMaskPadding), "tiles straight into LDS: head dims up to 128, no key-padding vector");
     constexpr bool DIRECT = TILES != kTilesRegs, WHOLE = TILES == kTilesDirect;
     using Cfg = TileCfg<DP>;
@@ -195,18 +203,23 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
     // Head dims above 128 do not have the registers for two score tiles and their operands in flight (O alone is 128
     // registers), nor does head dim 128 with a bias (two items' bias values) or with a key-padding mask: there an
     // item runs its three phases one after the other, and K is parked with V.
-    constexpr bool PIPE = DP <= 128 && !((((BIAS && !DIRECT) || MODE == kMaskPadding)) && DP == 128);
+    constexpr bool PIPE = DP <= 128 && !(((BIAS && !DIRECT) || MODE == kMaskPadding) && DP == 128);
+    static_assert(PIPE || !HALVES, "the halves meet once a tile");
 
     constexpr int kTilesLds = DIRECT ? Cfg::LDS_BYTES_DIRECT : Cfg::LDS_BYTES;  // BIAS: the four waves' bias values behind the tiles
-    __shared__ alignas(DIRECT || BIAS ? 1024 : 16) unsigned char lds[BIAS ? (kTilesLds + 1023) / 1024 * 1024 + 4 * Cfg::BIAS_BYTES : kTilesLds];
+    constexpr int kHalves = HALVES ? 2 : 1, kBiasAt = kHalves * ((kTilesLds + 1023) / 1024 * 1024);
+    static_assert(!HALVES || (kTilesLds % 1024 == 0 && kTilesLds >= 4 * 32 * DP * 4 && kTilesLds >= 4 * Cfg::REGION + 2048), "a half's partials fit over its tiles, their max and sum behind the output rows");
+    __shared__ alignas(DIRECT || BIAS ? 1024 : 16) unsigned char lds[BIAS ? kBiasAt + kHalves * 4 * Cfg::BIAS_BYTES : kHalves * kTilesLds];
     uint16_t* const Ks = (uint16_t*)lds;                      // [2][KT * LDK]
     uint16_t* const Vs = (uint16_t*)lds + 2 * KT * LDK;       // [2][KT * LDV]
     // DIRECT: [K stage 0][K stage 1][V stage 0][V stage 1], rows of ROWB bytes without padding
     constexpr int ROWB = DP * 2, STAGE_B = Cfg::STAGE_BYTES;
 
-    const int tid = threadIdx.x;
+    const int tid = HALVES ? threadIdx.x & 255 : threadIdx.x;  // within the half
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = HALVES ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+    const uint32_t half_at = (uint32_t)(half * kTilesLds);  // where its stages start
     const int col = lane & 31, hh = lane >> 5;
 
     // ---- which tile.  The grid is (unit within the batch, batch, rank of the query tile), dispatched x first: all
@@ -293,7 +306,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
     if constexpr (DIRECT && !WHOLE) {
 #pragma unroll
         for (int n = 0; n < NLD; n++) {
-            unsigned char* const at = lds + (wave + 4 * n) * 1024 + 16 * lane;
+            unsigned char* const at = lds + half_at + (wave + 4 * n) * 1024 + 16 * lane;
             const bool k_on = (dl_k_on[n] >> lane) & 1, v_on = (dl_v_on[n] >> lane) & 1;
 #pragma unroll
             for (int st = 0; st < 2; st++) {
@@ -306,7 +319,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
     auto dl_tile = [&](const u32x4_t& rs, const uint32_t (&lane_off)[NLD], const uint64_t (&on)[NLD], uint32_t tile_off, uint32_t stage_off) __attribute__((always_inline)) {
 #pragma unroll
         for (int n = 0; n < NLD; n++) {
-            const uint32_t block = lds_base + stage_off + (uint32_t)((wave + 4 * n) * 1024);
+            const uint32_t block = lds_base + half_at + stage_off + (uint32_t)((wave + 4 * n) * 1024);
             const uint32_t lane_at = DP == 96 ? lane_off[n] : lane_off[0];
             const uint32_t off = DP == 96 ? tile_off : tile_off + (uint32_t)(256 / SPR * n) * kv_pitch * 2u;
             if constexpr (WHOLE) t_buffer_to_lds(rs, lane_at, off, block);
@@ -318,7 +331,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
     // once the length is known, those of K are masked in the score tile whatever they hold.  (A span of the keys
     // starts where the sequence's own length puts it: its requests wait for the lengths.)
     const uint32_t tile_bytes_g = (uint32_t)KT * kv_pitch * 2u;  // from a tile's first row to the next tile's, in memory
-    if (!SPLIT && !WIN) {
+    if (!SPLIT && !WIN && !HALVES) {
         const uint32_t all_bytes = p.seq_kv > 0 ? ((uint32_t)(p.seq_kv - 1) * kv_pitch + (uint32_t)D) * 2u : 0u;
         if constexpr (DIRECT) {
             const u32x4_t Kall = t_make_rsrc(Kg, all_bytes), Vall = t_make_rsrc(Vg, all_bytes);
@@ -409,12 +422,23 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
         Kg += (size_t)key0 * (size_t)p.lkv.row_pitch;
         Vg += (size_t)key0 * (size_t)p.lkv.row_pitch;
     }
+    const int n_loop = HALVES ? (n_tiles + 1) / 2 : n_tiles;  // tiles between the workgroup's barriers
+    int half_key0 = 0;
+    if (HALVES) {  // this half's span of the walk, as a span of SPLIT; the second may be a tile shorter
+        half_key0 = half * n_loop * KT;
+        n_tiles = half ? n_tiles - n_loop : n_loop;
+        n_keys = min(n_keys, (half + 1) * n_loop * KT) - half_key0;
+        off -= half_key0;
+        Kg += (size_t)half_key0 * (size_t)p.lkv.row_pitch;
+        Vg += (size_t)half_key0 * (size_t)p.lkv.row_pitch;
+    }
     // A tile of padded query rows only (a padded batch has many: every tile behind a sequence's last row) has nothing
     // to load or walk: its rows get the fill value and the workgroup is done.
     if (!SPLIT && !PACKED && q0 >= n_q) {
         const uint32_t f2 = p.zero_padded_rows ? 0u : 0x7fc07fc0u;
         const u32x4_t val = {f2, f2, f2, f2};
         uint16_t* const ob = p.out + (size_t)b * p.lo.batch_stride + (size_t)h0 * p.lo.head_stride;
+        if (HALVES && half) return;
         for (int c = tid; c < TROWS * CH; c += TTHREADS) {
             const int row = c / CH, ch = c - row * CH;
             if (q0 + row < rows_total && 8 * ch < D) *(u32x4_t*)(ob + (size_t)(q0 + row) * p.lo.row_pitch + 8 * ch) = val;
@@ -432,7 +456,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
     const __amdgpu_buffer_rsrc_t Kbuf = __builtin_amdgcn_make_buffer_rsrc((void*)Kg, 0, slab_bytes, kBufferFlags);
     const __amdgpu_buffer_rsrc_t Vbuf = __builtin_amdgcn_make_buffer_rsrc((void*)Vg, 0, slab_bytes, kBufferFlags);
     const u32x4_t Kd = t_make_rsrc(Kg, slab_bytes), Vd = t_make_rsrc(Vg, slab_bytes);  // (DIRECT: the same descriptors as scalars)
-    if (DIRECT && (SPLIT || WIN)) {
+    if (DIRECT && (SPLIT || WIN || HALVES)) {
         dl_tile(Kd, dl_k, dl_k_on, 0u, 0u);
         dl_tile(Vd, dl_v, dl_v_on, 0u, 2u * STAGE_B);
         dl_tile(Kd, dl_k, dl_k_on, tile_bytes_g, STAGE_B);
@@ -465,7 +489,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
     bool valid = false;
     const float cc = BIAS ? kLog2e : p.scale_log2e;  // exp2 argument per unit of score
 
-    if (n_tiles > 0) {
+    if (n_loop > 0) {
         static_assert(CHUNKS % TTHREADS == 0, "every thread moves NL chunks of every tile");
         // Every request below is unconditional -- a tile index past the last tile is clamped to it, a chunk past the
         // head dim reads column 0 -- and only the LDS write is predicated.  With no branch around a load the compiler
@@ -549,13 +573,13 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
         // behind the tensor: those scores are masked.
         u32x4_t bias_rsrc = {0u, 0u, 0u, 0u};
         uint32_t bias_lane[2] = {0u, 0u}, bias_at = 0, bias_step = 0;
-        const uint32_t bias_lds = BIAS ? (uint32_t)((kTilesLds + 1023) / 1024 * 1024 + wave * Cfg::BIAS_BYTES) : 0u;
+        const uint32_t bias_lds = BIAS ? (uint32_t)(kBiasAt + (wave + 4 * half) * Cfg::BIAS_BYTES) : 0u;
         const bool bias_vec4 = BIAS && p.bias_vec4;
         if constexpr (BIAS) {
             const int r_first = q0 + 32 * wq, n_rows = max(min(32, rows_total - r_first), 0);
             const float* const bb = p.bias + ((size_t)b * p.heads + h0) * (size_t)p.bias_bh_stride + (size_t)min(r_first, rows_total - 1) * (size_t)p.seq_kv;
-            const uint32_t pitch = (uint32_t)p.seq_kv * 4u;
-            bias_rsrc = t_make_rsrc(bb, (uint32_t)n_rows * pitch);
+            const uint32_t pitch = (uint32_t)p.seq_kv * 4u, first = 4u * (uint32_t)min(half_key0, p.seq_kv);
+            bias_rsrc = t_make_rsrc((const char*)bb + first, n_rows > 0 ? (uint32_t)n_rows * pitch - first : 0u);
             if (bias_vec4) {  // instruction n: rows 8 n + lane / 8
                 const int row = lane >> 3, slot = (lane & 7) ^ (row >> 1);
                 bias_lane[0] = (uint32_t)row * pitch + 16u * (uint32_t)slot;
@@ -625,9 +649,9 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
         uint32_t k_base = 0, k_base1 = 0, v_base = 0;
         if constexpr (DIRECT) {
             const int j = lane & 15, g16 = (lane >> 4) & 1, vrow = (j >> 2) + 4 * hh, low = 2 * g16 + ((j & 3) >> 1);
-            k_base = (uint32_t)(col * ROWB + ((hh ^ swz_k(col)) * 16));
-            if constexpr (DP == 96) k_base1 = (uint32_t)(col * ROWB + (((2 + hh) ^ swz_k(col)) * 16));
-            v_base = (uint32_t)(2 * STAGE_B + vrow * ROWB + ((low ^ swz_v(vrow)) * 16) + 8 * (j & 1));
+            k_base = half_at + (uint32_t)(col * ROWB + ((hh ^ swz_k(col)) * 16));
+            if constexpr (DP == 96) k_base1 = half_at + (uint32_t)(col * ROWB + (((2 + hh) ^ swz_k(col)) * 16));
+            v_base = half_at + (uint32_t)(2 * STAGE_B + vrow * ROWB + ((low ^ swz_v(vrow)) * 16) + 8 * (j & 1));
         }
         // where the operands of item `item` of stage `st` start: with the lane's own offset (padded layout), or without
         // it (DIRECT: load_op adds the lane's swizzled offset)
@@ -659,7 +683,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
             if (n_keys < KT) {
 #pragma unroll
                 for (int n = 0; n < NLD; n++)
-                    if (dl_row[n] >= n_keys) *(u32x4_t*)(lds + 2 * STAGE_B + (wave + 4 * n) * 1024 + 16 * lane) = u32x4_t{0u, 0u, 0u, 0u};
+                    if (dl_row[n] >= n_keys) *(u32x4_t*)(lds + half_at + 2 * STAGE_B + (wave + 4 * n) * 1024 + 16 * lane) = u32x4_t{0u, 0u, 0u, 0u};
             }
             bias_first();
         } else {
@@ -1062,15 +1086,47 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
                 if (PF >= 3) walk_full(t0 + 2, std::integral_constant<int, 4 % PF>{}, std::integral_constant<int, 3 % PF>{}, (t0 + 2) & 1, std::false_type{});
             }
         }
-        for (; t0 < n_tiles; t0 += PF) {
+        for (; t0 < n_loop; t0 += PF) {
             walk_tile(t0, std::integral_constant<int, 2 % PF>{}, std::integral_constant<int, 1 % PF>{});
-            if (PF >= 2 && t0 + 1 < n_tiles) walk_tile(t0 + 1, std::integral_constant<int, 3 % PF>{}, std::integral_constant<int, 2 % PF>{});
-            if (PF >= 3 && t0 + 2 < n_tiles) walk_tile(t0 + 2, std::integral_constant<int, 4 % PF>{}, std::integral_constant<int, 3 % PF>{});
+            if (PF >= 2 && t0 + 1 < n_loop) walk_tile(t0 + 1, std::integral_constant<int, 3 % PF>{}, std::integral_constant<int, 2 % PF>{});
+            if (PF >= 3 && t0 + 2 < n_loop) walk_tile(t0 + 2, std::integral_constant<int, 4 % PF>{}, std::integral_constant<int, 3 % PF>{});
         }
         // a wave that walked every item of the workgroup still owes the last P.V
-        if (PIPE && n_it == n_tiles * NI && n_it > 0) drain(v_at((n_tiles - 1) & 1, NI - 1));
+        if (PIPE && n_it == n_loop * NI && n_it > 0) drain(v_at((n_loop - 1) & 1, NI - 1));
         if constexpr (BIAS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (requests behind the last item and the last tile)
         __syncthreads();  // the output rows are staged over the tiles
+        if constexpr (HALVES) {
+            // the second half's O (relative to its running max), max and lane's share of the row sum, as the registers hold
+            // them, over its tiles and behind the first half's output rows
+            f32x4_t* const part_o = (f32x4_t*)(lds + kTilesLds + wave * (32 * DP * 4)) + lane;
+            float* const part_ml = (float*)(lds + kTilesLds - 2048) + 128 * wave + lane;
+            if (half) {
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        part_o[64 * (4 * dt + j)] = f32x4_t{acc_o[dt][4 * j], acc_o[dt][4 * j + 1], acc_o[dt][4 * j + 2], acc_o[dt][4 * j + 3]};
+                part_ml[0] = m_run;
+                part_ml[64] = l_run;
+            }
+            __syncthreads();
+            if (half) return;
+            const float m_1 = part_ml[0], l_1 = part_ml[64];
+            const float m_new = t_vmax(m_run, m_1), m_use = m_new == neg_inf() ? 0.0f : m_new;
+            const float a_0 = __builtin_amdgcn_exp2f((m_run - m_use) * cc), a_1 = __builtin_amdgcn_exp2f((m_1 - m_use) * cc);
+            l_run = l_run * a_0 + l_1 * a_1;
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const f32x4_t o_1 = part_o[64 * (4 * dt + j)];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc_o[dt][4 * j + e] = acc_o[dt][4 * j + e] * a_0 + o_1[e] * a_1;
+                }
+        }
+    } else if (HALVES && half) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
     }
     // (a workgroup without tiles still has its early requests in flight: they land in its LDS)
     if constexpr (DIRECT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1108,7 +1164,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
     const float bad = (PACKED && l == 0.0f) ? 0.0f : quiet_nan();
     uint16_t* const obuf = (uint16_t*)(lds + wq * Cfg::REGION);
     const float fill = p.zero_padded_rows ? 0.0f : quiet_nan();
-    if (n_tiles > 0) {
+    if (n_loop > 0) {
         uint16_t* const orow = obuf + col * LDK + 4 * hh;
         if (__all(good && valid)) {
             // the common wave: one multiplication per element (a branch of its own: as a select inside one loop the
@@ -1154,7 +1210,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
             // no key tile walked: padded rows get the fill value, valid rows (which then see no key at all) NaN
             const uint32_t f2 = rr < n_q ? 0x7fc07fc0u : fill2;
             u32x4_t val = {f2, f2, f2, f2};
-            if (n_tiles > 0) val = *(const u32x4_t*)(src + RS * n * LDK);
+            if (n_loop > 0) val = *(const u32x4_t*)(src + RS * n * LDK);
             if (rr < rows_total && col_ok) *(u32x4_t*)dst = val;
             dst += step;
         }
@@ -1170,7 +1226,7 @@ __global__ __launch_bounds__(TileCfg<DP>::THREADS, BIAS && DP == 64 ? 2 : (TILES
             // when the rows are positions of a chunked decode
             const uint32_t f2 = sp < n_q ? (PACKED ? 0u : 0x7fc07fc0u) : fill2;
             u32x4_t val = {f2, f2, f2, f2};
-            if (n_tiles > 0) val = *(const u32x4_t*)(obuf + row * LDK + 8 * ch);
+            if (n_loop > 0) val = *(const u32x4_t*)(obuf + row * LDK + 8 * ch);
             if (rr < rows_total && 8 * ch < D) {
                 uint16_t* dst = p.out + (size_t)b * p.lo.batch_stride + (size_t)(h0 + gg) * p.lo.head_stride +
                                 (size_t)sp * p.lo.row_pitch + 8 * ch;
@@ -1748,9 +1804,9 @@ __global__ __launch_bounds__(256, 2) void flash_wide_bf16_kernel(FlashTileParams
     }
 }
 
-template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs>
+template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs, bool HALVES = false>
 hipError_t launch_one(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
-    hipLaunchKernelGGL((flash_tile_bf16_kernel<DP, MODE, BIAS, PACKED, SPLIT, WIN, TILES>), grid, dim3(TileCfg<DP>::THREADS), 0, stream, p);
+    hipLaunchKernelGGL((flash_tile_bf16_kernel<DP, MODE, BIAS, PACKED, SPLIT, WIN, TILES, HALVES>), grid, dim3(HALVES ? 512 : TileCfg<DP>::THREADS), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -1772,9 +1828,29 @@ hipError_t launch_tiles(hipStream_t stream, const FlashTileParams& p, dim3 grid)
     if (p.mask == kMaskCausal) return launch_one<DP, kMaskCausal, false, false, false, false, TILES>(stream, p, grid);
     return hipErrorInvalidValue;
 }
+// Two halves of the walk (head dims 64 and 128 exactly, up to 32, and 65 to 96) where every workgroup has a CU to itself and
+// the walk is long enough to pay for the meeting at its end, 0.6-1.4 us.  us, whole / halves, B H N head dim: causal 1 8 384
+// 64 8.0 / 8.1, 512 9.3 / 9.1, 1024 14.7 / 13.0, 4096 46.2 / 37.4; 1 8 256 128 8.8 / 10.3, 512 12.5 / 13.0, 1024 20.1 / 19.0,
+// 4096 63.9 / 54.3; 1 8 512 96 10.4 / 10.7; unmasked 1 12 1000 96 19.5 / 17.4; 1 8 3000 32 37.2 / 28.2; with a bias 1 8 256 64
+// 7.8 / 7.8, 512 11.5 / 10.3; 77 queries over 3001 keys, 24 heads of 32, 65.8 / 43.1.
+constexpr int kHalvesFrom64 = 512, kHalvesFrom = 768;  // keys, head dims up to 64 and above
+template <int DP, int TILES>
+hipError_t launch_halves(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
+    if (p.bias) return launch_one<DP, kMaskNone, true, false, false, false, TILES, true>(stream, p, grid);
+    if (p.mask == kMaskNone) return launch_one<DP, kMaskNone, false, false, false, false, TILES, true>(stream, p, grid);
+    return launch_one<DP, kMaskCausal, false, false, false, false, TILES, true>(stream, p, grid);
+}
+static bool takes_halves(const FlashTileParams& p, dim3 grid) {
+    return p.pack == 1 && !p.decode_rows && p.window == 0 && p.mask != kMaskPadding && p.seq_kv >= (p.dim <= 64 ? kHalvesFrom64 : kHalvesFrom) &&
+           (unsigned long long)grid.x * grid.y * grid.z <= (unsigned long long)p.n_cus;
+}
 template <int DP>
 hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
     if (p.mask == kMaskPadding) return launch_one<DP, kMaskPadding, false, false>(stream, p, grid);
+    if constexpr (DP <= 128) {
+        constexpr int kTiles = DP % 64 == 0 ? kTilesDirect : kTilesDirectPart;
+        if ((kTiles == kTilesDirectPart || p.dim == DP) && takes_halves(p, grid)) return launch_halves<DP, kTiles>(stream, p, grid);
+    }
     if constexpr (DP > 128) return launch_tiles<DP, kTilesRegs>(stream, p, grid);
     else return p.dim == DP ? launch_tiles<DP, kTilesDirect>(stream, p, grid) : launch_tiles<DP, kTilesDirectPart>(stream, p, grid);
 }

@@ -150,6 +150,7 @@ struct FlashTileParams {
     // reference's decode kernels leave it so), not the NaN row of flash_forward.  Implied by pack > 1; a group of one
     // head sets it.
     int decode_rows;
+    int n_cus;  // CUs of the device (0: unknown)
 };
 static_assert(offsetof(FlashTileParams, q) == 64 && offsetof(FlashTileParams, q_lens) == 128, "lines of the arguments");
 bool flash_tile_bf16_supported(int dim);

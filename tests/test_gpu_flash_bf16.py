@@ -479,3 +479,45 @@ def test_padding_mask_longer_than_the_persistent_kernel_holds(oracle):
     for i in (0, 1, 499, 500, 39999, 40000, 65535, 65536, 65999):
         want = oracle.gqa_forward_f32(q2[i], k2, v2, 1, 1, 1, 1, k2.shape[0], d)
         assert_bf16_parity(got[i], want, d, 1, f"row {i}")
+
+
+@pytest.mark.parametrize("d", [24, 32, 64, 80, 96, 128])
+@pytest.mark.parametrize("n", [512, 513, 576, 577, 767, 768, 769, 833, 1024, 1089])
+def test_two_halves_of_the_keys(oracle, n, d):
+    """Few workgroups and long walks: the tile kernel cuts the walk in two from 512 keys on at head dims up to 64, from 768
+    above.  Odd and even numbers of tiles, one key in the last tile; a padded batch whose sequences have none, one, two
+    and all of the tiles; an additive mask that hides the first, the last and every key of some rows' halves."""
+    h = 2
+    masks = {"none": ra.Mask.none(), "causal": ra.Mask.causal()}
+    shape, oshape = ra.AttentionShape.new(1, h, n, d), oracle.AttentionShape(1, h, n, d)
+    bits, f = zip(*(bf16_round(seeded_normal(h * n * d, s)) for s in (1, 2, 3)))
+    for name, mask in masks.items():
+        got = flash_bf16(shape, *bits, mask)
+        assert_bf16_parity(got, oracle.flash_forward_masked(oshape, *f, name), d, n, f"n={n} d={d} {name}")
+    lens = np.array([0, 1, 64, 65, n // 2, n], dtype=np.int32)
+    b = len(lens)
+    vb, vf = zip(*(bf16_round(seeded_normal(b * n * d, s)) for s in (4, 5, 6)))
+    dq, dk, dv, dl = (dev(x) for x in (*vb, lens))
+    out = ra.HipStorage(b * n * d * 2)
+    ra.flash_forward_varlen_bf16_dev(ra.AttentionShape.new(b, 1, n, d), dq, dk, dv, dl, out, zero_padded_rows=True)
+    ra.synchronize()
+    got = oracle.bf16_to_f32(out.download(np.uint16)).reshape(b, n, d)
+    for i, ln in enumerate(lens):
+        assert not got[i, ln:].any()
+        if ln:
+            q, k, v = (np.ascontiguousarray(x.reshape(b, n, d)[i, :ln]).ravel() for x in vf)
+            want = oracle.flash_forward_masked(oracle.AttentionShape(1, 1, int(ln), d), q, k, v, "causal")
+            assert_bf16_parity(got[i, :ln].ravel(), want, d, None, f"n={n} d={d} length {ln}")
+    tq = 70
+    rng = np.random.default_rng(n)
+    bias = rng.standard_normal((tq, n)).astype(np.float32)
+    bias[3, : n // 2 + 64] = -1.0e4
+    bias[4, n // 2 - 64:] = -np.inf
+    bias[5] = -np.inf
+    bias[6] = -1.0e4
+    dq, dk, dv, db = (dev(x) for x in (bits[0][: tq * h * d], bits[1], bits[2], bias))
+    out = ra.HipStorage(tq * h * d * 2)
+    ra.mha_forward_masked_bf16_dev(dq, dk, dv, out, 1, tq, n, h, d, db, bias.size)
+    ra.synchronize()
+    want = oracle.mha_forward_masked(f[0][: tq * h * d], f[1], f[2], 1, tq, n, h, d, bias)
+    assert_bf16_parity(oracle.bf16_to_f32(out.download(np.uint16)), want, d, None, f"n={n} d={d} bias")
