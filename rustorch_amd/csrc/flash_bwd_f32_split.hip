@@ -2,18 +2,21 @@
 // flash_bwd_f32.hip (its header has the formulas) for launches with enough rows to fill the chip with 128 a workgroup.
 //
 // A wave owns 32 rows (keys for dK/dV, queries for dQ), split once into registers as B operands; the four waves of a
-// workgroup walk the same tiles of 32 rows of the other side, which the workgroup splits into LDS: as rows (A operand of the
-// score-shaped products) and, where a gradient contracts over them, as columns (A operand of dV^T += dO^T P and the like,
-// the rows of a column in the order the weights sit in the accumulators).  Every output row has one owner: no atomics, the
-// same bits on every launch.
+// workgroup walk the same tiles of 32 rows of the other side, which the workgroup splits once into LDS: planes of rows, read as
+// rows (A operand of the score-shaped products) and, where a gradient contracts over them, as columns by the transposing reads
+// (A operand of dV^T += dO^T P and the like, in the order the weights sit in the accumulators).  Every output row has one
+// owner: no atomics, the same bits on every launch.
 //
-// What bounds them: matrix and vector instructions together, as in the forward kernel (counted: 38 % and 43 % of the clocks of
-// either kernel); at head dim 64 a tile is 72 (dQ) and 96 (dK/dV) matrix instructions of 32 clocks and about 580 and 745
-// vector ones of 4 per wave.  LDS holds two tiles of both streams for one workgroup a CU, and a wave takes the register
-// file of its SIMD; the moves that makes necessary are a tenth of the vector instructions.  Between two matrix instructions stands a
-// step of the next tile's split or of the weights (two matrix instructions behind each other hold the wave until the first
-// is done: 382 -> 370 us; without any order 418).  B=4 H=16 N=1024 D=64, dQ and dK/dV: 506 -> 370 us, B=2 N=2048 973 ->
-// 704, head dim 32 273 -> 216; relative error against 64 bits 5.9e-7 -> 4.5e-7, 7.3e-7 -> 5.9e-7, 5.5e-7 -> 4.4e-7.
+// What bounds them: a wave takes the register file of its SIMD (400 registers at head dim 64), so nothing covers what it waits
+// for; at head dim 64 a tile is 96 (dK/dV) and 72 (dQ) matrix instructions of 32 clocks and 520 and 400 vector ones of 4, each
+// kernel with room to run the one beside the other, and takes 4400 and 3500 clocks.  Hence: vector work between all matrix
+// instructions, in runs of independent instructions (SplitQuad); LDS writes one at a time; nothing loaded is looked at in
+// the step that requests it; owners and sums pinned to the accumulation registers, where the matrix instructions read them
+// and no vector instruction wants them.  Time of both, B=4 H=16 N=1024 D=64: f32 kernels 506 us, this form with columns of its
+// own in LDS 362, with the transposing reads 341, with every vector step beside a matrix instruction 336, without a wait
+// for the row statistic where it is requested 327, sums pinned 321, dQ in the same order 312, independent runs and single
+// writes 308.  B=2 N=2048 973, 689, 583; head dim 32 273, 214, 171.  (dQ with two waves a SIMD, 40 registers spilled: 318.)
+// Relative error against 64 bits 5.9e-7 -> 4.5e-7, 7.3e-7 -> 5.9e-7, 5.5e-7 -> 4.4e-7 (f32 kernels -> this).
 #include "rt_common.hpp"
 #include "rt_kernels.hpp"
 #include "rt_split.hpp"
@@ -21,6 +24,8 @@
 namespace rt {
 
 namespace {
+
+#define RT_INLINE __attribute__((always_inline))  // lambdas over the wave's registers: a call would put them in memory
 
 constexpr int kTile = 32;
 constexpr int kTermA[6] = {2, 1, 1, 0, 0, 0}, kTermB[6] = {0, 1, 0, 2, 1, 0};  // planes of the six terms, small ones first
@@ -38,81 +43,72 @@ __device__ __forceinline__ void check8(const float (&x)[8], float& chk) {
     chk = split_too_small(m) ? kSplitMost : __builtin_fmaxf(chk, m);
 }
 
-// One streamed matrix [N, D]: a tile's rows and columns on their way from memory into LDS.  Rows behind the last repeat it;
-// whoever reads the tile gives them weights of zero.
-template <int DT, bool kRowsOut, bool kColsOut>
+// One streamed matrix [N, D]: a tile's rows on their way from memory into LDS.  Rows behind the last repeat it; whoever reads
+// the tile gives them weights of zero.
+template <int DT>
 struct Stream {
-    static constexpr int DPAD = 32 * DT, LDK = DPAD + 8, LDV = kTile + 8;
-    static constexpr int RPL = kTile * LDK, CPL = DPAD * LDV;
-    static constexpr int SIZE = (kRowsOut ? 3 * RPL : 0) + (kColsOut ? 3 * CPL : 0);  // bf16 elements of a tile
-    static constexpr int COLS = kRowsOut ? 3 * RPL : 0;                               // where its columns begin
+    using Plane = SplitPlane<DT>;
+    static constexpr int DPAD = 32 * DT;
+    static constexpr int SIZE = 3 * Plane::SIZE;  // bf16 elements of a tile
     static constexpr int ITEMS = 4 * DPAD;
     f32x4_t r[2];
-    float c[8];
 
-    __device__ __forceinline__ void clear() {
-        r[0] = r[1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int e = 0; e < 8; e++) c[e] = 0.0f;
-    }
-    __device__ __forceinline__ void load(const float* __restrict__ src, int row0, int N, int D, int tid) {
+    __device__ __forceinline__ void clear() { r[0] = r[1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}; }
+    // `at`: byte offset of this thread's piece from a tile's first row.  A tile that ends within N and rows of DPAD columns,
+    // the usual case, cost two loads and no vector instruction.
+    static __device__ __forceinline__ uint32_t piece(int D, int tid) { return 4u * (uint32_t)(tid / (DPAD / 8) * D + 8 * (tid % (DPAD / 8))); }
+    __device__ __forceinline__ void load(const float* __restrict__ src, int row0, int N, int D, int tid, uint32_t at) {
         if (ITEMS % 256 != 0 && tid >= ITEMS) return;
-        if constexpr (kRowsOut) {
-            const int row = min(row0 + tid / (DPAD / 8), N - 1), d = 8 * (tid % (DPAD / 8));
-            const float* x = src + (size_t)row * D + d;
+        if (row0 + kTile <= N && D == DPAD) {  // uniform
+            const char* const x = (const char*)(src + (size_t)row0 * D);
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (d + 4 * u < D) z = *(const f32x4_t*)(x + 4 * u);
-                r[u] = z;
-            }
+            for (int u = 0; u < 2; u++) r[u] = *(const f32x4_t*)(x + at + 16 * u);
+            return;
         }
-        if constexpr (kColsOut) {
-            const int d = tid % DPAD, g = tid / DPAD;
-            const int first = row0 + 16 * (g >> 1) + 4 * (g & 1);
+        const int row = min(row0 + tid / (DPAD / 8), N - 1), d = 8 * (tid % (DPAD / 8));
+        const float* x = src + (size_t)row * D + d;
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int row = min(first + 8 * (e >> 2) + (e & 3), N - 1);
-                c[e] = d < D ? src[(size_t)row * D + d] : 0.0f;
-            }
+        for (int u = 0; u < 2; u++) {
+            f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (d + 4 * u < D) z = *(const f32x4_t*)(x + 4 * u);
+            r[u] = z;
         }
     }
-    // Splitting in twelve steps a row (or column) piece of eight elements: step x is term x % 3 of pair x / 3, the last writes.
+    // Splitting in ten steps a row piece of eight elements, five for either half.
+    static constexpr int STEPS = 2 * SplitQuad::STEPS;
     u32x4_t w[3];
-    SplitPair pair;
+    SplitQuad quad;
     float m;
-    template <bool kCol>
     __device__ __forceinline__ void step(int x, __bf16* buf, int tid, float& chk) {
-        const int e = x / 3, n = x % 3;
-        if (n == 0) pair.r = kCol ? split_f32x2_t{c[2 * e], c[2 * e + 1]} : split_f32x2_t{r[e >> 1][2 * (e & 1)], r[e >> 1][2 * (e & 1) + 1]};
-        w[n][e] = pair.step(n);
-        if (!kCol && n == 2) {  // the columns hold the same values
-            const float x0 = r[e >> 1][2 * (e & 1)], x1 = r[e >> 1][2 * (e & 1) + 1];
-            if (e == 0) m = 0.0f;
-            m = split_max(split_max(m, x0), x1);
-            if (e == 3) chk = split_too_small(m) ? kSplitMost : __builtin_fmaxf(chk, m);
-        }
-        if (x == 11 && (ITEMS % 256 == 0 || tid < ITEMS)) {
-            __bf16* at = kCol ? buf + COLS + (tid % DPAD) * LDV + 8 * (tid / DPAD)
-                              : buf + (tid / (DPAD / 8)) * LDK + 8 * (tid % (DPAD / 8));
+        const int h = x / SplitQuad::STEPS, k = x % SplitQuad::STEPS;
+        if (k == 0) {
 #pragma unroll
-            for (int u = 0; u < 3; u++) *(u32x4_t*)(at + u * (kCol ? CPL : RPL)) = w[u];
+            for (int i = 0; i < 4; i++) quad.r[i] = r[h][i];
         }
+        uint32_t a = 0, b = 0;
+        quad.step(k, a, b);
+        if (k % 2 == 0) {
+            w[k / 2][2 * h] = a;
+            w[k / 2][2 * h + 1] = b;
+        }
+        if (k == 3) {
+            m = split_max(split_max(h == 0 ? 0.0f : m, r[h][0]), r[h][1]);
+            m = split_max(split_max(m, r[h][2]), r[h][3]);
+        }
+        if (h == 1 && k % 2 == 0 && (ITEMS % 256 == 0 || tid < ITEMS))  // a plane at a time: three writes at once hold the wave
+            *(u32x4_t*)(buf + Plane::at(tid / (DPAD / 8), tid % (DPAD / 8)) + (k / 2) * Plane::SIZE) = w[k / 2];
+        if (x == STEPS - 1) chk = split_too_small(m) ? kSplitMost : __builtin_fmaxf(chk, m);
     }
     __device__ __forceinline__ void store(__bf16* buf, int tid, float& chk) {
 #pragma unroll
-        for (int x = 0; x < 12; x++)
-            if constexpr (kRowsOut) step<false>(x, buf, tid, chk);
-#pragma unroll
-        for (int x = 0; x < 12; x++)
-            if constexpr (kColsOut) step<true>(x, buf, tid, chk);
+        for (int x = 0; x < STEPS; x++) step(x, buf, tid, chk);
     }
-    // A operands: chunk j of plane a of row `col`; slots 16j + 8hh .. of plane a of column 32t + col
+    // A operands: chunk j of plane a of row `col`; chunk j of plane a of column 32t + lane % 32
     static __device__ __forceinline__ bf16x8_t row_frag(const __bf16* buf, int a, int j, int col, int hh) {
-        return *(const bf16x8_t*)(buf + a * RPL + col * LDK + 16 * j + 8 * hh);
+        return Plane::row_frag(buf + a * Plane::SIZE, j, col, hh);
     }
-    static __device__ __forceinline__ bf16x8_t col_frag(const __bf16* buf, int a, int t, int j, int col, int hh) {
-        return *(const bf16x8_t*)(buf + COLS + a * CPL + (32 * t + col) * LDV + 16 * j + 8 * hh);
+    static __device__ __forceinline__ bf16x8_t col_frag(const __bf16* buf, int a, int t, int j, int lane) {
+        return Plane::col_frag(buf + a * Plane::SIZE, t, j, lane);
     }
 };
 
@@ -154,16 +150,16 @@ __device__ __forceinline__ void owner_of_block(int& bh, int& blk) {
     }
 }
 
-// Two tiles of both streams in LDS (117 KB at head dim 64): one workgroup a CU, so a wave may have the whole register file.
+// One workgroup a CU at head dim 64, so a wave may have the whole register file.
 template <int DT>
 __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split_kernel(FlashBwdF32Params p) {
     constexpr int DPAD = 32 * DT, KS = DPAD / 16;
-    using St = Stream<DT, true, true>;
+    using St = Stream<DT>;
     constexpr int BUF = 2 * St::SIZE;  // Q, then dO
     __shared__ __attribute__((aligned(16))) __bf16 lds[2 * BUF];
     __shared__ __attribute__((aligned(16))) float stat[2][2][kTile];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hh = lane >> 5;
     const int N = p.seq, D = p.dim;
     int bh, blk;
@@ -204,20 +200,25 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
     q_in.clear();
     o_in.clear();
     float st = 0.0f;  // threads 0..31: the row statistic, 32..63: delta.  Rows beyond seq: +inf, their weights are zeros
-    auto load = [&](int row0) {
-        q_in.load(Qg, row0, N, D, tid);
-        o_in.load(dOg, row0, N, D, tid);
-        if (tid < 64) {
-            const int row = row0 + (tid & 31);
-            st = row < N ? (tid < 32 ? lse : delta)[row] : 0.0f;
-            chk = split_max(chk, st);
-            if (row >= N && tid < 32) st = -neg_inf();
+    const uint32_t piece = St::piece(D, tid);
+    const float* const st_src = tid < 32 ? lse : delta;
+    auto load = [&](int row0) RT_INLINE {
+        q_in.load(Qg, row0, N, D, tid, piece);
+        o_in.load(dOg, row0, N, D, tid, piece);
+        if (wave == 0) st = st_src[min(row0 + (tid & 31), N - 1)];
+    };
+    // (the loaded value is looked at here and not where it is requested: there the wave would wait for it)
+    auto put_stat = [&](int b, int row0) RT_INLINE {
+        if (wave == 0) {
+            const bool in = row0 + (tid & 31) < N;
+            chk = split_max(chk, in ? st : 0.0f);
+            stat[b][tid >> 5][tid & 31] = in ? st : (tid < 32 ? -neg_inf() : 0.0f);
         }
     };
-    auto store = [&](int b) {
+    auto store = [&](int b) RT_INLINE {
         q_in.store(lds + b * BUF, tid, chk);
         o_in.store(lds + b * BUF + St::SIZE, tid, chk);
-        if (tid < 64) stat[b][tid >> 5][tid & 31] = st;
+        put_stat(b, 0);
     };
     // P and dS of one pair of elements from the score-shaped products
     auto weight = [&](float s, float dp, float l, float dl, float& pv, float& ds) {
@@ -230,114 +231,122 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
     store(0);
     const bool uncarried = __syncthreads_or(!(chk < kSplitMost));  // seen already: no step of the loop below
     if (n_tiles > 1) load(kTile);
-    // In a step the next tile (in registers since the step before) is split between the instructions of the score-shaped
-    // products, and the second half of the weights is formed between those of the first half's gradient products: with one
-    // wave a SIMD nothing else would keep both units busy.  The scheduling barriers keep that order.
+    // A step's products, in the order S = Q K^T, dP = dO V^T, dV += P^T dO, dK += dS^T Q: no vector work stands alone.  The next tile (in
+    // registers since the step before) is split between the instructions of S, P is formed and split between those of dP and
+    // the first of dV, dS between those of dV and the first half of dK.  With one wave a SIMD nothing else would keep both
+    // units busy.  The scheduling barriers keep that order.
     for (int tile = 0; tile < (uncarried ? 0 : n_tiles); tile++) {
         const __bf16* qb = lds + (tile & 1) * BUF;
         const __bf16* ob = qb + St::SIZE;
         __bf16* nb = lds + ((tile + 1) & 1) * BUF;  // behind the last tile: a repeat that nobody reads
+        if constexpr (DT > 1) {
+#pragma unroll
+            for (int t = 0; t < DT; t++) asm volatile("" : "+a"(acc_dv[t]), "+a"(acc_dk[t]), "+a"(low_dv[t]), "+a"(low_dk[t]));
+#pragma unroll
+            for (int j = 0; j < KS; j++) asm volatile("" : "+a"(kf[j].p[0]), "+a"(kf[j].p[1]), "+a"(kf[j].p[2]), "+a"(vf[j].p[0]), "+a"(vf[j].p[1]), "+a"(vf[j].p[2]));
+        }
         f32x16_t s, dp;
         zero16(s);
         zero16(dp);
-        bf16x8_t qa[3][KS], oa[2][KS];
+        bf16x8_t fa[3][KS];
         // S in the order of terms of the forward kernel (there K is the A operand): the same bits, which is what makes
         // exp(S - L) of a dominant key one
-        auto read_q = [&](int a) {
+        auto read_plane = [&](const __bf16* buf, int a) RT_INLINE {
 #pragma unroll
-            for (int j = 0; j < KS; j++) qa[a][j] = St::row_frag(qb, a, j, col, hh);
+            for (int j = 0; j < KS; j++) fa[a][j] = St::row_frag(buf, a, j, col, hh);
         };
-        auto read_o = [&](int a) {
+        read_plane(qb, 0);
+        f32x4_t lv[4], dl[4];  // register i of S and dP holds query row 8 (i/4) + 4 hh + i%4 of the tile
+        u32x4_t pw[2][3], dw[2][3];
+        SplitQuad sp;
+        float y[4];
+        // 16 steps a chunk of P (from S, which becomes P), then 16 a chunk of dS: for four elements at a time the three
+        // instructions of each, then their split
+        auto weight_step = [&](int x) RT_INLINE {
+            const int j = (x / 16) & 1, e = (x / 8) & 1, k = x % 8, i0 = 8 * j + 4 * e, g = i0 >> 2;
+            if (k < 3) {
 #pragma unroll
-            for (int j = 0; j < KS; j++) oa[a & 1][j] = St::row_frag(ob, a, j, col, hh);
-        };
-        read_q(0);
-        read_o(2);
-        auto stage = [&](int n) {  // behind instruction n of 12 KS: its share of the 48 steps of the next tile's split
-#pragma unroll
-            for (int x = n * 48 / (12 * KS); x < (n + 1) * 48 / (12 * KS); x++) {
-                St& in = x < 24 ? q_in : o_in;
-                __bf16* to = nb + (x < 24 ? 0 : St::SIZE);
-                if ((x % 24) < 12) in.template step<false>(x % 12, to, tid, chk);
-                else in.template step<true>(x % 12, to, tid, chk);
+                for (int i = 0; i < 4; i++) {
+                    if (x < 32) {
+                        if (k == 0) y[i] = s[i0 + i] * p.scale - lv[g][i];
+                        if (k == 1) y[i] *= kLog2e;
+                        if (k == 2) sp.r[i] = s[i0 + i] = __builtin_amdgcn_exp2f(y[i]);
+                    } else {
+                        if (k == 0) y[i] = dp[i0 + i] - dl[g][i];
+                        if (k == 1) y[i] *= s[i0 + i];
+                        if (k == 2) sp.r[i] = y[i] * p.scale;
+                    }
+                }
+                return;
             }
+            uint32_t a = 0, b = 0;
+            sp.step(k - 3, a, b);
+            if ((k - 3) % 2) return;
+            u32x4_t& w = (x < 32 ? pw : dw)[j][(k - 3) / 2];
+            w[2 * e] = a;
+            w[2 * e + 1] = b;
+        };
+        auto weights = [&](int from, int to, int n, int of) RT_INLINE {  // the n-th of `of` shares of steps from .. to
+#pragma unroll
+            for (int x = from + (to - from) * n / of; x < from + (to - from) * (n + 1) / of; x++) weight_step(x);
             RT_ORDER();
         };
 #pragma unroll
         for (int n = 0; n < 6 * KS; n++) {
             const int term = n / KS, j = n % KS;
-            if (n == 0) read_q(1), read_o(1);
-            if (n == KS) read_q(2), read_o(0);
-            s = mfma_h(qa[kTermB[term]][j], kf[j].p[kTermA[term]], s);
-            stage(2 * n);
-            dp = mfma_h(oa[kTermA[term] & 1][j], vf[j].p[kTermB[term]], dp);
-            stage(2 * n + 1);
+            if (n == 0) read_plane(qb, 1);
+            if (n == KS) read_plane(qb, 2);
+            s = mfma_h(fa[kTermB[term]][j], kf[j].p[kTermA[term]], s);
+#pragma unroll
+            for (int x = n * 2 * St::STEPS / (6 * KS); x < (n + 1) * 2 * St::STEPS / (6 * KS); x++) {
+                if (x < St::STEPS) q_in.step(x, nb, tid, chk);
+                else o_in.step(x - St::STEPS, nb + St::SIZE, tid, chk);
+            }
+            RT_ORDER();
         }
-        if (tid < 64) stat[(tile + 1) & 1][tid >> 5][tid & 31] = st;
+        put_stat((tile + 1) & 1, (tile + 1) * kTile);  // (behind the last tile: nothing is read there)
         if (tile + 2 < n_tiles) load((tile + 2) * kTile);
-        // register i holds query row 8 (i/4) + 4 hh + i%4 of the tile
-        f32x4_t lv[4], dl[4];
+        read_plane(ob, 2);
 #pragma unroll
         for (int g = 0; g < 4; g++) {
             lv[g] = *(const f32x4_t*)(&stat[tile & 1][0][8 * g + 4 * hh]);
             dl[g] = *(const f32x4_t*)(&stat[tile & 1][1][8 * g + 4 * hh]);
         }
-        u32x4_t pw[2][3], dw[2][3];
-        SplitPair sp, sd;
-        auto weight_step = [&](int j, int x) {  // 24 steps a chunk, six a pair
-            const int e = x / 6, n = x % 6, i = 8 * j + 2 * e;
-            if (n < 2) {
-                float pv, ds;
-                weight(s[i + n], dp[i + n], lv[i >> 2][(i & 3) + n], dl[i >> 2][(i & 3) + n], pv, ds);
-                sp.r[n] = pv;
-                sd.r[n] = ds;
-            } else if (n == 2) {
-                pw[j][0][e] = sp.step(0);
-            } else if (n == 3) {
-                pw[j][1][e] = sp.step(1);
-            } else if (n == 4) {
-                pw[j][2][e] = sp.step(2);
-                dw[j][0][e] = sd.step(0);
-            } else {
-                dw[j][1][e] = sd.step(1);
-                dw[j][2][e] = sd.step(2);
-            }
-        };
-        bf16x8_t oc[DT][3], qc[DT][3];
-        auto read_cols = [&](int j, int t) {
+        bf16x8_t ca[DT][3];
+        auto read_cols = [&](const __bf16* buf, int j, int t) RT_INLINE {
 #pragma unroll
-            for (int a = 0; a < 3; a++) {
-                oc[t][a] = St::col_frag(ob, a, t, j, col, hh);
-                qc[t][a] = St::col_frag(qb, a, t, j, col, hh);
-            }
+            for (int a = 0; a < 3; a++) ca[t][a] = St::col_frag(buf, a, t, j, lane);
         };
 #pragma unroll
-        for (int t = 0; t < DT; t++) read_cols(0, t);
+        for (int n = 0; n < 6 * KS; n++) {
+            const int term = n / KS, j = n % KS;
+            if (n == 0) read_plane(ob, 1);
+            if (n == KS) read_plane(ob, 0);
+            if (n == 4 * KS) {
 #pragma unroll
-        for (int x = 0; x < 24; x++) weight_step(0, x);
-        RT_ORDER();
+                for (int t = 0; t < DT; t++) read_cols(ob, 0, t);
+            }
+            dp = mfma_h(fa[kTermA[term]][j], vf[j].p[kTermB[term]], dp);
+            weights(0, 24, n, 6 * KS);
+        }
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int g = 0; g < 2; g++)  // dV, then dK
 #pragma unroll
-            for (int t = 0; t < DT; t++) {
+            for (int j = 0; j < 2; j++)
 #pragma unroll
-                for (int term = 0; term < 6; term++) {
-                    const int n = 6 * t + term;
-                    auto form = [&](int n2) {  // behind instruction n2 of 12 DT: its share of the second chunk's weights
-                        if (j == 1) return;
+                for (int t = 0; t < DT; t++) {
 #pragma unroll
-                        for (int x = n2 * 24 / (12 * DT); x < (n2 + 1) * 24 / (12 * DT); x++) weight_step(1, x);
-                        RT_ORDER();
-                    };
-                    f32x16_t& ov = term == 5 ? acc_dv[t] : low_dv[t];
-                    f32x16_t& ok = term == 5 ? acc_dk[t] : low_dk[t];
-                    ov = mfma_h(oc[t][kTermA[term]], as_frag(pw[j][kTermB[term]]), ov);
-                    form(2 * n);
-                    ok = mfma_h(qc[t][kTermA[term]], as_frag(dw[j][kTermB[term]]), ok);
-                    form(2 * n + 1);
+                    for (int term = 0; term < 6; term++) {
+                        f32x16_t& o = term == 5 ? (g ? acc_dk[t] : acc_dv[t]) : (g ? low_dk[t] : low_dv[t]);
+                        o = mfma_h(ca[t][kTermA[term]], as_frag(g ? dw[j][kTermB[term]] : pw[j][kTermB[term]]), o);
+                        const int n = 6 * t + term;
+                        if (g == 0 && j == 0) weights(24, 36, n, 6 * DT);
+                        if (g == 0 && j == 1) weights(36, 48, n, 6 * DT);
+                        if (g == 1 && j == 0) weights(48, 64, n, 6 * DT);
+                    }
+                    if (j == 0) read_cols(g ? qb : ob, 1, t);
+                    else if (g == 0) read_cols(qb, 0, t);
                 }
-                if (j == 0) read_cols(1, t);
-            }
         __syncthreads();
     }
 
@@ -409,12 +418,11 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
 template <int DT>
 __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_kernel(FlashBwdF32Params p) {
     constexpr int DPAD = 32 * DT, KS = DPAD / 16;
-    using StK = Stream<DT, true, true>;
-    using StV = Stream<DT, true, false>;
-    constexpr int BUF = StK::SIZE + StV::SIZE;
+    using St = Stream<DT>;
+    constexpr int BUF = 2 * St::SIZE;  // K, then V
     __shared__ __attribute__((aligned(16))) __bf16 lds[2 * BUF];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hh = lane >> 5;
     const int N = p.seq, D = p.dim;
     int bh, blk;
@@ -456,17 +464,17 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_k
         zero16(acc[t]);
         zero16(low[t]);
     }
-    StK k_in;
-    StV v_in;
+    St k_in, v_in;
     k_in.clear();
     v_in.clear();
-    auto load = [&](int row0) {
-        k_in.load(Kg, row0, N, D, tid);
-        v_in.load(Vg, row0, N, D, tid);
+    const uint32_t piece = St::piece(D, tid);
+    auto load = [&](int row0) RT_INLINE {
+        k_in.load(Kg, row0, N, D, tid, piece);
+        v_in.load(Vg, row0, N, D, tid, piece);
     };
     auto store = [&](int b) {
         k_in.store(lds + b * BUF, tid, chk);
-        v_in.store(lds + b * BUF + StK::SIZE, tid, chk);
+        v_in.store(lds + b * BUF + St::SIZE, tid, chk);
     };
     // dS of one element from the score-shaped products; register i holds key 8 (i/4) + 4 hh + i%4 of the tile
     auto weight = [&](float s, float dp) {
@@ -486,78 +494,101 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_k
     store(0);
     const bool uncarried = __syncthreads_or(!(chk < kSplitMost));  // seen already: no step of the loop below
     if (n_tiles > 1) load(kTile);
-    for (int tile = 0; tile < (uncarried ? 0 : n_tiles); tile++) {  // a step as in the kernel above
+    for (int tile = 0; tile < (uncarried ? 0 : n_tiles); tile++) {  // a step as in the kernel above, in the order S, dP, dQ
         const __bf16* kb = lds + (tile & 1) * BUF;
-        const __bf16* vb = kb + StK::SIZE;
+        const __bf16* vb = kb + St::SIZE;
         __bf16* nb = lds + ((tile + 1) & 1) * BUF;
+        if constexpr (DT > 1) {
+#pragma unroll
+            for (int t = 0; t < DT; t++) asm volatile("" : "+a"(acc[t]), "+a"(low[t]));
+#pragma unroll
+            for (int j = 0; j < KS; j++) asm volatile("" : "+a"(qf[j].p[0]), "+a"(qf[j].p[1]), "+a"(qf[j].p[2]), "+a"(of[j].p[0]), "+a"(of[j].p[1]), "+a"(of[j].p[2]));
+        }
         f32x16_t s, dp;
         zero16(s);
         zero16(dp);
-        bf16x8_t ka[2][KS], va[2][KS];
-        auto read_rows = [&](int a) {
+        bf16x8_t fa[2][KS];
+        auto read_plane = [&](const __bf16* buf, int a) RT_INLINE {
 #pragma unroll
-            for (int j = 0; j < KS; j++) {
-                ka[a & 1][j] = StK::row_frag(kb, a, j, col, hh);
-                va[a & 1][j] = StV::row_frag(vb, a, j, col, hh);
-            }
+            for (int j = 0; j < KS; j++) fa[a & 1][j] = St::row_frag(buf, a, j, col, hh);
         };
-        read_rows(2);
-        auto stage = [&](int n) {  // behind instruction n of 12 KS: its share of the 36 steps of the next tile's split
+        read_plane(kb, 2);
 #pragma unroll
-            for (int x = n * 36 / (12 * KS); x < (n + 1) * 36 / (12 * KS); x++) {
-                if (x < 12) k_in.template step<false>(x % 12, nb, tid, chk);
-                else if (x < 24) k_in.template step<true>(x % 12, nb, tid, chk);
-                else v_in.template step<false>(x % 12, nb + StK::SIZE, tid, chk);
+        for (int n = 0; n < 6 * KS; n++) {
+            const int term = n / KS, j = n % KS;
+            if (n == 0) read_plane(kb, 1);
+            if (n == KS) read_plane(kb, 0);
+            s = mfma_h(fa[kTermA[term] & 1][j], qf[j].p[kTermB[term]], s);
+#pragma unroll
+            for (int x = n * 2 * St::STEPS / (6 * KS); x < (n + 1) * 2 * St::STEPS / (6 * KS); x++) {
+                if (x < St::STEPS) k_in.step(x, nb, tid, chk);
+                else v_in.step(x - St::STEPS, nb + St::SIZE, tid, chk);
             }
             RT_ORDER();
+        }
+        if (tile + 2 < n_tiles) load((tile + 2) * kTile);
+        read_plane(vb, 2);
+        hide_edge(s, tile * kTile);
+        u32x4_t dw[2][3];
+        SplitQuad sd;
+        float y[4];
+        // 12 steps of P (S becomes P), then 16 a chunk of dS, four elements at a time as in the kernel above
+        auto weight_step = [&](int x) RT_INLINE {
+            const int z = x < 12 ? x / 3 : (x - 12) / 8, k = x < 12 ? x % 3 : (x - 12) % 8, i0 = 4 * z;
+            if (k < 3) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (x < 12) {
+                        if (k == 0) y[i] = s[i0 + i] * p.scale - lse_q;
+                        if (k == 1) y[i] *= kLog2e;
+                        if (k == 2) s[i0 + i] = __builtin_amdgcn_exp2f(y[i]);
+                    } else {
+                        if (k == 0) y[i] = dp[i0 + i] - delta_q;
+                        if (k == 1) y[i] *= s[i0 + i];
+                        if (k == 2) sd.r[i] = y[i] * p.scale;
+                    }
+                }
+                return;
+            }
+            uint32_t a = 0, b = 0;
+            sd.step(k - 3, a, b);
+            if ((k - 3) % 2) return;
+            u32x4_t& w = dw[z / 2][(k - 3) / 2];
+            w[2 * (z & 1)] = a;
+            w[2 * (z & 1) + 1] = b;
+        };
+        auto weights = [&](int from, int to, int n, int of_n) RT_INLINE {
+#pragma unroll
+            for (int x = from + (to - from) * n / of_n; x < from + (to - from) * (n + 1) / of_n; x++) weight_step(x);
+            RT_ORDER();
+        };
+        bf16x8_t kc[DT][3];
+        auto read_cols = [&](int j, int t) RT_INLINE {
+#pragma unroll
+            for (int a = 0; a < 3; a++) kc[t][a] = St::col_frag(kb, a, t, j, lane);
         };
 #pragma unroll
         for (int n = 0; n < 6 * KS; n++) {
             const int term = n / KS, j = n % KS;
-            if (n == 0) read_rows(1);
-            if (n == KS) read_rows(0);
-            s = mfma_h(ka[kTermA[term] & 1][j], qf[j].p[kTermB[term]], s);
-            stage(2 * n);
-            dp = mfma_h(va[kTermA[term] & 1][j], of[j].p[kTermB[term]], dp);
-            stage(2 * n + 1);
-        }
-        if (tile + 2 < n_tiles) load((tile + 2) * kTile);
-        hide_edge(s, tile * kTile);
-        u32x4_t dw[2][3];
-        bf16x8_t kc[DT][3];
-        auto read_cols = [&](int j, int t) {
+            if (n == 0) read_plane(vb, 1);
+            if (n == KS) read_plane(vb, 0);
+            if (n == 4 * KS) {
 #pragma unroll
-            for (int a = 0; a < 3; a++) kc[t][a] = StK::col_frag(kb, a, t, j, col, hh);
-        };
-        SplitPair sd;
-        auto weight_step = [&](int j, int x) {  // 12 steps a chunk, three a pair
-            const int e = x / 3, n = x % 3, i = 8 * j + 2 * e;
-            if (n < 2) {
-                sd.r[n] = weight(s[i + n], dp[i + n]);
-            } else {
-#pragma unroll
-                for (int u = 0; u < 3; u++) dw[j][u][e] = sd.step(u);
+                for (int t = 0; t < DT; t++) read_cols(0, t);
             }
-        };
-#pragma unroll
-        for (int t = 0; t < DT; t++) read_cols(0, t);
-#pragma unroll
-        for (int x = 0; x < 12; x++) weight_step(0, x);
-        RT_ORDER();
+            dp = mfma_h(fa[kTermA[term] & 1][j], of[j].p[kTermB[term]], dp);
+            weights(0, 12, n, 6 * KS);
+        }
+        weights(12, 28, 0, 1);
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int t = 0; t < DT; t++) {
 #pragma unroll
                 for (int term = 0; term < 6; term++) {
-                    const int n = 6 * t + term;
                     f32x16_t& o = term == 5 ? acc[t] : low[t];
                     o = mfma_h(kc[t][kTermA[term]], as_frag(dw[j][kTermB[term]]), o);
-                    if (j == 0) {
-#pragma unroll
-                        for (int x = n * 12 / (6 * DT); x < (n + 1) * 12 / (6 * DT); x++) weight_step(1, x);
-                        RT_ORDER();
-                    }
+                    if (j == 0) weights(28, 44, 6 * t + term, 6 * DT);
                 }
                 if (j == 0) read_cols(1, t);
             }

@@ -36,6 +36,29 @@ struct SplitPair {
     }
 };
 
+// Four values on their way through the split, in five steps of two to six instructions: steps 0, 2 and 4 give the packed h, m
+// and l of either pair.  No instruction needs the one ahead of it: a wave alone on its SIMD issues a vector instruction
+// every 5 clocks where four chains alternate and every 8.6 in a single one (six of them behind a matrix instruction: 38 and
+// 55 clocks).
+struct SplitQuad {
+    static constexpr int STEPS = 5;
+    float r[4], u[4];
+    __device__ __forceinline__ void step(int k, uint32_t& w0, uint32_t& w1) {
+        if (k % 2 == 0) {
+            w0 = __builtin_bit_cast(uint32_t, __builtin_convertvector((split_f32x2_t{r[0], r[1]}), split_bf16x2_t));
+            w1 = __builtin_bit_cast(uint32_t, __builtin_convertvector((split_f32x2_t{r[2], r[3]}), split_bf16x2_t));
+            if (k == 4) return;
+            u[0] = bf16_lo(w0);
+            u[2] = bf16_lo(w1);
+            u[1] = bf16_hi(w0);
+            u[3] = bf16_hi(w1);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) r[i] -= u[i];
+        }
+    }
+};
+
 __device__ __forceinline__ void split2(float x0, float x1, uint32_t (&w)[3]) {
     SplitPair s{{x0, x1}};
 #pragma unroll
@@ -56,6 +79,35 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
     for (int n = 0; n < 3; n++) s.p[n] = __builtin_bit_cast(bf16x8_t, w[n]);
     return s;
 }
+
+// One of the three planes of a tile of 32 rows in LDS, rows of 32 DT bf16 without padding.  The same plane serves as rows
+// (16-byte reads of 16 rows at one slot) and, through the transposing reads, as columns (8 bytes of four rows, 64 bytes of
+// a row side by side): the XOR of the 16-byte slot index spreads the sixteen rows over all banks and keeps the 64 bytes of
+// four rows in four different quarters of them.
+template <int DT>
+struct SplitPlane {
+    static constexpr int DPAD = 32 * DT, SIZE = 32 * DPAD;  // in elements
+    static __device__ __forceinline__ int swizzle(int r) {
+        return DT == 4 ? 4 * (r & 3) + ((r >> 2) & 3) : (DT == 2 ? 4 * ((r >> 1) & 1) + ((r >> 2) & 3) : ((r >> 2) & 3));
+    }
+    static __device__ __forceinline__ int at(int row, int slot) { return row * DPAD + 8 * (slot ^ swizzle(row)); }
+    // A operand over the head dim: elements 16j + 8hh .. of row `col`
+    static __device__ __forceinline__ bf16x8_t row_frag(const __bf16* plane, int j, int col, int hh) {
+        return *(const bf16x8_t*)(plane + at(col, 2 * j + hh));
+    }
+    // A operand over the rows: column 32t + lane % 32, slot e of a lane row 16j + 4hh + 8 (e / 4) + e % 4 -- the order in which
+    // the score-shaped accumulators hold their rows
+    static __device__ __forceinline__ bf16x8_t col_frag(const __bf16* plane, int t, int j, int lane) {
+        typedef short s16x4_t __attribute__((ext_vector_type(4)));
+        const int l = lane & 15, row = (l >> 2) + 4 * (lane >> 5), slot = 4 * t + 2 * ((lane >> 4) & 1) + ((l & 3) >> 1);
+        auto read = [&](int r) __attribute__((always_inline)) {
+            const __bf16* const p = plane + at(r, slot) + 4 * (l & 1);
+            return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4_t __attribute__((address_space(3)))*)(p)));
+        };
+        const u32x2_t lo = read(16 * j + row), hi = read(16 * j + 8 + row);
+        return __builtin_bit_cast(bf16x8_t, u32x4_t{lo[0], lo[1], hi[0], hi[1]});
+    }
+};
 
 // A fixed place in the instruction order: what is written before it stays before it.
 #define RT_ORDER() __builtin_amdgcn_sched_barrier(0)
