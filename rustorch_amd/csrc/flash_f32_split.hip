@@ -1,16 +1,18 @@
 // f32 flash-attention forward on the bf16 matrix cores, every operand as three bf16 terms (rt_split.hpp).
 //
 // A workgroup of four waves owns 128 query rows, 32 a wave; all four walk the same key tiles of 32, which the workgroup
-// splits once and keeps in LDS as three planes of K (rows, the A operand of S^T = K Q^T) and three of V (columns, the A
-// operand of O^T = V^T P^T, the keys of a column in the order the weights sit in the score accumulators).  Q is split once
-// into registers, the weights where they are formed.
+// splits once and keeps in LDS as three planes of rows of K (the A operand of S^T = K Q^T) and three of V, read as columns by
+// the transposing reads (the A operand of O^T = V^T P^T, the keys of a column in the order the weights sit in the score
+// accumulators).  Q is split once into registers, the weights where they are formed.
 //
 // What bounds it: matrix and vector instructions together.  A tile of 32 keys is 48 matrix instructions of 32 clocks and
-// about 400 vector instructions of 4 per wave, and the two add up to the whole of the time (46 % and 55 % of the clocks),
-// whether a SIMD holds one wave or two (1.56 and 1.58 us a tile); 64 matrix instructions of 64 clocks in the f32 kernel.  B=4 H=16 N=1024 D=64: 181 ->
-// 102 us, causal 120 -> 69; B=2 N=2048 336 -> 189, causal 187 -> 119.  Relative error against 64 bits at those sizes
-// 4.2e-7 -> 1.7e-7 and 5.1e-7 -> 2.2e-7 (four instructions round a score at its size instead of 32, one addition a tile
-// the output instead of 16).  Above head dim 64 LDS holds one workgroup a CU: D=128 405 -> 218 us, causal 249 -> 133.
+// about 370 vector instructions of 4 per wave (1.5 us a tile on a SIMD, with one wave or two); 64 matrix instructions of 64
+// clocks in the f32 kernel.  The vector steps are runs of independent instructions between the matrix instructions
+// (SplitQuad).  B=4 H=16 N=1024 D=64: f32 kernel 181 us, V loaded and split by columns 99.3, by rows 96.4; causal 120, 67.1,
+// 65.4; B=2 N=2048 336, 187.8, 183.6; 5 x 16 heads N=777 D=80 unmasked 229 -> 202.  Above head dim 64 a wave has its SIMD to
+// itself: Q in the accumulation registers, D=128 f32 405, 212, 201 us, causal 249, 126, 118.5.  Relative error against 64 bits
+// 4.2e-7 -> 1.7e-7 and 5.1e-7 -> 2.2e-7 at the first and third size (four instructions round a score at its size instead of
+// 32, one addition a tile the output instead of 16).
 #include <type_traits>
 
 #include "rt_common.hpp"
@@ -29,14 +31,12 @@ template <int DT, bool kExactD, bool kCausal>
 __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kernel(FlashF32Params p) {
     constexpr int DPAD = 32 * DT;
     constexpr int KS = DPAD / 16;          // contraction chunks of the score product
-    constexpr int LDK = DPAD + 8;          // bf16 elements: 16-byte reads of 8 rows tile all banks
-    constexpr int LDV = kTile + 8;
-    constexpr int KPL = kTile * LDK, VPL = DPAD * LDV;  // one plane of each
-    constexpr int KBUF = 3 * KPL, VBUF = 3 * VPL;
+    using Plane = SplitPlane<DT>;
+    constexpr int BUF = 3 * Plane::SIZE;   // a tile of K or of V
     constexpr int ITEMS = 4 * DPAD;        // groups of 8 elements of a tile of K (or V)
     constexpr int NI = (ITEMS + 255) / 256;
     // tiles t and t + 1 of K, t to t + 2 of V
-    __shared__ __attribute__((aligned(16))) __bf16 lds[2 * KBUF + 3 * VBUF];
+    __shared__ __attribute__((aligned(16))) __bf16 lds[5 * BUF];
 
     const int Nq = p.seq, N = p.seq_kv ? p.seq_kv : p.seq;
     const int D = kExactD ? DPAD : p.dim;
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
         const int q0 = qblk * 4 * kTile, q0w = q0 + wave * kTile;
         const int q_row = q0w + col;
         float chk = 0.0f;  // the largest magnitude of everything this thread splits
-        float v_max = 0.0f;
+        uint32_t v_least = ~0u;  // the smallest magnitude of what it splits of V, zeros left out: 2 (bits of |x|) - 1
 
         // Q as B operand: chunk j, this lane's 8 elements d = 16j + 8hh ..
         Split8 qf[KS];
@@ -103,112 +103,72 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
         const int wave_end = q0w >= Nq ? 0 : (kCausal ? min(N, q0w + kTile) : N);
         const int n_wave = (wave_end + kTile - 1) / kTile;  // tiles this wave has scores in
 
-        // A tile's way into LDS: 8 elements of a K row per item, and 8 keys of a V column, in the order the weights sit in
-        // the score accumulators (slot 8g + e is key 16 (g/2) + 4 (g%2) + 8 (e/4) + e%4).  Rows behind the last key repeat
+        // A tile's way into LDS: 8 elements of a row per item, of K and of V.  Rows behind the last key repeat
         // it: their weights are exact zeros, and what a zero makes of its value the key itself has made of every row.
-        f32x4_t kreg[NI][2];
-        float vreg[NI][8];
+        f32x4_t kreg[NI][2], vreg[NI][2];
+        uint32_t at[NI];  // byte offsets of this thread's items from a tile's first row
 #pragma unroll
         for (int n = 0; n < NI; n++) {  // threads without an item split zeros
-            kreg[n][0] = kreg[n][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int e = 0; e < 8; e++) vreg[n][e] = 0.0f;
-        }
-        // byte offsets of this thread's items from a tile's first row; the rows of a V item follow at uniform steps
-        uint32_t k_off[NI], v_off[NI];
-#pragma unroll
-        for (int n = 0; n < NI; n++) {
+            kreg[n][0] = kreg[n][1] = vreg[n][0] = vreg[n][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
             const int idx = 256 * n + tid;
-            k_off[n] = 4u * ((uint32_t)(idx / (DPAD / 8)) * (uint32_t)kv_pitch + 8u * (uint32_t)(idx % (DPAD / 8)));
-            const int g = idx / DPAD;
-            v_off[n] = 4u * ((uint32_t)(16 * (g >> 1) + 4 * (g & 1)) * (uint32_t)kv_pitch + (uint32_t)(idx % DPAD));
+            at[n] = 4u * ((uint32_t)(idx / (DPAD / 8)) * (uint32_t)kv_pitch + 8u * (uint32_t)(idx % (DPAD / 8)));
         }
         auto load_tile = [&](int tile) RT_INLINE {
-            if (tile * kTile + kTile <= N) {  // wave-uniform
-                const char* kb = (const char*)(Kg + (size_t)tile * kTile * kv_pitch);
-                const char* vb = (const char*)(Vg + (size_t)tile * kTile * kv_pitch);
-#pragma unroll
-                for (int n = 0; n < NI; n++) {
-                    const int idx = 256 * n + tid;
-                    if (ITEMS % 256 == 0 || idx < ITEMS) {
-#pragma unroll
-                        for (int u = 0; u < 2; u++) {
-                            f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-                            if (kExactD || 8 * (idx % (DPAD / 8)) + 4 * u < D) z = *(const f32x4_t*)(kb + k_off[n] + 16 * u);
-                            kreg[n][u] = z;
-                        }
-#pragma unroll
-                        for (int e = 0; e < 8; e++) {
-                            const char* row = vb + (size_t)(8 * (e >> 2) + (e & 3)) * kv_pitch * 4;
-                            vreg[n][e] = (kExactD || idx % DPAD < D) ? *(const float*)(row + v_off[n]) : 0.0f;
-                        }
-                    }
-                }
-                return;
-            }
+            const bool inside = tile * kTile + kTile <= N;  // wave-uniform
+            const char* kb = (const char*)(Kg + (size_t)tile * kTile * kv_pitch);
+            const char* vb = (const char*)(Vg + (size_t)tile * kTile * kv_pitch);
 #pragma unroll
             for (int n = 0; n < NI; n++) {
-                const int idx = 256 * n + tid;
+                const int idx = 256 * n + tid, d = 8 * (idx % (DPAD / 8));
                 if (ITEMS % 256 == 0 || idx < ITEMS) {
-                    const int r = idx / (DPAD / 8), c = idx % (DPAD / 8);
-                    const float* kr = Kg + (size_t)min(tile * kTile + r, N - 1) * kv_pitch + 8 * c;
+                    const size_t off = inside ? (size_t)at[n] : 4 * ((size_t)(min(tile * kTile + idx / (DPAD / 8), N - 1) - tile * kTile) * kv_pitch + (size_t)d);
 #pragma unroll
                     for (int u = 0; u < 2; u++) {
-                        f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-                        if (kExactD || 8 * c + 4 * u < D) z = *(const f32x4_t*)(kr + 4 * u);
+                        f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f}, y = z;
+                        if (kExactD || d + 4 * u < D) {
+                            z = *(const f32x4_t*)(kb + off + 16 * u);
+                            y = *(const f32x4_t*)(vb + off + 16 * u);
+                        }
                         kreg[n][u] = z;
-                    }
-                    const int d = idx % DPAD, g = idx / DPAD;
-                    const int key0 = tile * kTile + 16 * (g >> 1) + 4 * (g & 1);
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const int key = min(key0 + 8 * (e >> 2) + (e & 3), N - 1);
-                        vreg[n][e] = (kExactD || d < D) ? Vg[(size_t)key * kv_pitch + d] : 0.0f;
+                        vreg[n][u] = y;
                     }
                 }
             }
         };
-        // Splitting: 24 NI steps, three for each pair of this thread's 8 NI (K and V of an item, four pairs each), then the writes.
-        struct Parts {
-            u32x4_t w[2 * NI][3];
-        };
-        SplitPair pair;
-        auto split_step = [&](Parts& o, int y) RT_INLINE {  // term y % 3 of pair y / 3
-            const int x = y / 3, u = y % 3, n = x / 8, e = x % 4;
-            const bool is_v = (x % 8) >= 4;
-            const float x0 = is_v ? vreg[n][2 * e] : kreg[n][e >> 1][2 * (e & 1)];
-            const float x1 = is_v ? vreg[n][2 * e + 1] : kreg[n][e >> 1][2 * (e & 1) + 1];
-            if (u == 0) pair.r = split_f32x2_t{x0, x1};
-            o.w[2 * n + (is_v ? 1 : 0)][u][e] = pair.step(u);
-            if (u < 2) return;
-            if (is_v) {  // scores of small keys are small whatever is lost of them; small values are the result's size
-                if (e == 0) v_max = 0.0f;
-                v_max = split_max(split_max(v_max, x0), x1);
-                if (e == 3) chk = split_too_small(v_max) ? kSplitMost : __builtin_fmaxf(chk, v_max);
-            } else {
-                chk = split_max(split_max(chk, x0), x1);
-            }
-        };
-        auto write_tile = [&](const Parts& o, __bf16* kbuf, __bf16* vbuf) RT_INLINE {
+        // Splitting: 20 NI steps, five (SplitQuad) for each half of this thread's K and V items; a plane is written as soon as
+        // both halves have given their part of it.
+        constexpr int kSplits = 4 * SplitQuad::STEPS * NI;
+        SplitQuad quad;
+        u32x4_t w[3];
+        auto split_step = [&](int x, __bf16* kbuf, __bf16* vbuf) RT_INLINE {
+            const int k = x % SplitQuad::STEPS, y = x / SplitQuad::STEPS, h = y & 1, n = y >> 2;
+            const bool is_v = (y & 2) != 0;
+            const f32x4_t& in = is_v ? vreg[n][h] : kreg[n][h];
+            if (k == 0) {
 #pragma unroll
-            for (int n = 0; n < NI; n++) {
-                const int idx = 256 * n + tid;
-                if (ITEMS % 256 == 0 || idx < ITEMS) {
-                    const int r = idx / (DPAD / 8), c = idx % (DPAD / 8), d = idx % DPAD, g = idx / DPAD;
-#pragma unroll
-                    for (int u = 0; u < 3; u++) {
-                        *(u32x4_t*)(kbuf + u * KPL + r * LDK + 8 * c) = o.w[2 * n][u];
-                        *(u32x4_t*)(vbuf + u * VPL + d * LDV + 8 * g) = o.w[2 * n + 1][u];
-                    }
-                }
+                for (int i = 0; i < 4; i++) quad.r[i] = in[i];
             }
+            uint32_t a = 0, b = 0;
+            quad.step(k, a, b);
+            if (k % 2 == 0) {
+                w[k / 2][2 * h] = a;
+                w[k / 2][2 * h + 1] = b;
+            } else if (k == 1) {
+                chk = split_max(split_max(chk, in[0]), in[1]);
+                chk = split_max(split_max(chk, in[2]), in[3]);
+            } else if (is_v) {  // scores of small keys are small whatever is lost of them; small values are the result's size
+#pragma unroll
+                for (int i = 0; i < 4; i++) v_least = min(v_least, (__float_as_uint(in[i]) << 1) - 1u);
+            }
+            const int idx = 256 * n + tid;
+            if (h == 1 && k % 2 == 0 && (ITEMS % 256 == 0 || idx < ITEMS))
+                *(u32x4_t*)((is_v ? vbuf : kbuf) + Plane::at(idx / (DPAD / 8), idx % (DPAD / 8)) + (k / 2) * Plane::SIZE) = w[k / 2];
         };
         auto store_tile = [&](__bf16* kbuf, __bf16* vbuf) RT_INLINE {
-            Parts o;
 #pragma unroll
-            for (int x = 0; x < 24 * NI; x++) split_step(o, x);
-            write_tile(o, kbuf, vbuf);
+            for (int x = 0; x < kSplits; x++) split_step(x, kbuf, vbuf);
         };
+        auto carried = [&]() RT_INLINE { return chk < kSplitMost && v_least >= kSplitLeast; };
 
         // A score tile (register i: key 8 (i/4) + 4 hh + i%4, query `col`): scaled and masked, then turned into weights.
         // weights() returns the factor the sums so far have to be multiplied by.
@@ -259,7 +219,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
         bf16x8_t kf[2][KS];
         auto read_plane = [&](const __bf16* kbuf, int a) RT_INLINE {
 #pragma unroll
-            for (int j = 0; j < KS; j++) kf[a & 1][j] = *(const bf16x8_t*)(kbuf + a * KPL + col * LDK + 8 * hh + 16 * j);
+            for (int j = 0; j < KS; j++) kf[a & 1][j] = Plane::row_frag(kbuf + a * Plane::SIZE, j, col, hh);
         };
         auto score_step = [&](const __bf16* kbuf, f32x16_t& s, int n) RT_INLINE {  // n: 0 .. 6 KS - 1, a constant
             const int term = n / KS, j = n % KS;
@@ -272,16 +232,16 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             for (int i = 0; i < 16; i++) x[i] = 0.0f;
         };
 
-        __bf16* const v_lds = lds + 2 * KBUF;
+        __bf16* const v_lds = lds + 2 * BUF;
         load_tile(0);
         store_tile(lds, v_lds);
         if (n_tiles > 1) {
             load_tile(1);
-            store_tile(lds + KBUF, v_lds + VBUF);
+            store_tile(lds + BUF, v_lds + BUF);
         }
         // Seen already: no step of the loop below, straight to the second pass, whose first tile may overwrite what a late
         // wave still reads here for scores that nobody uses then.
-        const bool uncarried = __syncthreads_or(!(chk < kSplitMost));
+        const bool uncarried = __syncthreads_or(!carried());
         f32x16_t s_next;
         zero16(s_next);
         read_plane(lds, 2);
@@ -292,9 +252,12 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
         // the tile after the next is split: the matrix instructions have vector work between them in the same wave.  The
         // scheduling barriers keep that order; left to itself the compiler puts the one kind behind the other.
         for (int tile = 0; tile < (uncarried ? 0 : n_tiles); tile++) {
-            const __bf16* kn = lds + ((tile + 1) & 1) * KBUF;  // behind the last tile: scores of no tile, not used
-            const __bf16* vb = v_lds + v_now * VBUF + col * LDV + 8 * hh;
-            const int v_put = v_now == 0 ? 2 : v_now - 1;  // (tile + 2) % 3
+            const __bf16* kn = lds + ((tile + 1) & 1) * BUF;  // behind the last tile: scores of no tile, not used
+            const __bf16* vb = v_lds + v_now * BUF;
+            if constexpr (DT > 2) {  // what only matrix instructions read goes to the accumulation registers (the sums too: 222 us for 201)
+#pragma unroll
+                for (int j = 0; j < KS; j++) asm volatile("" : "+a"(qf[j].p[0]), "+a"(qf[j].p[1]), "+a"(qf[j].p[2]));
+            }
             if (tile + 2 < n_tiles) load_tile(tile + 2);
             f32x16_t s = s_next;
             scale_mask(s, tile * kTile);
@@ -307,34 +270,43 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             rescale();
             u32x4_t pw[2][3];
             float part[2] = {0.0f, 0.0f};
-            SplitPair sp;
-            auto weight_step = [&](int x) RT_INLINE {  // 16 steps, two a pair
-                const int g = x / 2;
-                if (x % 2 == 0) {
+            SplitQuad sp;
+            float y[4];
+            auto weight_step = [&](int x) RT_INLINE {  // 32 steps: four weights at a time, the three instructions of each, their split
+                const int g = x / 8, k = x % 8;
+                if (k < 3) {
 #pragma unroll
-                    for (int u = 0; u < 2; u++) {
-                        const float e = __builtin_amdgcn_exp2f((s[2 * g + u] - m_use) * kLog2e);
-                        part[u] += e;
-                        sp.r[u] = e;
+                    for (int i = 0; i < 4; i++) {
+                        if (k == 0) y[i] = s[4 * g + i] - m_use;
+                        if (k == 1) y[i] *= kLog2e;
+                        if (k == 2) sp.r[i] = __builtin_amdgcn_exp2f(y[i]);
                     }
-                } else {
+                    if (k == 2) {
 #pragma unroll
-                    for (int u = 0; u < 3; u++) pw[g >> 2][u][g & 3] = sp.step(u);
+                        for (int i = 0; i < 4; i++) part[i & 1] += sp.r[i];
+                    }
+                    return;
                 }
+                uint32_t a = 0, b = 0;
+                sp.step(k - 3, a, b);
+                if ((k - 3) % 2) return;
+                pw[g >> 1][(k - 3) / 2][2 * (g & 1)] = a;
+                pw[g >> 1][(k - 3) / 2][2 * (g & 1) + 1] = b;
             };
             RT_ORDER();
 #pragma unroll
             for (int n = 0; n < 4 * KS; n++) {
                 score_step(kn, s_next, 2 * KS + n);
 #pragma unroll
-                for (int x = n * 16 / (4 * KS); x < (n + 1) * 16 / (4 * KS); x++) weight_step(x);
+                for (int x = n * 32 / (4 * KS); x < (n + 1) * 32 / (4 * KS); x++) weight_step(x);
                 RT_ORDER();
             }
             add_sum(part[0] + part[1]);
             // A tile's product in registers of its own, smallest terms first, then one addition to the sum: in the sum
             // itself each of the twelve instructions would round at its size, and the error against 64 bits grew above
             // that of the f32 kernel.
-            Parts kv_parts;
+            __bf16* const k_put = lds + (tile & 1) * BUF;
+            __bf16* const v_put = v_lds + (v_now == 0 ? 2 : v_now - 1) * BUF;  // tile + 2's
 #pragma unroll
             for (int t = 0; t < DT; t++) {
                 f32x16_t o;
@@ -343,28 +315,27 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
 #pragma unroll
                 for (int a = 2; a >= 0; a--)
 #pragma unroll
-                    for (int j = 0; j < 2; j++) v[a][j] = *(const bf16x8_t*)(vb + a * VPL + t * 32 * LDV + 16 * j);
+                    for (int j = 0; j < 2; j++) v[a][j] = Plane::col_frag(vb + a * Plane::SIZE, t, j, lane);
 #pragma unroll
                 for (int term = 0; term < 6; term++) {
 #pragma unroll
                     for (int j = 0; j < 2; j++) {
                         o = mfma_h(v[kPlaneA[term]][j], __builtin_bit_cast(bf16x8_t, pw[j][kPlaneC[term]]), o);
-                        // its share of the next tile's split: 24 NI steps behind 12 DT instructions
+                        // its share of the next tile's split, behind 12 DT instructions
                         const int n = (6 * t + term) * 2 + j;
 #pragma unroll
-                        for (int x = n * 24 * NI / (12 * DT); x < (n + 1) * 24 * NI / (12 * DT); x++) split_step(kv_parts, x);
+                        for (int x = n * kSplits / (12 * DT); x < (n + 1) * kSplits / (12 * DT); x++) split_step(x, k_put, v_put);
                         RT_ORDER();
                     }
                 }
 #pragma unroll
                 for (int i = 0; i < 16; i++) acc_o[t][i] += o[i];
             }
-            write_tile(kv_parts, lds + (tile & 1) * KBUF, v_lds + v_put * VBUF);
             v_now = v_now == 2 ? 0 : v_now + 1;
             __syncthreads();
         }
 
-        if (uncarried || __syncthreads_or(!(chk < kSplitMost))) {
+        if (uncarried || __syncthreads_or(!carried())) {
             // something here the split does not carry: the rows once more in f32, the tiles through LDS two at a time.  For a
             // launch (B=4 H=16 N=1024 D=64) 158 us where the first tiles show it, 240 where only the last does; straight from
             // memory 770; the f32 kernel alone 181.

@@ -2,7 +2,7 @@
 //
 // x = h + m + l with h = bf16(x), m = bf16(x - h), l = bf16(x - h - m), each rounded to nearest: the differences are
 // exact, and 3 x 8 bits of significand hold all 24 of x (below 2^-109 the last term meets the smallest bf16: an
-// absolute error of 2^-134; a workgroup that reads a group of values below 2^-80 goes by split_too_small).  A product x * y is then the six terms hh, hm, mh, hl, mm, lh; what is left out, ml + lm + ll,
+// absolute error of 2^-134; a workgroup that reads values so small goes by split_too_small or kSplitLeast).  A product x * y is then the six terms hh, hm, mh, hl, mm, lh; what is left out, ml + lm + ll,
 // is below 2^-26 |x y|, less than half of an f32 rounding.  Every term is exact in the f32 accumulator of
 // v_mfma_f32_32x32x16_bf16, whose rate is 16 times that of v_mfma_f32_32x32x2_f32: six of them are 2.7 times the f32 rate.
 //
@@ -119,6 +119,8 @@ __device__ __forceinline__ f32x16_t mfma_h(bf16x8_t a, bf16x8_t b, f32x16_t acc)
 constexpr float kSplitMost = 0x1p30f;  // the magnitude from which on the split products are not used
 // The same for values so small that the last term of the split would count (largest of a group of eight; zeros are fine).
 __device__ __forceinline__ bool split_too_small(float group_max) { return group_max < 0x1p-80f && group_max > 0.0f; }
+// ... and for single values: 2 (bits of |x|) - 1 of 2^-100, from which on the last term of x is no subnormal.
+constexpr uint32_t kSplitLeast = ((uint32_t)(127 - 100) << 24) - 1u;
 // The larger magnitude; a NaN is not seen.
 __device__ __forceinline__ float split_max(float m, float x) { return __builtin_fmaxf(m, __builtin_fabsf(x)); }
 
