@@ -133,6 +133,45 @@ __device__ __forceinline__ u32x4_t t_make_rsrc(const void* base, uint32_t bytes)
                    (uint32_t)__builtin_amdgcn_readfirstlane(bytes), kBufferFlags};
 }
 
+// Where a workgroup works that takes the `pos`-th of the query tiles of `batch` <= 64 sequences, ordered by tile number downwards
+// (tile L of every sequence that has one, by sequence), then those of padded rows only, by tile number.  Lane i holds
+// sequence i; a binary search over the tile number, a sum over the lanes a step.
+struct TilePlace {
+    int b, qtile, len;
+};
+__device__ __forceinline__ int t_lane_sum(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1, 2, 4, 8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return __builtin_amdgcn_readlane(x, 63);
+}
+__device__ __forceinline__ TilePlace t_place_by_length(const int32_t* lens, int batch, int seq, int pos, int lane) {
+    const int len = lane < batch ? min(max(lens[lane], 0), seq) : 0;
+    const int n = (len + TROWS - 1) / TROWS, n_all = (seq + TROWS - 1) / TROWS;  // tiles with valid rows, and all of them
+    const int valid = t_lane_sum(n);
+    const bool padded = pos >= valid;
+    // tiles in front of those numbered L: of higher number, or (padded rows only) of lower
+    auto ahead = [&](int L) __attribute__((always_inline)) { return t_lane_sum(padded ? (lane < batch ? max(L - n, 0) : 0) : max(n - 1 - L, 0)); };
+    const int at = padded ? pos - valid : pos;
+    int lo = 0, hi = n_all - 1;
+    while (lo < hi) {  // padded: the highest L with ahead(L) <= at; else the lowest
+        const int mid = padded ? (lo + hi + 1) >> 1 : (lo + hi) >> 1;
+        const bool in = ahead(mid) <= at;
+        if (padded) {
+            if (in) lo = mid; else hi = mid - 1;
+        } else {
+            if (in) hi = mid; else lo = mid + 1;
+        }
+    }
+    uint64_t has = __ballot(padded ? (lane < batch && n <= lo) : n > lo);  // the sequences with a tile of that number
+    for (int k = at - ahead(lo); k > 0; k--) has &= has - 1;
+    const int b = has ? __builtin_ctzll(has) : 0;
+    return TilePlace{b, lo, __builtin_amdgcn_readlane(len, b)};
+}
+
 // How K/V tiles come into LDS: through registers, or straight there with rows of DP columns or with rows of fewer.
 enum TileWay : int { kTilesRegs = 0, kTilesDirect = 1, kTilesDirectPart = 2 };
 
@@ -233,11 +272,21 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     // The heads of a GQA group follow one another at a distance of kv_heads in the grid, so that a group lands on one XCD
     // (or on those its kv heads leave it) and shares its keys through that L2: grid position x is head x / kv_heads of
     // group x % kv_heads (kv_magic = 2^32 / kv_heads + 1, exact below 2^16 heads; 0 where every head has its own keys).
-    const int b = blockIdx.y;
+    int b = blockIdx.y;
     const int gx = PACKED ? 0 : (int)__umulhi(blockIdx.x, p.kv_magic);
     const int kvh = (int)blockIdx.x - gx * p.kv_heads;
     const int hx = PACKED ? kvh : kvh * p.group + gx;
     const int zz = p.n_qtiles - 1 - (int)blockIdx.z;
+    // A padded batch by length (n_qtiles < 0, tiles_by_length): the position within (batch, rank) is a place in the list of
+    // all sequences' query tiles by their number, which is their cost: the last tile of the longest sequence first, the tiles
+    // of padded rows only last.  Ranked within their own sequence, the second and third tile of the longest one waited behind
+    // first tiles of short ones.
+    constexpr bool kByLength = kCausal && !PACKED && !SPLIT && !WIN;
+    TilePlace place{-1, 0, 0};
+    if (kByLength && p.n_qtiles < 0) {
+        place = t_place_by_length(p.q_lens, (int)gridDim.y, p.seq_q, (int)(blockIdx.y + gridDim.y * blockIdx.z), lane);
+        b = place.b;
+    }
     const int h0 = PACKED ? hx * G : hx;  // head of a row with g = 0
     const int D = p.dim;
 
@@ -364,7 +413,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     auto len_at = [](const int32_t* a, int i) __attribute__((always_inline)) {
         return ((const __attribute__((address_space(4))) int32_t*)(uintptr_t)a)[i];
     };
-    const int q_len_raw = p.q_lens ? len_at(p.q_lens, b) : p.seq_q;
+    const int q_len_raw = p.q_lens ? (kByLength && place.b >= 0 ? place.len : len_at(p.q_lens, b)) : p.seq_q;
     // (a padded batch of self-attention hands over one array for both: one dependent load instead of two in a row)
     const int kv_len_raw = p.kv_lens ? (p.kv_lens == p.q_lens ? q_len_raw : len_at(p.kv_lens, b)) : p.seq_kv;
     const int n_q = min(max(q_len_raw, 0), p.seq_q);  // valid query positions
@@ -379,6 +428,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         const int n_qt = (n_q * G + TROWS - 1) / TROWS;  // tiles with valid rows
         const int rank = (int)blockIdx.z;
         qtile = rank < n_qt ? n_qt - 1 - rank : rank;
+        if (kByLength && place.b >= 0) qtile = place.qtile;
     }
     const int q0 = qtile * TROWS;
     // which 32 query rows of the tile a wave owns.  Wave w runs on SIMD w % 4, and under a causal mask the rows at
@@ -1900,6 +1950,17 @@ hipError_t launch_flash_wide_bf16(hipStream_t stream, const FlashTileParams& par
     return hipGetLastError();
 }
 
+// A padded batch's query tiles in one order over all sequences (at most 64: a lane each): where they do not fit the chip at
+// once, and the walks are long enough to pay for the wait for the lengths ahead of the first request for keys, about 1 us.
+// us, by sequence / by length: B H N shortest head dim 16 16 1024 128 64 29.8 / 27.7, at 128 52.3 / 48.6, 32 8 2000 300 64 82 / 76,
+// 8 32 4096 1000 128 608 / 575; with fewer than eight tiles 64 8 500 64 96 34.7 / 34.6, 12 16 700 100 32 11.9 / 12.6, 22 16 300 60
+// 80 16.3 / 18.6.
+static bool tiles_by_length(const FlashTileParams& p, long long n_qtiles) {
+    return p.q_lens && p.kv_lens == p.q_lens && p.seq_q == p.seq_kv && p.mask == kMaskCausal && p.pack == 1 && !p.decode_rows && p.window == 0 &&
+           p.batch > 1 && p.batch <= 64 && n_qtiles >= 8 &&
+           n_qtiles * p.batch * p.heads > (long long)p.n_cus * flash_tile_bf16_workgroups(p.dim);
+}
+
 hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& params) {
     FlashTileParams p = params;
     if (p.batch == 0 || p.heads == 0 || p.seq_q == 0) return hipSuccess;
@@ -1916,6 +1977,7 @@ hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& par
         return hipErrorInvalidValue;  // the chunked decode only
     if (p.batch > 65535 || n_qtiles * p.n_splits > 65535 || heads_u > 65535 || p.group < 1) return hipErrorInvalidValue;  // grid limits
     set_grid_order(p, n_qtiles * p.n_splits);
+    if (tiles_by_length(p, n_qtiles)) p.n_qtiles = -1;
     dim3 grid((unsigned)heads_u, (unsigned)p.batch, (unsigned)(n_qtiles * p.n_splits));
     if (p.dim <= 32) return launch_dp<32>(stream, p, grid);
     if (p.dim <= 64) return launch_dp<64>(stream, p, grid);

@@ -113,7 +113,7 @@ struct FlashTileParams {
     int seq_kv, dim;
     int kv_heads, group;
     uint32_t kv_magic;        // set by the launcher: 2^32 / kv_heads + 1, for a division by a multiply (0 when group is 1)
-    int n_qtiles;             // set by the launcher: the grid's z
+    int n_qtiles;             // set by the launcher: the grid's z, or -1: query tiles of a padded batch by their number
     // ---- second line
     const uint16_t* q;
     uint16_t* out;

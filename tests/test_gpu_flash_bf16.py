@@ -521,3 +521,34 @@ def test_two_halves_of_the_keys(oracle, n, d):
     ra.synchronize()
     want = oracle.mha_forward_masked(f[0][: tq * h * d], f[1], f[2], 1, tq, n, h, d, bias)
     assert_bf16_parity(oracle.bf16_to_f32(out.download(np.uint16)), want, d, None, f"n={n} d={d} bias")
+
+
+@pytest.mark.parametrize("d", [64, 128, 200])
+@pytest.mark.parametrize("lens", [[1024] * 12, [0, 1024, 1, 128, 129, 1023, 896, 897, 1024, 5, 700, 0], [3] * 11 + [1024],
+                                  [0] * 12, list(range(16, 1024, 16))])
+def test_padded_batch_ordered_by_length(oracle, lens, d):
+    """More query tiles than fit the chip at once and eight or more a sequence: every tile is taken once, whichever
+    sequences have it, and rows behind a sequence's last get the fill value."""
+    b, h, n = len(lens), 16 if len(lens) < 40 else 4, 1024
+    rng = np.random.default_rng(d)
+    bits, f = zip(*(bf16_round(rng.standard_normal((b, h, n, d), dtype=np.float32)) for _ in range(3)))
+    f = [x.reshape(b, h, n, d) for x in f]
+    dq, dk, dv, dl = (dev(x) for x in (*bits, np.asarray(lens, dtype=np.int32)))
+    out = ra.HipStorage(b * h * n * d * 2)
+    out.upload(np.full(b * h * n * d, 0x7B7B, dtype=np.uint16))
+    ra.flash_forward_varlen_bf16_dev(ra.AttentionShape.new(b, h, n, d), dq, dk, dv, dl, out, zero_padded_rows=True)
+    ra.synchronize()
+    got = oracle.bf16_to_f32(out.download(np.uint16)).reshape(b, h, n, d)
+    assert np.isfinite(got).all()
+    for i, ln in enumerate(lens):
+        assert not got[i, :, ln:].any()
+    for i in sorted({0, b // 2, b - 1, int(np.argmax(lens))}):  # whole sequences of some heads; the last valid tile of the others
+        ln = lens[i]
+        if ln == 0:
+            continue
+        q, k, v = (np.ascontiguousarray(x[i, 1, :ln]).ravel() for x in f)
+        want = oracle.flash_forward_masked(oracle.AttentionShape(1, 1, ln, d), q, k, v, "causal")
+        assert_bf16_parity(got[i, 1, :ln].ravel(), want, d, None, f"length {ln} d={d}")
+    for i, ln in enumerate(lens):  # row r weighs row 0 .. r: the first row is V's
+        if ln:
+            assert max_abs(got[i, :, 0], f[2][i, :, 0]) <= TOL
