@@ -490,31 +490,40 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
 
 }  // namespace
 
-// Which of the two kernels has less to do on its busiest SIMD, in tile steps of this file's kernel.  This one spreads
-// 32-row workgroups whose waves share the keys, so it is near the mean of the chip; the split kernel owns 128 rows a
-// workgroup and walks all their keys, at 0.58 of the time per step at head dim 64 (1.6 against 2.83 us per tile of 32 x 32
-// and SIMD) and 0.68 at 32 (1.08 against 1.6); half a step more of fixed cost here.  Without a mask the gradients follow
-// the same rule, so that they form the scores in the order in which the row statistic was formed: their kernels take 0.73
-// and 0.79 of a step, and the line lies where forward and gradients together break even (0.69 and 0.76).  Both sides of it
-// at head dim 64, us here / there: one sequence of 8 heads, 2048 keys 99 / 99 (gradients 250 / 336), causal 55 / 99; 4096
-// keys 331 / 197, causal 175 / 193; 2 x 12 heads, 999 keys 76 / 55 (gradients 200 / 178), causal 50 / 53; 8 x 16 heads,
-// 256 keys 32 / 22 (gradients 89 / 66), causal 31 / 22.  Head dim 128: 8 heads, 2048 keys 191 / 192, 16 heads, 1500 keys
-// 219 / 146, causal 135 / 144; 4 x 16 heads, 1024 keys 405 / 218, causal 249 / 133.
+// Which of the two kernels has less to do on its busiest SIMD, in tile steps of this file's kernel.  The split kernel owns 128
+// rows a workgroup and walks all their keys.
+//
+// Causal, and head dims above 64: this file's kernel spreads 32-row workgroups whose waves share the keys, so it is near the
+// mean of the chip; the split kernel takes 0.58 of the time per step at head dim 64 (1.6 against 2.83 us per tile of 32 x 32
+// and SIMD) and 0.68 at 32 (1.08 against 1.6); half a step more of fixed cost here.  us here / there, head dim 64 causal: one
+// sequence of 8 heads, 2048 keys 55 / 99, 4096 175 / 193; 2 x 12 heads, 999 keys 50 / 53; 8 x 16 heads, 256 keys 31 / 22.
+// Head dim 128: 8 heads, 2048 keys 191 / 192, 16 heads, 1500 keys 219 / 146, causal 135 / 144; 4 x 16 heads, 1024 keys
+// 405 / 218, causal 249 / 133.
+//
+// Without a mask up to head dim 64 the gradients follow the same rule, so that they form the scores in the order in which the
+// row statistic was formed, and the line lies where forward and gradients together break even.  Every workgroup has the
+// same to do there: rounds of 32-row workgroups (one a CU in the gradients at head dim 64, two at 32) with a quarter of the
+// tiles each, against rounds of 128-row ones at 0.5 (0.345) of a step.  us here / there, forward and gradients, B H N at head
+// dim 64: 8 8 256 60 / 63, 8 16 100 37 / 42, 4 8 256 38 / 62, 2 8 512 62 / 100, 1 8 1000 112 / 179; 2 8 1024 181 / 180, 1 8 2048
+// 341 / 336, 2 12 400 91 / 86, 3 16 165 60 / 50, 8 16 200 107 / 64, 1 12 1500 395 / 256; at 32: 4 12 300 46 / 55, 1 8 2048
+// 189 / 260, 4 16 1024 336 / 234.
 static bool flash_f32_split_pays(const FlashF32Params& p) {
     const double n_cus = p.n_cus > 0 ? p.n_cus : 256;
     const long long keys = p.seq_kv ? p.seq_kv : p.seq;
     const double tiles = (double)((keys + 31) / 32), blocks = (p.seq + 127) / 128, n_bh = (double)p.heads * p.batch;
     const bool causal = p.mask == kMaskCausal;
-    const double here = n_bh * ((p.seq + 31) / 32) * (causal ? (tiles + 1) / 2 : tiles) / (4 * n_cus);
     const double per_cu = n_bh * blocks / n_cus;
+    if (!causal && p.dim <= 64) {
+        const double rounds = __builtin_ceil(n_bh * ((p.seq + 31) / 32) / (p.dim > 32 ? n_cus : 2 * n_cus));
+        return __builtin_ceil(per_cu) * tiles * (p.dim > 32 ? 0.5 : 0.345) < 1.02 * rounds * __builtin_ceil(tiles / 4) - 0.2;
+    }
+    const double here = n_bh * ((p.seq + 31) / 32) * (causal ? (tiles + 1) / 2 : tiles) / (4 * n_cus);
     double there = __builtin_ceil(per_cu) * tiles;
     if (causal) {
         if (p.dim <= 64) there = __builtin_fmax(tiles, 1.1 * per_cu * (tiles + 4) / 2);
         else there = per_cu > 1 ? __builtin_ceil(per_cu / 2) * (tiles + 4) : tiles;  // two blocks a workgroup
     }
-    if (p.dim > 64) return there * 0.55 < here + 0.5;
-    const double step = p.dim > 32 ? (causal ? 0.58 : 0.69) : (causal ? 0.68 : 0.76);
-    return there * step < here + 0.5;
+    return there * (p.dim > 64 ? 0.55 : (p.dim > 32 ? 0.58 : 0.68)) < here + 0.5;
 }
 
 // (above head dim 64 the gradients have no such form, and a row statistic they read is formed as they form the scores)
