@@ -526,9 +526,38 @@ static bool flash_f32_split_pays(const FlashF32Params& p) {
     return there * (p.dim > 64 ? 0.55 : (p.dim > 32 ? 0.58 : 0.68)) < here + 0.5;
 }
 
+// The same question between the two forms of the split products (flash_f32_split.hip: 128 query rows a workgroup, or 32 and
+// waves that share the keys), up to head dim 64 and for a forward without row statistic, in us beside the launch.  At head
+// dim 64 a tile step of 128 rows takes 1.41 us (1.45 causal, with what its rows of unequal length leave idle), one of the
+// four waves' 3.8 with two workgroups on a CU and 2.2 with one; causal 1.9 a step of the chip's mean and 2.3 for each
+// workgroup of a CU; at 32 0.87 and 1.05, causal 1.02 and 1.05 with 1.3 a workgroup.  us, 128 rows / shared keys, B H N at
+// head dim 64: 1 8 2048 94 / 69, causal 91 / 43; 8 8 256 17.0 / 14.5; 2 12 400 23 / 19; 1 12 1500 69 / 72; 5 12 300 20 / 25; 4 16 1024
+// 95 / 129, causal 63 / 85; causal 1 8 4096 173 / 128, 2 12 999 49 / 38, 4 16 512 29 / 32, 8 16 256 19 / 24; at 32: 8 16 300 24 / 21,
+// 4 16 1024 63 / 73, causal 1 8 4096 144 / 78, 2 16 2048 80 / 83.
+static bool flash_f32_rows_pay(const FlashF32Params& p) {
+    const double n_cus = p.n_cus > 0 ? p.n_cus : 256;
+    const long long keys = p.seq_kv ? p.seq_kv : p.seq;
+    const double tiles = (double)((keys + 31) / 32), n_bh = (double)p.heads * p.batch, groups = n_bh * ((p.seq + 31) / 32);
+    const double per_cu = n_bh * ((p.seq + 127) / 128) / n_cus, share = __builtin_ceil(tiles / 4);
+    if (p.mask == kMaskCausal) {
+        const double rows = __builtin_fmax(tiles, 1.1 * per_cu * (tiles + 4) / 2), mean = groups * (tiles + 1) / (8 * n_cus);
+        return p.dim > 32 ? 1.45 * rows < 1.9 * mean + 2.3 * groups / n_cus : 1.02 * rows + 2 < 1.05 * mean + 1.3 * groups / n_cus;
+    }
+    const double rows = __builtin_ceil(per_cu) * tiles;
+    if (p.dim <= 32) return 0.87 * rows < 1.05 * share * groups / n_cus;
+    const double full = __builtin_floor(groups / (2 * n_cus)), rest = groups - full * 2 * n_cus;
+    return 1.41 * rows < share * (3.8 * full + (rest > n_cus ? 3.8 : (rest > 0 ? 2.2 : 0.0)));
+}
+
+constexpr int kSplitKeysFrom = 129;  // keys: below, a wave has one tile at most, and the f32 kernel is level (128 7.1 / 7.4 us)
+static bool flash_f32_takes_split_keys(const FlashF32Params& p) {
+    return (p.seq_kv ? p.seq_kv : p.seq) >= kSplitKeysFrom && flash_f32_split_keys_supported(p);
+}
+
 // (above head dim 64 the gradients have no such form, and a row statistic they read is formed as they form the scores)
 bool flash_f32_takes_split(const FlashF32Params& p, bool with_lse) {
-    return p.dim % 4 == 0 && p.dim <= (with_lse ? 64 : 128) && !p.bias && p.mask != kMaskPadding && flash_f32_split_pays(p);
+    if (p.dim % 4 != 0 || p.dim > (with_lse ? 64 : 128) || p.bias || p.mask == kMaskPadding) return false;
+    return flash_f32_split_pays(p) && (with_lse || !flash_f32_takes_split_keys(p) || flash_f32_rows_pay(p));
 }
 
 hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p) {
@@ -548,6 +577,7 @@ hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p) {
         const bool exact = (p.dim % 32 == 0), pad = (p.mask == kMaskPadding);
         if (p.bias && p.mask != kMaskNone) return hipErrorInvalidValue;  // a bias comes without a mask kind
         if (flash_f32_takes_split(p, p.lse != nullptr)) return launch_flash_f32_split(stream, p);
+        if (flash_f32_takes_split_keys(p)) return launch_flash_f32_split_keys(stream, p);
         const int mode = pad ? 2 : (p.mask == kMaskCausal ? 1 : (p.bias ? 3 : 0));
         auto launch = [&](auto dt_c, auto exact_c) {
             constexpr int kDT = decltype(dt_c)::value;

@@ -410,6 +410,393 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
     }
 }
 
+// 16 bytes per lane from a buffer straight into LDS, lane l at lds_block + 16 l (wave-uniform); past the end of the
+// descriptor zeros.  The lanes outside `on` bring nothing.  Awaited by hand (vmcnt): the compiler does not know of it.
+__device__ __forceinline__ void tile_to_lds(uint64_t on, const u32x4_t& rsrc, uint32_t lane_off, uint32_t off, uint32_t lds_block) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block), so = __builtin_amdgcn_readfirstlane(off);
+    uint64_t all;
+    asm volatile("s_mov_b32 m0, %1\n\ts_and_saveexec_b64 %0, %5\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\ts_mov_b64 exec, %0"
+                 : "=&s"(all)
+                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so), "s"(on)
+                 : "memory", "scc");
+}
+
+// The same products for launches with few rows: a workgroup owns 32 query rows and its four waves share the keys, wave w
+// tiles w, w + 4, ..; each walks alone, without a barrier, and the four (O, m, l) are folded through LDS at the end, as in
+// flash_fwd_f32_splitk_kernel.  A wave's tile of K and its tile of V lie in LDS of its own as they are in memory (16-byte
+// slots of a row XORed with bits of the row), brought there straight; K is requested again once its scores are formed, V
+// once it has been multiplied.  Every wave splits what it reads itself, between the matrix instructions of the piece before.
+//
+// What bounds it: the vector unit, with two workgroups a CU: about 700 instructions a tile and wave, half of them splits of K
+// and V that a workgroup of 128 rows shares.  us, f32 kernel -> this, B H N head dim: causal 1 8 2048 64 55.0 -> 42.9, 2 12 999 64
+// 51.5 -> 39.3, 1 4 3664 32 60.2 -> 48.9; unmasked 1 8 1024 64 28.5 -> 22.9, 1 8 512 64 16.6 -> 13.9; 1 8 2048 64 90.2 -> 68.7 (from 128
+// rows a workgroup).
+template <int DT, bool kExactD, bool kCausal>
+__global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF32Params p) {
+    static_assert(DT <= 2, "two workgroups a CU");
+    constexpr int DPAD = 32 * DT, KS = DPAD / 16, SL = DPAD / 4, NREQ = 4 * DT, ROWB = DPAD * 4;
+    constexpr int TILE = 32 * DPAD;  // floats
+    constexpr int NW = 4, LDO = DPAD + 4;
+    __shared__ __attribute__((aligned(1024))) float lds[NW * 2 * TILE];
+    __shared__ float red_m[NW][kTile], red_l[NW][kTile], fin_inv[kTile];
+    static_assert(2 * TILE >= 32 * LDO, "a wave's partial O fits over its tiles");
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31, hh = lane >> 5;
+    const int Nq = p.seq, N = p.seq_kv ? p.seq_kv : p.seq;
+    const int D = kExactD ? DPAD : p.dim;
+    // (batch, head) and query tile as in flash_fwd_f32_splitk_kernel: a head's tiles on one XCD, and where all workgroups
+    // are resident at once a long and a short one on a CU
+    const int nq = (int)gridDim.x, n_bh = (int)(gridDim.y * gridDim.z);
+    int h = blockIdx.y, b = blockIdx.z;
+    int qtile = nq - 1 - (int)blockIdx.x;
+    if ((n_bh & 7) == 0) {
+        const int lin = (int)blockIdx.x + nq * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z);
+        const int xcd = lin & 7, r = lin >> 3, half = (nq * (n_bh >> 3)) >> 1;
+        const int bh = (r / nq) * 8 + xcd;
+        qtile = nq - 1 - r % nq;
+        if (p.zigzag && r >= half && (half % nq == 0 || nq == 2 * half)) qtile = (r - half) % nq;
+        h = bh % (int)gridDim.y;
+        b = bh / (int)gridDim.y;
+    } else if (p.zigzag && ((h + b * (int)gridDim.y) * 2 >= n_bh)) {
+        qtile = (int)blockIdx.x;
+    }
+    const int q0 = qtile * kTile, q_row = q0 + col;
+    const int kvh = h / p.group;
+    const float* __restrict__ Qg = p.q + (size_t)b * p.lq.batch_stride + (size_t)h * p.lq.head_stride;
+    const float* __restrict__ Kg = p.k + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
+    const float* __restrict__ Vg = p.v + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
+    float* __restrict__ Og = p.out + (size_t)b * p.lo.batch_stride + (size_t)h * p.lo.head_stride;
+    const size_t q_pitch = p.lq.row_pitch, o_pitch = p.lo.row_pitch;
+
+    const int kv_end = kCausal ? min(N, q0 + kTile) : N;
+    const int n_tiles = (kv_end + kTile - 1) / kTile;
+
+    // ---- a wave's tiles: instruction n brings chunks 64 n .. + 63 of 16 bytes, chunk c slot c % SL of row c / SL
+    auto swizzle = [](int r) RT_INLINE { return DT == 2 ? (r & 15) : ((r >> 1) & 7); };
+    unsigned char* const Kw = (unsigned char*)(lds + wave * 2 * TILE);
+    unsigned char* const Vw = Kw + TILE * 4;
+    const uint32_t k_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)Kw, v_lds = k_lds + TILE * 4;
+    const uint32_t pitch_b = (uint32_t)p.lkv.row_pitch * 4u;
+    uint32_t lane_off[NREQ];
+    uint64_t on[NREQ];
+#pragma unroll
+    for (int n = 0; n < NREQ; n++) {
+        const int c = 64 * n + lane, row = c / SL, slot = (c % SL) ^ swizzle(row);
+        lane_off[n] = (uint32_t)row * pitch_b + 16u * (uint32_t)slot;
+        on[n] = kExactD ? ~0ull : __ballot(4 * slot < D);
+        if (!kExactD && 4 * slot >= D) *(u32x4_t*)(Kw + 16 * c) = *(u32x4_t*)(Vw + 16 * c) = u32x4_t{0u, 0u, 0u, 0u};
+    }
+    auto rsrc_of = [&](const float* base) RT_INLINE {
+        const uint64_t a = (uint64_t)(uintptr_t)base;
+        return u32x4_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
+                       (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(N - 1) * pitch_b + 4u * (uint32_t)D), 0x00020000u};
+    };
+    const u32x4_t k_rsrc = rsrc_of(Kg), v_rsrc = rsrc_of(Vg);
+    // (rows behind the last are zeros: their scores are masked, and their weights are zeros.  Tiles behind the last bring
+    // nothing but are requested all the same, so that a wait can count.)
+    auto request = [&](const u32x4_t& rs, uint32_t at, int tile) RT_INLINE {
+        const uint32_t off = (uint32_t)tile * (uint32_t)kTile * pitch_b;
+#pragma unroll
+        for (int n = 0; n < NREQ; n++) tile_to_lds(on[n], rs, lane_off[n], off, at + 1024u * (uint32_t)n);
+    };
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    request(k_rsrc, k_lds, wave);
+    request(v_rsrc, v_lds, wave);
+
+    // ---- operands out of LDS
+    const uint32_t k_base = (uint32_t)(col * ROWB + (((2 * hh) ^ swizzle(col)) * 16));
+    auto read_k = [&](int j, float (&x)[8]) RT_INLINE {  // elements 16j + 8hh .. of key `col`
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const f32x4_t z = *(const f32x4_t*)(Kw + (k_base ^ (uint32_t)((4 * j + u) * 16)));
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[4 * u + i] = z[i];
+        }
+    };
+    auto read_v = [&](int t, int j, float (&x)[8]) RT_INLINE {  // keys 16j + 4hh + 8 (e / 4) + e % 4 of column 32t + col
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int key = 16 * j + 4 * hh + 8 * (e >> 2) + (e & 3);
+            x[e] = *(const float*)(Vw + key * ROWB + ((((32 * t + col) >> 2) ^ swizzle(key)) * 16) + 4 * (col & 3));
+        }
+    };
+
+    float chk = 0.0f;
+    uint32_t v_least = ~0u;
+    Split8 qf[KS];
+#pragma unroll
+    for (int j = 0; j < KS; j++) {
+        float x[8];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+            const int d = 16 * j + 8 * hh + 4 * u;
+            if (q_row < Nq && d < D) z = *(const f32x4_t*)(Qg + (size_t)q_row * q_pitch + d);
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[4 * u + i] = z[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) chk = split_max(chk, x[i]);
+        qf[j] = split8(x);
+    }
+
+    f32x16_t acc_o[DT];
+    auto zero16 = [](f32x16_t& x) RT_INLINE {
+#pragma unroll
+        for (int i = 0; i < 16; i++) x[i] = 0.0f;
+    };
+#pragma unroll
+    for (int t = 0; t < DT; t++) zero16(acc_o[t]);
+    float m_run = neg_inf(), l_run = 0.0f, l_low = 0.0f;
+
+    auto scale_mask = [&](f32x16_t& s, int kv0) RT_INLINE {
+#pragma unroll
+        for (int i = 0; i < 16; i++) s[i] *= p.scale;
+        if ((kv0 + kTile > N) || (kCausal && kv0 + kTile - 1 > q0)) {
+            asm volatile("");  // a branch: the selects cost more than the jump
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int kr = kv0 + 8 * (i >> 2) + 4 * hh + (i & 3);
+                if (kr >= N || (kCausal && kr > q_row)) s[i] = neg_inf();
+            }
+        }
+    };
+    float alpha = 0.0f;
+    auto take_max = [&](const f32x16_t& s) RT_INLINE {
+        float m_tile = neg_inf();  // NaN never wins, as in the reference's `if x > m`
+#pragma unroll
+        for (int i = 0; i < 16; i++) m_tile = __builtin_fmaxf(m_tile, s[i]);
+        auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(m_tile), __float_as_uint(m_tile), false, false);
+        const float m_new = __builtin_fmaxf(__builtin_fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])), m_run);
+        const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
+        alpha = (m_run == neg_inf()) ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_use) * kLog2e);
+        m_run = m_new;
+        return m_use;
+    };
+    auto add_sum = [&](float tile_l) RT_INLINE {
+        const float add = tile_l - l_low * alpha, before = l_run * alpha;
+        l_run = before + add;
+        l_low = (l_run - before) - add;
+    };
+    auto rescale = [&]() RT_INLINE {
+        if (__any(alpha != 1.0f)) {
+#pragma unroll
+            for (int t = 0; t < DT; t++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc_o[t][i] *= alpha;
+        }
+    };
+
+    // An operand on its way through the split: eight values, ten steps (two SplitQuads in turn)
+    struct Piece {
+        float x[8];
+        u32x4_t w[3];
+        SplitQuad quad;
+    };
+    auto piece_step = [&](Piece& o, int x, bool is_v) RT_INLINE {
+        const int hf = x / SplitQuad::STEPS, k = x % SplitQuad::STEPS;
+        if (k == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) o.quad.r[i] = o.x[4 * hf + i];
+        }
+        uint32_t a = 0, b2 = 0;
+        o.quad.step(k, a, b2);
+        if (k % 2 == 0) {
+            o.w[k / 2][2 * hf] = a;
+            o.w[k / 2][2 * hf + 1] = b2;
+        } else if (k == 1) {
+            chk = split_max(split_max(chk, o.x[4 * hf]), o.x[4 * hf + 1]);
+            chk = split_max(split_max(chk, o.x[4 * hf + 2]), o.x[4 * hf + 3]);
+        } else if (is_v) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) v_least = min(v_least, (__float_as_uint(o.x[4 * hf + i]) << 1) - 1u);
+        }
+    };
+    constexpr int kPiece = 2 * SplitQuad::STEPS;
+    constexpr int kPlaneA[6] = {2, 1, 1, 0, 0, 0}, kPlaneC[6] = {0, 1, 0, 2, 1, 0};  // the six terms, the small ones first
+    auto frag = [](u32x4_t x) RT_INLINE { return __builtin_bit_cast(bf16x8_t, x); };
+
+    for (int tile = wave; tile < n_tiles; tile += NW) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NREQ) : "memory");  // K; V may still be on its way
+        // S, the large terms and the small ones in registers of their own; the next chunk of K is split meanwhile
+        f32x16_t s, s_low;
+        zero16(s);
+        zero16(s_low);
+        Piece pc[2];
+        read_k(0, pc[0].x);
+#pragma unroll
+        for (int x = 0; x < kPiece; x++) piece_step(pc[0], x, false);
+#pragma unroll
+        for (int j = 0; j < KS; j++) {
+            if (j + 1 < KS) read_k(j + 1, pc[(j + 1) & 1].x);
+#pragma unroll
+            for (int term = 0; term < 6; term++) {
+                f32x16_t& to = term == 5 ? s : s_low;
+                to = mfma_h(frag(pc[j & 1].w[kPlaneA[term]]), qf[j].p[kPlaneC[term]], to);
+                if (j + 1 < KS) {
+#pragma unroll
+                    for (int x = term * kPiece / 6; x < (term + 1) * kPiece / 6; x++) piece_step(pc[(j + 1) & 1], x, false);
+                }
+                RT_ORDER();
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // K has been read
+        request(k_rsrc, k_lds, tile + NW);
+#pragma unroll
+        for (int i = 0; i < 16; i++) s[i] += s_low[i];
+        scale_mask(s, tile * kTile);
+        const float m_use = take_max(s);
+        rescale();
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NREQ) : "memory");  // V; the next K may be on its way
+        read_v(0, 0, pc[0].x);
+        u32x4_t pw[2][3];
+        float part[2] = {0.0f, 0.0f};
+        SplitQuad sp;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            float y[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) y[i] = (s[4 * g + i] - m_use) * kLog2e;
+#pragma unroll
+            for (int i = 0; i < 4; i++) sp.r[i] = __builtin_amdgcn_exp2f(y[i]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) part[i & 1] += sp.r[i];
+#pragma unroll
+            for (int k = 0; k < SplitQuad::STEPS; k++) {
+                uint32_t a = 0, b2 = 0;
+                sp.step(k, a, b2);
+                if (k % 2) continue;
+                pw[g >> 1][k / 2][2 * (g & 1)] = a;
+                pw[g >> 1][k / 2][2 * (g & 1) + 1] = b2;
+            }
+        }
+        add_sum(part[0] + part[1]);
+#pragma unroll
+        for (int x = 0; x < kPiece; x++) piece_step(pc[0], x, true);
+        // O: a tile's product in registers of its own, the small terms of both halves of the keys first, then one addition
+#pragma unroll
+        for (int t = 0; t < DT; t++) {
+            f32x16_t o;
+            zero16(o);
+            read_v(t, 1, pc[1].x);
+#pragma unroll
+            for (int term = 0; term < 5; term++) {
+                o = mfma_h(frag(pc[0].w[kPlaneA[term]]), frag(pw[0][kPlaneC[term]]), o);
+#pragma unroll
+                for (int x = term * kPiece / 5; x < (term + 1) * kPiece / 5; x++) piece_step(pc[1], x, true);
+                RT_ORDER();
+            }
+            const bf16x8_t head = frag(pc[0].w[0]);
+            if (t + 1 < DT) read_v(t + 1, 0, pc[0].x);
+#pragma unroll
+            for (int term = 0; term < 5; term++) {
+                o = mfma_h(frag(pc[1].w[kPlaneA[term]]), frag(pw[1][kPlaneC[term]]), o);
+                if (t + 1 < DT) {
+#pragma unroll
+                    for (int x = term * kPiece / 5; x < (term + 1) * kPiece / 5; x++) piece_step(pc[0], x, true);
+                }
+                RT_ORDER();
+            }
+            o = mfma_h(head, frag(pw[0][0]), o);
+            o = mfma_h(frag(pc[1].w[0]), frag(pw[1][0]), o);
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc_o[t][i] += o[i];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // V has been read
+        request(v_rsrc, v_lds, tile + NW);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing on its way into LDS that is used otherwise from here on
+
+    if (__syncthreads_or(!(chk < kSplitMost && v_least >= kSplitLeast))) {
+        // something here the split does not carry: the rows once more in f32, out of the same tiles
+#pragma unroll
+        for (int t = 0; t < DT; t++) zero16(acc_o[t]);
+        m_run = neg_inf();
+        l_run = l_low = 0.0f;
+        float q[16 * DT];
+        f32_row<DT>(q, Qg + (size_t)q_row * q_pitch, q_row < Nq, D, hh);
+        for (int tile = wave; tile < n_tiles; tile += NW) {
+            request(k_rsrc, k_lds, tile);
+            request(v_rsrc, v_lds, tile);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            f32x16_t s;
+            zero16(s);
+#pragma unroll
+            for (int j = 0; j < 4 * DT; j++) {  // contraction order 8j + 4hh + i, as f32_row holds the queries
+                const f32x4_t a = *(const f32x4_t*)(Kw + col * ROWB + (((2 * j + hh) ^ swizzle(col)) * 16));
+#pragma unroll
+                for (int i = 0; i < 4; i++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], q[4 * j + i], s, 0, 0, 0);
+            }
+            scale_mask(s, tile * kTile);
+            const float m_use = take_max(s);
+            float tile_l = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                s[i] = __builtin_amdgcn_exp2f((s[i] - m_use) * kLog2e);
+                tile_l += s[i];
+            }
+            add_sum(tile_l);
+            rescale();
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int key = 8 * (i >> 2) + 4 * hh + (i & 3);
+#pragma unroll
+                for (int t = 0; t < DT; t++) {
+                    const float a = *(const float*)(Vw + key * ROWB + ((((32 * t + col) >> 2) ^ swizzle(key)) * 16) + 4 * (col & 3));
+                    acc_o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, s[i], acc_o[t], 0, 0, 0);
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+    }
+
+    // ---- the four partial states (as in flash_fwd_f32_splitk_kernel)
+    {
+        const float l = l_run + other_half(l_run);
+        if (hh == 0) {
+            red_m[wave][col] = m_run;
+            red_l[wave][col] = l;
+        }
+    }
+    __syncthreads();
+    float m_all = neg_inf();
+#pragma unroll
+    for (int w2 = 0; w2 < NW; w2++) m_all = __builtin_fmaxf(m_all, red_m[w2][col]);
+    float l_all = 0.0f, my_f = 0.0f;
+#pragma unroll
+    for (int w2 = 0; w2 < NW; w2++) {
+        const float mw = red_m[w2][col];
+        const float f = (mw == neg_inf()) ? 0.0f : expf(mw - m_all);  // an empty partial weighs nothing
+        l_all += red_l[w2][col] * f;
+        if (w2 == wave) my_f = f;
+    }
+    if (wave == 0 && hh == 0) {
+        const bool good = (l_all > 0.0f) && (fabsf(l_all) != __uint_as_float(0x7f800000u)) && (l_all == l_all);
+        fin_inv[col] = good ? 1.0f / l_all : quiet_nan();
+    }
+    float* const Ow = (float*)Kw;  // this wave's weighted O, as rows [col][d]
+#pragma unroll
+    for (int t = 0; t < DT; t++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            *(f32x4_t*)(Ow + col * LDO + t * 32 + 8 * g + 4 * hh) =
+                f32x4_t{acc_o[t][4 * g] * my_f, acc_o[t][4 * g + 1] * my_f, acc_o[t][4 * g + 2] * my_f, acc_o[t][4 * g + 3] * my_f};
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < DT; n++) {
+        const int idx = 256 * n + tid, r = idx / SL, c = idx % SL;
+        f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w2 = 0; w2 < NW; w2++) sum += *(const f32x4_t*)(lds + w2 * 2 * TILE + r * LDO + 4 * c);
+        const float inv = fin_inv[r];  // NaN marks a row without a valid sum
+        f32x4_t o;
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[i] = (inv == inv) ? sum[i] * inv : quiet_nan();
+        if (q0 + r < Nq && 4 * c < D) *(f32x4_t*)(Og + (size_t)(q0 + r) * o_pitch + 4 * c) = o;
+    }
+}
+
 }  // namespace
 
 hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p_in) {
@@ -442,6 +829,30 @@ hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p_in
         case 4: launch_dt(std::integral_constant<int, 4>{}); break;
         default: return hipErrorInvalidValue;
     }
+    return hipGetLastError();
+}
+
+bool flash_f32_split_keys_supported(const FlashF32Params& p) {
+    const long long keys = p.seq_kv ? p.seq_kv : p.seq;
+    return p.dim <= 64 && p.dim % 4 == 0 && (p.mask == kMaskNone || p.mask == kMaskCausal) && !p.bias && !p.lse && keys > 0 &&
+           (unsigned long long)(keys + 256) * (unsigned long long)p.lkv.row_pitch * 4ull < (1ull << 32);  // 32-bit offsets
+}
+
+hipError_t launch_flash_f32_split_keys(hipStream_t stream, const FlashF32Params& p_in) {
+    FlashF32Params p = p_in;
+    if (!flash_f32_split_keys_supported(p)) return hipErrorInvalidValue;
+    dim3 grid((p.seq + kTile - 1) / kTile, p.heads, p.batch), block(256);
+    p.zigzag = (p.mask == kMaskCausal) && ((long long)grid.x * grid.y * grid.z <= 2ll * p.n_cus) ? 1 : 0;
+    auto launch = [&](auto dt_c, auto exact_c) {
+        constexpr int kDT = decltype(dt_c)::value;
+        constexpr bool kEx = decltype(exact_c)::value;
+        if (p.mask == kMaskCausal) hipLaunchKernelGGL((flash_fwd_f32_split_keys_kernel<kDT, kEx, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((flash_fwd_f32_split_keys_kernel<kDT, kEx, false>), grid, block, 0, stream, p);
+    };
+    if (p.dim == 32) launch(std::integral_constant<int, 1>{}, std::true_type{});
+    else if (p.dim < 32) launch(std::integral_constant<int, 1>{}, std::false_type{});
+    else if (p.dim == 64) launch(std::integral_constant<int, 2>{}, std::true_type{});
+    else launch(std::integral_constant<int, 2>{}, std::false_type{});
     return hipGetLastError();
 }
 

@@ -318,3 +318,78 @@ def test_the_rule_turns_away_what_the_kernels_do_not_take():
     for d, with_lse in ((62, False), (132, False), (256, False), (68, True), (128, True)):
         assert not ra.debug_f32_split_products(big(8, 16, 1024, d), with_lse=with_lse)
     assert not ra.debug_f32_split_products(big(1, 1, 64, 64))
+
+
+# ---- few rows: workgroups of 32 whose waves share the keys
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [4, 20, 32, 36, 60, 64])
+@pytest.mark.parametrize("b,h,n", [(1, 1, 129), (1, 8, 160), (2, 3, 161), (1, 4, 255), (1, 8, 257), (1, 2, 500), (3, 1, 513)])
+def test_few_rows_against_64_bits(b, h, n, d, causal):
+    """One to five tiles a wave, the last one with 1, 31 and 32 keys, head dims that fill the 32 or 64 columns and do not."""
+    assert not ra.debug_f32_split_products(ra.AttentionShape.new(b, h, n, d), ra.Mask.causal() if causal else ra.Mask.none())
+    q, k, v = inputs(b, h, n, d)
+    got, want = run(q, k, v, causal), attention64(q, k, v, causal)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+    assert np.abs(got - want).max() <= 5e-6
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,hkv,n,d", [(8, 2, 200, 64), (4, 1, 333, 20), (6, 3, 161, 32)])
+def test_few_rows_of_grouped_heads_and_rows_apart(h, hkv, n, d, causal):
+    """What lies behind a head's columns in a [batch, seq, heads, dim] row is another head's, here NaN."""
+    b = 2
+    q = seeded_normal((b, h, n, d), 1).reshape(b, h, n, d)
+    k, v = (seeded_normal((b, hkv, n, d), i).reshape(b, hkv, n, d) for i in (2, 3))
+    if hkv > 1:
+        k[:, 1], v[:, 1] = np.nan, np.nan
+    want = attention64(q, np.repeat(k, h // hkv, axis=1), np.repeat(v, h // hkv, axis=1), causal)
+    shape, mask = ra.AttentionShape.new(b, h, n, d), ra.Mask.causal() if causal else ra.Mask.none()
+    got = []
+    for layout, call in ((np.ascontiguousarray, ra.flash_forward_f32_dev), (bnhd, ra.flash_forward_bnhd_f32_dev)):
+        out = ra.HipStorage(q.size * 4)
+        call(shape, dev(layout(q)), dev(layout(k)), dev(layout(v)), out, mask, n_kv_heads=hkv)
+        ra.synchronize()
+        got.append(layout(out.download(np.float32).reshape(layout(q).shape)))
+    assert np.array_equal(got[0], got[1], equal_nan=True)
+    assert np.array_equal(np.isnan(got[0]), np.isnan(want))
+    ok = ~np.isnan(want)
+    assert np.linalg.norm((got[0] - want)[ok]) <= 1e-6 * np.linalg.norm(want[ok])
+
+
+@pytest.mark.parametrize("t_q,t_kv,d", [(1, 300, 64), (33, 129, 60), (70, 1000, 32)])
+def test_few_rows_keys_of_another_length(t_q, t_kv, d):
+    b, h = 2, 3
+    q = seeded_normal((b, h, t_q, d), 1).reshape(b, h, t_q, d)
+    k, v = (seeded_normal((b, h, t_kv, d), i).reshape(b, h, t_kv, d) for i in (2, 3))
+    out = ra.HipStorage(q.size * 4)
+    ra.mha_forward_masked_f32_dev(dev(bnhd(q)), dev(bnhd(k)), dev(bnhd(v)), out, b, t_q, t_kv, h, d)
+    ra.synchronize()
+    got, want = bnhd(out.download(np.float32).reshape(b, t_q, h, d)), attention64(q, k, v, False)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("what", ["q inf", "k inf", "v inf", "q nan", "k nan", "v nan", "k large", "v small", "v zero"])
+def test_few_rows_what_the_split_does_not_carry(what, causal):
+    """Infinities, values from 2^30 on and values of V below 2^-100 send the workgroups that read them to the f32 products; NaN
+    is carried.  Zeros are neither small nor large."""
+    b, h, n, d = 1, 2, 300, 64
+    q, k, v = inputs(b, h, n, d)
+    x = {"q": q, "k": k, "v": v}[what[0]]
+    value = {"inf": np.inf, "nan": np.nan, "large": np.float32(2.0) ** 40, "small": np.float32(1e-33), "zero": 0.0}[what.split()[1]]
+    if what[2:] in ("small", "zero"):
+        x[0, 0] = value
+    else:
+        x[0, 1, 37, 5] = value
+    got = run(q, k, v, causal)
+    want = attention64(q, k, v, causal)
+    if what == "v small":
+        assert np.linalg.norm(got[0, 0].astype(np.float64) - want[0, 0]) <= 1e-6 * np.linalg.norm(want[0, 0])
+    if what in ("v inf", "v nan") and causal:  # rows of the tile that do not see the key: zero times its value, as in every f32 kernel
+        assert np.isfinite(got[0, 1, 64:, :5]).all() and not np.isfinite(got[0, 1, 37:, 5]).any()
+        return
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = np.isfinite(want)
+    assert np.abs(got - want)[ok].max() <= 5e-6
