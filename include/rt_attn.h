@@ -166,7 +166,8 @@ int rt_flash_backward_f32_dev(void *stream, const rt_attention_shape *shape, con
 /* The saved-forward form of the backward, which the header of cpu_backward.rs describes for a GPU path
  * (cpu_backward.rs:3-4, :29-35: "from a saved forward pass (Q, K, V, the softmax statistics m and l, and the upstream
  * gradient dO)"; the reference's CPU function recomputes instead).  rt_flash_forward_stats_f32_dev is the unmasked
- * forward that also writes the row statistic lse[b,h,i] = m_i + ln(l_i) ([batch,heads,seq] f32);
+ * forward that also writes the row statistic lse[b,h,i] = m_i + ln(l_i) ([batch,heads,seq] f32), formed from the scores as
+ * the gradients form them (the plain forward may run another kernel, and its output then differs in the last bits);
  * rt_flash_backward_saved_f32_dev takes that `out` and `lse` back and skips the recomputation.  `workspace`:
  * batch*heads*seq floats (RT_ERR_WORKSPACE_TOO_SMALL otherwise).  dim <= 512 (tuned up to 128). */
 int rt_flash_forward_stats_f32_dev(void *stream, const rt_attention_shape *shape, const float *q, const float *k,

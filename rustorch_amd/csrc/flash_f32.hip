@@ -549,9 +549,16 @@ static bool flash_f32_rows_pay(const FlashF32Params& p) {
     return 1.41 * rows < share * (3.8 * full + (rest > n_cus ? 3.8 : (rest > 0 ? 2.2 : 0.0)));
 }
 
-constexpr int kSplitKeysFrom = 129;  // keys: below, a wave has one tile at most, and the f32 kernel is level (128 7.1 / 7.4 us)
+// Keys from which the shared keys pay: with 128 a wave has one tile at most, and the f32 kernel is level (7.1 / 7.4 us).
+// Unmasked up to head dim 32 it is level up to 256 (us, f32 kernel / shared keys, B H N: 1 8 256 6.9 / 6.8, 2 12 256 7.0 / 6.9,
+// 8 8 256 10.0 / 9.4) and keeps those calls, which then give the bits of the forward that keeps its row statistic; against
+// 128 rows a workgroup they pay there as well (1 8 160 10.5 / 6.7).
+constexpr int kSplitKeysFrom = 129, kSplitKeysFrom32 = 257;
 static bool flash_f32_takes_split_keys(const FlashF32Params& p) {
-    return (p.seq_kv ? p.seq_kv : p.seq) >= kSplitKeysFrom && flash_f32_split_keys_supported(p);
+    if (!flash_f32_split_keys_supported(p)) return false;
+    const long long keys = p.seq_kv ? p.seq_kv : p.seq;
+    const bool level = p.mask == kMaskNone && p.dim <= 32 && !flash_f32_split_pays(p);
+    return keys >= (level ? kSplitKeysFrom32 : kSplitKeysFrom);
 }
 
 // (above head dim 64 the gradients have no such form, and a row statistic they read is formed as they form the scores)

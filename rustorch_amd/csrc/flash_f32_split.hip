@@ -493,8 +493,9 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
                        (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(N - 1) * pitch_b + 4u * (uint32_t)D), 0x00020000u};
     };
     const u32x4_t k_rsrc = rsrc_of(Kg), v_rsrc = rsrc_of(Vg);
-    // (rows behind the last are zeros: their scores are masked, and their weights are zeros.  Tiles behind the last bring
-    // nothing but are requested all the same, so that a wait can count.)
+    // (rows behind the last are zeros: their scores are masked, and their weights are zeros.  Tiles behind the last, whose
+    // offset lies past the descriptor's end, bring zeros too, without a read, but are requested all the same, so that a wait
+    // can count.)
     auto request = [&](const u32x4_t& rs, uint32_t at, int tile) RT_INLINE {
         const uint32_t off = (uint32_t)tile * (uint32_t)kTile * pitch_b;
 #pragma unroll
