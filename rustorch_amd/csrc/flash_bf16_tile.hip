@@ -283,6 +283,8 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     // first tiles of short ones.
     constexpr bool kByLength = kCausal && !PACKED && !SPLIT && !WIN;
     TilePlace place{-1, 0, 0};
+    // (what the first requests need of the arguments is loaded ahead of the branch, not once more behind it)
+    if (kByLength) asm volatile("" ::"s"(p.k), "s"(p.v), "s"(p.lkv.batch_stride), "s"(p.lkv.head_stride), "s"(p.lkv.row_pitch), "s"(p.seq_kv), "s"(p.dim));
     if (kByLength && p.n_qtiles < 0) {
         place = t_place_by_length(p.q_lens, (int)gridDim.y, p.seq_q, (int)(blockIdx.y + gridDim.y * blockIdx.z), lane);
         b = place.b;
@@ -338,7 +340,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     uint64_t dl_k_on[NLD], dl_v_on[NLD];        // and the lanes whose chunk lies within the head dim
 #pragma unroll
     for (int n = 0; n < NLD; n++) {
-        const int c = 64 * (wave + 4 * n) + lane, row = c / SPR, slot = c - row * SPR;
+        const int c = 64 * (wave + 4 * n) + lane, row = (int)((uint32_t)c / SPR), slot = c - row * SPR;
         dl_row[n] = row;
         const int sk = slot ^ swz_k(row), sv = slot ^ swz_v(row);
         dl_k[n] = (uint32_t)row * kv_pitch * 2u + (uint32_t)(16 * sk);
@@ -830,11 +832,12 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
                 for (int ks = 0; ks < KS; ks++)
                     s_a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, load_op(2 * ks, k_at(0, 0), nullptr)), qreg[ks], s_a, 0, 0, 0);
                 // The running max starts at the max of item 0, taken here, so that the first step already runs the
-                // fast path (without it the step would form P twice and rescale an O that is still zero).  The bias and the
-                // masks go on a copy: the step applies them to the scores.
-                f32x16_t s_0 = s_a;
-                mask_item(0, 0, s_0);
-                const float m0 = t_max_with_other_half(t_max16(s_0));
+                // fast path (without it the step would form P twice and rescale an O that is still zero).  A bias goes on a
+                // copy: the step applies it to the scores.  (Masks applied twice change nothing.)
+                f32x16_t s_0;
+                if (BIAS) s_0 = s_a;
+                mask_item(0, 0, BIAS ? s_0 : s_a);
+                const float m0 = t_max_with_other_half(t_max16(BIAS ? s_0 : s_a));
                 if (m0 > neg_inf()) {  // (false for -inf and for NaN: such a row waits for the slow path)
                     m_run = m0;
                     neg_mc = -m0 * cc;
