@@ -823,27 +823,47 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         bf16x8_t p_a[2], p_b[2];  // P(j - 1) and P(j)
         p_a[0] = p_a[1] = p_b[0] = p_b[1] = __builtin_bit_cast(bf16x8_t, u32x4_t{0u, 0u, 0u, 0u});
 
-        // S(0), before the pipeline starts
-        {
+        // A window: the items ahead of the first that a row of the wave sees are left out (1.5 of 10.5 items a wave at 256
+        // keys, 1.5 and more of 4.5 at 64, each on the slow path of rows without a maximum); the wave only keeps its part of
+        // the movement.  us, B H N hd window: 3 12 3001 80 77 35.1 -> 33.3, 2 32 3000 32 500 29.8 -> 27.8.
+        const int j_first = WIN && n_it > 0 ? max(min(n_keys - 1, q0 + 32 * wq + off) - p.window + 1, 0) >> 5 : 0;
+        // Its last rows' first key lies in the item behind, but for a window of 1 mod 32: they get their running max from that
+        // item's scores, once the first step has made them (late_max).  Without a max the wave took the slow path twice, 4 us
+        // of 45 at 4 16 4096 64 256 (40.6 at 257 keys).  Both together: 45.1 -> 42.0, 2 16 2048 64 300 15.7 -> 14.1, 1 32 1000
+        // 128 64 10.9 -> 9.9, 2 32 3000 32 500 30.2 -> 27.3, 1 8 16000 128 2500 165.5 -> 163.8.
+        const bool late = WIN && PIPE && n_it > j_first + 1 && wave_lo_max > 32 * j_first + 31;
+
+        // S of the wave's first item (0, or under a window the first that a row of it sees), before its pipeline starts
 #pragma unroll
-            for (int i = 0; i < 16; i++) s_a[i] = s_b[i] = 0.0f;
-            if (PIPE && n_it > 0) {
+        for (int i = 0; i < 16; i++) s_a[i] = s_b[i] = 0.0f;
+        auto first_scores = [&](int it, int k0, const uint16_t* kp, f32x16_t& s) __attribute__((always_inline)) {
 #pragma unroll
-                for (int ks = 0; ks < KS; ks++)
-                    s_a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, load_op(2 * ks, k_at(0, 0), nullptr)), qreg[ks], s_a, 0, 0, 0);
-                // The running max starts at the max of item 0, taken here, so that the first step already runs the
-                // fast path (without it the step would form P twice and rescale an O that is still zero).  A bias goes on a
-                // copy: the step applies it to the scores.  (Masks applied twice change nothing.)
-                f32x16_t s_0;
-                if (BIAS) s_0 = s_a;
-                mask_item(0, 0, BIAS ? s_0 : s_a);
-                const float m0 = t_max_with_other_half(t_max16(BIAS ? s_0 : s_a));
-                if (m0 > neg_inf()) {  // (false for -inf and for NaN: such a row waits for the slow path)
-                    m_run = m0;
-                    neg_mc = -m0 * cc;
-                }
+            for (int ks = 0; ks < KS; ks++)
+                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, load_op(2 * ks, kp, nullptr)), qreg[ks], s, 0, 0, 0);
+            // The running max starts at the max of this item, taken here, so that the first step already runs the
+            // fast path (without it the step would form P twice and rescale an O that is still zero).  A bias goes on a
+            // copy: the step applies it to the scores.  (Masks applied twice change nothing.)
+            f32x16_t s_0;
+            if (BIAS) s_0 = s;
+            mask_item(it, k0, BIAS ? s_0 : s);
+            const float m0 = t_max_with_other_half(t_max16(BIAS ? s_0 : s));
+            if (m0 > neg_inf()) {  // (false for -inf and for NaN: such a row waits for the slow path)
+                m_run = m0;
+                neg_mc = -m0 * cc;
+            } else if (late) {
+                neg_mc = 0.0f;  // every score of the row is masked, and weighs exp2(-inf + 0)
             }
-        }
+        };
+        auto late_max = [&](int it, int k0, f32x16_t& s) __attribute__((always_inline)) {
+            if (!late) return;
+            mask_item(it, k0, s);
+            const float m1 = t_max_with_other_half(t_max16(s));
+            if (m_run == neg_inf()) {
+                m_run = m1;
+                neg_mc = (m1 == neg_inf()) ? (valid ? __uint_as_float(0x7f800000u) : 0.0f) : -m1 * cc;
+            }
+        };
+        if (PIPE && !WIN && n_it > 0) first_scores(0, 0, k_at(0, 0), s_a);
 
         // O^T += V(j-1)^T . P(j-1)^T alone: behind the wave's last item
         auto drain = [&](const uint16_t* vp) __attribute__((always_inline)) {
@@ -1073,6 +1093,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
                 step(0, k0, k_at(st, 1), (!kLater && t == 0) ? v_at(st, 0) : v_at(st ^ 1, NI - 1), s_a, s_b, p_a, p_b, std::integral_constant<int, 0>{});
                 meet(std::true_type{});
                 park_next(t, kset_c, vset_c, st_c);
+                if (WIN && !kLater && t * NI == j_first) late_max(1, k0 + 32, s_b);
                 step(1, k0 + 32, k_at(st ^ 1, 0), v_at(st, 0), s_b, s_a, p_b, p_a, std::integral_constant<int, DIRECT ? 2 * NLD : 0>{});
             } else {
                 step_a(0, k0, k_at(st ^ 1, 0), (!kLater && t == 0) ? v_at(st, 0) : v_at(st ^ 1, 0));
@@ -1096,14 +1117,33 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             }
             keep_cur = keep_next;
         };
-        int t0 = 0;  // t0 % PF == 0 throughout: the set indices below are compile-time
+        int t0 = 0;  // t0 % PF == 0 throughout (DIRECT knows no sets): the set indices below are compile-time
+        if constexpr (WIN && PIPE) {
+            static_assert(!WIN || !PIPE || (DIRECT && NI == 2), "a window's pipelined walk moves its tiles straight to LDS");
+            using IC0 = std::integral_constant<int, 0>;
+            for (; t0 < j_first / NI; t0++) {
+                meet(std::false_type{});
+                park_next(t0, IC0{}, IC0{}, t0 & 1);
+            }
+            const int st = t0 & 1;
+            if (j_first & 1) {
+                first_scores(1, 32 * j_first, k_at(st, 1), s_b);
+                meet(std::false_type{});
+                park_next(t0, IC0{}, IC0{}, st);
+                step(1, 32 * j_first, k_at(st ^ 1, 0), v_at(st, 0), s_b, s_a, p_b, p_a, IC0{});
+                late_max(0, 32 * j_first + 32, s_a);
+                t0++;
+            } else if (n_it > 0) {
+                first_scores(0, 32 * j_first, k_at(st, 0), s_a);
+            }
+        }
         if (!PIPE) {
             static_assert(PIPE || PF == 1, "the unpipelined walk keeps one register set");
             for (int t = 0; t < n_tiles; t++) {
                 const int st = t & 1;
 #pragma unroll
                 for (int it = 0; it < NI; it++)
-                    if (t * NI + it < n_it)
+                    if (t * NI + it < n_it && t * NI + it >= j_first)
                         step_simple(it, t * KT + 32 * it, k_at(st, it), v_at(st, it));
                 park_k(kreg[0], st ^ 1);
                 park_v(std::integral_constant<int, 0>{}, st ^ 1);
@@ -1116,13 +1156,14 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         }
         const int t_full = PIPE ? n_it / NI : 0;
         if constexpr (DIRECT && !BIAS) {
-            // (the others have no register to spare for the second copy of the tile's code)  Tile 0 on its own, then the tiles in pairs (odd, even) whose LDS stages are compile-time
+            // (the others have no register to spare for the second copy of the tile's code)  Tile 0 (under a window the first
+            // one where it is even) on its own, then the tiles in pairs (odd, even) whose LDS stages are compile-time
             // constants, then what is left of the tiles the wave walks in full
             using IC0 = std::integral_constant<int, 0>;
             using IC1 = std::integral_constant<int, 1>;
-            if (PIPE && t0 < t_full) {
-                walk_full(0, IC0{}, IC0{}, IC0{}, std::false_type{});
-                t0 = 1;
+            if (PIPE && t0 < t_full && (!WIN || (t0 & 1) == 0)) {
+                walk_full(WIN ? t0 : 0, IC0{}, IC0{}, IC0{}, std::false_type{});
+                t0++;
             }
             for (; PIPE && t0 + 2 <= t_full; t0 += 2) {
                 walk_full(t0, IC0{}, IC0{}, IC1{}, std::true_type{});

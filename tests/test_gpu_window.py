@@ -40,6 +40,16 @@ def test_window_matches_the_masked_path_of_multi_head_attention(oracle, b, n, h,
     assert_bf16_parity(got.reshape(b, n, h * d), want.reshape(b, n, h * d), h * d, None, f"window {window}", block_rows=64)
 
 
+@pytest.mark.parametrize("d", [32, 64, 80, 128])
+@pytest.mark.parametrize("window", [30, 31, 32, 34, 63, 96, 97, 159, 191, 257])
+def test_window_where_a_waves_first_item_moves(oracle, d, window):
+    """A wave starts at the 32-key item of its first row's first key: every place of it within a tile, and sequences that
+    end within a wave's rows."""
+    for n in (450, 513):
+        got, want, _ = window_bnhd(oracle, 1, n, 2, 1, d, window, 5 * window + n)
+        assert_bf16_parity(got.reshape(1, n, 2 * d), want.reshape(1, n, 2 * d), 2 * d, None, f"window {window}", block_rows=64)
+
+
 def test_window_of_one_is_v_and_a_window_of_the_sequence_is_the_causal_mask(oracle):
     b, n, h, d = 1, 200, 2, 64
     got, want, (qb, k_rep, v_rep) = window_bnhd(oracle, b, n, h, h, d, 1, 3)
