@@ -552,3 +552,15 @@ def test_padded_batch_ordered_by_length(oracle, lens, d):
     for i, ln in enumerate(lens):  # row r weighs row 0 .. r: the first row is V's
         if ln:
             assert max_abs(got[i, :, 0], f[2][i, :, 0]) <= TOL
+
+
+@pytest.mark.parametrize("h,n,d", [(55, 520, 32), (100, 513, 24), (24, 1282, 64), (24, 1408, 80), (32, 1345, 128), (16, 2200, 128)])
+def test_two_halves_of_the_keys_in_two_rounds(oracle, h, n, d):
+    """Causal launches of one to 1.9 workgroups a CU: the second round of workgroups starts where the first ends."""
+    bits, f = zip(*(bf16_round(seeded_normal(h * n * d, s)) for s in (1, 2, 3)))
+    got = flash_bf16(ra.AttentionShape.new(1, h, n, d), *bits, ra.Mask.causal()).reshape(h, n, d)
+    for i in (0, 7, h // 2, h - 1):
+        q, k, v = (np.ascontiguousarray(x.reshape(h, n, d)[i]).ravel() for x in f)
+        want = oracle.flash_forward_masked(oracle.AttentionShape(1, 1, n, d), q, k, v, "causal")
+        assert_bf16_parity(got[i].ravel(), want, d, n, f"head {i}")
+    assert np.isfinite(got).all()
