@@ -1922,7 +1922,7 @@ hipError_t launch_tiles(hipStream_t stream, const FlashTileParams& p, dim3 grid)
     if (p.mask == kMaskCausal) return launch_one<DP, kMaskCausal, false, false, false, false, TILES>(stream, p, grid);
     return hipErrorInvalidValue;
 }
-// Two halves of the walk (head dims 64 and 128 exactly, up to 32, and 65 to 96) where every workgroup has a CU to itself and
+// Two halves of the walk (head dims 64 and 128 exactly, up to 32, and 65 to 96): where every workgroup has a CU to itself and
 // the walk is long enough to pay for the meeting at its end, 0.6-1.4 us.  us, whole / halves, B H N head dim: causal 1 8 384
 // 64 8.0 / 8.1, 512 9.3 / 9.1, 1024 14.7 / 13.0, 4096 46.2 / 37.4; 1 8 256 128 8.8 / 10.3, 512 12.5 / 13.0, 1024 20.1 / 19.0,
 // 4096 63.9 / 54.3; 1 8 512 96 10.4 / 10.7; unmasked 1 12 1000 96 19.5 / 17.4; 1 8 3000 32 37.2 / 28.2; with a bias 1 8 256 64
@@ -1934,13 +1934,14 @@ hipError_t launch_halves(hipStream_t stream, const FlashTileParams& p, dim3 grid
     if (p.mask == kMaskNone) return launch_one<DP, kMaskNone, false, false, false, false, TILES, true>(stream, p, grid);
     return launch_one<DP, kMaskCausal, false, false, false, false, TILES, true>(stream, p, grid);
 }
-// Up to 1.9 causal workgroups a CU: the long tiles are dispatched first, so that a long walk in halves and a short one behind it
-// take a CU no longer than the longest walk whole, with its neighbour beside it -- from as many query tiles on as pay for two
-// meetings a CU, and above head dim 64 from more where the heads do not divide by the eight XCDs and one gets more of the
-// long tiles, or where nearly every CU takes two.  us, whole / halves, causal B H N: head dim 128 1 32 1501 34.5 / 29.5, 1 16 2500 51.3 / 42.5, 2 8 3000 62.1 / 50.5,
-// 1 12 4096 72.0 / 63.1, 5 8 1400 34.4 / 33.1, 1 10 6000 128 / 106, but 1 28 1600 31.0 / 32.8, 1 28 2048 42.2 / 43.7, 1 40 1409 34.6 / 34.9,
-// 4 12 1024 23.8 / 27.1, 1 32 2048 (two a CU) 44.3 / 44.8; 64 1 32 1501 24.8 / 20.0, 1 28 1600 21.0 / 19.6, but 4 12 1024 15.9 / 16.7; 32
-// 4 16 640 8.9 / 8.6, 5 8 1400 19.9 / 16.6.  Without a mask every walk is as long and halves are slower: 128 1 16 2500 64.6 / 77.0.
+// Up to 1.9 causal workgroups a CU: the long tiles are dispatched first, so that a long walk in halves and a short one behind
+// it take a CU no longer than the longest walk whole, with its neighbour beside it -- from as many query tiles on as pay for
+// two meetings a CU, and above head dim 64 from more where the heads do not divide by the eight XCDs and one gets more of the
+// long tiles, or where nearly every CU takes two.  us, whole / halves, causal B H N: head dim 128 1 32 1501 34.5 / 29.5,
+// 1 16 2500 51.3 / 42.5, 2 8 3000 62.1 / 50.5, 1 12 4096 72.0 / 63.1, 5 8 1400 34.4 / 33.1, 1 10 6000 128 / 106, but 1 28 1600
+// 31.0 / 32.8, 1 28 2048 42.2 / 43.7, 1 40 1409 34.6 / 34.9, 4 12 1024 23.8 / 27.1, 1 32 2048 (two a CU) 44.3 / 44.8; 64
+// 1 32 1501 24.8 / 20.0, 1 28 1600 21.0 / 19.6, but 4 12 1024 15.9 / 16.7; 32 4 16 640 8.9 / 8.6, 5 8 1400 19.9 / 16.6.  Without
+// a mask every walk is as long and halves are slower: 128 1 16 2500 64.6 / 77.0.
 static bool takes_halves(const FlashTileParams& p, dim3 grid) {
     if (p.pack != 1 || p.decode_rows || p.window != 0 || p.mask == kMaskPadding || p.seq_kv < (p.dim <= 64 ? kHalvesFrom64 : kHalvesFrom)) return false;
     const unsigned long long units = (unsigned long long)grid.x * grid.y, n = units * grid.z, n_cus = (unsigned long long)p.n_cus;
