@@ -825,12 +825,14 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
 
         // A window: the items ahead of the first that a row of the wave sees are left out (1.5 of 10.5 items a wave at 256
         // keys, 1.5 and more of 4.5 at 64, each on the slow path of rows without a maximum); the wave only keeps its part of
-        // the movement.  us, B H N hd window: 3 12 3001 80 77 35.1 -> 33.3, 2 32 3000 32 500 29.8 -> 27.8.
+        // the movement.
         const int j_first = WIN && n_it > 0 ? max(min(n_keys - 1, q0 + 32 * wq + off) - p.window + 1, 0) >> 5 : 0;
         // Its last rows' first key lies in the item behind, but for a window of 1 mod 32: they get their running max from that
-        // item's scores, once the first step has made them (late_max).  Without a max the wave took the slow path twice, 4 us
-        // of 45 at 4 16 4096 64 256 (40.6 at 257 keys).  Both together: 45.1 -> 42.0, 2 16 2048 64 300 15.7 -> 14.1, 1 32 1000
-        // 128 64 10.9 -> 9.9, 2 32 3000 32 500 30.2 -> 27.3, 1 8 16000 128 2500 165.5 -> 163.8.
+        // item's scores, once the first step has made them (late_max, on every way into the walk: a row without a maximum
+        // weighs its keys by exp2 of the plain scores).  Without a max the wave took the slow path twice.  Both together, us
+        // with inputs that change from pass to pass, B H N hd window: 4 16 4096 64 256 49.2 -> 47.8, 2 16 2048 64 300 17.7 ->
+        // 17.1, 1 32 1000 128 64 11.7 -> 10.6, 2 32 3000 32 500 34.7 -> 33.4, 1 8 16000 128 2500 165.2 -> 160.9, 3 12 3001 80
+        // 77 30.1 -> 27.8, 4 28 1900 96 150 49.1 -> 45.4.
         const bool late = WIN && PIPE && n_it > j_first + 1 && wave_lo_max > 32 * j_first + 31;
 
         // S of the wave's first item (0, or under a window the first that a row of it sees), before its pipeline starts
@@ -1093,7 +1095,6 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
                 step(0, k0, k_at(st, 1), (!kLater && t == 0) ? v_at(st, 0) : v_at(st ^ 1, NI - 1), s_a, s_b, p_a, p_b, std::integral_constant<int, 0>{});
                 meet(std::true_type{});
                 park_next(t, kset_c, vset_c, st_c);
-                if (WIN && !kLater && t * NI == j_first) late_max(1, k0 + 32, s_b);
                 step(1, k0 + 32, k_at(st ^ 1, 0), v_at(st, 0), s_b, s_a, p_b, p_a, std::integral_constant<int, DIRECT ? 2 * NLD : 0>{});
             } else {
                 step_a(0, k0, k_at(st ^ 1, 0), (!kLater && t == 0) ? v_at(st, 0) : v_at(st ^ 1, 0));
@@ -1135,6 +1136,14 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
                 t0++;
             } else if (n_it > 0) {
                 first_scores(0, 32 * j_first, k_at(st, 0), s_a);
+                if (n_it > j_first + 1) {  // (V of the tile itself has landed by the barrier only, but for tile 0)
+                    step(0, 32 * j_first, k_at(st, 1), t0 == 0 ? v_at(0, 0) : v_at(st ^ 1, 1), s_a, s_b, p_a, p_b, IC0{});
+                    meet(std::true_type{});
+                    park_next(t0, IC0{}, IC0{}, st);
+                    late_max(1, 32 * j_first + 32, s_b);
+                    step(1, 32 * j_first + 32, k_at(st ^ 1, 0), v_at(st, 0), s_b, s_a, p_b, p_a, IC0{});
+                    t0++;
+                }
             }
         }
         if (!PIPE) {
@@ -1156,13 +1165,13 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         }
         const int t_full = PIPE ? n_it / NI : 0;
         if constexpr (DIRECT && !BIAS) {
-            // (the others have no register to spare for the second copy of the tile's code)  Tile 0 (under a window the first
-            // one where it is even) on its own, then the tiles in pairs (odd, even) whose LDS stages are compile-time
-            // constants, then what is left of the tiles the wave walks in full
+            // (the others have no register to spare for the second copy of the tile's code)  Tile 0 (under a window the one
+            // behind the first where it is even) on its own, then the tiles in pairs (odd, even) whose LDS stages are
+            // compile-time constants, then what is left of the tiles the wave walks in full
             using IC0 = std::integral_constant<int, 0>;
             using IC1 = std::integral_constant<int, 1>;
             if (PIPE && t0 < t_full && (!WIN || (t0 & 1) == 0)) {
-                walk_full(WIN ? t0 : 0, IC0{}, IC0{}, IC0{}, std::false_type{});
+                walk_full(WIN ? t0 : 0, IC0{}, IC0{}, IC0{}, std::integral_constant<bool, WIN>{});
                 t0++;
             }
             for (; PIPE && t0 + 2 <= t_full; t0 += 2) {

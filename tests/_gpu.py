@@ -52,6 +52,25 @@ def assert_decode_parity(got, want, dim, label=""):
     assert_bf16_parity(got, want, dim, None, label, block_rows=1, min_elems=64)
 
 
+def assert_within_rounding(got, want, sizes, label=""):
+    """Element by element: a bf16 output is off by its own rounding and by that of the weights, 2^-8 of the value and of
+    `sizes`, the same attention over |V|; 2^-13 of both for the f32 scores (a sum of d products of up to 2^10 in f32, on
+    either side) and exponentials.  A row that has lost its maximum or a key is off by its own size."""
+    got, want, sizes = (np.asarray(x, dtype=np.float64).ravel() for x in (got, want, sizes))
+    assert same_nan_pattern(got, want), f"{label}: NaN pattern differs"
+    over = np.abs(got - want) / ((2.0 ** -8 + 2.0 ** -13) * (np.abs(want) + sizes))
+    worst = int(np.nanargmax(over))
+    assert over[worst] <= 1.0, f"{label}: element {worst} is {got[worst]} and not {want[worst]}, {over[worst]:.2f} of the bound"
+
+
+def with_common_offset(q, k, d, scaled):
+    """q and k [.., d] with one column such that every scaled score is the other columns' minus `scaled`."""
+    a = np.float32(np.sqrt(scaled * np.sqrt(d)))
+    q, k = q.copy(), k.copy()
+    q[..., d // 2], k[..., d // 2] = -a, a
+    return q, k
+
+
 def flash_bf16(shape, q_bits, k_bits, v_bits, mask=None, n_kv_heads=0):
     """Run the bf16 device entry point on host bit-pattern arrays; returns f32 values of the bf16 output."""
     dq, dk, dv = dev(q_bits), dev(k_bits), dev(v_bits)

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import rustorch_amd as ra
-from _gpu import assert_bf16_parity, bf16_round, dev
+from _gpu import assert_bf16_parity, assert_within_rounding, bf16_round, dev, with_common_offset
 from _util import seeded_normal
 
 pytestmark = pytest.mark.gpu
@@ -48,6 +48,30 @@ def test_window_where_a_waves_first_item_moves(oracle, d, window):
     for n in (450, 513):
         got, want, _ = window_bnhd(oracle, 1, n, 2, 1, d, window, 5 * window + n)
         assert_bf16_parity(got.reshape(1, n, 2 * d), want.reshape(1, n, 2 * d), 2 * d, None, f"window {window}", block_rows=64)
+
+
+@pytest.mark.parametrize("d", [32, 64, 80, 128])
+@pytest.mark.parametrize("q_times,offset", [(2.5, 0.0), (3.5, 0.0), (8.0, 0.0), (1.0, 130.0), (3.5, 130.0)])
+def test_window_with_scores_of_any_size(oracle, d, q_times, offset):
+    """Rows whose running max moves far, and rows whose scores all lie near -130, where weights formed without a max are
+    all zero.  Past the start of the sequence the four waves of a workgroup start at the items f .. f + 3 of its tiles, f = 0
+    (windows 34, 50, 64, 100, 300) or 1 (80, 150, 270), and their last rows see their first key an item later."""
+    n, h = 450, 2
+    for window in (34, 50, 64, 80, 100, 150, 270, 300):
+        q, k, v = (seeded_normal((n, h, d), 31 * window + i) for i in range(3))
+        q *= np.float32(q_times)
+        if offset:
+            q, k = with_common_offset(q, k, d, offset)
+        (qb, qf), (kb, kf), (vb, vf) = (bf16_round(x.ravel()) for x in (q, k, v))
+        out = ra.HipStorage(n * h * d * 2)
+        dq, dk, dv = dev(qb), dev(kb), dev(vb)
+        ra.flash_forward_window_bf16_dev(ra.AttentionShape.new(1, h, n, d), dq, dk, dv, out, window, bnhd=True)
+        ra.synchronize()
+        got = oracle.bf16_to_f32(out.download(np.uint16))
+        mask = oracle.sliding_window_mask(n, window)
+        want = oracle.mha_forward_masked(qf, kf, vf, 1, n, n, h, d, attn_mask=mask)
+        sizes = oracle.mha_forward_masked(qf, kf, np.abs(vf), 1, n, n, h, d, attn_mask=mask)
+        assert_within_rounding(got, want, sizes, f"window {window}")
 
 
 def test_window_of_one_is_v_and_a_window_of_the_sequence_is_the_causal_mask(oracle):
