@@ -721,219 +721,6 @@ def main():
                             "traffic": profile_traffic("flash_bwd_f32_b1_h8_n2048_d64.md", "backward_step"),
                             "kernels": "flash_fwd_f32_split_kernel<2> + flash_bwd_f32_dq_split_kernel<2> (with the delta prologue) "
                                        "+ flash_bwd_f32_dkdv_split_kernel<2> (one event pair around the timed steps)"}}
-        # the reference's own call: one sequence per launch (LlmKernels::gqa_decode_online_bf16), back to back on the
-        # stream as a decode loop issues it, on sequence 0's cache
-        single = {}
-        d_o1 = ra.HipStorage(Hq * Dd * 2)
-        for kv_len in (512, 2048, 8192):
-            t1 = time_steps(hip, stream,
-                            lambda i: K.gqa_decode_online_bf16(stream, d_q, sets[i % n_sets][0], sets[i % n_sets][1], d_o1,
-                                                               Hq, Hkv, kv_len, Dd, Lmax),
-                            args.steps, args.warmup, spread_steps=0)
-            single[str(kv_len)] = {"us_per_call": t1.mean_ms * 1e3,
-                                   "GB/s": (2 * Hkv * kv_len * Dd * 2 + 2 * Hq * Dd * 2) / (t1.mean_ms * 1e-3) / 1e9}
-        decode["single_sequence"] = dict(single, note="rt_gqa_decode_online_bf16, 32 q / 8 kv heads, D=128: one launch "
-                                                      "per call, issued back to back from the host")
-        # several new positions of ONE sequence against its long cache, each causal to itself (the reference's
-        # gqa_decode_batched_f32 call shape): the keys are cut into spans, a second kernel folds the partials.  Every
-        # call reads another sequence's slab of the rotated caches (192 slabs of 34 MB), so none finds its keys in
-        # the last-level cache.
-        chunk = {}
-        slab_bytes = Hkv * Lmax * Dd * 2
-        for s_new in (4, 16):
-            q_c = oracle.f32_to_bf16(np.random.default_rng(90 + s_new).standard_normal(s_new * Hq * Dd, dtype=np.float32))
-            d_qc = ra.HipStorage.from_numpy(q_c)
-            d_oc = ra.HipStorage(s_new * Hq * Dd * 2)
-
-            def launch_chunk(i, d_qc=d_qc, d_oc=d_oc, s_new=s_new):
-                k_, v_ = sets[(i // Bd) % n_sets]
-                off = (i % Bd) * slab_bytes
-                K.gqa_decode_chunk_bf16(stream, d_qc, k_.ptr + off, v_.ptr + off, d_oc, Lmax, 1, s_new, Hq, Hkv, Dd, Lmax)
-
-            tc = time_steps(hip, stream, launch_chunk, args.steps, args.warmup)
-            bytes_c = float(2 * Hkv * Lmax * Dd * 2 + 2 * s_new * Hq * Dd * 2)
-            leg_c = {"us_per_call": tc.mean_ms * 1e3, **spread(tc.per), **tc.settle(), "algorithmic_bytes": bytes_c,
-                     "roofline": {"bound": "hbm", "achieved": bytes_c / (tc.mean_ms * 1e-3) / 1e9, "peak": PEAK_HBM_GBS,
-                                  "unit": "GB/s", "frac": bytes_c / (tc.mean_ms * 1e-3) / 1e9 / PEAK_HBM_GBS,
-                                  "traffic": profile_traffic("chunk_decode_b1_hq32_hkv8_d128_ctx8192.md", f"chunk_{s_new}"),
-                                  "kernels": "flash_tile_bf16_kernel<128, causal, packed, split, direct> + flash_split_merge_kernel "
-                                             "(one event pair around the timed calls)"}}
-            if not args.no_cpu:
-                K.gqa_decode_chunk_bf16(stream, d_qc, sets[0][0], sets[0][1], d_oc, Lmax, 1, s_new, Hq, Hkv, Dd, Lmax)
-                hip.sync()
-                got_c = oracle.bf16_to_f32(d_oc.download(np.uint16))
-                n_slab = Hkv * Lmax * Dd
-                t0 = time.perf_counter()
-                want_c = oracle.gqa_decode_chunk_bf16(q_c, kc[:n_slab], vc[:n_slab], [Lmax], 1, s_new, Hq, Hkv, Dd, Lmax,
-                                                      threads=threads)
-                cpu_c = time.perf_counter() - t0
-                err_c = float(np.abs(got_c - want_c).max())
-                rel_c = oracle.rel_fro_blocks(got_c, want_c, Dd, block_rows=1, min_elems=64)
-                leg_c["parity_max_abs"], leg_c["parity_rel_fro"] = err_c, rel_c
-                leg_c["cpu_baseline"] = {"value": bytes_c / cpu_c / 1e9, "unit": "GB/s", "cores": min(threads, Hq),
-                                         "kind": "port",
-                                         "sample": f"one call ({cpu_c * 1e3:.0f} ms): the shader's four phases per (position, "
-                                                   f"head), one task per head; K and V are read once per query head and "
-                                                   f"position there, once per kv head in the byte count"}
-                if not (err_c <= oracle.BF16_MAX_ABS and rel_c <= oracle.BF16_REL_FRO):
-                    print(f"PARITY FAILURE: chunk decode seq_new={s_new} max-abs {err_c}, relative {rel_c}", file=sys.stderr)
-                    sys.exit(1)
-            chunk[str(s_new)] = leg_c
-        decode["chunk_decode"] = dict(chunk, config={"workload": "bf16 chunked causal decode of one sequence: batch 1, 32 q / 8 kv "
-                                                                 "heads, D=128, seq_new new positions (4, 16) over a cache "
-                                                                 "that holds 8192 keys with them (pos_base = 8192 - seq_new), "
-                                                                 "rt_gqa_decode_chunk_bf16 with a host length"})
-        # ---- the step ahead of decode attention (q/k RMSNorm + RoPE + cache append, one launch): a decode step of
-        # the batch, and a prompt of the headline shape
-        prep = {}
-        rope_p = ra.RoPE(Dd, Lmax)
-        rope_p.device_tables()
-        d_g = ra.HipStorage.from_numpy(np.ones(Dd, dtype=np.float32) + 0.01 * np.arange(Dd, dtype=np.float32) / Dd)
-        for name, (pb, pseq) in (("decode_step", (Bd, 1)), ("prompt", (4, 4096))):
-            rng_r = np.random.default_rng(4242 + pseq)
-            pq = oracle.f32_to_bf16(rng_r.standard_normal(pb * Hq * pseq * Dd, dtype=np.float32))
-            pk, pv = (oracle.f32_to_bf16(rng_r.standard_normal(pb * Hkv * pseq * Dd, dtype=np.float32)) for _ in range(2))
-            d_pq, d_pk, d_pv = (ra.HipStorage.from_numpy(x) for x in (pq, pk, pv))
-            k_, v_ = sets[0]  # (pb sequences of the first cache set: positions 0 .. pseq - 1 are overwritten)
-            launch_p = lambda i: K.qk_norm_rope_kv_append_bf16(stream, d_pq, d_pk, d_pv, k_, v_, 0, rope_p, pb, Hq, Hkv, Dd,
-                                                               Lmax, q_gamma=d_g, k_gamma=d_g, seq=pseq)
-            tp = time_steps(hip, stream, launch_p, args.steps, args.warmup)
-            bytes_p = float(pb * pseq * Dd * 2 * (2 * Hq + 4 * Hkv))  # q in and out, k and v in, two cache rows out
-            leg_p = {"us_per_call": tp.mean_ms * 1e3, **spread(tp.per), **tp.settle(), "algorithmic_bytes": bytes_p,
-                     "roofline": {"bound": "hbm", "achieved": bytes_p / (tp.mean_ms * 1e-3) / 1e9, "peak": PEAK_HBM_GBS,
-                                  "unit": "GB/s", "frac": bytes_p / (tp.mean_ms * 1e-3) / 1e9 / PEAK_HBM_GBS,
-                                  "traffic": profile_traffic("prepare_hq32_hkv8_d128.md", name),
-                                  "kernel": "prompt_prepare_kernel<64, 128>" if pseq >= 32 else "decode_prepare_kernel"}}
-            if not args.no_cpu:
-                # q is rewritten in place: a fresh copy of the inputs, one call, every bit against the oracle
-                d_pq.upload(pq)
-                launch_p(0)
-                hip.sync()
-                kc_w = np.zeros(pb * Hkv * pseq * Dd, dtype=np.uint16)  # the oracle's cache holds the new rows only
-                vc_w = np.zeros_like(kc_w)
-                oro_p = oracle.RoPE(Dd, Lmax)
-                oro_p.cos, oro_p.sin = rope_p.cos.copy(), rope_p.sin.copy()
-                g_host = d_g.download(np.float32)
-                t0 = time.perf_counter()
-                want_q = oracle.decode_prepare_bf16(pq, pk, pv, kc_w, vc_w, np.zeros(pb, dtype=np.int32), g_host, g_host, 1e-6,
-                                                    oro_p, pb, Hq, Hkv, Dd, pseq, seq=pseq)
-                cpu_p = time.perf_counter() - t0
-                got_q = d_pq.download(np.uint16)
-                got_kc = k_.download(np.uint16, pb * Hkv * Lmax * Dd).reshape(pb * Hkv, Lmax, Dd)[:, :pseq]
-                got_vc = v_.download(np.uint16, pb * Hkv * Lmax * Dd).reshape(pb * Hkv, Lmax, Dd)[:, :pseq]
-                same = (np.array_equal(got_q, want_q) and np.array_equal(got_kc, kc_w.reshape(pb * Hkv, pseq, Dd))
-                        and np.array_equal(got_vc, vc_w.reshape(pb * Hkv, pseq, Dd)))
-                leg_p["parity_bit_exact"] = bool(same)
-                leg_p["cpu_baseline"] = {"value": bytes_p / cpu_p / 1e9, "unit": "GB/s", "cores": 1, "kind": "port",
-                                         "sample": f"the whole call once ({cpu_p * 1e3:.0f} ms), single-threaded loops as in "
-                                                   f"the reference's decode_step"}
-                if not same:
-                    print(f"PARITY FAILURE: prepare ({name}) differs from the oracle's bits", file=sys.stderr)
-                    sys.exit(1)
-            prep[name] = leg_p
-            del d_pq, d_pk, d_pv
-        decode["prepare"] = dict(prep, config={"workload": "rt_qk_norm_rope_kv_append_bf16, 32 q / 8 kv heads, D=128, both "
-                                                           "gammas: decode_step = batch 64, one new token each; prompt = "
-                                                           "batch 4, 4096 new tokens each at position 0"})
-        if not args.no_cpu:
-            got = oracle.bf16_to_f32(d_o.download(np.uint16))
-            t0 = time.perf_counter()
-            want = oracle.gqa_decode_batched_bf16(qd, kc, vc, lens, Bd, Hq, Hkv, Dd, Lmax, threads=threads)
-            cpu_s = time.perf_counter() - t0
-            err = float(np.abs(got - want).max())
-            rel = oracle.rel_fro_blocks(got, want, Dd, block_rows=1, min_elems=64)  # per (sequence, head) row
-            decode["parity_max_abs"] = err
-            decode["parity_rel_fro"] = rel
-            decode["cpu_baseline"] = {"value": alg_bytes / cpu_s / 1e9, "unit": "GB/s", "cores": threads,
-                                      "kind": "port",
-                                      "sample": f"the whole decode step once ({cpu_s:.1f} s): trim + decode_attn_row "
-                                                f"per (sequence, kv head) task, f32 on bf16-rounded inputs; the "
-                                                f"reference runs seq_q = 1 on a single thread"}
-            if not (err <= oracle.BF16_MAX_ABS and rel <= oracle.BF16_REL_FRO):
-                print(f"PARITY FAILURE: decode max-abs {err}, relative Frobenius error per row {rel}", file=sys.stderr)
-                sys.exit(1)
-
-    # ------------------------------------------------------------------ f32 prefill, the reference's own CPU-runnable case
-    f32 = None
-    if args.only in (None, "f32"):
-        Bf, Hf, Nf, Df = 1, 8, 2048, 64
-        rng_f = np.random.default_rng(77)
-        qf, kf, vf = (rng_f.standard_normal(Bf * Hf * Nf * Df, dtype=np.float32) for _ in range(3))
-        dqf, dkf, dvf = (ra.HipStorage.from_numpy(x) for x in (qf, kf, vf))
-        dof = ra.HipStorage(Bf * Hf * Nf * Df * 4)
-        shape_f = ra.AttentionShape.new(Bf, Hf, Nf, Df)
-        causal_f = ra.Mask.causal()
-        tm = time_steps(hip, stream, lambda i: ra.flash_forward_f32_dev(shape_f, dqf, dkf, dvf, dof, causal_f, stream=stream),
-                        args.steps, args.warmup)
-        flops_f = 4.0 * Bf * Hf * Df * (Nf * (Nf + 1) / 2.0)
-        f32 = {"metric": "f32 prefill attn TFLOP/s", "value": flops_f / (tm.wall_ms / args.steps * 1e-3) / 1e12,
-               "unit": "TFLOP/s", "ms_per_step": tm.wall_ms / args.steps, "kernel_ms_mean": tm.mean_ms, **spread(tm.per),
-               **tm.settle(),
-               "config": {"workload": "f32 causal flash-attention forward, B=1 H=8 N=2048 D=64, N(0,1) inputs (seed 77), "
-                                      "tensors resident in HBM", "flop_convention": "4*B*H*D*N*(N+1)/2 (causal-counted)"},
-               "roofline": {"bound": "mfma", "achieved": flops_f / (tm.mean_ms * 1e-3) / 1e12, "peak": PEAK_F32_TFLOPS,
-                            "unit": "TFLOP/s", "frac": flops_f / (tm.mean_ms * 1e-3) / 1e12 / PEAK_F32_TFLOPS,
-                            "traffic": profile_traffic("flash_fwd_f32_b1_h8_n2048_d64.md", "flash_fwd_f32_split_keys_kernel<2,exact,causal>"), "kernel": "flash_fwd_f32_split_keys_kernel<2, exact, causal>"}}
-        if not args.no_cpu:
-            got = dof.download(np.float32)
-            oracle.flash_forward_masked(oracle.AttentionShape(Bf, Hf, Nf, Df), qf, kf, vf, "causal", threads=threads)  # warm
-            reps = 5
-            t0 = time.perf_counter()
-            for _ in range(reps):
-                want = oracle.flash_forward_masked(oracle.AttentionShape(Bf, Hf, Nf, Df), qf, kf, vf, "causal",
-                                                   threads=threads)
-            cpu_s = (time.perf_counter() - t0) / reps
-            err = float(np.abs(got - want).max())
-            f32["parity_max_abs"] = err
-            f32["parity_rel_fro"] = oracle.rel_fro_blocks(got, want, Df, Nf)
-            f32["cpu_baseline"] = {"value": flops_f / cpu_s / 1e12, "unit": "TFLOP/s", "cores": min(threads, Bf * Hf),
-                                   "kind": "port",
-                                   "sample": f"the whole workload, mean of {reps} runs ({cpu_s * 1e3:.0f} ms each): one task "
-                                             f"per (b,h) slab as rayon does, so at most B*H = 8 threads work; every tile "
-                                             f"computed, causal-counted FLOPs, as in the reference"}
-            if not err <= 1e-5:
-                print(f"PARITY FAILURE: f32 prefill max-abs {err}", file=sys.stderr)
-                sys.exit(1)
-        del dqf, dkf, dvf, dof
-
-    # ------------------------------------------------------------------ f32 backward on the same shape (unmasked, as the reference's)
-    bwd = None
-    if args.only in (None, "bwd"):
-        Bb, Hb, Nb, Db = 1, 8, 2048, 64
-        rng_b = np.random.default_rng(78)
-        n_b = Bb * Hb * Nb * Db
-        host = [rng_b.uniform(-1.0, 1.0, n_b).astype(np.float32) for _ in range(4)]  # q, k, v, dO
-        d_in = [ra.HipStorage.from_numpy(x) for x in host]
-        d_g = [ra.HipStorage(n_b * 4) for _ in range(3)]
-        shape_b = ra.AttentionShape.new(Bb, Hb, Nb, Db)
-        ws_b = ra.flash_backward_workspace_bytes(shape_b)
-        d_ws = ra.HipStorage(ws_b)
-        tm = time_steps(hip, stream, lambda i: ra.flash_backward_f32_dev(shape_b, *d_in, *d_g, d_ws, ws_b, stream=stream),
-                        args.steps, args.warmup)
-        flops_b = 10.0 * Bb * Hb * Db * float(Nb) * Nb
-        # the same gradients from a saved forward (O and m + ln l kept from the forward pass): no recomputation
-        d_o, d_lse = ra.HipStorage(n_b * 4), ra.HipStorage(Bb * Hb * Nb * 4)
-        ra.flash_forward_stats_f32_dev(shape_b, d_in[0], d_in[1], d_in[2], d_o, d_lse, stream=stream)
-        tm_saved = time_steps(hip, stream,
-                              lambda i: ra.flash_backward_saved_f32_dev(shape_b, d_in[0], d_in[1], d_in[2], d_o, d_lse,
-                                                                        d_in[3], *d_g, d_ws, ws_b, stream=stream),
-                              args.steps, args.warmup, spread_steps=0)
-        bwd = {"metric": "f32 attention backward TFLOP/s", "value": flops_b / (tm.wall_ms / args.steps * 1e-3) / 1e12,
-               "unit": "TFLOP/s", "ms_per_step": tm.wall_ms / args.steps, "kernel_ms_mean": tm.mean_ms, **spread(tm.per),
-               **tm.settle(),
-               "saved_forward": {"kernel_ms_mean": tm_saved.mean_ms, "tflops": flops_b / (tm_saved.mean_ms * 1e-3) / 1e12,
-                                 "note": "rt_flash_backward_saved_f32_dev: O and the row statistic come from the forward "
-                                         "pass instead of being recomputed (dQ, which also forms delta, then dK/dV)"},
-               "config": {"workload": "f32 unmasked attention backward (dQ, dK, dV from Q, K, V, dO), B=1 H=8 N=2048 D=64, "
-                                      "U(-1,1) inputs (seed 78), tensors resident in HBM",
-                          "flop_convention": "10*B*H*N*N*D: the five N x N x D products of the backward; the step also "
-                                             "re-runs the forward (2 products) and computes the scores twice (7 products "
-                                             "in the two backward kernels), none of which is counted"},
-               "roofline": {"bound": "mfma", "achieved": flops_b / (tm.mean_ms * 1e-3) / 1e12, "peak": PEAK_F32_TFLOPS,
-                            "unit": "TFLOP/s", "frac": flops_b / (tm.mean_ms * 1e-3) / 1e12 / PEAK_F32_TFLOPS,
-                            "traffic": profile_traffic("flash_bwd_f32_b1_h8_n2048_d64.md", "backward_step"),
-                            "kernels": "flash_fwd_f32_splitk_kernel<2> + flash_bwd_f32_dq_kernel<2> (with the delta prologue) "
-                                       "+ flash_bwd_f32_dkdv_kernel<2> (one event pair around the timed steps)"}}
         if not args.no_cpu:
             n_slab = Bb * Hb  # the reference's backward is a single-threaded loop; the whole workload is a second or two
             slab = Nb * Db
