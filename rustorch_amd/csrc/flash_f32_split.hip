@@ -169,6 +169,17 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             for (int x = 0; x < kSplits; x++) split_step(x, kbuf, vbuf);
         };
         auto carried = [&]() RT_INLINE { return chk < kSplitMost && v_least >= kSplitLeast; };
+        // of this lane's results: one that is no larger than what a small value of V may have lost of itself
+        auto small_result = [&]() RT_INLINE {
+            const float least = (l_run + other_half(l_run)) * kSplitLeastResult;
+            bool small = false;
+#pragma unroll
+            for (int t = 0; t < DT; t++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    if (kExactD || 32 * t + 8 * (i >> 2) + 4 * hh + (i & 3) < D) small |= __builtin_fabsf(acc_o[t][i]) < least;
+            return small && q_row < Nq;
+        };
 
         // A score tile (register i: key 8 (i/4) + 4 hh + i%4, query `col`): scaled and masked, then turned into weights.
         // weights() returns the factor the sums so far have to be multiplied by.
@@ -240,8 +251,17 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             store_tile(lds + BUF, v_lds + BUF);
         }
         // Seen already: no step of the loop below, straight to the second pass, whose first tile may overwrite what a late
-        // wave still reads here for scores that nobody uses then.
-        const bool uncarried = __syncthreads_or(!carried());
+        // wave still reads here for scores that nobody uses then.  (Small values of V alone: only where the tile split last has no
+        // others.)
+        bool uncarried = __syncthreads_or(!carried());
+        if (uncarried) {
+            float v_most = 0.0f;
+#pragma unroll
+            for (int n = 0; n < NI; n++)
+#pragma unroll
+                for (int i = 0; i < 8; i++) v_most = split_max(v_most, vreg[n][i >> 2][i & 3]);
+            uncarried = __syncthreads_or(!(chk < kSplitMost)) || !__syncthreads_or(v_most >= kSplitLeastResult);
+        }
         f32x16_t s_next;
         zero16(s_next);
         read_plane(lds, 2);
@@ -335,7 +355,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             __syncthreads();
         }
 
-        if (uncarried || __syncthreads_or(!carried())) {
+        if (uncarried || (__syncthreads_or(!carried()) && __syncthreads_or(!(chk < kSplitMost) || small_result()))) {
             // something here the split does not carry: the rows once more in f32, the tiles through LDS two at a time.  For a
             // launch (B=4 H=16 N=1024 D=64) 158 us where the first tiles show it, 240 where only the last does; straight from
             // memory 770; the f32 kernel alone 181.
@@ -709,7 +729,18 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing on its way into LDS that is used otherwise from here on
 
-    if (__syncthreads_or(!(chk < kSplitMost && v_least >= kSplitLeast))) {
+    bool uncarried = !(chk < kSplitMost);
+    if (__any(v_least < kSplitLeast)) {  // small values of V: where a result of this wave's keys is no larger than what they may have lost
+        const float least = (l_run + other_half(l_run)) * kSplitLeastResult;
+        bool small = false;
+#pragma unroll
+        for (int t = 0; t < DT; t++)
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if (kExactD || 32 * t + 8 * (i >> 2) + 4 * hh + (i & 3) < D) small |= __builtin_fabsf(acc_o[t][i]) < least;
+        uncarried |= small && q_row < Nq && m_run != neg_inf();  // (a row that sees none of them loses nothing)
+    }
+    if (__syncthreads_or(uncarried)) {
         // something here the split does not carry: the rows once more in f32, out of the same tiles
 #pragma unroll
         for (int t = 0; t < DT; t++) zero16(acc_o[t]);

@@ -2,8 +2,9 @@
 //
 // x = h + m + l with h = bf16(x), m = bf16(x - h), l = bf16(x - h - m), each rounded to nearest: the differences are
 // exact, and 3 x 8 bits of significand hold all 24 of x (below 2^-109 the last term meets the smallest bf16: an
-// absolute error of 2^-134; a workgroup that reads values so small goes by split_too_small or kSplitLeast).  A product x * y is then the six terms hh, hm, mh, hl, mm, lh; what is left out, ml + lm + ll,
-// is below 2^-26 |x y|, less than half of an f32 rounding.  Every term is exact in the f32 accumulator of
+// absolute error of 2^-134; a workgroup that reads values so small goes by split_too_small or kSplitLeast).  A product
+// x * y is then the six terms hh, hm, mh, hl, mm, lh; what is left out, ml + lm + ll, is below 2^-26 |x y|, less than
+// half of an f32 rounding.  Every term is exact in the f32 accumulator of
 // v_mfma_f32_32x32x16_bf16, whose rate is 16 times that of v_mfma_f32_32x32x2_f32: six of them are 2.7 times the f32 rate.
 //
 // NaN survives the split as three NaN, and whatever f32 arithmetic makes NaN of it comes out NaN here.  Infinities do not
@@ -119,8 +120,15 @@ __device__ __forceinline__ f32x16_t mfma_h(bf16x8_t a, bf16x8_t b, f32x16_t acc)
 constexpr float kSplitMost = 0x1p30f;  // the magnitude from which on the split products are not used
 // The same for values so small that the last term of the split would count (largest of a group of eight; zeros are fine).
 __device__ __forceinline__ bool split_too_small(float group_max) { return group_max < 0x1p-80f && group_max > 0.0f; }
-// ... and for single values: 2 (bits of |x|) - 1 of 2^-100, from which on the last term of x is no subnormal.
+// ... and for single values of V: 2 (bits of |x|) - 1 of 2^-100, from which on the last term of x is no subnormal.  Where one
+// is smaller the results decide: a value, and each of its products, loses 2^-126 at most, so that a result (before it is
+// divided by the row sum) of 2^-80 of that sum is off by less than 2^-26 of itself at 2^16 keys.  A subnormal in V leaves
+// every row on the split products whose results are not small themselves; turned away by the value alone it cost each
+// workgroup that read it the f32 pass.  us, one in every head, before -> now, clean: causal B=1 H=8 N=2048 D=64 83.7 -> 44.2,
+// 44.7; B=4 H=16 N=1024 D=64 239.9 -> 101.3, 101.0; causal D=128 272 -> 125, 126.  In a column of zeros, whose results it is,
+// it costs the f32 pass behind the other (154 -> 240).
 constexpr uint32_t kSplitLeast = ((uint32_t)(127 - 100) << 24) - 1u;
+constexpr float kSplitLeastResult = 0x1p-80f;
 // The larger magnitude; a NaN is not seen.
 __device__ __forceinline__ float split_max(float m, float x) { return __builtin_fmaxf(m, __builtin_fabsf(x)); }
 

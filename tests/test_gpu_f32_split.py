@@ -165,6 +165,40 @@ def test_small_values():
     assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("b,h,n,d", [(8, 16, 256, 64), (8, 32, 353, 32), (8, 16, 256, 128), (8, 16, 225, 60), (1, 2, 300, 64), (1, 8, 257, 20)])
+def test_a_small_value_of_v_among_others(b, h, n, d, causal):
+    """A subnormal in V leaves the split products to every row whose results are not small themselves: the other columns have
+    the bits they have with a zero in its place.  Under the causal mask row 0 is V's first, and its workgroup goes the f32 way."""
+    q, k, v = inputs(b, h, n, d)
+    rows = 128 if ra.debug_f32_split_products(ra.AttentionShape.new(b, h, n, d), ra.Mask.causal() if causal else ra.Mask.none()) else 32
+    col = d // 3
+    others = np.arange(d) != col
+    for key, value in ((0, 2.0 ** -110 * (1 + 2.0 ** -23)), (n // 2, 1e-40), (n - 1, 1e-40)):
+        usual = v[0, 1, key, col]
+        v[0, 1, key, col] = value
+        got, want = run(q, k, v, causal), attention64(q, k, v, causal)
+        v[0, 1, key, col] = 0.0
+        zero = run(q, k, v, causal)
+        v[0, 1, key, col] = usual
+        first = rows if causal and key == 0 else 0
+        assert np.array_equal(got[0, 1, first:, others], zero[0, 1, first:, others])
+        assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+        if first:
+            assert got[0, 1, 0, col] == np.float32(value)
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_small_columns_of_v(d):
+    """One column small throughout beside others of the usual size: its results keep their precision."""
+    q, k, v = inputs(8, 16, 256, d)
+    v[2, 7, :, 5] *= np.float32(2.0 ** -115)
+    for causal in (False, True):
+        got, want = run(q, k, v, causal)[2, 7].astype(np.float64), attention64(q, k, v, causal)[2, 7]
+        assert np.linalg.norm((got - want)[:, 5]) <= 1e-6 * np.linalg.norm(want[:, 5])
+        assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
 def run_backward(q, k, v, d_out):
     b, h, n, d = q.shape
     shape = ra.AttentionShape.new(b, h, n, d)
