@@ -1946,17 +1946,19 @@ hipError_t launch_halves(hipStream_t stream, const FlashTileParams& p, dim3 grid
 // Up to 1.9 causal workgroups a CU: the long tiles are dispatched first, so that a long walk in halves and a short one behind
 // it take a CU no longer than the longest walk whole, with its neighbour beside it -- from as many query tiles on as pay for
 // two meetings a CU, and above head dim 64 from more where the heads do not divide by the eight XCDs and one gets more of the
-// long tiles, or where nearly every CU takes two.  us, whole / halves, causal B H N: head dim 128 1 32 1501 34.5 / 29.5,
-// 1 16 2500 51.3 / 42.5, 2 8 3000 62.1 / 50.5, 1 12 4096 72.0 / 63.1, 5 8 1400 34.4 / 33.1, 1 10 6000 128 / 106, but 1 28 1600
-// 31.0 / 32.8, 1 28 2048 42.2 / 43.7, 1 40 1409 34.6 / 34.9, 4 12 1024 23.8 / 27.1, 1 32 2048 (two a CU) 44.3 / 44.8; 64
-// 1 32 1501 24.8 / 20.0, 1 28 1600 21.0 / 19.6, but 4 12 1024 15.9 / 16.7; 32 4 16 640 8.9 / 8.6, 5 8 1400 19.9 / 16.6.  Without
-// a mask every walk is as long and halves are slower: 128 1 16 2500 64.6 / 77.0.
+// long tiles, where the heads of one tile number take more than an eighth of the CUs and the second round starts among tiles
+// half as long as the longest, or where nearly every CU takes two.  us, whole / halves, causal, inputs that change from pass
+// to pass, B H N: head dim 128 1 24 1300 29.2 / 27.0, 1 32 1523 36.8 / 33.3, 1 32 1684 40.2 / 39.5, 1 24 2150 48.6 / 42.2,
+// 1 26 2246 53.4 / 51.9, 2 8 3612 76.8 / 65.7, but 5 8 1300 32.5 / 35.2, 5 8 1400 35.7 / 36.2, 4 12 1276 33.9 / 37.8, 1 28 2048
+// 42.2 / 43.7, 1 28 2224 51.6 / 52.4; 96 1 32 1523 31.1 / 27.6, but 2 20 1283 27.2 / 28.2; 80 1 26 2246 44.8 / 40.1; 64 1 24 1466
+// 24.1 / 19.8, 1 40 1461 25.8 / 25.0, 1 44 1350 25.5 / 25.0, but 4 16 854 17.7 / 18.5; 32 1 80 582 10.8 / 9.9, 1 96 582 10.95 /
+// 10.90.  Without a mask every walk is as long and halves are slower: 128 1 16 2500 64.6 / 77.0.
 static bool takes_halves(const FlashTileParams& p, dim3 grid) {
     if (p.pack != 1 || p.decode_rows || p.window != 0 || p.mask == kMaskPadding || p.seq_kv < (p.dim <= 64 ? kHalvesFrom64 : kHalvesFrom)) return false;
     const unsigned long long units = (unsigned long long)grid.x * grid.y, n = units * grid.z, n_cus = (unsigned long long)p.n_cus;
     if (n <= n_cus) return true;
     if (p.mask != kMaskCausal || 10 * n > 19 * n_cus) return false;
-    if (p.dim > 64) return grid.z >= 18 || (grid.z >= 11 && units % 8 == 0 && 4 * n <= 7 * n_cus);
+    if (p.dim > 64) return grid.z >= 18 || (grid.z >= 11 && units % 8 == 0 && 8 * units <= n_cus && 4 * n <= 7 * n_cus);
     return grid.z >= (p.dim <= 32 ? 5 : 11);
 }
 template <int DP>

@@ -564,3 +564,15 @@ def test_two_halves_of_the_keys_in_two_rounds(oracle, h, n, d):
         want = oracle.flash_forward_masked(oracle.AttentionShape(1, 1, n, d), q, k, v, "causal")
         assert_bf16_parity(got[i].ravel(), want, d, n, f"head {i}")
     assert np.isfinite(got).all()
+
+
+@pytest.mark.parametrize("h,n,d,halves", [(40, 1300, 128, False), (40, 1400, 96, False), (32, 1300, 128, True), (24, 1400, 80, True),
+                                          (40, 1400, 64, True), (64, 800, 64, False)])
+def test_which_causal_launches_walk_in_halves(force_kernel, h, n, d, halves):
+    """The fold of two halves is another order of additions: a launch walks whole where its bits are those of one of twice as
+    many heads, which has two workgroups a CU and more."""
+    force_kernel("tile")
+    q, k, v = (bf16_round(seeded_normal(h * n * d, s))[0] for s in (1, 2, 3))
+    one = flash_bf16(ra.AttentionShape.new(1, h, n, d), q, k, v, ra.Mask.causal())
+    two = flash_bf16(ra.AttentionShape.new(2, h, n, d), *(np.tile(x, 2) for x in (q, k, v)), ra.Mask.causal())
+    assert np.array_equal(one, two[: one.size]) != halves
