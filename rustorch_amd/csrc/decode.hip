@@ -191,7 +191,6 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(AttnRowsParams p) {
 // Lane l holds column h = l % 16 and the 8 keys 16*rt + 4*(l/16) + i of the step, which as they
 // stand are the 8 contraction slots of its B operand for the second product; the V operand is
 // fetched with the same slot -> key map.
-constexpr uint32_t kBufferFlags = 0x00020000u;  // dword 3 of a raw buffer descriptor: 32-bit data format, no swizzle
 constexpr int kDecRows = 32;     // key rows per step
 constexpr int kDecSpanMin = 8;   // a wave takes at least this many steps (bounds the partials per segment); batches
 constexpr int kDecSpanMinOne = 2;  // the same for a single sequence, where the latency of one call is what counts

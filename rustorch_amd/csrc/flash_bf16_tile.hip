@@ -30,7 +30,6 @@ namespace rt {
 
 namespace {
 
-constexpr uint32_t kBufferFlags = 0x00020000u;  // dword 3 of a raw buffer descriptor: 32-bit data format, no swizzle
 constexpr int TROWS = 128;  // query rows per workgroup: four waves' worth, each wave 32
 constexpr float kTileTrigSum = 65536.0f;  // a lane's 16-key share of a row sum above this sends the wave to the slow path
 
@@ -92,46 +91,6 @@ struct TileCfg {
     static constexpr int OCC_DIRECT = DP <= 64 ? 3 : 2;
     static constexpr int BIAS_BYTES = 32 * 32 * 4;  // a wave's bias values of an item: 32 rows of 32 keys
 };
-
-// 16 bytes per lane from a buffer straight into LDS: lane l lands at LDS byte address lds_block + 16 l (lds_block is
-// wave-uniform and goes through M0); a lane whose offset lies past the end of the descriptor lands zeros.  Issued as
-// inline assembly so that the compiler's counter bookkeeping does not make every later LDS read wait for it:
-// completion is awaited explicitly (s_waitcnt vmcnt(0) before the barrier that publishes the tile).  Loads the
-// compiler does not know of can only make its own vmcnt waits longer, never shorter: the counter retires in order.
-// (The statement counts as a writer of memory, which keeps the compiler from moving LDS reads across it.)
-__device__ __forceinline__ void t_buffer_to_lds(const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
-    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
-    const uint32_t so = __builtin_amdgcn_readfirstlane(tile_off);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :
-                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so)
-                 : "memory");
-}
-// the same for the lanes of `on` alone (what the others would have brought stays as it is in LDS); no branch around it
-__device__ __forceinline__ void t_buffer_to_lds_of(uint64_t on, const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
-    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
-    const uint32_t so = __builtin_amdgcn_readfirstlane(tile_off);
-    uint64_t all;
-    asm volatile("s_mov_b32 m0, %1\n\ts_and_saveexec_b64 %0, %5\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\ts_mov_b64 exec, %0"
-                 : "=&s"(all)
-                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so), "s"(on)
-                 : "memory", "scc");
-}
-// the same, 4 bytes per lane: lane l lands at lds_block + 4 l
-__device__ __forceinline__ void t_buffer_to_lds_b32(const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
-    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
-    const uint32_t so = __builtin_amdgcn_readfirstlane(tile_off);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-                 :
-                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so)
-                 : "memory");
-}
-// a raw buffer descriptor as four scalars: base, no stride, `bytes` addressable
-__device__ __forceinline__ u32x4_t t_make_rsrc(const void* base, uint32_t bytes) {
-    const uint64_t a = (uint64_t)(uintptr_t)base;
-    return u32x4_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
-                   (uint32_t)__builtin_amdgcn_readfirstlane(bytes), kBufferFlags};
-}
 
 // Where a workgroup works that takes the `pos`-th of the query tiles of `batch` <= 64 sequences, ordered by tile number downwards
 // (tile L of every sequence that has one, by sequence), then those of padded rows only, by tile number.  Lane i holds
@@ -373,8 +332,8 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             const uint32_t block = lds_base + half_at + stage_off + (uint32_t)((wave + 4 * n) * 1024);
             const uint32_t lane_at = DP == 96 ? lane_off[n] : lane_off[0];
             const uint32_t off = DP == 96 ? tile_off : tile_off + (uint32_t)(256 / SPR * n) * kv_pitch * 2u;
-            if constexpr (WHOLE) t_buffer_to_lds(rs, lane_at, off, block);
-            else t_buffer_to_lds_of(on[DP == 96 ? n : 0], rs, lane_at, off, block);
+            if constexpr (WHOLE) buffer_to_lds(rs, lane_at, off, block);
+            else buffer_to_lds_of(on[DP == 96 ? n : 0], rs, lane_at, off, block);
         }
     };
     // Tile 0 (K and V) and K of tile 1 are requested before the sequence lengths have arrived (a dependent load
@@ -385,7 +344,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     if (!SPLIT && !WIN && !HALVES) {
         const uint32_t all_bytes = p.seq_kv > 0 ? ((uint32_t)(p.seq_kv - 1) * kv_pitch + (uint32_t)D) * 2u : 0u;
         if constexpr (DIRECT) {
-            const u32x4_t Kall = t_make_rsrc(Kg, all_bytes), Vall = t_make_rsrc(Vg, all_bytes);
+            const u32x4_t Kall = make_rsrc(Kg, all_bytes), Vall = make_rsrc(Vg, all_bytes);
             dl_tile(Kall, dl_k, dl_k_on, 0u, 0u);
             dl_tile(Vall, dl_v, dl_v_on, 0u, 2u * STAGE_B);
             dl_tile(Kall, dl_k, dl_k_on, tile_bytes_g, STAGE_B);
@@ -507,7 +466,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     const uint32_t slab_bytes = n_keys > 0 ? ((uint32_t)(n_keys - 1) * kv_pitch + (uint32_t)D) * 2u : 0u;
     const __amdgpu_buffer_rsrc_t Kbuf = __builtin_amdgcn_make_buffer_rsrc((void*)Kg, 0, slab_bytes, kBufferFlags);
     const __amdgpu_buffer_rsrc_t Vbuf = __builtin_amdgcn_make_buffer_rsrc((void*)Vg, 0, slab_bytes, kBufferFlags);
-    const u32x4_t Kd = t_make_rsrc(Kg, slab_bytes), Vd = t_make_rsrc(Vg, slab_bytes);  // (DIRECT: the same descriptors as scalars)
+    const u32x4_t Kd = make_rsrc(Kg, slab_bytes), Vd = make_rsrc(Vg, slab_bytes);  // (DIRECT: the same descriptors as scalars)
     if (DIRECT && (SPLIT || WIN || HALVES)) {
         dl_tile(Kd, dl_k, dl_k_on, 0u, 0u);
         dl_tile(Vd, dl_v, dl_v_on, 0u, 2u * STAGE_B);
@@ -631,7 +590,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             const int r_first = q0 + 32 * wq, n_rows = max(min(32, rows_total - r_first), 0);
             const float* const bb = p.bias + ((size_t)b * p.heads + h0) * (size_t)p.bias_bh_stride + (size_t)min(r_first, rows_total - 1) * (size_t)p.seq_kv;
             const uint32_t pitch = (uint32_t)p.seq_kv * 4u, first = 4u * (uint32_t)min(half_key0, p.seq_kv);
-            bias_rsrc = t_make_rsrc((const char*)bb + first, n_rows > 0 ? (uint32_t)n_rows * pitch - first : 0u);
+            bias_rsrc = make_rsrc((const char*)bb + first, n_rows > 0 ? (uint32_t)n_rows * pitch - first : 0u);
             if (bias_vec4) {  // instruction n: rows 8 n + lane / 8
                 const int row = lane >> 3, slot = (lane & 7) ^ (row >> 1);
                 bias_lane[0] = (uint32_t)row * pitch + 16u * (uint32_t)slot;
@@ -649,11 +608,11 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             if (bias_vec4) {
 #pragma unroll
                 for (int n = 0; n < 4; n++)
-                    t_buffer_to_lds(bias_rsrc, bias_lane[n & 1], k_off + (uint32_t)n * bias_step, lds_base + bias_lds + 1024u * (uint32_t)n);
+                    buffer_to_lds(bias_rsrc, bias_lane[n & 1], k_off + (uint32_t)n * bias_step, lds_base + bias_lds + 1024u * (uint32_t)n);
             } else {
 #pragma unroll
                 for (int n = 0; n < 16; n++)
-                    t_buffer_to_lds_b32(bias_rsrc, bias_lane[0] + (bias_lane[1] ^ (16u * (uint32_t)(n & 7))), k_off + (uint32_t)n * bias_step,
+                    buffer_to_lds_b32(bias_rsrc, bias_lane[0] + (bias_lane[1] ^ (16u * (uint32_t)(n & 7))), k_off + (uint32_t)n * bias_step,
                                         lds_base + bias_lds + 256u * (uint32_t)n);
             }
         };
@@ -1950,9 +1909,10 @@ hipError_t launch_halves(hipStream_t stream, const FlashTileParams& p, dim3 grid
 // half as long as the longest, or where nearly every CU takes two.  us, whole / halves, causal, inputs that change from pass
 // to pass, B H N: head dim 128 1 24 1300 29.2 / 27.0, 1 32 1523 36.8 / 33.3, 1 32 1684 40.2 / 39.5, 1 24 2150 48.6 / 42.2,
 // 1 26 2246 53.4 / 51.9, 2 8 3612 76.8 / 65.7, but 5 8 1300 32.5 / 35.2, 5 8 1400 35.7 / 36.2, 4 12 1276 33.9 / 37.8, 1 28 2048
-// 42.2 / 43.7, 1 28 2224 51.6 / 52.4; 96 1 32 1523 31.1 / 27.6, but 2 20 1283 27.2 / 28.2; 80 1 26 2246 44.8 / 40.1; 64 1 24 1466
-// 24.1 / 19.8, 1 40 1461 25.8 / 25.0, 1 44 1350 25.5 / 25.0, but 4 16 854 17.7 / 18.5; 32 1 80 582 10.8 / 9.9, 1 96 582 10.95 /
-// 10.90.  Without a mask every walk is as long and halves are slower: 128 1 16 2500 64.6 / 77.0.
+// 42.2 / 43.7, 1 28 2224 51.6 / 52.4; 96 1 32 1523 31.1 / 27.6, but 2 20 1283 27.2 / 28.2; 80 1 26 2246 44.8 / 40.1 (and 5 8 1400
+// 30.1 / 28.5, left out with its like); 64 1 24 1466 24.1 / 19.8, 1 40 1461 25.8 / 25.0, 1 44 1350 25.5 / 25.0, but 4 16 854 17.7 /
+// 18.5; 32 1 80 582 10.8 / 9.9, 1 96 582 10.95 / 10.90.  Without a mask every walk is as long and halves are slower: 128
+// 1 16 2500 64.6 / 77.0.
 static bool takes_halves(const FlashTileParams& p, dim3 grid) {
     if (p.pack != 1 || p.decode_rows || p.window != 0 || p.mask == kMaskPadding || p.seq_kv < (p.dim <= 64 ? kHalvesFrom64 : kHalvesFrom)) return false;
     const unsigned long long units = (unsigned long long)grid.x * grid.y, n = units * grid.z, n_cus = (unsigned long long)p.n_cus;

@@ -430,17 +430,6 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
     }
 }
 
-// 16 bytes per lane from a buffer straight into LDS, lane l at lds_block + 16 l (wave-uniform); past the end of the
-// descriptor zeros.  The lanes outside `on` bring nothing.  Awaited by hand (vmcnt): the compiler does not know of it.
-__device__ __forceinline__ void tile_to_lds(uint64_t on, const u32x4_t& rsrc, uint32_t lane_off, uint32_t off, uint32_t lds_block) {
-    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block), so = __builtin_amdgcn_readfirstlane(off);
-    uint64_t all;
-    asm volatile("s_mov_b32 m0, %1\n\ts_and_saveexec_b64 %0, %5\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\ts_mov_b64 exec, %0"
-                 : "=&s"(all)
-                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so), "s"(on)
-                 : "memory", "scc");
-}
-
 // The same products for launches with few rows: a workgroup owns 32 query rows and its four waves share the keys, wave w
 // tiles w, w + 4, ..; each walks alone, without a barrier, and the four (O, m, l) are folded through LDS at the end, as in
 // flash_fwd_f32_splitk_kernel.  A wave's tile of K and its tile of V lie in LDS of its own as they are in memory (16-byte
@@ -507,19 +496,15 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
         on[n] = kExactD ? ~0ull : __ballot(4 * slot < D);
         if (!kExactD && 4 * slot >= D) *(u32x4_t*)(Kw + 16 * c) = *(u32x4_t*)(Vw + 16 * c) = u32x4_t{0u, 0u, 0u, 0u};
     }
-    auto rsrc_of = [&](const float* base) RT_INLINE {
-        const uint64_t a = (uint64_t)(uintptr_t)base;
-        return u32x4_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
-                       (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(N - 1) * pitch_b + 4u * (uint32_t)D), 0x00020000u};
-    };
-    const u32x4_t k_rsrc = rsrc_of(Kg), v_rsrc = rsrc_of(Vg);
+    const uint32_t kv_bytes = (uint32_t)(N - 1) * pitch_b + 4u * (uint32_t)D;
+    const u32x4_t k_rsrc = make_rsrc(Kg, kv_bytes), v_rsrc = make_rsrc(Vg, kv_bytes);
     // (rows behind the last are zeros: their scores are masked, and their weights are zeros.  Tiles behind the last, whose
     // offset lies past the descriptor's end, bring zeros too, without a read, but are requested all the same, so that a wait
     // can count.)
     auto request = [&](const u32x4_t& rs, uint32_t at, int tile) RT_INLINE {
         const uint32_t off = (uint32_t)tile * (uint32_t)kTile * pitch_b;
 #pragma unroll
-        for (int n = 0; n < NREQ; n++) tile_to_lds(on[n], rs, lane_off[n], off, at + 1024u * (uint32_t)n);
+        for (int n = 0; n < NREQ; n++) buffer_to_lds_of(on[n], rs, lane_off[n], off, at + 1024u * (uint32_t)n);
     };
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     request(k_rsrc, k_lds, wave);

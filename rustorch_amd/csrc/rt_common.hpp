@@ -32,6 +32,48 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 __device__ __forceinline__ float bf16_lo(uint32_t packed) { return __uint_as_float(packed << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t packed) { return __uint_as_float(packed & 0xffff0000u); }
 
+constexpr uint32_t kBufferFlags = 0x00020000u;  // dword 3 of a raw buffer descriptor: 32-bit data format, no swizzle
+
+// 16 bytes per lane from a buffer straight into LDS: lane l lands at LDS byte address lds_block + 16 l (lds_block is
+// wave-uniform and goes through M0); a lane whose offset lies past the end of the descriptor lands zeros.  Issued as
+// inline assembly so that the compiler's counter bookkeeping does not make every later LDS read wait for it:
+// completion is awaited explicitly (s_waitcnt vmcnt before the barrier that publishes the tile).  Loads the
+// compiler does not know of can only make its own vmcnt waits longer, never shorter: the counter retires in order.
+// (The statement counts as a writer of memory, which keeps the compiler from moving LDS reads across it.)
+__device__ __forceinline__ void buffer_to_lds(const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
+    const uint32_t so = __builtin_amdgcn_readfirstlane(tile_off);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so)
+                 : "memory");
+}
+// the same for the lanes of `on` alone (what the others would have brought stays as it is in LDS); no branch around it
+__device__ __forceinline__ void buffer_to_lds_of(uint64_t on, const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
+    const uint32_t so = __builtin_amdgcn_readfirstlane(tile_off);
+    uint64_t all;
+    asm volatile("s_mov_b32 m0, %1\n\ts_and_saveexec_b64 %0, %5\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\ts_mov_b64 exec, %0"
+                 : "=&s"(all)
+                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so), "s"(on)
+                 : "memory", "scc");
+}
+// the same, 4 bytes per lane: lane l lands at lds_block + 4 l
+__device__ __forceinline__ void buffer_to_lds_b32(const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
+    const uint32_t so = __builtin_amdgcn_readfirstlane(tile_off);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+                 :
+                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so)
+                 : "memory");
+}
+// a raw buffer descriptor as four scalars: base, no stride, `bytes` addressable
+__device__ __forceinline__ u32x4_t make_rsrc(const void* base, uint32_t bytes) {
+    const uint64_t a = (uint64_t)(uintptr_t)base;
+    return u32x4_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
+                   (uint32_t)__builtin_amdgcn_readfirstlane(bytes), kBufferFlags};
+}
+
 // Value held by the lane 32 positions away (the other half of the wave).
 __device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32, 64); }
 
