@@ -54,7 +54,7 @@ def assert_decode_parity(got, want, dim, label=""):
 
 def assert_within_rounding(got, want, sizes, label=""):
     """Element by element: a bf16 output is off by its own rounding and by that of the weights, 2^-8 of the value and of
-    `sizes`, the same attention over |V|; 2^-13 of both for the f32 scores (a sum of d products of up to 2^10 in f32, on
+    `sizes`, the same attention over |V|; 2^-13 of both for the f32 scores (a sum of d products of up to 2^11 in f32, on
     either side) and exponentials.  A row that has lost its maximum or a key is off by its own size."""
     got, want, sizes = (np.asarray(x, dtype=np.float64).ravel() for x in (got, want, sizes))
     assert same_nan_pattern(got, want), f"{label}: NaN pattern differs"

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import rustorch_amd as ra
-from _gpu import dev
+from _gpu import dev, with_common_offset
 from _util import seeded_normal
 
 pytestmark = pytest.mark.gpu
@@ -402,6 +402,23 @@ def test_few_rows_keys_of_another_length(t_q, t_kv, d):
     ra.synchronize()
     got, want = bnhd(out.download(np.float32).reshape(b, t_q, h, d)), attention64(q, k, v, False)
     assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("b,h,n,d", [(1, 2, 300, 64), (1, 4, 500, 20), (8, 16, 256, 64), (8, 32, 353, 32), (8, 16, 256, 128)])
+@pytest.mark.parametrize("q_times,offset", [(2.5, 0.0), (8.0, 0.0), (1.0, 130.0), (3.5, 130.0)])
+def test_scores_of_any_size(b, h, n, d, causal, q_times, offset):
+    """Waves whose keys' maxima lie far apart, and scores that all lie near -130.  A scaled score is off by about eight
+    roundings at the size of its products' magnitudes together, a weight by that share of itself, and a result by twice
+    that (numerator and row sum) of the attention over |V|; 2^-20 for everything else."""
+    q, k, v = inputs(b, h, n, d)
+    q *= np.float32(q_times)
+    if offset:
+        q, k = with_common_offset(q, k, d, offset)
+    got, want = run(q, k, v, causal), attention64(q, k, v, causal)
+    sizes = attention64(q, k, np.abs(v), causal)
+    scores = (np.abs(q).astype(np.float64) @ np.swapaxes(np.abs(k), -1, -2).astype(np.float64)).max(axis=-1, keepdims=True) / np.sqrt(d)
+    assert (np.abs(got - want) <= (2 * 8 * 2.0 ** -24 * scores + 2.0 ** -20) * sizes).all()
 
 
 @pytest.mark.parametrize("causal", [False, True])

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import rustorch_amd as ra
-from _gpu import assert_bf16_parity, bf16_round, dev, flash_bf16, max_abs
+from _gpu import assert_bf16_parity, assert_within_rounding, bf16_round, dev, flash_bf16, max_abs, with_common_offset
 from _util import seeded_normal
 
 pytestmark = pytest.mark.gpu
@@ -521,6 +521,35 @@ def test_two_halves_of_the_keys(oracle, n, d):
     ra.synchronize()
     want = oracle.mha_forward_masked(f[0][: tq * h * d], f[1], f[2], 1, tq, n, h, d, bias)
     assert_bf16_parity(oracle.bf16_to_f32(out.download(np.uint16)), want, d, None, f"n={n} d={d} bias")
+
+
+@pytest.mark.parametrize("d", [24, 64, 80, 128])
+@pytest.mark.parametrize("q_times,offset", [(2.5, 0.0), (8.0, 0.0), (1.0, 130.0), (3.5, 130.0)])
+def test_two_halves_with_scores_of_any_size(oracle, d, q_times, offset):
+    """Halves whose maxima lie far apart, rows that no key of one half counts for, and scores that all lie near -130; under a
+    causal mask the rows of a second half that see none of it, with a bias the rows one half of which is hidden."""
+    h, n, tq = 2, 833, 70
+    q, k, v = (seeded_normal((h, n, d), i) for i in (1, 2, 3))
+    q *= np.float32(q_times)
+    if offset:
+        q, k = with_common_offset(q, k, d, offset)
+    bits, f = zip(*(bf16_round(x.ravel()) for x in (q, k, v)))
+    shape, oshape = ra.AttentionShape.new(1, h, n, d), oracle.AttentionShape(1, h, n, d)
+    for name, mask in (("none", ra.Mask.none()), ("causal", ra.Mask.causal())):
+        want, sizes = (oracle.flash_forward_masked(oshape, f[0], f[1], x, name) for x in (f[2], np.abs(f[2])))
+        assert_within_rounding(flash_bf16(shape, *bits, mask), want, sizes, name)
+    bias = np.random.default_rng(n).standard_normal((tq, n)).astype(np.float32)
+    bias[3, : n // 2 + 64] = -1.0e4
+    bias[4, n // 2 - 64:] = -1.0e4
+    bias[5, ::2] += 60.0
+    bnhd = [x.reshape(h, n, d).transpose(1, 0, 2) for x in bits], [x.reshape(h, n, d).transpose(1, 0, 2) for x in f]
+    (qb, kb, vb), (qf, kf, vf) = ([x[0][:tq].ravel(), x[1].ravel(), x[2].ravel()] for x in bnhd)
+    out = ra.HipStorage(tq * h * d * 2)
+    dq, dk, dv, db = dev(qb), dev(kb), dev(vb), dev(bias)
+    ra.mha_forward_masked_bf16_dev(dq, dk, dv, out, 1, tq, n, h, d, db, bias.size)
+    ra.synchronize()
+    want, sizes = (oracle.mha_forward_masked(qf, kf, x, 1, tq, n, h, d, bias) for x in (vf, np.abs(vf)))
+    assert_within_rounding(oracle.bf16_to_f32(out.download(np.uint16)), want, sizes, "bias")
 
 
 @pytest.mark.parametrize("d", [64, 128, 200])
