@@ -198,7 +198,12 @@ int rt_flash_forward_f32_dev(void *stream, const rt_attention_shape *shape, uint
  * evenly over them, a 4-wave tile kernel for everything else, and a form of the tile kernel with 64 query rows per wave
  * for dim 64, which runs only when it is asked for;
  * rt_debug_force_bf16_prefill_kernel forces one of them where it applies.  The remaining dims and alignments run on
- * a one-workgroup-per-row kernel with the same masks and row rules (correct at any speed, not tuned). */
+ * a one-workgroup-per-row kernel with the same masks and row rules (correct at any speed, not tuned).
+ * The last bits of a sequence's rows may depend on what else is in the launch: which kernel serves it, and, where the tile
+ * kernel has few workgroups a compute unit, whether it walks the keys in two halves that are folded at the end (another
+ * order of the same additions), follow from the number of heads, sequences and rows together.  That holds for the
+ * [batch, seq, heads, dim], the padded and the masked bf16 entries below as well, and for f32 prefill, whose kernels are
+ * chosen by the same numbers.  The same call on the same device gives the same bits every time. */
 int rt_flash_forward_bf16_dev(void *stream, const rt_attention_shape *shape, uint64_t n_kv_heads, const void *q,
                               const void *k, const void *v, int mask_kind, const uint8_t *keep, void *out,
                               rt_err_detail *err);

@@ -9,8 +9,9 @@
 // list, this one is built for many short jobs: a workgroup of four waves owns 128 query rows (32 per wave) of one
 // (batch, head) and is gone when they are done; several workgroups share a CU, so one workgroup's set-up, softmax
 // and output overlap with another's matrix work without any hand-written interleaving, and the hardware
-// dispatcher balances jobs of unequal length.  Keys are walked KT at a time through a double-buffered LDS tile
-// (global -> registers -> LDS, one workgroup barrier per tile); per 32-key item a wave computes
+// dispatcher balances jobs of unequal length.  Keys are walked KT at a time through a double-buffered LDS tile (straight
+// from memory, or through registers above head dim 128 and under a key-padding vector; one workgroup barrier per tile);
+// per 32-key item a wave computes
 //
 //   S^T[kv, q]  = K[kv, :] . Q[q, :]      v_mfma_f32_32x32x16_bf16, A = K tile (LDS), B = Q (registers)
 //   online softmax on S^T (a lane holds 16 scores of query row lane % 32; row max / sum are in-lane plus one
@@ -19,8 +20,8 @@
 //
 // with P fed to the second product straight from the score registers (the accumulator layout of the first
 // product is a B operand of the second under a fixed permutation of the contraction slots, which the V operand
-// read applies as well).  LDS rows are padded so that the 16-byte K reads and the transposing V reads are free
-// of bank conflicts.
+// read applies as well).  LDS rows are padded, or their 16-byte slots XORed with bits of the row, so that the 16-byte K
+// reads and the transposing V reads are free of bank conflicts.
 #include "rt_common.hpp"
 #include "rt_kernels.hpp"
 
@@ -199,9 +200,10 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     constexpr int PF = Cfg::PF;        // register sets of tiles in flight behind the two LDS stages
     static_assert(2 * DT == KS, "one P.V matrix instruction per score matrix instruction");
     // Head dims above 128 do not have the registers for two score tiles and their operands in flight (O alone is 128
-    // registers), nor does head dim 128 with a bias (two items' bias values) or with a key-padding mask: there an
-    // item runs its three phases one after the other, and K is parked with V.
-    constexpr bool PIPE = DP <= 128 && !(((BIAS && !DIRECT) || MODE == kMaskPadding) && DP == 128);
+    // registers), nor does head dim 128 with a key-padding mask: there an item runs its three phases one after the other,
+    // and K is parked with V.
+    constexpr bool PIPE = DP <= 128 && !(MODE == kMaskPadding && DP == 128);
+    static_assert(!BIAS || DIRECT || DP > 128, "a bias up to head dim 128 comes with tiles straight to LDS");
     static_assert(PIPE || !HALVES, "the halves meet once a tile");
 
     constexpr int kTilesLds = DIRECT ? Cfg::LDS_BYTES_DIRECT : Cfg::LDS_BYTES;  // BIAS: the four waves' bias values behind the tiles
@@ -579,9 +581,10 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         // (8 rows a load instruction, or 2 where the rows are not 16-byte aligned), and from there into the order the scores
         // sit in; the 16-byte slots of a row are XORed with bits of the row, as those of a K tile of 128-byte rows.  Read
         // from its row in memory by each lane, 16 bytes of 32 rows at a time, the bias kept the address unit busy for half
-        // of the launch and the waves waiting for 54 % of theirs: B=4 H=16 T=1024 hd=64 47.4 -> 28.3 us, 1023 keys (4-byte
-        // requests) 93.9 -> 34.9, one matrix a head at B=4 H=16 T=770 hd=96 119 -> 58.3.  Keys behind the last one read the next row, or zeros
-        // behind the tensor: those scores are masked.
+        // of the launch and the waves waiting for 54 % of theirs: B=4 H=16 T=1024 hd=64 47.4 -> 28.3 us with warm inputs and
+        // 47.3 -> 29.9 with inputs that change from pass to pass; warm, 1023 keys (4-byte requests) 93.9 -> 34.9, one matrix a
+        // head at B=4 H=16 T=770 hd=96 119 -> 58.3.  Keys behind the last one read the next row, or zeros behind the tensor:
+        // those scores are masked.
         u32x4_t bias_rsrc = {0u, 0u, 0u, 0u};
         uint32_t bias_lane[2] = {0u, 0u}, bias_at = 0, bias_step = 0;
         const uint32_t bias_lds = BIAS ? (uint32_t)(kBiasAt + (wave + 4 * half) * Cfg::BIAS_BYTES) : 0u;
@@ -1978,10 +1981,13 @@ hipError_t launch_flash_wide_bf16(hipStream_t stream, const FlashTileParams& par
 }
 
 // A padded batch's query tiles in one order over all sequences (at most 64: a lane each): where they do not fit the chip at
-// once, and the walks are long enough to pay for the wait for the lengths ahead of the first request for keys, about 1 us.
-// us, by sequence / by length: B H N shortest head dim 16 16 1024 128 64 29.8 / 27.7, at 128 52.3 / 48.6, 32 8 2000 300 64 82 / 76,
-// 8 32 4096 1000 128 608 / 575; with fewer than eight tiles 64 8 500 64 96 34.7 / 34.6, 12 16 700 100 32 11.9 / 12.6, 22 16 300 60
-// 80 16.3 / 18.6.
+// once, and the walks are long enough to pay for the wait for the lengths ahead of the first request for keys, 1 to 1.5 us.
+// us, by sequence / by length, inputs that change from pass to pass, lengths spread evenly up to N and standing in any order
+// in the batch, B H N shortest head dim: 16 16 1024 128 64 31.1 / 29.9, at 128 59.5 / 59.2, 32 8 2000 300 64 89.9 / 84.5, 8 32
+// 4096 1000 128 683 / 626, 20 8 3000 1000 128 240 / 223, 2 16 4000 800 64 61.6 / 54.1, 24 12 1236 176 32 32.1 / 30.2.  What the
+// order gains depends on where the long sequences stand; where they had fallen well the wait is what is left: 6 8 2246 1123
+// 64 38.9 / 40.6, 3 16 3107 443 64 50.6 / 52.6, 3 32 1702 425 256 136 / 139, 30 12 1800 900 64 136 / 138.  With fewer than eight
+// tiles 64 8 500 64 96 34.7 / 34.6, 12 16 700 100 32 11.9 / 12.6, 22 16 300 60 80 16.3 / 18.6.
 static bool tiles_by_length(const FlashTileParams& p, long long n_qtiles) {
     return p.q_lens && p.kv_lens == p.q_lens && p.seq_q == p.seq_kv && p.mask == kMaskCausal && p.pack == 1 && !p.decode_rows && p.window == 0 &&
            p.batch > 1 && p.batch <= 64 && n_qtiles >= 8 &&
