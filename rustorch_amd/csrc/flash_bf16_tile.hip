@@ -94,42 +94,51 @@ struct TileCfg {
 };
 
 // Where a workgroup works that takes the `pos`-th of the query tiles of `batch` <= 64 sequences, ordered by tile number downwards
-// (tile L of every sequence that has one, by sequence), then those of padded rows only, by tile number.  Lane i holds
-// sequence i; a binary search over the tile number, a sum over the lanes a step.
+// (tile L of every sequence that has one, by sequence), then those of padded rows only, by tile number upwards.  Lane i holds
+// sequence i: a ballot per tile number gives the sequences that have it, four numbers without a branch between.  It stands
+// ahead of the first request for keys, so what bounds it is its own latency: a binary search over the number, a sum over the
+// lanes a step, took 0.3 to 1 us more of a launch (below).
 struct TilePlace {
     int b, qtile, len;
 };
-__device__ __forceinline__ int t_lane_sum(int x) {
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1, 2, 4, 8
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return __builtin_amdgcn_readlane(x, 63);
-}
 __device__ __forceinline__ TilePlace t_place_by_length(const int32_t* lens, int batch, int seq, int pos, int lane) {
     const int len = lane < batch ? min(max(lens[lane], 0), seq) : 0;
-    const int n = (len + TROWS - 1) / TROWS, n_all = (seq + TROWS - 1) / TROWS;  // tiles with valid rows, and all of them
-    const int valid = t_lane_sum(n);
-    const bool padded = pos >= valid;
-    // tiles in front of those numbered L: of higher number, or (padded rows only) of lower
-    auto ahead = [&](int L) __attribute__((always_inline)) { return t_lane_sum(padded ? (lane < batch ? max(L - n, 0) : 0) : max(n - 1 - L, 0)); };
-    const int at = padded ? pos - valid : pos;
-    int lo = 0, hi = n_all - 1;
-    while (lo < hi) {  // padded: the highest L with ahead(L) <= at; else the lowest
-        const int mid = padded ? (lo + hi + 1) >> 1 : (lo + hi) >> 1;
-        const bool in = ahead(mid) <= at;
-        if (padded) {
-            if (in) lo = mid; else hi = mid - 1;
-        } else {
-            if (in) hi = mid; else lo = mid + 1;
+    const int n_all = (seq + TROWS - 1) / TROWS;
+    const uint32_t n = (uint32_t)(len + TROWS - 1) / TROWS;                    // its tiles with valid rows,
+    const uint32_t m = lane < batch ? (uint32_t)n_all - n : 0u;                // and the others: the last m of n_all
+    int at = pos, k = 0;  // k: tiles passed by, of n_all with valid rows (from the highest down) and n_all without
+    uint64_t has = 0;
+    auto find = [&](auto with) __attribute__((always_inline)) {  // with(k): the sequences that have the k-th; true when the place is among them
+        for (k = 0; k < n_all; k += 4) {
+            int c[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) c[j] = __builtin_popcountll(with(k + j));
+            const int all = c[0] + c[1] + c[2] + c[3];
+            if (at < all) {
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    if (at < c[j]) break;
+                    at -= c[j];
+                    k++;
+                }
+                has = with(k);
+                return true;
+            }
+            at -= all;
         }
+        return false;
+    };
+    int tile;
+    if (find([&](int i) __attribute__((always_inline)) { return __ballot((uint32_t)(n_all - 1 - i) < n); })) {  // (below tile 0: none)
+        tile = n_all - 1 - k;
+    } else {
+        find([&](int i) __attribute__((always_inline)) { return __ballot((uint32_t)(n_all - 1 - i) < m); });
+        tile = k;
     }
-    uint64_t has = __ballot(padded ? (lane < batch && n <= lo) : n > lo);  // the sequences with a tile of that number
-    for (int k = at - ahead(lo); k > 0; k--) has &= has - 1;
-    const int b = has ? __builtin_ctzll(has) : 0;
-    return TilePlace{b, lo, __builtin_amdgcn_readlane(len, b)};
+    const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0u));
+    const uint64_t one = has & __ballot(below == at);
+    const int b = one ? __builtin_ctzll(one) : 0;
+    return TilePlace{b, tile, __builtin_amdgcn_readlane(len, b)};
 }
 
 // How K/V tiles come into LDS: through registers, or straight there with rows of DP columns or with rows of fewer.
@@ -1981,13 +1990,15 @@ hipError_t launch_flash_wide_bf16(hipStream_t stream, const FlashTileParams& par
 }
 
 // A padded batch's query tiles in one order over all sequences (at most 64: a lane each): where they do not fit the chip at
-// once, and the walks are long enough to pay for the wait for the lengths ahead of the first request for keys, 1 to 1.5 us.
-// us, by sequence / by length, inputs that change from pass to pass, lengths spread evenly up to N and standing in any order
-// in the batch, B H N shortest head dim: 16 16 1024 128 64 31.1 / 29.9, at 128 59.5 / 59.2, 32 8 2000 300 64 89.9 / 84.5, 8 32
-// 4096 1000 128 683 / 626, 20 8 3000 1000 128 240 / 223, 2 16 4000 800 64 61.6 / 54.1, 24 12 1236 176 32 32.1 / 30.2.  What the
-// order gains depends on where the long sequences stand; where they had fallen well the wait is what is left: 6 8 2246 1123
-// 64 38.9 / 40.6, 3 16 3107 443 64 50.6 / 52.6, 3 32 1702 425 256 136 / 139, 30 12 1800 900 64 136 / 138.  With fewer than eight
-// tiles 64 8 500 64 96 34.7 / 34.6, 12 16 700 100 32 11.9 / 12.6, 22 16 300 60 80 16.3 / 18.6.
+// once, and the walks are long enough to pay for the wait for the lengths ahead of the first request for keys.  us, by
+// sequence / by length (with the binary search), inputs that change from pass to pass, lengths spread evenly up to N and
+// standing in any order in the batch, B H N shortest head dim: 16 16 1024 170 64 34.5 / 32.8 (33.5), 32 8 2000 333 64 90.2 / 85.0
+// (86.3), 20 8 3000 500 128 210 / 193 (193), 4 16 4000 666 128 142.3 / 128.4 (127.2), 22 40 949 158 64 103.5 / 93.9 (97.0), 2 16
+// 4000 666 64 61.0 / 53.4 (53.8), 12 16 2048 1024 64 90.6 / 89.2 (91.2).  What the order gains depends on where the long
+// sequences stand and how far the lengths lie apart; what is left otherwise is the wait: 3 16 3107 517 64 51.4 / 53.0 (53.4),
+// 14 8 1174 195 64 23.9 / 24.5 (25.1), 3 32 1702 283 256 124.2 / 130.6 (130.7), and lengths all equal 16 16 1024 64 55.1 / 55.9
+// (56.6), 22 40 949 64 184 / 188 (191), 14 8 1174 64 34.4 / 36.1 (37.3).  With fewer than eight tiles (with the search) 64 8 500
+// 64 96 34.7 / 34.6, 12 16 700 100 32 11.9 / 12.6, 22 16 300 60 80 16.3 / 18.6.
 static bool tiles_by_length(const FlashTileParams& p, long long n_qtiles) {
     return p.q_lens && p.kv_lens == p.q_lens && p.seq_q == p.seq_kv && p.mask == kMaskCausal && p.pack == 1 && !p.decode_rows && p.window == 0 &&
            p.batch > 1 && p.batch <= 64 && n_qtiles >= 8 &&

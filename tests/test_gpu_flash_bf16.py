@@ -583,6 +583,30 @@ def test_padded_batch_ordered_by_length(oracle, lens, d):
             assert max_abs(got[i, :, 0], f[2][i, :, 0]) <= TOL
 
 
+@pytest.mark.parametrize("n,h,lens", [(1153, 32, [1153, 1, 1024, 1025, 640, 0, 129]), (1281, 8, [1281] * 11), (2100, 16, [700, 2100, 2049, 128]),
+                                      (9000, 4, [9000, 130, 8900])])
+def test_padded_batch_ordered_by_length_of_more_tiles(oracle, n, h, lens):
+    """Ten to 71 tiles a sequence, counts that are and are not multiples of four: the first and last row of every tile of every
+    sequence, in the first and last head, through the reference's single-row attention."""
+    b, d = len(lens), 64
+    rng = np.random.default_rng(n)
+    bits, f = zip(*(bf16_round(rng.standard_normal((b, h, n, d), dtype=np.float32)) for _ in range(3)))
+    q, k, v = (x.reshape(b, h, n, d) for x in f)
+    dq, dk, dv, dl = (dev(x) for x in (*bits, np.asarray(lens, dtype=np.int32)))
+    out = ra.HipStorage(b * h * n * d * 2)
+    out.upload(np.full(b * h * n * d, 0x7B7B, dtype=np.uint16))
+    ra.flash_forward_varlen_bf16_dev(ra.AttentionShape.new(b, h, n, d), dq, dk, dv, dl, out, zero_padded_rows=True)
+    ra.synchronize()
+    got = oracle.bf16_to_f32(out.download(np.uint16)).reshape(b, h, n, d)
+    for i, ln in enumerate(lens):
+        assert not got[i, :, ln:].any()
+        for row in sorted({r for t in range(0, ln, 128) for r in (t, min(t + 127, ln - 1))}):
+            for head in (0, h - 1):
+                want, sizes = (oracle.gqa_forward_f32(q[i, head, row], k[i, head, : row + 1], x[i, head, : row + 1], 1, 1, 1, 1, row + 1, d)
+                               for x in (v, np.abs(v)))
+                assert_within_rounding(got[i, head, row], want, sizes, f"sequence {i} head {head} row {row}")
+
+
 @pytest.mark.parametrize("h,n,d", [(55, 520, 32), (100, 513, 24), (24, 1282, 64), (24, 1408, 80), (32, 1345, 128), (16, 2200, 128)])
 def test_two_halves_of_the_keys_in_two_rounds(oracle, h, n, d):
     """Causal launches of one to 1.9 workgroups a CU: the second round of workgroups starts where the first ends."""
