@@ -691,7 +691,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void flash_fwd_bf16_kernel(FlashBf16Pa
             for (int n = 0; n < 32 / RPI; n++) {
                 u32x4_t v = *(const u32x4_t __attribute__((address_space(3)))*)(uintptr_t)(rd + (uint32_t)(n * RPI * ROWB));
                 if (qw_out + n * RPI + r0 < N)
-                    *(u32x4_t*)(gp + (size_t)n * RPI * o_pitch_b + (slot_off ^ (uint32_t)(swz_o(n * RPI) * 16))) = v;
+                    store_past(gp + (size_t)n * RPI * o_pitch_b + (slot_off ^ (uint32_t)(swz_o(n * RPI) * 16)), v);
             }
         }
     }

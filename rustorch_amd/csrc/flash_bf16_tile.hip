@@ -463,7 +463,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         if (HALVES && half) return;
         for (int c = tid; c < TROWS * CH; c += TTHREADS) {
             const int row = c / CH, ch = c - row * CH;
-            if (q0 + row < rows_total && 8 * ch < D) *(u32x4_t*)(ob + (size_t)(q0 + row) * p.lo.row_pitch + 8 * ch) = val;
+            if (q0 + row < rows_total && 8 * ch < D) store_past(ob + (size_t)(q0 + row) * p.lo.row_pitch + 8 * ch, val);
         }
         // (the early requests land in this workgroup's LDS: not to be left in flight when it is handed on)
         if constexpr (DIRECT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1285,7 +1285,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             const uint32_t f2 = rr < n_q ? 0x7fc07fc0u : fill2;
             u32x4_t val = {f2, f2, f2, f2};
             if (n_loop > 0) val = *(const u32x4_t*)(src + RS * n * LDK);
-            if (rr < rows_total && col_ok) *(u32x4_t*)dst = val;
+            if (rr < rows_total && col_ok) store_past(dst, val);
             dst += step;
         }
     } else {
@@ -1304,7 +1304,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             if (rr < rows_total && 8 * ch < D) {
                 uint16_t* dst = p.out + (size_t)b * p.lo.batch_stride + (size_t)(h0 + gg) * p.lo.head_stride +
                                 (size_t)sp * p.lo.row_pitch + 8 * ch;
-                *(u32x4_t*)dst = val;
+                store_past(dst, val);
             }
         }
     }
