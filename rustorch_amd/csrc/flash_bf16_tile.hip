@@ -1214,17 +1214,24 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         // The partial of this span: O as accumulated (relative to the running max as it stands), that max in the exp2
         // domain, the row sum.  A workgroup without tiles, or a row that saw no key of the span, leaves (0, -inf, 0).
         // Stored as it stands in the registers, 32 rows to a block: eight columns of the 32 rows are 1 KB in one piece
-        // (row by row, 16 bytes here and there, the stores took 1-2 us of a short span).
+        // (row by row, 16 bytes here and there, the stores took 1-2 us of a short span).  Above head dim 64 they go out at device
+        // scope, so that the end of the launch has no megabytes in the L2s to write back: us, 32 / 8 heads of 128, 64 positions
+        // over 8192 keys 22.1 -> 21.3, 16 15.3 -> 15.05; 28 / 4 heads, 200 over 3000 26.6 -> 23.5.  (Past the caches: 23.3 there,
+        // 17.1 for 16.5 with 3 positions of 5 sequences over 1109 keys of 256.)  At head dim 64 the partials are few enough for
+        // the write-back to be the shorter way: 16 heads, 2 positions over 900 keys 10.1, 10.4 at device scope.
+        constexpr int kPartScope = DP > 64 ? 16 : 0;  // sc1
         const int r = q0 + 32 * wq + col;
         if (r < rows_total) {
             const size_t block = (((size_t)b * p.kv_heads + kvh) * (size_t)((rows_total + 31) / 32) + (size_t)(q0 / 32 + wq)) * (size_t)p.n_splits + (size_t)split;
-            float* const po = p.part_o + block * (size_t)(32 * D) + 4 * lane;
+            const __amdgpu_buffer_rsrc_t po = __builtin_amdgcn_make_buffer_rsrc(p.part_o + block * (size_t)(32 * D), 0, 128u * (uint32_t)D, kBufferFlags);
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
                 for (int j = 0; j < 4; j++)
                     if (32 * dt + 8 * j < D)
-                        *(f32x4_t*)(po + 256 * (4 * dt + j)) = f32x4_t{acc_o[dt][4 * j], acc_o[dt][4 * j + 1], acc_o[dt][4 * j + 2], acc_o[dt][4 * j + 3]};
+                        __builtin_amdgcn_raw_buffer_store_b128(
+                            __builtin_bit_cast(u32x4_t, f32x4_t{acc_o[dt][4 * j], acc_o[dt][4 * j + 1], acc_o[dt][4 * j + 2], acc_o[dt][4 * j + 3]}), po,
+                            16u * (uint32_t)lane, 1024u * (uint32_t)(4 * dt + j), kPartScope);
             p.part_ml[64 * block + lane] = hh == 0 ? m_run * cc : l;
         }
         return;
