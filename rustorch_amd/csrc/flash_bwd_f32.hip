@@ -4,11 +4,12 @@
 // The reference rebuilds the full seq x seq matrices P, dP and dS per (batch, head).  Here nothing of that
 // size exists: the forward kernel is run once more to leave O and the row statistic L_i = m_i + ln(l_i), and
 //
-//   delta_i = sum_j P_ij dP_ij = dO_i . O_i                                   (prologue of flash_bwd_f32_dq_kernel)
+//   delta_i = sum_j P_ij dP_ij = dO_i . O_i                                   (prologue of flash_bwd_f32_dq_kernel; in one
+//                                                                              launch with it the dK/dV side forms its own)
 //   P_ij    = exp(scale * Q_i.K_j - L_i),   dP_ij = dO_i . V_j,   dS_ij = P_ij (dP_ij - delta_i)
 //   dQ_i = scale * sum_j dS_ij K_j                                            (flash_bwd_f32_dq_kernel)
-//   dV_j = sum_i P_ij dO_i,   dK_j = scale * sum_i dS_ij Q_i                  (flash_bwd_f32_dkdv_kernel, launched second:
-//                                                                              it reads the delta the dQ kernel left)
+//   dV_j = sum_i P_ij dO_i,   dK_j = scale * sum_i dS_ij Q_i                  (flash_bwd_f32_dkdv_kernel; launched second it
+//                                                                              reads the delta the dQ kernel left)
 //
 // are recomputed 32 x 32 tile by tile on the f32 matrix cores (v_mfma_f32_32x32x2_f32).  Each output row is owned
 // by exactly one workgroup, so there are no atomics and the result does not depend on scheduling.
@@ -23,6 +24,8 @@
 //                  dV^T[d, kv] += dO^T.P,  dK^T[d, kv] += Q^T.dS   (A = the same LDS tiles read along d)
 //   dQ kernel:     S^T[kv, q] = K.Q^T and dP^T[kv, q] = V.dO^T     (A = K / V tile from LDS, B = Q / dO registers)
 //                  dQ^T[d, q] += K^T.dS^T                          (A = the K tile read along d)
+#include <type_traits>
+
 #include "rt_common.hpp"
 #include "rt_kernels.hpp"
 
@@ -133,35 +136,36 @@ __device__ __forceinline__ void spill_transposed(float* tile, const f32x16_t* ac
         }
 }
 
-// Which (batch*head, owner tile) a workgroup takes.  Workgroups are dealt round-robin to the 8 XCDs, each with its own
-// L2: when the (batch, head) pairs divide evenly, XCD x takes the pairs bh = x (mod 8) one after the other, so that a
-// pair's four input tensors are fetched into one L2 only.
-__device__ __forceinline__ void owner_of_block(int& bh, int& tile) {
-    const int nt = (int)gridDim.x, n_bh = (int)(gridDim.y * gridDim.z);
-    bh = (int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z;
-    tile = (int)blockIdx.x;
-    if ((n_bh & 7) == 0) {
-        const int lin = (int)blockIdx.x + nt * bh;
-        const int xcd = lin & 7, r = lin >> 3;
-        bh = (r / nt) * 8 + xcd;
-        tile = r % nt;
-    }
+// Which (batch*head, owner tile) the workgroup at position `lin` of `nt` tiles times `n_bh` pairs takes.  Workgroups are dealt
+// round-robin to the 8 XCDs, each with its own L2: when the (batch, head) pairs divide evenly, XCD x takes the pairs bh = x
+// (mod 8) one after the other, so that a pair's four input tensors are fetched into one L2 only.
+__device__ __forceinline__ void owner_of_block(int lin, int nt, int n_bh, int& bh, int& tile) {
+    const bool by_xcd = (n_bh & 7) == 0;
+    const int r = by_xcd ? lin >> 3 : lin;
+    bh = r / nt;
+    tile = r % nt;
+    if (by_xcd) bh = 8 * bh + (lin & 7);
 }
 
-template <int DT>  // DT = ceil(dim / 32); the head dim is zero-padded to DPAD = 32 * DT in LDS
-__global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dkdv_kernel(FlashBwdF32Params p) {
+template <int DT>
+struct BwdTiles {  // LDS of a workgroup: two tiles a wave
+    static constexpr int LD = 32 * DT + 4;  // 16-byte reads of 16 rows tile all banks
+    static constexpr int TILE = kRows * LD;
+    static constexpr int FLOATS = kNW * 2 * TILE;
+};
+
+// kOwnDelta: delta is formed here, of the tile's rows of dO and O (16-byte loads), and not read.
+template <int DT, bool kOwnDelta>  // DT = ceil(dim / 32); the head dim is zero-padded to DPAD = 32 * DT in LDS
+__device__ __forceinline__ void bwd_f32_dkdv(const FlashBwdF32Params& p, int lin, int nt, float* lds, float (*stat)[2][kRows]) {
     constexpr int DPAD = 32 * DT;
-    constexpr int LD = DPAD + 4;  // 16-byte reads of 16 rows tile all banks
-    constexpr int TILE = kRows * LD;
-    __shared__ __attribute__((aligned(16))) float lds[kNW * 2 * TILE];
-    __shared__ float stat[kNW][2][kRows];
+    constexpr int LD = BwdTiles<DT>::LD, TILE = BwdTiles<DT>::TILE;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, hh = lane >> 5;
     const int N = p.seq, D = p.dim;
-    const bool vec = p.vec != 0;
+    const bool vec = kOwnDelta || p.vec != 0;
     int bh_i, tile_i;
-    owner_of_block(bh_i, tile_i);
+    owner_of_block(lin, nt, p.batch * p.heads, bh_i, tile_i);
     const int kv0 = tile_i * kRows;
     const size_t bh = (size_t)bh_i;
     const size_t base = bh * (size_t)N * D;
@@ -171,6 +175,7 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dkdv_ker
     const float* __restrict__ dOg = p.d_out + base;
     const float* __restrict__ lse = p.lse + bh * (size_t)N;
     const float* __restrict__ delta = p.delta + bh * (size_t)N;
+    const float* __restrict__ Og = p.o + base;
     float* Qt = lds + wave * 2 * TILE;  // this wave's Q tile
     float* Ot = Qt + TILE;              // this wave's dO tile
 
@@ -207,7 +212,7 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dkdv_ker
     auto load_stats = [&](int q0n) {
         const bool ok = q0n + col < N;
         nl = ok ? lse[q0n + col] : -neg_inf();
-        nd = ok ? delta[q0n + col] : 0.0f;
+        if constexpr (!kOwnDelta) nd = ok ? delta[q0n + col] : 0.0f;
     };
     if (wave < n_qt) {
         if (vec) {
@@ -226,6 +231,19 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dkdv_ker
         } else {
             stage_tile<DPAD, LD>(Qt, Qg, q0, N, D, lane, false);
             stage_tile<DPAD, LD>(Ot, dOg, q0, N, D, lane, false);
+        }
+        if constexpr (kOwnDelta) {  // as the dQ kernel forms it
+            nd = 0.0f;
+            if (q0 + col < N) {
+                const float* const o_row = Og + (size_t)(q0 + col) * D;
+#pragma unroll 2  // (all at once: 29 registers spilled at head dim 64, 124 at 128)
+                for (int d = 4 * hh; d < D; d += 8) {
+                    const f32x4_t a = *(const f32x4_t*)(o_row + d), c = *(const f32x4_t*)(Ot + col * LD + d);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) nd = __builtin_fmaf(a[i], c[i], nd);
+                }
+            }
+            nd += other_half(nd);
         }
         if (hh == 0) {
             stat[wave][0][col] = nl;
@@ -281,18 +299,16 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dkdv_ker
 }
 
 template <int DT>
-__global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dq_kernel(FlashBwdF32Params p) {
+__device__ __forceinline__ void bwd_f32_dq(const FlashBwdF32Params& p, int lin, int nt, float* lds) {
     constexpr int DPAD = 32 * DT;
-    constexpr int LD = DPAD + 4;
-    constexpr int TILE = kRows * LD;
-    __shared__ __attribute__((aligned(16))) float lds[kNW * 2 * TILE];
+    constexpr int LD = BwdTiles<DT>::LD, TILE = BwdTiles<DT>::TILE;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, hh = lane >> 5;
     const int N = p.seq, D = p.dim;
     const bool vec = p.vec != 0;
     int bh_i, tile_i;
-    owner_of_block(bh_i, tile_i);
+    owner_of_block(lin, nt, p.batch * p.heads, bh_i, tile_i);
     const int q0 = tile_i * kRows;
     const size_t bh = (size_t)bh_i;
     const size_t base = bh * (size_t)N * D;
@@ -413,6 +429,29 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dq_kerne
     reduce_store<DPAD, LD, 2 * TILE>(lds, 0, p.dq + base, q0, N, D, tid, vec);
 }
 
+__device__ __forceinline__ int linear_block() { return (int)blockIdx.x + (int)gridDim.x * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z); }
+
+template <int DT>
+__global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dkdv_kernel(FlashBwdF32Params p) {
+    __shared__ __attribute__((aligned(16))) float lds[BwdTiles<DT>::FLOATS];
+    __shared__ float stat[kNW][2][kRows];
+    bwd_f32_dkdv<DT, false>(p, linear_block(), (int)gridDim.x, lds, stat);
+}
+template <int DT>
+__global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dq_kernel(FlashBwdF32Params p) {
+    __shared__ __attribute__((aligned(16))) float lds[BwdTiles<DT>::FLOATS];
+    bwd_f32_dq<DT>(p, linear_block(), (int)gridDim.x, lds);
+}
+// Both in one launch (bwd_f32_one_launch), dK/dV, the longer one, first: grid x holds the owner tiles of both.
+template <int DT>
+__global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_both_kernel(FlashBwdF32Params p) {
+    __shared__ __attribute__((aligned(16))) float lds[BwdTiles<DT>::FLOATS];
+    __shared__ float stat[kNW][2][kRows];
+    const int nt = (int)gridDim.x / 2, lin = linear_block(), n = nt * p.batch * p.heads;
+    if (lin < n) bwd_f32_dkdv<DT, true>(p, lin, nt, lds, stat);
+    else bwd_f32_dq<DT>(p, lin - n, nt, lds);
+}
+
 // ---- any head dim up to 512: one workgroup per row, any speed ------------------------------------------------------
 // The gradients of cpu_backward.rs:46-185 for the head dims the tiled kernels above do not hold in registers.  The dQ
 // kernel owns a query row i (and leaves delta_i = dO_i . O_i for the second kernel), the dK/dV kernel a key row j;
@@ -524,6 +563,15 @@ __global__ __launch_bounds__(256) void flash_bwd_rows_dkdv_kernel(FlashBwdF32Par
 
 }  // namespace
 
+// The gradients in one launch?  dQ and dK/dV have `blocks` workgroups each, of which a CU holds `per_cu`.  A launch that leaves
+// CUs idle takes as long as one of its workgroups, whatever the others do: where the workgroups of both are resident at once
+// they run side by side, and a small call pays for one launch instead of two.  For that dK/dV has to form delta itself, O
+// being one more tensor to read, 2 % of its time.  With more workgroups than places the two are level.  us of the gradients,
+// two launches -> one, B H N head dim: 1 8 18 64 15.0 -> 7.9, 1 8 126 64 19.2 -> 10.6, 2 8 512 64 43.7 -> 38.2, 1 4 2000 64
+// 153 -> 136, 1 8 300 32 20.7 -> 11.5, 1 8 500 128 78.9 -> 50.5, 1 4 700 96 89.8 -> 61.0; with 128 rows a workgroup 2 8 655 64
+// 92.5 -> 53.8, 1 8 2048 64 247 -> 163, 3 16 165 64 39.0 -> 22.4.
+bool bwd_f32_one_launch(long long blocks, int per_cu, int n_cus) { return 2 * blocks <= (long long)per_cu * (n_cus > 0 ? n_cus : 256); }
+
 size_t flash_bwd_f32_workspace_floats(int batch, int heads, int seq, int dim) {
     return (size_t)batch * heads * seq * ((size_t)dim + 2);
 }
@@ -587,24 +635,21 @@ hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Param
         if (flash_f32_takes_split(f, true)) return launch_flash_bwd_f32_split(stream, p);
     }
     dim3 grid((p.seq + kRows - 1) / kRows, p.heads, p.batch), block(256);
-    const int dt = (p.dim + 31) / 32;
-    switch (dt) {
-        case 1:
-            hipLaunchKernelGGL(flash_bwd_f32_dq_kernel<1>, grid, block, 0, stream, p);
-            hipLaunchKernelGGL(flash_bwd_f32_dkdv_kernel<1>, grid, block, 0, stream, p);
-            break;
-        case 2:
-            hipLaunchKernelGGL(flash_bwd_f32_dq_kernel<2>, grid, block, 0, stream, p);
-            hipLaunchKernelGGL(flash_bwd_f32_dkdv_kernel<2>, grid, block, 0, stream, p);
-            break;
-        case 3:
-            hipLaunchKernelGGL(flash_bwd_f32_dq_kernel<3>, grid, block, 0, stream, p);
-            hipLaunchKernelGGL(flash_bwd_f32_dkdv_kernel<3>, grid, block, 0, stream, p);
-            break;
-        case 4:
-            hipLaunchKernelGGL(flash_bwd_f32_dq_kernel<4>, grid, block, 0, stream, p);
-            hipLaunchKernelGGL(flash_bwd_f32_dkdv_kernel<4>, grid, block, 0, stream, p);
-            break;
+    const bool both = p.vec && aligned(p.o) && bwd_f32_one_launch((long long)grid.x * grid.y * grid.z, p.dim <= 64 ? 2 : 1, p.n_cus);
+    auto launch = [&](auto dt_c) {
+        constexpr int kDT = decltype(dt_c)::value;
+        if (both) {
+            hipLaunchKernelGGL(flash_bwd_f32_both_kernel<kDT>, dim3(2 * grid.x, grid.y, grid.z), block, 0, stream, p);
+            return;
+        }
+        hipLaunchKernelGGL(flash_bwd_f32_dq_kernel<kDT>, grid, block, 0, stream, p);
+        hipLaunchKernelGGL(flash_bwd_f32_dkdv_kernel<kDT>, grid, block, 0, stream, p);
+    };
+    switch ((p.dim + 31) / 32) {
+        case 1: launch(std::integral_constant<int, 1>{}); break;
+        case 2: launch(std::integral_constant<int, 2>{}); break;
+        case 3: launch(std::integral_constant<int, 3>{}); break;
+        case 4: launch(std::integral_constant<int, 4>{}); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

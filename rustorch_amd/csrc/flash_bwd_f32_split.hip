@@ -17,6 +17,8 @@
 // for the row statistic where it is requested 327, sums pinned 321, dQ in the same order 312, independent runs and single
 // writes 308.  B=2 N=2048 973, 689, 583; head dim 32 273, 214, 171.  (dQ with two waves a SIMD, 40 registers spilled: 318.)
 // Relative error against 64 bits 5.9e-7 -> 4.5e-7, 7.3e-7 -> 5.9e-7, 5.5e-7 -> 4.4e-7 (f32 kernels -> this).
+#include <type_traits>
+
 #include "rt_common.hpp"
 #include "rt_kernels.hpp"
 #include "rt_split.hpp"
@@ -138,32 +140,42 @@ __device__ __forceinline__ void store_rows(float* __restrict__ dst, const f32x16
 
 __device__ __forceinline__ bf16x8_t as_frag(u32x4_t x) { return __builtin_bit_cast(bf16x8_t, x); }
 
-// (batch, head) and 128-row block of a workgroup: pairs on one XCD each where they divide by eight
-__device__ __forceinline__ void owner_of_block(int& bh, int& blk) {
-    const int nt = (int)gridDim.x, n_bh = (int)(gridDim.y * gridDim.z);
-    bh = (int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z;
-    blk = (int)blockIdx.x;
-    if ((n_bh & 7) == 0) {
-        const int lin = (int)blockIdx.x + nt * bh, xcd = lin & 7, r = lin >> 3;
-        bh = (r / nt) * 8 + xcd;
-        blk = r % nt;
-    }
+// (batch, head) and 128-row block of the workgroup at position `lin` of `nt` blocks times `n_bh` pairs: pairs on one XCD each
+// where they divide by eight
+__device__ __forceinline__ void owner_of_block(int lin, int nt, int n_bh, int& bh, int& blk) {
+    const bool by_xcd = (n_bh & 7) == 0;
+    const int r = by_xcd ? lin >> 3 : lin;
+    bh = r / nt;
+    blk = r % nt;
+    if (by_xcd) bh = 8 * bh + (lin & 7);
+}
+__device__ __forceinline__ int linear_block() { return (int)blockIdx.x + (int)gridDim.x * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z); }
+
+// the sum of x over groups of 4 or 8 neighbouring lanes, in each of them
+template <int N>
+__device__ __forceinline__ float lanes_sum(float x) {
+    auto dpp = [](float y, auto ctrl) { return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(y), decltype(ctrl)::value, 0xf, 0xf, true)); };
+    x += dpp(x, std::integral_constant<int, 0xb1>{});  // quad_perm 1, 0, 3, 2
+    x += dpp(x, std::integral_constant<int, 0x4e>{});  // quad_perm 2, 3, 0, 1
+    if (N == 8) x += dpp(x, std::integral_constant<int, 0x141>{});  // row_half_mirror: the other quad
+    return x;
 }
 
-// One workgroup a CU at head dim 64, so a wave may have the whole register file.
 template <int DT>
-__global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split_kernel(FlashBwdF32Params p) {
+constexpr int kLdsHalfs = 4 * Stream<DT>::SIZE;  // two tiles of either streamed matrix
+
+// kOwnDelta: delta is formed here, a tile's with its rows of dO and O, and not read.
+template <int DT, bool kOwnDelta>
+__device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int lin, int nt, __bf16* lds, float (*stat)[2][kTile]) {
     constexpr int DPAD = 32 * DT, KS = DPAD / 16;
     using St = Stream<DT>;
     constexpr int BUF = 2 * St::SIZE;  // Q, then dO
-    __shared__ __attribute__((aligned(16))) __bf16 lds[2 * BUF];
-    __shared__ __attribute__((aligned(16))) float stat[2][2][kTile];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hh = lane >> 5;
     const int N = p.seq, D = p.dim;
     int bh, blk;
-    owner_of_block(bh, blk);
+    owner_of_block(lin, nt, p.batch * p.heads, bh, blk);
     const int key = blk * 4 * kTile + wave * kTile + col;
     const size_t base = (size_t)bh * N * D;
     const float* __restrict__ Qg = p.q + base;
@@ -172,6 +184,7 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
     const float* __restrict__ dOg = p.d_out + base;
     const float* __restrict__ lse = p.lse + (size_t)bh * N;
     const float* __restrict__ delta = p.delta + (size_t)bh * N;
+    const float* __restrict__ Og = p.o + base;
 
     float chk = 0.0f;
     Split8 kf[KS], vf[KS];
@@ -196,20 +209,39 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
         zero16(low_dk[t]);
     }
 
-    St q_in, o_in;
+    St q_in, o_in, out_in;  // out_in: O, for delta; read and multiplied, never split
     q_in.clear();
     o_in.clear();
+    out_in.clear();
     float st = 0.0f;  // threads 0..31: the row statistic, 32..63: delta.  Rows beyond seq: +inf, their weights are zeros
     const uint32_t piece = St::piece(D, tid);
     const float* const st_src = tid < 32 ? lse : delta;
     auto load = [&](int row0) RT_INLINE {
         q_in.load(Qg, row0, N, D, tid, piece);
         o_in.load(dOg, row0, N, D, tid, piece);
+        if constexpr (kOwnDelta) out_in.load(Og, row0, N, D, tid, piece);
         if (wave == 0) st = st_src[min(row0 + (tid & 31), N - 1)];
     };
     // (the loaded value is looked at here and not where it is requested: there the wave would wait for it)
     auto put_stat = [&](int b, int row0) RT_INLINE {
-        if (wave == 0) {
+        if constexpr (kOwnDelta) {
+            constexpr int LANES = DPAD / 8;  // of a row
+            float x = 0.0f, y = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                x = __builtin_fmaf(o_in.r[0][i], out_in.r[0][i], x);
+                y = __builtin_fmaf(o_in.r[1][i], out_in.r[1][i], y);
+            }
+            const int row = tid / LANES;
+            x = row0 + row < N ? lanes_sum<LANES>(x + y) : 0.0f;
+            chk = split_max(chk, x);
+            if (tid % LANES == 0 && (St::ITEMS % 256 == 0 || tid < St::ITEMS)) stat[b][1][row] = x;
+            if (tid < 32) {
+                const bool in = row0 + tid < N;
+                chk = split_max(chk, in ? st : 0.0f);
+                stat[b][0][tid] = in ? st : -neg_inf();
+            }
+        } else if (wave == 0) {
             const bool in = row0 + (tid & 31) < N;
             chk = split_max(chk, in ? st : 0.0f);
             stat[b][tid >> 5][tid & 31] = in ? st : (tid < 32 ? -neg_inf() : 0.0f);
@@ -360,7 +392,7 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
         // launch of both kernels (B=4 H=16 N=1024 D=64) 551 us where the first tiles show it, 684 where only the last does;
         // straight from memory 2880; the f32 kernels alone 506.
         using Tile = F32Tile<DT>;
-        static_assert(4 * Tile::SIZE * sizeof(float) <= sizeof(lds), "two tiles of Q and dO");
+        static_assert(4 * Tile::SIZE * sizeof(float) <= kLdsHalfs<DT> * sizeof(__bf16), "two tiles of Q and dO");
         float* const f32_lds = (float*)lds;
 #pragma unroll
         for (int t = 0; t < DT; t++) {
@@ -377,7 +409,17 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
             ot.load(dOg, (size_t)D, q0, N, D, tid);
             if (tid < 64) {
                 const int row = q0 + (tid & 31);
-                st_f = row < N ? (tid < 32 ? lse : delta)[row] : (tid < 32 ? -neg_inf() : 0.0f);
+                st_f = tid < 32 ? -neg_inf() : 0.0f;
+                if (row < N) {
+                    if (!kOwnDelta || tid < 32) {
+                        st_f = (tid < 32 ? lse : delta)[row];
+                    } else {
+                        f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+                        for (int d = 0; d < D; d += 4)
+                            sum += *(const f32x4_t*)(dOg + (size_t)row * D + d) * *(const f32x4_t*)(Og + (size_t)row * D + d);
+                        st_f = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+                    }
+                }
             }
         };
         auto store_f = [&](int b2) {
@@ -416,17 +458,16 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
 }
 
 template <int DT>
-__global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_kernel(FlashBwdF32Params p) {
+__device__ __forceinline__ void bwd_dq_split(const FlashBwdF32Params& p, int lin, int nt, __bf16* lds) {
     constexpr int DPAD = 32 * DT, KS = DPAD / 16;
     using St = Stream<DT>;
     constexpr int BUF = 2 * St::SIZE;  // K, then V
-    __shared__ __attribute__((aligned(16))) __bf16 lds[2 * BUF];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hh = lane >> 5;
     const int N = p.seq, D = p.dim;
     int bh, blk;
-    owner_of_block(bh, blk);
+    owner_of_block(lin, nt, p.batch * p.heads, bh, blk);
     const int q_row = blk * 4 * kTile + wave * kTile + col;
     const bool q_ok = q_row < N;
     const size_t base = (size_t)bh * N * D;
@@ -599,7 +640,7 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_k
     for (int t = 0; t < DT; t++) acc[t] += low[t];
     if (uncarried || __syncthreads_or(!(chk < kSplitMost))) {  // as in the kernel above
         using Tile = F32Tile<DT>;
-        static_assert(4 * Tile::SIZE * sizeof(float) <= sizeof(lds), "two tiles of K and V");
+        static_assert(4 * Tile::SIZE * sizeof(float) <= kLdsHalfs<DT> * sizeof(__bf16), "two tiles of K and V");
         float* const f32_lds = (float*)lds;
 #pragma unroll
         for (int t = 0; t < DT; t++) zero16(acc[t]);
@@ -637,19 +678,45 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_k
     store_rows<DT>(p.dq + base, acc, q_row, hh, N, D);
 }
 
+// One workgroup a CU at head dim 64, so a wave may have the whole register file.
+template <int DT>
+__global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split_kernel(FlashBwdF32Params p) {
+    __shared__ __attribute__((aligned(16))) __bf16 lds[kLdsHalfs<DT>];
+    __shared__ __attribute__((aligned(16))) float stat[2][2][kTile];
+    bwd_dkdv_split<DT, false>(p, linear_block(), (int)gridDim.x, lds, stat);
+}
+template <int DT>
+__global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_kernel(FlashBwdF32Params p) {
+    __shared__ __attribute__((aligned(16))) __bf16 lds[kLdsHalfs<DT>];
+    bwd_dq_split<DT>(p, linear_block(), (int)gridDim.x, lds);
+}
+// Both in one launch, dK/dV, the longer one, first: grid x holds the owner blocks of both.
+template <int DT>
+__global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_both_split_kernel(FlashBwdF32Params p) {
+    __shared__ __attribute__((aligned(16))) __bf16 lds[kLdsHalfs<DT>];
+    __shared__ __attribute__((aligned(16))) float stat[2][2][kTile];
+    const int nt = (int)gridDim.x / 2, lin = linear_block(), n = nt * p.batch * p.heads;
+    if (lin < n) bwd_dkdv_split<DT, true>(p, lin, nt, lds, stat);
+    else bwd_dq_split<DT>(p, lin - n, nt, lds);
+}
+
 }  // namespace
 
 hipError_t launch_flash_bwd_f32_split(hipStream_t stream, const FlashBwdF32Params& p) {
     dim3 grid((p.seq + 4 * kTile - 1) / (4 * kTile), p.heads, p.batch), block(256);
-    if (p.dim <= 32) {
-        hipLaunchKernelGGL(flash_bwd_f32_dq_split_kernel<1>, grid, block, 0, stream, p);
-        hipLaunchKernelGGL(flash_bwd_f32_dkdv_split_kernel<1>, grid, block, 0, stream, p);
-    } else if (p.dim <= 64) {
-        hipLaunchKernelGGL(flash_bwd_f32_dq_split_kernel<2>, grid, block, 0, stream, p);
-        hipLaunchKernelGGL(flash_bwd_f32_dkdv_split_kernel<2>, grid, block, 0, stream, p);
-    } else {
-        return hipErrorInvalidValue;
-    }
+    const bool both = bwd_f32_one_launch((long long)grid.x * grid.y * grid.z, p.dim <= 32 ? 2 : 1, p.n_cus);
+    auto launch = [&](auto dt_c) {
+        constexpr int kDT = decltype(dt_c)::value;
+        if (both) {
+            hipLaunchKernelGGL(flash_bwd_f32_both_split_kernel<kDT>, dim3(2 * grid.x, grid.y, grid.z), block, 0, stream, p);
+            return;
+        }
+        hipLaunchKernelGGL(flash_bwd_f32_dq_split_kernel<kDT>, grid, block, 0, stream, p);
+        hipLaunchKernelGGL(flash_bwd_f32_dkdv_split_kernel<kDT>, grid, block, 0, stream, p);
+    };
+    if (p.dim <= 32) launch(std::integral_constant<int, 1>{});
+    else if (p.dim <= 64) launch(std::integral_constant<int, 2>{});
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

@@ -503,10 +503,9 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
 // Without a mask up to head dim 64 the gradients follow the same rule, so that they form the scores in the order in which the
 // row statistic was formed, and the line lies where forward and gradients together break even.  Every workgroup has the
 // same to do there: rounds of 32-row workgroups (one a CU in the gradients at head dim 64, two at 32) with a quarter of the
-// tiles each, against rounds of 128-row ones at 0.5 (0.345) of a step.  us here / there, forward and gradients, B H N at head
-// dim 64: 8 8 256 60 / 63, 8 16 100 37 / 42, 4 8 256 38 / 62, 2 8 512 62 / 100, 1 8 1000 112 / 179; 2 8 1024 181 / 180, 1 8 2048
-// 341 / 336, 2 12 400 91 / 86, 3 16 165 60 / 50, 8 16 200 107 / 64, 1 12 1500 395 / 256; at 32: 4 12 300 46 / 55, 1 8 2048
-// 189 / 260, 4 16 1024 336 / 234.
+// tiles each, against rounds of 128-row ones at 0.5 (0.345) of a step.  us here / there, forward and gradients (in a launch each), B H N
+// at head dim 64: 4 12 283 72 / 70, 8 16 200 107 / 64, 1 12 1500 395 / 256; at 32: 4 12 300 46 / 55, 8 16 200 59 / 40, 4 16 1024 336 / 234;
+// with the gradients in one launch (flash_f32_gradients_join) 4 8 256 34 / 47, 4 8 128 18 / 28.
 static bool flash_f32_split_pays(const FlashF32Params& p) {
     const double n_cus = p.n_cus > 0 ? p.n_cus : 256;
     const long long keys = p.seq_kv ? p.seq_kv : p.seq;
@@ -561,9 +560,21 @@ static bool flash_f32_takes_split_keys(const FlashF32Params& p) {
     return keys >= (level ? kSplitKeysFrom32 : kSplitKeysFrom);
 }
 
+// Unmasked, head dims 33 to 64, for a forward whose row statistic the gradients read: the gradients' two kernels run side by
+// side in one launch (bwd_f32_one_launch) with 128 rows a workgroup, and with 32 would not.  us, forward + gradients, f32 / 128
+// rows, B H N at head dim 64: 8 8 256 18.0 + 43.0 / 17.7 + 29.8, 4 8 384 22.3 + 56.7 / 22.5 + 36.8, 2 8 640 32.2 + 86.3 / 32.6 + 51.7,
+// 8 16 100 11.3 + 26.6 / 11.9 + 18.9, 1 4 3000 127 + 368 / 129 + 209.  With 32 in one launch as well: 2 8 512 55 / 70, 1 8 1000
+// 99 / 125.  At head dim 32 the forward loses most of what the gradients gain (1 8 2048 50 + 138 / 75 + 109).
+static bool flash_f32_gradients_join(const FlashF32Params& p) {
+    const long long n_bh = (long long)p.heads * p.batch;
+    return p.mask == kMaskNone && p.dim > 32 && p.dim <= 64 && !bwd_f32_one_launch(n_bh * ((p.seq + 31) / 32), 2, p.n_cus) &&
+           bwd_f32_one_launch(n_bh * ((p.seq + 127) / 128), 1, p.n_cus);
+}
+
 // (above head dim 64 the gradients have no such form, and a row statistic they read is formed as they form the scores)
 bool flash_f32_takes_split(const FlashF32Params& p, bool with_lse) {
     if (p.dim % 4 != 0 || p.dim > (with_lse ? 64 : 128) || p.bias || p.mask == kMaskPadding) return false;
+    if (with_lse && flash_f32_gradients_join(p)) return true;
     return flash_f32_split_pays(p) && (with_lse || !flash_f32_takes_split_keys(p) || flash_f32_rows_pay(p));
 }
 

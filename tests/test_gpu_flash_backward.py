@@ -216,3 +216,58 @@ def test_saved_forward_form_checks_workspace():
     with pytest.raises(ra.DeviceError) as ei:
         ra.flash_backward_saved_f32_dev(shape, *([buf] * 9), buf, 63)
     assert ei.value.status == L.RT_ERR_WORKSPACE_TOO_SMALL
+
+
+# ---- dQ and dK/dV in one launch -------------------------------------------------------------------------------
+
+
+@pytest.mark.parametrize("bhnd", [
+    (8, 32, 20, 64), (8, 32, 33, 64),    # 32 rows a workgroup: all resident at once, and one tile a head more than that
+    (4, 8, 250, 40), (1, 8, 250, 100), (2, 20, 97, 96),  # the last tile short, padded head dims; one launch, one, two
+    (5, 13, 40, 32),                     # head pairs not a multiple of eight
+    (8, 16, 128, 64), (2, 16, 321, 64), (5, 13, 130, 60), (8, 16, 200, 32),  # 128 rows a workgroup: one row or a few in the last
+    (8, 16, 129, 64),                    # as many blocks as the CUs hold of one kernel: two launches
+])
+def test_gradients_in_one_launch(oracle, bhnd):
+    b, h, n, d = bhnd
+    shape = ra.AttentionShape.new(*bhnd)
+    bufs = [seeded_normal(shape.buffer_len(), s) for s in (71, 72, 73, 74)]
+    got = ra.flash_backward(shape, *bufs)
+    again = ra.flash_backward(shape, *bufs)
+    want = oracle.flash_backward(oracle.AttentionShape(*bhnd), *bufs)
+    for name, g, a, w in zip(("dq", "dk", "dv"), got, again, want):
+        assert np.array_equal(g, a), name
+        # as test_backward_matches_oracle_on_normal_inputs
+        assert max_abs(g, w) <= 1e-5 * max(1.0, float(np.abs(w).max())) * 4, name
+
+
+@pytest.mark.parametrize("what", ["key inf", "d_out nan", "d_out inf", "d_out small"])
+@pytest.mark.parametrize("bhnd", [(2, 16, 320, 64), (8, 16, 224, 32), (2, 8, 96, 64)])
+def test_gradients_in_one_launch_of_values_beyond_the_split(oracle, bhnd, what):
+    """One head holds them; the others keep their bits, and it has what f32 arithmetic makes of them (delta among it, which
+    the dK/dV side forms itself)."""
+    b, h, n, d = bhnd
+    shape = ra.AttentionShape.new(*bhnd)
+    x = [seeded_normal(shape.buffer_len(), s).reshape(bhnd) for s in (71, 72, 73, 74)]
+    clean = [g.reshape(bhnd) for g in ra.flash_backward(shape, *[a.ravel() for a in x])]
+    q, k, v, d_out = x
+    at = (1, 5)
+    if what == "key inf":
+        q[at][:, 9] = -np.abs(q[at][:, 9]) - np.float32(0.1)
+        k[at][40, 9] = np.inf
+    elif what == "d_out small":
+        d_out[at] *= np.float32(2.0 ** -115)
+    else:
+        d_out[at][n - 1, 3] = np.nan if what == "d_out nan" else np.inf
+    got = [g.reshape(bhnd) for g in ra.flash_backward(shape, *[a.ravel() for a in x])]
+    one = [np.ascontiguousarray(a[at]).ravel() for a in x]
+    want = oracle.flash_backward(oracle.AttentionShape(1, 1, n, d), *one)
+    other = np.ones((b, h), dtype=bool)
+    other[at] = False
+    for name, g, c, w in zip(("dq", "dk", "dv"), got, clean, want):
+        assert np.array_equal(g[other], c[other]), name
+        gs, ws = g[at].astype(np.float64), w.reshape(n, d).astype(np.float64)
+        fin = np.isfinite(ws)
+        assert np.array_equal(np.isfinite(gs), fin), name
+        if fin.any():  # the gradients' bound of the f32 kernels against 64 bits, twice: the oracle sums in f32 as well
+            assert np.linalg.norm((gs - ws)[fin]) <= 4e-6 * np.linalg.norm(ws[fin]), name
