@@ -181,11 +181,9 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             return small && q_row < Nq;
         };
 
-        // A score tile (register i: key 8 (i/4) + 4 hh + i%4, query `col`): scaled and masked, then turned into weights.
-        // weights() returns the factor the sums so far have to be multiplied by.
-        auto scale_mask = [&](f32x16_t& s, int kv0) RT_INLINE {
-#pragma unroll
-            for (int i = 0; i < 16; i++) s[i] *= p.scale;
+        // A score tile (register i: key 8 (i/4) + 4 hh + i%4, query `col`): masked, then turned into weights.  The maximum is
+        // scaled, the scores are where it is subtracted.
+        auto hide = [&](f32x16_t& s, int kv0) RT_INLINE {
             if ((kv0 + kTile > N) || (kCausal && kv0 + kTile - 1 > q0w)) {
                 asm volatile("");  // a branch: the selects cost more than the jump
 #pragma unroll
@@ -200,7 +198,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
 #pragma unroll
             for (int i = 0; i < 16; i++) m_tile = __builtin_fmaxf(m_tile, s[i]);
             auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(m_tile), __float_as_uint(m_tile), false, false);
-            return __builtin_fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+            return __builtin_fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) * p.scale;
         };
         // the maximum goes to m_run; returns what is subtracted from the scores
         float alpha = 0.0f;
@@ -280,7 +278,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
             }
             if (tile + 2 < n_tiles) load_tile(tile + 2);
             f32x16_t s = s_next;
-            scale_mask(s, tile * kTile);
+            hide(s, tile * kTile);
             read_plane(kn, 2);
             zero16(s_next);
             // a third of the score product beside the row maximum, the rest beside the weights, two at a time
@@ -297,7 +295,7 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
                 if (k < 3) {
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        if (k == 0) y[i] = s[4 * g + i] - m_use;
+                        if (k == 0) y[i] = __builtin_fmaf(s[4 * g + i], p.scale, -m_use);
                         if (k == 1) y[i] *= kLog2e;
                         if (k == 2) sp.r[i] = __builtin_amdgcn_exp2f(y[i]);
                     }
@@ -390,12 +388,12 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
                     f32x16_t s;
                     zero16(s);
                     f32_rows<DT>(s, kb, q, col_f, hh_f);
-                    scale_mask(s, tile * kTile);
+                    hide(s, tile * kTile);
                     const float m_use = take_max(row_max(s));
                     float tile_l = 0.0f;
 #pragma unroll
                     for (int i = 0; i < 16; i++) {
-                        s[i] = __builtin_amdgcn_exp2f((s[i] - m_use) * kLog2e);
+                        s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], p.scale, -m_use) * kLog2e);
                         tile_l += s[i];
                     }
                     add_sum(tile_l);
@@ -556,9 +554,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
     for (int t = 0; t < DT; t++) zero16(acc_o[t]);
     float m_run = neg_inf(), l_run = 0.0f, l_low = 0.0f;
 
-    auto scale_mask = [&](f32x16_t& s, int kv0) RT_INLINE {
-#pragma unroll
-        for (int i = 0; i < 16; i++) s[i] *= p.scale;
+    auto hide = [&](f32x16_t& s, int kv0) RT_INLINE {  // (scaled where the maximum is subtracted)
         if ((kv0 + kTile > N) || (kCausal && kv0 + kTile - 1 > q0)) {
             asm volatile("");  // a branch: the selects cost more than the jump
 #pragma unroll
@@ -574,7 +570,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
 #pragma unroll
         for (int i = 0; i < 16; i++) m_tile = __builtin_fmaxf(m_tile, s[i]);
         auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(m_tile), __float_as_uint(m_tile), false, false);
-        const float m_new = __builtin_fmaxf(__builtin_fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])), m_run);
+        const float m_new = __builtin_fmaxf(__builtin_fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) * p.scale, m_run);
         const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
         alpha = (m_run == neg_inf()) ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_use) * kLog2e);
         m_run = m_new;
@@ -625,10 +621,10 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
 
     for (int tile = wave; tile < n_tiles; tile += NW) {
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NREQ) : "memory");  // K; V may still be on its way
-        // S, the large terms and the small ones in registers of their own; the next chunk of K is split meanwhile
-        f32x16_t s, s_low;
+        // S, the small terms of all chunks ahead of the large ones; the next chunk of K is split meanwhile
+        f32x16_t s;
         zero16(s);
-        zero16(s_low);
+        bf16x8_t head[KS];
         Piece pc[2];
         read_k(0, pc[0].x);
 #pragma unroll
@@ -637,21 +633,21 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
         for (int j = 0; j < KS; j++) {
             if (j + 1 < KS) read_k(j + 1, pc[(j + 1) & 1].x);
 #pragma unroll
-            for (int term = 0; term < 6; term++) {
-                f32x16_t& to = term == 5 ? s : s_low;
-                to = mfma_h(frag(pc[j & 1].w[kPlaneA[term]]), qf[j].p[kPlaneC[term]], to);
+            for (int term = 0; term < 5; term++) {
+                s = mfma_h(frag(pc[j & 1].w[kPlaneA[term]]), qf[j].p[kPlaneC[term]], s);
                 if (j + 1 < KS) {
 #pragma unroll
-                    for (int x = term * kPiece / 6; x < (term + 1) * kPiece / 6; x++) piece_step(pc[(j + 1) & 1], x, false);
+                    for (int x = term * kPiece / 5; x < (term + 1) * kPiece / 5; x++) piece_step(pc[(j + 1) & 1], x, false);
                 }
                 RT_ORDER();
             }
+            head[j] = frag(pc[j & 1].w[0]);
         }
+#pragma unroll
+        for (int j = 0; j < KS; j++) s = mfma_h(head[j], qf[j].p[0], s);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // K has been read
         request(k_rsrc, k_lds, tile + NW);
-#pragma unroll
-        for (int i = 0; i < 16; i++) s[i] += s_low[i];
-        scale_mask(s, tile * kTile);
+        hide(s, tile * kTile);
         const float m_use = take_max(s);
         rescale();
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NREQ) : "memory");  // V; the next K may be on its way
@@ -663,7 +659,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
         for (int g = 0; g < 4; g++) {
             float y[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) y[i] = (s[4 * g + i] - m_use) * kLog2e;
+            for (int i = 0; i < 4; i++) y[i] = __builtin_fmaf(s[4 * g + i], p.scale, -m_use) * kLog2e;
 #pragma unroll
             for (int i = 0; i < 4; i++) sp.r[i] = __builtin_amdgcn_exp2f(y[i]);
 #pragma unroll
@@ -745,12 +741,12 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
 #pragma unroll
                 for (int i = 0; i < 4; i++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], q[4 * j + i], s, 0, 0, 0);
             }
-            scale_mask(s, tile * kTile);
+            hide(s, tile * kTile);
             const float m_use = take_max(s);
             float tile_l = 0.0f;
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                s[i] = __builtin_amdgcn_exp2f((s[i] - m_use) * kLog2e);
+                s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], p.scale, -m_use) * kLog2e);
                 tile_l += s[i];
             }
             add_sum(tile_l);
