@@ -1864,26 +1864,29 @@ RT_API int rt_gqa_decode_naive_bf16(void* stream, const void* q, const void* k_c
 }
 
 namespace {
-// Into how many spans the keys of a chunk's units are cut: the cheapest of a workgroup's tile steps (1.15 us at head dim
-// 128 with a CU to itself, half as much again for every workgroup that shares it) plus, when there are spans, the merge
-// launch (4 us) and the partials' way to memory and back (4.5 TB/s).  Over 30 shapes (2 to 512 positions, 700 to 8192
-// keys, head dims 64 to 256) its choice is within 3 % of the best count measured, 6 % at one of them.  One sequence, 32
-// heads over 8, 8192 keys: 16 positions 119 -> 15.3 us (32 spans), 128 positions 123 -> 29.3 us (8), 512 positions 122
-// -> 74 us (4).
-// Units that fill the chip by themselves are not cut, and no span is shorter than two key tiles.
+// Into how many spans the keys of a chunk's units are cut: the cheapest of a workgroup's tile steps (0.75 us at head dim 64,
+// 1.1 at 128, with a CU to itself, half as much again for every workgroup that shares it; above head dim 64, where no third one
+// covers its set-up, each costs 0.8 us besides) plus, when there are spans, the merge launch (3 us) and the partials' way to memory
+// and back (3 TB/s).  Over 36 shapes (2 to 341 positions, 130 to 8192 keys, head dims 64 to 256) its choice is within 2 % of
+// the best count measured.  One sequence, 32 heads over 8 of 128, 8192 keys: 16 positions 119 -> 14.9 us (32 spans), 100
+// positions 28.5 (8).  Short walks are cut to single tiles: 16 heads of 64, 2 positions over 900 keys, us by spans 1 16.3, 5 10.1,
+// 8 9.3, 15 7.9; 8 x 16 heads of 64, 4 over 800, 1 14.6, 2 14.2, 4 12.6; 32 / 8 of 128, 4 over 200, 1 9.6, 4 8.6; but, for their
+// partials, 16 over 1000, 8 10.5, 16 10.9.
+// Units that fill the chip by themselves are not cut.
 long long chunk_splits(long long slabs, long long rows, int head_dim, long long keys) {
     const long long key_tile = rt::flash_tile_bf16_key_tile(head_dim), tiles = (keys + key_tile - 1) / key_tile;
     const long long units = slabs * ((rows + 127) / 128);
     if (units >= g_num_cus || tiles < 4) return 1;
     const long long occ = rt::flash_tile_bf16_workgroups(head_dim);
-    const float step_us = 1.15f * (float)key_tile * (float)head_dim / (64.0f * 128.0f);
-    const float partial_us = (float)(slabs * rows) * (float)(head_dim + 2) * (2 * sizeof(float)) / 4.5e6f;
+    const float step_us = 0.4f + 0.7f * (float)key_tile * (float)head_dim / (64.0f * 128.0f);
+    const float partial_us = (float)(slabs * rows) * (float)(head_dim + 2) * (2 * sizeof(float)) / 3.0e6f;
     long long best = 1;
     float best_us = 0.0f;
-    for (long long n = 1; n <= std::min<long long>(tiles / 2, 64) && (n - 1) * units < occ * g_num_cus; n++) {
+    for (long long n = 1; n <= std::min<long long>(tiles, 64) && (n - 1) * units < occ * g_num_cus; n++) {
         const long long per_cu = (units * n + g_num_cus - 1) / g_num_cus, rounds = per_cu / occ, rest = per_cu % occ;
         const float load = 0.5f * (float)(rounds * (occ + 1) + (rest ? rest + 1 : 0));
-        const float us = (float)((tiles + n - 1) / n) * step_us * load + (n > 1 ? 4.0f + (float)n * partial_us : 0.0f);
+        const float us = (float)((tiles + n - 1) / n) * step_us * load + (head_dim > 64 ? 1.6f * (load - 1.0f) : 0.0f) +
+                         (n > 1 ? 3.0f + (float)n * partial_us : 0.0f);
         if (n == 1 || us < best_us) {
             best = n;
             best_us = us;

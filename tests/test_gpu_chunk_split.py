@@ -36,6 +36,22 @@ def test_spans_fold_to_the_whole(oracle, b, s, hq, hkv, d, max_seq, lens):
     assert_bf16_parity(oracle.bf16_to_f32(out.download(np.uint16)), want, d, None, f"s={s} hq={hq} d={d}")
 
 
+@pytest.mark.parametrize("b,s,hq,hkv,d,max_seq,lens", [
+    (1, 2, 16, 16, 64, 900, [900]),           # as many spans as tiles, the last of four keys
+    (1, 4, 8, 2, 64, 1473, [1473]),           # the last of one
+    (3, 4, 32, 8, 128, 200, [200, 65, 4]),    # spans without keys, and of the new positions alone
+    (1, 8, 16, 2, 256, 300, [300]),           # tiles of 32 keys
+    (2, 5, 12, 12, 80, 321, [320, 257]),      # columns past the head dim
+    (4, 4, 16, 16, 64, 800, [800, 1, 0, 449]),  # two workgroups a CU, positions without keys
+])
+def test_spans_of_a_tile(oracle, b, s, hq, hkv, d, max_seq, lens):
+    (q, k, v), (dq, dk, dv), out = tensors(b, s, hq, hkv, d, max_seq)
+    K.gqa_decode_chunk_bf16(None, dq, dk, dv, out, dev(np.asarray(lens, dtype=np.int32)), b, s, hq, hkv, d, max_seq)
+    ra.synchronize()
+    want = oracle.gqa_decode_chunk_bf16(q, k, v, lens, b, s, hq, hkv, d, max_seq)
+    assert_bf16_parity(oracle.bf16_to_f32(out.download(np.uint16)), want, d, None, f"s={s} hq={hq} d={d}")
+
+
 def test_a_captured_call_stays_within_the_fixed_scratch(oracle):
     b, s, hq, hkv, d, max_seq = 1, 100, 16, 2, 256, 2048
     (q, k, v), (dq, dk, dv), out = tensors(b, s, hq, hkv, d, max_seq)
