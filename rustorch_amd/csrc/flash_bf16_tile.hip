@@ -215,7 +215,18 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     static_assert(!BIAS || DIRECT || DP > 128, "a bias up to head dim 128 comes with tiles straight to LDS");
     static_assert(PIPE || !HALVES, "the halves meet once a tile");
 
-    constexpr int kTilesLds = DIRECT ? Cfg::LDS_BYTES_DIRECT : Cfg::LDS_BYTES;  // BIAS: the four waves' bias values behind the tiles
+    // QLDS: the query rows come through LDS as well, whole lines an instruction, over V(1), whose request comes behind the first
+    // barrier only, and as many bytes behind it.  Read straight into the operands, 16 bytes of 32 rows at a time, every line was
+    // asked for by four instructions (eight at head dim 128).  us, inputs that change from pass to pass, bhnd / bnhd, before ->
+    // now: window 256, 4 16 4096 64 43.9 -> 42.5 / 47.0 -> 45.2, window 64 34.2 -> 32.9 / 37.0 -> 34.8, window 126, 5 12 7697 128
+    // 113.2 -> 107.6 / 120.2 -> 112.8; causal 2 32/8 1501 128 46.3 -> 45.3 / 46.7 -> 45.8, 4 16 1024 64 16.7 -> 16.4; masked 4 16
+    // 1024 64 31.2 -> 30.5.  Past the caches as well under a window at head dim 64 (42.7 -> 41.4 / 45.5 -> 45.2); elsewhere that is
+    // slower (causal 2 32/8 1501 128 45.2 -> 47.4).  Not where rows run over a group's heads, nor beside a bias at head dim 128, where two
+    // workgroups a CU would not fit.
+    constexpr bool QLDS = DIRECT && !PACKED && !(BIAS && DP == 128);
+    constexpr int kQAt = 3 * Cfg::STAGE_BYTES;
+    static_assert(!QLDS || KT * 2 == TROWS, "half of the query rows fit a stage");
+    constexpr int kTilesLds = QLDS ? (5 * Cfg::STAGE_BYTES > 4 * Cfg::REGION ? 5 * Cfg::STAGE_BYTES : 4 * Cfg::REGION) : DIRECT ? Cfg::LDS_BYTES_DIRECT : Cfg::LDS_BYTES;  // BIAS: the four waves' bias values behind the tiles
     constexpr int kHalves = HALVES ? 2 : 1, kBiasAt = kHalves * ((kTilesLds + 1023) / 1024 * 1024);
     static_assert(!HALVES || (kTilesLds % 1024 == 0 && kTilesLds >= 4 * 32 * DP * 4 && kTilesLds >= 4 * Cfg::REGION + 2048), "a half's partials fit over its tiles, their max and sum behind the output rows");
     __shared__ alignas(DIRECT || BIAS ? 1024 : 16) unsigned char lds[BIAS ? kBiasAt + kHalves * 4 * Cfg::BIAS_BYTES : kHalves * kTilesLds];
@@ -645,8 +656,25 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
 
         // ---- Q as B operand: column q = lane % 32, contraction slots 16 ks + 8 hh .. + 8
         bf16x8_t qreg[KS];
+        if constexpr (QLDS) {
+            // instruction n: chunks 64 n .. + 63 of the wave's 32 rows, swizzled as those of a K tile (zeros behind the last row
+            // and behind the head dim)
+            const int r_first = q0 + 32 * wq, n_rows = max(min(32, rows_total - r_first), 0);
+            const uint32_t q_pitch = (uint32_t)p.lq.row_pitch;
+            const u32x4_t Qd = make_rsrc(p.q + (size_t)b * p.lq.batch_stride + (size_t)h0 * p.lq.head_stride + (size_t)min(r_first, rows_total - 1) * q_pitch,
+                                         n_rows > 0 ? ((uint32_t)(n_rows - 1) * q_pitch + (uint32_t)D) * 2u : 0u);
+#pragma unroll
+            for (int n = 0; n < CH / 2; n++) {
+                const int c = 64 * n + lane, row = (int)((uint32_t)c / CH), slot = (c - row * CH) ^ swz_k(row);
+                const uint32_t at = 8 * slot < D ? (uint32_t)row * q_pitch * 2u + 16u * (uint32_t)slot : 0x7fffffffu;
+                const uint32_t block = lds_base + half_at + (uint32_t)(kQAt + wave * 32 * ROWB + 1024 * n);
+                if constexpr (WIN && DP <= 64) buffer_to_lds_past(Qd, at, 0u, block);
+                else buffer_to_lds(Qd, at, 0u, block);
+            }
+        }
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
+            if constexpr (QLDS) break;
             // Unconditional loads (a row past the tensor is read from the tensor's last row, a chunk past the head dim
             // from its last chunk): a load under a per-lane test costs a branch of its own.  A row that does not exist
             // has every score masked and is not written, so what it holds does not matter; the columns past the head
@@ -703,6 +731,13 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             // tile 0 and K(1) have landed (and the queries); V rows of tile 0 past the last key, requested before the
             // lengths were known, are zeroed by the lane that fetched them
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if constexpr (QLDS) {
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++) {
+                    const unsigned char* const at = lds + kQAt + wave * 32 * ROWB;
+                    qreg[ks] = *(const bf16x8_t*)(at + (DP == 96 ? ((ks & 1) ? k_base1 : k_base) + (uint32_t)(64 * (ks >> 1)) : k_base ^ (uint32_t)(32 * ks)));
+                }
+            }
             if (n_keys < KT) {
 #pragma unroll
                 for (int n = 0; n < NLD; n++)

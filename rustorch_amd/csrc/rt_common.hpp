@@ -48,6 +48,15 @@ __device__ __forceinline__ void buffer_to_lds(const u32x4_t& rsrc, uint32_t lane
                  : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so)
                  : "memory");
 }
+// the same past the caches (`nt`), for what no other workgroup reads
+__device__ __forceinline__ void buffer_to_lds_past(const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
+    const uint32_t so = __builtin_amdgcn_readfirstlane(tile_off);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 :
+                 : "s"(m), "v"(lane_off), "s"(rsrc), "s"(so)
+                 : "memory");
+}
 // the same for the lanes of `on` alone (what the others would have brought stays as it is in LDS); no branch around it
 __device__ __forceinline__ void buffer_to_lds_of(uint64_t on, const u32x4_t& rsrc, uint32_t lane_off, uint32_t tile_off, uint32_t lds_block) {
     const uint32_t m = __builtin_amdgcn_readfirstlane(lds_block);
