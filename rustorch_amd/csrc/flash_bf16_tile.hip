@@ -220,7 +220,8 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     // asked for by four instructions (eight at head dim 128).  us, inputs that change from pass to pass, bhnd / bnhd, before ->
     // now: window 256, 4 16 4096 64 43.9 -> 42.5 / 47.0 -> 45.2, window 64 34.2 -> 32.9 / 37.0 -> 34.8, window 126, 5 12 7697 128
     // 113.2 -> 107.6 / 120.2 -> 112.8; causal 2 32/8 1501 128 46.3 -> 45.3 / 46.7 -> 45.8, 4 16 1024 64 16.7 -> 16.4; masked 4 16
-    // 1024 64 31.2 -> 30.5.  Past the caches as well under a window at head dim 64 (42.7 -> 41.4 / 45.5 -> 45.2); elsewhere that is
+    // 1024 64 31.2 -> 30.5.  Past the caches as well under a window up to head dim 64 where the
+    // workgroups do not fit the chip at once (42.7 -> 41.4 / 45.5 -> 45.2; 1 8/2 852 64 window 104 7.7 -> 7.8); elsewhere that is
     // slower (causal 2 32/8 1501 128 45.2 -> 47.4).  Not where rows run over a group's heads, nor beside a bias at head dim 128, where two
     // workgroups a CU would not fit.
     constexpr bool QLDS = DIRECT && !PACKED && !(BIAS && DP == 128);
@@ -661,6 +662,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             // and behind the head dim)
             const int r_first = q0 + 32 * wq, n_rows = max(min(32, rows_total - r_first), 0);
             const uint32_t q_pitch = (uint32_t)p.lq.row_pitch;
+            const bool many = WIN && (uint64_t)gridDim.x * gridDim.y * gridDim.z > (uint64_t)p.n_cus * Cfg::OCC_DIRECT;
             const u32x4_t Qd = make_rsrc(p.q + (size_t)b * p.lq.batch_stride + (size_t)h0 * p.lq.head_stride + (size_t)min(r_first, rows_total - 1) * q_pitch,
                                          n_rows > 0 ? ((uint32_t)(n_rows - 1) * q_pitch + (uint32_t)D) * 2u : 0u);
 #pragma unroll
@@ -668,7 +670,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
                 const int c = 64 * n + lane, row = (int)((uint32_t)c / CH), slot = (c - row * CH) ^ swz_k(row);
                 const uint32_t at = 8 * slot < D ? (uint32_t)row * q_pitch * 2u + 16u * (uint32_t)slot : 0x7fffffffu;
                 const uint32_t block = lds_base + half_at + (uint32_t)(kQAt + wave * 32 * ROWB + 1024 * n);
-                if constexpr (WIN && DP <= 64) buffer_to_lds_past(Qd, at, 0u, block);
+                if (WIN && DP <= 64 && many) buffer_to_lds_past(Qd, at, 0u, block);
                 else buffer_to_lds(Qd, at, 0u, block);
             }
         }
