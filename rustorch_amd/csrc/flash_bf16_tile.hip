@@ -10,7 +10,8 @@
 // (batch, head) and is gone when they are done; several workgroups share a CU, so one workgroup's set-up, softmax
 // and output overlap with another's matrix work without any hand-written interleaving, and the hardware
 // dispatcher balances jobs of unequal length.  Keys are walked KT at a time through a double-buffered LDS tile (straight
-// from memory, or through registers above head dim 128 and under a key-padding vector; one workgroup barrier per tile);
+// from memory, or through registers above head dim 128 and under a key-padding vector whose bits do not fit LDS; one workgroup
+// barrier per tile);
 // per 32-key item a wave computes
 //
 //   S^T[kv, q]  = K[kv, :] . Q[q, :]      v_mfma_f32_32x32x16_bf16, A = K tile (LDS), B = Q (registers)
@@ -172,7 +173,7 @@ enum TileWay : int { kTilesRegs = 0, kTilesDirect = 1, kTilesDirectPart = 2 };
 // moved by that many keys, as for a span of SPLIT), and an item that holds keys below some row's window is masked on
 // that side as well.
 //
-// DIRECT (head dims up to 128, no key-padding vector): the tiles travel from memory straight into LDS
+// DIRECT (head dims up to 128): the tiles travel from memory straight into LDS
 // (buffer_load_dwordx4 ... lds) instead of through registers and LDS writes.  After a tile's barrier the waves request
 // K(t+2) and V(t+1) into the stages K(t) and V(t-1) have just left and wait for their own requests ahead of the next
 // tile's barrier.  LDS rows are unpadded (a landing block of 1 KB is contiguous) and their 16-byte slots are XORed
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     static_assert(!SPLIT || (PACKED && !BIAS && MODE == kMaskCausal), "the split over the keys serves the chunked decode");
     static_assert(!WIN || (!PACKED && !BIAS && !SPLIT && MODE == kMaskCausal), "the window is a causal mask's");
     static_assert(!HALVES || (TILES != kTilesRegs && !PACKED && !SPLIT && !WIN), "halves of the walk: tiles straight to LDS, rows of one head");
-    static_assert(TILES == kTilesRegs || (DP <= 128 && MODE != kMaskPadding), "tiles straight into LDS: head dims up to 128, no key-padding vector");
+    static_assert(TILES == kTilesRegs || DP <= 128, "tiles straight into LDS: head dims up to 128");
     constexpr bool DIRECT = TILES != kTilesRegs, WHOLE = TILES == kTilesDirect;
     using Cfg = TileCfg<DP>;
     constexpr int KT = Cfg::KT, LDK = Cfg::LDK, LDV = Cfg::LDV, NI = Cfg::NI, TTHREADS = Cfg::THREADS;
@@ -209,9 +210,9 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     constexpr int PF = Cfg::PF;        // register sets of tiles in flight behind the two LDS stages
     static_assert(2 * DT == KS, "one P.V matrix instruction per score matrix instruction");
     // Head dims above 128 do not have the registers for two score tiles and their operands in flight (O alone is 128
-    // registers), nor does head dim 128 with a key-padding mask: there an item runs its three phases one after the other,
-    // and K is parked with V.
-    constexpr bool PIPE = DP <= 128 && !(MODE == kMaskPadding && DP == 128);
+    // registers), nor does head dim 128 with a key-padding mask and tiles through registers: there an item runs its three phases
+    // one after the other, and K is parked with V.
+    constexpr bool PIPE = DP <= 128 && !(MODE == kMaskPadding && DP == 128 && !DIRECT);
     static_assert(!BIAS || DIRECT || DP > 128, "a bias up to head dim 128 comes with tiles straight to LDS");
     static_assert(PIPE || !HALVES, "the halves meet once a tile");
 
@@ -507,7 +508,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             if ((tid + TTHREADS * n) / CH >= n_keys) vreg[0][n] = u32x4_t{0u, 0u, 0u, 0u};
     }
 
-    if (MODE == kMaskPadding && n_keys > 0) {  // keep bytes past the last key count as kept: `lim` masks those keys
+    if (MODE == kMaskPadding && !DIRECT && n_keys > 0) {  // keep bytes past the last key count as kept: `lim` masks those keys
         const int j = lane & (KT - 1);
         const uint32_t kb = p.keep[min(j, n_keys - 1)];
         keep_raw[0] = j < n_keys ? kb : 1u;
@@ -557,6 +558,12 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             for (int n = 0; n < NL; n++)
                 if (D == DP || ld_on[n]) *(u32x4_t*)(lds + st * (KT * LDK * 2) + st_k[n]) = src[n];
         };
+        // Mask::Padding, DIRECT: a bit per key in LDS, behind V(1)'s stage, where half of the query rows came in; a wave reads
+        // the word of its next item a step ahead
+        constexpr bool KEEP_BITS = MODE == kMaskPadding && DIRECT;
+        static_assert(!KEEP_BITS || QLDS, "the bits take the query rows' place");
+        constexpr int kKeepAt = 4 * Cfg::STAGE_BYTES;
+        uint32_t keep_word_next = ~0u;
         uint64_t keep_cur = ~0ull, keep_next = ~0ull;  // keep bits of the tile whose items are in their softmax step, and of the next
         auto park_v = [&](auto set_c, int st) __attribute__((always_inline)) {
             constexpr int SET = decltype(set_c)::value;
@@ -648,8 +655,8 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
 
         // Mask::Padding hiding the reference's whole first key tile: every row NaN (the tiled recurrence of
         // cpu_forward.rs:268-425 takes exp(-inf - (-inf)) on that tile and never recovers)
-        if (MODE == kMaskPadding) {
-            const int lead = p.ref_bc < n_keys ? p.ref_bc : n_keys;
+        const int lead = p.ref_bc < n_keys ? p.ref_bc : n_keys;
+        if (MODE == kMaskPadding && !KEEP_BITS) {
             bool any = false;
             for (int j = lane; j < lead; j += kWave) any |= (p.keep[j] != 0);
             poison = !__any(any);
@@ -718,6 +725,21 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         };
 
 
+        constexpr int KB = 8;  // ballots of a wave whose bytes are requested together
+        uint32_t keep_byte[KB];
+        auto keep_load = [&](int base) __attribute__((always_inline)) {  // keys base + 256 i + 64 wave + lane
+#pragma unroll
+            for (int i = 0; i < KB; i++) {
+                const int first = base + 256 * i + 64 * wave;
+                keep_byte[i] = 1u;  // (keys past the end are masked by `lim`)
+                if (first < n_keys) {
+                    const uint32_t x = p.keep[min(first + lane, n_keys - 1)];
+                    keep_byte[i] = first + lane < n_keys ? x : 1u;
+                }
+            }
+        };
+        if constexpr (KEEP_BITS) keep_load(0);
+
         // K(0), V(0) -> stage 0, K(1) -> stage 1; then the register sets take K(2) .. K(1 + PF) and V(1) .. V(PF)
         // (K(j) travels in set j % PF, and so does V(j))
         f32x4_t bv[4] = {};  // bias values of the item whose softmax step comes next
@@ -746,6 +768,20 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
                     if (dl_row[n] >= n_keys) *(u32x4_t*)(lds + half_at + 2 * STAGE_B + (wave + 4 * n) * 1024 + 16 * lane) = u32x4_t{0u, 0u, 0u, 0u};
             }
             bias_first();
+            if constexpr (KEEP_BITS) {
+                __syncthreads();  // every wave has read its query rows
+                for (int base = 0;;) {
+#pragma unroll
+                    for (int i = 0; i < KB; i++) {
+                        const int first = base + 256 * i + 64 * wave;
+                        const uint64_t bits = __ballot(keep_byte[i] != 0);
+                        if (lane == 0 && first < n_keys) *(u32x2_t*)(lds + kKeepAt + first / 8) = u32x2_t{(uint32_t)bits, (uint32_t)(bits >> 32)};
+                    }
+                    base += 256 * KB;
+                    if (base >= n_keys) break;
+                    keep_load(base);
+                }
+            }
         } else {
             park_k(kreg[0], 0);
             park_v(std::integral_constant<int, 0>{}, 0);
@@ -766,6 +802,13 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             }
         }
         __syncthreads();
+        if constexpr (KEEP_BITS) {
+            keep_word_next = *(const uint32_t*)(lds + kKeepAt);
+            bool any = false;
+            for (int j = lane; 32 * j < lead; j += kWave)
+                any |= (*(const uint32_t*)(lds + kKeepAt + 4 * j) & (lead - 32 * j >= 32 ? ~0u : (1u << (lead - 32 * j)) - 1u)) != 0;
+            poison = !__any(any);
+        }
 
         // ---- pieces of a step
         // the bias, then the masks, on the scores of the item whose keys start at k0 (item `it` of its tile)
@@ -787,7 +830,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
                 for (int i = 0; i < 16; i++) sc[i] = (8 * (i >> 2) + (i & 3) < room_lo) ? neg_inf() : sc[i];
             }
             if (MODE == kMaskPadding) {
-                const uint32_t keep_word = (uint32_t)(keep_cur >> (32 * it));
+                const uint32_t keep_word = KEEP_BITS ? (uint32_t)__builtin_amdgcn_readfirstlane(keep_word_next) : (uint32_t)(keep_cur >> (32 * it));
                 if (keep_word != 0xffffffffu) {
                     const uint32_t mine = keep_word >> (4 * hh);  // bit 8(i/4) + i%4 of `mine` is key 8(i/4) + 4hh + i%4
 #pragma unroll
@@ -969,6 +1012,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         auto step = [&](int it, int k0, const uint16_t* kp, const uint16_t* vp, f32x16_t& s_cur, f32x16_t& s_next,
                         bf16x8_t (&p_prev)[2], bf16x8_t (&p_new)[2], auto wait_c) __attribute__((always_inline)) {
             mask_item(it, k0, s_cur);
+            if constexpr (KEEP_BITS) keep_word_next = *(const uint32_t*)(lds + kKeepAt + min((k0 >> 5) + 1, (n_keys - 1) >> 5) * 4);
 #pragma unroll
             for (int i = 0; i < 16; i++) s_next[i] = 0.0f;
             u32x4_t ops[NM];
@@ -1928,7 +1972,7 @@ hipError_t launch_one(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
     return hipGetLastError();
 }
 
-// Tiles straight to LDS wherever the kernel has that form: head dims up to 128 without a key-padding vector.
+// Tiles straight to LDS wherever the kernel has that form: head dims up to 128.
 template <int DP, int TILES>
 hipError_t launch_tiles(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
     if (p.n_splits > 1) {  // (rows packed over a group of one head are rows of that head)
@@ -1979,7 +2023,19 @@ static bool takes_halves(const FlashTileParams& p, dim3 grid) {
 }
 template <int DP>
 hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
-    if (p.mask == kMaskPadding) return launch_one<DP, kMaskPadding, false, false>(stream, p, grid);
+    if (p.mask == kMaskPadding) {
+        // Tiles straight to LDS and a bit per key, as far as the bits fit a stage (from 32768 keys at DP 32 to 131072 at 128).  us,
+        // a byte a lane with tiles through registers -> this, the last eighth of the keys hidden, B H N head dim: 2 12 2032 128
+        // 72.7 -> 60.7 (no mask 57.0), 1 12 1866 96 43.6 -> 35.9, 3 16 1117 80 33.9 -> 29.5, 4 16 2048 64 87.5 -> 80.3, 8 16 512 64 15.6 ->
+        // 14.3, 2 16 3000 32 64.3 -> 63.5.  A single tile at head dim 128 stays: 5 16 42 128 6.2, 6.4.
+        if constexpr (DP <= 128) {
+            if (p.seq_kv <= 8 * TileCfg<DP>::STAGE_BYTES && (DP < 128 || p.seq_kv > TileCfg<DP>::KT)) {
+                if (p.dim == DP) return launch_one<DP, kMaskPadding, false, false, false, false, kTilesDirect>(stream, p, grid);
+                return launch_one<DP, kMaskPadding, false, false, false, false, kTilesDirectPart>(stream, p, grid);
+            }
+        }
+        return launch_one<DP, kMaskPadding, false, false>(stream, p, grid);
+    }
     if constexpr (DP <= 128) {
         constexpr int kTiles = DP % 64 == 0 ? kTilesDirect : kTilesDirectPart;
         if ((kTiles == kTilesDirectPart || p.dim == DP) && takes_halves(p, grid)) return launch_halves<DP, kTiles>(stream, p, grid);

@@ -629,3 +629,29 @@ def test_which_causal_launches_walk_in_halves(force_kernel, h, n, d, halves):
     one = flash_bf16(ra.AttentionShape.new(1, h, n, d), q, k, v, ra.Mask.causal())
     two = flash_bf16(ra.AttentionShape.new(2, h, n, d), *(np.tile(x, 2) for x in (q, k, v)), ra.Mask.causal())
     assert np.array_equal(one, two[: one.size]) != halves
+
+
+@pytest.mark.parametrize("n,d", [(2047, 64), (2048, 128), (2049, 80), (2049, 32), (4100, 64), (64, 128), (65, 128), (32768, 32), (32769, 32)])
+def test_padding_bits(oracle, force_kernel, n, d):
+    """A key-padding vector as bits in LDS: more keys than one set of requests brings, hidden items and tiles, the last word not
+    whole, and either side of the lines to the form that reads bytes.  Sampled rows, as above."""
+    force_kernel("tile")
+    b, h = 1, 2
+    (qb, qf), (kb, kf), (vb, vf) = inputs((b, h, n, d), (b, h, n, d), (94, 95, 96))
+    keep = np.random.default_rng(n).random(n) < 0.6
+    keep[n // 3:n // 3 + 200] = False
+    keep[5] = True
+    got = flash_bf16(ra.AttentionShape.new(b, h, n, d), qb, kb, vb, ra.Mask.padding(keep)).reshape(h, n, d)
+    assert np.isfinite(got).all()
+    for head in range(h):
+        q2, k2, v2 = (x.reshape(h, n, d)[head] for x in (qf, kf, vf))
+        k2, v2 = k2[keep], v2[keep]
+        for i in sorted({0, 31, 32, n // 2, n - 2, n - 1}):
+            want = oracle.gqa_forward_f32(q2[i], k2, v2, 1, 1, 1, 1, k2.shape[0], d)
+            assert_bf16_parity(got[head, i], want, d, 1, f"n={n} d={d} row {i}")
+    first = np.ones(n, bool)
+    first[:64] = False  # the reference's first key tile hidden: every row NaN
+    if n > 64:
+        assert np.isnan(flash_bf16(ra.AttentionShape.new(b, h, n, d), qb, kb, vb, ra.Mask.padding(first))).all()
+        first[63] = True
+        assert np.isfinite(flash_bf16(ra.AttentionShape.new(b, h, n, d), qb, kb, vb, ra.Mask.padding(first))).all()
