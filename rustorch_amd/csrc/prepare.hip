@@ -113,9 +113,10 @@ __global__ __launch_bounds__(64) void decode_prepare_kernel(DecodePrepareParams 
 // and nothing is kept there for the rows that come behind), and V, which is only passed through, comes with `nt`.
 // B=4, 32 + 8 heads, 4096 tokens, D=128, us with 6 sets of inputs in turn: plain 92.7; rows out `nt` 87.9, `sc1` 89.7,
 // `nt sc1` 83.8, V's loads `nt` too 80.3, q's and k's as well 82.8.  (The compiler has a builtin for both bits on buffer stores.)
+template <bool kPast>
 __device__ __forceinline__ void put16(__amdgpu_buffer_rsrc_t rs, uint32_t byte, u32x4_t v) {
     constexpr int kNt = 2, kSc1 = 16;
-    __builtin_amdgcn_raw_buffer_store_b128(v, rs, byte, 0, kNt | kSc1);
+    __builtin_amdgcn_raw_buffer_store_b128(v, rs, byte, 0, kPast ? kNt | kSc1 : 0);
 }
 
 // The same arithmetic for a prompt.  With many consecutive tokens per head the one-wave kernel above is bound by its
@@ -128,7 +129,7 @@ __device__ __forceinline__ void put16(__amdgpu_buffer_rsrc_t rs, uint32_t byte, 
 // DMAX; every pointer 16-byte aligned.  Grid (token blocks, heads, batch), token blocks fastest: workgroups go round-robin
 // to the 8 XCDs in that order, so all heads of a token block run on one XCD and its cos / sin rows are fetched into one
 // L2, once (with the heads fastest every XCD fetched every table row: 76 MB more on the prompt above).
-template <int ROWS, int DMAX>
+template <int ROWS, int DMAX, bool kPast>
 __global__ __launch_bounds__(256) void prompt_prepare_kernel(DecodePrepareParams p) {
     __shared__ uint32_t rows_w[ROWS * (DMAX + 2) / 2];
     __shared__ float inv[ROWS];
@@ -211,14 +212,14 @@ __global__ __launch_bounds__(256) void prompt_prepare_kernel(DecodePrepareParams
             o0[e] = pack_bf16x2(x0[i0] * c0 - x1[i0] * s0, x0[i1] * c1 - x1[i1] * s1);
             o1[e] = pack_bf16x2(x1[i0] * c0 + x0[i0] * s0, x1[i1] * c1 + x0[i1] * s1);
         }
-        put16(dst_rs, (uint32_t)(r * D + k0) * 2u, o0);
-        put16(dst_rs, (uint32_t)(r * D + half + k0) * 2u, o1);
+        put16<kPast>(dst_rs, (uint32_t)(r * D + k0) * 2u, o0);
+        put16<kPast>(dst_rs, (uint32_t)(r * D + half + k0) * 2u, o1);
     }
     if (!is_q) {
         const uint16_t* vs = p.v_in + kv_row;
         uint16_t* vd = p.v_cache + (((size_t)b * p.n_kv + kvh) * (size_t)p.max_seq + (size_t)(pos0 + sq0)) * D;
         const __amdgpu_buffer_rsrc_t vd_rs = __builtin_amdgcn_make_buffer_rsrc(vd, 0, (uint32_t)(n_rows * D) * 2u, kBufferFlags);
-        for (int c = tid; c < n_rows * CH; c += 256) put16(vd_rs, 16u * (uint32_t)c, __builtin_nontemporal_load((const u32x4_t*)(vs + 8 * (size_t)c)));
+        for (int c = tid; c < n_rows * CH; c += 256) put16<kPast>(vd_rs, 16u * (uint32_t)c, kPast ? __builtin_nontemporal_load((const u32x4_t*)(vs + 8 * (size_t)c)) : *(const u32x4_t*)(vs + 8 * (size_t)c));
     }
 }
 
@@ -236,10 +237,17 @@ hipError_t launch_decode_prepare(hipStream_t stream, const DecodePrepareParams& 
                          aligned16(p.v_in) && aligned16(p.k_cache) && aligned16(p.v_cache) && aligned16(p.cos_table) &&
                          aligned16(p.sin_table) && aligned16(p.q_gamma) && aligned16(p.k_gamma) && p.n_heads + p.n_kv <= 65535;
     if (wide_ok) {
+        // past the caches where the rows written do not fit the L2s, 8 of 4 MB: us, plainly / past, 32 / 8 heads of 128: 1 x 70
+        // tokens 6.3 / 7.3, 1 x 2048 (25 MB) 13.4 / 14.0, 1 x 4096 (50 MB) 28.6 / 24.0, 2 x 3000 42.3 / 35.8; 4 x 8 of 256, 301 15.8 / 18.4
+        const double written = 2.0 * p.batch * p.seq * (double)p.head_dim * (p.n_heads + 2.0 * p.n_kv);
+        const bool past = written > 32.0 * (1 << 20);
+        const dim3 grid((p.seq + 63) / 64, p.n_heads + p.n_kv, p.batch), block(256);
         if (p.head_dim <= 128) {
-            hipLaunchKernelGGL((prompt_prepare_kernel<64, 128>), dim3((p.seq + 63) / 64, p.n_heads + p.n_kv, p.batch), dim3(256), 0, stream, p);
+            if (past) hipLaunchKernelGGL((prompt_prepare_kernel<64, 128, true>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((prompt_prepare_kernel<64, 128, false>), grid, block, 0, stream, p);
         } else {
-            hipLaunchKernelGGL((prompt_prepare_kernel<64, 256>), dim3((p.seq + 63) / 64, p.n_heads + p.n_kv, p.batch), dim3(256), 0, stream, p);
+            if (past) hipLaunchKernelGGL((prompt_prepare_kernel<64, 256, true>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((prompt_prepare_kernel<64, 256, false>), grid, block, 0, stream, p);
         }
         return hipGetLastError();
     }
