@@ -10,9 +10,8 @@
 // (batch, head) and is gone when they are done; several workgroups share a CU, so one workgroup's set-up, softmax
 // and output overlap with another's matrix work without any hand-written interleaving, and the hardware
 // dispatcher balances jobs of unequal length.  Keys are walked KT at a time through a double-buffered LDS tile (straight
-// from memory, or through registers above head dim 128 and under a key-padding vector whose bits do not fit LDS; one workgroup
-// barrier per tile);
-// per 32-key item a wave computes
+// from memory, or through registers above head dim 128 and under a key-padding vector whose bits do not fit LDS; one
+// workgroup barrier per tile); per 32-key item a wave computes
 //
 //   S^T[kv, q]  = K[kv, :] . Q[q, :]      v_mfma_f32_32x32x16_bf16, A = K tile (LDS), B = Q (registers)
 //   online softmax on S^T (a lane holds 16 scores of query row lane % 32; row max / sum are in-lane plus one
@@ -191,7 +190,7 @@ enum TileWay : int { kTilesRegs = 0, kTilesDirect = 1, kTilesDirectPart = 2 };
 // the split form's merge does.  For launches that leave a CU one workgroup: its waves, alone on their SIMDs, take 800
 // clocks an item at head dim 64 where three of them together take 500 each, and 2100 with a bias, whose latency one wave
 // does not hide.  (launch_halves has the figures.)
-template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs, bool HALVES = false>
+template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs, bool HALVES = false, bool QROWS = true>
 __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : BIAS && DP == 64 ? 2 : (TILES ? TileCfg<DP>::OCC_DIRECT : TileCfg<DP>::OCC)) void flash_tile_bf16_kernel(FlashTileParams p) {
     static_assert(!SPLIT || (PACKED && !BIAS && MODE == kMaskCausal), "the split over the keys serves the chunked decode");
     static_assert(!WIN || (!PACKED && !BIAS && !SPLIT && MODE == kMaskCausal), "the window is a causal mask's");
@@ -223,9 +222,10 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     // 113.2 -> 107.6 / 120.2 -> 112.8; causal 2 32/8 1501 128 46.3 -> 45.3 / 46.7 -> 45.8, 4 16 1024 64 16.7 -> 16.4; masked 4 16
     // 1024 64 31.2 -> 30.5.  Past the caches as well under a window up to head dim 64 where the
     // workgroups do not fit the chip at once (42.7 -> 41.4 / 45.5 -> 45.2; 1 8/2 852 64 window 104 7.7 -> 7.8); elsewhere that is
-    // slower (causal 2 32/8 1501 128 45.2 -> 47.4).  Not where rows run over a group's heads, nor beside a bias at head dim 128, where two
-    // workgroups a CU would not fit.
-    constexpr bool QLDS = DIRECT && !PACKED && !(BIAS && DP == 128);
+    // slower (causal 2 32/8 1501 128 45.2 -> 47.4).  Not where rows run over a group's heads, nor up to head dim 32, whose rows are half
+    // a line (2 32 3000 32 window 500 26.9 -> 27.3), nor beside a bias at head dim 128, where two workgroups a CU would not fit, or up to
+    // 64 (QROWS) where a third one would be there: masked 9 16 1261 x 309 64 39.5 -> 42.0, 6 16 900 x 200 15.7 -> 16.7.
+    constexpr bool QLDS = DIRECT && !PACKED && !(BIAS && DP == 128) && (DP > 32 || MODE == kMaskPadding) && QROWS;
     constexpr int kQAt = 3 * Cfg::STAGE_BYTES;
     static_assert(!QLDS || KT * 2 == TROWS, "half of the query rows fit a stage");
     constexpr int kTilesLds = QLDS ? (5 * Cfg::STAGE_BYTES > 4 * Cfg::REGION ? 5 * Cfg::STAGE_BYTES : 4 * Cfg::REGION) : DIRECT ? Cfg::LDS_BYTES_DIRECT : Cfg::LDS_BYTES;  // BIAS: the four waves' bias values behind the tiles
@@ -1392,7 +1392,8 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             if (rr < rows_total && 8 * ch < D) {
                 uint16_t* dst = p.out + (size_t)b * p.lo.batch_stride + (size_t)(h0 + gg) * p.lo.head_stride +
                                 (size_t)sp * p.lo.row_pitch + 8 * ch;
-                store_past(dst, val);
+                if constexpr (WIN && DP > 128) *(u32x4_t*)dst = val;  // (4 40/8 2653 256 window 476: 425 us, past the caches 437)
+                else store_past(dst, val);
             }
         }
     }
@@ -1966,9 +1967,9 @@ __global__ __launch_bounds__(256, 2) void flash_wide_bf16_kernel(FlashTileParams
     }
 }
 
-template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs, bool HALVES = false>
+template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs, bool HALVES = false, bool QROWS = true>
 hipError_t launch_one(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
-    hipLaunchKernelGGL((flash_tile_bf16_kernel<DP, MODE, BIAS, PACKED, SPLIT, WIN, TILES, HALVES>), grid, dim3(HALVES ? 512 : TileCfg<DP>::THREADS), 0, stream, p);
+    hipLaunchKernelGGL((flash_tile_bf16_kernel<DP, MODE, BIAS, PACKED, SPLIT, WIN, TILES, HALVES, QROWS>), grid, dim3(HALVES ? 512 : TileCfg<DP>::THREADS), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -1985,7 +1986,11 @@ hipError_t launch_tiles(hipStream_t stream, const FlashTileParams& p, dim3 grid)
     }
     if (p.pack > 1 || p.decode_rows) return launch_one<DP, kMaskCausal, false, true, false, false, TILES>(stream, p, grid);
     if (p.window > 0) return launch_one<DP, kMaskCausal, false, false, false, true, TILES>(stream, p, grid);
-    if (p.bias) return launch_one<DP, kMaskNone, true, false, false, false, TILES>(stream, p, grid);
+    if (p.bias) {
+        if (DP == 64 && (unsigned long long)grid.x * grid.y * grid.z > 2ull * (unsigned long long)p.n_cus)
+            return launch_one<DP, kMaskNone, true, false, false, false, TILES, false, DP != 64>(stream, p, grid);
+        return launch_one<DP, kMaskNone, true, false, false, false, TILES>(stream, p, grid);
+    }
     if (p.mask == kMaskNone) return launch_one<DP, kMaskNone, false, false, false, false, TILES>(stream, p, grid);
     if (p.mask == kMaskCausal) return launch_one<DP, kMaskCausal, false, false, false, false, TILES>(stream, p, grid);
     return hipErrorInvalidValue;
