@@ -148,3 +148,14 @@ def test_prepare_then_decode_matches_cpu_decode_step(oracle):
     want = oracle.gqa_decode_batched_bf16(want_q, want_kc, want_vc, positions + 1, b_, hq, hkv, d, lmax)
     got = oracle.bf16_to_f32(dout.download(np.uint16))
     assert_decode_parity(got, want, d)
+
+
+@pytest.mark.parametrize("d,seq", [(128, 2731), (128, 2730), (64, 5461), (64, 5462)])
+def test_prompt_either_side_of_the_rows_that_fit_the_caches(oracle, d, seq):
+    """32 MiB of rows written is where the stores change: 32 query heads and twice 8 key heads, just below and just above."""
+    hq, hkv = 32, 8
+    assert (2 * seq * d * (hq + 2 * hkv) > 32 << 20) == (seq in (2731, 5462))
+    rng = np.random.default_rng(seq)
+    positions = np.array([1], np.int32)
+    rope, oro, q, k, v, kc, vc, qg, kg = _case(oracle, rng, 1, hq, hkv, d, seq + 2, positions, (True, True), seq=seq)
+    _run(oracle, rope, oro, q, k, v, kc, vc, qg, kg, positions, 1, hq, hkv, d, seq + 2, 1e-6, seq=seq)

@@ -655,3 +655,19 @@ def test_padding_bits(oracle, force_kernel, n, d):
         assert np.isnan(flash_bf16(ra.AttentionShape.new(b, h, n, d), qb, kb, vb, ra.Mask.padding(first))).all()
         first[63] = True
         assert np.isfinite(flash_bf16(ra.AttentionShape.new(b, h, n, d), qb, kb, vb, ra.Mask.padding(first))).all()
+
+
+@pytest.mark.parametrize("b,tq,tkv", [(16, 129, 70), (17, 129, 70), (17, 256, 128), (17, 130, 1)])
+def test_bias_either_side_of_two_workgroups_a_cu(oracle, b, tq, tkv):
+    """Beside a bias at head dim 64, launches of more than two workgroups a CU (512 of 128 query rows) read their rows into the
+    operands, the others through LDS; a last workgroup of one row, and of all."""
+    h, d = 16, 64
+    rng = np.random.default_rng(b + tq)
+    bits, f = zip(*inputs((b * tq * h * d,), (b * tkv * h * d,)))
+    bias = rng.standard_normal((tq, tkv)).astype(np.float32)
+    dq, dk, dv, db = (dev(x) for x in (*bits, bias))
+    out = ra.HipStorage.zeros(2 * b * tq * h * d)
+    ra.mha_forward_masked_bf16_dev(dq, dk, dv, out, b, tq, tkv, h, d, db, bias.size)
+    ra.synchronize()
+    want = oracle.mha_forward_masked(*f, b, tq, tkv, h, d, bias)
+    assert_bf16_parity(oracle.bf16_to_f32(out.download(np.uint16)), want, d, None, f"b={b} tq={tq} tkv={tkv}")
