@@ -22,6 +22,7 @@
 // product is a B operand of the second under a fixed permutation of the contraction slots, which the V operand
 // read applies as well).  LDS rows are padded, or their 16-byte slots XORed with bits of the row, so that the 16-byte K
 // reads and the transposing V reads are free of bank conflicts.
+#include "flash_tile_lds.hpp"
 #include "rt_common.hpp"
 #include "rt_kernels.hpp"
 
@@ -75,7 +76,7 @@ __device__ __forceinline__ float t_max16(const f32x16_t& s) {
 
 template <int DP>
 struct TileCfg {
-    static constexpr int KT = DP <= 128 ? 64 : 32;  // keys per LDS tile
+    static constexpr int KT = TileLds<DP>::KT;  // keys per LDS tile
     static constexpr int NI = KT / 32;              // 32-key items per tile
     static constexpr int THREADS = 256;
     static constexpr int LDK = DP + 8;                        // +16 B: 16 rows x 16 B tile all 64 banks
@@ -87,7 +88,7 @@ struct TileCfg {
     static constexpr int REGION = 32 * LDK * 2;                           // a wave's staged output rows
     static constexpr int LDS_BYTES = TILE_BYTES > 4 * REGION ? TILE_BYTES : 4 * REGION;
     // DIRECT: unpadded tiles (rows of DP * 2 bytes, 16-byte slots swizzled), filled by loads that go straight to LDS
-    static constexpr int STAGE_BYTES = KT * DP * 2;
+    static constexpr int STAGE_BYTES = TileLds<DP>::STAGE_BYTES;
     static constexpr int LDS_BYTES_DIRECT = 4 * STAGE_BYTES > 4 * REGION ? 4 * STAGE_BYTES : 4 * REGION;
     static constexpr int OCC_DIRECT = DP <= 64 ? 3 : 2;
     static constexpr int BIAS_BYTES = 32 * 32 * 4;  // a wave's bias values of an item: 32 rows of 32 keys
@@ -226,7 +227,6 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     // a line (2 32 3000 32 window 500 26.9 -> 27.3), nor beside a bias at head dim 128, where two workgroups a CU would not fit, or up to
     // 64 (QROWS) where a third one would be there: masked 9 16 1261 x 309 64 39.5 -> 42.0, 6 16 900 x 200 15.7 -> 16.7.
     constexpr bool QLDS = DIRECT && !PACKED && !(BIAS && DP == 128) && (DP > 32 || MODE == kMaskPadding) && QROWS;
-    constexpr int kQAt = 3 * Cfg::STAGE_BYTES;
     static_assert(!QLDS || KT * 2 == TROWS, "half of the query rows fit a stage");
     constexpr int kTilesLds = QLDS ? (5 * Cfg::STAGE_BYTES > 4 * Cfg::REGION ? 5 * Cfg::STAGE_BYTES : 4 * Cfg::REGION) : DIRECT ? Cfg::LDS_BYTES_DIRECT : Cfg::LDS_BYTES;  // BIAS: the four waves' bias values behind the tiles
     constexpr int kHalves = HALVES ? 2 : 1, kBiasAt = kHalves * ((kTilesLds + 1023) / 1024 * 1024);
@@ -234,8 +234,8 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     __shared__ alignas(DIRECT || BIAS ? 1024 : 16) unsigned char lds[BIAS ? kBiasAt + kHalves * 4 * Cfg::BIAS_BYTES : kHalves * kTilesLds];
     uint16_t* const Ks = (uint16_t*)lds;                      // [2][KT * LDK]
     uint16_t* const Vs = (uint16_t*)lds + 2 * KT * LDK;       // [2][KT * LDV]
-    // DIRECT: [K stage 0][K stage 1][V stage 0][V stage 1], rows of ROWB bytes without padding
-    constexpr int ROWB = DP * 2, STAGE_B = Cfg::STAGE_BYTES;
+    using Lds = TileLds<DP>;  // DIRECT
+    constexpr int ROWB = Lds::ROW_BYTES, STAGE_B = Lds::STAGE_BYTES;
 
     const int tid = HALVES ? threadIdx.x & 255 : threadIdx.x;  // within the half
     const int lane = tid & 63;
@@ -305,18 +305,9 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         ld_off[n] = ((uint32_t)row * kv_pitch + (ld_on[n] ? (uint32_t)(8 * ch) : 0u)) * 2u;
     }
     u32x4_t k1[NL];
-    // DIRECT: a wave's load instruction fills 1 KB of LDS with 64 chunks of 16 bytes, lane l the 16 bytes at 16 l;
-    // instruction n of wave w fills block w + 4 n of a stage: chunk 64 (w + 4 n) + l, which is slot chunk % SPR of row
-    // chunk / SPR.  Bank conflicts are avoided by an XOR of the slot index with bits of the row (K rows are read 16 at a
-    // time at one slot, V rows 4 at a time over 4 adjacent slots by the transposing reads; four rows of 64 or of 192 bytes
-    // start at four different quarters of the banks, which is all that V asks for), applied on the way in: the lane fetches
-    // the slot that belongs at its LDS position.  Slots behind the head dim are not requested: they are zero from the start.
-    constexpr int SPR = DP / 8;                // 16-byte slots per row
-    constexpr int NLD = KT * SPR / 256;        // load instructions per wave, matrix and tile
-    auto swz_k = [](int r) __attribute__((always_inline)) {
-        return DP == 128 ? (r & 15) : (DP == 64 ? ((r >> 1) & 7) : ((r >> 2) & 3));
-    };
-    auto swz_v = [](int r) __attribute__((always_inline)) { return DP == 128 ? 4 * (r & 3) : (DP == 64 ? 4 * ((r >> 1) & 1) : 0); };
+    // DIRECT: which chunk of a tile each lane of a load instruction fetches, and where it lands (flash_tile_lds.hpp).  Slots
+    // behind the head dim are not requested.
+    constexpr int SPR = Lds::SPR, NLD = Lds::REQUESTS;
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
     int dl_row[NLD];                            // row of the lane's chunk of instruction n,
     uint32_t dl_k[NLD], dl_v[NLD];              // its byte offsets from a tile's first row in K and in V,
@@ -325,7 +316,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     for (int n = 0; n < NLD; n++) {
         const int c = 64 * (wave + 4 * n) + lane, row = (int)((uint32_t)c / SPR), slot = c - row * SPR;
         dl_row[n] = row;
-        const int sk = slot ^ swz_k(row), sv = slot ^ swz_v(row);
+        const int sk = slot ^ Lds::swz_k(row), sv = slot ^ Lds::swz_v(row);
         dl_k[n] = (uint32_t)row * kv_pitch * 2u + (uint32_t)(16 * sk);
         dl_v[n] = (uint32_t)row * kv_pitch * 2u + (uint32_t)(16 * sv);
         dl_k_on[n] = __ballot(8 * sk < D);
@@ -340,20 +331,17 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     if constexpr (DIRECT && !WHOLE) {
 #pragma unroll
         for (int n = 0; n < NLD; n++) {
-            unsigned char* const at = lds + half_at + (wave + 4 * n) * 1024 + 16 * lane;
-            const bool k_on = (dl_k_on[n] >> lane) & 1, v_on = (dl_v_on[n] >> lane) & 1;
+            unsigned char* const at = lds + half_at + Lds::block(wave, n) + 16 * lane;
 #pragma unroll
-            for (int st = 0; st < 2; st++) {
-                if (!k_on) *(u32x4_t*)(at + st * STAGE_B) = u32x4_t{0u, 0u, 0u, 0u};
-                if (!v_on) *(u32x4_t*)(at + (2 + st) * STAGE_B) = u32x4_t{0u, 0u, 0u, 0u};
-            }
+            for (int st = 0; st < Lds::CLEARED; st++)
+                if (!(((st < 2 ? dl_k_on : dl_v_on)[n] >> lane) & 1)) *(u32x4_t*)(at + st * STAGE_B) = u32x4_t{0u, 0u, 0u, 0u};
         }
     }
     // the tile whose first row lies tile_off bytes into the descriptor -> the stage at stage_off
     auto dl_tile = [&](const u32x4_t& rs, const uint32_t (&lane_off)[NLD], const uint64_t (&on)[NLD], uint32_t tile_off, uint32_t stage_off) __attribute__((always_inline)) {
 #pragma unroll
         for (int n = 0; n < NLD; n++) {
-            const uint32_t block = lds_base + half_at + stage_off + (uint32_t)((wave + 4 * n) * 1024);
+            const uint32_t block = lds_base + half_at + stage_off + (uint32_t)Lds::block(wave, n);
             const uint32_t lane_at = DP == 96 ? lane_off[n] : lane_off[0];
             const uint32_t off = DP == 96 ? tile_off : tile_off + (uint32_t)(256 / SPR * n) * kv_pitch * 2u;
             if constexpr (WHOLE) buffer_to_lds(rs, lane_at, off, block);
@@ -562,7 +550,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         // the word of its next item a step ahead
         constexpr bool KEEP_BITS = MODE == kMaskPadding && DIRECT;
         static_assert(!KEEP_BITS || QLDS, "the bits take the query rows' place");
-        constexpr int kKeepAt = 4 * Cfg::STAGE_BYTES;
+        constexpr int kKeepAt = Lds::KEEP_AT;
         uint32_t keep_word_next = ~0u;
         uint64_t keep_cur = ~0ull, keep_next = ~0ull;  // keep bits of the tile whose items are in their softmax step, and of the next
         auto park_v = [&](auto set_c, int st) __attribute__((always_inline)) {
@@ -673,10 +661,10 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             const u32x4_t Qd = make_rsrc(p.q + (size_t)b * p.lq.batch_stride + (size_t)h0 * p.lq.head_stride + (size_t)min(r_first, rows_total - 1) * q_pitch,
                                          n_rows > 0 ? ((uint32_t)(n_rows - 1) * q_pitch + (uint32_t)D) * 2u : 0u);
 #pragma unroll
-            for (int n = 0; n < CH / 2; n++) {
-                const int c = 64 * n + lane, row = (int)((uint32_t)c / CH), slot = (c - row * CH) ^ swz_k(row);
+            for (int n = 0; n < Lds::Q_REQUESTS; n++) {
+                const int c = 64 * n + lane, row = (int)((uint32_t)c / CH), slot = (c - row * CH) ^ Lds::swz_k(row);
                 const uint32_t at = 8 * slot < D ? (uint32_t)row * q_pitch * 2u + 16u * (uint32_t)slot : 0x7fffffffu;
-                const uint32_t block = lds_base + half_at + (uint32_t)(kQAt + wave * 32 * ROWB + 1024 * n);
+                const uint32_t block = lds_base + half_at + (uint32_t)Lds::q_block(wave, n);
                 if (WIN && DP <= 64 && many) buffer_to_lds_past(Qd, at, 0u, block);
                 else buffer_to_lds(Qd, at, 0u, block);
             }
@@ -709,9 +697,9 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         uint32_t k_base = 0, k_base1 = 0, v_base = 0;
         if constexpr (DIRECT) {
             const int j = lane & 15, g16 = (lane >> 4) & 1, vrow = (j >> 2) + 4 * hh, low = 2 * g16 + ((j & 3) >> 1);
-            k_base = half_at + (uint32_t)(col * ROWB + ((hh ^ swz_k(col)) * 16));
-            if constexpr (DP == 96) k_base1 = half_at + (uint32_t)(col * ROWB + (((2 + hh) ^ swz_k(col)) * 16));
-            v_base = half_at + (uint32_t)(2 * STAGE_B + vrow * ROWB + ((low ^ swz_v(vrow)) * 16) + 8 * (j & 1));
+            k_base = half_at + (uint32_t)(col * ROWB + ((hh ^ Lds::swz_k(col)) * 16));
+            if constexpr (DP == 96) k_base1 = half_at + (uint32_t)(col * ROWB + (((2 + hh) ^ Lds::swz_k(col)) * 16));
+            v_base = half_at + (uint32_t)(Lds::V_AT + vrow * ROWB + ((low ^ Lds::swz_v(vrow)) * 16) + 8 * (j & 1));
         }
         // where the operands of item `item` of stage `st` start: with the lane's own offset (padded layout), or without
         // it (DIRECT: load_op adds the lane's swizzled offset)
@@ -758,14 +746,14 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             if constexpr (QLDS) {
 #pragma unroll
                 for (int ks = 0; ks < KS; ks++) {
-                    const unsigned char* const at = lds + kQAt + wave * 32 * ROWB;
+                    const unsigned char* const at = lds + Lds::q_block(wave, 0);
                     qreg[ks] = *(const bf16x8_t*)(at + (DP == 96 ? ((ks & 1) ? k_base1 : k_base) + (uint32_t)(64 * (ks >> 1)) : k_base ^ (uint32_t)(32 * ks)));
                 }
             }
             if (n_keys < KT) {
 #pragma unroll
                 for (int n = 0; n < NLD; n++)
-                    if (dl_row[n] >= n_keys) *(u32x4_t*)(lds + half_at + 2 * STAGE_B + (wave + 4 * n) * 1024 + 16 * lane) = u32x4_t{0u, 0u, 0u, 0u};
+                    if (dl_row[n] >= n_keys) *(u32x4_t*)(lds + half_at + Lds::V_AT + Lds::block(wave, n) + 16 * lane) = u32x4_t{0u, 0u, 0u, 0u};
             }
             bias_first();
             if constexpr (KEEP_BITS) {

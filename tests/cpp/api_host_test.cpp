@@ -11,6 +11,7 @@
 #include <functional>
 
 #include "../../include/rt_attn.h"
+#include "../../rustorch_amd/csrc/flash_tile_lds.hpp"
 #include "../../rustorch_amd/csrc/rt_kernels.hpp"
 
 static int g_failed = 0;
@@ -317,6 +318,40 @@ static void the_prefill_plan_deals_as_the_kernel_does() {
     CHECK(ranked > 0);
 }
 
+// bf16 tile kernel, tiles straight to LDS: ahead of its first barrier no 16 bytes of LDS are written by two waves, nor twice by
+// one (a request's arrival has no order with a wave's own clearing), and a wave's query rows are its own requests' alone.
+template <int DP>
+static void one_writer(int dim) {
+    using L = rt::TileLds<DP>;
+    std::vector<int> writer(5 * L::STAGE_BYTES / 16, -1);
+    auto write = [&](int at, int wave) {
+        CHECK(at % 16 == 0 && at + 16 <= 5 * L::STAGE_BYTES && writer[(size_t)at / 16] == -1);
+        writer[(size_t)at / 16] = wave;
+    };
+    for (int wave = 0; wave < 4; wave++)
+        for (int lane = 0; lane < 64; lane++) {
+            for (int n = 0; n < L::REQUESTS; n++) {
+                const int at = L::block(wave, n) + 16 * lane, row = at / L::ROW_BYTES, slot = at / 16 % L::SPR;
+                CHECK(row < L::KT);
+                for (int stage = 0; stage < 4; stage++) {  // K(0), K(1) and V(0) are requested, V(1) behind the barrier
+                    const bool inside = 8 * (slot ^ (stage < 2 ? L::swz_k(row) : L::swz_v(row))) < dim;
+                    if ((inside && stage < 3) || (!inside && stage < L::CLEARED)) write(stage * L::STAGE_BYTES + at, wave);
+                }
+            }
+            for (int n = 0; n < L::Q_REQUESTS; n++) write(L::q_block(wave, n) + 16 * lane, wave);
+        }
+    for (int at = 0; at < 2 * L::STAGE_BYTES; at += 16) CHECK(writer[(size_t)at / 16] >= 0);  // K: whole rows
+    for (int row = 0; row < 128; row++)
+        for (int slot = 0; slot < L::SPR; slot++) CHECK(writer[(size_t)(L::Q_AT / 16 + row * L::SPR + slot)] == row / 32);
+    CHECK(L::KEEP_AT == L::Q_AT + L::STAGE_BYTES && L::V_AT + L::STAGE_BYTES == L::Q_AT);
+}
+static void a_tiles_lds_has_one_writer() {
+    for (int dim = 8; dim <= 32; dim += 8) one_writer<32>(dim);
+    for (int dim = 40; dim <= 64; dim += 8) one_writer<64>(dim);
+    for (int dim = 72; dim <= 96; dim += 8) one_writer<96>(dim);
+    for (int dim = 104; dim <= 128; dim += 8) one_writer<128>(dim);
+}
+
 int main(int argc, char** argv) {
     fake::on_launch() = note_launch;
     const std::map<std::string, std::function<void()>> tests = {
@@ -325,6 +360,7 @@ int main(int argc, char** argv) {
         {"calls_on_the_per_thread_stream_take_turns", calls_on_the_per_thread_stream_take_turns},
         {"host_slices_follow_the_current_device", host_slices_follow_the_current_device},
         {"the_prefill_plan_deals_as_the_kernel_does", the_prefill_plan_deals_as_the_kernel_does},
+        {"a_tiles_lds_has_one_writer", a_tiles_lds_has_one_writer},
         {"no_thread_spins_through_the_kernel", no_thread_spins_through_the_kernel},
         {"a_host_without_threads_copies_by_itself", a_host_without_threads_copies_by_itself},
         {"a_host_without_memory_is_an_error", a_host_without_memory_is_an_error},
