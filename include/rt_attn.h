@@ -157,7 +157,8 @@ int rt_flash_backward_f32(const rt_attention_shape *shape, const float *q, size_
 
 /* flash_backward (cpu_backward.rs:46-185) on device-resident f32 tensors.  `workspace` is device memory of at least
  * rt_flash_backward_workspace_bytes(shape) bytes, 16-byte aligned (the recomputed forward output and two per-row
- * statistics); RT_ERR_WORKSPACE_TOO_SMALL otherwise.  Everything runs on `stream`. */
+ * statistics); RT_ERR_WORKSPACE_TOO_SMALL otherwise.  Everything runs on `stream`.  dk and dv may lie exactly over k and v
+ * (in either order); no other buffers of a call may share memory. */
 size_t rt_flash_backward_workspace_bytes(const rt_attention_shape *shape);
 int rt_flash_backward_f32_dev(void *stream, const rt_attention_shape *shape, const float *q, const float *k,
                               const float *v, const float *d_out, float *dq, float *dk, float *dv, void *workspace,
@@ -169,7 +170,8 @@ int rt_flash_backward_f32_dev(void *stream, const rt_attention_shape *shape, con
  * forward that also writes the row statistic lse[b,h,i] = m_i + ln(l_i) ([batch,heads,seq] f32), formed from the scores as
  * the gradients form them (the plain forward may run another kernel, and its output then differs in the last bits);
  * rt_flash_backward_saved_f32_dev takes that `out` and `lse` back and skips the recomputation.  `workspace`:
- * batch*heads*seq floats (RT_ERR_WORKSPACE_TOO_SMALL otherwise).  dim <= 512 (tuned up to 128). */
+ * batch*heads*seq floats (RT_ERR_WORKSPACE_TOO_SMALL otherwise).  One of the gradients may lie exactly over `out`, and dk and dv
+ * over k and v, as above.  dim <= 512 (tuned up to 128). */
 int rt_flash_forward_stats_f32_dev(void *stream, const rt_attention_shape *shape, const float *q, const float *k,
                                    const float *v, float *out, float *lse, rt_err_detail *err);
 int rt_flash_backward_saved_f32_dev(void *stream, const rt_attention_shape *shape, const float *q, const float *k,

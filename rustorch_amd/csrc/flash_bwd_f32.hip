@@ -635,7 +635,7 @@ hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Param
         if (flash_f32_takes_split(f, true)) return launch_flash_bwd_f32_split(stream, p);
     }
     dim3 grid((p.seq + kRows - 1) / kRows, p.heads, p.batch), block(256);
-    const bool both = p.vec && aligned(p.o) && bwd_f32_one_launch((long long)grid.x * grid.y * grid.z, p.dim <= 64 ? 2 : 1, p.n_cus);
+    const bool both = p.vec && aligned(p.o) && bwd_f32_one_launch((long long)grid.x * grid.y * grid.z, p.dim <= 64 ? 2 : 1, p.n_cus) && bwd_f32_apart(p);
     auto launch = [&](auto dt_c) {
         constexpr int kDT = decltype(dt_c)::value;
         if (both) {

@@ -704,7 +704,7 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_both_split
 
 hipError_t launch_flash_bwd_f32_split(hipStream_t stream, const FlashBwdF32Params& p) {
     dim3 grid((p.seq + 4 * kTile - 1) / (4 * kTile), p.heads, p.batch), block(256);
-    const bool both = bwd_f32_one_launch((long long)grid.x * grid.y * grid.z, p.dim <= 32 ? 2 : 1, p.n_cus);
+    const bool both = bwd_f32_one_launch((long long)grid.x * grid.y * grid.z, p.dim <= 32 ? 2 : 1, p.n_cus) && bwd_f32_apart(p);
     auto launch = [&](auto dt_c) {
         constexpr int kDT = decltype(dt_c)::value;
         if (both) {

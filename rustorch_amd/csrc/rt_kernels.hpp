@@ -81,9 +81,22 @@ hipError_t launch_flash_bwd_f32(hipStream_t stream, const FlashBwdF32Params& p, 
 // `delta` is B*H*N floats of scratch.  Runs dQ (which also leaves delta) and dK/dV.
 hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Params& p, const float* o, const float* lse,
                                       float* delta);
-// Its form on the bf16 matrix cores: p.o, p.lse and p.delta set, dim <= 64 and a multiple of 4, all tensors 16-byte aligned.
 // dQ and dK/dV of `blocks` workgroups each, `per_cu` of them on a CU: in one launch?
 bool bwd_f32_one_launch(long long blocks, int per_cu, int n_cus);
+// Do the gradients share no memory with what the kernels read, nor with each other?  Only then may dQ and dK/dV run side by side:
+// one behind the other, dQ may lie over O, and dK and dV over O, K and V, whose last reader is the workgroup that writes them.
+inline bool bwd_f32_apart(const FlashBwdF32Params& p) {
+    const size_t rows = (size_t)p.batch * p.heads * p.seq, n = rows * (size_t)p.dim;
+    const struct {
+        const float* at;
+        size_t n;
+    } x[9] = {{p.dq, n}, {p.dk, n}, {p.dv, n}, {p.q, n}, {p.k, n}, {p.v, n}, {p.d_out, n}, {p.o, n}, {p.lse, rows}};
+    for (int i = 0; i < 3; i++)
+        for (int j = i + 1; j < 9; j++)
+            if ((uintptr_t)x[i].at < (uintptr_t)(x[j].at + x[j].n) && (uintptr_t)x[j].at < (uintptr_t)(x[i].at + x[i].n)) return false;
+    return true;
+}
+// Its form on the bf16 matrix cores: p.o, p.lse and p.delta set, dim <= 64 and a multiple of 4, all tensors 16-byte aligned.
 hipError_t launch_flash_bwd_f32_split(hipStream_t stream, const FlashBwdF32Params& p);
 
 struct FlashBf16Params {

@@ -28,10 +28,17 @@ static std::mutex g_mutex;
 static std::vector<rt::DecodeSplitParams> g_decode;
 static std::vector<rt::FlashTileParams> g_tile;
 static int g_rows = 0;
+static bool g_f32_split = false;
+static std::vector<std::string> g_bwd;  // the gradients' kernels, as launched: "both", "dq", "dkdv"
 
 // the kernels of decode.hip, by their names
 static void note_launch(const std::string& name, dim3 grid, void** args, hipStream_t s) {
     if (name.find("attn_rows") != std::string::npos) g_rows++;
+    for (const char* k : {"both", "dq", "dkdv"})
+        if (name.find(std::string("flash_bwd_f32_") + k) != std::string::npos || name.find(std::string("flash_bwd_rows_") + k) != std::string::npos) {
+            fake::Inside here;
+            g_bwd.push_back(k);
+        }
     if (name.find("decode_latency") == std::string::npos && name.find("decode_split") == std::string::npos) return;
     fake::log("decode", s);
     std::lock_guard<std::mutex> lock(g_mutex);
@@ -45,7 +52,7 @@ hipError_t launch_flash_f32(hipStream_t s, const FlashF32Params& p) {
     for (size_t i = 0; i < n; i++) p.out[i] = p.q[i] + 2.0f * p.k[i] + 4.0f * p.v[i];
     return hipSuccess;
 }
-bool flash_f32_takes_split(const FlashF32Params&, bool) { return false; }
+bool flash_f32_takes_split(const FlashF32Params&, bool) { return g_f32_split; }
 hipError_t launch_flash_tile_bf16(hipStream_t s, const FlashTileParams& p) {
     fake::log("tile", s);
     fake::Inside here;
@@ -53,9 +60,6 @@ hipError_t launch_flash_tile_bf16(hipStream_t s, const FlashTileParams& p) {
     g_tile.push_back(p);
     return hipSuccess;
 }
-size_t flash_bwd_f32_workspace_floats(int, int, int, int) { return 64; }
-hipError_t launch_flash_bwd_f32(hipStream_t, const FlashBwdF32Params&, float*) { return hipSuccess; }
-hipError_t launch_flash_bwd_f32_saved(hipStream_t, const FlashBwdF32Params&, const float*, const float*, float*) { return hipSuccess; }
 bool flash_tile_bf16_supported(int dim) { return dim <= 256 && dim % 8 == 0; }
 int flash_tile_bf16_key_tile(int) { return 64; }
 int flash_tile_bf16_workgroups(int) { return 2; }
@@ -352,6 +356,37 @@ static void a_tiles_lds_has_one_writer() {
     for (int dim = 104; dim <= 128; dim += 8) one_writer<128>(dim);
 }
 
+// The gradients run side by side only where they share no memory with what either kernel reads, nor with each other.
+static void gradients_that_share_memory_take_turns() {
+    const std::vector<std::string> one = {"both"}, two = {"dq", "dkdv"};
+    for (bool split : {false, true})
+        for (int dim : {64, 32, 200}) {
+            g_f32_split = split;
+            const rt_attention_shape shape = {1, 8, 100, (uint64_t)dim};
+            const size_t rows = 800, n = rows * (size_t)dim;
+            std::vector<float> memory(9 * (n + 64));
+            float* x[9];  // q k v d_out o dq dk dv, and the row statistic
+            for (int i = 0; i < 9; i++) x[i] = (float*)(((uintptr_t)memory.data() + 63) / 64 * 64) + i * n;  // side by side
+            std::vector<float> ws(rows);
+            auto launched = [&](float* dq, float* dk, float* dv) {
+                g_bwd.clear();
+                CHECK(rt_flash_backward_saved_f32_dev(nullptr, &shape, x[0], x[1], x[2], x[4], x[8], x[3], dq, dk, dv, ws.data(),
+                                                      rows * sizeof(float), nullptr) == RT_OK);
+                return g_bwd;
+            };
+            CHECK(launched(x[5], x[6], x[7]) == (dim <= 128 ? one : two));
+            CHECK(launched(x[5], x[1], x[2]) == two);              // dk over k, dv over v
+            CHECK(launched(x[5], x[2], x[7]) == two);
+            CHECK(launched(x[4], x[6], x[7]) == two);              // dq over out, dk over out, dv over out
+            CHECK(launched(x[5], x[4], x[7]) == two);
+            CHECK(launched(x[5], x[6], x[4]) == two);
+            CHECK(launched(x[5], x[5], x[7]) == two);              // one buffer for two gradients
+            CHECK(launched(x[5], x[6], x[6] + n - 4) == two);      // the last four values
+            CHECK(launched(x[5], x[6], x[8] - n + 4) == two);      // the statistic's first
+        }
+    g_f32_split = false;
+}
+
 int main(int argc, char** argv) {
     fake::on_launch() = note_launch;
     const std::map<std::string, std::function<void()>> tests = {
@@ -361,6 +396,7 @@ int main(int argc, char** argv) {
         {"host_slices_follow_the_current_device", host_slices_follow_the_current_device},
         {"the_prefill_plan_deals_as_the_kernel_does", the_prefill_plan_deals_as_the_kernel_does},
         {"a_tiles_lds_has_one_writer", a_tiles_lds_has_one_writer},
+        {"gradients_that_share_memory_take_turns", gradients_that_share_memory_take_turns},
         {"no_thread_spins_through_the_kernel", no_thread_spins_through_the_kernel},
         {"a_host_without_threads_copies_by_itself", a_host_without_threads_copies_by_itself},
         {"a_host_without_memory_is_an_error", a_host_without_memory_is_an_error},

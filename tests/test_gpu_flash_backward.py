@@ -241,6 +241,31 @@ def test_gradients_in_one_launch(oracle, bhnd):
         assert max_abs(g, w) <= 1e-5 * max(1.0, float(np.abs(w).max())) * 4, name
 
 
+@pytest.mark.parametrize("over", ["dk k, dv v", "dk v, dv k", "dq out", "dk out", "dv out"])
+@pytest.mark.parametrize("bhnd", [(1, 8, 250, 100), (8, 16, 128, 64), (1, 2, 40, 320)])
+def test_gradients_over_tensors_their_owner_reads_last(bhnd, over):
+    """Sizes whose gradients run side by side where the tensors lie apart; here they may not."""
+    b, h, n, d = bhnd
+    shape = ra.AttentionShape.new(*bhnd)
+    bufs = [seeded_normal(shape.buffer_len(), s) for s in (71, 72, 73, 74)]
+    want = ra.flash_backward(shape, *bufs)
+    t = dict(zip(("q", "k", "v", "d_out"), [dev(x) for x in bufs]))
+    t["out"], lse = ra.HipStorage.zeros(shape.buffer_len() * 4), ra.HipStorage.zeros(b * h * n * 4)
+    ra.flash_forward_stats_f32_dev(shape, t["q"], t["k"], t["v"], t["out"], lse)
+    for name in ("dq", "dk", "dv"):
+        t[name] = ra.HipStorage.zeros(shape.buffer_len() * 4)
+    for pair in over.split(", "):
+        name, at = pair.split()
+        t[name] = t[at]
+    ws = ra.HipStorage.zeros(b * h * n * 4)
+    ra.flash_backward_saved_f32_dev(shape, t["q"], t["k"], t["v"], t["out"], lse, t["d_out"], t["dq"], t["dk"], t["dv"], ws,
+                                    ws.byte_len)
+    ra.synchronize()
+    for name, w in zip(("dq", "dk", "dv"), want):
+        # as test_backward_matches_oracle_on_normal_inputs: delta may be summed in another order
+        assert max_abs(t[name].download(np.float32), w) <= 1e-5 * max(1.0, float(np.abs(w).max())) * 4, name
+
+
 @pytest.mark.parametrize("what", ["key inf", "d_out nan", "d_out inf", "d_out small"])
 @pytest.mark.parametrize("bhnd", [(2, 16, 320, 64), (8, 16, 224, 32), (2, 8, 96, 64)])
 def test_gradients_in_one_launch_of_values_beyond_the_split(oracle, bhnd, what):
