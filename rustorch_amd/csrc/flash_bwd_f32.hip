@@ -298,7 +298,8 @@ __device__ __forceinline__ void bwd_f32_dkdv(const FlashBwdF32Params& p, int lin
     reduce_store<DPAD, LD, 2 * TILE>(lds, 0, p.dk + base, kv0, N, D, tid, vec);
 }
 
-template <int DT>
+// kLeaveDelta: for a dK/dV kernel that runs behind this one
+template <int DT, bool kLeaveDelta>
 __device__ __forceinline__ void bwd_f32_dq(const FlashBwdF32Params& p, int lin, int nt, float* lds) {
     constexpr int DPAD = 32 * DT;
     constexpr int LD = BwdTiles<DT>::LD, TILE = BwdTiles<DT>::TILE;
@@ -348,8 +349,8 @@ __device__ __forceinline__ void bwd_f32_dq(const FlashBwdF32Params& p, int lin, 
         }
     }
     // delta of the owner rows, dO_i . O_i: a lane adds up the half of row `col` it holds of dO, the other half sits
-    // in lane + 32.  Every wave of the workgroup needs all 32 values and computes them itself; wave 0 leaves them in
-    // memory for the dK/dV kernel.  (Rows beyond seq and columns beyond dim are staged as zeros.)
+    // in lane + 32.  Every wave of the workgroup needs all 32 values and computes them itself; kLeaveDelta: wave 0
+    // leaves them in memory for the dK/dV kernel.  (Rows beyond seq and columns beyond dim are staged as zeros.)
     if (vec) store_tile_regs<DPAD, LD>(Kt, r_o, lane);
     else stage_tile<DPAD, LD>(Kt, Og, q0, N, D, lane, false);
     float delta_q = 0.0f;
@@ -360,7 +361,7 @@ __device__ __forceinline__ void bwd_f32_dq(const FlashBwdF32Params& p, int lin, 
         for (int i = 0; i < 4; i++) delta_q = __builtin_fmaf(a[i], oreg[4 * j + i], delta_q);
     }
     delta_q += __shfl_xor(delta_q, 32, 64);
-    if (wave == 0 && hh == 0 && q_ok) p.delta[bh * (size_t)N + q0 + col] = delta_q;
+    if (kLeaveDelta && wave == 0 && hh == 0 && q_ok) p.delta[bh * (size_t)N + q0 + col] = delta_q;
     // have the statistic land here: a wait for it inside the loop would also wait for the tile prefetched there
     asm volatile("" : "+v"(lse_q), "+v"(delta_q));
 
@@ -440,7 +441,7 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dkdv_ker
 template <int DT>
 __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_dq_kernel(FlashBwdF32Params p) {
     __shared__ __attribute__((aligned(16))) float lds[BwdTiles<DT>::FLOATS];
-    bwd_f32_dq<DT>(p, linear_block(), (int)gridDim.x, lds);
+    bwd_f32_dq<DT, true>(p, linear_block(), (int)gridDim.x, lds);
 }
 // Both in one launch (bwd_f32_one_launch), dK/dV, the longer one, first: grid x holds the owner tiles of both.
 template <int DT>
@@ -449,7 +450,7 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_bwd_f32_both_ker
     __shared__ float stat[kNW][2][kRows];
     const int nt = (int)gridDim.x / 2, lin = linear_block(), n = nt * p.batch * p.heads;
     if (lin < n) bwd_f32_dkdv<DT, true>(p, lin, nt, lds, stat);
-    else bwd_f32_dq<DT>(p, lin - n, nt, lds);
+    else bwd_f32_dq<DT, false>(p, lin - n, nt, lds);
 }
 
 // ---- any head dim up to 512: one workgroup per row, any speed ------------------------------------------------------

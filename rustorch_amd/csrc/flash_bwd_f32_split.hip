@@ -215,7 +215,7 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
     out_in.clear();
     float st = 0.0f;  // threads 0..31: the row statistic, 32..63: delta.  Rows beyond seq: +inf, their weights are zeros
     const uint32_t piece = St::piece(D, tid);
-    const float* const st_src = tid < 32 ? lse : delta;
+    const float* const st_src = kOwnDelta || tid < 32 ? lse : delta;  // (kOwnDelta: the upper half's is not used)
     auto load = [&](int row0) RT_INLINE {
         q_in.load(Qg, row0, N, D, tid, piece);
         o_in.load(dOg, row0, N, D, tid, piece);
@@ -457,7 +457,8 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
     store_rows<DT>(p.dk + base, acc_dk, key, hh, N, D);
 }
 
-template <int DT>
+// kLeaveDelta: for a dK/dV kernel that runs behind this one
+template <int DT, bool kLeaveDelta>
 __device__ __forceinline__ void bwd_dq_split(const FlashBwdF32Params& p, int lin, int nt, __bf16* lds) {
     constexpr int DPAD = 32 * DT, KS = DPAD / 16;
     using St = Stream<DT>;
@@ -494,7 +495,7 @@ __device__ __forceinline__ void bwd_dq_split(const FlashBwdF32Params& p, int lin
         for (int i = 0; i < 8; i++) delta_q = __builtin_fmaf(y[i], x[i], delta_q);
     }
     delta_q += other_half(delta_q);
-    if (hh == 0 && q_ok) p.delta[(size_t)bh * N + q_row] = delta_q;
+    if (kLeaveDelta && hh == 0 && q_ok) p.delta[(size_t)bh * N + q_row] = delta_q;
     float lse_q = q_ok ? p.lse[(size_t)bh * N + q_row] : 0.0f;
     chk = split_max(split_max(chk, lse_q), delta_q);
     if (!q_ok) lse_q = -neg_inf();  // weights of zero
@@ -688,7 +689,7 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dkdv_split
 template <int DT>
 __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_dq_split_kernel(FlashBwdF32Params p) {
     __shared__ __attribute__((aligned(16))) __bf16 lds[kLdsHalfs<DT>];
-    bwd_dq_split<DT>(p, linear_block(), (int)gridDim.x, lds);
+    bwd_dq_split<DT, true>(p, linear_block(), (int)gridDim.x, lds);
 }
 // Both in one launch, dK/dV, the longer one, first: grid x holds the owner blocks of both.
 template <int DT>
@@ -697,7 +698,7 @@ __global__ __launch_bounds__(256, DT == 1 ? 2 : 1) void flash_bwd_f32_both_split
     __shared__ __attribute__((aligned(16))) float stat[2][2][kTile];
     const int nt = (int)gridDim.x / 2, lin = linear_block(), n = nt * p.batch * p.heads;
     if (lin < n) bwd_dkdv_split<DT, true>(p, lin, nt, lds, stat);
-    else bwd_dq_split<DT>(p, lin - n, nt, lds);
+    else bwd_dq_split<DT, false>(p, lin - n, nt, lds);
 }
 
 }  // namespace

@@ -70,7 +70,7 @@ struct FlashBwdF32Params {
     // filled by the launcher
     const float* o;
     const float* lse;
-    float* delta;  // written by the dQ kernel (its owner rows), read by the dK/dV kernel where that runs after it
+    float* delta;  // written by the dQ kernel (its owner rows) and read by the dK/dV kernel where that runs after it
     int vec;
 };
 // Floats of scratch launch_flash_bwd_f32 needs (O, the row statistic and delta).
@@ -78,7 +78,7 @@ size_t flash_bwd_f32_workspace_floats(int batch, int heads, int seq, int dim);
 // dim <= 128.  Runs the forward kernel, then dQ (which also leaves delta) and dK/dV on `stream`.
 hipError_t launch_flash_bwd_f32(hipStream_t stream, const FlashBwdF32Params& p, float* workspace);
 // The same from a saved forward: `o` [B,H,N,D] and `lse` [B,H,N] as launch_flash_f32 leaves them (FlashF32Params::lse);
-// `delta` is B*H*N floats of scratch.  Runs dQ (which also leaves delta) and dK/dV.
+// `delta` is B*H*N floats of scratch, used where they run one behind the other.  Runs dQ and dK/dV.
 hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Params& p, const float* o, const float* lse,
                                       float* delta);
 // dQ and dK/dV of `blocks` workgroups each, `per_cu` of them on a CU: in one launch?

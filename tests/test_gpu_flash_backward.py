@@ -241,6 +241,21 @@ def test_gradients_in_one_launch(oracle, bhnd):
         assert max_abs(g, w) <= 1e-5 * max(1.0, float(np.abs(w).max())) * 4, name
 
 
+@pytest.mark.parametrize("bhnd,used", [((1, 8, 250, 100), False), ((8, 16, 128, 64), False), ((8, 16, 129, 64), True)])
+def test_gradients_in_one_launch_share_no_scratch(bhnd, used):
+    b, h, n, d = bhnd
+    shape = ra.AttentionShape.new(*bhnd)
+    q, k, v, d_out = [dev(seeded_normal(shape.buffer_len(), s)) for s in (71, 72, 73, 74)]
+    out, lse, ws = (ra.HipStorage.zeros(x * 4) for x in (shape.buffer_len(), b * h * n, b * h * n))
+    grads = [ra.HipStorage.zeros(shape.buffer_len() * 4) for _ in range(3)]
+    ra.flash_forward_stats_f32_dev(shape, q, k, v, out, lse)
+    fill = np.full(b * h * n, 0x7fc12345, dtype=np.uint32)
+    ws.upload(fill)
+    ra.flash_backward_saved_f32_dev(shape, q, k, v, out, lse, d_out, *grads, ws, ws.byte_len)
+    ra.synchronize()
+    assert (ws.download(np.uint32) != fill).all() == used and (ws.download(np.uint32) != fill).any() == used
+
+
 @pytest.mark.parametrize("over", ["dk k, dv v", "dk v, dv k", "dq out", "dk out", "dv out"])
 @pytest.mark.parametrize("bhnd", [(1, 8, 250, 100), (8, 16, 128, 64), (1, 2, 40, 320)])
 def test_gradients_over_tensors_their_owner_reads_last(bhnd, over):
