@@ -38,24 +38,27 @@ constexpr int kNW = 4;  // waves per workgroup
 
 template <int DPAD>
 struct TileRegs;
-template <int DPAD>
+template <int DPAD, bool kRepeat = false>
 __device__ __forceinline__ void load_tile_regs(TileRegs<DPAD>& t, const float* __restrict__ src, int row0, int N, int D,
                                                int lane);
 template <int DPAD, int LD>
 __device__ __forceinline__ void store_tile_regs(float* dst, const TileRegs<DPAD>& t, int lane);
 
-// Copies rows [row0, row0 + 32) x [0, dim) of a [seq, dim] matrix into a 32 x LD LDS tile, zero beyond seq and dim.
-template <int DPAD, int LD>
+// Copies rows [row0, row0 + 32) x [0, dim) of a [seq, dim] matrix into a 32 x LD LDS tile, zero beyond dim and seq.  kRepeat: rows
+// beyond seq repeat the last one.  Query rows that meet a key do: their statistic gives them weights of zero where the last row
+// has a weight at all, but a row of zeros would make NaN of an infinite key.
+template <int DPAD, int LD, bool kRepeat = false>
 __device__ __forceinline__ void stage_tile(float* dst, const float* __restrict__ src, int row0, int N, int D, int lane,
                                            bool vec) {
     if (vec) {
         TileRegs<DPAD> t;
-        load_tile_regs<DPAD>(t, src, row0, N, D, lane);
+        load_tile_regs<DPAD, kRepeat>(t, src, row0, N, D, lane);
         store_tile_regs<DPAD, LD>(dst, t, lane);
     } else {
         for (int idx = lane; idx < kRows * DPAD; idx += kWave) {
             const int r = idx / DPAD, d = idx - r * DPAD;
-            dst[r * LD + d] = (row0 + r < N && d < D) ? src[(size_t)(row0 + r) * D + d] : 0.0f;
+            const int row = kRepeat ? min(row0 + r, N - 1) : row0 + r;
+            dst[r * LD + d] = (row < N && d < D) ? src[(size_t)row * D + d] : 0.0f;
         }
     }
 }
@@ -66,7 +69,7 @@ template <int DPAD>
 struct TileRegs {
     f32x4_t r[kRows * (DPAD / 4) / kWave];
 };
-template <int DPAD>
+template <int DPAD, bool kRepeat>
 __device__ __forceinline__ void load_tile_regs(TileRegs<DPAD>& t, const float* __restrict__ src, int row0, int N, int D,
                                                int lane) {
     constexpr int CH = DPAD / 4;
@@ -80,9 +83,9 @@ __device__ __forceinline__ void load_tile_regs(TileRegs<DPAD>& t, const float* _
     }
 #pragma unroll
     for (int n = 0; n < kRows * CH / kWave; n++) {
-        const int idx = kWave * n + lane, r = idx / CH, c = idx % CH;
+        const int idx = kWave * n + lane, c = idx % CH, row = kRepeat ? min(row0 + idx / CH, N - 1) : row0 + idx / CH;
         f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (row0 + r < N && 4 * c < D) z = *(const f32x4_t*)(src + (size_t)(row0 + r) * D + 4 * c);
+        if (row < N && 4 * c < D) z = *(const f32x4_t*)(src + (size_t)row * D + 4 * c);
         t.r[n] = z;
     }
 }
@@ -216,7 +219,7 @@ __device__ __forceinline__ void bwd_f32_dkdv(const FlashBwdF32Params& p, int lin
     };
     if (wave < n_qt) {
         if (vec) {
-            load_tile_regs<DPAD>(ra, Qg, wave * kRows, N, D, lane);
+            load_tile_regs<DPAD, true>(ra, Qg, wave * kRows, N, D, lane);
             if constexpr (kPrefetchBoth) load_tile_regs<DPAD>(rb, dOg, wave * kRows, N, D, lane);
         }
         load_stats(wave * kRows);
@@ -229,7 +232,7 @@ __device__ __forceinline__ void bwd_f32_dkdv(const FlashBwdF32Params& p, int lin
             if constexpr (kPrefetchBoth) store_tile_regs<DPAD, LD>(Ot, rb, lane);
             else stage_tile<DPAD, LD>(Ot, dOg, q0, N, D, lane, true);
         } else {
-            stage_tile<DPAD, LD>(Qt, Qg, q0, N, D, lane, false);
+            stage_tile<DPAD, LD, true>(Qt, Qg, q0, N, D, lane, false);
             stage_tile<DPAD, LD>(Ot, dOg, q0, N, D, lane, false);
         }
         if constexpr (kOwnDelta) {  // as the dQ kernel forms it
@@ -251,7 +254,7 @@ __device__ __forceinline__ void bwd_f32_dkdv(const FlashBwdF32Params& p, int lin
         }
         if (more) {
             if (vec) {
-                load_tile_regs<DPAD>(ra, Qg, q0 + kNW * kRows, N, D, lane);
+                load_tile_regs<DPAD, true>(ra, Qg, q0 + kNW * kRows, N, D, lane);
                 if constexpr (kPrefetchBoth) load_tile_regs<DPAD>(rb, dOg, q0 + kNW * kRows, N, D, lane);
             }
             load_stats(q0 + kNW * kRows);

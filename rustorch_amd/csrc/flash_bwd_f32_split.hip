@@ -405,7 +405,7 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
         Tile qt, ot;
         float st_f = 0.0f;
         auto load_f = [&](int q0) {
-            qt.load(Qg, (size_t)D, q0, N, D, tid);
+            qt.template load<true>(Qg, (size_t)D, q0, N, D, tid);
             ot.load(dOg, (size_t)D, q0, N, D, tid);
             if (tid < 64) {
                 const int row = q0 + (tid & 31);

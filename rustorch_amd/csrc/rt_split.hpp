@@ -132,16 +132,17 @@ constexpr float kSplitLeastResult = 0x1p-80f;
 // The larger magnitude; a NaN is not seen.
 __device__ __forceinline__ float split_max(float m, float x) { return __builtin_fmaxf(m, __builtin_fabsf(x)); }
 
-// A tile of 32 rows in f32 on its way through the 256 threads of a workgroup into LDS, zeros beyond the last row and D: for
-// the rows that are done once more.  16-byte loads; a row's start is 4 banks behind the one before it.
+// A tile of 32 rows in f32 on its way through the 256 threads of a workgroup into LDS, zeros beyond D and the last row (kRepeat:
+// copies of the last row, for query rows that meet a key that may be infinite): for the rows that are done once more.  16-byte loads; a row's start is 4 banks behind the one before it.
 template <int DT>
 struct F32Tile {
     static constexpr int CH = 8 * DT, LD = 32 * DT + 4, SIZE = 32 * LD;
     f32x4_t r[DT];
+    template <bool kRepeat = false>
     __device__ __forceinline__ void load(const float* __restrict__ src, size_t pitch, int row0, int N, int D, int tid) {
 #pragma unroll
         for (int n = 0; n < DT; n++) {
-            const int idx = 256 * n + tid, row = row0 + idx / CH, d = 4 * (idx % CH);
+            const int idx = 256 * n + tid, row = kRepeat ? min(row0 + idx / CH, N - 1) : row0 + idx / CH, d = 4 * (idx % CH);
             f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
             if (row < N && d < D) z = *(const f32x4_t*)(src + (size_t)row * pitch + d);
             r[n] = z;

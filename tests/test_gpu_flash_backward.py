@@ -311,3 +311,28 @@ def test_gradients_in_one_launch_of_values_beyond_the_split(oracle, bhnd, what):
         assert np.array_equal(np.isfinite(gs), fin), name
         if fin.any():  # the gradients' bound of the f32 kernels against 64 bits, twice: the oracle sums in f32 as well
             assert np.linalg.norm((gs - ws)[fin]) <= 4e-6 * np.linalg.norm(ws[fin]), name
+
+
+@pytest.mark.parametrize("bhnd", [
+    (2, 8, 90, 64), (1, 4, 70, 100), (1, 2, 45, 33), (40, 8, 33, 24),      # the f32 kernels: one launch, two, element by element
+    (2, 16, 310, 64), (8, 16, 210, 32), (8, 16, 129, 64), (1, 2, 35, 200),  # the split ones' second pass; a workgroup per row
+])
+def test_an_infinite_key_behind_a_short_last_tile(oracle, bhnd):
+    """A key that every query scores -inf weighs nothing: its rows of dK and dV are zeros, the others those of the keys without
+    it.  (dQ is NaN where it is infinite itself.)"""
+    b, h, n, d = bhnd
+    shape = ra.AttentionShape.new(*bhnd)
+    x = [seeded_normal(shape.buffer_len(), s).reshape(bhnd) for s in (71, 72, 73, 74)]
+    q, k, v, d_out = x
+    at = (b - 1, h - 1)
+    q[at][:, 9] = -np.abs(q[at][:, 9]) - np.float32(0.1)
+    k[at][n // 2, 9] = np.inf
+    got = [g.reshape(bhnd)[at].astype(np.float64) for g in ra.flash_backward(shape, *[a.ravel() for a in x])]
+    one = [np.ascontiguousarray(a[at]).ravel() for a in x]
+    want = [w.reshape(n, d).astype(np.float64) for w in oracle.flash_backward(oracle.AttentionShape(1, 1, n, d), *one)]
+    assert np.isfinite(want[1]).all() and np.isfinite(want[2]).all()
+    for name, g, w in zip(("dq", "dk", "dv"), got, want):
+        fin = np.isfinite(w)
+        assert np.array_equal(np.isfinite(g), fin), name
+        # as test_gradients_in_one_launch_of_values_beyond_the_split
+        assert np.linalg.norm((g - w)[fin]) <= 4e-6 * np.linalg.norm(w[fin]), name
