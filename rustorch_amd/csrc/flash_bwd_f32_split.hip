@@ -222,20 +222,23 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
         if constexpr (kOwnDelta) out_in.load(Og, row0, N, D, tid, piece);
         if (wave == 0) st = st_src[min(row0 + (tid & 31), N - 1)];
     };
+    auto put_delta = [&](int b, int row0) RT_INLINE {  // of the tile's rows of dO and O as they came; returns it
+        constexpr int LANES = DPAD / 8;  // of a row
+        float x = 0.0f, y = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            x = __builtin_fmaf(o_in.r[0][i], out_in.r[0][i], x);
+            y = __builtin_fmaf(o_in.r[1][i], out_in.r[1][i], y);
+        }
+        const int row = tid / LANES;
+        x = row0 + row < N ? lanes_sum<LANES>(x + y) : 0.0f;
+        if (tid % LANES == 0 && (St::ITEMS % 256 == 0 || tid < St::ITEMS)) stat[b][1][row] = x;
+        return x;
+    };
     // (the loaded value is looked at here and not where it is requested: there the wave would wait for it)
     auto put_stat = [&](int b, int row0) RT_INLINE {
         if constexpr (kOwnDelta) {
-            constexpr int LANES = DPAD / 8;  // of a row
-            float x = 0.0f, y = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                x = __builtin_fmaf(o_in.r[0][i], out_in.r[0][i], x);
-                y = __builtin_fmaf(o_in.r[1][i], out_in.r[1][i], y);
-            }
-            const int row = tid / LANES;
-            x = row0 + row < N ? lanes_sum<LANES>(x + y) : 0.0f;
-            chk = split_max(chk, x);
-            if (tid % LANES == 0 && (St::ITEMS % 256 == 0 || tid < St::ITEMS)) stat[b][1][row] = x;
+            chk = split_max(chk, put_delta(b, row0));
             if (tid < 32) {
                 const bool in = row0 + tid < N;
                 chk = split_max(chk, in ? st : 0.0f);
@@ -407,28 +410,23 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
         auto load_f = [&](int q0) {
             qt.template load<true>(Qg, (size_t)D, q0, N, D, tid);
             ot.load(dOg, (size_t)D, q0, N, D, tid);
-            if (tid < 64) {
+            if constexpr (kOwnDelta) {  // dO once more, as the sum over neighbouring lanes wants it (a row a lane: 409 us, B=1 H=8 N=2048 D=64; this 354)
+                o_in.load(dOg, q0, N, D, tid, piece);
+                out_in.load(Og, q0, N, D, tid, piece);
+            }
+            if (tid < (kOwnDelta ? 32 : 64)) {
                 const int row = q0 + (tid & 31);
-                st_f = tid < 32 ? -neg_inf() : 0.0f;
-                if (row < N) {
-                    if (!kOwnDelta || tid < 32) {
-                        st_f = (tid < 32 ? lse : delta)[row];
-                    } else {
-                        f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
-                        for (int d = 0; d < D; d += 4)
-                            sum += *(const f32x4_t*)(dOg + (size_t)row * D + d) * *(const f32x4_t*)(Og + (size_t)row * D + d);
-                        st_f = (sum[0] + sum[1]) + (sum[2] + sum[3]);
-                    }
-                }
+                st_f = row < N ? st_src[row] : (tid < 32 ? -neg_inf() : 0.0f);
             }
         };
-        auto store_f = [&](int b2) {
+        auto store_f = [&](int b2, int q0) {
             qt.store(f32_lds + b2 * 2 * Tile::SIZE, tid);
             ot.store(f32_lds + b2 * 2 * Tile::SIZE + Tile::SIZE, tid);
-            if (tid < 64) stat[b2][tid >> 5][tid & 31] = st_f;
+            if constexpr (kOwnDelta) put_delta(b2, q0);
+            if (tid < (kOwnDelta ? 32 : 64)) stat[b2][tid >> 5][tid & 31] = st_f;
         };
         load_f(0);
-        store_f(0);
+        store_f(0, 0);
         __syncthreads();
         for (int tile = 0; tile < n_tiles; tile++) {
             const float* qb = f32_lds + (tile & 1) * 2 * Tile::SIZE;
@@ -449,7 +447,7 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
             }
             f32_cols<DT>(acc_dv, ob, s, col, hh);
             f32_cols<DT>(acc_dk, qb, dp, col, hh);
-            if (tile + 1 < n_tiles) store_f((tile + 1) & 1);
+            if (tile + 1 < n_tiles) store_f((tile + 1) & 1, (tile + 1) * kTile);
             __syncthreads();
         }
     }

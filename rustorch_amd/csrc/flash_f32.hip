@@ -564,7 +564,9 @@ static bool flash_f32_takes_split_keys(const FlashF32Params& p) {
 // side in one launch (bwd_f32_one_launch) with 128 rows a workgroup, and with 32 would not.  us, forward + gradients, f32 / 128
 // rows, B H N at head dim 64: 8 8 256 18.0 + 43.0 / 17.7 + 29.8, 4 8 384 22.3 + 56.7 / 22.5 + 36.8, 2 8 640 32.2 + 86.3 / 32.6 + 51.7,
 // 8 16 100 11.3 + 26.6 / 11.9 + 18.9, 1 4 3000 127 + 368 / 129 + 209.  With 32 in one launch as well: 2 8 512 55 / 70, 1 8 1000
-// 99 / 125.  At head dim 32 the forward loses most of what the gradients gain (1 8 2048 50 + 138 / 75 + 109).
+// 99 / 125.  The forward alone is level to 0.6 us longer, and inputs that the split does not carry, which the f32 form takes as
+// they are, pay for its second pass: 2 8 640 32.3 + 85.7 / 82.2 + 114.4, 8 16 100 12.1 + 27.1 / 17.5 + 33.1.  At head dim 32 the
+// forward loses most of what the gradients gain (1 8 2048 50 + 138 / 75 + 109).
 static bool flash_f32_gradients_join(const FlashF32Params& p) {
     const long long n_bh = (long long)p.heads * p.batch;
     return p.mask == kMaskNone && p.dim > 32 && p.dim <= 64 && !bwd_f32_one_launch(n_bh * ((p.seq + 31) / 32), 2, p.n_cus) &&
