@@ -133,3 +133,23 @@ def test_window_errors():
     with pytest.raises(ra.DeviceError) as ei:
         ra.flash_forward_window_bf16_dev(shape, z.ptr + 2, z, z, z, 4)
     assert ei.value.status == 21
+
+
+@pytest.mark.parametrize("n,d", [(1537, 64), (769, 128), (1229, 80), (3073, 32), (400, 256)])
+def test_output_rows_either_side_of_the_caches(n, d):
+    """Two sequences write more than the 6 MiB from which on output rows go past the caches (up to head dim 128), either by itself
+    less: the same bits, every row written."""
+    b, h, window = 2, 16, 300
+    assert d > 128 or 2 * b * h * n * d > 6 << 20 >= 2 * h * n * d
+    bits = [bf16_round(seeded_normal((b, n, h, d), i))[0].reshape(b, -1) for i in range(3)]
+
+    def run(*x):
+        out = ra.HipStorage(2 * x[0].size)
+        out.upload(np.full(x[0].size, 0x7B7B, dtype=np.uint16))
+        ra.flash_forward_window_bf16_dev(ra.AttentionShape.new(x[0].shape[0], h, n, d), *[dev(a) for a in x], out, window, h, True)
+        ra.synchronize()
+        return out.download(np.uint16)
+
+    whole = run(*bits)
+    assert np.array_equal(whole, np.concatenate([run(*[a[i:i + 1] for a in bits]) for i in range(b)]))
+    assert not (whole == 0x7B7B).any()
