@@ -237,10 +237,14 @@ hipError_t launch_decode_prepare(hipStream_t stream, const DecodePrepareParams& 
                          aligned16(p.v_in) && aligned16(p.k_cache) && aligned16(p.v_cache) && aligned16(p.cos_table) &&
                          aligned16(p.sin_table) && aligned16(p.q_gamma) && aligned16(p.k_gamma) && p.n_heads + p.n_kv <= 65535;
     if (wide_ok) {
-        // past the caches where the rows written do not fit the L2s, 8 of 4 MB: us, plainly / past, 32 / 8 heads of 128: 1 x 70
-        // tokens 6.3 / 7.3, 1 x 2048 (25 MB) 13.4 / 14.0, 1 x 4096 (50 MB) 28.6 / 24.0, 2 x 3000 42.3 / 35.8; 4 x 8 of 256, 301 15.8 / 18.4
+        // past the caches from twice what the L2s hold, 8 of 4 MB.  us, plainly / past, inputs that change from pass to pass, 32 / 8
+        // heads of 128, caches as long as the prompt, caches of 8192 tokens: 1 x 70 tokens (0.8 MB) 6.3 / 7.3; 1 x 3000 (37 MB)
+        // 16.1 / 18.5, 16.1 / 18.3; 1 x 4096 (50 MB) 20.8 / 22.4, 21.0 / 22.6; 4 x 1024 (50 MB) 21.8 / 26.0, 29.4 / 26.2; 8 x 1024, head dim
+        // 64 (50 MB) 19.6 / 25.1, 24.1 / 25.4; 2 x 3000 (74 MB) 37.5 / 34.7, 37.4 / 34.4; 16 x 512 (101 MB) 50.9 / 45.3, 48.6 / 45.6; 4 x
+        // 4096 (201 MB) 91.2 / 79.5, 92.5 / 80.3.  Between the copies that bring the inputs and the attention that reads the rows it is
+        // level at every one of these sizes (4 x 4096 639.0 / 638.3, 16 x 512 137.0 / 136.8, 2 x 3000 210.0 / 211.7)
         const double written = 2.0 * p.batch * p.seq * (double)p.head_dim * (p.n_heads + 2.0 * p.n_kv);
-        const bool past = written > 32.0 * (1 << 20);
+        const bool past = written > 64.0 * (1 << 20);
         const dim3 grid((p.seq + 63) / 64, p.n_heads + p.n_kv, p.batch), block(256);
         if (p.head_dim <= 128) {
             if (past) hipLaunchKernelGGL((prompt_prepare_kernel<64, 128, true>), grid, block, 0, stream, p);

@@ -150,11 +150,12 @@ def test_prepare_then_decode_matches_cpu_decode_step(oracle):
     assert_decode_parity(got, want, d)
 
 
-@pytest.mark.parametrize("d,seq", [(128, 2731), (128, 2730), (64, 5461), (64, 5462)])
+@pytest.mark.parametrize("d,seq", [(128, 2731), (128, 2730), (64, 5461), (64, 5462), (128, 5462), (128, 5461), (64, 10922), (64, 10923)])
 def test_prompt_either_side_of_the_rows_that_fit_the_caches(oracle, d, seq):
-    """32 MiB of rows written is where the stores change: 32 query heads and twice 8 key heads, just below and just above."""
+    """64 MiB of rows written is where the stores change: 32 query heads and twice 8 key heads, just below and just above
+    (and around half of them)."""
     hq, hkv = 32, 8
-    assert (2 * seq * d * (hq + 2 * hkv) > 32 << 20) == (seq in (2731, 5462))
+    assert (2 * seq * d * (hq + 2 * hkv) > 64 << 20) == ((d, seq) in ((128, 5462), (64, 10923)))
     rng = np.random.default_rng(seq)
     positions = np.array([1], np.int32)
     rope, oro, q, k, v, kc, vc, qg, kg = _case(oracle, rng, 1, hq, hkv, d, seq + 2, positions, (True, True), seq=seq)
