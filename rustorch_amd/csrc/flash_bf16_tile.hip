@@ -2063,8 +2063,9 @@ hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
 }  // namespace
 
 bool flash_tile_bf16_supported(int dim) { return dim > 0 && dim <= 256 && dim % 8 == 0; }
-int flash_tile_bf16_key_tile(int dim) { return dim <= 128 ? 64 : 32; }
-int flash_tile_bf16_workgroups(int dim) { return dim <= 64 ? 3 : (dim <= 128 ? 2 : 1); }
+static_assert(flash_tile_bf16_key_tile(128) == TileCfg<128>::KT && flash_tile_bf16_key_tile(136) == TileCfg<256>::KT, "the host's rule of the key tile");
+static_assert(flash_tile_bf16_workgroups(64) == TileCfg<64>::OCC && flash_tile_bf16_workgroups(72) == TileCfg<96>::OCC && flash_tile_bf16_workgroups(136) == TileCfg<256>::OCC,
+              "the host's rule of the workgroups a CU");
 // The kernel addresses the keys of one (batch, kv head) with 32-bit byte offsets (tile offset + lane offset, the
 // requests that run a few tiles past the last one included).
 bool flash_tile_bf16_addressable(long long seq_kv, long long row_pitch) {

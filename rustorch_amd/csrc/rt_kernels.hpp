@@ -174,8 +174,8 @@ struct FlashTileParams {
 static_assert(offsetof(FlashTileParams, q) == 64 && offsetof(FlashTileParams, q_lens) == 128 && offsetof(FlashTileParams, keep) == 192, "lines of the arguments");
 bool flash_tile_bf16_supported(int dim);
 // keys per LDS tile of the tile kernel at head dim `dim` (the unit the split over the keys is cut in)
-int flash_tile_bf16_key_tile(int dim);
-int flash_tile_bf16_workgroups(int dim);  // that share a CU
+constexpr int flash_tile_bf16_key_tile(int dim) { return dim <= 128 ? 64 : 32; }
+constexpr int flash_tile_bf16_workgroups(int dim) { return dim <= 64 ? 3 : (dim <= 128 ? 2 : 1); }  // that share a CU
 hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& p);
 bool flash_tile_bf16_addressable(long long seq_kv, long long row_pitch);  // K/V slabs below 4 GiB (32-bit offsets)
 inline bool flash_tile_bf16_bias_addressable(long long seq_kv) { return seq_kv < (1ll << 24); }  // 32 rows of an additive bias likewise

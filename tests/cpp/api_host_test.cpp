@@ -61,8 +61,6 @@ hipError_t launch_flash_tile_bf16(hipStream_t s, const FlashTileParams& p) {
     return hipSuccess;
 }
 bool flash_tile_bf16_supported(int dim) { return dim <= 256 && dim % 8 == 0; }
-int flash_tile_bf16_key_tile(int) { return 64; }
-int flash_tile_bf16_workgroups(int) { return 2; }
 bool flash_tile_bf16_addressable(long long, long long) { return true; }
 bool flash_wide_bf16_supported(const FlashTileParams&) { return false; }
 hipError_t launch_flash_wide_bf16(hipStream_t, const FlashTileParams&) { return hipSuccess; }
@@ -356,6 +354,37 @@ static void a_tiles_lds_has_one_writer() {
     for (int dim = 104; dim <= 128; dim += 8) one_writer<128>(dim);
 }
 
+// How many spans a chunk's keys are cut into, of every case of tests/test_gpu_chunk_split.py and on either side of the rule's ends.
+static void a_chunks_keys_are_cut_as_its_tests_say() {
+    hipStream_t s;
+    CHECK(hipStreamCreate(&s) == hipSuccess);
+    auto spans = [&](int batch, int seq_new, int heads, int kv, int dim, int keys) {
+        g_tile.clear();
+        CHECK(rt_gqa_decode_chunk_bf16(s, g_buf, g_buf, g_buf, g_buf, (const int32_t*)g_buf, 0, batch, seq_new, heads, kv, dim, keys, nullptr) == RT_OK);
+        return g_tile.size() == 1 ? g_tile[0].n_splits : -1;
+    };
+    // test_spans_fold_to_the_whole
+    CHECK(spans(1, 1, 7, 1, 128, 1024) == 16);
+    CHECK(spans(1, 11, 6, 2, 128, 1500) == 24);
+    CHECK(spans(2, 43, 3, 1, 96, 700) == 11);
+    CHECK(spans(1, 31, 1, 1, 8, 4096) == 64);
+    CHECK(spans(1, 3, 64, 2, 200, 2000) == 21);
+    CHECK(spans(1, 100, 16, 2, 256, 2048) == 8);
+    // test_spans_of_a_tile: as many as tiles, but for two of them
+    CHECK(spans(1, 2, 16, 16, 64, 900) == 15);
+    CHECK(spans(1, 4, 8, 2, 64, 1473) == 24);
+    CHECK(spans(3, 4, 32, 8, 128, 200) <= 1);
+    CHECK(spans(1, 8, 16, 2, 256, 300) == 10);
+    CHECK(spans(2, 5, 12, 12, 80, 321) == 6);
+    CHECK(spans(4, 4, 16, 16, 64, 800) == 7);
+    CHECK(spans(3, 2, 8, 8, 64, 900) == 15);
+    CHECK(spans(2, 4, 16, 16, 64, 800) == 13);
+    CHECK(spans(1, 4, 32, 8, 128, 200) == 4);
+    // units that fill the chip, and fewer than four tiles, are not cut
+    CHECK(spans(16, 2, 16, 16, 64, 4096) <= 1 && spans(8, 2, 16, 16, 64, 4096) > 1);
+    CHECK(spans(1, 4, 32, 8, 128, 192) <= 1 && spans(1, 4, 32, 8, 128, 193) == 4);
+}
+
 // The gradients run side by side only where they share no memory with what either kernel reads, nor with each other.
 static void gradients_that_share_memory_take_turns() {
     const std::vector<std::string> one = {"both"}, two = {"dq", "dkdv"};
@@ -397,6 +426,7 @@ int main(int argc, char** argv) {
         {"the_prefill_plan_deals_as_the_kernel_does", the_prefill_plan_deals_as_the_kernel_does},
         {"a_tiles_lds_has_one_writer", a_tiles_lds_has_one_writer},
         {"gradients_that_share_memory_take_turns", gradients_that_share_memory_take_turns},
+        {"a_chunks_keys_are_cut_as_its_tests_say", a_chunks_keys_are_cut_as_its_tests_say},
         {"no_thread_spins_through_the_kernel", no_thread_spins_through_the_kernel},
         {"a_host_without_threads_copies_by_itself", a_host_without_threads_copies_by_itself},
         {"a_host_without_memory_is_an_error", a_host_without_memory_is_an_error},
