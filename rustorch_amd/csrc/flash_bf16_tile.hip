@@ -191,7 +191,7 @@ enum TileWay : int { kTilesRegs = 0, kTilesDirect = 1, kTilesDirectPart = 2 };
 // the split form's merge does.  For launches that leave a CU one workgroup: its waves, alone on their SIMDs, take 800
 // clocks an item at head dim 64 where three of them together take 500 each, and 2100 with a bias, whose latency one wave
 // does not hide.  (launch_halves has the figures.)
-template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs, bool HALVES = false, bool QROWS = true>
+template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs, bool HALVES = false, bool QROWS = true, bool PAST = false>
 __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : BIAS && DP == 64 ? 2 : (TILES ? TileCfg<DP>::OCC_DIRECT : TileCfg<DP>::OCC)) void flash_tile_bf16_kernel(FlashTileParams p) {
     static_assert(!SPLIT || (PACKED && !BIAS && MODE == kMaskCausal), "the split over the keys serves the chunked decode");
     static_assert(!WIN || (!PACKED && !BIAS && !SPLIT && MODE == kMaskCausal), "the window is a causal mask's");
@@ -455,17 +455,9 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         Kg += (size_t)half_key0 * (size_t)p.lkv.row_pitch;
         Vg += (size_t)half_key0 * (size_t)p.lkv.row_pitch;
     }
-    // Output rows past the caches or plainly, as out_goes_past has it (the empty statements keep the two kinds of store from being
-    // merged into one).  Above head dim 128 without the choice: plainly under a window (4 40/8 2653 256 window 476 425 us, past the caches 437),
-    // past the caches otherwise (1 8/2 1024 256 46.9 -> 46.7).
-    auto store_row = [&](uint16_t* dst, u32x4_t v) __attribute__((always_inline)) {
-        if (DP > 128 ? !WIN : p.out_past != 0) {
-            if (DP <= 128) asm volatile("");
-            store_past(dst, v);
-            if (DP <= 128) asm volatile("");
-        } else {
-            *(u32x4_t*)dst = v;
-        }
+    auto store_row = [&](uint16_t* dst, u32x4_t v) __attribute__((always_inline)) {  // PAST: past the caches (out_goes_past)
+        if constexpr (PAST) store_past(dst, v);
+        else *(u32x4_t*)dst = v;
     };
     // A tile of padded query rows only (a padded batch has many: every tile behind a sequence's last row) has nothing
     // to load or walk: its rows get the fill value and the workgroup is done.
@@ -1366,27 +1358,15 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         const size_t step = (size_t)RS * (size_t)p.lo.row_pitch;
         const uint16_t* src = obuf + row0 * LDK + 8 * ch;
         const bool col_ok = 8 * ch < D;
-        auto rows = [&](auto past_c) __attribute__((always_inline)) {
 #pragma unroll
-            for (int n = 0; n < CH / 2; n++) {
-                const int rr = rr0 + RS * n;
-                // no key tile walked: padded rows get the fill value, valid rows (which then see no key at all) NaN
-                const uint32_t f2 = rr < n_q ? 0x7fc07fc0u : fill2;
-                u32x4_t val = {f2, f2, f2, f2};
-                if (n_loop > 0) val = *(const u32x4_t*)(src + RS * n * LDK);
-                if (rr < rows_total && col_ok) {
-                    if constexpr (decltype(past_c)::value) store_past(dst, val);
-                    else *(u32x4_t*)dst = val;
-                }
-                dst += step;
-            }
-        };
-        if (p.out_past) {  // (a copy of the code for either: a branch a store cost small calls 2 to 4 %)
-            asm volatile("" ::: "memory");
-            rows(std::true_type{});
-            asm volatile("" ::: "memory");
-        } else {
-            rows(std::false_type{});
+        for (int n = 0; n < CH / 2; n++) {
+            const int rr = rr0 + RS * n;
+            // no key tile walked: padded rows get the fill value, valid rows (which then see no key at all) NaN
+            const uint32_t f2 = rr < n_q ? 0x7fc07fc0u : fill2;
+            u32x4_t val = {f2, f2, f2, f2};
+            if (n_loop > 0) val = *(const u32x4_t*)(src + RS * n * LDK);
+            if (rr < rows_total && col_ok) store_row(dst, val);
+            dst += step;
         }
     } else {
 #pragma unroll
@@ -1978,9 +1958,32 @@ __global__ __launch_bounds__(256, 2) void flash_wide_bf16_kernel(FlashTileParams
     }
 }
 
+// Output rows past the caches (store_past), up to head dim 128?  The call is never longer for it, but what it gains by not waiting
+// for the write-back the kernel that reads the rows next pays in part, or, where they would have stayed in the L2s for it, in
+// full and more.  us, plainly / past, the call, and it with a product of its rows and a [heads * dim, heads * dim] matrix behind it, by
+// MB written: 1 (1 16 512 64) 8.57 / 8.56, 25.2 / 25.2; 2 (1 32/8 256 128) 8.38 / 8.38, 30.5 / 31.4; 4 (masked 2 16 1024 64) 17.7 / 17.5, 29.6 /
+// 30.9, (window 300, 2 16 2000 32) 13.2 / 12.8, 24.0 / 25.3; 5 (window 256, 1 16 2500 64) 12.0 / 11.6, 24.6 / 25.9; 5.7 (2 16 700 80) 16.0 / 15.9,
+// 29.0 / 30.7; 6.5 (1 40/8 640 128) 14.9 / 14.4, 61.1 / 61.0; 8 (1 32/8 1024 128) 19.7 / 18.8, 59.1 / 58.7, (window 256, 2 16 2048 64) 13.2 / 12.6,
+// 27.7 / 27.9; 24 (2 32/8 1501 128) 45.3 / 44.5, 132.7 / 133.3; 32 (window 256, 4 16 4096 64) 41.0 / 39.2, 79.8 / 79.8, (padded, 16 16 1024 64)
+// 28.2 / 26.2, 82.4 / 81.9; 48 (2 32/8 3000 128) 148.9 / 145.5, 315.6 / 319.1.  From 6 MB on the call gains 1 to 8 % and the two together are level;
+// below, the two together lose up to 6 % for a call that gains up to 4.  Two kernels (PAST): where one chose by a branch around its
+// stores, 2 32/8 1501 128 took 45.9 for 45.6, small calls with a branch a store 2 to 4 % longer.  Above head dim 128 without the choice: plainly
+// under a window (4 40/8 2653 256 window 476 425 us, past the caches 437), past the caches otherwise (1 8/2 1024 256 46.9 -> 46.7).
+static bool out_goes_past(const FlashTileParams& p) {
+    const double written = 2.0 * p.batch * p.heads * (double)p.seq_q * p.dim;
+    return written > 6.0 * (1 << 20);
+}
+
 template <int DP, int MODE, bool BIAS, bool PACKED, bool SPLIT = false, bool WIN = false, int TILES = kTilesRegs, bool HALVES = false, bool QROWS = true>
 hipError_t launch_one(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
-    hipLaunchKernelGGL((flash_tile_bf16_kernel<DP, MODE, BIAS, PACKED, SPLIT, WIN, TILES, HALVES, QROWS>), grid, dim3(HALVES ? 512 : TileCfg<DP>::THREADS), 0, stream, p);
+    const dim3 block(HALVES ? 512 : TileCfg<DP>::THREADS);
+    if constexpr (DP > 128) {
+        hipLaunchKernelGGL((flash_tile_bf16_kernel<DP, MODE, BIAS, PACKED, SPLIT, WIN, TILES, HALVES, QROWS, !SPLIT && !WIN>), grid, block, 0, stream, p);
+    } else if (!SPLIT && out_goes_past(p)) {  // (a span leaves partials)
+        hipLaunchKernelGGL((flash_tile_bf16_kernel<DP, MODE, BIAS, PACKED, SPLIT, WIN, TILES, HALVES, QROWS, !SPLIT>), grid, block, 0, stream, p);
+    } else {
+        hipLaunchKernelGGL((flash_tile_bf16_kernel<DP, MODE, BIAS, PACKED, SPLIT, WIN, TILES, HALVES, QROWS, false>), grid, block, 0, stream, p);
+    }
     return hipGetLastError();
 }
 
@@ -2122,20 +2125,6 @@ static bool tiles_by_length(const FlashTileParams& p, long long n_qtiles) {
            n_qtiles * p.batch * p.heads > (long long)p.n_cus * flash_tile_bf16_workgroups(p.dim);
 }
 
-// Output rows past the caches (store_past), up to head dim 128?  The call is never longer for it, but what it gains by not waiting
-// for the write-back the kernel that reads the rows next pays in part, or, where they would have stayed in the L2s for it, in
-// full and more.  us, plainly / past, the call, and it with a product of its rows and a [heads * dim, heads * dim] matrix behind it, by
-// MB written: 1 (1 16 512 64) 8.57 / 8.56, 25.2 / 25.2; 2 (1 32/8 256 128) 8.38 / 8.38, 30.5 / 31.4; 4 (masked 2 16 1024 64) 17.7 / 17.5, 29.6 /
-// 30.9, (window 300, 2 16 2000 32) 13.2 / 12.8, 24.0 / 25.3; 5 (window 256, 1 16 2500 64) 12.0 / 11.6, 24.6 / 25.9; 5.7 (2 16 700 80) 16.0 / 15.9,
-// 29.0 / 30.7; 6.5 (1 40/8 640 128) 14.9 / 14.4, 61.1 / 61.0; 8 (1 32/8 1024 128) 19.7 / 18.8, 59.1 / 58.7, (window 256, 2 16 2048 64) 13.2 / 12.6,
-// 27.7 / 27.9; 24 (2 32/8 1501 128) 45.3 / 44.5, 132.7 / 133.3; 32 (window 256, 4 16 4096 64) 41.0 / 39.2, 79.8 / 79.8, (padded, 16 16 1024 64)
-// 28.2 / 26.2, 82.4 / 81.9; 48 (2 32/8 3000 128) 148.9 / 145.5, 315.6 / 319.1.  From 6 MB on the call gains 1 to 8 % and the two together are level;
-// below, the two together lose up to 6 % for a call that gains up to 4.
-static bool out_goes_past(const FlashTileParams& p) {
-    const double written = 2.0 * p.batch * p.heads * (double)p.seq_q * p.dim;
-    return written > 6.0 * (1 << 20);
-}
-
 hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& params) {
     FlashTileParams p = params;
     if (p.batch == 0 || p.heads == 0 || p.seq_q == 0) return hipSuccess;
@@ -2153,7 +2142,6 @@ hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& par
     if (p.batch > 65535 || n_qtiles * p.n_splits > 65535 || heads_u > 65535 || p.group < 1) return hipErrorInvalidValue;  // grid limits
     set_grid_order(p, n_qtiles * p.n_splits);
     if (tiles_by_length(p, n_qtiles)) p.n_qtiles = -1;
-    p.out_past = out_goes_past(p);
     dim3 grid((unsigned)heads_u, (unsigned)p.batch, (unsigned)(n_qtiles * p.n_splits));
     if (p.dim <= 32) return launch_dp<32>(stream, p, grid);
     if (p.dim <= 64) return launch_dp<64>(stream, p, grid);

@@ -155,7 +155,6 @@ struct FlashTileParams {
     int n_splits;
     float* part_o;
     float* part_ml;
-    int out_past;             // set by the launcher: output rows go past the caches
     // ---- what only some forms read
     const uint8_t* keep;      // kMaskPadding: device, seq_kv bytes
     const float* bias;        // optional additive score bias, f32 rows of seq_kv per query position, added after scaling
@@ -171,7 +170,7 @@ struct FlashTileParams {
     int decode_rows;
     int n_cus;  // CUs of the device (0: unknown)
 };
-static_assert(offsetof(FlashTileParams, q) == 64 && offsetof(FlashTileParams, q_lens) == 128 && offsetof(FlashTileParams, keep) == 192, "lines of the arguments");
+static_assert(offsetof(FlashTileParams, q) == 64 && offsetof(FlashTileParams, q_lens) == 128, "lines of the arguments");
 bool flash_tile_bf16_supported(int dim);
 // keys per LDS tile of the tile kernel at head dim `dim` (the unit the split over the keys is cut in)
 constexpr int flash_tile_bf16_key_tile(int dim) { return dim <= 128 ? 64 : 32; }
