@@ -73,12 +73,24 @@ template <int DPAD, bool kRepeat>
 __device__ __forceinline__ void load_tile_regs(TileRegs<DPAD>& t, const float* __restrict__ src, int row0, int N, int D,
                                                int lane) {
     constexpr int CH = DPAD / 4;
-    if (D == DPAD && row0 + kRows <= N) {
+    if ((!kRepeat || DPAD == 128) && D == DPAD && row0 + kRows <= N) {
         // the whole tile is there and contiguous (row pitch == DPAD): one per-lane address, constant offsets, and no
         // per-load bounds test (a wave-uniform condition)
         const f32x4_t* base = (const f32x4_t*)(src + (size_t)row0 * DPAD) + lane;
 #pragma unroll
         for (int n = 0; n < kRows * CH / kWave; n++) t.r[n] = base[kWave * n];
+        return;
+    }
+    if (kRepeat && D == DPAD) {
+        // Every row is there: no test a load, 32-bit offsets.  Whole tiles as well, but at 128: us of the gradients' second kernel, this
+        // way for the short tile alone / for all, 3 x 8 heads of 96, N=1000 189 / 184; a training step of 2 x 8 of 128, 1250 680 / 687
+        const f32x4_t* base = (const f32x4_t*)(src + (size_t)row0 * DPAD);
+        const int last = N - 1 - row0;
+#pragma unroll
+        for (int n = 0; n < kRows * CH / kWave; n++) {
+            const int idx = kWave * n + lane;
+            t.r[n] = base[min(idx / CH, last) * CH + idx % CH];
+        }
         return;
     }
 #pragma unroll
