@@ -88,7 +88,7 @@ __device__ __forceinline__ u32x4_t make_rsrc(const void* base, uint32_t bytes) {
 // meanwhile have that much less room.  us, plainly -> past the caches, bf16: padded batch of 16 x 16 heads, N=1024 D=64 30.1 ->
 // 26.9; window 256, 4 x 16 heads, N=4096 D=64 45.9 -> 41.9; causal 2 x 32 / 8 heads, N=1501 D=128 46.8 -> 45.8.  (What the next
 // kernel pays for it, and from which size on it is worth it, stands at out_goes_past; the persistent kernel, which takes calls that
-// write 16 MB or more, stores this way always.)  For whole lines:
+// write 11 MB or more, stores this way always.)  For whole lines:
 // the f32 kernels' pieces of 32 bytes a row took longer that way (train, 4 x 16 heads, N=1024 D=64 411 -> 418).
 template <typename T>
 __device__ __forceinline__ void store_past(void* dst, T v) { __builtin_nontemporal_store(v, (T*)dst); }
