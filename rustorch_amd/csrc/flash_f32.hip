@@ -526,18 +526,31 @@ static bool flash_f32_split_pays(const FlashF32Params& p) {
 }
 
 // The same question between the two forms of the split products (flash_f32_split.hip: 128 query rows a workgroup, or 32 and
-// waves that share the keys), up to head dim 64 and for a forward without row statistic, in us beside the launch.  At head
+// waves that share the keys), for a forward without row statistic, in us beside the launch.  At head
 // dim 64 a tile step of 128 rows takes 1.41 us (1.45 causal, with what its rows of unequal length leave idle), one of the
 // four waves' 3.8 with two workgroups on a CU and 2.2 with one; causal 1.9 a step of the chip's mean and 2.3 for each
 // workgroup of a CU; at 32 0.87 and 1.05, causal 1.02 and 1.05 with 1.3 a workgroup.  us, 128 rows / shared keys, B H N at
 // head dim 64: 1 8 2048 94 / 69, causal 91 / 43; 8 8 256 17.0 / 14.5; 2 12 400 23 / 19; 1 12 1500 69 / 72; 5 12 300 20 / 25; 4 16 1024
 // 95 / 129, causal 63 / 85; causal 1 8 4096 173 / 128, 2 12 999 49 / 38, 4 16 512 29 / 32, 8 16 256 19 / 24; at 32: 8 16 300 24 / 21,
 // 4 16 1024 63 / 73, causal 1 8 4096 144 / 78, 2 16 2048 80 / 83.
+// Above head dim 64 one workgroup of either form fills a CU: a tile step of 128 rows takes 2.45 us (2.8 above 96), one of the
+// four waves' 3.6 (4.5), and a workgroup of them 4.5 (5.5) beside its steps; causal blocks of 128 rows go two to a workgroup
+// from one a CU on, those of 32 come near the chip's mean but for the longest.  us, f32 kernel / 128 rows / shared keys, B H N at head dim
+// 128: 1 8 2048 193 / 174 / 145; 2 8 1024 102 / 92 / 81; 4 8 400 57 / 44 / 48; 2 12 700 117 / 67 / 94; 1 8 161 17.4 / 24.6 / 16.6; causal
+// 1 8 3438 297 / 284 / 223; 1 12 1500 142 / 128 / 109; 1 16 2048 220 / 175 / 168; 2 16 1500 258 / 156 / 206; at 96: 1 8 1024 43.7 / 82.7 /
+// 35.8; 8 8 200 29.5 / 25.8 / 25.7; 1 16 2048 317 / 163 / 216; causal 2 12 999 96 / 85 / 70; 4 12 600 78 / 55 / 61.
 static bool flash_f32_rows_pay(const FlashF32Params& p) {
     const double n_cus = p.n_cus > 0 ? p.n_cus : 256;
     const long long keys = p.seq_kv ? p.seq_kv : p.seq;
     const double tiles = (double)((keys + 31) / 32), n_bh = (double)p.heads * p.batch, groups = n_bh * ((p.seq + 31) / 32);
     const double per_cu = n_bh * ((p.seq + 127) / 128) / n_cus, share = __builtin_ceil(tiles / 4);
+    if (p.dim > 64) {
+        const double row_step = p.dim > 96 ? 2.8 : 2.45, key_step = p.dim > 96 ? 4.5 : 3.6, own = p.dim > 96 ? 5.5 : 4.5;
+        if (p.mask == kMaskCausal)
+            return row_step * (per_cu > 1 ? __builtin_ceil(per_cu / 2) * (tiles + 4) : tiles) <
+                   __builtin_fmax(key_step * share, key_step * groups * (tiles + 1) / (8 * n_cus) + own * groups / n_cus);
+        return row_step * __builtin_ceil(per_cu) * tiles + 2 < __builtin_ceil(groups / n_cus) * (key_step * share + own) - own;
+    }
     if (p.mask == kMaskCausal) {
         const double rows = __builtin_fmax(tiles, 1.1 * per_cu * (tiles + 4) / 2), mean = groups * (tiles + 1) / (8 * n_cus);
         return p.dim > 32 ? 1.45 * rows < 1.9 * mean + 2.3 * groups / n_cus : 1.02 * rows + 2 < 1.05 * mean + 1.3 * groups / n_cus;
@@ -548,7 +561,8 @@ static bool flash_f32_rows_pay(const FlashF32Params& p) {
     return 1.41 * rows < share * (3.8 * full + (rest > n_cus ? 3.8 : (rest > 0 ? 2.2 : 0.0)));
 }
 
-// Keys from which the shared keys pay: with 128 a wave has one tile at most, and the f32 kernel is level (7.1 / 7.4 us).
+// Keys from which the shared keys pay: with 128 a wave has one tile at most, and the f32 kernel is level (7.1 / 7.4 us; at head dim
+// 128 11.9 / 12.5).
 // Unmasked up to head dim 32 it is level up to 256 (us, f32 kernel / shared keys, B H N: 1 8 256 6.9 / 6.8, 2 12 256 7.0 / 6.9,
 // 8 8 256 10.0 / 9.4) and keeps those calls, which then give the bits of the forward that keeps its row statistic; against
 // 128 rows a workgroup they pay there as well (1 8 160 10.5 / 6.7).
@@ -577,6 +591,7 @@ static bool flash_f32_gradients_join(const FlashF32Params& p) {
 bool flash_f32_takes_split(const FlashF32Params& p, bool with_lse) {
     if (p.dim % 4 != 0 || p.dim > (with_lse ? 64 : 128) || p.bias || p.mask == kMaskPadding) return false;
     if (with_lse && flash_f32_gradients_join(p)) return true;
+    if (p.dim > 64 && p.mask == kMaskNone && !with_lse && flash_f32_takes_split_keys(p)) return flash_f32_rows_pay(p);  // either is ahead of the f32 kernel
     return flash_f32_split_pays(p) && (with_lse || !flash_f32_takes_split_keys(p) || flash_f32_rows_pay(p));
 }
 

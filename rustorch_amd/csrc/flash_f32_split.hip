@@ -434,13 +434,15 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
 // slots of a row XORed with bits of the row), brought there straight; K is requested again once its scores are formed, V
 // once it has been multiplied.  Every wave splits what it reads itself, between the matrix instructions of the piece before.
 //
-// What bounds it: the vector unit, with two workgroups a CU: about 700 instructions a tile and wave, half of them splits of K
+// What bounds it: the vector unit, with two workgroups a CU up to head dim 64 and one above (a wave then has its SIMD to itself, Q in
+// the accumulation registers): at head dim 64 about 700 instructions a tile and wave, half of them splits of K
 // and V that a workgroup of 128 rows shares.  us, f32 kernel -> this, B H N head dim: causal 1 8 2048 64 55.0 -> 42.9, 2 12 999 64
-// 51.5 -> 39.3, 1 4 3664 32 60.2 -> 48.9; unmasked 1 8 1024 64 28.5 -> 22.9, 1 8 512 64 16.6 -> 13.9; 1 8 2048 64 90.2 -> 68.7 (from 128
-// rows a workgroup).
+// 51.5 -> 39.3, 1 4 3664 32 60.2 -> 48.9, 1 8 3438 128 297 -> 223, 1 12 1500 96 120 -> 83, 2 4 333 68 19.5 -> 16.2; unmasked 1 8 1024 64
+// 28.5 -> 22.9, 1 8 512 64 16.6 -> 13.9, 1 8 1024 96 43.7 -> 35.8; 1 8 2048 64 90.2 -> 68.7 (from 128 rows a workgroup).  Eight waves that
+// share them, one workgroup a CU: 1 8 2048 64 42.6 -> 42.8, 4096 128 -> 140, unmasked 1 4 1024 22.2 -> 20.2, not kept.  Relative error
+// against 64 bits at head dim 128, N = 2048 unmasked 5.8e-7 -> 2.0e-7.
 template <int DT, bool kExactD, bool kCausal>
-__global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF32Params p) {
-    static_assert(DT <= 2, "two workgroups a CU");
+__global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_keys_kernel(FlashF32Params p) {
     constexpr int DPAD = 32 * DT, KS = DPAD / 16, SL = DPAD / 4, NREQ = 4 * DT, ROWB = DPAD * 4;
     constexpr int TILE = 32 * DPAD;  // floats
     constexpr int NW = 4, LDO = DPAD + 4;
@@ -480,7 +482,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
     const int n_tiles = (kv_end + kTile - 1) / kTile;
 
     // ---- a wave's tiles: instruction n brings chunks 64 n .. + 63 of 16 bytes, chunk c slot c % SL of row c / SL
-    auto swizzle = [](int r) RT_INLINE { return DT == 2 ? (r & 15) : ((r >> 1) & 7); };
+    auto swizzle = [](int r) RT_INLINE { return DT % 2 == 0 ? (r & 15) : ((r >> 1) & 7); };
     unsigned char* const Kw = (unsigned char*)(lds + wave * 2 * TILE);
     unsigned char* const Vw = Kw + TILE * 4;
     const uint32_t k_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)Kw, v_lds = k_lds + TILE * 4;
@@ -513,7 +515,9 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_f32_split_keys_kernel(FlashF
     auto read_k = [&](int j, float (&x)[8]) RT_INLINE {  // elements 16j + 8hh .. of key `col`
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            const f32x4_t z = *(const f32x4_t*)(Kw + (k_base ^ (uint32_t)((4 * j + u) * 16)));
+            // (rows of 24 slots, DT 3: only the lower three bits of a slot are XORed)
+            const uint32_t at = DT == 3 ? (k_base ^ (uint32_t)((4 * (j & 1) + u) * 16)) + (uint32_t)(128 * (j >> 1)) : k_base ^ (uint32_t)((4 * j + u) * 16);
+            const f32x4_t z = *(const f32x4_t*)(Kw + at);
 #pragma unroll
             for (int i = 0; i < 4; i++) x[4 * u + i] = z[i];
         }
@@ -847,7 +851,7 @@ hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p_in
 
 bool flash_f32_split_keys_supported(const FlashF32Params& p) {
     const long long keys = p.seq_kv ? p.seq_kv : p.seq;
-    return p.dim <= 64 && p.dim % 4 == 0 && (p.mask == kMaskNone || p.mask == kMaskCausal) && !p.bias && !p.lse && keys > 0 &&
+    return p.dim <= 128 && p.dim % 4 == 0 && (p.mask == kMaskNone || p.mask == kMaskCausal) && !p.bias && !p.lse && keys > 0 &&
            (unsigned long long)(keys + 256) * (unsigned long long)p.lkv.row_pitch * 4ull < (1ull << 32);  // 32-bit offsets
 }
 
@@ -855,17 +859,24 @@ hipError_t launch_flash_f32_split_keys(hipStream_t stream, const FlashF32Params&
     FlashF32Params p = p_in;
     if (!flash_f32_split_keys_supported(p)) return hipErrorInvalidValue;
     dim3 grid((p.seq + kTile - 1) / kTile, p.heads, p.batch), block(256);
-    p.zigzag = (p.mask == kMaskCausal) && ((long long)grid.x * grid.y * grid.z <= 2ll * p.n_cus) ? 1 : 0;
+    p.zigzag = (p.mask == kMaskCausal) && ((long long)grid.x * grid.y * grid.z <= (p.dim <= 64 ? 2ll : 1ll) * p.n_cus) ? 1 : 0;
     auto launch = [&](auto dt_c, auto exact_c) {
         constexpr int kDT = decltype(dt_c)::value;
         constexpr bool kEx = decltype(exact_c)::value;
         if (p.mask == kMaskCausal) hipLaunchKernelGGL((flash_fwd_f32_split_keys_kernel<kDT, kEx, true>), grid, block, 0, stream, p);
         else hipLaunchKernelGGL((flash_fwd_f32_split_keys_kernel<kDT, kEx, false>), grid, block, 0, stream, p);
     };
-    if (p.dim == 32) launch(std::integral_constant<int, 1>{}, std::true_type{});
-    else if (p.dim < 32) launch(std::integral_constant<int, 1>{}, std::false_type{});
-    else if (p.dim == 64) launch(std::integral_constant<int, 2>{}, std::true_type{});
-    else launch(std::integral_constant<int, 2>{}, std::false_type{});
+    auto launch_dt = [&](auto dt_c) {
+        if (p.dim % 32 == 0) launch(dt_c, std::true_type{});
+        else launch(dt_c, std::false_type{});
+    };
+    switch ((p.dim + 31) / 32) {
+        case 1: launch_dt(std::integral_constant<int, 1>{}); break;
+        case 2: launch_dt(std::integral_constant<int, 2>{}); break;
+        case 3: launch_dt(std::integral_constant<int, 3>{}); break;
+        case 4: launch_dt(std::integral_constant<int, 4>{}); break;
+        default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 

@@ -50,7 +50,7 @@ struct FlashF32Params {
 hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p);
 // The form on the bf16 matrix cores: dim <= 128 and a multiple of 4, 16-byte aligned rows, mask none or causal, no bias.
 hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p);
-// ... and for few rows: dim <= 64, no row statistic
+// ... and for few rows: no row statistic
 bool flash_f32_split_keys_supported(const FlashF32Params& p);
 hipError_t launch_flash_f32_split_keys(hipStream_t stream, const FlashF32Params& p);
 bool flash_f32_takes_split(const FlashF32Params& p, bool with_lse);  // by sizes and mask; for 16-byte aligned rows

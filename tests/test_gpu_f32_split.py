@@ -444,3 +444,49 @@ def test_few_rows_what_the_split_does_not_carry(what, causal):
     assert np.array_equal(np.isnan(got), np.isnan(want))
     ok = np.isfinite(want)
     assert np.abs(got - want)[ok].max() <= 5e-6
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("b,h,hkv,n,d", [
+    (1, 1, 1, 129, 128),   # one key in the second tile of the first wave
+    (1, 8, 8, 161, 96),    # rows of 24 slots in LDS
+    (2, 4, 1, 333, 68),    # grouped heads, the least of the padded columns
+    (1, 4, 2, 257, 100),
+    (1, 8, 8, 545, 80),    # three tiles a wave, then five
+    (2, 8, 8, 640, 128),   # more workgroups than CUs
+])
+def test_few_rows_above_head_dim_64(b, h, hkv, n, d, causal):
+    """The edges of tiles and of the padded columns, both layouts (what lies behind a head's columns there is another head's)."""
+    assert not ra.debug_f32_split_products(ra.AttentionShape.new(b, h, n, d), ra.Mask.causal() if causal else ra.Mask.none())
+    q = seeded_normal((b, h, n, d), 1).reshape(b, h, n, d)
+    k, v = (seeded_normal((b, hkv, n, d), i).reshape(b, hkv, n, d) for i in (2, 3))
+    want = attention64(q, np.repeat(k, h // hkv, axis=1), np.repeat(v, h // hkv, axis=1), causal)
+    shape, mask = ra.AttentionShape.new(b, h, n, d), ra.Mask.causal() if causal else ra.Mask.none()
+    got = []
+    for layout, call in ((np.ascontiguousarray, ra.flash_forward_f32_dev), (bnhd, ra.flash_forward_bnhd_f32_dev)):
+        out = ra.HipStorage(q.size * 4)
+        out.upload(np.full(q.size, 7.0, dtype=np.float32))
+        call(shape, dev(layout(q)), dev(layout(k)), dev(layout(v)), out, mask, n_kv_heads=hkv)
+        ra.synchronize()
+        got.append(layout(out.download(np.float32).reshape(layout(q).shape)))
+    assert np.array_equal(got[0], got[1])
+    assert np.linalg.norm(got[0] - want) <= 1e-6 * np.linalg.norm(want)
+    assert np.abs(got[0] - want).max() <= 5e-6
+
+
+@pytest.mark.parametrize("d", [96, 128])
+@pytest.mark.parametrize("what", ["k inf", "v inf", "q nan", "v small"])
+def test_few_rows_above_head_dim_64_what_the_split_does_not_carry(what, d):
+    """The second pass in f32 out of tiles of these widths: rows that see the value are what 64 bits make of them, the rest as they were."""
+    q, k, v = inputs(1, 2, 300, d)
+    x = {"q": q, "k": k, "v": v}[what[0]]
+    if what == "v small":
+        x[0, 0] = np.float32(1e-33)
+    else:
+        x[0, 1, 0 if what == "v inf" else 37, d - 1] = np.inf if what[2:] == "inf" else np.nan  # (every row sees key 0)
+    got, want = run(q, k, v, True), attention64(q, k, v, True)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    for head in range(2):
+        ok = np.isfinite(want[0, head])
+        err = np.linalg.norm((got[0, head].astype(np.float64) - want[0, head])[ok])
+        assert err <= 1e-6 * np.linalg.norm(want[0, head][ok])
