@@ -640,7 +640,7 @@ hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Param
     auto aligned = [](const void* ptr) { return (uintptr_t)ptr % 16 == 0; };
     p.vec = (p.dim % 4 == 0) && aligned(p.q) && aligned(p.k) && aligned(p.v) && aligned(p.d_out) && aligned(p.dq) &&
             aligned(p.dk) && aligned(p.dv);
-    if (p.vec && aligned(p.o)) {  // many rows: the bf16 matrix cores, by the rule of the forward
+    if (p.vec && aligned(p.o) && (unsigned long long)p.seq * (unsigned)p.dim * 4 < (1ull << 31)) {  // many rows: the bf16 matrix cores, by the rule of the forward
         FlashF32Params f{};
         f.batch = p.batch;
         f.heads = p.heads;

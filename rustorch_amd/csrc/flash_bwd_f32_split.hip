@@ -11,11 +11,12 @@
 // for; at head dim 64 a tile is 96 (dK/dV) and 72 (dQ) matrix instructions of 32 clocks and 520 and 400 vector ones of 4, each
 // kernel with room to run the one beside the other, and takes 4400 and 3500 clocks.  Hence: vector work between all matrix
 // instructions, in runs of independent instructions (SplitQuad); LDS writes one at a time; nothing loaded is looked at in
-// the step that requests it; owners and sums pinned to the accumulation registers, where the matrix instructions read them
-// and no vector instruction wants them.  Time of both, B=4 H=16 N=1024 D=64: f32 kernels 506 us, this form with columns of its
+// the step that requests it, nor copied there; owners pinned to the accumulation registers, where the matrix instructions read them
+// and no vector instruction wants them; sums wherever the vector unit need not fetch them.  Time of both, B=4 H=16 N=1024 D=64: f32 kernels 506 us, this form with columns of its
 // own in LDS 362, with the transposing reads 341, with every vector step beside a matrix instruction 336, without a wait
 // for the row statistic where it is requested 327, sums pinned 321, dQ in the same order 312, independent runs and single
-// writes 308.  B=2 N=2048 973, 689, 583; head dim 32 273, 214, 171.  (dQ with two waves a SIMD, 40 registers spilled: 318.)
+// writes 308.  B=2 N=2048 973, 689, 583; head dim 32 273, 214, 171.  (dQ with two waves a SIMD, 40 registers spilled: 318.)  On another
+// card: tiles loaded without a branch and owners all at once 327 -> 318, sums not pinned 313; 2 x 12 heads N=400 39.3 -> 37.1.
 // Relative error against 64 bits 5.9e-7 -> 4.5e-7, 7.3e-7 -> 5.9e-7, 5.5e-7 -> 4.4e-7 (f32 kernels -> this).
 #include <type_traits>
 
@@ -45,47 +46,61 @@ __device__ __forceinline__ void check8(const float (&x)[8], float& chk) {
     chk = split_too_small(m) ? kSplitMost : __builtin_fmaxf(chk, m);
 }
 
-// One streamed matrix [N, D]: a tile's rows on their way from memory into LDS.  Rows behind the last repeat it; whoever reads
-// the tile gives them weights of zero.
+// One streamed matrix [N, D]: a tile's rows on their way from memory into LDS, in pieces of eight elements of a row, kN a thread.
+// Rows behind the last repeat it; whoever reads the tile gives them weights of zero.
 template <int DT>
 struct Stream {
     using Plane = SplitPlane<DT>;
-    static constexpr int DPAD = 32 * DT;
+    static constexpr int DPAD = 32 * DT, CH = DPAD / 8, ITEMS = kTile * CH, kN = (ITEMS + 255) / 256;
     static constexpr int SIZE = 3 * Plane::SIZE;  // bf16 elements of a tile
-    static constexpr int ITEMS = 4 * DPAD;
-    f32x4_t r[2];
+    f32x4_t r[kN][2];
+    __amdgpu_buffer_rsrc_t rs;
+    int pitch, last;
 
-    __device__ __forceinline__ void clear() { r[0] = r[1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}; }
-    // `at`: byte offset of this thread's piece from a tile's first row.  A tile that ends within N and rows of DPAD columns,
-    // the usual case, cost two loads and no vector instruction.
-    static __device__ __forceinline__ uint32_t piece(int D, int tid) { return 4u * (uint32_t)(tid / (DPAD / 8) * D + 8 * (tid % (DPAD / 8))); }
-    __device__ __forceinline__ void load(const float* __restrict__ src, int row0, int N, int D, int tid, uint32_t at) {
-        if (ITEMS % 256 != 0 && tid >= ITEMS) return;
-        if (row0 + kTile <= N && D == DPAD) {  // uniform
-            const char* const x = (const char*)(src + (size_t)row0 * D);
+    // Where a thread's pieces lie in a row: byte offsets of either half, past every descriptor where the row has no such elements.
+    struct Place {
+        uint32_t at[kN][2];
+        __device__ __forceinline__ Place(int D, int tid) {
 #pragma unroll
-            for (int u = 0; u < 2; u++) r[u] = *(const f32x4_t*)(x + at + 16 * u);
-            return;
+            for (int n = 0; n < kN; n++)
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const int d = 8 * ((256 * n + tid) % CH) + 4 * u;
+                    at[n][u] = d < D ? 4u * (uint32_t)d : 0x80000000u;
+                }
         }
-        const int row = min(row0 + tid / (DPAD / 8), N - 1), d = 8 * (tid % (DPAD / 8));
-        const float* x = src + (size_t)row * D + d;
+    };
+    static __device__ __forceinline__ bool has(int n, int tid) { return ITEMS % 256 == 0 || 256 * n + tid < ITEMS; }
+
+    // (N rows of D f32, less than 2 GiB)
+    __device__ __forceinline__ Stream(const float* src, int N, int D)
+        : rs(__builtin_amdgcn_make_buffer_rsrc((void*)src, 0, 4u * (uint32_t)N * (uint32_t)D, kBufferFlags)), pitch(4 * D), last(N - 1) {
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (d + 4 * u < D) z = *(const f32x4_t*)(x + 4 * u);
-            r[u] = z;
+        for (int n = 0; n < kN; n++) r[n][0] = r[n][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    // Without a branch around a load, or two ways to one: where those met, the registers were copied, and the copies waited for the
+    // loads just requested.
+    __device__ __forceinline__ void load(int tile, const Place& place, int tid) {
+        const int row0 = min(kTile * tile, last), left = last - row0;
+        const uint32_t so = (uint32_t)row0 * (uint32_t)pitch;
+#pragma unroll
+        for (int n = 0; n < kN; n++) {
+            const uint32_t row = (uint32_t)min((256 * n + tid) / CH, left);
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                r[n][u] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, __umul24(row, (uint32_t)pitch) + place.at[n][u], so, 0));
         }
     }
-    // Splitting in ten steps a row piece of eight elements, five for either half.
-    static constexpr int STEPS = 2 * SplitQuad::STEPS;
+    // Splitting in ten steps a piece, five for either half.
+    static constexpr int STEPS = 2 * SplitQuad::STEPS * kN;
     u32x4_t w[3];
     SplitQuad quad;
     float m;
     __device__ __forceinline__ void step(int x, __bf16* buf, int tid, float& chk) {
-        const int h = x / SplitQuad::STEPS, k = x % SplitQuad::STEPS;
+        const int n = x / (2 * SplitQuad::STEPS), h = x / SplitQuad::STEPS % 2, k = x % SplitQuad::STEPS;
         if (k == 0) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) quad.r[i] = r[h][i];
+            for (int i = 0; i < 4; i++) quad.r[i] = r[n][h][i];
         }
         uint32_t a = 0, b = 0;
         quad.step(k, a, b);
@@ -94,12 +109,15 @@ struct Stream {
             w[k / 2][2 * h + 1] = b;
         }
         if (k == 3) {
-            m = split_max(split_max(h == 0 ? 0.0f : m, r[h][0]), r[h][1]);
-            m = split_max(split_max(m, r[h][2]), r[h][3]);
+            m = split_max(split_max(h == 0 ? 0.0f : m, r[n][h][0]), r[n][h][1]);
+            m = split_max(split_max(m, r[n][h][2]), r[n][h][3]);
+            asm volatile("" : "+v"(m));  // here: put off behind the next tile's loads, it would keep them out of these registers
         }
-        if (h == 1 && k % 2 == 0 && (ITEMS % 256 == 0 || tid < ITEMS))  // a plane at a time: three writes at once hold the wave
-            *(u32x4_t*)(buf + Plane::at(tid / (DPAD / 8), tid % (DPAD / 8)) + (k / 2) * Plane::SIZE) = w[k / 2];
-        if (x == STEPS - 1) chk = split_too_small(m) ? kSplitMost : __builtin_fmaxf(chk, m);
+        if (h == 1 && k % 2 == 0 && has(n, tid)) {  // a plane at a time: three writes at once hold the wave
+            const int idx = 256 * n + tid;
+            *(u32x4_t*)(buf + Plane::at(idx / CH, idx % CH) + (k / 2) * Plane::SIZE) = w[k / 2];
+        }
+        if (h == 1 && k == 4) chk = split_too_small(m) ? kSplitMost : __builtin_fmaxf(chk, m);
     }
     __device__ __forceinline__ void store(__bf16* buf, int tid, float& chk) {
 #pragma unroll
@@ -114,16 +132,41 @@ struct Stream {
     }
 };
 
-// 8 elements of a row, zeros beyond seq and dim
-__device__ __forceinline__ void load8(float (&x)[8], const float* __restrict__ src, int row, int d, int N, int D) {
+// The owners' rows: this lane's elements 16j + 8hh .. of row `row` of N rows of D, zeros beyond seq and dim, without a branch, so that
+// all are on their way together.
+template <int KS>
+struct OwnerRow {
+    f32x4_t x[KS][2];
+    __device__ __forceinline__ void load(const float* src, int row, int N, int D, int hh) {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, 4u * (uint32_t)N * (uint32_t)D, kBufferFlags);
+        const uint32_t at = row < N ? 4u * (uint32_t)row * (uint32_t)D : 0x80000000u;
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-        f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (row < N && d + 4 * u < D) z = *(const f32x4_t*)(src + (size_t)row * D + d + 4 * u);
+        for (int j = 0; j < KS; j++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) x[4 * u + i] = z[i];
+            for (int u = 0; u < 2; u++) {
+                const int d = 16 * j + 8 * hh + 4 * u;
+                x[j][u] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, d < D ? at + 4u * (uint32_t)d : 0x80000000u, 0, 0));
+            }
     }
-}
+    __device__ __forceinline__ void split(Split8 (&s)[KS], float& chk) const {
+#pragma unroll
+        for (int j = 0; j < KS; j++) {
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) y[i] = x[j][i >> 2][i & 3];
+            check8(y, chk);
+            s[j] = split8(y);
+        }
+    }
+    __device__ __forceinline__ float dot(const OwnerRow& o) const {
+        float sum = 0.0f;
+#pragma unroll
+        for (int j = 0; j < KS; j++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) sum = __builtin_fmaf(o.x[j][i >> 2][i & 3], x[j][i >> 2][i & 3], sum);
+        return sum;
+    }
+};
 
 // accumulators (d = 32t + 8g + 4hh + i of row `row`) to row `row` of a [seq, dim] matrix
 template <int DT>
@@ -188,15 +231,12 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
 
     float chk = 0.0f;
     Split8 kf[KS], vf[KS];
-#pragma unroll
-    for (int j = 0; j < KS; j++) {
-        float x[8];
-        load8(x, Kg, key, 16 * j + 8 * hh, N, D);
-        check8(x, chk);
-        kf[j] = split8(x);
-        load8(x, Vg, key, 16 * j + 8 * hh, N, D);
-        check8(x, chk);
-        vf[j] = split8(x);
+    {
+        OwnerRow<KS> k, v;
+        k.load(Kg, key, N, D, hh);
+        v.load(Vg, key, N, D, hh);
+        k.split(kf, chk);
+        v.split(vf, chk);
     }
     // Each sum in two register sets: the large terms (hh), and the five small ones.  The large set is rounded twice a tile
     // instead of twelve times, and no vector instruction touches either.
@@ -209,26 +249,23 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
         zero16(low_dk[t]);
     }
 
-    St q_in, o_in, out_in;  // out_in: O, for delta; read and multiplied, never split
-    q_in.clear();
-    o_in.clear();
-    out_in.clear();
+    const typename St::Place place(D, tid);
+    St q_in(Qg, N, D), o_in(dOg, N, D), out_in(Og, N, D);  // out_in: O, for delta; read and multiplied, never split
     float st = 0.0f;  // threads 0..31: the row statistic, 32..63: delta.  Rows beyond seq: +inf, their weights are zeros
-    const uint32_t piece = St::piece(D, tid);
-    const float* const st_src = kOwnDelta || tid < 32 ? lse : delta;  // (kOwnDelta: the upper half's is not used)
-    auto load = [&](int row0) RT_INLINE {
-        q_in.load(Qg, row0, N, D, tid, piece);
-        o_in.load(dOg, row0, N, D, tid, piece);
-        if constexpr (kOwnDelta) out_in.load(Og, row0, N, D, tid, piece);
-        if (wave == 0) st = st_src[min(row0 + (tid & 31), N - 1)];
+    const float* const st_src = kOwnDelta || lane < 32 ? lse : delta;  // (kOwnDelta: the upper half's is not used)
+    auto load = [&](int tile) RT_INLINE {
+        q_in.load(tile, place, tid);
+        o_in.load(tile, place, tid);
+        if constexpr (kOwnDelta) out_in.load(tile, place, tid);
+        st = st_src[min(tile * kTile + (lane & 31), N - 1)];  // (in every wave: no branch around a load)
     };
     auto put_delta = [&](int b, int row0) RT_INLINE {  // of the tile's rows of dO and O as they came; returns it
         constexpr int LANES = DPAD / 8;  // of a row
         float x = 0.0f, y = 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            x = __builtin_fmaf(o_in.r[0][i], out_in.r[0][i], x);
-            y = __builtin_fmaf(o_in.r[1][i], out_in.r[1][i], y);
+            x = __builtin_fmaf(o_in.r[0][0][i], out_in.r[0][0][i], x);
+            y = __builtin_fmaf(o_in.r[0][1][i], out_in.r[0][1][i], y);
         }
         const int row = tid / LANES;
         x = row0 + row < N ? lanes_sum<LANES>(x + y) : 0.0f;
@@ -265,7 +302,7 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
     load(0);
     store(0);
     const bool uncarried = __syncthreads_or(!(chk < kSplitMost));  // seen already: no step of the loop below
-    if (n_tiles > 1) load(kTile);
+    load(1);
     // A step's products, in the order S = Q K^T, dP = dO V^T, dV += P^T dO, dK += dS^T Q: no vector work stands alone.  The next tile (in
     // registers since the step before) is split between the instructions of S, P is formed and split between those of dP and
     // the first of dV, dS between those of dV and the first half of dK.  With one wave a SIMD nothing else would keep both
@@ -275,8 +312,6 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
         const __bf16* ob = qb + St::SIZE;
         __bf16* nb = lds + ((tile + 1) & 1) * BUF;  // behind the last tile: a repeat that nobody reads
         if constexpr (DT > 1) {
-#pragma unroll
-            for (int t = 0; t < DT; t++) asm volatile("" : "+a"(acc_dv[t]), "+a"(acc_dk[t]), "+a"(low_dv[t]), "+a"(low_dk[t]));
 #pragma unroll
             for (int j = 0; j < KS; j++) asm volatile("" : "+a"(kf[j].p[0]), "+a"(kf[j].p[1]), "+a"(kf[j].p[2]), "+a"(vf[j].p[0]), "+a"(vf[j].p[1]), "+a"(vf[j].p[2]));
         }
@@ -340,7 +375,7 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
             RT_ORDER();
         }
         put_stat((tile + 1) & 1, (tile + 1) * kTile);  // (behind the last tile: nothing is read there)
-        if (tile + 2 < n_tiles) load((tile + 2) * kTile);
+        load(tile + 2);  // (behind the last tile: its last row, which nobody reads)
         read_plane(ob, 2);
 #pragma unroll
         for (int g = 0; g < 4; g++) {
@@ -411,8 +446,8 @@ __device__ __forceinline__ void bwd_dkdv_split(const FlashBwdF32Params& p, int l
             qt.template load<true>(Qg, (size_t)D, q0, N, D, tid);
             ot.load(dOg, (size_t)D, q0, N, D, tid);
             if constexpr (kOwnDelta) {  // dO once more, as the sum over neighbouring lanes wants it (a row a lane: 409 us, B=1 H=8 N=2048 D=64; this 354)
-                o_in.load(dOg, q0, N, D, tid, piece);
-                out_in.load(Og, q0, N, D, tid, piece);
+                o_in.load(q0 / kTile, place, tid);
+                out_in.load(q0 / kTile, place, tid);
             }
             if (tid < (kOwnDelta ? 32 : 64)) {
                 const int row = q0 + (tid & 31);
@@ -479,18 +514,14 @@ __device__ __forceinline__ void bwd_dq_split(const FlashBwdF32Params& p, int lin
     // the owner rows, and delta = dO . O of each: half a row in this lane, half in lane + 32
     float chk = 0.0f, delta_q = 0.0f;
     Split8 qf[KS], of[KS];
-#pragma unroll
-    for (int j = 0; j < KS; j++) {
-        float x[8], y[8];
-        load8(x, Qg, q_row, 16 * j + 8 * hh, N, D);
-        check8(x, chk);
-        qf[j] = split8(x);
-        load8(x, dOg, q_row, 16 * j + 8 * hh, N, D);
-        check8(x, chk);
-        of[j] = split8(x);
-        load8(y, Og, q_row, 16 * j + 8 * hh, N, D);
-#pragma unroll
-        for (int i = 0; i < 8; i++) delta_q = __builtin_fmaf(y[i], x[i], delta_q);
+    {
+        OwnerRow<KS> q, g, o;
+        q.load(Qg, q_row, N, D, hh);
+        g.load(dOg, q_row, N, D, hh);
+        o.load(Og, q_row, N, D, hh);
+        q.split(qf, chk);
+        g.split(of, chk);
+        delta_q = g.dot(o);
     }
     delta_q += other_half(delta_q);
     if (kLeaveDelta && hh == 0 && q_ok) p.delta[(size_t)bh * N + q_row] = delta_q;
@@ -504,13 +535,11 @@ __device__ __forceinline__ void bwd_dq_split(const FlashBwdF32Params& p, int lin
         zero16(acc[t]);
         zero16(low[t]);
     }
-    St k_in, v_in;
-    k_in.clear();
-    v_in.clear();
-    const uint32_t piece = St::piece(D, tid);
-    auto load = [&](int row0) RT_INLINE {
-        k_in.load(Kg, row0, N, D, tid, piece);
-        v_in.load(Vg, row0, N, D, tid, piece);
+    const typename St::Place place(D, tid);
+    St k_in(Kg, N, D), v_in(Vg, N, D);
+    auto load = [&](int tile) RT_INLINE {
+        k_in.load(tile, place, tid);
+        v_in.load(tile, place, tid);
     };
     auto store = [&](int b) {
         k_in.store(lds + b * BUF, tid, chk);
@@ -533,14 +562,12 @@ __device__ __forceinline__ void bwd_dq_split(const FlashBwdF32Params& p, int lin
     load(0);
     store(0);
     const bool uncarried = __syncthreads_or(!(chk < kSplitMost));  // seen already: no step of the loop below
-    if (n_tiles > 1) load(kTile);
+    load(1);
     for (int tile = 0; tile < (uncarried ? 0 : n_tiles); tile++) {  // a step as in the kernel above, in the order S, dP, dQ
         const __bf16* kb = lds + (tile & 1) * BUF;
         const __bf16* vb = kb + St::SIZE;
         __bf16* nb = lds + ((tile + 1) & 1) * BUF;
         if constexpr (DT > 1) {
-#pragma unroll
-            for (int t = 0; t < DT; t++) asm volatile("" : "+a"(acc[t]), "+a"(low[t]));
 #pragma unroll
             for (int j = 0; j < KS; j++) asm volatile("" : "+a"(qf[j].p[0]), "+a"(qf[j].p[1]), "+a"(qf[j].p[2]), "+a"(of[j].p[0]), "+a"(of[j].p[1]), "+a"(of[j].p[2]));
         }
@@ -566,7 +593,7 @@ __device__ __forceinline__ void bwd_dq_split(const FlashBwdF32Params& p, int lin
             }
             RT_ORDER();
         }
-        if (tile + 2 < n_tiles) load((tile + 2) * kTile);
+        load(tile + 2);  // (behind the last tile: its last row, which nobody reads)
         read_plane(vb, 2);
         hide_edge(s, tile * kTile);
         u32x4_t dw[2][3];
