@@ -236,7 +236,8 @@ int rt_debug_force_bf16_prefill_kernel(int which);
 /* No counterpart in the reference: for measurements and tests.  1 if an f32 forward of this shape (seq_kv keys; 0: seq) on
  * 16-byte aligned tensors runs on the bf16 matrix cores, operands as three bf16 terms, in workgroups of 128 query rows; 0
  * if not: few rows without the row statistic have the same products in workgroups of 32 rows, the rest
- * the f32 matrix cores.  with_lse != 0: the forward that keeps the row statistic, and the gradients.  Asks no device:
+ * the f32 matrix cores.  with_lse != 0: the forward that keeps the row statistic, and the gradients, up to
+ * head dim 64 (0 above, where the gradients have a form of their own).  Asks no device:
  * before the first call on one the answer is that of 256 compute units. */
 int rt_debug_f32_split_products(const rt_attention_shape *shape, uint64_t seq_kv, int mask_kind, int with_lse);
 

@@ -588,6 +588,23 @@ __global__ __launch_bounds__(256) void flash_bwd_rows_dkdv_kernel(FlashBwdF32Par
 // 92.5 -> 53.8, 1 8 2048 64 247 -> 163, 3 16 165 64 39.0 -> 22.4.
 bool bwd_f32_one_launch(long long blocks, int per_cu, int n_cus) { return 2 * blocks <= (long long)per_cu * (n_cus > 0 ? n_cus : 256); }
 
+// Head dims above 64: do the gradients run on the split products (flash_bwd_f32_wide.hpp)?  In us: a workgroup of 128 rows takes 9 and 3.5
+// a tile of 32 (7 and 2.8 up to 96) for dQ or dK and two thirds of it for dV, side by side where they fill less than the chip;
+// the f32 kernels' workgroups of 32 rows 5 and 8.5 (6.9) for every four tiles, dQ and dK/dV one behind the other, or, where both fit the chip,
+// 6 and 12 (10 and 7) for the two.  us of the gradients, f32 / split, B H N head dim: 4 16 1024 128 1084 / 740, 96 868 / 587; 4 16 453
+// 80 297 / 142; 2 8 640 128 176 / 89; 1 4 2500 128 633 / 296; 2 8 300 96 51 / 42; 8 16 128 128 60 / 58; and on the other side 1 8
+// 500 128 52 / 65, 3 4 202 128 31 / 38, 8 16 64 128 29 / 36, 1 8 250 96 24 / 33.
+bool flash_f32_gradients_wide(const FlashF32Params& p) {
+    if (p.dim <= 64 || p.dim > 128 || p.dim % 4 != 0 || p.mask != kMaskNone || p.bias || (unsigned long long)p.seq * (unsigned)p.dim * 4 >= (1ull << 31)) return false;
+    const double n_cus = p.n_cus > 0 ? p.n_cus : 256, tiles = (p.seq + 31) / 32, n_bh = (double)p.heads * p.batch;
+    const double n = n_bh * ((p.seq + 127) / 128), small = n_bh * tiles, steps = __builtin_ceil(tiles / 4);
+    const bool high = p.dim > 96;
+    const double one = high ? 9 + 3.5 * tiles : 7 + 2.8 * tiles;
+    const double wide = 3 * n <= n_cus ? one + 6 : n < n_cus ? one * __builtin_fmax(1.66, 2.66 * n / n_cus) + 8 : one * 1.15 * 2.66 * __builtin_ceil(n / n_cus);
+    const double f32 = 2 * small <= n_cus ? (high ? 6 + 12 * steps : 10 + 7 * steps) : 2 * __builtin_ceil(small / n_cus) * (5 + (high ? 8.5 : 6.9) * steps);
+    return wide < f32;
+}
+
 size_t flash_bwd_f32_workspace_floats(int batch, int heads, int seq, int dim) {
     return (size_t)batch * heads * seq * ((size_t)dim + 2);
 }
@@ -648,6 +665,7 @@ hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Param
         f.dim = p.dim;
         f.mask = kMaskNone;
         f.n_cus = p.n_cus;
+        if (flash_f32_gradients_wide(f) && bwd_f32_apart(p)) return launch_flash_bwd_f32_wide(stream, p);
         if (flash_f32_takes_split(f, true)) return launch_flash_bwd_f32_split(stream, p);
     }
     dim3 grid((p.seq + kRows - 1) / kRows, p.heads, p.batch), block(256);

@@ -747,3 +747,5 @@ hipError_t launch_flash_bwd_f32_split(hipStream_t stream, const FlashBwdF32Param
 }
 
 }  // namespace rt
+
+#include "flash_bwd_f32_wide.hpp"

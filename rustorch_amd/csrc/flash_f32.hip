@@ -562,16 +562,16 @@ static bool flash_f32_rows_pay(const FlashF32Params& p) {
 }
 
 // Keys from which the shared keys pay: with 128 a wave has one tile at most, and the f32 kernel is level (7.1 / 7.4 us; at head dim
-// 128 11.9 / 12.5).
+// 128 11.9 / 12.5, and with two tiles a wave at most nearly so: 17.4 / 16.5).
 // Unmasked up to head dim 32 it is level up to 256 (us, f32 kernel / shared keys, B H N: 1 8 256 6.9 / 6.8, 2 12 256 7.0 / 6.9,
 // 8 8 256 10.0 / 9.4) and keeps those calls, which then give the bits of the forward that keeps its row statistic; against
 // 128 rows a workgroup they pay there as well (1 8 160 10.5 / 6.7).
-constexpr int kSplitKeysFrom = 129, kSplitKeysFrom32 = 257;
+constexpr int kSplitKeysFrom = 129, kSplitKeysFrom32 = 257, kSplitKeysFrom128 = 225;
 static bool flash_f32_takes_split_keys(const FlashF32Params& p) {
-    if (!flash_f32_split_keys_supported(p)) return false;
+    if (!flash_f32_split_keys_supported(p) || p.lse) return false;
     const long long keys = p.seq_kv ? p.seq_kv : p.seq;
     const bool level = p.mask == kMaskNone && p.dim <= 32 && !flash_f32_split_pays(p);
-    return keys >= (level ? kSplitKeysFrom32 : kSplitKeysFrom);
+    return keys >= (level ? kSplitKeysFrom32 : p.dim > 96 ? kSplitKeysFrom128 : kSplitKeysFrom);
 }
 
 // Unmasked, head dims 33 to 64, for a forward whose row statistic the gradients read: the gradients' two kernels run side by
@@ -587,7 +587,7 @@ static bool flash_f32_gradients_join(const FlashF32Params& p) {
            bwd_f32_one_launch(n_bh * ((p.seq + 127) / 128), 1, p.n_cus);
 }
 
-// (above head dim 64 the gradients have no such form, and a row statistic they read is formed as they form the scores)
+// (above head dim 64 with the row statistic: flash_f32_gradients_wide, flash_bwd_f32.hip)
 bool flash_f32_takes_split(const FlashF32Params& p, bool with_lse) {
     if (p.dim % 4 != 0 || p.dim > (with_lse ? 64 : 128) || p.bias || p.mask == kMaskPadding) return false;
     if (with_lse && flash_f32_gradients_join(p)) return true;
@@ -611,6 +611,8 @@ hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p) {
         pz.zigzag = (p.mask == kMaskCausal) && ((long long)grid.x * grid.y * grid.z <= resident) ? 1 : 0;
         const bool exact = (p.dim % 32 == 0), pad = (p.mask == kMaskPadding);
         if (p.bias && p.mask != kMaskNone) return hipErrorInvalidValue;  // a bias comes without a mask kind
+        if (p.lse && flash_f32_gradients_wide(p))  // the statistic of scores formed as the gradients form them
+            return flash_f32_rows_pay(p) || !flash_f32_split_keys_supported(p) ? launch_flash_f32_split(stream, p) : launch_flash_f32_split_keys(stream, p);
         if (flash_f32_takes_split(p, p.lse != nullptr)) return launch_flash_f32_split(stream, p);
         if (flash_f32_takes_split_keys(p)) return launch_flash_f32_split_keys(stream, p);
         const int mode = pad ? 2 : (p.mask == kMaskCausal ? 1 : (p.bias ? 3 : 0));

@@ -50,10 +50,11 @@ struct FlashF32Params {
 hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p);
 // The form on the bf16 matrix cores: dim <= 128 and a multiple of 4, 16-byte aligned rows, mask none or causal, no bias.
 hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p);
-// ... and for few rows: no row statistic
+// ... and for few rows
 bool flash_f32_split_keys_supported(const FlashF32Params& p);
 hipError_t launch_flash_f32_split_keys(hipStream_t stream, const FlashF32Params& p);
 bool flash_f32_takes_split(const FlashF32Params& p, bool with_lse);  // by sizes and mask; for 16-byte aligned rows
+bool flash_f32_gradients_wide(const FlashF32Params& p);  // the same of launch_flash_bwd_f32_wide
 
 // Backward of unmasked f32 attention; every tensor is [batch, heads, seq, dim] row-major and contiguous.
 struct FlashBwdF32Params {
@@ -98,6 +99,8 @@ inline bool bwd_f32_apart(const FlashBwdF32Params& p) {
 }
 // Its form on the bf16 matrix cores: p.o, p.lse and p.delta set, dim <= 64 and a multiple of 4, all tensors 16-byte aligned.
 hipError_t launch_flash_bwd_f32_split(hipStream_t stream, const FlashBwdF32Params& p);
+// ... and for 64 < dim <= 128; the gradients share no memory with what is read, nor with each other (bwd_f32_apart)
+hipError_t launch_flash_bwd_f32_wide(hipStream_t stream, const FlashBwdF32Params& p);
 
 struct FlashBf16Params {
     const uint16_t* q;

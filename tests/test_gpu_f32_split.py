@@ -448,7 +448,8 @@ def test_few_rows_what_the_split_does_not_carry(what, causal):
 
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("b,h,hkv,n,d", [
-    (1, 1, 1, 129, 128),   # one key in the second tile of the first wave
+    (1, 1, 1, 129, 96),    # one key in the second tile of the first wave
+    (1, 1, 1, 225, 128),   # one key in the eighth tile
     (1, 8, 8, 161, 96),    # rows of 24 slots in LDS
     (2, 4, 1, 333, 68),    # grouped heads, the least of the padded columns
     (1, 4, 2, 257, 100),
@@ -490,3 +491,76 @@ def test_few_rows_above_head_dim_64_what_the_split_does_not_carry(what, d):
         ok = np.isfinite(want[0, head])
         err = np.linalg.norm((got[0, head].astype(np.float64) - want[0, head])[ok])
         assert err <= 1e-6 * np.linalg.norm(want[0, head][ok])
+
+
+# ---- gradients above head dim 64: dK and dV in workgroups of their own
+
+WIDE = [
+    (2, 8, 300, 96),    # all three in one launch, the last tile of 12 rows, the last workgroup of 44
+    (4, 8, 225, 68),    # one row in the last tile, most of the third column block empty
+    (2, 8, 640, 128),   # whole tiles
+    (6, 16, 200, 128),  # one launch of more workgroups than CUs
+    (4, 16, 453, 80),   # dQ ahead of dK and dV
+    (8, 17, 257, 100),  # head pairs not a multiple of eight, one row in the last workgroup
+    (8, 16, 128, 96),   # four tiles
+]
+
+
+@pytest.mark.parametrize("b,h,n,d", WIDE)
+def test_wide_gradients_against_64_bits(b, h, n, d):
+    """The bound of test_gradients_against_64_bits."""
+    x = inputs(b, h, n, d) + [seeded_normal((b, h, n, d), 4).reshape(b, h, n, d)]
+    got = run_backward(*x)
+    for name, g, w in zip(("dq", "dk", "dv"), got, gradients64(*x)):
+        assert np.linalg.norm(g - w) <= 2e-6 * np.linalg.norm(w), name
+    for g, again in zip(got, run_backward(*x)):
+        assert np.array_equal(g, again)
+
+
+@pytest.mark.parametrize("b,h,n,d", [(2, 8, 300, 96), (8, 16, 200, 128)])
+@pytest.mark.parametrize("what", ["key inf", "value inf", "d_out nan", "query nan", "small"])
+def test_wide_gradients_of_values_the_split_does_not_carry(b, h, n, d, what):
+    """Only the head that holds them changes, and its workgroups that read them do their rows once more in f32."""
+    x = inputs(b, h, n, d) + [seeded_normal((b, h, n, d), 4).reshape(b, h, n, d)]
+    q, k, v, d_out = x
+    at = (1, 5)
+    if what == "key inf":
+        q[at][:, 9] = -np.abs(q[at][:, 9]) - 0.1
+        k[at][n - 1, 9] = np.inf
+    elif what == "value inf":
+        v[at][40, 9] = np.inf
+    elif what == "d_out nan":
+        d_out[at][17, 3] = np.nan
+    elif what == "query nan":
+        q[at][17, 3] = np.nan
+    else:
+        d_out[at] *= np.float32(2.0 ** -115)
+    got, want = run_backward(*x), gradients64(*x)
+    other = np.ones((b, h), dtype=bool)
+    other[at] = False
+    for name, g, w in zip(("dq", "dk", "dv"), got, want):
+        assert np.linalg.norm(g[other] - w[other]) <= 2e-6 * np.linalg.norm(w[other]), name
+        gs, ws = g[at].astype(np.float64), w[at]
+        fin = np.isfinite(ws)
+        assert np.array_equal(np.isfinite(gs), fin), name
+        assert not fin.any() or np.linalg.norm((gs - ws)[fin]) <= 2e-6 * np.linalg.norm(ws[fin]), name
+
+
+@pytest.mark.parametrize("over", ["dk k", "dk v, dv k", "dq out", "dv k"])
+def test_wide_gradients_over_what_they_read(over):
+    """Tensors that share memory take the f32 kernels, one behind the other."""
+    b, h, n, d = 2, 8, 300, 96
+    x = inputs(b, h, n, d) + [seeded_normal((b, h, n, d), 4).reshape(b, h, n, d)]
+    shape = ra.AttentionShape.new(b, h, n, d)
+    t = dict(zip(("q", "k", "v", "d_out"), (dev(y.ravel()) for y in x)))
+    t["out"], lse, ws = ra.HipStorage(4 * b * h * n * d), ra.HipStorage(4 * b * h * n), ra.HipStorage(4 * b * h * n)
+    g = {y: ra.HipStorage(4 * b * h * n * d) for y in ("dq", "dk", "dv")}
+    ra.flash_forward_stats_f32_dev(shape, t["q"], t["k"], t["v"], t["out"], lse)
+    for pair in over.split(", "):
+        a, z = pair.split()
+        g[a] = t[z]
+    ra.flash_backward_saved_f32_dev(shape, t["q"], t["k"], t["v"], t["out"], lse, t["d_out"], g["dq"], g["dk"], g["dv"], ws, ws.byte_len)
+    ra.synchronize()
+    for name, w in zip(("dq", "dk", "dv"), gradients64(*x)):
+        got = g[name].download(np.float32).reshape(b, h, n, d)
+        assert np.linalg.norm(got - w) <= 2e-6 * np.linalg.norm(w), name
