@@ -74,9 +74,9 @@ __device__ __forceinline__ float t_max16(const f32x16_t& s) {
     return __builtin_fmaxf(t_max3(t0, t1, t2), s[15]);
 }
 
-template <int DP>
+template <int DP, bool DIRECT = false>
 struct TileCfg {
-    static constexpr int KT = TileLds<DP>::KT;  // keys per LDS tile
+    static constexpr int KT = DP > 128 && !DIRECT ? 32 : TileLds<DP>::KT;  // keys per LDS tile
     static constexpr int NI = KT / 32;              // 32-key items per tile
     static constexpr int THREADS = 256;
     static constexpr int LDK = DP + 8;                        // +16 B: 16 rows x 16 B tile all 64 banks
@@ -90,7 +90,7 @@ struct TileCfg {
     // DIRECT: unpadded tiles (rows of DP * 2 bytes, 16-byte slots swizzled), filled by loads that go straight to LDS
     static constexpr int STAGE_BYTES = TileLds<DP>::STAGE_BYTES;
     static constexpr int LDS_BYTES_DIRECT = 4 * STAGE_BYTES > 4 * REGION ? 4 * STAGE_BYTES : 4 * REGION;
-    static constexpr int OCC_DIRECT = DP <= 64 ? 3 : 2;
+    static constexpr int OCC_DIRECT = OCC;
     static constexpr int BIAS_BYTES = 32 * 32 * 4;  // a wave's bias values of an item: 32 rows of 32 keys
 };
 
@@ -173,14 +173,15 @@ enum TileWay : int { kTilesRegs = 0, kTilesDirect = 1, kTilesDirectPart = 2 };
 // moved by that many keys, as for a span of SPLIT), and an item that holds keys below some row's window is masked on
 // that side as well.
 //
-// DIRECT (head dims up to 128): the tiles travel from memory straight into LDS
+// DIRECT: the tiles travel from memory straight into LDS
 // (buffer_load_dwordx4 ... lds) instead of through registers and LDS writes.  After a tile's barrier the waves request
 // K(t+2) and V(t+1) into the stages K(t) and V(t-1) have just left and wait for their own requests ahead of the next
 // tile's barrier.  LDS rows are unpadded (a landing block of 1 KB is contiguous) and their 16-byte slots are XORed
 // with bits of the row, as in flash_bf16.hip.  Same instructions on the same operands otherwise: the same bits.
 // Measured against the register path, interleaved in one process: 3-5 % on short or padded sequences (B=16 H=16
 // N=1024: 52.3 -> 49.3 us), 7-9 % on long ones (B=4 H=32 N=4096: 306 -> 283 us), 4-7 % at head dim 128, 10-11 % at 96 and
-// 80 (B=2 H=16 N=4096: 123.5 -> 111.8 and 119.6 -> 107.7), 5 % at 32 (58.4 -> 55.8); three stages per matrix or four
+// 80 (B=2 H=16 N=4096: 123.5 -> 111.8 and 119.6 -> 107.7), 5 % at 32 (58.4 -> 55.8), 20-40 % at 256 (takes_tiles_direct), where it
+// is what leaves the registers for the pipelined walk: 512 of them, a wave a SIMD; three stages per matrix or four
 // workgroups per CU (head dim 64) are no faster.  Head dims between the tile widths have a form of their own
 // (kTilesDirectPart), whose requests leave the lanes behind the head dim out: two scalar instructions a request, which
 // cost the masked form at head dim 64 6 % where the kernel of whole rows had them too (28.3 -> 29.9 us; a branch 31.1).
@@ -196,9 +197,8 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     static_assert(!SPLIT || (PACKED && !BIAS && MODE == kMaskCausal), "the split over the keys serves the chunked decode");
     static_assert(!WIN || (!PACKED && !BIAS && !SPLIT && MODE == kMaskCausal), "the window is a causal mask's");
     static_assert(!HALVES || (TILES != kTilesRegs && !PACKED && !SPLIT && !WIN), "halves of the walk: tiles straight to LDS, rows of one head");
-    static_assert(TILES == kTilesRegs || DP <= 128, "tiles straight into LDS: head dims up to 128");
     constexpr bool DIRECT = TILES != kTilesRegs, WHOLE = TILES == kTilesDirect;
-    using Cfg = TileCfg<DP>;
+    using Cfg = TileCfg<DP, DIRECT>;
     constexpr int KT = Cfg::KT, LDK = Cfg::LDK, LDV = Cfg::LDV, NI = Cfg::NI, TTHREADS = Cfg::THREADS;
     constexpr int KS = DP / 16;        // contraction steps of the score product
     constexpr int DT = DP / 32;        // 32-row tiles of O^T
@@ -209,11 +209,11 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     constexpr bool kCausal = MODE == kMaskCausal;
     constexpr int PF = Cfg::PF;        // register sets of tiles in flight behind the two LDS stages
     static_assert(2 * DT == KS, "one P.V matrix instruction per score matrix instruction");
-    // Head dims above 128 do not have the registers for two score tiles and their operands in flight (O alone is 128
-    // registers), nor does head dim 128 with a key-padding mask and tiles through registers: there an item runs its three phases
-    // one after the other, and K is parked with V.
-    constexpr bool PIPE = DP <= 128 && !(MODE == kMaskPadding && DP == 128 && !DIRECT);
-    static_assert(!BIAS || DIRECT || DP > 128, "a bias up to head dim 128 comes with tiles straight to LDS");
+    // Through registers, head dims above 128 do not have those for two score tiles and their operands in flight beside the tiles'
+    // own (O alone is 128, and a wave has a SIMD to itself), nor does head dim 128 with a key-padding mask: there an item runs its
+    // three phases one after the other, and K is parked with V.
+    constexpr bool PIPE = DIRECT || DP < 128 || (DP == 128 && MODE != kMaskPadding);
+    static_assert(!BIAS || (DP <= 128) == DIRECT, "a bias comes with tiles straight to LDS up to head dim 128, through registers above");
     static_assert(PIPE || !HALVES, "the halves meet once a tile");
 
     // QLDS: the query rows come through LDS as well, whole lines an instruction, over V(1), whose request comes behind the first
@@ -321,11 +321,11 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         dl_v[n] = (uint32_t)row * kv_pitch * 2u + (uint32_t)(16 * sv);
         dl_k_on[n] = __ballot(8 * sk < D);
         dl_v_on[n] = __ballot(8 * sv < D);
-        if (DP != 96 && n > 0) {  // (the same columns, 256 / SPR rows on: known to the compiler)
-            dl_k[n] = dl_k[0] + (uint32_t)(256 / SPR * n) * kv_pitch * 2u;
-            dl_v[n] = dl_v[0] + (uint32_t)(256 / SPR * n) * kv_pitch * 2u;
-            dl_k_on[n] = dl_k_on[0];
-            dl_v_on[n] = dl_v_on[0];
+        if (n >= Lds::SETS) {  // (the same columns, rows on: known to the compiler)
+            dl_k[n] = dl_k[n % Lds::SETS] + (uint32_t)Lds::rows_on(n) * kv_pitch * 2u;
+            dl_v[n] = dl_v[n % Lds::SETS] + (uint32_t)Lds::rows_on(n) * kv_pitch * 2u;
+            dl_k_on[n] = dl_k_on[n % Lds::SETS];
+            dl_v_on[n] = dl_v_on[n % Lds::SETS];
         }
     }
     if constexpr (DIRECT && !WHOLE) {
@@ -342,10 +342,10 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
 #pragma unroll
         for (int n = 0; n < NLD; n++) {
             const uint32_t block = lds_base + half_at + stage_off + (uint32_t)Lds::block(wave, n);
-            const uint32_t lane_at = DP == 96 ? lane_off[n] : lane_off[0];
-            const uint32_t off = DP == 96 ? tile_off : tile_off + (uint32_t)(256 / SPR * n) * kv_pitch * 2u;
+            const uint32_t lane_at = lane_off[n % Lds::SETS];
+            const uint32_t off = tile_off + (uint32_t)Lds::rows_on(n) * kv_pitch * 2u;
             if constexpr (WHOLE) buffer_to_lds(rs, lane_at, off, block);
-            else buffer_to_lds_of(on[DP == 96 ? n : 0], rs, lane_at, off, block);
+            else buffer_to_lds_of(on[n % Lds::SETS], rs, lane_at, off, block);
         }
     };
     // Tile 0 (K and V) and K of tile 1 are requested before the sequence lengths have arrived (a dependent load
@@ -682,7 +682,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
             // dim must be zero.
             const int d0 = 16 * ks + 8 * hh;
             u32x4_t z = {0u, 0u, 0u, 0u};
-            if constexpr (DP <= 128) {
+            if constexpr (DP <= 128 || DIRECT) {
                 z = *(const u32x4_t*)(p.q + q_off + min(d0, D - 8));
                 if (D < DP && d0 >= D) z = u32x4_t{0u, 0u, 0u, 0u};
             } else {  // (head dim 256 has no register to spare for the clamped addresses)
@@ -1348,7 +1348,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
     }
     // (the same wave wrote and now reads: no barrier needed, the LDS queue is in order)
     const uint32_t fill2 = t_cvt_pk_bf16(fill, fill);
-    if constexpr (!PACKED && 64 % CH == 0 && DP <= 128) {
+    if constexpr (!PACKED && 64 % CH == 0 && (DP <= 128 || DIRECT)) {
         // rows of one head, and a wave's store instruction covers whole rows: lane l moves chunk l % CH of the rows
         // l / CH, l / CH + 64 / CH, ... -- one address, then a constant step
         constexpr int RS = 64 / CH;  // rows per store instruction
@@ -1987,9 +1987,8 @@ hipError_t launch_one(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
     return hipGetLastError();
 }
 
-// Tiles straight to LDS wherever the kernel has that form: head dims up to 128.
 template <int DP, int TILES>
-hipError_t launch_tiles(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
+hipError_t launch_packed(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
     if (p.n_splits > 1) {  // (rows packed over a group of one head are rows of that head)
         hipError_t e = launch_one<DP, kMaskCausal, false, true, true, false, TILES>(stream, p, grid);
         if (e != hipSuccess) return e;
@@ -1998,9 +1997,15 @@ hipError_t launch_tiles(hipStream_t stream, const FlashTileParams& p, dim3 grid)
         else hipLaunchKernelGGL(flash_split_merge_kernel<false>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, stream, p);
         return hipGetLastError();
     }
-    if (p.pack > 1 || p.decode_rows) return launch_one<DP, kMaskCausal, false, true, false, false, TILES>(stream, p, grid);
+    return launch_one<DP, kMaskCausal, false, true, false, false, TILES>(stream, p, grid);
+}
+template <int DP, int TILES>
+hipError_t launch_tiles(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
+    if (p.n_splits > 1 || p.pack > 1 || p.decode_rows) return launch_packed<DP, TILES>(stream, p, grid);
     if (p.window > 0) return launch_one<DP, kMaskCausal, false, false, false, true, TILES>(stream, p, grid);
-    if (p.bias) {
+    if constexpr (DP > 128 && TILES != kTilesRegs) {
+        if (p.bias) return hipErrorInvalidValue;  // (takes_tiles_direct)
+    } else if (p.bias) {
         if (DP == 64 && (unsigned long long)grid.x * grid.y * grid.z > 2ull * (unsigned long long)p.n_cus)
             return launch_one<DP, kMaskNone, true, false, false, false, TILES, false, DP != 64>(stream, p, grid);
         return launch_one<DP, kMaskNone, true, false, false, false, TILES>(stream, p, grid);
@@ -2040,6 +2045,18 @@ static bool takes_halves(const FlashTileParams& p, dim3 grid) {
     if (p.dim > 64) return grid.z >= 18 || (grid.z >= 11 && units % 8 == 0 && 8 * units <= n_cus && 4 * n <= 7 * n_cus);
     return grid.z >= (p.dim <= 32 ? 5 : 11);
 }
+// Head dims above 128: the pipelined walk over tiles of 64 keys straight to LDS, one workgroup a CU, or the walk over tiles of 32
+// through registers, whose phases follow one another (one wave a SIMD as well: O takes 128 registers).  The first from 96 keys a walk
+// on, 256 a span where more than two waves of a tile have rows; not with a bias, whose LDS leaves the query rows to be read into the operands and whose values spill.  us,
+// registers / LDS, B H N at head dim 256: causal 4 32 2048 410 / 338, 3 40/8 724 71.7 / 56.7, 1 8/2 1024 46.5 / 32.7, 2 16 100 11.7 / 10.5,
+// but 1 16 65 9.9 / 10.3, 1 16 40 8.4 / 8.6, 1 16 16 7.4 / 8.5; none 2 16 2048 177 / 130, a padding mask 202 / 138; window 476, 4 40/8
+// 2653 427 / 353; padded 5 8 2817 124 / 96, 9 32 1483 266 / 237; head dim 160 2 16 1100 49.7 / 39.6; with a bias 4 8 1024 57.2 / 65.0, 1 8
+// 77 x 513 38.6 / 52.1.  A chunk's positions over a cache, whole: 2 16 200 over 1500 34.0 / 29.4, 12 32/8 10 over 4314 95.0 / 91.6, 9 8 8 over
+// 20 7.8 / 9.2, 1 12 211 over 214 15.7 / 14.8, 4 32 339 over 342 33.9 / 34.4; in spans of 256 keys 1 16/2 100 over 2048 29.1 / 26.1, of 64 rows 1 32/8
+// 16 over 8192 22.2 / 22.5, of 32 keys 10.2 / 11.4.
+static bool takes_tiles_direct(const FlashTileParams& p) {
+    return !p.bias && (p.n_splits > 1 ? p.seq_kv / p.n_splits >= 256 && p.seq_q * p.pack > 64 : p.seq_kv >= 96);
+}
 template <int DP>
 hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
     if (p.mask == kMaskPadding) {
@@ -2047,11 +2064,9 @@ hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
         // a byte a lane with tiles through registers -> this, the last eighth of the keys hidden, B H N head dim: 2 12 2032 128
         // 72.7 -> 60.7 (no mask 57.0), 1 12 1866 96 43.6 -> 35.9, 3 16 1117 80 33.9 -> 29.5, 4 16 2048 64 87.5 -> 80.3, 8 16 512 64 15.6 ->
         // 14.3, 2 16 3000 32 64.3 -> 63.5.  A single tile at head dim 128 stays: 5 16 42 128 6.2, 6.4.
-        if constexpr (DP <= 128) {
-            if (p.seq_kv <= 8 * TileCfg<DP>::STAGE_BYTES && (DP < 128 || p.seq_kv > TileCfg<DP>::KT)) {
-                if (p.dim == DP) return launch_one<DP, kMaskPadding, false, false, false, false, kTilesDirect>(stream, p, grid);
-                return launch_one<DP, kMaskPadding, false, false, false, false, kTilesDirectPart>(stream, p, grid);
-            }
+        if (p.seq_kv <= 8 * TileCfg<DP>::STAGE_BYTES && (DP < 128 || (DP == 128 ? p.seq_kv > TileCfg<DP>::KT : takes_tiles_direct(p)))) {
+            if (p.dim == DP) return launch_one<DP, kMaskPadding, false, false, false, false, kTilesDirect>(stream, p, grid);
+            return launch_one<DP, kMaskPadding, false, false, false, false, kTilesDirectPart>(stream, p, grid);
         }
         return launch_one<DP, kMaskPadding, false, false>(stream, p, grid);
     }
@@ -2059,8 +2074,10 @@ hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
         constexpr int kTiles = DP % 64 == 0 ? kTilesDirect : kTilesDirectPart;
         if ((kTiles == kTilesDirectPart || p.dim == DP) && takes_halves(p, grid)) return launch_halves<DP, kTiles>(stream, p, grid);
     }
-    if constexpr (DP > 128) return launch_tiles<DP, kTilesRegs>(stream, p, grid);
-    else return p.dim == DP ? launch_tiles<DP, kTilesDirect>(stream, p, grid) : launch_tiles<DP, kTilesDirectPart>(stream, p, grid);
+    if constexpr (DP > 128) {
+        if (!takes_tiles_direct(p)) return launch_tiles<DP, kTilesRegs>(stream, p, grid);
+    }
+    return p.dim == DP ? launch_tiles<DP, kTilesDirect>(stream, p, grid) : launch_tiles<DP, kTilesDirectPart>(stream, p, grid);
 }
 
 }  // namespace

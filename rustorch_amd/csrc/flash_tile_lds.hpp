@@ -1,4 +1,4 @@
-// Where the bf16 tile kernel keeps what lies in LDS when its tiles travel straight there (head dims up to 128): plain
+// Where the bf16 tile kernel keeps what lies in LDS when its tiles travel straight there: plain
 // arithmetic, so that a host test can hold every wave's writes against each other.
 //
 //   [K stage 0][K stage 1][V stage 0][V stage 1]   a stage: KT rows of DP columns without padding
@@ -16,15 +16,19 @@ namespace rt {
 
 template <int DP>
 struct TileLds {
-    static constexpr int KT = DP <= 128 ? 64 : 32;  // keys per tile
-    static constexpr int SPR = DP / 8;              // 16-byte slots per row
+    static constexpr int KT = 64;      // keys per tile
+    static constexpr int SPR = DP / 8;  // 16-byte slots per row
     static constexpr int ROW_BYTES = 2 * DP, STAGE_BYTES = KT * ROW_BYTES;
     static constexpr int REQUESTS = KT * SPR / 256;  // load instructions per wave, matrix and tile
     static constexpr int K_AT = 0, V_AT = 2 * STAGE_BYTES, Q_AT = 3 * STAGE_BYTES, KEEP_AT = 4 * STAGE_BYTES;
     static constexpr int Q_REQUESTS = SPR / 2;  // per wave, of its own 32 query rows
 
-    static constexpr int swz_k(int row) { return DP == 128 ? (row & 15) : (DP == 64 ? ((row >> 1) & 7) : ((row >> 2) & 3)); }
-    static constexpr int swz_v(int row) { return DP == 128 ? 4 * (row & 3) : (DP == 64 ? 4 * ((row >> 1) & 1) : 0); }
+    static constexpr int swz_k(int row) { return DP >= 128 ? (row & 15) : (DP == 64 ? ((row >> 1) & 7) : ((row >> 2) & 3)); }
+    static constexpr int swz_v(int row) { return DP >= 128 ? 4 * (row & 3) : (DP == 64 ? 4 * ((row >> 1) & 1) : 0); }
+    // Instructions n and n + SETS of a wave fetch the same columns, rows_on(n + SETS) - rows_on(n) rows apart: the lane's part of
+    // the address is that of instruction n % SETS (whose own rows it holds).
+    static constexpr int SETS = DP == 96 ? REQUESTS : (DP == 256 ? 2 : 1);
+    static constexpr int rows_on(int n) { return (n - n % SETS) * 256 / SPR; }
 
     static constexpr int block(int wave, int n) { return 1024 * (wave + 4 * n); }                      // within a stage
     static constexpr int q_block(int wave, int n) { return Q_AT + wave * 32 * ROW_BYTES + 1024 * n; }

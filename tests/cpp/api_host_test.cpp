@@ -352,6 +352,7 @@ static void a_tiles_lds_has_one_writer() {
     for (int dim = 40; dim <= 64; dim += 8) one_writer<64>(dim);
     for (int dim = 72; dim <= 96; dim += 8) one_writer<96>(dim);
     for (int dim = 104; dim <= 128; dim += 8) one_writer<128>(dim);
+    for (int dim = 136; dim <= 256; dim += 8) one_writer<256>(dim);
 }
 
 // How many spans a chunk's keys are cut into, of every case of tests/test_gpu_chunk_split.py and on either side of the rule's ends.
