@@ -791,7 +791,9 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_keys
     if (wave == 0 && hh == 0) {
         const bool good = (l_all > 0.0f) && (fabsf(l_all) != __uint_as_float(0x7f800000u)) && (l_all == l_all);
         fin_inv[col] = good ? 1.0f / l_all : quiet_nan();
-        if (p.lse && q_row < Nq) p.lse[((size_t)b * p.heads + h) * (size_t)Nq + q_row] = m_all + logf(l_all);
+        if constexpr (DT > 2) {  // (head dims up to 64 keep no statistic here, and a late argument read is 0.3 us of a launch)
+            if (p.lse && q_row < Nq) p.lse[((size_t)b * p.heads + h) * (size_t)Nq + q_row] = m_all + logf(l_all);
+        }
     }
     float* const Ow = (float*)Kw;  // this wave's weighted O, as rows [col][d]
 #pragma unroll
@@ -852,7 +854,7 @@ hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p_in
 
 bool flash_f32_split_keys_supported(const FlashF32Params& p) {
     const long long keys = p.seq_kv ? p.seq_kv : p.seq;
-    return p.dim <= 128 && p.dim % 4 == 0 && (p.mask == kMaskNone || p.mask == kMaskCausal) && !p.bias && keys > 0 &&
+    return p.dim <= 128 && p.dim % 4 == 0 && (p.mask == kMaskNone || p.mask == kMaskCausal) && !p.bias && (!p.lse || p.dim > 64) && keys > 0 &&
            (unsigned long long)(keys + 256) * (unsigned long long)p.lkv.row_pitch * 4ull < (1ull << 32);  // 32-bit offsets
 }
 
