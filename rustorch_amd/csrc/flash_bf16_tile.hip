@@ -598,45 +598,49 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         // BIAS (scores = (q . k) * scale + bias, crates/rustorch-nn/src/attention.rs:378-392, kept in the natural domain so
         // that a bias of -1e4 weighs as it does in the reference): f32 rows of seq_kv per (batch, head), or one matrix for
         // all.  An item's 32 rows of 32 keys go from memory to the wave's own 4 KB of LDS as whole 128-byte pieces of a row
-        // (8 rows a load instruction, or 2 where the rows are not 16-byte aligned), and from there into the order the scores
+        // (8 rows a load instruction), and from there into the order the scores
         // sit in; the 16-byte slots of a row are XORed with bits of the row, as those of a K tile of 128-byte rows.  Read
         // from its row in memory by each lane, 16 bytes of 32 rows at a time, the bias kept the address unit busy for half
         // of the launch and the waves waiting for 54 % of theirs: B=4 H=16 T=1024 hd=64 47.4 -> 28.3 us with warm inputs and
-        // 47.3 -> 29.9 with inputs that change from pass to pass; warm, 1023 keys (4-byte requests) 93.9 -> 34.9, one matrix a
-        // head at B=4 H=16 T=770 hd=96 119 -> 58.3.  Keys behind the last one read the next row, or zeros behind the tensor:
+        // 47.3 -> 29.9 with inputs that change from pass to pass.  Keys behind the last one read the next row, or zeros behind the tensor:
         // those scores are masked.
+        // A row may start at any multiple of 4 bytes: a 16-byte request asks for no more of its address.  The one chunk that must
+        // not be asked for whole is that which ends behind the tensor: the wave of the tensor's last row takes an item that is short
+        // of 32 keys 4 bytes a lane, 2 rows an instruction.  us, every request for an unaligned tensor that way -> now, B H T head dim,
+        // one matrix for all: 4 16 1023 64 36.8 -> 33.0 (1024 keys 30.2), 13 12 1662 32 190 -> 182 (1664 144), 4 12 1662 128 113 -> 103, 1 12
+        // 161 32 7.9 -> 7.1, 4 8 1023 256 62.8 -> 58.9; one a head: 2 8 466 80 17.3 -> 15.5, 1 8 77 x 513 64 14.3 -> 12.5.
         u32x4_t bias_rsrc = {0u, 0u, 0u, 0u};
         uint32_t bias_lane[2] = {0u, 0u}, bias_at = 0, bias_step = 0;
         const uint32_t bias_lds = BIAS ? (uint32_t)(kBiasAt + (wave + 4 * half) * Cfg::BIAS_BYTES) : 0u;
-        const bool bias_vec4 = BIAS && p.bias_vec4;
+        int bias_whole = 0;      // items before it are asked for 16 bytes a lane
+        bool bias_pieces = false;  // the last item asked for was not
         if constexpr (BIAS) {
             const int r_first = q0 + 32 * wq, n_rows = max(min(32, rows_total - r_first), 0);
             const float* const bb = p.bias + ((size_t)b * p.heads + h0) * (size_t)p.bias_bh_stride + (size_t)min(r_first, rows_total - 1) * (size_t)p.seq_kv;
             const uint32_t pitch = (uint32_t)p.seq_kv * 4u, first = 4u * (uint32_t)min(half_key0, p.seq_kv);
-            bias_rsrc = make_rsrc((const char*)bb + first, n_rows > 0 ? (uint32_t)n_rows * pitch - first : 0u);
-            if (bias_vec4) {  // instruction n: rows 8 n + lane / 8
-                const int row = lane >> 3, slot = (lane & 7) ^ (row >> 1);
-                bias_lane[0] = (uint32_t)row * pitch + 16u * (uint32_t)slot;
-                bias_lane[1] = (uint32_t)row * pitch + 16u * (uint32_t)(slot ^ 4);
-                bias_step = 8u * pitch;
-            } else {  // instruction n: rows 2 n + lane / 32
-                bias_lane[0] = (uint32_t)(lane >> 5) * pitch;
-                bias_lane[1] = 4u * (uint32_t)(lane & 31);
-                bias_step = 2u * pitch;
-            }
+            const bool ends = !p.bias_vec4 && r_first + n_rows == rows_total && (p.bias_bh_stride == 0 || (b == (int)gridDim.y - 1 && h0 == p.heads - 1));
+            bias_whole = ends ? (p.seq_kv - half_key0) >> 5 : 0x7fffffff;
+            bias_rsrc = make_rsrc((const char*)bb + first, n_rows > 0 ? (uint32_t)n_rows * pitch - first + (ends || p.bias_vec4 ? 0u : 12u) : 0u);
+            // instruction n: rows 8 n + lane / 8
+            const int row = lane >> 3, slot = (lane & 7) ^ (row >> 1);
+            bias_lane[0] = (uint32_t)row * pitch + 16u * (uint32_t)slot;
+            bias_lane[1] = (uint32_t)row * pitch + 16u * (uint32_t)(slot ^ 4);
+            bias_step = 8u * pitch;
             bias_at = bias_lds + (uint32_t)(col * 128 + ((hh ^ ((col >> 1) & 7)) * 16));
         }
         auto bias_request = [&](int item) __attribute__((always_inline)) {
             const uint32_t k_off = 128u * (uint32_t)item;
-            if (bias_vec4) {
+            bias_pieces = item >= bias_whole;
+            if (__builtin_expect(!bias_pieces, 1)) {
 #pragma unroll
                 for (int n = 0; n < 4; n++)
                     buffer_to_lds(bias_rsrc, bias_lane[n & 1], k_off + (uint32_t)n * bias_step, lds_base + bias_lds + 1024u * (uint32_t)n);
-            } else {
+            } else {  // instruction n: rows 2 n + lane / 32
+                const uint32_t pitch = (uint32_t)p.seq_kv * 4u;
 #pragma unroll
                 for (int n = 0; n < 16; n++)
-                    buffer_to_lds_b32(bias_rsrc, bias_lane[0] + (bias_lane[1] ^ (16u * (uint32_t)(n & 7))), k_off + (uint32_t)n * bias_step,
-                                        lds_base + bias_lds + 256u * (uint32_t)n);
+                    buffer_to_lds_b32(bias_rsrc, (uint32_t)(lane >> 5) * pitch + ((4u * (uint32_t)(lane & 31)) ^ (16u * (uint32_t)(n & 7))), k_off + (uint32_t)(2 * n) * pitch,
+                                      lds_base + bias_lds + 256u * (uint32_t)n);
             }
         };
         auto bias_read = [&](f32x4_t (&bv)[4]) __attribute__((always_inline)) {
@@ -1120,7 +1124,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         // the tile's requests)
         auto meet = [&](auto stepped_c) __attribute__((always_inline)) {
             if constexpr (DIRECT && BIAS && decltype(stepped_c)::value) {
-                if (bias_vec4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+                if (!bias_pieces) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
                 else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
             } else if constexpr (DIRECT) {
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

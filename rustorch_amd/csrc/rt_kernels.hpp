@@ -162,7 +162,7 @@ struct FlashTileParams {
     const uint8_t* keep;      // kMaskPadding: device, seq_kv bytes
     const float* bias;        // optional additive score bias, f32 rows of seq_kv per query position, added after scaling
     long long bias_bh_stride; // elements between the biases of consecutive (batch, head) pairs; 0 = one for all
-    int bias_vec4;            // bias rows may be read 16 bytes at a time (base and seq_kv * 4 bytes both 16-byte aligned)
+    int bias_vec4;            // base and seq_kv * 4 bytes both 16-byte aligned: no 16-byte piece of a row lies partly behind the last
     float scale;              // 1/sqrt(dim)
     int ref_bc;
     int batch, heads;

@@ -101,6 +101,14 @@ def test_additive_mask_at_the_edges_of_items(oracle, d, tq, tkv, lead):
         assert_bf16_parity(got, want, d, None, f"tq={tq} tkv={tkv} d={d} lead={lead} per_head={per_head}")
 
 
+@pytest.mark.parametrize("d", [32, 64, 96, 256])
+@pytest.mark.parametrize("tq,tkv,lead", [(129, 545, 0), (64, 513, 1), (33, 770, 2), (100, 1023, 3), (40, 800, 1), (97, 831, 1)])
+def test_additive_mask_of_any_alignment_over_many_keys(oracle, d, tq, tkv, lead):
+    """Walks in two halves and whole, rows that start at any multiple of 4 bytes, a last item of 1, 2, 31 or 32 keys; what lies
+    around the mask in memory is NaN."""
+    test_additive_mask_at_the_edges_of_items(oracle, d, tq, tkv, lead)
+
+
 def test_masked_bf16_errors():
     z = ra.HipStorage(1 << 16)
     with pytest.raises(ra.DeviceError) as ei:  # head dim above 512
