@@ -195,6 +195,10 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, hh = lane >> 5;
+    // the arguments, requested together: left to itself the compiler loads a field where it is first used, and waits for it there
+    asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.out), "s"(p.lse), "s"(p.heads), "s"(p.group), "s"(p.seq), "s"(p.seq_kv), "s"(p.dim), "s"(p.scale),
+                 "s"(p.zigzag), "s"(p.dealt), "s"(p.blocks_magic), "s"(p.heads_magic), "s"(p.lq.batch_stride), "s"(p.lq.head_stride), "s"(p.lq.row_pitch));
+    asm volatile("" ::"s"(p.lkv.batch_stride), "s"(p.lkv.head_stride), "s"(p.lkv.row_pitch), "s"(p.lo.batch_stride), "s"(p.lo.head_stride), "s"(p.lo.row_pitch));
     const int Nq = p.seq, N = p.seq_kv ? p.seq_kv : p.seq;  // N: keys (== queries unless cross-attention)
     const int D = kExactD ? DPAD : p.dim;
     // Which (batch, head, query tile) this workgroup takes.  Workgroups are dealt round-robin to the 8 XCDs, each
@@ -205,19 +209,19 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
     const int nq = (int)gridDim.x, n_bh = (int)(gridDim.y * gridDim.z);
     int h = blockIdx.y, b = blockIdx.z;
     int qtile = nq - 1 - (int)blockIdx.x;
-    if ((n_bh & 7) == 0) {
+    if (p.dealt) {
         const int lin = (int)blockIdx.x + nq * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z);
         const int xcd = lin & 7, r = lin >> 3, half = (nq * (n_bh >> 3)) >> 1;
-        int bh = (r / nq) * 8 + xcd;
-        qtile = nq - 1 - r % nq;
-        if (p.zigzag && r >= half && (half % nq == 0 || nq == 2 * half)) qtile = (r - half) % nq;
-        h = bh % (int)gridDim.y;
-        b = bh / (int)gridDim.y;
+        const int at = div_magic(r, p.blocks_magic), bh = at * 8 + xcd;
+        qtile = nq - 1 - (r - at * nq);
+        if (p.zigzag && r >= half && (div_magic(half, p.blocks_magic) * nq == half || nq == 2 * half)) qtile = (r - half) - div_magic(r - half, p.blocks_magic) * nq;
+        b = div_magic(bh, p.heads_magic);
+        h = bh - b * (int)gridDim.y;
     } else if (p.zigzag && ((h + b * (int)gridDim.y) * 2 >= n_bh)) {
         qtile = (int)blockIdx.x;
     }
     const int q0 = qtile * kRows;
-    const int kvh = h / p.group;
+    const int kvh = p.group == 1 ? h : h / p.group;
     const float* __restrict__ Qg = p.q + (size_t)b * p.lq.batch_stride + (size_t)h * p.lq.head_stride;
     const float* __restrict__ Kg = p.k + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
     const float* __restrict__ Vg = p.v + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
@@ -251,17 +255,7 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
         }
     }
 
-    // Q as B operand, in registers: qreg[4j + i] = Q[q0 + col][8j + 4hh + i]
     const int q_row = q0 + col;
-    float qreg[DPAD / 2];
-#pragma unroll
-    for (int j = 0; j < DPAD / 8; j++) {
-        f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (q_row < Nq && 8 * j + 4 * hh < D) z = *(const f32x4_t*)(Qg + (size_t)q_row * q_pitch + 8 * j + 4 * hh);
-#pragma unroll
-        for (int i = 0; i < 4; i++) qreg[4 * j + i] = z[i];
-    }
-
     f32x16_t acc_o[DT];
 #pragma unroll
     for (int t = 0; t < DT; t++)
@@ -286,15 +280,13 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
     const int ld_r = lane / CH, ld_c = lane % CH;
     const bool ld_col_ok = kExactD || 4 * ld_c < D;  // this lane's 16-byte column exists
     const uint32_t ld_off = (uint32_t)ld_r * (uint32_t)kv_pitch * 4u + (uint32_t)ld_c * 16u;  // bytes; a few rows: fits
+    // A tile that is not whole goes through descriptors that end with the last key's row: a row behind it and a column behind the
+    // head dim come back as zeros without a read, and no load stands behind a test of its own.
     f32x4_t kreg[NLD], vreg[NLD];
+    const uint32_t pitch_b = (uint32_t)kv_pitch * 4u;
     auto issue_loads = [&](int tile) {
-        if constexpr (kEvenRows) {
-            if (tile * kRows + kRows <= N) {  // whole tile present (wave-uniform): no per-load bounds test
-                if (!ld_col_ok) {
-#pragma unroll
-                    for (int n = 0; n < NLD; n++) kreg[n] = vreg[n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                    return;
-                }
+        if constexpr (kEvenRows && kExactD) {
+            if (tile * kRows + kRows <= N) {  // (wave-uniform)
                 const char* kb = (const char*)Kg + (size_t)tile * kRows * kv_pitch * sizeof(float) + ld_off;
                 const char* vb = (const char*)Vg + (size_t)tile * kRows * kv_pitch * sizeof(float) + ld_off;
 #pragma unroll
@@ -306,29 +298,37 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
                 return;
             }
         }
+        const size_t base = (size_t)tile * kRows * kv_pitch;
+        const uint32_t bytes = (uint32_t)(min(N - tile * kRows, kRows) - 1) * pitch_b + 4u * (uint32_t)D;
+        const __amdgpu_buffer_rsrc_t kb = __builtin_amdgcn_make_buffer_rsrc((void*)(Kg + base), 0, bytes, kBufferFlags);
+        const __amdgpu_buffer_rsrc_t vb = __builtin_amdgcn_make_buffer_rsrc((void*)(Vg + base), 0, bytes, kBufferFlags);
 #pragma unroll
         for (int n = 0; n < NLD; n++) {
-            f32x4_t zk = {0.0f, 0.0f, 0.0f, 0.0f}, zv = zk;
+            uint32_t off, step = 0;
             if constexpr (kEvenRows) {
-                const int row0 = tile * kRows + RPL * n;  // uniform
-                const size_t base = (size_t)row0 * kv_pitch * sizeof(float);
-                if (row0 + ld_r < N && ld_col_ok) {  // rows past the end are zeros (and masked below)
-                    zk = *(const f32x4_t*)((const char*)Kg + base + ld_off);
-                    zv = *(const f32x4_t*)((const char*)Vg + base + ld_off);
-                }
+                off = ld_col_ok ? ld_off : 0x7fffffffu;
+                step = (uint32_t)(RPL * n) * pitch_b;  // uniform
             } else {
                 const int idx = 64 * n + lane, r = idx / CH, c = idx % CH;
-                const int kr = tile * kRows + r;
-                if (kr < N && 4 * c < D) {
-                    zk = *(const f32x4_t*)(Kg + (size_t)kr * kv_pitch + 4 * c);
-                    zv = *(const f32x4_t*)(Vg + (size_t)kr * kv_pitch + 4 * c);
-                }
+                off = kExactD || 4 * c < D ? (uint32_t)r * pitch_b + 16u * (uint32_t)c : 0x7fffffffu;
             }
-            kreg[n] = zk;
-            vreg[n] = zv;
+            kreg[n] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(kb, off, step, 0));
+            vreg[n] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(vb, off, step, 0));
         }
     };
     if (wave < n_tiles) issue_loads(wave);
+
+    // Q as B operand, in registers (requested behind the first tile): qreg[4j + i] = Q[q0 + col][8j + 4hh + i]
+    const float* const q_at = Qg + (size_t)min(q_row, Nq - 1) * q_pitch;  // (a row behind the last repeats it and is not written)
+    float qreg[DPAD / 2];
+#pragma unroll
+    for (int j = 0; j < DPAD / 8; j++) {
+        const int d = 8 * j + 4 * hh;
+        f32x4_t z = *(const f32x4_t*)(q_at + (kExactD ? d : min(d, D - 4)));
+        if (!kExactD && d >= D) z = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; i++) qreg[4 * j + i] = z[i];
+    }
 
     for (int tile = wave; tile < n_tiles; tile += NW) {
         const int kv0 = tile * kRows;
@@ -609,6 +609,7 @@ hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p) {
         // 8 (dim <= 64) or 4 waves fit on a CU: is every workgroup resident from the start?
         const long long resident = (long long)p.n_cus * (dt <= 2 ? 2 : 1);
         pz.zigzag = (p.mask == kMaskCausal) && ((long long)grid.x * grid.y * grid.z <= resident) ? 1 : 0;
+        deal_to_xcds(pz, grid.x);
         const bool exact = (p.dim % 32 == 0), pad = (p.mask == kMaskPadding);
         if (p.bias && p.mask != kMaskNone) return hipErrorInvalidValue;  // a bias comes without a mask kind
         if (p.lse && flash_f32_gradients_wide(p))  // the statistic of scores formed as the gradients form them

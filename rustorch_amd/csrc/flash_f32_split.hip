@@ -38,6 +38,10 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
     // tiles t and t + 1 of K, t to t + 2 of V
     __shared__ __attribute__((aligned(16))) __bf16 lds[5 * BUF];
 
+    // the arguments, requested together: left to itself the compiler loads a field where it is first used, and waits for it there
+    asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.out), "s"(p.lse), "s"(p.heads), "s"(p.group), "s"(p.seq), "s"(p.seq_kv), "s"(p.dim), "s"(p.scale),
+                 "s"(p.zigzag), "s"(p.dealt), "s"(p.blocks_magic), "s"(p.heads_magic), "s"(p.lq.batch_stride), "s"(p.lq.head_stride), "s"(p.lq.row_pitch));
+    asm volatile("" ::"s"(p.lkv.batch_stride), "s"(p.lkv.head_stride), "s"(p.lkv.row_pitch), "s"(p.lo.batch_stride), "s"(p.lo.head_stride), "s"(p.lo.row_pitch));
     const int Nq = p.seq, N = p.seq_kv ? p.seq_kv : p.seq;
     const int D = kExactD ? DPAD : p.dim;
     // p.zigzag 2 (head dims above 64): a workgroup takes two blocks of a head, a long and a short one, in turn
@@ -45,18 +49,18 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
     int h = blockIdx.y, b = blockIdx.z;
     int x = (int)blockIdx.x;
     bool short_first = false;
-    if ((n_bh & 7) == 0) {                // a head's workgroups on one XCD: its K and V come into one L2
+    if (p.dealt) {                        // a head's workgroups on one XCD: its K and V come into one L2
         const int lin = (int)blockIdx.x + nq * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z);
         const int xcd = lin & 7, r = lin >> 3, half = (nq * (n_bh >> 3)) >> 1;
-        const int bh = (r / nq) * 8 + xcd;
-        x = r % nq;
+        const int at = div_magic(r, p.blocks_magic), bh = at * 8 + xcd;
+        x = r - at * nq;
         // all resident at once: list positions r and r + half share a CU, a long one and a short one of them
-        short_first = p.zigzag == 1 && r >= half && half % nq == 0;
-        h = bh % (int)gridDim.y;
-        b = bh / (int)gridDim.y;
+        short_first = p.zigzag == 1 && r >= half && div_magic(half, p.blocks_magic) * nq == half;
+        b = div_magic(bh, p.heads_magic);
+        h = bh - b * (int)gridDim.y;
     }
     int qblk = short_first ? x : n_blk - 1 - x;  // longest causal rows first
-    const int kvh = h / p.group;
+    const int kvh = p.group == 1 ? h : h / p.group;
     const float* __restrict__ Qg = p.q + (size_t)b * p.lq.batch_stride + (size_t)h * p.lq.head_stride;
     const float* __restrict__ Kg = p.k + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
     const float* __restrict__ Vg = p.v + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
@@ -74,15 +78,17 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
         uint32_t v_least = ~0u;  // the smallest magnitude of what it splits of V, zeros left out: 2 (bits of |x|) - 1
 
         // Q as B operand: chunk j, this lane's 8 elements d = 16j + 8hh ..
+        // (rows behind the last repeat it, so that no load stands behind a test; nothing of theirs is written)
+        const float* const q_at = Qg + (size_t)min(q_row, Nq - 1) * q_pitch;
         Split8 qf[KS];
 #pragma unroll
         for (int j = 0; j < KS; j++) {
             float x[8];
 #pragma unroll
             for (int u = 0; u < 2; u++) {
-                f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
                 const int d = 16 * j + 8 * hh + 4 * u;
-                if (q_row < Nq && d < D) z = *(const f32x4_t*)(Qg + (size_t)q_row * q_pitch + d);
+                f32x4_t z = *(const f32x4_t*)(q_at + (kExactD ? d : min(d, D - 4)));
+                if (!kExactD && d >= D) z = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int i = 0; i < 4; i++) x[4 * u + i] = z[i];
             }
@@ -459,19 +465,19 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_keys
     const int nq = (int)gridDim.x, n_bh = (int)(gridDim.y * gridDim.z);
     int h = blockIdx.y, b = blockIdx.z;
     int qtile = nq - 1 - (int)blockIdx.x;
-    if ((n_bh & 7) == 0) {
+    if (p.dealt) {
         const int lin = (int)blockIdx.x + nq * ((int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z);
         const int xcd = lin & 7, r = lin >> 3, half = (nq * (n_bh >> 3)) >> 1;
-        const int bh = (r / nq) * 8 + xcd;
-        qtile = nq - 1 - r % nq;
-        if (p.zigzag && r >= half && (half % nq == 0 || nq == 2 * half)) qtile = (r - half) % nq;
-        h = bh % (int)gridDim.y;
-        b = bh / (int)gridDim.y;
+        const int at = div_magic(r, p.blocks_magic), bh = at * 8 + xcd;
+        qtile = nq - 1 - (r - at * nq);
+        if (p.zigzag && r >= half && (div_magic(half, p.blocks_magic) * nq == half || nq == 2 * half)) qtile = (r - half) - div_magic(r - half, p.blocks_magic) * nq;
+        b = div_magic(bh, p.heads_magic);
+        h = bh - b * (int)gridDim.y;
     } else if (p.zigzag && ((h + b * (int)gridDim.y) * 2 >= n_bh)) {
         qtile = (int)blockIdx.x;
     }
     const int q0 = qtile * kTile, q_row = q0 + col;
-    const int kvh = h / p.group;
+    const int kvh = p.group == 1 ? h : h / p.group;
     const float* __restrict__ Qg = p.q + (size_t)b * p.lq.batch_stride + (size_t)h * p.lq.head_stride;
     const float* __restrict__ Kg = p.k + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
     const float* __restrict__ Vg = p.v + (size_t)b * p.lkv.batch_stride + (size_t)kvh * p.lkv.head_stride;
@@ -532,15 +538,16 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_keys
 
     float chk = 0.0f;
     uint32_t v_least = ~0u;
+    const float* const q_at = Qg + (size_t)min(q_row, Nq - 1) * q_pitch;  // (as in the kernel above)
     Split8 qf[KS];
 #pragma unroll
     for (int j = 0; j < KS; j++) {
         float x[8];
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
             const int d = 16 * j + 8 * hh + 4 * u;
-            if (q_row < Nq && d < D) z = *(const f32x4_t*)(Qg + (size_t)q_row * q_pitch + d);
+            f32x4_t z = *(const f32x4_t*)(q_at + (kExactD ? d : min(d, D - 4)));
+            if (!kExactD && d >= D) z = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int i = 0; i < 4; i++) x[4 * u + i] = z[i];
         }
@@ -832,6 +839,7 @@ hipError_t launch_flash_f32_split(hipStream_t stream, const FlashF32Params& p_in
         p.zigzag = 2;
         grid.x = (grid.x + 1) / 2;
     }
+    deal_to_xcds(p, grid.x);
     auto launch = [&](auto dt_c, auto exact_c) {
         constexpr int kDT = decltype(dt_c)::value;
         constexpr bool kEx = decltype(exact_c)::value;
@@ -863,6 +871,7 @@ hipError_t launch_flash_f32_split_keys(hipStream_t stream, const FlashF32Params&
     if (!flash_f32_split_keys_supported(p)) return hipErrorInvalidValue;
     dim3 grid((p.seq + kTile - 1) / kTile, p.heads, p.batch), block(256);
     p.zigzag = (p.mask == kMaskCausal) && ((long long)grid.x * grid.y * grid.z <= (p.dim <= 64 ? 2ll : 1ll) * p.n_cus) ? 1 : 0;
+    deal_to_xcds(p, grid.x);
     auto launch = [&](auto dt_c, auto exact_c) {
         constexpr int kDT = decltype(dt_c)::value;
         constexpr bool kEx = decltype(exact_c)::value;

@@ -93,6 +93,9 @@ __device__ __forceinline__ u32x4_t make_rsrc(const void* base, uint32_t bytes) {
 template <typename T>
 __device__ __forceinline__ void store_past(void* dst, T v) { __builtin_nontemporal_store(v, (T*)dst); }
 
+// x / d by the multiplier 2^32 / d + 1 (exact where x d < 2^32), or by one for the multiplier 0
+__device__ __forceinline__ int div_magic(int x, uint32_t magic) { return magic ? (int)__umulhi((uint32_t)x, magic) : x; }
+
 // Value held by the lane 32 positions away (the other half of the wave).
 __device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32, 64); }
 

@@ -45,7 +45,21 @@ struct FlashF32Params {
     long long bias_bh_stride;  // elements between the biases of consecutive (batch, head) pairs; 0 = one for all
     // optional [batch, heads, seq] output: the row statistic m + ln(l) of the softmax (what a backward pass needs)
     float* lse;
+    // set by the launcher: 2^32 / d + 1 of the blocks a head and of `heads`, for divisions by a multiply where (batch, head) pairs
+    // are dealt to the eight XCDs (`dealt`; 0 for a division by one)
+    uint32_t blocks_magic, heads_magic;
+    int dealt;
 };
+// The same, for `blocks` workgroups a head: where the pairs divide by eight and the multiplies are exact.  (A division is a
+// chain of twenty dependent instructions ahead of a workgroup's first request: four of them 0.2 us.)
+inline void deal_to_xcds(FlashF32Params& p, unsigned blocks) {
+    const unsigned long long n_bh = (unsigned long long)p.heads * (unsigned long long)p.batch, d = 1ull << 32;
+    p.dealt = 0;
+    if (n_bh % 8 != 0 || (unsigned long long)blocks * blocks * (n_bh / 8) >= d || n_bh * (unsigned long long)p.heads >= d) return;
+    p.blocks_magic = blocks > 1 ? (uint32_t)(d / blocks) + 1u : 0u;
+    p.heads_magic = p.heads > 1 ? (uint32_t)(d / (unsigned long long)p.heads) + 1u : 0u;
+    p.dealt = 1;
+}
 // dim <= 256 (the tiled four-wave kernel up to 128).  Returns hipErrorInvalidValue for an unsupported dim.
 hipError_t launch_flash_f32(hipStream_t stream, const FlashF32Params& p);
 // The form on the bf16 matrix cores: dim <= 128 and a multiple of 4, 16-byte aligned rows, mask none or causal, no bias.
