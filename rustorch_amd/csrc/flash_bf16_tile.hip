@@ -613,14 +613,13 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         uint32_t bias_lane[2] = {0u, 0u}, bias_at = 0, bias_step = 0;
         const uint32_t bias_lds = BIAS ? (uint32_t)(kBiasAt + (wave + 4 * half) * Cfg::BIAS_BYTES) : 0u;
         int bias_whole = 0;      // items before it are asked for 16 bytes a lane
-        bool bias_pieces = false;  // the last item asked for was not
         if constexpr (BIAS) {
             const int r_first = q0 + 32 * wq, n_rows = max(min(32, rows_total - r_first), 0);
             const float* const bb = p.bias + ((size_t)b * p.heads + h0) * (size_t)p.bias_bh_stride + (size_t)min(r_first, rows_total - 1) * (size_t)p.seq_kv;
             const uint32_t pitch = (uint32_t)p.seq_kv * 4u, first = 4u * (uint32_t)min(half_key0, p.seq_kv);
             const bool ends = !p.bias_vec4 && r_first + n_rows == rows_total && (p.bias_bh_stride == 0 || (b == (int)gridDim.y - 1 && h0 == p.heads - 1));
             bias_whole = ends ? (p.seq_kv - half_key0) >> 5 : 0x7fffffff;
-            bias_rsrc = make_rsrc((const char*)bb + first, n_rows > 0 ? (uint32_t)n_rows * pitch - first + (ends || p.bias_vec4 ? 0u : 12u) : 0u);
+            bias_rsrc = make_rsrc((const char*)bb + first, n_rows > 0 ? (uint32_t)n_rows * pitch - first + (ends || p.bias_vec4 ? 0u : min(12u, pitch)) : 0u);
             // instruction n: rows 8 n + lane / 8
             const int row = lane >> 3, slot = (lane & 7) ^ (row >> 1);
             bias_lane[0] = (uint32_t)row * pitch + 16u * (uint32_t)slot;
@@ -630,8 +629,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         }
         auto bias_request = [&](int item) __attribute__((always_inline)) {
             const uint32_t k_off = 128u * (uint32_t)item;
-            bias_pieces = item >= bias_whole;
-            if (__builtin_expect(!bias_pieces, 1)) {
+            if (__builtin_expect(item < bias_whole, 1)) {
 #pragma unroll
                 for (int n = 0; n < 4; n++)
                     buffer_to_lds(bias_rsrc, bias_lane[n & 1], k_off + (uint32_t)n * bias_step, lds_base + bias_lds + 1024u * (uint32_t)n);
@@ -1124,8 +1122,7 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
         // the tile's requests)
         auto meet = [&](auto stepped_c) __attribute__((always_inline)) {
             if constexpr (DIRECT && BIAS && decltype(stepped_c)::value) {
-                if (!bias_pieces) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-                else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+                asm volatile("s_waitcnt vmcnt(4)" ::: "memory");  // (of a last item's sixteen pieces it waits for twelve)
             } else if constexpr (DIRECT) {
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             }

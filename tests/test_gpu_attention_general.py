@@ -102,10 +102,11 @@ def test_additive_mask_at_the_edges_of_items(oracle, d, tq, tkv, lead):
 
 
 @pytest.mark.parametrize("d", [32, 64, 96, 256])
-@pytest.mark.parametrize("tq,tkv,lead", [(129, 545, 0), (64, 513, 1), (33, 770, 2), (100, 1023, 3), (40, 800, 1), (97, 831, 1)])
+@pytest.mark.parametrize("tq,tkv,lead", [(129, 545, 0), (64, 513, 1), (33, 770, 2), (100, 1023, 3), (40, 800, 1), (97, 831, 1), (33, 1, 1), (65, 2, 3),
+                                           (34, 3, 1)])
 def test_additive_mask_of_any_alignment_over_many_keys(oracle, d, tq, tkv, lead):
-    """Walks in two halves and whole, rows that start at any multiple of 4 bytes, a last item of 1, 2, 31 or 32 keys; what lies
-    around the mask in memory is NaN."""
+    """Walks in two halves and whole, rows that start at any multiple of 4 bytes, a last item of 1, 2, 31 or 32 keys, rows shorter
+    than a request with a single one behind a wave's; what lies around the mask in memory is NaN."""
     test_additive_mask_at_the_edges_of_items(oracle, d, tq, tkv, lead)
 
 
