@@ -1395,65 +1395,77 @@ __global__ __launch_bounds__(HALVES ? 512 : TileCfg<DP>::THREADS, HALVES ? 2 : B
 // kernel would have written the row.  No partial with a key (every m is -inf): the position sees no key at all, a row
 // of zeros.  A wave takes eight columns of 32 rows, as the partials hold them: 1 KB a load, and a lane's weights are its
 // own row's.  With many partials the four waves of a workgroup share them out (PARTS) and meet in LDS: a wave has eight
-// loads of each kind in flight, and a latency for every eight is what the kernel takes.
+// loads of each kind in flight, and a latency for every eight is what the kernel takes, beside what stands ahead of the
+// first of them: the grid is (columns, row block, (sequence, kv head)) and the arguments are the kernel's own, so that
+// no division and no second round of argument loads does; partials behind the last are zeros by the descriptor, no branch.  us
+// of the whole call, before -> now, new positions over context: 32 / 8 heads of 128, 16 over 8192 14.76 -> 14.45, 4 x 8 over 1024 12.25 ->
+// 11.62; 28 / 4 of 128, 4 over 300 8.75 -> 8.27; 2 x 16 / 2 of 256, 5 over 3000 15.73 -> 15.40.
+struct SplitMergeParams {
+    const float *part_o, *part_ml;
+    int n, dim, blocks, rows;  // partials, head dim, blocks of 32 rows and rows of a (sequence, kv head)
+    uint16_t* out;
+    long long batch_stride, head_stride, row_pitch;
+    int pack, kv_heads;
+    uint32_t pack_magic, kv_magic;  // div_magic
+};
+
 template <bool PARTS>
-__global__ __launch_bounds__(256) void flash_split_merge_kernel(FlashTileParams p) {
+__global__ __launch_bounds__(256) void flash_split_merge_kernel(SplitMergeParams p) {
     constexpr int kGroup = 8;
     __shared__ float fold[PARTS ? 3 : 1][6][64];
-    const int D = p.dim, G = p.pack, n = p.n_splits, lane = threadIdx.x % 64;
+    const int D = p.dim, n = p.n, lane = threadIdx.x % 64;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const uint32_t rows_total = (uint32_t)p.seq_q * (uint32_t)G, blocks = (rows_total + 31) / 32, pieces = (uint32_t)D / 8;
-    const uint32_t item = PARTS ? blockIdx.x : 4 * blockIdx.x + wave;
-    if (item >= (uint32_t)p.batch * (uint32_t)p.kv_heads * blocks * pieces) return;  // (PARTS: one item per workgroup, all there)
-    const uint32_t block = item / pieces, piece = item - block * pieces, bk = block / blocks;
-    const uint32_t r = (block - bk * blocks) * 32 + (lane & 31);
-    const uint32_t b = bk / (uint32_t)p.kv_heads, kvh = bk - b * (uint32_t)p.kv_heads;
-    const bool row_in = r < rows_total;
-    const float* const ml = p.part_ml + (size_t)block * n * 64 + (lane & 31);
-    const float* const po = p.part_o + (size_t)block * n * (32 * D) + 256 * piece + 4 * lane;
+    const uint32_t piece = PARTS ? blockIdx.x : 4 * blockIdx.x + wave;
+    asm volatile("" ::"s"(p.part_o), "s"(p.part_ml), "s"(n), "s"(D), "s"(p.blocks), "s"(p.out), "s"(p.batch_stride), "s"(p.head_stride), "s"(p.row_pitch), "s"(p.pack), "s"(p.kv_heads),
+                 "s"(p.pack_magic), "s"(p.kv_magic), "s"(p.rows));  // (loaded in one go)
+    if (!PARTS && piece >= (uint32_t)D / 8) return;
+    const size_t block = (size_t)(blockIdx.z * (uint32_t)p.blocks + blockIdx.y) * (uint32_t)n;
+    const uint32_t o_bytes = 128u * (uint32_t)D;
+    const __amdgpu_buffer_rsrc_t ml = __builtin_amdgcn_make_buffer_rsrc((void*)(p.part_ml + block * 64), 0, (uint32_t)n * 256u, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t po = __builtin_amdgcn_make_buffer_rsrc((void*)(p.part_o + block * (uint32_t)(32 * D)), 0, (uint32_t)n * o_bytes, kBufferFlags);
+    const uint32_t ml_lane = 4u * (uint32_t)(lane & 31), po_lane = 1024u * piece + 16u * (uint32_t)lane;
 
     constexpr int STEP = PARTS ? 4 : 1;
     float m_all = neg_inf(), l_all = 0.0f;
     f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
     bool nan_m = false;
-    if (row_in) {
-        for (int k0 = PARTS ? (int)wave : 0; k0 < n; k0 += kGroup * STEP) {
-            float mv[kGroup], lv[kGroup];
-            f32x4_t ov[kGroup];
+    int k0 = PARTS ? (int)wave : 0;  // (below n: PARTS comes with more than eight)
+    do {
+        float mv[kGroup], lv[kGroup];
+        f32x4_t ov[kGroup];
 #pragma unroll
-            for (int j = 0; j < kGroup; j++) {
-                const int k = k0 + STEP * j;
-                mv[j] = neg_inf();
-                lv[j] = 0.0f;
-                ov[j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                if (k < n) {
-                    mv[j] = ml[64 * k];
-                    lv[j] = ml[64 * k + 32];
-                    ov[j] = *(const f32x4_t*)(po + (size_t)k * (32 * D));
-                }
-            }
-            float m_new = m_all;
-#pragma unroll
-            for (int j = 0; j < kGroup; j++) {
-                m_new = fmaxf(m_new, mv[j]);
-                nan_m |= mv[j] != mv[j];
-            }
-            const float m_use = m_new == neg_inf() ? 0.0f : m_new;
-            const float rescale = m_all == neg_inf() ? 0.0f : __builtin_amdgcn_exp2f(m_all - m_use);
-            l_all *= rescale;
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[e] *= rescale;
-#pragma unroll
-            for (int j = 0; j < kGroup; j++) {
-                // an empty partial (m = -inf) is the identity
-                const float w = mv[j] == neg_inf() ? 0.0f : __builtin_amdgcn_exp2f(mv[j] - m_use);
-                l_all += lv[j] * w;
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[e] += ov[j][e] * w;
-            }
-            m_all = m_new;
+        for (int j = 0; j < kGroup; j++) {
+            const uint32_t k = (uint32_t)(k0 + STEP * j);
+            mv[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ml, ml_lane + 256u * k, 0, 0));
+            lv[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ml, ml_lane + 256u * k + 128u, 0, 0));
+            ov[j] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(po, po_lane + o_bytes * k, 0, 0));
         }
-    }
+        __builtin_amdgcn_sched_barrier(0);  // (all on their way before the first is awaited)
+#pragma unroll
+        for (int j = 0; j < kGroup; j++)
+            if (k0 + STEP * j >= n) mv[j] = neg_inf();
+        float m_new = m_all;
+#pragma unroll
+        for (int j = 0; j < kGroup; j++) {
+            m_new = fmaxf(m_new, mv[j]);
+            nan_m |= mv[j] != mv[j];
+        }
+        const float m_use = m_new == neg_inf() ? 0.0f : m_new;
+        const float rescale = m_all == neg_inf() ? 0.0f : __builtin_amdgcn_exp2f(m_all - m_use);
+        l_all *= rescale;
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[e] *= rescale;
+#pragma unroll
+        for (int j = 0; j < kGroup; j++) {
+            // an empty partial (m = -inf) is the identity
+            const float w = mv[j] == neg_inf() ? 0.0f : __builtin_amdgcn_exp2f(mv[j] - m_use);
+            l_all += lv[j] * w;
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[e] += ov[j][e] * w;
+        }
+        m_all = m_new;
+        k0 += kGroup * STEP;
+    } while (k0 < n);
     if constexpr (PARTS) {
         if (wave > 0) {
             fold[wave - 1][0][lane] = nan_m ? __builtin_nanf("") : m_all;
@@ -1483,10 +1495,11 @@ __global__ __launch_bounds__(256) void flash_split_merge_kernel(FlashTileParams 
         }
         m_all = m_new;
     }
-    if (!row_in) return;
-    const uint32_t s_pos = r / (uint32_t)G, g = r - s_pos * (uint32_t)G;
-    uint16_t* const dst = p.out + (size_t)b * p.lo.batch_stride + (size_t)(kvh * G + g) * p.lo.head_stride +
-                          (size_t)s_pos * p.lo.row_pitch + 8 * piece + 4 * (lane >> 5);
+    const int r = (int)blockIdx.y * 32 + (lane & 31), bk = (int)blockIdx.z;
+    if (r >= p.rows) return;
+    const int b = div_magic(bk, p.kv_magic), kvh = bk - b * p.kv_heads, s_pos = div_magic(r, p.pack_magic), g = r - s_pos * p.pack;
+    uint16_t* const dst = p.out + (size_t)b * p.batch_stride + (size_t)(kvh * p.pack + g) * p.head_stride + (size_t)s_pos * p.row_pitch +
+                          8 * piece + 4 * (lane >> 5);
     uint2 x = make_uint2(0u, 0u);
     if (m_all != neg_inf() || nan_m) {
         x.x = (uint32_t)f32_to_bf16_bits(acc[0] / l_all) | (uint32_t)f32_to_bf16_bits(acc[1] / l_all) << 16;
@@ -1993,9 +2006,13 @@ hipError_t launch_packed(hipStream_t stream, const FlashTileParams& p, dim3 grid
     if (p.n_splits > 1) {  // (rows packed over a group of one head are rows of that head)
         hipError_t e = launch_one<DP, kMaskCausal, false, true, true, false, TILES>(stream, p, grid);
         if (e != hipSuccess) return e;
-        const size_t items = (size_t)p.batch * p.kv_heads * (((size_t)p.seq_q * p.pack + 31) / 32) * (size_t)(p.dim / 8);
-        if (p.n_splits > 8) hipLaunchKernelGGL(flash_split_merge_kernel<true>, dim3((unsigned)items), dim3(256), 0, stream, p);
-        else hipLaunchKernelGGL(flash_split_merge_kernel<false>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, stream, p);
+        auto magic = [](int d) { return d > 1 ? (uint32_t)(0x100000000ull / (unsigned)d) + 1u : 0u; };
+        const int rows = p.seq_q * p.pack, blocks = (rows + 31) / 32, pieces = p.dim / 8;
+        const SplitMergeParams m{p.part_o, p.part_ml, p.n_splits, p.dim, blocks, rows, p.out, p.lo.batch_stride, p.lo.head_stride, p.lo.row_pitch,
+                                 p.pack, p.kv_heads, magic(p.pack), magic(p.kv_heads)};
+        const dim3 at((unsigned)(p.n_splits > 8 ? pieces : (pieces + 3) / 4), (unsigned)blocks, (unsigned)(p.batch * p.kv_heads));
+        if (p.n_splits > 8) hipLaunchKernelGGL(flash_split_merge_kernel<true>, at, dim3(256), 0, stream, m);
+        else hipLaunchKernelGGL(flash_split_merge_kernel<false>, at, dim3(256), 0, stream, m);
         return hipGetLastError();
     }
     return launch_one<DP, kMaskCausal, false, true, false, false, TILES>(stream, p, grid);
@@ -2157,6 +2174,10 @@ hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& par
     if (p.n_splits < 1) p.n_splits = 1;
     if (p.n_splits > 1 && (p.pack != p.group || p.bias || p.mask != kMaskCausal || !p.part_o || !p.part_ml))
         return hipErrorInvalidValue;  // the chunked decode only
+    // (what is cut leaves CUs idle: fewer than 2^15 rows and slabs.  The merge's grid, its offsets and its divisions need no more.)
+    if (p.n_splits > 1 && ((long long)p.batch * p.kv_heads > 65535 || (rows + 31) / 32 > 65535 || rows * (long long)p.pack >= 1ll << 32 ||
+                           (long long)p.batch * p.kv_heads * p.kv_heads >= 1ll << 32 || (long long)p.n_splits * p.dim >= 1ll << 25))
+        return hipErrorInvalidValue;
     if (p.batch > 65535 || n_qtiles * p.n_splits > 65535 || heads_u > 65535 || p.group < 1) return hipErrorInvalidValue;  // grid limits
     set_grid_order(p, n_qtiles * p.n_splits);
     if (tiles_by_length(p, n_qtiles)) p.n_qtiles = -1;
