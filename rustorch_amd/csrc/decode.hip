@@ -559,7 +559,10 @@ __global__ __launch_bounds__(64) void decode_split_kernel(DecodeSplitParams p) {
 // whose partials the workgroup that finishes last folds.  Bound by its chain of waits: 4.2 us for one split (arguments,
 // rows, products, fold of the waves), 3 us more for a fold across workgroups (stores out, counter, loads back).  32 / 8
 // heads of 128, us per call, before (split + merge kernel) and now: 4 sequences of 64-512 16.7 / 8.1, 128 of 32-256
-// 26.7 / 17.9, one of 2048 9.3 / 8.5.
+// 26.7 / 17.9, one of 2048 9.3 / 8.5.  Ahead of the first row stand one round of argument loads and the length, no division; q
+// is asked for before either.  When q followed the rows, by lanes of the group only, its second half was not asked for until the
+// rows and the first half were there: 8 sequences of 100-1000, 32 / 8 of 128 10.03 -> 9.11, 2 of 30-900, 16 of 256 14.19 -> 12.84, 128 of
+// 32-500, 16 / 2 of 64 6.62 -> 6.53.
 constexpr int kLatWaves = 4;
 constexpr int kLatMaxSplits = 24;
 static_assert(kLatMaxSplits <= 64, "the fold gives every split a lane, a segment's word eight bits of count");
@@ -578,22 +581,30 @@ __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSp
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int hcol = lane & 15, g4 = lane >> 4;
     const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
-    const int G = p.heads / p.kv_heads;
+    // (the arguments in one go, q ahead of the length and without a branch, which would have its two loads wait for the rows)
+    asm volatile("" ::"s"(p.q), "s"(p.k_cache), "s"(p.v_cache), "s"(p.out), "s"(p.kv_lens), "s"(p.kv_len), "s"(p.ws), "s"(p.batch), "s"(p.heads), "s"(p.kv_heads),
+                 "s"(p.max_seq), "s"(p.scale_log2e), "s"(p.n_splits), "s"(p.launch_id), "s"(p.group), "s"(p.splits_magic));
+    const int G = p.group;
     const int seg = b * p.kv_heads + kvh;
     const uint32_t n_slots = (uint32_t)p.batch * p.heads * p.n_splits, ml_byte = n_slots * HD * 4;
+    const __amdgpu_buffer_rsrc_t q_rs = __builtin_amdgcn_make_buffer_rsrc((void*)(p.q + (size_t)seg * G * HD), 0, 2 * G * HD, kBufferFlags);
+    bf16x8_t qreg[T::KS];  // (zeros beyond the group)
+#pragma unroll
+    for (int ks = 0; ks < T::KS; ks++)
+        qreg[ks] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(q_rs, 2 * (hcol * HD + 32 * ks + 8 * g4), 0, 0));
     SegWord word;
     if (tid == 0 && p.n_splits > 1)
         word.request((word_t*)((unsigned char*)p.ws + (size_t)n_slots * (HD + 2) * 4 + (size_t)seg * kWordPitch), p.launch_id);
-    const int len = dec_len(p, b), steps = dec_steps(len);
-    const int per = max((steps + p.n_splits - 1) / p.n_splits, kLatWaves);
-    const int n_act = (steps + per - 1) / per;  // splits that hold keys
+    __builtin_amdgcn_sched_barrier(0);
+    const int len = min(max(p.kv_lens ? *(const __attribute__((address_space(4))) int32_t*)(p.kv_lens + b) : p.kv_len, 0), p.max_seq), steps = dec_steps(len);
+    const int per = max(div_magic(steps + p.n_splits - 1, p.splits_magic), kLatWaves);
     uint16_t* const out = p.out + (size_t)seg * G * HD;
-    if (split >= n_act) {
+    if (split * per >= steps) {
         if (steps == 0 && split == 0)  // no key: rows of zeros (gqa.rs:261; llm_kernels.rs:456)
             for (int i = tid; i < G * HD / 4; i += NT) *(u32x2_t*)(out + 4 * i) = u32x2_t{0u, 0u};
         return;
     }
-    const bool counts = tid == 0 && n_act > 1;
+    const bool counts = tid == 0 && steps > per;
     const int t1 = min(steps, (split + 1) * per);
     uint16_t* const Kw = (uint16_t*)lds + wave * T::HALFS;
     uint16_t* const Vw = Kw + kDecRows * T::LDK;
@@ -604,9 +615,7 @@ __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSp
     int t = split * per + wave;
     if (t < t1) {  // (so it is for wave 0)
         u32x4_t kreg[T::NLD], vreg[T::NLD];
-        bf16x8_t qreg[T::KS];
         dec_load<HD>(p, b, kvh, t, len, lane, kreg, vreg);
-        dec_load_q<HD>(p, b, kvh, lane, qreg);
         if (counts) word.replace();
         for (; t < t1; t += kLatWaves) {
             dec_park<HD>(Kw, Vw, lane, kreg, vreg);
@@ -615,6 +624,7 @@ __global__ __launch_bounds__(64 * kLatWaves) void decode_latency_kernel(DecodeSp
         }
     }
 
+    const int n_act = (steps + per - 1) / per;  // splits that hold keys
     // ---- fold the four waves
     const float l_wave = state.l_total(), m_wave = state.m * c;  // exp2 domain from here on
     if (g4 == 0) {
@@ -824,7 +834,10 @@ __global__ __launch_bounds__(256) void kv_block_append_kernel(T* __restrict__ k_
 template <int HD>
 hipError_t launch_split_hd(hipStream_t stream, const DecodeSplitParams& p) {
     if (p.n_splits > 0) {
-        hipLaunchKernelGGL(decode_latency_kernel<HD>, dim3(p.n_splits, p.kv_heads, p.batch), dim3(64 * kLatWaves), 0, stream, p);
+        DecodeSplitParams lp = p;
+        lp.group = p.heads / p.kv_heads;
+        lp.splits_magic = p.n_splits > 1 ? (uint32_t)((1ull << 32) / (unsigned)p.n_splits) + 1u : 0u;
+        hipLaunchKernelGGL(decode_latency_kernel<HD>, dim3(p.n_splits, p.kv_heads, p.batch), dim3(64 * kLatWaves), 0, stream, lp);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(decode_split_kernel<HD>, dim3(p.n_waves), dim3(64), 0, stream, p);

@@ -267,6 +267,9 @@ struct DecodeSplitParams {
     // 0: the split kernel followed by the merge kernel.
     int n_splits;
     uint64_t launch_id;
+    // set by the launcher for the latency form: heads / kv_heads, and n_splits as a multiplier (div_magic: 24 splits of 2^26 steps are exact)
+    int group;
+    uint32_t splits_magic;
 };
 bool decode_split_supported(int heads, int kv_heads, int dim);
 int decode_split_span_min(int batch);
