@@ -21,55 +21,68 @@ namespace {
 
 constexpr int kPrepMaxD = 512;
 
-// grid (n_heads + n_kv, seq, batch), one wave per head row; lane l holds the pairs (k, k + D/2), k = l + 64 j.  What
-// bounds a decode step's launch is its chain of waits, so everything it reads is requested at once (the row, gamma, the
-// table row, V) and the one serial part, the sum of squares in index order, adds squares that the lanes have formed in
-// parallel, four per LDS read: 3.4 -> 2.9 us for 32 + 8 heads of 128.
-constexpr int kPrepPairs = kPrepMaxD / 2 / kWave;
+// grid (n_heads + n_kv, seq, batch), one wave per head row; lane l holds the pairs (k, k + D/2), k = l + 64 j, j < PAIRS.  What
+// bounds a decode step's launch is its chain of waits, so everything it reads is requested at once (the arguments in one go; then
+// the row, gamma and V, which no position is needed for, then the table row) and the one serial part, the sum of squares in index
+// order, adds squares that the lanes have formed in parallel, four per LDS read.  The requests go through descriptors: what a lane
+// or a head does not have (pairs behind the last, gamma, V beside q) is a zero and no branch.  Where each pair stood behind a test, the
+// second waited for the first, and V for the row: in a recorded graph, us a launch, 32 + 8 heads of 128 2.56 -> 2.26, without gamma 1.95 ->
+// 1.88, 64 sequences of them 3.43 -> 3.06, 16 + 2 of 256 3.29 -> 2.96.
+template <int PAIRS>
 __global__ __launch_bounds__(64) void decode_prepare_kernel(DecodePrepareParams p) {
-    __shared__ __attribute__((aligned(16))) float squares[kPrepMaxD];
+    __shared__ __attribute__((aligned(16))) float squares[2 * PAIRS * kWave];
     const int lane = threadIdx.x;
     const int h = blockIdx.x, sq = blockIdx.y, b = blockIdx.z;
+    asm volatile("" ::"s"(p.q), "s"(p.k_in), "s"(p.v_in), "s"(p.k_cache), "s"(p.v_cache), "s"(p.positions), "s"(p.q_gamma), "s"(p.k_gamma), "s"(p.cos_table), "s"(p.sin_table),
+                 "s"(p.eps), "s"(p.pos), "s"(p.seq), "s"(p.n_heads), "s"(p.n_kv), "s"(p.head_dim), "s"(p.max_seq), "s"(p.table_rows));
     const int D = p.head_dim, half = D / 2, S = p.seq;
-    const int pos0 = p.positions ? p.positions[b] : p.pos;
-    // a sequence whose rows would leave the cache or the tables writes nothing (the host checks a scalar position;
-    // positions that live on the device are the caller's to keep in range)
-    if (pos0 < 0 || pos0 + S > p.max_seq || pos0 + S > p.table_rows) return;
-    const int pos = pos0 + sq;
     const bool is_q = h < p.n_heads;
     const int kvh = h - p.n_heads;
     const size_t q_row = (((size_t)b * p.n_heads + h) * S + sq) * D;
     const size_t kv_row = (((size_t)b * p.n_kv + kvh) * S + sq) * D;
-    const size_t cache_row = (((size_t)b * p.n_kv + kvh) * (size_t)p.max_seq + (size_t)pos) * D;
-    const uint16_t* src = is_q ? p.q + q_row : p.k_in + kv_row;
     const float* gamma = is_q ? p.q_gamma : p.k_gamma;
-    const float* cs = p.cos_table + (size_t)pos * half;
-    const float* sn = p.sin_table + (size_t)pos * half;
+    auto rows = [](const void* base, int bytes) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, kBufferFlags); };
+    const __amdgpu_buffer_rsrc_t src = rows(is_q ? p.q + q_row : p.k_in + kv_row, 2 * D), gm = rows(gamma, gamma ? 4 * D : 0),
+                                 vs = rows(is_q ? p.q : p.v_in + kv_row, is_q ? 0 : 2 * D);
+    auto bf16_at = [](__amdgpu_buffer_rsrc_t rs, int k) { return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, 2 * k, 0, 0); };
+    auto f32_at = [](__amdgpu_buffer_rsrc_t rs, int k) { return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, 4 * k, 0, 0)); };
 
-    float x0[kPrepPairs], x1[kPrepPairs], c[kPrepPairs], si[kPrepPairs], g0[kPrepPairs], g1[kPrepPairs];
-    uint16_t v0[kPrepPairs], v1[kPrepPairs];
+    float x0[PAIRS], x1[PAIRS], c[PAIRS], si[PAIRS], g0[PAIRS], g1[PAIRS];
+    uint16_t r0[PAIRS], r1[PAIRS], v0[PAIRS], v1[PAIRS];
 #pragma unroll
-    for (int j = 0; j < kPrepPairs; j++) {
+    for (int j = 0; j < PAIRS; j++) {
         const int k = lane + kWave * j;
-        if (k >= half) break;
-        x0[j] = bf16_bits_to_f32(src[k]);
-        x1[j] = bf16_bits_to_f32(src[k + half]);
-        if (gamma) {
-            g0[j] = gamma[k];
-            g1[j] = gamma[k + half];
-        }
-        c[j] = cs[k];
-        si[j] = sn[k];
-        if (!is_q) {
-            v0[j] = p.v_in[kv_row + k];
-            v1[j] = p.v_in[kv_row + k + half];
-        }
+        r0[j] = bf16_at(src, k);
+        r1[j] = bf16_at(src, k + half);
+        g0[j] = f32_at(gm, k);
+        g1[j] = f32_at(gm, k + half);
+        v0[j] = bf16_at(vs, k);
+        v1[j] = bf16_at(vs, k + half);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int pos0 = p.positions ? *(const __attribute__((address_space(4))) int32_t*)(p.positions + b) : p.pos;
+    // a sequence whose rows would leave the cache or the tables writes nothing (the host checks a scalar position;
+    // positions that live on the device are the caller's to keep in range)
+    if (pos0 < 0 || pos0 + S > p.max_seq || pos0 + S > p.table_rows) return;
+    const int pos = pos0 + sq;
+    const size_t cache_row = (((size_t)b * p.n_kv + kvh) * (size_t)p.max_seq + (size_t)pos) * D;
+    const __amdgpu_buffer_rsrc_t cs = rows(p.cos_table + (size_t)pos * half, 4 * half), sn = rows(p.sin_table + (size_t)pos * half, 4 * half);
+#pragma unroll
+    for (int j = 0; j < PAIRS; j++) {
+        c[j] = f32_at(cs, lane + kWave * j);
+        si[j] = f32_at(sn, lane + kWave * j);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (all on their way before the first is awaited)
+#pragma unroll
+    for (int j = 0; j < PAIRS; j++) {
+        x0[j] = bf16_bits_to_f32(r0[j]);
+        x1[j] = bf16_bits_to_f32(r1[j]);
     }
     if (gamma) {
         // rms_norm_inplace (model.rs:862-885): sq accumulates in index order; every lane walks the whole row (broadcast
         // reads), which keeps the reference's summation order without a serial section
 #pragma unroll
-        for (int j = 0; j < kPrepPairs; j++) {
+        for (int j = 0; j < PAIRS; j++) {
             const int k = lane + kWave * j;
             if (k >= half) break;
             squares[k] = x0[j] * x0[j];
@@ -89,15 +102,14 @@ __global__ __launch_bounds__(64) void decode_prepare_kernel(DecodePrepareParams 
         const float inv_d = 1.0f / (float)D;
         const float inv_rms = 1.0f / sqrtf(sum * inv_d + p.eps);
 #pragma unroll
-        for (int j = 0; j < kPrepPairs; j++) {
-            if (lane + kWave * j >= half) break;
+        for (int j = 0; j < PAIRS; j++) {
             x0[j] = x0[j] * inv_rms * g0[j];
             x1[j] = x1[j] * inv_rms * g1[j];
         }
     }
     uint16_t* dst = is_q ? p.q + q_row : p.k_cache + cache_row;
 #pragma unroll
-    for (int j = 0; j < kPrepPairs; j++) {
+    for (int j = 0; j < PAIRS; j++) {
         const int k = lane + kWave * j;
         if (k >= half) break;
         dst[k] = f32_to_bf16_bits(x0[j] * c[j] - x1[j] * si[j]);
@@ -255,7 +267,10 @@ hipError_t launch_decode_prepare(hipStream_t stream, const DecodePrepareParams& 
         }
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(decode_prepare_kernel, dim3(p.n_heads + p.n_kv, p.seq, p.batch), dim3(64), 0, stream, p);
+    const dim3 grid(p.n_heads + p.n_kv, p.seq, p.batch), block(64);
+    if (p.head_dim <= 2 * kWave) hipLaunchKernelGGL(decode_prepare_kernel<1>, grid, block, 0, stream, p);
+    else if (p.head_dim <= 4 * kWave) hipLaunchKernelGGL(decode_prepare_kernel<2>, grid, block, 0, stream, p);
+    else hipLaunchKernelGGL(decode_prepare_kernel<kPrepMaxD / 2 / kWave>, grid, block, 0, stream, p);
     return hipGetLastError();
 }
 

@@ -53,6 +53,13 @@ def test_matches_oracle_bit_for_bit(oracle, norms, b_, hq, hkv, d, lmax):
     _run(oracle, rope, oro, q, k, v, kc, vc, qg, kg, positions, b_, hq, hkv, d, lmax, 1e-6)
 
 
+@pytest.mark.parametrize("norms", [(True, True), (False, False), (False, True)])
+@pytest.mark.parametrize("d", [2, 126, 128, 130, 254, 256, 510, 512])
+def test_head_dims_at_the_edges_of_a_lanes_pairs(oracle, norms, d):
+    """One, two and four pairs a lane, the last of them for every lane, for some and for one."""
+    test_matches_oracle_bit_for_bit(oracle, norms, 3, 4, 2, d, 12)
+
+
 @pytest.mark.parametrize("norms", [(True, True), (False, False), (True, False)])
 @pytest.mark.parametrize("b_,hq,hkv,d,lmax,seq", [(2, 3, 1, 16, 24, 5), (2, 8, 2, 128, 700, 300), (1, 4, 4, 64, 64, 64),
                                                   (2, 4, 2, 256, 400, 257), (1, 2, 1, 96, 1100, 1024), (2, 2, 2, 72, 80, 40),
