@@ -206,39 +206,36 @@ __device__ __forceinline__ size_t dec_slots(const DecodeSplitParams& p) {
                      : (size_t)p.batch * p.heads * p.n_part;
 }
 
-__device__ __forceinline__ int wave_sum_i(int x) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
-    return x;
-}
-__device__ __forceinline__ int wave_incl_scan_i(int x, int lane) {
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        int y = __shfl_up(x, off, 64);
-        if (lane >= off) x += y;
-    }
+// x summed up to and with each lane, the lanes of a row of 16 first, then across rows (no LDS: a sum by shuffles took 0.3 us, and
+// the kernels below had three behind one another)
+__device__ __forceinline__ int wave_incl_scan_i(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15, into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31, into rows 2 and 3
     return x;
 }
 
-// Steps of all sequences (each counted kv_heads times) and the span every wave takes.
-__device__ __forceinline__ void dec_total(const DecodeSplitParams& p, int lane, int& total, int& span) {
-    int t = 0;
-    for (int r = 0; r < p.batch; r += 64) {
-        int i = r + lane;
-        t += wave_sum_i(i < p.batch ? p.kv_heads * dec_steps(dec_len(p, i)) : 0);
-    }
-    total = t;
-    span = max((t + p.n_waves - 1) / p.n_waves, p.span_min);
+// Both kernels of the split decode read the lengths once and sum them once for all that they need of them.  Read and summed for the
+// total, for the place of a sequence and for its own length in turn, the calls took, us, before -> now: 64 sequences of 512-8192, 32 / 8
+// heads of 128 178.6 -> 177.5, 128 of 200-1500 81.1 -> 78.8, 100 of 500-4000, 16 / 2 of 64 26.5 -> 24.9; recorded, one of 2048 8.43 -> 7.70, one of
+// 8192, 16 / 2 of 256 16.3 -> 15.0.
+// The lengths of the 64 sequences from r on, a lane each (zero behind the last), and their steps (each counted kv_heads
+// times), each and summed up.
+struct DecLens {
+    int len, steps, incl;
+};
+__device__ __forceinline__ DecLens dec_lens(const DecodeSplitParams& p, int lane, int r) {
+    DecLens x;
+    x.len = r + lane < p.batch ? dec_len(p, r + lane) : 0;
+    x.steps = p.kv_heads * dec_steps(x.len);
+    x.incl = wave_incl_scan_i(x.steps);
+    return x;
 }
-// First step (in the flat list) of sequence b.
-__device__ __forceinline__ int dec_seq_start(const DecodeSplitParams& p, int lane, int b) {
-    int t = 0;
-    for (int r = 0; r < b; r += 64) {
-        int i = r + lane;
-        t += wave_sum_i(i < b ? p.kv_heads * dec_steps(dec_len(p, i)) : 0);
-    }
-    return t;
-}
+// The span every wave takes of `total` steps.
+__device__ __forceinline__ int dec_span(const DecodeSplitParams& p, int total) { return max((total + p.n_waves - 1) / p.n_waves, p.span_min); }
 
 // Geometry of a wave's private LDS tile, and the step both decode kernels run on it.
 template <int HD>
@@ -457,8 +454,10 @@ __global__ __launch_bounds__(64) void decode_split_kernel(DecodeSplitParams p) {
     const int G = p.heads / p.kv_heads;
     const int Hkv = p.kv_heads;
 
-    int total, span;
-    dec_total(p, lane, total, span);
+    const DecLens head = dec_lens(p, lane, 0);
+    int total = __builtin_amdgcn_readlane(head.incl, 63);
+    for (int r = 64; r < p.batch; r += 64) total += __builtin_amdgcn_readlane(dec_lens(p, lane, r).incl, 63);
+    const int span = dec_span(p, total);
     const int first = w * span;
     const int last = min(total, first + span);
     if (first >= last) return;
@@ -467,22 +466,18 @@ __global__ __launch_bounds__(64) void decode_split_kernel(DecodeSplitParams p) {
     DecCursor cur;
     int seq_start;  // flat index of the first step of sequence cur.b
     {
-        int base = 0, b = 0, found_start = 0;
-        for (int r = 0; r < p.batch; r += 64) {
-            int i = r + lane;
-            int st = i < p.batch ? Hkv * dec_steps(dec_len(p, i)) : 0;
-            int incl = wave_incl_scan_i(st, lane) + base;
-            int cnt = __popcll(__ballot(i < p.batch && incl <= first));  // sequences of this round that end before `first`
-            if (cnt < 64) {
-                b = r + cnt;
-                found_start = cnt == 0 ? base : __shfl(incl, cnt - 1, 64);
-                break;
-            }
-            base = __shfl(incl, 63, 64);
+        DecLens x = head;
+        int base = 0, r = 0, cnt;
+        for (;;) {
+            cnt = __popcll(__ballot(base + x.incl <= first));  // sequences of this round that end at or before `first`; lanes
+            if (cnt < 64) break;                               // behind the last repeat the total, which is above it
+            base += __builtin_amdgcn_readlane(x.incl, 63);
+            r += 64;
+            x = dec_lens(p, lane, r);
         }
-        cur.b = b;
-        seq_start = found_start;
-        cur.len_b = dec_len(p, b);
+        cur.b = r + cnt;
+        seq_start = base + __builtin_amdgcn_readlane(x.incl, cnt) - __builtin_amdgcn_readlane(x.steps, cnt);
+        cur.len_b = __builtin_amdgcn_readlane(x.len, cnt);
         cur.steps_b = dec_steps(cur.len_b);
         int local = first - seq_start;
         cur.kvh = local / cur.steps_b;
@@ -729,12 +724,22 @@ __global__ __launch_bounds__((HD < 64 ? 64 : HD) * NS) void decode_merge_kernel(
     constexpr int TD = HD < 64 ? 64 : HD;  // threads per sub-state
     const int h = blockIdx.x, b = blockIdx.y, d = threadIdx.x % TD, sub = threadIdx.x / TD;
     const int lane = threadIdx.x & 63;
+    asm volatile("" ::"s"(p.out), "s"(p.kv_lens), "s"(p.kv_len), "s"(p.ws), "s"(p.batch), "s"(p.heads), "s"(p.kv_heads), "s"(p.max_seq), "s"(p.n_part), "s"(p.span_min),
+                 "s"(p.n_waves), "s"(p.compact));  // (loaded in one go)
+    __builtin_amdgcn_sched_barrier(0);
     const int G = p.heads / p.kv_heads;
     const int kvh = h / G;
-    int total, span;
-    dec_total(p, lane, total, span);
-    const int steps_b = dec_steps(dec_len(p, b));
-    const int seg_first = dec_seq_start(p, lane, b) + kvh * steps_b;
+    int total = 0, seq_start = 0, len_b = 0;
+    for (int r = 0; r < p.batch; r += 64) {
+        const DecLens x = dec_lens(p, lane, r);
+        if ((unsigned)(b - r) < 64u) {
+            len_b = __builtin_amdgcn_readlane(x.len, b - r);
+            seq_start = total + __builtin_amdgcn_readlane(x.incl, b - r) - __builtin_amdgcn_readlane(x.steps, b - r);
+        }
+        total += __builtin_amdgcn_readlane(x.incl, 63);
+    }
+    const int span = dec_span(p, total), steps_b = dec_steps(len_b);
+    const int seg_first = seq_start + kvh * steps_b;
     const int w_first = seg_first / span;
     const int n_valid = steps_b > 0 ? (seg_first + steps_b - 1) / span - w_first + 1 : 0;
     const float* ws_o = p.ws;

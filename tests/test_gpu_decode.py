@@ -122,6 +122,26 @@ def test_gqa_decode_batched_matches_oracle(oracle, b, hq, hkv, d, max_seq, lens)
             assert (g4[i] == 0).all()
 
 
+def test_split_decode_of_more_sequences_than_lanes(oracle):
+    """Lengths summed 64 at a time: sequences without keys on either side of a round's edge, at both ends and for a whole round,
+    and batches that end with a round, one behind it and in the middle of the third."""
+    hq, hkv, d, max_seq = 4, 2, 64, 2600
+    kb, _ = bf16_round(seeded_normal((130, hkv, max_seq, d), 2))
+    vb, _ = bf16_round(seeded_normal((130, hkv, max_seq, d), 3))
+    for b, none in ((130, [0, 63, 64, 129]), (130, range(64, 128)), (130, range(0, 65)), (128, [127]), (65, [])):
+        lens = np.random.default_rng(b).integers(1, 400, size=b)
+        lens[b // 2] = max_seq
+        lens[list(none)] = 0
+        lens[1] = 33 if 1 not in none else 0
+        qb, _ = bf16_round(seeded_normal((b, hq, d), 1))
+        n = b * hkv * max_seq * d
+        k, v = kb.reshape(-1)[:n], vb.reshape(-1)[:n]
+        got = run_batched(oracle, qb, k, v, lens, b, hq, hkv, d, max_seq)
+        want = oracle.gqa_decode_batched_bf16(qb, k, v, np.asarray(lens, dtype=np.int32), b, hq, hkv, d, max_seq)
+        assert_decode_parity(got, want, d, f"b={b} none={list(none)}")
+        assert not got.reshape(b, -1)[list(none)].any()
+
+
 def test_decode_split_equals_unsplit(oracle):
     """Split-K invariance: the batched (chunked) path and the single-pass reference call agree for
     lengths on both sides of every chunk boundary."""
