@@ -141,97 +141,135 @@ __device__ __forceinline__ void put16(__amdgpu_buffer_rsrc_t rs, uint32_t byte, 
 // DMAX; every pointer 16-byte aligned.  Grid (token blocks, heads, batch), token blocks fastest: workgroups go round-robin
 // to the 8 XCDs in that order, so all heads of a token block run on one XCD and its cos / sin rows are fetched into one
 // L2, once (with the heads fastest every XCD fetched every table row: 76 MB more on the prompt above).
+// A thread asks for its rows and V at once and for the tables in two halves, the second in the rows' registers: 62 at DMAX 128, so that a
+// CU holds eight workgroups (with all tables at once 74, six of them, which 1 x 3000 tokens notice).  One chunk behind the other,
+// each with a division ahead of it, and the tables behind the sums: us, 4 x 4096 tokens, 32 / 8 heads of 128 80.3 -> 71.5, without gamma 72.4 ->
+// 69.5, 1 x 1000 9.9 -> 8.3, 1 x 100 6.3 -> 5.3; 4 x 16 / 2 of 256, 4096 86.7 -> 66.6.
 template <int ROWS, int DMAX, bool kPast>
 __global__ __launch_bounds__(256) void prompt_prepare_kernel(DecodePrepareParams p) {
+    constexpr int NC = ROWS * DMAX / 8 / 256, NP = NC / 2;  // 16-byte chunks of the rows, and pairs of them, a thread takes
     __shared__ uint32_t rows_w[ROWS * (DMAX + 2) / 2];
     __shared__ float inv[ROWS];
+    __shared__ alignas(16) float gam[DMAX];
     const int tid = threadIdx.x;
     const int h = blockIdx.y, b = blockIdx.z;
+    asm volatile("" ::"s"(p.q), "s"(p.k_in), "s"(p.v_in), "s"(p.k_cache), "s"(p.v_cache), "s"(p.positions), "s"(p.q_gamma), "s"(p.k_gamma), "s"(p.cos_table), "s"(p.sin_table),
+                 "s"(p.eps), "s"(p.pos), "s"(p.seq), "s"(p.n_heads), "s"(p.n_kv), "s"(p.head_dim), "s"(p.max_seq), "s"(p.table_rows), "s"(p.chunk_magic), "s"(p.pair_magic));
     const int sq0 = (int)blockIdx.x * ROWS;
     const int D = p.head_dim, half = D / 2, S = p.seq;
     const int pitch_w = (D + 2) / 2;  // words per row in LDS
     const int CH = D / 8;             // 16-byte chunks per row
-    const int pos0 = p.positions ? p.positions[b] : p.pos;
-    if (pos0 < 0 || pos0 + S > p.max_seq || pos0 + S > p.table_rows) return;  // as in the one-wave kernel
+    const int HP = half / 8;          // chunk pairs (k .. k + 8, k + half .. k + half + 8) per row
+    if (sq0 >= S) return;
     const int n_rows = min(ROWS, S - sq0);
     const bool is_q = h < p.n_heads;
     const int kvh = h - p.n_heads;
     const size_t q_row = (((size_t)b * p.n_heads + h) * S + sq0) * D;
     const size_t kv_row = (((size_t)b * p.n_kv + kvh) * S + sq0) * D;
-    const uint16_t* src = is_q ? p.q + q_row : p.k_in + kv_row;
     const float* gamma = is_q ? p.q_gamma : p.k_gamma;
+    const int row_bytes = n_rows * D * 2;
+    auto rsrc = [](const void* base, int bytes) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, kBufferFlags); };
+    const __amdgpu_buffer_rsrc_t src = rsrc(is_q ? p.q + q_row : p.k_in + kv_row, row_bytes), gm = rsrc(gamma, gamma ? 4 * D : 0),
+                                 vs = rsrc(is_q ? p.q : p.v_in + kv_row, is_q ? 0 : row_bytes);
+    u32x4_t x[NC], v[NC];  // chunk c = tid + 256 i of the block's rows, which follow one another
+#pragma unroll
+    for (int i = 0; i < NC; i++) x[i] = __builtin_amdgcn_raw_buffer_load_b128(src, 16 * (tid + 256 * i), 0, 0);
+    const float g = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(gm, 4 * tid, 0, 0));
+#pragma unroll
+    for (int i = 0; i < NC; i++) v[i] = __builtin_amdgcn_raw_buffer_load_b128(vs, 16 * (tid + 256 * i), 0, kPast ? 2 : 0);
+    __builtin_amdgcn_sched_barrier(0);
+    const int pos0 = p.positions ? *(const __attribute__((address_space(4))) int32_t*)(p.positions + b) : p.pos;
+    if (pos0 < 0 || pos0 + S > p.max_seq || pos0 + S > p.table_rows) return;  // as in the one-wave kernel
+    const size_t table_row = (size_t)(pos0 + sq0) * half, cache_row = (((size_t)b * p.n_kv + kvh) * (size_t)p.max_seq + (size_t)(pos0 + sq0)) * D;
+    const __amdgpu_buffer_rsrc_t cs = rsrc(p.cos_table + table_row, row_bytes), sn = rsrc(p.sin_table + table_row, row_bytes);  // (half as many, twice as wide)
+    f32x4_t ct[NP][2], st[NP][2];  // of pair c = tid + 256 i: eight values of each table, which follow one another likewise
+    auto tables = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            ct[i][e] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(cs, 32 * (tid + 256 * i) + 16 * e, 0, 0));
+            st[i][e] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sn, 32 * (tid + 256 * i) + 16 * e, 0, 0));
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < NP / 2; i++) tables(i);
+    __builtin_amdgcn_sched_barrier(0);  // (all on their way before the first is awaited)
 
-    for (int c = tid; c < n_rows * CH; c += 256) {
-        const int r = c / CH, ch = c - r * CH;
-        const u32x4_t v = *(const u32x4_t*)(src + (size_t)r * D + 8 * ch);
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+        const int c = tid + 256 * i;
+        if (c >= n_rows * CH) break;
+        const int r = (int)(((uint32_t)c * p.chunk_magic) >> 20), ch = c - r * CH;
         uint32_t* w = rows_w + r * pitch_w + 4 * ch;  // (rows start on odd words: four 4-byte writes)
-        w[0] = v[0];
-        w[1] = v[1];
-        w[2] = v[2];
-        w[3] = v[3];
+        w[0] = x[i][0];
+        w[1] = x[i][1];
+        w[2] = x[i][2];
+        w[3] = x[i][3];
     }
+    if (tid < DMAX) gam[tid] = g;
+    __builtin_amdgcn_sched_barrier(0);  // (these in the rows' registers)
+#pragma unroll
+    for (int i = NP / 2; i < NP; i++) tables(i);
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
+    if (!is_q) {
+        const __amdgpu_buffer_rsrc_t vd = rsrc(p.v_cache + cache_row, row_bytes);
+#pragma unroll
+        for (int i = 0; i < NC; i++) put16<kPast>(vd, 16u * (uint32_t)(tid + 256 * i), v[i]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     if (gamma) {
         for (int r = tid; r < n_rows; r += 256) {
             const uint32_t* w = rows_w + r * pitch_w;
             float sq = 0.0f;
             for (int j = 0; j < half; j++) {  // elements 2j and 2j + 1, in index order
-                const uint32_t x = w[j];
-                const float v0 = bf16_lo(x), v1 = bf16_hi(x);
+                const uint32_t y = w[j];
+                const float v0 = bf16_lo(y), v1 = bf16_hi(y);
                 sq = sq + v0 * v0;
                 sq = sq + v1 * v1;
             }
             const float inv_d = 1.0f / (float)D;
             inv[r] = 1.0f / sqrtf(sq * inv_d + p.eps);
         }
-        __syncthreads();
     }
-    uint16_t* dst = is_q ? p.q + q_row
-                         : p.k_cache + (((size_t)b * p.n_kv + kvh) * (size_t)p.max_seq + (size_t)(pos0 + sq0)) * D;
-    const __amdgpu_buffer_rsrc_t dst_rs = __builtin_amdgcn_make_buffer_rsrc(dst, 0, (uint32_t)(n_rows * D) * 2u, kBufferFlags);
-    const int HP = half / 8;  // chunk pairs (k .. k + 8, k + half .. k + half + 8) per row
-    for (int c = tid; c < n_rows * HP; c += 256) {
-        const int r = c / HP, k0 = 8 * (c - r * HP);
+    if (gamma) __syncthreads();
+    const __amdgpu_buffer_rsrc_t dst = rsrc(is_q ? p.q + q_row : p.k_cache + cache_row, row_bytes);
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        const int c = tid + 256 * i;
+        if (c >= n_rows * HP) break;
+        const int r = (int)(((uint32_t)c * p.pair_magic) >> 20), k0 = 8 * (c - r * HP);
         const uint32_t* w = rows_w + r * pitch_w;
         float x0[8], x1[8];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const uint32_t a = w[k0 / 2 + e], bb = w[(half + k0) / 2 + e];
-            x0[2 * e] = bf16_lo(a);
-            x0[2 * e + 1] = bf16_hi(a);
-            x1[2 * e] = bf16_lo(bb);
-            x1[2 * e + 1] = bf16_hi(bb);
+            const uint32_t y = w[k0 / 2 + e], z = w[(half + k0) / 2 + e];
+            x0[2 * e] = bf16_lo(y);
+            x0[2 * e + 1] = bf16_hi(y);
+            x1[2 * e] = bf16_lo(z);
+            x1[2 * e + 1] = bf16_hi(z);
         }
         if (gamma) {
             const float inv_rms = inv[r];
-            const f32x4_t g0a = *(const f32x4_t*)(gamma + k0), g0b = *(const f32x4_t*)(gamma + k0 + 4);
-            const f32x4_t g1a = *(const f32x4_t*)(gamma + half + k0), g1b = *(const f32x4_t*)(gamma + half + k0 + 4);
+            auto times = [&](float (&y)[8], const float* at) __attribute__((always_inline)) {
+                const f32x4_t ga = *(const f32x4_t*)at, gb = *(const f32x4_t*)(at + 4);
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                x0[e] = x0[e] * inv_rms * (e < 4 ? g0a[e] : g0b[e - 4]);
-                x1[e] = x1[e] * inv_rms * (e < 4 ? g1a[e] : g1b[e - 4]);
-            }
+                for (int e = 0; e < 8; e++) y[e] = y[e] * inv_rms * (e < 4 ? ga[e] : gb[e - 4]);
+            };
+            times(x0, gam + k0);
+            __builtin_amdgcn_sched_barrier(0);
+            times(x1, gam + half + k0);
         }
-        const size_t trow = (size_t)(pos0 + sq0 + r) * half + k0;
-        const f32x4_t ca = *(const f32x4_t*)(p.cos_table + trow), cb = *(const f32x4_t*)(p.cos_table + trow + 4);
-        const f32x4_t sa = *(const f32x4_t*)(p.sin_table + trow), sb = *(const f32x4_t*)(p.sin_table + trow + 4);
         u32x4_t o0, o1;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int i0 = 2 * e, i1 = 2 * e + 1;
-            const float c0 = i0 < 4 ? ca[i0] : cb[i0 - 4], c1 = i1 < 4 ? ca[i1] : cb[i1 - 4];
-            const float s0 = i0 < 4 ? sa[i0] : sb[i0 - 4], s1 = i1 < 4 ? sa[i1] : sb[i1 - 4];
+            const float c0 = ct[i][i0 / 4][i0 % 4], c1 = ct[i][i1 / 4][i1 % 4], s0 = st[i][i0 / 4][i0 % 4], s1 = st[i][i1 / 4][i1 % 4];
             o0[e] = pack_bf16x2(x0[i0] * c0 - x1[i0] * s0, x0[i1] * c1 - x1[i1] * s1);
             o1[e] = pack_bf16x2(x1[i0] * c0 + x0[i0] * s0, x1[i1] * c1 + x0[i1] * s1);
         }
-        put16<kPast>(dst_rs, (uint32_t)(r * D + k0) * 2u, o0);
-        put16<kPast>(dst_rs, (uint32_t)(r * D + half + k0) * 2u, o1);
-    }
-    if (!is_q) {
-        const uint16_t* vs = p.v_in + kv_row;
-        uint16_t* vd = p.v_cache + (((size_t)b * p.n_kv + kvh) * (size_t)p.max_seq + (size_t)(pos0 + sq0)) * D;
-        const __amdgpu_buffer_rsrc_t vd_rs = __builtin_amdgcn_make_buffer_rsrc(vd, 0, (uint32_t)(n_rows * D) * 2u, kBufferFlags);
-        for (int c = tid; c < n_rows * CH; c += 256) put16<kPast>(vd_rs, 16u * (uint32_t)c, kPast ? __builtin_nontemporal_load((const u32x4_t*)(vs + 8 * (size_t)c)) : *(const u32x4_t*)(vs + 8 * (size_t)c));
+        put16<kPast>(dst, (uint32_t)(r * D + k0) * 2u, o0);
+        put16<kPast>(dst, (uint32_t)(r * D + half + k0) * 2u, o1);
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -250,20 +288,28 @@ hipError_t launch_decode_prepare(hipStream_t stream, const DecodePrepareParams& 
                          aligned16(p.sin_table) && aligned16(p.q_gamma) && aligned16(p.k_gamma) && p.n_heads + p.n_kv <= 65535;
     if (wide_ok) {
         // past the caches from twice what the L2s hold, 8 of 4 MB.  us, plainly / past, inputs that change from pass to pass, 32 / 8
-        // heads of 128, caches as long as the prompt, caches of 8192 tokens: 1 x 70 tokens (0.8 MB) 6.3 / 7.3; 1 x 3000 (37 MB)
-        // 16.1 / 18.5, 16.1 / 18.3; 1 x 4096 (50 MB) 20.8 / 22.4, 21.0 / 22.6; 4 x 1024 (50 MB) 21.8 / 26.0, 29.4 / 26.2; 8 x 1024, head dim
-        // 64 (50 MB) 19.6 / 25.1, 24.1 / 25.4; 2 x 3000 (74 MB) 37.5 / 34.7, 37.4 / 34.4; 16 x 512 (101 MB) 50.9 / 45.3, 48.6 / 45.6; 4 x
-        // 4096 (201 MB) 91.2 / 79.5, 92.5 / 80.3.  Between the copies that bring the inputs and the attention that reads the rows it is
-        // level at every one of these sizes (4 x 4096 639.0 / 638.3, 16 x 512 137.0 / 136.8, 2 x 3000 210.0 / 211.7)
+        // heads of 128: 1 x 2000 tokens (25 MB) 11.2 / 12.8; 1 x 3000 (37 MB) 16.4 / 19.7; 1 x 4096 (50 MB) 17.9 / 22.7; 4 x 1024 (50 MB) 17.9 /
+        // 22.8; 8 x 16 / 16 of 64, 1024 (50 MB) 20.3 / 23.1; of 256, 4 x 16 / 2, 2500 (51 MB) 41.8 / 41.8, 4 x 8 / 8, 1100 (54 MB) 27.7 / 27.0.
+        // Before a thread asked for all its rows at once: 2 x 3000 (74 MB) 37.5 / 34.7, 16 x 512 (101 MB) 50.9 / 45.3, 4 x 4096 (201 MB) 91.2 /
+        // 79.5; between the copies that bring the inputs and the attention that reads the rows level at every one of these sizes
         const double written = 2.0 * p.batch * p.seq * (double)p.head_dim * (p.n_heads + 2.0 * p.n_kv);
         const bool past = written > 64.0 * (1 << 20);
-        const dim3 grid((p.seq + 63) / 64, p.n_heads + p.n_kv, p.batch), block(256);
+        // Token blocks up to a multiple of eight, so that every head's land on the XCD that has their table rows (those behind the
+        // last token end at once), where that adds a fifth at most.  us, as they are / so, 1 x 32 / 8 heads of 128: 550 tokens (9 blocks)
+        // 6.5 / 7.4, 1100 (18) 8.8 / 9.3, 1300 (21) 10.5 / 9.9, 2200 (35) 13.4 / 12.8, 2600 (41) 14.7 / 13.9, 3000 (47) 16.4 / 14.6.
+        int blocks = (p.seq + 63) / 64;
+        const int eights = (blocks + 7) / 8 * 8;
+        if (5 * (eights - blocks) <= blocks) blocks = eights;
+        const dim3 grid(blocks, p.n_heads + p.n_kv, p.batch), block(256);
+        DecodePrepareParams pp = p;
+        pp.chunk_magic = (1u << 20) / (uint32_t)(p.head_dim / 8) + 1u;  // (exact: c d < 2^20)
+        pp.pair_magic = (1u << 20) / (uint32_t)(p.head_dim / 16) + 1u;
         if (p.head_dim <= 128) {
-            if (past) hipLaunchKernelGGL((prompt_prepare_kernel<64, 128, true>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((prompt_prepare_kernel<64, 128, false>), grid, block, 0, stream, p);
+            if (past) hipLaunchKernelGGL((prompt_prepare_kernel<64, 128, true>), grid, block, 0, stream, pp);
+            else hipLaunchKernelGGL((prompt_prepare_kernel<64, 128, false>), grid, block, 0, stream, pp);
         } else {
-            if (past) hipLaunchKernelGGL((prompt_prepare_kernel<64, 256, true>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((prompt_prepare_kernel<64, 256, false>), grid, block, 0, stream, p);
+            if (past) hipLaunchKernelGGL((prompt_prepare_kernel<64, 256, true>), grid, block, 0, stream, pp);
+            else hipLaunchKernelGGL((prompt_prepare_kernel<64, 256, false>), grid, block, 0, stream, pp);
         }
         return hipGetLastError();
     }

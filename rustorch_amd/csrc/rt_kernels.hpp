@@ -313,6 +313,7 @@ struct DecodePrepareParams {
     float eps;
     int pos;
     int batch, seq, n_heads, n_kv, head_dim, max_seq, table_rows;
+    uint32_t chunk_magic, pair_magic;  // set by the launcher of a prompt: 2^20 / d + 1 of a row's 16-byte chunks, and of half of them
 };
 // head_dim even and <= 512; seq, batch <= 65535
 hipError_t launch_decode_prepare(hipStream_t stream, const DecodePrepareParams& p);

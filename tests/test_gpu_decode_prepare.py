@@ -63,7 +63,9 @@ def test_head_dims_at_the_edges_of_a_lanes_pairs(oracle, norms, d):
 @pytest.mark.parametrize("norms", [(True, True), (False, False), (True, False)])
 @pytest.mark.parametrize("b_,hq,hkv,d,lmax,seq", [(2, 3, 1, 16, 24, 5), (2, 8, 2, 128, 700, 300), (1, 4, 4, 64, 64, 64),
                                                   (2, 4, 2, 256, 400, 257), (1, 2, 1, 96, 1100, 1024), (2, 2, 2, 72, 80, 40),
-                                                  (1, 6, 2, 32, 40, 33), (3, 2, 1, 128, 31, 31)])
+                                                  (1, 6, 2, 32, 40, 33), (3, 2, 1, 128, 31, 31),
+                                                  # rows of fewer chunks than a thread's share, a last block of one token; blocks up to eight
+                                                  (2, 3, 1, 80, 500, 449), (1, 2, 2, 144, 140, 129), (2, 2, 1, 240, 1400, 1345)])
 def test_several_new_tokens_match_oracle_bit_for_bit(oracle, b_, hq, hkv, d, lmax, seq, norms):
     """A prompt: [batch, heads, seq, head_dim] inputs, token s at position p + s and cache row p + s.  From 32 tokens
     on, head dims that are a multiple of 16 up to 256 take the kernel that moves 64 consecutive tokens of a head
