@@ -290,8 +290,8 @@ hipError_t launch_decode_prepare(hipStream_t stream, const DecodePrepareParams& 
         // past the caches from twice what the L2s hold, 8 of 4 MB.  us, plainly / past, inputs that change from pass to pass, 32 / 8
         // heads of 128: 1 x 2000 tokens (25 MB) 11.2 / 12.8; 1 x 3000 (37 MB) 16.4 / 19.7; 1 x 4096 (50 MB) 17.9 / 22.7; 4 x 1024 (50 MB) 17.9 /
         // 22.8; 8 x 16 / 16 of 64, 1024 (50 MB) 20.3 / 23.1; of 256, 4 x 16 / 2, 2500 (51 MB) 41.8 / 41.8, 4 x 8 / 8, 1100 (54 MB) 27.7 / 27.0.
-        // Before a thread asked for all its rows at once: 2 x 3000 (74 MB) 37.5 / 34.7, 16 x 512 (101 MB) 50.9 / 45.3, 4 x 4096 (201 MB) 91.2 /
-        // 79.5; between the copies that bring the inputs and the attention that reads the rows level at every one of these sizes
+        // 1 x 5500 (68 MB) 27.9 / 29.2; 2 x 3000 (74 MB) 31.3 / 31.4; 16 x 512 (101 MB) 43.1 / 38.8; 4 x 4096 (201 MB) 79.5 / 71.7.  Before a
+        // thread asked for all its rows at once it was level between the copies that bring the inputs and the attention that reads the rows
         const double written = 2.0 * p.batch * p.seq * (double)p.head_dim * (p.n_heads + 2.0 * p.n_kv);
         const bool past = written > 64.0 * (1 << 20);
         // Token blocks up to a multiple of eight, so that every head's land on the XCD that has their table rows (those behind the
