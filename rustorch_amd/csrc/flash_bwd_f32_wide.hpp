@@ -22,6 +22,14 @@ namespace {
 
 enum Role { kDQ, kDK, kDV };  // the gradient of a workgroup's rows
 
+// dK and dV: dS and P are split at 2^17 times their size, so that whatever f32 holds of them (2^-126 on) keeps 24 bits.  The last term of a
+// split meets the smallest bf16 below 2^-109, and the rows of a key that every query weighs with 2^-123 were off by 2^-12 of themselves, where f32
+// leaves 2^-18 (the exponent's rounding).  (A row of dQ has weights that sum to one, beside which such small ones are nothing.)  dS has the
+// factor in its scale, P takes 16 multiplies a tile: grads, us, without / with, B H N head dim: 8 16 96 128 41.9 / 42.0, 8 16 96 96 35.1 / 35.7, 4 16 453
+// 80 137.7 / 138.1, 16 16 64 128 52.0 / 52.3.  What goes in stays below 2^27 for it: 2^(3 x 27 + 7) of a product of three over the head dim, times a
+// scale below 2^-3 and 2^17, is below 2^125 over the 2^23 rows that 2 GiB hold.
+constexpr float kLift = 0x1p17f, kWideMost = 0x1p27f;
+
 template <int DT>
 constexpr int kWideHalfs = 6 * Stream<DT>::SIZE;  // three tiles of either streamed matrix
 
@@ -185,7 +193,7 @@ __device__ __forceinline__ void bwd_role(const FlashBwdF32Params& p, int lin, in
             y_in.store(ybuf(i), tid, chk);
         }
     }
-    const bool uncarried = __syncthreads_or(!(chk < kSplitMost));  // seen already: no step of the loop below
+    const bool uncarried = __syncthreads_or(!(chk < kWideMost));  // seen already: no step of the loop below
     f32x16_t s;
     if (!uncarried) {
         x_in.load(kAhead, place, tid);
@@ -198,6 +206,7 @@ __device__ __forceinline__ void bwd_role(const FlashBwdF32Params& p, int lin, in
     // A step: dP of this tile beside its P; the scores of the next tile beside this tile's dS; the gradients beside the split of
     // the tile after the next.  Its one barrier, a third into the first product, stands between the writes of the step before and
     // the first read of what they wrote, and between the last reads of the tile before and the writes over it.
+    const float ds_scale = kQ ? p.scale : p.scale * kLift;
     int b0 = 0;  // tile % 3
     for (int tile = 0; tile < (uncarried ? 0 : n_tiles); tile++) {
         const int b1 = b0 == 2 ? 0 : b0 + 1, b2 = b1 == 2 ? 0 : b1 + 1;
@@ -235,7 +244,8 @@ __device__ __forceinline__ void bwd_role(const FlashBwdF32Params& p, int lin, in
             for (int i = 0; i < 4; i++) {
                 if (k == 0) y[i] = s[4 * z + i] * p.scale - (kQ ? lse_q : lv[z][i]);
                 if (k == 1) y[i] *= kLog2e;
-                if (k == 2) sq.r[i] = s[4 * z + i] = __builtin_amdgcn_exp2f(y[i]);
+                if (k == 2) s[4 * z + i] = __builtin_amdgcn_exp2f(y[i]);
+                if (k == 2 && !kDP) sq.r[i] = s[4 * z + i] * kLift;
             }
         };
         auto ds_step = [&](int x) RT_INLINE {
@@ -245,7 +255,7 @@ __device__ __forceinline__ void bwd_role(const FlashBwdF32Params& p, int lin, in
             for (int i = 0; i < 4; i++) {
                 if (k == 0) y[i] = dp[4 * z + i] - (kQ ? delta_q : dl[z][i]);
                 if (k == 1) y[i] *= s[4 * z + i];
-                if (k == 2) sq.r[i] = y[i] * p.scale;
+                if (k == 2) sq.r[i] = y[i] * ds_scale;
             }
         };
         auto shares = [&](auto step, int steps, int n, int of) RT_INLINE {  // the n-th of `of` shares
@@ -308,7 +318,14 @@ __device__ __forceinline__ void bwd_role(const FlashBwdF32Params& p, int lin, in
         b0 = b1;
     }
 
-    if (uncarried || __syncthreads_or(!(chk < kSplitMost))) {
+    if constexpr (!kQ) {
+#pragma unroll
+        for (int t = 0; t < DT; t++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[t][i] *= 1.0f / kLift;
+    }
+
+    if (uncarried || __syncthreads_or(!(chk < kWideMost))) {
         // something here the split does not carry: the rows once more in f32, the tiles through LDS two at a time
         using Tile = F32Tile<DT>;
         static_assert(4 * Tile::SIZE * sizeof(float) <= kWideHalfs<DT> * sizeof(__bf16), "two tiles of either matrix");

@@ -564,3 +564,24 @@ def test_wide_gradients_over_what_they_read(over):
     for name, w in zip(("dq", "dk", "dv"), gradients64(*x)):
         got = g[name].download(np.float32).reshape(b, h, n, d)
         assert np.linalg.norm(got - w) <= 2e-6 * np.linalg.norm(w), name
+@pytest.mark.parametrize("b,h,n,d", [(2, 8, 300, 96), (8, 16, 200, 128)])
+def test_wide_gradients_of_a_key_that_no_query_weighs(b, h, n, d):
+    """Every weight of the key is about e^-85 = 2^-123, as f32 has it: its rows of dK and dV hold what f32 makes of them.  The weights' error
+    is that of the exponent, a difference of f32 values of 85 (a score that is rounded twice, the statistic, their difference and the
+    product with log2 e: 5 x 2^-18 of the weight); three bf16 terms of a weight that small leave out up to 2^-11 of it."""
+    x = inputs(b, h, n, d) + [seeded_normal((b, h, n, d), 4).reshape(b, h, n, d)]
+    q, k, v, d_out = x
+    at, key = (1, 5), 40
+    q[at][:, 9], k[at][:, 9] = 4.0, 0.0
+    k[at][key] = 0.0
+    k[at][key, 9] = np.float32(-79.0 * np.sqrt(d) / 4.0)
+    got, want = run_backward(*x), gradients64(*x)
+    for name, g, w in zip(("dq", "dk", "dv"), got, want):
+        assert np.linalg.norm(g - w) <= 2e-6 * np.linalg.norm(w), name
+        if name == "dq":
+            continue
+        row, wrow = g[at][key].astype(np.float64), w[at][key]
+        assert 2.0 ** -126 < np.abs(wrow).max() < 2.0 ** -110
+        assert np.linalg.norm(row - wrow) <= 5 * 2.0 ** -18 * np.linalg.norm(wrow), name
+
+
