@@ -665,7 +665,7 @@ hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Param
         f.dim = p.dim;
         f.mask = kMaskNone;
         f.n_cus = p.n_cus;
-        if (flash_f32_gradients_wide(f) && bwd_f32_apart(p)) return launch_flash_bwd_f32_wide(stream, p);
+        if (flash_f32_gradients_wide(f) && bwd_f32_apart(p, true)) return launch_flash_bwd_f32_wide(stream, p);
         if (flash_f32_takes_split(f, true)) return launch_flash_bwd_f32_split(stream, p);
     }
     dim3 grid((p.seq + kRows - 1) / kRows, p.heads, p.batch), block(256);

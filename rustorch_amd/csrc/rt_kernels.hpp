@@ -85,7 +85,8 @@ struct FlashBwdF32Params {
     // filled by the launcher
     const float* o;
     const float* lse;
-    float* delta;  // written by the dQ kernel (its owner rows) and read by the dK/dV kernel where that runs after it
+    float* delta;  // dO . O of every row: written by the dQ kernel (its owner rows), or above head dim 64 where all three run side by side by
+                   // a launch ahead of them, and read by the kernels that run after it; not used where dQ and dK/dV run side by side otherwise
     int vec;
 };
 // Floats of scratch launch_flash_bwd_f32 needs (O, the row statistic and delta).
@@ -93,27 +94,28 @@ size_t flash_bwd_f32_workspace_floats(int batch, int heads, int seq, int dim);
 // dim <= 128.  Runs the forward kernel, then dQ (which also leaves delta) and dK/dV on `stream`.
 hipError_t launch_flash_bwd_f32(hipStream_t stream, const FlashBwdF32Params& p, float* workspace);
 // The same from a saved forward: `o` [B,H,N,D] and `lse` [B,H,N] as launch_flash_f32 leaves them (FlashF32Params::lse);
-// `delta` is B*H*N floats of scratch, used where they run one behind the other.  Runs dQ and dK/dV.
+// `delta` is B*H*N floats of scratch.  Runs dQ and dK/dV.
 hipError_t launch_flash_bwd_f32_saved(hipStream_t stream, const FlashBwdF32Params& p, const float* o, const float* lse,
                                       float* delta);
 // dQ and dK/dV of `blocks` workgroups each, `per_cu` of them on a CU: in one launch?
 bool bwd_f32_one_launch(long long blocks, int per_cu, int n_cus);
 // Do the gradients share no memory with what the kernels read, nor with each other?  Only then may dQ and dK/dV run side by side:
 // one behind the other, dQ may lie over O, and dK and dV over O, K and V, whose last reader is the workgroup that writes them.
-inline bool bwd_f32_apart(const FlashBwdF32Params& p) {
+// with_delta: delta is read beside the writes as well (the wide form; the others that run side by side have no use for it).
+inline bool bwd_f32_apart(const FlashBwdF32Params& p, bool with_delta = false) {
     const size_t rows = (size_t)p.batch * p.heads * p.seq, n = rows * (size_t)p.dim;
     const struct {
         const float* at;
         size_t n;
-    } x[9] = {{p.dq, n}, {p.dk, n}, {p.dv, n}, {p.q, n}, {p.k, n}, {p.v, n}, {p.d_out, n}, {p.o, n}, {p.lse, rows}};
+    } x[10] = {{p.dq, n}, {p.dk, n}, {p.dv, n}, {p.q, n}, {p.k, n}, {p.v, n}, {p.d_out, n}, {p.o, n}, {p.lse, rows}, {p.delta, rows}};
     for (int i = 0; i < 3; i++)
-        for (int j = i + 1; j < 9; j++)
+        for (int j = i + 1; j < (with_delta ? 10 : 9); j++)
             if ((uintptr_t)x[i].at < (uintptr_t)(x[j].at + x[j].n) && (uintptr_t)x[j].at < (uintptr_t)(x[i].at + x[i].n)) return false;
     return true;
 }
 // Its form on the bf16 matrix cores: p.o, p.lse and p.delta set, dim <= 64 and a multiple of 4, all tensors 16-byte aligned.
 hipError_t launch_flash_bwd_f32_split(hipStream_t stream, const FlashBwdF32Params& p);
-// ... and for 64 < dim <= 128; the gradients share no memory with what is read, nor with each other (bwd_f32_apart)
+// ... and for 64 < dim <= 128; the gradients share no memory with what is read, delta included, nor with each other (bwd_f32_apart)
 hipError_t launch_flash_bwd_f32_wide(hipStream_t stream, const FlashBwdF32Params& p);
 
 struct FlashBf16Params {

@@ -29,12 +29,12 @@ static std::vector<rt::DecodeSplitParams> g_decode;
 static std::vector<rt::FlashTileParams> g_tile;
 static int g_rows = 0;
 static bool g_f32_split = false;
-static std::vector<std::string> g_bwd;  // the gradients' kernels, as launched: "both", "dq", "dkdv"
+static std::vector<std::string> g_bwd;  // the gradients' kernels, as launched: "both", "dq", "dkdv", "delta"
 
 // the kernels of decode.hip, by their names
 static void note_launch(const std::string& name, dim3 grid, void** args, hipStream_t s) {
     if (name.find("attn_rows") != std::string::npos) g_rows++;
-    for (const char* k : {"both", "dq", "dkdv"})
+    for (const char* k : {"both", "dq", "dkdv", "delta"})
         if (name.find(std::string("flash_bwd_f32_") + k) != std::string::npos || name.find(std::string("flash_bwd_rows_") + k) != std::string::npos) {
             fake::Inside here;
             g_bwd.push_back(k);
@@ -417,6 +417,24 @@ static void gradients_that_share_memory_take_turns() {
     g_f32_split = false;
 }
 
+// Above head dim 64 the gradients that run side by side read delta from the workspace: one that shares memory with a gradient gives
+// the call to the kernels that have no use for it.
+static void wide_gradients_read_the_workspace() {
+    const rt_attention_shape shape = {1, 8, 16, 96};
+    const size_t rows = 128, n = rows * 96;
+    std::vector<float> memory(10 * (n + 64));
+    float* x[10];  // q k v d_out o dq dk dv, the row statistic and a workspace
+    for (int i = 0; i < 10; i++) x[i] = (float*)(((uintptr_t)memory.data() + 63) / 64 * 64) + i * n;
+    auto launched = [&](float* ws) {
+        g_bwd.clear();
+        CHECK(rt_flash_backward_saved_f32_dev(nullptr, &shape, x[0], x[1], x[2], x[4], x[8], x[3], x[5], x[6], x[7], ws, rows * sizeof(float), nullptr) == RT_OK);
+        return g_bwd;
+    };
+    const std::vector<std::string> wide = {"delta", "dkdv"}, f32 = {"both"};
+    CHECK(launched(x[9]) == wide);
+    for (int i = 5; i < 8; i++) CHECK(launched(x[i]) == f32 && launched(x[i] + n - 4) == f32);
+}
+
 int main(int argc, char** argv) {
     fake::on_launch() = note_launch;
     const std::map<std::string, std::function<void()>> tests = {
@@ -427,6 +445,7 @@ int main(int argc, char** argv) {
         {"the_prefill_plan_deals_as_the_kernel_does", the_prefill_plan_deals_as_the_kernel_does},
         {"a_tiles_lds_has_one_writer", a_tiles_lds_has_one_writer},
         {"gradients_that_share_memory_take_turns", gradients_that_share_memory_take_turns},
+        {"wide_gradients_read_the_workspace", wide_gradients_read_the_workspace},
         {"a_chunks_keys_are_cut_as_its_tests_say", a_chunks_keys_are_cut_as_its_tests_say},
         {"no_thread_spins_through_the_kernel", no_thread_spins_through_the_kernel},
         {"a_host_without_threads_copies_by_itself", a_host_without_threads_copies_by_itself},

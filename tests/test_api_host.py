@@ -16,6 +16,7 @@ CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
     "the_prefill_plan_deals_as_the_kernel_does",
     "a_tiles_lds_has_one_writer",
     "gradients_that_share_memory_take_turns",
+    "wide_gradients_read_the_workspace",
     "a_chunks_keys_are_cut_as_its_tests_say",
     "no_thread_spins_through_the_kernel",
     "a_host_without_threads_copies_by_itself",
