@@ -1874,7 +1874,7 @@ namespace {
 // partials, 16 over 1000, 8 10.5, 16 10.9.
 // Units that fill the chip by themselves are not cut.
 long long chunk_splits(long long slabs, long long rows, int head_dim, long long keys) {
-    const long long key_tile = rt::flash_tile_bf16_key_tile(head_dim), tiles = (keys + key_tile - 1) / key_tile;
+    const long long key_tile = rt::flash_tile_bf16_key_tile(head_dim, false), tiles = (keys + key_tile - 1) / key_tile;
     const long long units = slabs * ((rows + 127) / 128);
     if (units >= g_num_cus || tiles < 4) return 1;
     const long long occ = rt::flash_tile_bf16_workgroups(head_dim);

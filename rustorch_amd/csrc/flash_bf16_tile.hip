@@ -2072,9 +2072,12 @@ static bool takes_halves(const FlashTileParams& p, dim3 grid) {
 // 77 x 513 38.6 / 52.1.  A chunk's positions over a cache, whole: 2 16 200 over 1500 34.0 / 29.4, 12 32/8 10 over 4314 95.0 / 91.6, 9 8 8 over
 // 20 7.8 / 9.2, 1 12 211 over 214 15.7 / 14.8, 4 32 339 over 342 33.9 / 34.4; in spans of 256 keys 1 16/2 100 over 2048 29.1 / 26.1, of 64 rows 1 32/8
 // 16 over 8192 22.2 / 22.5, of 32 keys 10.2 / 11.4.
-static bool takes_tiles_direct(const FlashTileParams& p) {
-    return !p.bias && (p.n_splits > 1 ? p.seq_kv / p.n_splits >= 256 && p.seq_q * p.pack > 64 : p.seq_kv >= 96);
-}
+// A chunk whose lengths are on the device stays with the registers: seq_kv is the cache's size there, and a length that the launch does not
+// know may be short.  us, max_seq 8192, all lengths alike, at 20, 100, 300, 1000 and 8000 keys, registers / LDS: 32 32/8 16 positions 9.8 /
+// 14.5, 14.8 / 15.5, 26.0 / 26.2, 60.7 / 60.4, 384 / 378; 9 8 8 10.3 / 12.2, 11.4 / 11.7, 13.7 / 14.5, 23.3 / 25.7, 112 / 112; 32 16 100 - ,
+// 29.8 / 33.9, 48.8 / 51.1, 119 / 117, 827 / 746; 4 16/2 200 - , - , 30.1 / 30.3, 42.3 / 38.5, 172 / 122.  (A padded batch is as long as its longest
+// sequence: 5 8 of 2817, lengths 352 to 2817 119 / 97, one of 2817 and the rest 20 116 / 87; all 20, which nobody pads so far, 16.7 / 17.7.)
+static bool takes_tiles_direct(const FlashTileParams& p) { return flash_tile_bf16_direct(p); }
 template <int DP>
 hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
     if (p.mask == kMaskPadding) {
@@ -2101,7 +2104,9 @@ hipError_t launch_dp(hipStream_t stream, const FlashTileParams& p, dim3 grid) {
 }  // namespace
 
 bool flash_tile_bf16_supported(int dim) { return dim > 0 && dim <= 256 && dim % 8 == 0; }
-static_assert(flash_tile_bf16_key_tile(128) == TileCfg<128>::KT && flash_tile_bf16_key_tile(136) == TileCfg<256>::KT, "the host's rule of the key tile");
+static_assert(flash_tile_bf16_key_tile(128, false) == TileCfg<128, true>::KT && flash_tile_bf16_key_tile(136, false) == TileCfg<256>::KT &&
+                  flash_tile_bf16_key_tile(136, true) == TileCfg<256, true>::KT,
+              "the host's rule of the key tile");
 static_assert(flash_tile_bf16_workgroups(64) == TileCfg<64>::OCC && flash_tile_bf16_workgroups(72) == TileCfg<96>::OCC && flash_tile_bf16_workgroups(136) == TileCfg<256>::OCC,
               "the host's rule of the workgroups a CU");
 // The kernel addresses the keys of one (batch, kv head) with 32-bit byte offsets (tile offset + lane offset, the

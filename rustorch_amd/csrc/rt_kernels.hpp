@@ -191,8 +191,17 @@ struct FlashTileParams {
 };
 static_assert(offsetof(FlashTileParams, q) == 64 && offsetof(FlashTileParams, q_lens) == 128, "lines of the arguments");
 bool flash_tile_bf16_supported(int dim);
+// Head dims above 128: does a walk over `keys` keys, or over a span of them (n_splits > 1, `rows` rows a kv head), bring its tiles straight
+// to LDS?  (Why the lines lie there: takes_tiles_direct, flash_bf16_tile.hip.)
+constexpr bool flash_tile_bf16_direct(long long rows, long long keys, long long n_splits) {
+    return n_splits > 1 ? keys / n_splits >= 256 && rows > 64 : keys >= 96;
+}
+inline bool flash_tile_bf16_direct(const FlashTileParams& p) {
+    if (p.bias || ((p.pack > 1 || p.decode_rows) && p.kv_lens)) return false;
+    return flash_tile_bf16_direct((long long)p.seq_q * p.pack, p.seq_kv, p.n_splits);
+}
 // keys per LDS tile of the tile kernel at head dim `dim` (the unit the split over the keys is cut in)
-constexpr int flash_tile_bf16_key_tile(int dim) { return dim <= 128 ? 64 : 32; }
+constexpr int flash_tile_bf16_key_tile(int dim, bool direct) { return dim <= 128 || direct ? 64 : 32; }
 constexpr int flash_tile_bf16_workgroups(int dim) { return dim <= 64 ? 3 : (dim <= 128 ? 2 : 1); }  // that share a CU
 hipError_t launch_flash_tile_bf16(hipStream_t stream, const FlashTileParams& p);
 bool flash_tile_bf16_addressable(long long seq_kv, long long row_pitch);  // K/V slabs below 4 GiB (32-bit offsets)

@@ -4,6 +4,7 @@
 #include "fake_hip.hpp"
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cstdint>
 #include <cstdio>
@@ -386,6 +387,24 @@ static void a_chunks_keys_are_cut_as_its_tests_say() {
     CHECK(spans(1, 4, 32, 8, 128, 192) <= 1 && spans(1, 4, 32, 8, 128, 193) == 4);
 }
 
+// Head dims above 128: a chunk whose lengths the launch does not know may be short, whatever the cache holds, and keeps the form for it.
+static void a_chunk_of_unknown_lengths_keeps_the_short_walk() {
+    hipStream_t s;
+    CHECK(hipStreamCreate(&s) == hipSuccess);
+    for (int dim : {136, 160, 256})
+        for (auto [batch, seq_new, heads, kv] : {std::array{9, 8, 8, 8}, std::array{32, 100, 16, 16}, std::array{4, 200, 16, 2}, std::array{1, 100, 16, 2}, std::array{32, 16, 32, 8}})
+            for (bool device : {true, false}) {
+                g_tile.clear();
+                CHECK(rt_gqa_decode_chunk_bf16(s, g_buf, g_buf, g_buf, g_buf, device ? (const int32_t*)g_buf : nullptr, 8192, batch, seq_new, heads, kv, dim,
+                                               8192, nullptr) == RT_OK);
+                CHECK(g_tile.size() == 1);
+                if (g_tile.size() != 1) continue;
+                const rt::FlashTileParams& p = g_tile[0];
+                const long long rows = (long long)seq_new * (heads / kv);
+                CHECK(rt::flash_tile_bf16_direct(p) == (!device && (p.n_splits <= 1 || (8192 / p.n_splits >= 256 && rows > 64))));
+            }
+}
+
 // The gradients run side by side only where they share no memory with what either kernel reads, nor with each other.
 static void gradients_that_share_memory_take_turns() {
     const std::vector<std::string> one = {"both"}, two = {"dq", "dkdv"};
@@ -447,6 +466,7 @@ int main(int argc, char** argv) {
         {"gradients_that_share_memory_take_turns", gradients_that_share_memory_take_turns},
         {"wide_gradients_read_the_workspace", wide_gradients_read_the_workspace},
         {"a_chunks_keys_are_cut_as_its_tests_say", a_chunks_keys_are_cut_as_its_tests_say},
+        {"a_chunk_of_unknown_lengths_keeps_the_short_walk", a_chunk_of_unknown_lengths_keeps_the_short_walk},
         {"no_thread_spins_through_the_kernel", no_thread_spins_through_the_kernel},
         {"a_host_without_threads_copies_by_itself", a_host_without_threads_copies_by_itself},
         {"a_host_without_memory_is_an_error", a_host_without_memory_is_an_error},
