@@ -240,6 +240,9 @@ int rt_debug_force_bf16_prefill_kernel(int which);
  * head dim 64 (0 above, where the gradients have a form of their own).  Asks no device:
  * before the first call on one the answer is that of 256 compute units. */
 int rt_debug_f32_split_products(const rt_attention_shape *shape, uint64_t seq_kv, int mask_kind, int with_lse);
+/* The same of the gradients above head dim 64: 1 if those of this shape, on 16-byte aligned tensors that share no memory, run on
+ * the bf16 matrix cores in that form of their own. */
+int rt_debug_f32_wide_gradients(const rt_attention_shape *shape);
 
 /* No counterpart in the reference, whose CPU loop needs none: on != 0 makes every causal prefill entry (f32 and bf16,
  * every layout, padded batches included) follow its kernel with a pass that reads V once and writes NaN into each

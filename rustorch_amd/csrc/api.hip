@@ -1184,6 +1184,18 @@ RT_API int rt_debug_f32_split_products(const rt_attention_shape* shape, uint64_t
     return rt::flash_f32_takes_split(p, with_lse != 0) ? 1 : 0;
 }
 
+RT_API int rt_debug_f32_wide_gradients(const rt_attention_shape* shape) {
+    if (!shape || !fits_int(shape->batch) || !fits_int(shape->heads) || !fits_int(shape->seq) || shape->dim == 0 || shape->dim > 512) return 0;
+    rt::FlashF32Params p{};
+    p.batch = (int)shape->batch;
+    p.heads = (int)shape->heads;
+    p.seq = (int)shape->seq;
+    p.dim = (int)shape->dim;
+    p.mask = rt::kMaskNone;
+    p.n_cus = g_num_cus;
+    return rt::flash_f32_gradients_wide(p) ? 1 : 0;
+}
+
 RT_API int rt_set_strict_non_finite_v(int on) { return g_strict_v.exchange(on ? 1 : 0); }
 
 static int flash_bf16_common(void* stream, const rt_attention_shape* shape, uint64_t n_kv_heads, const void* q,

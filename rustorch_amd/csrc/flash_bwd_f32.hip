@@ -593,7 +593,11 @@ bool bwd_f32_one_launch(long long blocks, int per_cu, int n_cus) { return 2 * bl
 // the f32 kernels' workgroups of 32 rows 5 and 8.5 (6.9) for every four tiles, dQ and dK/dV one behind the other, or, where both fit the chip,
 // 6 and 12 (10 and 7) for the two.  us of the gradients, f32 / split, B H N head dim: 4 16 1024 128 1084 / 740, 96 868 / 587; 4 16 453
 // 80 297 / 142; 2 8 640 128 176 / 89; 1 4 2500 128 633 / 296; 2 8 300 96 51 / 42; 8 16 128 128 60 / 58; and on the other side 1 8
-// 500 128 52 / 65, 3 4 202 128 31 / 38, 8 16 64 128 29 / 36, 1 8 250 96 24 / 33.
+// 500 128 52 / 65, 3 4 202 128 31 / 38, 8 16 64 128 29 / 36, 1 8 250 96 24 / 33.  Of one to three tiles, and in brackets with the
+// forward that follows them: 1 8 16 96 14.2 / 11.5; 4 8 32 96 13.1 / 12.1 (22.1 / 21.9); 5 17 32 68 16.8 / 12.2 (25.8 / 22.5); 5 17 64 96 23.8 /
+// 19.6 (32.7 / 29.5), 128 28.1 / 23.2 (38.3 / 35.7); 16 16 64 96 45.2 / 42.8 (61.5 / 55.8), 128 54.8 / 53.0 (74.0 / 68.2); 8 16 96 128 54.1 / 42.8
+// (73.5 / 59.3); on the other side 8 16 32 96 13.7 / 18.9, 1 8 64 96 13.1 / 16.3, 4 8 96 128 16.9 / 24.5, 16 16 32 128 28.6 / 35.0.  Level: 5 17
+// 32 96 14.5 / 13.7 (23.3 / 23.4).
 bool flash_f32_gradients_wide(const FlashF32Params& p) {
     if (p.dim <= 64 || p.dim > 128 || p.dim % 4 != 0 || p.mask != kMaskNone || p.bias || (unsigned long long)p.seq * (unsigned)p.dim * 4 >= (1ull << 31)) return false;
     const double n_cus = p.n_cus > 0 ? p.n_cus : 256, tiles = (p.seq + 31) / 32, n_bh = (double)p.heads * p.batch;

@@ -131,6 +131,12 @@ def debug_f32_split_products(shape, mask=None, seq_kv: int = 0, with_lse: bool =
     return bool(L.lib().rt_debug_f32_split_products(C.byref(s), seq_kv, mask.kind if mask else L.RT_MASK_NONE, int(with_lse)))
 
 
+def debug_f32_wide_gradients(shape) -> bool:
+    """Whether the f32 gradients of `shape`, a head dim above 64, run on the bf16 matrix cores (measurement / test query)."""
+    s = shape._c()
+    return bool(L.lib().rt_debug_f32_wide_gradients(C.byref(s)))
+
+
 def set_strict_non_finite_v(on: bool) -> bool:
     """Causal prefill entries follow the reference for non-finite V at hidden keys (every row NaN in that column,
     cpu_forward.rs:268-425) at the cost of one more pass over V.  Returns the previous setting."""

@@ -503,7 +503,30 @@ WIDE = [
     (4, 16, 453, 80),   # dQ ahead of dK and dV
     (8, 17, 257, 100),  # head pairs not a multiple of eight, one row in the last workgroup
     (8, 16, 128, 96),   # four tiles
+    (1, 8, 3, 68),      # a few rows
+    (1, 8, 18, 96),     # one tile: no step has a next one
+    (4, 8, 32, 80),
+    (16, 16, 33, 128),  # two, the last of a row, dQ ahead of dK and dV
+    (5, 17, 64, 96),    # two, all three in one launch
+    (16, 16, 64, 96),
+    (5, 17, 95, 100),   # three
+    (16, 16, 96, 128),
 ]
+NOT_WIDE = [(8, 16, 32, 96), (1, 8, 64, 96), (4, 8, 96, 128), (16, 16, 32, 128), (1, 8, 250, 96), (8, 16, 64, 128)]
+
+
+def test_the_rule_of_the_wide_gradients():
+    """On a device of 256 compute units."""
+    for shapes, wide in ((WIDE, True), (NOT_WIDE, False)):
+        for b, h, n, d in shapes:
+            assert ra.debug_f32_wide_gradients(ra.AttentionShape.new(b, h, n, d)) == wide, (b, h, n, d)
+    for d in (64, 66, 130, 132, 256):
+        assert not ra.debug_f32_wide_gradients(ra.AttentionShape.new(4, 16, 1024, d))
+
+
+@pytest.mark.parametrize("b,h,n,d", NOT_WIDE)
+def test_few_tiles_stay_with_the_f32_gradients(b, h, n, d):
+    test_wide_gradients_against_64_bits(b, h, n, d)
 
 
 @pytest.mark.parametrize("b,h,n,d", WIDE)
@@ -546,24 +569,6 @@ def test_wide_gradients_of_values_the_split_does_not_carry(b, h, n, d, what):
         assert not fin.any() or np.linalg.norm((gs - ws)[fin]) <= 2e-6 * np.linalg.norm(ws[fin]), name
 
 
-@pytest.mark.parametrize("over", ["dk k", "dk v, dv k", "dq out", "dv k"])
-def test_wide_gradients_over_what_they_read(over):
-    """Tensors that share memory take the f32 kernels, one behind the other."""
-    b, h, n, d = 2, 8, 300, 96
-    x = inputs(b, h, n, d) + [seeded_normal((b, h, n, d), 4).reshape(b, h, n, d)]
-    shape = ra.AttentionShape.new(b, h, n, d)
-    t = dict(zip(("q", "k", "v", "d_out"), (dev(y.ravel()) for y in x)))
-    t["out"], lse, ws = ra.HipStorage(4 * b * h * n * d), ra.HipStorage(4 * b * h * n), ra.HipStorage(4 * b * h * n)
-    g = {y: ra.HipStorage(4 * b * h * n * d) for y in ("dq", "dk", "dv")}
-    ra.flash_forward_stats_f32_dev(shape, t["q"], t["k"], t["v"], t["out"], lse)
-    for pair in over.split(", "):
-        a, z = pair.split()
-        g[a] = t[z]
-    ra.flash_backward_saved_f32_dev(shape, t["q"], t["k"], t["v"], t["out"], lse, t["d_out"], g["dq"], g["dk"], g["dv"], ws, ws.byte_len)
-    ra.synchronize()
-    for name, w in zip(("dq", "dk", "dv"), gradients64(*x)):
-        got = g[name].download(np.float32).reshape(b, h, n, d)
-        assert np.linalg.norm(got - w) <= 2e-6 * np.linalg.norm(w), name
 @pytest.mark.parametrize("b,h,n,d", [(2, 8, 300, 96), (8, 16, 200, 128)])
 def test_wide_gradients_of_a_key_that_no_query_weighs(b, h, n, d):
     """Every weight of the key is about e^-85 = 2^-123, as f32 has it: its rows of dK and dV hold what f32 makes of them.  The weights' error
@@ -585,3 +590,21 @@ def test_wide_gradients_of_a_key_that_no_query_weighs(b, h, n, d):
         assert np.linalg.norm(row - wrow) <= 5 * 2.0 ** -18 * np.linalg.norm(wrow), name
 
 
+@pytest.mark.parametrize("over", ["dk k", "dk v, dv k", "dq out", "dv k"])
+def test_wide_gradients_over_what_they_read(over):
+    """Tensors that share memory take the f32 kernels, one behind the other."""
+    b, h, n, d = 2, 8, 300, 96
+    x = inputs(b, h, n, d) + [seeded_normal((b, h, n, d), 4).reshape(b, h, n, d)]
+    shape = ra.AttentionShape.new(b, h, n, d)
+    t = dict(zip(("q", "k", "v", "d_out"), (dev(y.ravel()) for y in x)))
+    t["out"], lse, ws = ra.HipStorage(4 * b * h * n * d), ra.HipStorage(4 * b * h * n), ra.HipStorage(4 * b * h * n)
+    g = {y: ra.HipStorage(4 * b * h * n * d) for y in ("dq", "dk", "dv")}
+    ra.flash_forward_stats_f32_dev(shape, t["q"], t["k"], t["v"], t["out"], lse)
+    for pair in over.split(", "):
+        a, z = pair.split()
+        g[a] = t[z]
+    ra.flash_backward_saved_f32_dev(shape, t["q"], t["k"], t["v"], t["out"], lse, t["d_out"], g["dq"], g["dk"], g["dv"], ws, ws.byte_len)
+    ra.synchronize()
+    for name, w in zip(("dq", "dk", "dv"), gradients64(*x)):
+        got = g[name].download(np.float32).reshape(b, h, n, d)
+        assert np.linalg.norm(got - w) <= 2e-6 * np.linalg.norm(w), name
