@@ -110,6 +110,21 @@ def test_additive_mask_of_any_alignment_over_many_keys(oracle, d, tq, tkv, lead)
     test_additive_mask_at_the_edges_of_items(oracle, d, tq, tkv, lead)
 
 
+@pytest.mark.parametrize("d", [32, 64, 96, 256])
+@pytest.mark.parametrize("tq,tkv", [(33, 1), (65, 1), (100, 1), (64, 2), (97, 3)])
+def test_additive_mask_of_a_key_or_two_hides_rows(oracle, d, tq, tkv):
+    """Rows shorter than a request: what hides a wave's last rows arrives.  A row hidden altogether is NaN; one that lost its
+    mask on the way would be V."""
+    b, h = 2, 3
+    for per_head in (False, True):
+        mask = np.zeros((b * h, tq, tkv) if per_head else (tq, tkv), dtype=np.float32)
+        mask[..., [r for r in range(tq) if r % 32 in (0, 29, 30, 31)], :] = -np.inf
+        mask[..., tq - 1, :] = -np.inf
+        got = run_masked(oracle, b, tq, tkv, h, d, mask).reshape(b, tq, h * d)
+        hidden = np.isinf(mask.reshape(-1, tq, tkv)[0, :, 0])
+        assert np.isnan(got[:, hidden]).all() and np.isfinite(got[:, ~hidden]).all()
+
+
 def test_masked_bf16_errors():
     z = ra.HipStorage(1 << 16)
     with pytest.raises(ra.DeviceError) as ei:  # head dim above 512
