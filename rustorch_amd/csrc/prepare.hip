@@ -287,11 +287,13 @@ hipError_t launch_decode_prepare(hipStream_t stream, const DecodePrepareParams& 
                          aligned16(p.v_in) && aligned16(p.k_cache) && aligned16(p.v_cache) && aligned16(p.cos_table) &&
                          aligned16(p.sin_table) && aligned16(p.q_gamma) && aligned16(p.k_gamma) && p.n_heads + p.n_kv <= 65535;
     if (wide_ok) {
-        // past the caches from twice what the L2s hold, 8 of 4 MB.  us, plainly / past, inputs that change from pass to pass, 32 / 8
-        // heads of 128: 1 x 2000 tokens (25 MB) 11.2 / 12.8; 1 x 3000 (37 MB) 16.4 / 19.7; 1 x 4096 (50 MB) 17.9 / 22.7; 4 x 1024 (50 MB) 17.9 /
-        // 22.8; 8 x 16 / 16 of 64, 1024 (50 MB) 20.3 / 23.1; of 256, 4 x 16 / 2, 2500 (51 MB) 41.8 / 41.8, 4 x 8 / 8, 1100 (54 MB) 27.7 / 27.0.
-        // 1 x 5500 (68 MB) 27.9 / 29.2; 2 x 3000 (74 MB) 31.3 / 31.4; 16 x 512 (101 MB) 43.1 / 38.8; 4 x 4096 (201 MB) 79.5 / 71.7.  Before a
-        // thread asked for all its rows at once it was level between the copies that bring the inputs and the attention that reads the rows
+        // past the caches from twice what the L2s hold, 8 of 4 MB.  us, plainly / past, buffers of four calls in turn, and the copies that
+        // bring the inputs and the call together, 32 / 8 heads of 128: 1 x 4096 tokens (50 MB) 18.1 / 22.6, 35.4 / 35.3; 1 x 4500 (55) 23.5 / 25.2,
+        // 38.9 / 39.1; 1 x 5000 (61) 28.0 / 27.1, 42.2 / 42.0; 1 x 5500 (68) 30.4 / 29.0, 46.1 / 45.6; 2 x 3000 (74) 33.2 / 31.5, 50.9 / 49.9; 2 x 3500
+        // (86) 38.9 / 35.6, 62.6 / 56.1; 16 x 512 (101) 44.1 / 39.0, 85.2 / 63.8; 4 x 4096 (201) 79.0 / 72.0; 8 x 16 / 16 of 64, 1300 (64) 35.6 / 32.0,
+        // 45.0 / 44.1; of 256, 4 x 8 / 8, 1300 (64) 35.0 / 30.3, 46.8 / 45.8, 4 x 16 / 2, 3500 (143) 64.8 / 59.5, 110.1 / 107.9.  Inputs that still lie in the
+        // last-level cache favour plain rows: 1 x 5500 27.9 / 29.2, 2 x 3000 31.3 / 31.4 behind other calls' copies, and a call repeated on one set of
+        // buffers, which no prompt is, 23.0 / 28.2, 25.0 / 30.8, 16 x 512 32.1 / 38.4
         const double written = 2.0 * p.batch * p.seq * (double)p.head_dim * (p.n_heads + 2.0 * p.n_kv);
         const bool past = written > 64.0 * (1 << 20);
         // Token blocks up to a multiple of eight, so that every head's land on the XCD that has their table rows (those behind the
