@@ -1885,6 +1885,11 @@ namespace {
 // 8 9.3, 15 7.9; 8 x 16 heads of 64, 4 over 800, 1 14.6, 2 14.2, 4 12.6; 32 / 8 of 128, 4 over 200, 1 9.6, 4 8.6; but, for their
 // partials, 16 over 1000, 8 10.5, 16 10.9.
 // Units that fill the chip by themselves are not cut.
+// Above head dim 128 all of it is the times of tiles through registers, 32 keys each.  Where a span takes tiles of 64 straight to LDS instead
+// (flash_tile_bf16_direct) the counts are as good: of those measured over 23 shapes the choice is within 5 % of the best, but for two
+// (12 and 14 %).  A last span that 64 keys leave empty stays: with one span less, sequences, positions, heads, head
+// dim, keys, spans: 2 54 16/2 160 6507 16 28.0, 15 25.0; but 1 64 28/4 160 4234 15 23.0, 14 25.2; 1 161 8/2 256 5973 17 26.0, 16 29.4; 3 39 8/2 160 7262 21
+// 23.4, 20 22.7, 19 23.2.
 long long chunk_splits(long long slabs, long long rows, int head_dim, long long keys) {
     const long long key_tile = rt::flash_tile_bf16_key_tile(head_dim, false), tiles = (keys + key_tile - 1) / key_tile;
     const long long units = slabs * ((rows + 127) / 128);
