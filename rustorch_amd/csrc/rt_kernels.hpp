@@ -191,14 +191,18 @@ struct FlashTileParams {
 };
 static_assert(offsetof(FlashTileParams, q) == 64 && offsetof(FlashTileParams, q_lens) == 128, "lines of the arguments");
 bool flash_tile_bf16_supported(int dim);
-// Head dims above 128: does a walk over `keys` keys, or over a span of them (n_splits > 1, `rows` rows a kv head), bring its tiles straight
-// to LDS?  (Why the lines lie there: takes_tiles_direct, flash_bf16_tile.hip.)
-constexpr bool flash_tile_bf16_direct(long long rows, long long keys, long long n_splits) {
-    return n_splits > 1 ? keys / n_splits >= 256 && rows > 64 : keys >= 96;
-}
+// Head dims above 128: tiles straight to LDS?  (Why the lines lie there: takes_tiles_direct, flash_bf16_tile.hip.)
 inline bool flash_tile_bf16_direct(const FlashTileParams& p) {
-    if (p.bias || ((p.pack > 1 || p.decode_rows) && p.kv_lens)) return false;
-    return flash_tile_bf16_direct((long long)p.seq_q * p.pack, p.seq_kv, p.n_splits);
+    const bool packed = p.pack > 1 || p.decode_rows;
+    const long long rows = (long long)p.seq_q * p.pack, keys = p.seq_kv, units = (long long)p.batch * (packed ? p.kv_heads : p.heads) * ((rows + 127) / 128);
+    if (p.bias || (packed && p.kv_lens)) return false;
+    if (p.n_splits > 1) return keys / p.n_splits >= 256 && rows > 64;
+    if (keys < 96) return false;
+    if (4 * units <= 3ll * (p.n_cus > 0 ? p.n_cus : 256) || p.mask == kMaskPadding) return true;
+    if (packed) return p.dim <= 160 ? keys >= 300 : p.dim <= 192 ? keys >= 700 : rows > 64 && keys >= 1000;
+    if (p.window > 0) return p.window >= 96;
+    if (p.q_lens) return keys >= 512;
+    return keys >= (p.mask == kMaskCausal ? (p.group > 1 ? 160 : 288) : (p.group > 1 ? 96 : 200));
 }
 // keys per LDS tile of the tile kernel at head dim `dim` (the unit the split over the keys is cut in)
 constexpr int flash_tile_bf16_key_tile(int dim, bool direct) { return dim <= 128 || direct ? 64 : 32; }

@@ -401,7 +401,7 @@ static void a_chunk_of_unknown_lengths_keeps_the_short_walk() {
                 if (g_tile.size() != 1) continue;
                 const rt::FlashTileParams& p = g_tile[0];
                 const long long rows = (long long)seq_new * (heads / kv);
-                CHECK(rt::flash_tile_bf16_direct(p) == (!device && (p.n_splits <= 1 || (8192 / p.n_splits >= 256 && rows > 64))));
+                CHECK(rt::flash_tile_bf16_direct(p) == (!device && (p.n_splits <= 1 ? dim <= 160 || rows > 64 : 8192 / p.n_splits >= 256 && rows > 64)));
             }
 }
 
@@ -436,6 +436,51 @@ static void gradients_that_share_memory_take_turns() {
     g_f32_split = false;
 }
 
+// Head dims above 128, either side of the lines between the two forms of the tile kernel: workgroups that leave the chip room or fill it.
+static void wide_heads_take_the_form_that_pays() {
+    struct Case {
+        int batch, heads, group, seq, dim, mask, window;
+        bool lens, direct;
+    };
+    for (const Case& c : {Case{2, 16, 1, 95, 256, rt::kMaskCausal, 0, false, false}, Case{2, 16, 1, 96, 256, rt::kMaskCausal, 0, false, true},
+                          Case{12, 16, 1, 128, 256, rt::kMaskCausal, 0, false, true}, Case{13, 16, 1, 128, 256, rt::kMaskCausal, 0, false, false},
+                          Case{32, 16, 1, 256, 256, rt::kMaskCausal, 0, false, false}, Case{32, 16, 1, 300, 256, rt::kMaskCausal, 0, false, true},
+                          Case{8, 32, 4, 128, 256, rt::kMaskCausal, 0, false, false}, Case{8, 32, 4, 160, 256, rt::kMaskCausal, 0, false, true},
+                          Case{32, 16, 1, 160, 160, rt::kMaskNone, 0, false, false}, Case{32, 16, 1, 200, 160, rt::kMaskNone, 0, false, true},
+                          Case{8, 32, 4, 97, 256, rt::kMaskNone, 0, false, true}, Case{32, 16, 1, 128, 256, rt::kMaskPadding, 0, false, true},
+                          Case{4, 16, 1, 1000, 256, rt::kMaskCausal, 64, false, false}, Case{4, 16, 1, 1000, 256, rt::kMaskCausal, 128, false, true},
+                          Case{1, 16, 1, 1000, 256, rt::kMaskCausal, 64, false, true}, Case{16, 16, 1, 320, 256, rt::kMaskCausal, 0, true, false},
+                          Case{16, 16, 1, 600, 256, rt::kMaskCausal, 0, true, true}, Case{4, 16, 1, 200, 256, rt::kMaskCausal, 0, true, true}}) {
+        rt::FlashTileParams p{};
+        p.batch = c.batch;
+        p.heads = c.heads;
+        p.group = c.group;
+        p.kv_heads = c.heads / c.group;
+        p.pack = 1;
+        p.seq_q = p.seq_kv = c.seq;
+        p.dim = c.dim;
+        p.mask = c.mask;
+        p.window = c.window;
+        p.n_cus = 256;
+        int32_t lens = 0;
+        if (c.lens) p.q_lens = p.kv_lens = &lens;
+        CHECK(rt::flash_tile_bf16_direct(p) == c.direct);
+    }
+    hipStream_t s;
+    CHECK(hipStreamCreate(&s) == hipSuccess);
+    struct Chunk {
+        int batch, seq_new, heads, kv, dim, keys;
+        bool direct;
+    };
+    for (const Chunk& c : {Chunk{32, 100, 16, 16, 160, 200, false}, Chunk{32, 100, 16, 16, 160, 300, true}, Chunk{32, 30, 8, 8, 192, 400, false},
+                           Chunk{32, 30, 8, 8, 192, 700, true}, Chunk{32, 100, 16, 16, 256, 500, false}, Chunk{32, 100, 16, 16, 256, 1000, true},
+                           Chunk{64, 4, 32, 8, 256, 2000, false}, Chunk{4, 300, 16, 16, 256, 300, true}}) {
+        g_tile.clear();
+        CHECK(rt_gqa_decode_chunk_bf16(s, g_buf, g_buf, g_buf, g_buf, nullptr, c.keys, c.batch, c.seq_new, c.heads, c.kv, c.dim, 2048, nullptr) == RT_OK);
+        CHECK(g_tile.size() == 1 && g_tile[0].n_splits <= 1 && rt::flash_tile_bf16_direct(g_tile[0]) == c.direct);
+    }
+}
+
 // Above head dim 64 the gradients that run side by side read delta from the workspace: one that shares memory with a gradient gives
 // the call to the kernels that have no use for it.
 static void wide_gradients_read_the_workspace() {
@@ -466,6 +511,7 @@ int main(int argc, char** argv) {
         {"gradients_that_share_memory_take_turns", gradients_that_share_memory_take_turns},
         {"wide_gradients_read_the_workspace", wide_gradients_read_the_workspace},
         {"a_chunks_keys_are_cut_as_its_tests_say", a_chunks_keys_are_cut_as_its_tests_say},
+        {"wide_heads_take_the_form_that_pays", wide_heads_take_the_form_that_pays},
         {"a_chunk_of_unknown_lengths_keeps_the_short_walk", a_chunk_of_unknown_lengths_keeps_the_short_walk},
         {"no_thread_spins_through_the_kernel", no_thread_spins_through_the_kernel},
         {"a_host_without_threads_copies_by_itself", a_host_without_threads_copies_by_itself},

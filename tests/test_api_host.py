@@ -18,6 +18,7 @@ CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
     "gradients_that_share_memory_take_turns",
     "wide_gradients_read_the_workspace",
     "a_chunks_keys_are_cut_as_its_tests_say",
+    "wide_heads_take_the_form_that_pays",
     "a_chunk_of_unknown_lengths_keeps_the_short_walk",
     "no_thread_spins_through_the_kernel",
     "a_host_without_threads_copies_by_itself",

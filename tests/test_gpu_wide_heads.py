@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import rustorch_amd as ra
-from _gpu import assert_bf16_parity, bf16_round, flash_bf16
+from _gpu import assert_bf16_parity, bf16_round, dev, flash_bf16
 from _util import seeded_normal
 from test_gpu_attention_general import run_chunk
 from test_gpu_flash_bf16 import run_varlen
@@ -27,6 +27,36 @@ def test_masks_at_the_edges_of_tiles(oracle, n, d):
         want = oracle.flash_forward_masked(oracle.AttentionShape(b, h, n, d), qf, kf, vf, om)
         assert_bf16_parity(got, want, d, n, f"n={n} d={d} mask={mask.kind}")
         assert np.array_equal(got, flash_bf16(shape, qb, kb, vb, mask)), "two launches, two results"
+
+
+@pytest.mark.parametrize("d", [136, 256])
+@pytest.mark.parametrize("n", [129, 199, 200, 287, 288, 321])
+def test_workgroups_that_fill_the_chip(oracle, n, d):
+    """Either side of the lines there.  All heads have the same rows, so that one stands for all."""
+    b, h = 14, 16
+    one = [bf16_round(seeded_normal((1, 1, n, d), n + i)) for i in range(3)]
+    q, k, v = (np.ascontiguousarray(np.broadcast_to(x[0].reshape(1, 1, n, d), (b, h, n, d))) for x in one)
+    for mask, om in ((ra.Mask.none(), None), (ra.Mask.causal(), "causal")):
+        got = np.asarray(flash_bf16(ra.AttentionShape.new(b, h, n, d), q, k, v, mask)).reshape(b * h, n * d)
+        assert (got == got[0]).all()
+        want = oracle.flash_forward_masked(oracle.AttentionShape(1, 1, n, d), *(x[1].ravel() for x in one), om)
+        assert_bf16_parity(got[0], want, d, n, f"n={n} d={d} {om}")
+
+
+@pytest.mark.parametrize("b,s,hq,hkv,d,keys", [(25, 8, 8, 8, 136, 299), (25, 8, 8, 8, 136, 300), (25, 8, 8, 8, 256, 300), (13, 66, 16, 16, 256, 999), (13, 66, 16, 16, 256, 1000)])
+def test_chunks_that_fill_the_chip(oracle, b, s, hq, hkv, d, keys):
+    qb, kb, vb = (bf16_round(seeded_normal(shape, i))[0] for i, shape in enumerate([(1, s, 1, d), (1, 1, keys, d), (1, 1, keys, d)]))
+    q = np.ascontiguousarray(np.broadcast_to(qb.reshape(1, s, 1, d), (b, s, hq, d)))
+    k, v = (np.ascontiguousarray(np.broadcast_to(x.reshape(1, 1, keys, d), (b, hkv, keys, d))) for x in (kb, vb))
+    out = ra.HipStorage(q.size * 2)
+    out.upload(np.full(q.size, 0x7B7B, dtype=np.uint16))
+    dq, dk, dv = dev(q), dev(k), dev(v)
+    ra.LlmKernels().gqa_decode_chunk_bf16(None, dq, dk, dv, out, keys, b, s, hq, hkv, d, keys)
+    ra.synchronize()
+    got = oracle.bf16_to_f32(out.download(np.uint16)).reshape(b, s, hq, d)
+    assert (got == got[:1, :, :1]).all()
+    want = oracle.gqa_decode_chunk_bf16(qb, kb, vb, [keys], 1, s, 1, 1, d, keys)
+    assert_bf16_parity(got[0, :, 0].ravel(), want, d, None, f"s={s} d={d} keys={keys}")
 
 
 @pytest.mark.parametrize("d", [152, 256])
