@@ -8,8 +8,8 @@
 // with one barrier, inside the first product, and everything a product starts with read from LDS in the product ahead of it.  A gradient's
 // tile sum is formed in registers of its own, small terms first, and added once (rounded once a tile at its size).
 //
-// What bounds it: a wave takes its SIMD's register file and issues an instruction every 5 clocks, some 1000 a tile at head dim 128 with
-// 144 matrix instructions of 32 clocks among them, under a clock of 2.0 to 2.2 GHz.  us of both gradients, B=4 H=16 N=1024: head dim 128
+// What bounds it: a wave has its SIMD to itself and waits alone.  At head dim 128 a tile of dQ takes 8.4 k clocks, the matrix pipe 4.6 k of them (144
+// instructions of 32) and the vector unit 3.1 k; one of dK or dV 7.5 k, 3.8 k and 2.9 k (counters, B=4 H=16 N=1024, clock 2.0 GHz).  us of both gradients, B=4 H=16 N=1024: head dim 128
 // f32 kernels 1087, this 863 with sums in the accumulation registers (the vector unit reads none of those), 798 -> 765 with
 // them in its own, 740 without copies of loaded registers and owners loaded one behind the other; 96 868, 669, 649, 587.  Relative error
 // against 64 bits 6.5e-7 -> 4.2e-7, 6.1e-7 -> 4.1e-7.
