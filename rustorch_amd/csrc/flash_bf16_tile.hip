@@ -2079,10 +2079,12 @@ static bool takes_halves(const FlashTileParams& p, dim3 grid) {
 // Spans of a chunk: from 256 keys a span on, where more than two waves of a tile have rows: 1 16/2 100 over 2048 29.1 / 26.1, of 64 rows 1 32/8
 // 16 over 8192 22.2 / 22.5, of 32 keys 10.2 / 11.4.  Not with a bias, whose LDS leaves the query rows to be read into the operands and whose
 // values spill: 4 8 1024 57.2 / 65.0, 1 8 77 x 513 38.6 / 52.1.
-// A chunk whose lengths are on the device stays with the registers: seq_kv is the cache's size there, and a length that the launch does not
-// know may be short.  max_seq 8192, all lengths alike, at 20, 100, 300, 1000 and 8000 keys: 32 32/8 16 positions 9.8 / 14.5, 14.8 / 15.5, 26.0 /
-// 26.2, 60.7 / 60.4, 384 / 378; 9 8 8 10.3 / 12.2, 11.4 / 11.7, 13.7 / 14.5, 23.3 / 25.7, 112 / 112; 32 16 100 - , 29.8 / 33.9, 48.8 / 51.1, 119 / 117,
-// 827 / 746; 4 16/2 200 - , - , 30.1 / 30.3, 42.3 / 38.5, 172 / 122.  (A padded batch is as long as its longest sequence: 5 8 of 2817, lengths
+// A chunk whose lengths are on the device is taken to be as long as its new positions, from 256 of them on, not as the cache: a length that the
+// launch does not know may be short.  max_seq 8192, all lengths alike, at 20, 100, 300, 1000 and 8000 keys: 32 32/8 16 positions 9.8 / 14.5,
+// 14.8 / 15.5, 26.0 / 26.2, 60.7 / 60.4, 384 / 378; 9 8 8 10.3 / 12.2, 11.4 / 11.7, 13.7 / 14.5, 23.3 / 25.7, 112 / 112; 32 16 100 - , 29.8 /
+// 33.9, 48.8 / 51.1, 119 / 117, 827 / 746; 4 16/2 200 - , - , 30.1 / 30.3, 42.3 / 38.5, 172 / 122; 5 28 96 at 96 and 4000 11.8 / 13.4, 164 / 150; 4 16 300 at
+// 300, 1000 and 8000 19.5 / 17.6, 46.4 / 39.2, 319 / 248; 2 16/8 1024 at 1024 and 8000 49.1 / 41.5, 321 / 247.
+// (A padded batch is as long as its longest sequence: 5 8 of 2817, lengths
 // 352 to 2817 119 / 97, one of 2817 and the rest 20 116 / 87; all 20, which nobody pads so far, 16.7 / 17.7.)
 static bool takes_tiles_direct(const FlashTileParams& p) { return flash_tile_bf16_direct(p); }
 template <int DP>

@@ -193,11 +193,11 @@ static_assert(offsetof(FlashTileParams, q) == 64 && offsetof(FlashTileParams, q_
 bool flash_tile_bf16_supported(int dim);
 // Head dims above 128: tiles straight to LDS?  (Why the lines lie there: takes_tiles_direct, flash_bf16_tile.hip.)
 inline bool flash_tile_bf16_direct(const FlashTileParams& p) {
-    const bool packed = p.pack > 1 || p.decode_rows;
-    const long long rows = (long long)p.seq_q * p.pack, keys = p.seq_kv, units = (long long)p.batch * (packed ? p.kv_heads : p.heads) * ((rows + 127) / 128);
-    if (p.bias || (packed && p.kv_lens)) return false;
-    if (p.n_splits > 1) return keys / p.n_splits >= 256 && rows > 64;
-    if (keys < 96) return false;
+    const bool packed = p.pack > 1 || p.decode_rows, unknown = packed && p.kv_lens;  // lengths on the device: the new positions' at least
+    const long long rows = (long long)p.seq_q * p.pack, keys = unknown ? p.seq_q : p.seq_kv, units = (long long)p.batch * (packed ? p.kv_heads : p.heads) * ((rows + 127) / 128);
+    if (p.bias) return false;
+    if (p.n_splits > 1) return !unknown && keys / p.n_splits >= 256 && rows > 64;
+    if (keys < (unknown ? 256 : 96)) return false;
     if (4 * units <= 3ll * (p.n_cus > 0 ? p.n_cus : 256) || p.mask == kMaskPadding) return true;
     if (packed) return p.dim <= 160 ? keys >= 300 : p.dim <= 192 ? keys >= 700 : rows > 64 && keys >= 1000;
     if (p.window > 0) return p.window >= 96;

@@ -387,22 +387,25 @@ static void a_chunks_keys_are_cut_as_its_tests_say() {
     CHECK(spans(1, 4, 32, 8, 128, 192) <= 1 && spans(1, 4, 32, 8, 128, 193) == 4);
 }
 
-// Head dims above 128: a chunk whose lengths the launch does not know may be short, whatever the cache holds, and keeps the form for it.
+// Head dims above 128: a chunk whose lengths the launch does not know may be short, whatever the cache holds, and keeps the form for it; as
+// long as its new positions it is.
 static void a_chunk_of_unknown_lengths_keeps_the_short_walk() {
     hipStream_t s;
     CHECK(hipStreamCreate(&s) == hipSuccess);
-    for (int dim : {136, 160, 256})
-        for (auto [batch, seq_new, heads, kv] : {std::array{9, 8, 8, 8}, std::array{32, 100, 16, 16}, std::array{4, 200, 16, 2}, std::array{1, 100, 16, 2}, std::array{32, 16, 32, 8}})
-            for (bool device : {true, false}) {
-                g_tile.clear();
-                CHECK(rt_gqa_decode_chunk_bf16(s, g_buf, g_buf, g_buf, g_buf, device ? (const int32_t*)g_buf : nullptr, 8192, batch, seq_new, heads, kv, dim,
-                                               8192, nullptr) == RT_OK);
-                CHECK(g_tile.size() == 1);
-                if (g_tile.size() != 1) continue;
-                const rt::FlashTileParams& p = g_tile[0];
-                const long long rows = (long long)seq_new * (heads / kv);
-                CHECK(rt::flash_tile_bf16_direct(p) == (!device && (p.n_splits <= 1 ? dim <= 160 || rows > 64 : 8192 / p.n_splits >= 256 && rows > 64)));
-            }
+    auto direct = [&](int batch, int seq_new, int heads, int kv, int dim, bool device) {
+        g_tile.clear();
+        CHECK(rt_gqa_decode_chunk_bf16(s, g_buf, g_buf, g_buf, g_buf, device ? (const int32_t*)g_buf : nullptr, 8192, batch, seq_new, heads, kv, dim, 8192,
+                                       nullptr) == RT_OK);
+        CHECK(g_tile.size() == 1);
+        return rt::flash_tile_bf16_direct(g_tile[0]);
+    };
+    for (int dim : {136, 160, 256}) {
+        for (auto [batch, seq_new, heads, kv] : {std::array{9, 8, 8, 8}, std::array{32, 100, 16, 16}, std::array{4, 200, 16, 2}, std::array{1, 100, 16, 2}, std::array{32, 16, 32, 8},
+                                                 std::array{5, 96, 28, 28}, std::array{4, 255, 16, 16}})
+            CHECK(!direct(batch, seq_new, heads, kv, dim, true));
+        CHECK(direct(4, 300, 16, 16, dim, true) && direct(2, 1024, 16, 8, dim, true) && direct(1, 1024, 32, 8, dim, true) && direct(8, 1100, 16, 4, dim, true));
+        CHECK(direct(32, 100, 16, 16, dim, false) && direct(4, 200, 16, 2, dim, false) && direct(1, 100, 16, 2, dim, false) && direct(5, 96, 28, 28, dim, false));
+    }
 }
 
 // The gradients run side by side only where they share no memory with what either kernel reads, nor with each other.

@@ -517,7 +517,7 @@ NOT_WIDE = [(8, 16, 32, 96), (1, 8, 64, 96), (4, 8, 96, 128), (16, 16, 32, 128),
 
 def test_the_rule_of_the_wide_gradients():
     """On a device of 256 compute units."""
-    for shapes, wide in ((WIDE, True), (NOT_WIDE, False)):
+    for shapes, wide in ((WIDE + [(8, 16, 200, 128)], True), (NOT_WIDE, False)):
         for b, h, n, d in shapes:
             assert ra.debug_f32_wide_gradients(ra.AttentionShape.new(b, h, n, d)) == wide, (b, h, n, d)
     for d in (64, 66, 130, 132, 256):

@@ -94,3 +94,19 @@ def test_padded_batch(oracle, d):
 ])
 def test_chunks(oracle, b, s, hq, hkv, d, max_seq, lens):
     run_chunk(oracle, b, s, hq, hkv, d, max_seq, lens)
+
+
+@pytest.mark.parametrize("b,s,hq,hkv,d,max_seq,lens", [
+    (1, 130, 4, 1, 256, 500, [500]),        # whole, more rows than a tile
+    (4, 40, 16, 16, 200, 200, [200] * 4),
+    (1, 100, 16, 2, 256, 2047, [2047]),     # spans of fewer than 256 keys,
+    (1, 100, 16, 2, 256, 2049, [2049]),     # and of more; the last of a key
+    (1, 200, 16, 2, 160, 4000, [3333]),
+])
+def test_chunks_of_a_length_the_launch_knows(oracle, b, s, hq, hkv, d, max_seq, lens):
+    run_chunk(oracle, b, s, hq, hkv, d, max_seq, lens, scalar_len=True)
+
+
+@pytest.mark.parametrize("s,lens", [(255, [700, 300, 255, 400]), (256, [700, 256, 1, 321]), (300, [700, 301, 300, 0])])
+def test_chunks_of_many_positions_and_unknown_lengths(oracle, s, lens):
+    run_chunk(oracle, 4, s, 16, 16, 136, 700, lens)
