@@ -196,13 +196,16 @@ inline bool flash_tile_bf16_direct(const FlashTileParams& p) {
     const bool packed = p.pack > 1 || p.decode_rows, unknown = packed && p.kv_lens;  // lengths on the device: the new positions' at least
     const long long rows = (long long)p.seq_q * p.pack, keys = unknown ? p.seq_q : p.seq_kv, units = (long long)p.batch * (packed ? p.kv_heads : p.heads) * ((rows + 127) / 128);
     if (p.bias) return false;
-    if (p.n_splits > 1) return !unknown && keys / p.n_splits >= 256 && rows > 64;
-    if (keys < (unknown ? 256 : 96)) return false;
-    if (4 * units <= 3ll * (p.n_cus > 0 ? p.n_cus : 256) || p.mask == kMaskPadding) return true;
+    if (p.n_splits > 1) return !unknown && keys / p.n_splits >= 256 && rows > 96;
+    const long long n_cus = p.n_cus > 0 ? p.n_cus : 256;
+    if (keys < (unknown ? 256 : packed ? 140 : p.q_lens && 2 * units > n_cus ? 160 : 96)) return false;
+    if (4 * units <= 3 * n_cus || p.mask == kMaskPadding) return true;
+    if (packed && p.pack > 1 && rows > 64) return keys >= 250;
     if (packed) return p.dim <= 160 ? keys >= 300 : p.dim <= 192 ? keys >= 700 : rows > 64 && keys >= 1000;
-    if (p.window > 0) return p.window >= 96;
-    if (p.q_lens) return keys >= 512;
-    return keys >= (p.mask == kMaskCausal ? (p.group > 1 ? 160 : 288) : (p.group > 1 ? 96 : 200));
+    if (p.window > 0) return (p.group > 1 && p.heads >= 16) || (p.dim > 240 && p.window >= 256);
+    if (p.q_lens) return keys >= (p.dim <= 224 ? 352 : 512);
+    if (p.mask == kMaskCausal) return keys >= (p.group == 1 ? 288 : p.dim > 240 ? 129 : 96);
+    return p.group > 1 || keys <= 128 || keys > 160;
 }
 // keys per LDS tile of the tile kernel at head dim `dim` (the unit the split over the keys is cut in)
 constexpr int flash_tile_bf16_key_tile(int dim, bool direct) { return dim <= 128 || direct ? 64 : 32; }

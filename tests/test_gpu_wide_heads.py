@@ -67,10 +67,20 @@ def test_windows(oracle, d, window):
         assert_bf16_parity(got.reshape(1, n, 2 * d), want.reshape(1, n, 2 * d), 2 * d, None, f"n={n} window {window}", block_rows=64)
 
 
+def test_windows_that_fill_the_chip(oracle):
+    for hkv in (16, 8):  # through registers, and straight to LDS
+        got, want, _ = window_bnhd(oracle, 7, 193, 16, hkv, 136, 97, hkv)
+        assert_bf16_parity(got.reshape(7, 193, 16 * 136), want.reshape(7, 193, 16 * 136), 16 * 136, None, f"kv heads {hkv}", block_rows=64)
+
+
+@pytest.mark.parametrize("n,d", [(193, 136), (353, 136)])
+def test_padded_batches_that_fill_the_chip(oracle, n, d):
+    test_padded_batch(oracle, d, 13, 8, n, [n, 0, 1, 64, 65, 129, n - 1] + [n // 2] * 6)
+
+
 @pytest.mark.parametrize("d", [168, 256])
-def test_padded_batch(oracle, d):
-    b, h, n = 6, 2, 200
-    lens = np.array([200, 0, 1, 64, 65, 129], dtype=np.int32)
+def test_padded_batch(oracle, d, b=6, h=2, n=200, lens=(200, 0, 1, 64, 65, 129)):
+    lens = np.array(lens, dtype=np.int32)
     (qb, qf), (kb, kf), (vb, vf) = (bf16_round(seeded_normal((b, h, n, d), i)) for i in range(3))
     kb, vb = (x.copy().reshape(b, h, n, d) for x in (kb, vb))
     for i, m in enumerate(lens):  # what lies behind a sequence is not read, or weighs nothing
