@@ -10,6 +10,8 @@
 // of squares is taken sequentially, products and sums are rounded separately (this file is compiled with
 // floating-point contraction off) -- and rounded to bf16 once, so the result is the bf16 rounding of what the
 // CPU path computes on the same bf16 inputs, bit for bit.
+#include <type_traits>
+
 #include "rt_common.hpp"
 #include "rt_kernels.hpp"
 
@@ -280,7 +282,7 @@ bool aligned16(const void* a) { return ((uintptr_t)a & 15) == 0; }
 hipError_t launch_decode_prepare(hipStream_t stream, const DecodePrepareParams& p) {
     if (p.batch == 0 || p.seq == 0 || p.n_heads + p.n_kv == 0 || p.head_dim == 0) return hipSuccess;
     if (p.head_dim > kPrepMaxD || (p.head_dim & 1) || p.seq > 65535 || p.batch > 65535) return hipErrorInvalidValue;
-    // a prompt: the kernel that moves 64 consecutive tokens of a head through LDS, where its loads and stores are whole
+    // a prompt: the kernel that moves 64 or 128 consecutive tokens of a head through LDS, where its loads and stores are whole
     // 16-byte chunks (64 rows: 17 or 33 KB of LDS, so that four to eight workgroups share a CU; with 256 rows the same
     // prompt took 113 us instead of 80)
     const bool wide_ok = p.seq >= 32 && p.head_dim % 16 == 0 && p.head_dim <= 256 && aligned16(p.q) && aligned16(p.k_in) &&
@@ -296,23 +298,30 @@ hipError_t launch_decode_prepare(hipStream_t stream, const DecodePrepareParams& 
         // buffers, which no prompt is, 23.0 / 28.2, 25.0 / 30.8, 16 x 512 32.1 / 38.4
         const double written = 2.0 * p.batch * p.seq * (double)p.head_dim * (p.n_heads + 2.0 * p.n_kv);
         const bool past = written > 64.0 * (1 << 20);
-        // Token blocks up to a multiple of eight, so that every head's land on the XCD that has their table rows (those behind the
-        // last token end at once), where that adds a fifth at most.  us, as they are / so, 1 x 32 / 8 heads of 128: 550 tokens (9 blocks)
-        // 6.5 / 7.4, 1100 (18) 8.8 / 9.3, 1300 (21) 10.5 / 9.9, 2200 (35) 13.4 / 12.8, 2600 (41) 14.7 / 13.9, 3000 (47) 16.4 / 14.6.
-        int blocks = (p.seq + 63) / 64;
-        const int eights = (blocks + 7) / 8 * 8;
-        if (5 * (eights - blocks) <= blocks) blocks = eights;
-        const dim3 grid(blocks, p.n_heads + p.n_kv, p.batch), block(256);
         DecodePrepareParams pp = p;
         pp.chunk_magic = (1u << 20) / (uint32_t)(p.head_dim / 8) + 1u;  // (exact: c d < 2^20)
         pp.pair_magic = (1u << 20) / (uint32_t)(p.head_dim / 16) + 1u;
-        if (p.head_dim <= 128) {
-            if (past) hipLaunchKernelGGL((prompt_prepare_kernel<64, 128, true>), grid, block, 0, stream, pp);
-            else hipLaunchKernelGGL((prompt_prepare_kernel<64, 128, false>), grid, block, 0, stream, pp);
-        } else {
-            if (past) hipLaunchKernelGGL((prompt_prepare_kernel<64, 256, true>), grid, block, 0, stream, pp);
-            else hipLaunchKernelGGL((prompt_prepare_kernel<64, 256, false>), grid, block, 0, stream, pp);
-        }
+        auto launch = [&](auto rows_c, auto dmax_c) {
+            constexpr int kRows = decltype(rows_c)::value, kDMax = decltype(dmax_c)::value;
+            // Token blocks up to a multiple of eight, so that every head's land on the XCD that has their table rows (those behind the
+            // last token end at once), where that adds a fifth at most.  us, as they are / so, 1 x 32 / 8 heads of 128: 550 tokens (9 blocks)
+            // 6.5 / 7.4, 1100 (18) 8.8 / 9.3, 1300 (21) 10.5 / 9.9, 2200 (35) 13.4 / 12.8, 2600 (41) 14.7 / 13.9, 3000 (47) 16.4 / 14.6.
+            int blocks = (p.seq + kRows - 1) / kRows;
+            const int eights = (blocks + 7) / 8 * 8;
+            if (5 * (eights - blocks) <= blocks) blocks = eights;
+            const dim3 grid(blocks, p.n_heads + p.n_kv, p.batch), block(256);
+            if (past) hipLaunchKernelGGL((prompt_prepare_kernel<kRows, kDMax, true>), grid, block, 0, stream, pp);
+            else hipLaunchKernelGGL((prompt_prepare_kernel<kRows, kDMax, false>), grid, block, 0, stream, pp);
+        };
+        // A thread asks for as many chunks as its widest row needs: narrow heads have a form of their own, or half and three quarters of those
+        // requests are for nothing.  us, chunks in a loop (before) / rows of up to 128 / of up to 64 / 128 rows of up to 32, recorded: 3 x 16 / 16 heads of 64,
+        // 6807 tokens 50.2 / 56.1 / 47.2, 1 x 32 / 8, 1000 5.9 / 5.6 / 5.1, without gamma 4.9 / 4.7 / 4.2; of 48, 2 x 32 / 8, 3000 14.0 / 15.0 / 13.1; of 32, 3 x
+        // 16 / 16, 6807 31.9 / 38.0 / 30.0 / 27.0, 4 x 16 / 16, 700 without gamma 6.0 / 6.7 / 5.6 / 4.9, 1 x 32 / 8, 100 3.49 / 3.35 / 3.16 / 3.37.  (128 rows of up to
+        // 64: 49.1 and 6.0 us on the first two, 256 of up to 32 30.7 on the fourth.)
+        if (p.head_dim <= 32) launch(std::integral_constant<int, 128>{}, std::integral_constant<int, 32>{});
+        else if (p.head_dim <= 64) launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 64>{});
+        else if (p.head_dim <= 128) launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 128>{});
+        else launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 256>{});
         return hipGetLastError();
     }
     const dim3 grid(p.n_heads + p.n_kv, p.seq, p.batch), block(64);

@@ -68,7 +68,7 @@ def test_head_dims_at_the_edges_of_a_lanes_pairs(oracle, norms, d):
                                                   (2, 3, 1, 80, 500, 449), (1, 2, 2, 144, 140, 129), (2, 2, 1, 240, 1400, 1345)])
 def test_several_new_tokens_match_oracle_bit_for_bit(oracle, b_, hq, hkv, d, lmax, seq, norms):
     """A prompt: [batch, heads, seq, head_dim] inputs, token s at position p + s and cache row p + s.  From 32 tokens
-    on, head dims that are a multiple of 16 up to 256 take the kernel that moves 64 consecutive tokens of a head
+    on, head dims that are a multiple of 16 up to 256 take the kernel that moves 64 (128 up to head dim 32) consecutive tokens of a head
     through LDS; the others (and head dim 72 here) the one-wave-per-row kernel: the same
     bits either way."""
     rng = np.random.default_rng(300 + seq)
@@ -76,6 +76,14 @@ def test_several_new_tokens_match_oracle_bit_for_bit(oracle, b_, hq, hkv, d, lma
     positions[-1] = lmax - seq
     rope, oro, q, k, v, kc, vc, qg, kg = _case(oracle, rng, b_, hq, hkv, d, lmax, positions, norms, seq=seq)
     _run(oracle, rope, oro, q, k, v, kc, vc, qg, kg, positions, b_, hq, hkv, d, lmax, 1e-6, seq=seq)
+
+
+@pytest.mark.parametrize("norms", [(True, True), (False, False)])
+@pytest.mark.parametrize("d", [16, 32, 48, 64, 80])
+@pytest.mark.parametrize("seq", [32, 63, 64, 65, 127, 128, 129, 1000])
+def test_prompts_of_narrow_heads(oracle, seq, d, norms):
+    """Blocks of 64 and of 128 tokens, the last of one or of all but one."""
+    test_several_new_tokens_match_oracle_bit_for_bit(oracle, 2, 3, 1, d, seq + 5, seq, norms)
 
 
 def test_prompt_overflow_is_reported_for_the_last_token():
