@@ -23,11 +23,12 @@ namespace {
 enum Role { kDQ, kDK, kDV };  // the gradient of a workgroup's rows
 
 // dK and dV: dS and P are split at 2^17 times their size, so that whatever f32 holds of them (2^-126 on) keeps 24 bits.  The last term of a
-// split meets the smallest bf16 below 2^-109, and the rows of a key that every query weighs with 2^-123 were off by 2^-12 of themselves, where f32
-// leaves 2^-18 (the exponent's rounding).  (A row of dQ has weights that sum to one, beside which such small ones are nothing.)  dS has the
-// factor in its scale, P takes 16 multiplies a tile: grads, us, without / with, B H N head dim: 8 16 96 128 41.9 / 42.0, 8 16 96 96 35.1 / 35.7, 4 16 453
-// 80 137.7 / 138.1, 16 16 64 128 52.0 / 52.3.  What goes in stays below 2^27 for it: 2^(3 x 27 + 7) of a product of three over the head dim, times a
-// scale below 2^-3 and 2^17, is below 2^125 over the 2^23 rows that 2 GiB hold.
+// split meets the smallest bf16 below 2^-109, and the rows of a key that every query weighs with 2^-123 were off by 2^-12 of themselves, where
+// f32 leaves 2^-18 (the exponent's rounding).  (A row of dQ has weights that sum to one, beside which such small ones are nothing.)  dS has
+// the factor in its scale, P takes 16 multiplies a tile: training steps, us, without / with, B H N head dim: 1 12 903 96 196.3 / 200.0, 4 8
+// 376 80 94.1 / 96.2, 8 16 96 96 49.5 / 50.1, 4 16 453 80 183.0 / 183.7, 2 8 640 128 136.6 / 136.7.  What goes in stays below 2^27 for it:
+// 2^(3 x 27 + 7) of a product of three over the head dim, times a scale below 2^-3 and 2^17, is below 2^125 over the 2^23 rows that 2 GiB
+// hold.
 constexpr float kLift = 0x1p17f, kWideMost = 0x1p27f;
 
 template <int DT>
@@ -228,29 +229,33 @@ __device__ __forceinline__ void bwd_role(const FlashBwdF32Params& p, int lin, in
         SplitQuad sq;
         float y[4];
         f32x16_t dp, s_next;
-        // eight steps for four elements: the three instructions of each, then (kSplit) their split
-        auto split_part = [&](int x) RT_INLINE {
-            const int z = x / 8, k = x % 8 - 3;
+        // eight steps for four elements, of P (dV) nine: the three instructions of each, the factor of P in a step of its own (one behind the
+        // exponentials it waits for them, 1 x 12 heads of 96, N=903 201 us for 196), then the five of their split
+        constexpr int kPSteps = 9;
+        auto split_part = [&](int z, int k) RT_INLINE {
             uint32_t a = 0, b = 0;
             sq.step(k, a, b);
             if (k % 2) return;
             w[z / 2][k / 2][2 * (z & 1)] = a;
             w[z / 2][k / 2][2 * (z & 1) + 1] = b;
         };
-        auto p_step = [&](int x) RT_INLINE {
-            const int z = x / 8, k = x % 8;
-            if (k >= 3) return split_part(x);
+        auto p_part = [&](int z, int k) RT_INLINE {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 if (k == 0) y[i] = s[4 * z + i] * p.scale - (kQ ? lse_q : lv[z][i]);
                 if (k == 1) y[i] *= kLog2e;
                 if (k == 2) s[4 * z + i] = __builtin_amdgcn_exp2f(y[i]);
-                if (k == 2 && !kDP) sq.r[i] = s[4 * z + i] * kLift;
+                if (k == 3) sq.r[i] = s[4 * z + i] * kLift;
             }
+        };
+        auto p_step = [&](int x) RT_INLINE {
+            const int z = x / kPSteps, k = x % kPSteps;
+            if (k < 4) p_part(z, k);
+            else split_part(z, k - 4);
         };
         auto ds_step = [&](int x) RT_INLINE {
             const int z = x / 8, k = x % 8;
-            if (k >= 3) return split_part(x);
+            if (k >= 3) return split_part(z, k - 3);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 if (k == 0) y[i] = dp[4 * z + i] - (kQ ? delta_q : dl[z][i]);
@@ -262,8 +267,7 @@ __device__ __forceinline__ void bwd_role(const FlashBwdF32Params& p, int lin, in
 #pragma unroll
             for (int x = steps * n / of; x < steps * (n + 1) / of; x++) step(x);
         };
-        // P without its split: only the first three of eight steps count
-        auto p_only = [&](int x) RT_INLINE { p_step(x / 3 * 8 + x % 3); };
+        auto p_only = [&](int x) RT_INLINE { p_part(x / 3, x % 3); };  // P without its split
         if constexpr (kDP) {
             product(dp, ybuf(b0), yo, 0, [&](int n) RT_INLINE {
                 if (n == 2 * KS - 1) __syncthreads();
@@ -288,13 +292,13 @@ __device__ __forceinline__ void bwd_role(const FlashBwdF32Params& p, int lin, in
             if (more) {
                 product(s_next, xbuf(b1), xo, 1, [&](int n) RT_INLINE {
                     if (n == 2 * KS - 1) __syncthreads();
-                    shares(p_step, 32, n, 6 * KS);
+                    shares(p_step, 4 * kPSteps, n, 6 * KS);
                     if (n == 5 * KS) read_cols(ybuf(b0), 0, 0);
                 });
             } else {
                 zero16(s_next);
                 __syncthreads();
-                shares(p_step, 32, 0, 1);
+                shares(p_step, 4 * kPSteps, 0, 1);
                 read_cols(ybuf(b0), 0, 0);
             }
         }
