@@ -2074,19 +2074,20 @@ static bool takes_halves(const FlashTileParams& p, dim3 grid) {
 // / 338, head dim 160 32 16 160 45.5 / 48.3, 256 59.4 / 57.7; four query heads a kv head, whose keys the L2s have, 8 32/8 97 12.6 / 12.4, 128 13.7 /
 // 14.2 (at 224 1.02 times as fast), 160 24.0 / 23.4, 3 40/8 724 71.7 / 56.7.  None: of 129 to 160 keys, five tiles or three, 32 16 160 55.6 / 57.5,
 // else 97 26.3 / 25.5, 200 70.8 / 72.1 (head dim 160 62.1 / 59.2), 256 86.2 / 80.6, 2 16 2048 177 / 130, shared 8 32/8 97 12.9 / 11.5.  A padding
-// mask ahead from 97 keys on (32 16 128 34.4 / 31.8, 2 16 2048 202 / 138).  Padded, lengths from a sixth of N: 40 12 260 57.4 / 62.4, 400 86.6 /
-// 90.4, 600 131.9 / 129.1, 9 32 1483 266 / 237, head dim 160 16 16 320 33.5 / 34.0, 600 70.1 / 64.5.  Windows, of which a workgroup walks a few tiles
-// whatever N is: with keys of their own a window of 130, 8 16 3594 at head dim 224 316 / 367, of 228, 5 12 2530 at 208 136 / 143, of 434, 5 16 1424
-// at 240 119 / 124, at 256 157, 4 32 1357 123 / 134, 278, 6 12 2854 183 / 179; shared by two heads an XCD or more 476, 4 40/8 2653 427 / 353, 102, 3
-// 40/8 1562 127 / 112, by one 131, 36 8/2 1186 at 240 256 / 278.
+// mask ahead from 97 keys on (32 16 128 34.4 / 31.8, 2 16 2048 202 / 138).  Padded, lengths from a sixth of N: heads that do not divide by the XCDs
+// 40 12 260 57.4 / 62.4, 400 86.6 / 90.4, 600 131.9 / 129.1, others 23 16 246 41.0 / 40.7, 27 8 370 42.9 / 40.4, 9 32 1483 266 / 237, head dim 160 16
+// 16 320 33.5 / 34.0, 600 70.1 / 64.5.  Windows, of which a workgroup walks a few tiles whatever N is: with keys of their own a window of 130, 8 16
+// 3594 at head dim 224 316 / 367, of 228, 5 12 2530 at 208 136 / 143, of 434, 5 16 1424 at 240 119 / 124, at 256 157, 4 32 1357 123 / 134, 278, 6 12
+// 2854 183 / 179; shared by two heads an XCD or more 476, 4 40/8 2653 427 / 353, 102, 3 40/8 1562 127 / 112, by one 131, 36 8/2 1186 at 240 256 /
+// 278.
 // A chunk: 32 16 100 positions over 500 63.5 / 66.3, 1000 118 / 111, 64 32/8 4 over 500 57.1 / 61.0, 2000 181 / 184, 32 8 30 at head dim 224 over
 // 1000 46.7 / 48.0, 192 over 400 23.1 / 23.9, 700 34.0 / 32.0, 160 32 16 100 over 200 33.0 / 35.7, 300 40.6 / 39.2, 64 32/8 4 over 300 39.3 / 35.9;
-// more than 64 rows of shared kv heads, times as fast, 6 28/4 219 at 240 over 219 0.98, 21 32/8 71 over 288 1.05, 3 32/8 336 at 240 over 782 1.27.
-// Over 600 drawn calls that fill the chip two of the 300 that the rule sends straight to LDS lose more than 2 % (3.3), and the mean gain of those is
-// 1.13.
-// Spans of a chunk: from 256 keys a span and 97 rows on: 1 16/2 100 over 2048 29.1 / 26.1, of 87 rows 1 32 87 over 2812 30.1 / 31.8, of 64 1 32/8 16
-// over 8192 22.2 / 22.5, of 32 keys 10.2 / 11.4.  Not with a bias, whose LDS leaves the query rows to be read into the operands and whose values
-// spill: 4 8 1024 57.2 / 65.0, 1 8 77 x 513 38.6 / 52.1.
+// more than 64 rows of shared kv heads, or a workgroup for each CU at most, times as fast, 6 28/4 219 at 240 over 219 0.98, 15 8 219 over 969 1.12,
+// 21 32/8 71 over 288 1.05, 3 32/8 336 at 240 over 782 1.27. Over 600 drawn calls that fill the chip two of the 300 that the rule sends straight to
+// LDS lose more than 2 % (3.3), and the mean gain of those is 1.13.
+// Spans of a chunk: from 256 keys a span and 97 rows on, 65 of shared kv heads: 1 16/2 100 over 2048 29.1 / 26.1, of 72 rows 11 32/8 18 over 6304 138
+// / 130, of 87 1 32 87 over 2812 30.1 / 31.8, of 64 1 32/8 16 over 8192 22.2 / 22.5, of 32 keys 10.2 / 11.4.  Not with a bias, whose LDS leaves the
+// query rows to be read into the operands and whose values spill: 4 8 1024 57.2 / 65.0, 1 8 77 x 513 38.6 / 52.1.
 // A chunk whose lengths are on the device is taken to be as long as its new positions, from 256 of them on, not as the cache: a length that the
 // launch does not know may be short.  max_seq 8192, all lengths alike, at 20, 100, 300, 1000 and 8000 keys: 32 32/8 16 positions 9.8 / 14.5, 14.8 /
 // 15.5, 26.0 / 26.2, 60.7 / 60.4, 384 / 378; 9 8 8 10.3 / 12.2, 11.4 / 11.7, 13.7 / 14.5, 23.3 / 25.7, 112 / 112; 32 16 100 - , 29.8 / 33.9, 48.8 /

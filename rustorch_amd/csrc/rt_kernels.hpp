@@ -196,14 +196,14 @@ inline bool flash_tile_bf16_direct(const FlashTileParams& p) {
     const bool packed = p.pack > 1 || p.decode_rows, unknown = packed && p.kv_lens;  // lengths on the device: the new positions' at least
     const long long rows = (long long)p.seq_q * p.pack, keys = unknown ? p.seq_q : p.seq_kv, units = (long long)p.batch * (packed ? p.kv_heads : p.heads) * ((rows + 127) / 128);
     if (p.bias) return false;
-    if (p.n_splits > 1) return !unknown && keys / p.n_splits >= 256 && rows > 96;
+    if (p.n_splits > 1) return !unknown && keys / p.n_splits >= 256 && rows > (p.pack > 1 ? 64 : 96);
     const long long n_cus = p.n_cus > 0 ? p.n_cus : 256;
     if (keys < (unknown ? 256 : packed ? 140 : p.q_lens && 2 * units > n_cus ? 160 : 96)) return false;
     if (4 * units <= 3 * n_cus || p.mask == kMaskPadding) return true;
-    if (packed && p.pack > 1 && rows > 64) return keys >= 250;
+    if (packed && rows > 64 && (p.pack > 1 || units <= n_cus)) return keys >= 250;
     if (packed) return p.dim <= 160 ? keys >= 300 : p.dim <= 192 ? keys >= 700 : rows > 64 && keys >= 1000;
     if (p.window > 0) return (p.group > 1 && p.heads >= 16) || (p.dim > 240 && p.window >= 256);
-    if (p.q_lens) return keys >= (p.dim <= 224 ? 352 : 512);
+    if (p.q_lens) return keys >= (p.dim <= 224 || p.heads % 8 == 0 ? 352 : 512);
     if (p.mask == kMaskCausal) return keys >= (p.group == 1 ? 288 : p.dim > 240 ? 129 : 96);
     return p.group > 1 || keys <= 128 || keys > 160;
 }

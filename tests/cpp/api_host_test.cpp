@@ -456,7 +456,7 @@ static void wide_heads_take_the_form_that_pays() {
                           Case{4, 16, 1, 1000, 224, rt::kMaskCausal, 256, false, false}, Case{4, 40, 5, 1000, 224, rt::kMaskCausal, 64, false, true},
                           Case{8, 8, 4, 1000, 224, rt::kMaskCausal, 64, false, false},
                           Case{1, 16, 1, 1000, 256, rt::kMaskCausal, 64, false, true}, Case{16, 16, 1, 351, 160, rt::kMaskCausal, 0, true, false}, Case{16, 16, 1, 352, 160, rt::kMaskCausal, 0, true, true},
-                          Case{16, 16, 1, 511, 256, rt::kMaskCausal, 0, true, false}, Case{5, 16, 1, 159, 256, rt::kMaskCausal, 0, true, false}, Case{4, 16, 1, 159, 256, rt::kMaskCausal, 0, true, true},
+                          Case{16, 16, 1, 352, 256, rt::kMaskCausal, 0, true, true}, Case{16, 12, 1, 511, 256, rt::kMaskCausal, 0, true, false}, Case{5, 16, 1, 159, 256, rt::kMaskCausal, 0, true, false}, Case{4, 16, 1, 159, 256, rt::kMaskCausal, 0, true, true},
                           Case{16, 16, 1, 600, 256, rt::kMaskCausal, 0, true, true}, Case{4, 16, 1, 200, 256, rt::kMaskCausal, 0, true, true}}) {
         rt::FlashTileParams p{};
         p.batch = c.batch;
@@ -482,7 +482,8 @@ static void wide_heads_take_the_form_that_pays() {
     for (const Chunk& c : {Chunk{32, 100, 16, 16, 160, 200, false}, Chunk{32, 100, 16, 16, 160, 300, true}, Chunk{32, 30, 8, 8, 192, 400, false},
                            Chunk{32, 30, 8, 8, 192, 700, true}, Chunk{32, 100, 16, 16, 256, 500, false}, Chunk{32, 100, 16, 16, 256, 1000, true},
                            Chunk{64, 4, 32, 8, 256, 2000, false}, Chunk{4, 300, 16, 16, 256, 300, true},
-                           Chunk{32, 30, 32, 8, 256, 249, false}, Chunk{32, 30, 32, 8, 256, 250, true}, Chunk{16, 10, 8, 8, 256, 139, false}, Chunk{16, 10, 8, 8, 256, 140, true}}) {
+                           Chunk{32, 30, 32, 8, 256, 249, false}, Chunk{32, 30, 32, 8, 256, 250, true}, Chunk{16, 66, 16, 16, 256, 249, false}, Chunk{16, 66, 16, 16, 256, 250, true},
+                           Chunk{17, 66, 16, 16, 256, 999, false}, Chunk{16, 10, 8, 8, 256, 139, false}, Chunk{16, 10, 8, 8, 256, 140, true}}) {
         g_tile.clear();
         CHECK(rt_gqa_decode_chunk_bf16(s, g_buf, g_buf, g_buf, g_buf, nullptr, c.keys, c.batch, c.seq_new, c.heads, c.kv, c.dim, 2048, nullptr) == RT_OK);
         CHECK(g_tile.size() == 1 && g_tile[0].n_splits <= 1 && rt::flash_tile_bf16_direct(g_tile[0]) == c.direct);
