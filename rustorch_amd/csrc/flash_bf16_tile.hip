@@ -2083,8 +2083,8 @@ static bool takes_halves(const FlashTileParams& p, dim3 grid) {
 // A chunk: 32 16 100 positions over 500 63.5 / 66.3, 1000 118 / 111, 64 32/8 4 over 500 57.1 / 61.0, 2000 181 / 184, 32 8 30 at head dim 224 over
 // 1000 46.7 / 48.0, 192 over 400 23.1 / 23.9, 700 34.0 / 32.0, 160 32 16 100 over 200 33.0 / 35.7, 300 40.6 / 39.2, 64 32/8 4 over 300 39.3 / 35.9;
 // more than 64 rows of shared kv heads, or a workgroup for each CU at most, times as fast, 6 28/4 219 at 240 over 219 0.98, 15 8 219 over 969 1.12,
-// 21 32/8 71 over 288 1.05, 3 32/8 336 at 240 over 782 1.27. Over 600 drawn calls that fill the chip two of the 300 that the rule sends straight to
-// LDS lose more than 2 % (3.3), and the mean gain of those is 1.13.
+// 21 32/8 71 over 288 1.05, 3 32/8 336 at 240 over 782 1.27. Over 1040 drawn calls that fill the chip three of the 587 that the rule sends straight
+// to LDS are more than 2 % slower (3.9, 3.3, 2.1), and the mean gain of the 587 is 1.14.
 // Spans of a chunk: from 256 keys a span and 97 rows on, 65 of shared kv heads: 1 16/2 100 over 2048 29.1 / 26.1, of 72 rows 11 32/8 18 over 6304 138
 // / 130, of 87 1 32 87 over 2812 30.1 / 31.8, of 64 1 32/8 16 over 8192 22.2 / 22.5, of 32 keys 10.2 / 11.4.  Not with a bias, whose LDS leaves the
 // query rows to be read into the operands and whose values spill: 4 8 1024 57.2 / 65.0, 1 8 77 x 513 38.6 / 52.1.
