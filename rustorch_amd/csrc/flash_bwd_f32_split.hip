@@ -57,7 +57,8 @@ struct Stream {
     __amdgpu_buffer_rsrc_t rs;
     int pitch, last;
 
-    // Where a thread's pieces lie in a row: byte offsets of either half, past every descriptor where the row has no such elements.
+    // Where a thread's pieces lie in a row: byte offsets of either half, past every descriptor where the row has no such elements or the
+    // tile no such piece.
     struct Place {
         uint32_t at[kN][2];
         __device__ __forceinline__ Place(int D, int tid) {
@@ -66,7 +67,7 @@ struct Stream {
 #pragma unroll
                 for (int u = 0; u < 2; u++) {
                     const int d = 8 * ((256 * n + tid) % CH) + 4 * u;
-                    at[n][u] = d < D ? 4u * (uint32_t)d : 0x80000000u;
+                    at[n][u] = has(n, tid) && d < D ? 4u * (uint32_t)d : 0x80000000u;
                 }
         }
     };
