@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
     __shared__ float fin_inv[kRows];
 
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hh = lane >> 5;
     // the arguments, requested together: left to itself the compiler loads a field where it is first used, and waits for it there
     asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.out), "s"(p.lse), "s"(p.heads), "s"(p.group), "s"(p.seq), "s"(p.seq_kv), "s"(p.dim), "s"(p.scale),
@@ -280,24 +280,14 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
     const int ld_r = lane / CH, ld_c = lane % CH;
     const bool ld_col_ok = kExactD || 4 * ld_c < D;  // this lane's 16-byte column exists
     const uint32_t ld_off = (uint32_t)ld_r * (uint32_t)kv_pitch * 4u + (uint32_t)ld_c * 16u;  // bytes; a few rows: fits
-    // A tile that is not whole goes through descriptors that end with the last key's row: a row behind it and a column behind the
-    // head dim come back as zeros without a read, and no load stands behind a test of its own.
+    // Through descriptors that end with the tile's last key: a row behind it and a column behind the head dim come back as zeros
+    // without a read, and no load stands behind a test of its own.  The wave's number is known to be uniform: where it was not, each
+    // request was a loop over the lanes that agree on a descriptor.  us, so (whole tiles through pointers) -> now, B H N head dim: causal 1 4 30 128 10.4 ->
+    // 8.8, 1 8 40 32 5.5 -> 5.1; unmasked 1 8 161 128 16.8 -> 15.8, 1 8 250 20 7.4 -> 6.8, 1 8 60 96 9.0 -> 8.1, with the row statistic 3 5 777 32 24.5
+    // -> 23.4; a padding mask 1 8 2048 64 89.7 -> 82.1, 2 8 777 64 41.5 -> 37.3, 2 8 600 96 60.1 -> 54.2.
     f32x4_t kreg[NLD], vreg[NLD];
     const uint32_t pitch_b = (uint32_t)kv_pitch * 4u;
     auto issue_loads = [&](int tile) {
-        if constexpr (kEvenRows && kExactD) {
-            if (tile * kRows + kRows <= N) {  // (wave-uniform)
-                const char* kb = (const char*)Kg + (size_t)tile * kRows * kv_pitch * sizeof(float) + ld_off;
-                const char* vb = (const char*)Vg + (size_t)tile * kRows * kv_pitch * sizeof(float) + ld_off;
-#pragma unroll
-                for (int n = 0; n < NLD; n++) {
-                    const size_t step = (size_t)(RPL * n) * kv_pitch * sizeof(float);  // uniform
-                    kreg[n] = *(const f32x4_t*)(kb + step);
-                    vreg[n] = *(const f32x4_t*)(vb + step);
-                }
-                return;
-            }
-        }
         const size_t base = (size_t)tile * kRows * kv_pitch;
         const uint32_t bytes = (uint32_t)(min(N - tile * kRows, kRows) - 1) * pitch_b + 4u * (uint32_t)D;
         const __amdgpu_buffer_rsrc_t kb = __builtin_amdgcn_make_buffer_rsrc((void*)(Kg + base), 0, bytes, kBufferFlags);
@@ -496,9 +486,9 @@ __global__ __launch_bounds__(256, (DT <= 2 ? 2 : 1)) void flash_fwd_f32_splitk_k
 // Causal, and head dims above 64: this file's kernel spreads 32-row workgroups whose waves share the keys, so it is near the
 // mean of the chip; the split kernel takes 0.58 of the time per step at head dim 64 (1.6 against 2.83 us per tile of 32 x 32
 // and SIMD) and 0.68 at 32 (1.08 against 1.6); half a step more of fixed cost here.  us here / there, head dim 64 causal: one
-// sequence of 8 heads, 2048 keys 55 / 99, 4096 175 / 193; 2 x 12 heads, 999 keys 50 / 53; 8 x 16 heads, 256 keys 31 / 22.
-// Head dim 128: 8 heads, 2048 keys 191 / 192, 16 heads, 1500 keys 219 / 146, causal 135 / 144; 4 x 16 heads, 1024 keys
-// 405 / 218, causal 249 / 133.
+// sequence of 8 heads, 2048 keys 52 / 91, 4096 159 / 173; 2 x 12 heads, 999 keys 46 / 49; 8 x 16 heads, 256 keys 27 / 19.
+// Head dim 128: 8 heads, 2048 keys 178 / 174, 16 heads, 1500 keys 203 / 122; 4 x 16 heads, 1024 keys 395 / 198, causal
+// 239 / 119.
 //
 // Without a mask up to head dim 64 the gradients follow the same rule, so that they form the scores in the order in which the
 // row statistic was formed, and the line lies where forward and gradients together break even.  Every workgroup has the
@@ -536,9 +526,9 @@ static bool flash_f32_split_pays(const FlashF32Params& p) {
 // Above head dim 64 one workgroup of either form fills a CU: a tile step of 128 rows takes 2.45 us (2.8 above 96), one of the
 // four waves' 3.6 (4.5), and a workgroup of them 4.5 (5.5) beside its steps; causal blocks of 128 rows go two to a workgroup
 // from one a CU on, those of 32 come near the chip's mean but for the longest.  us, f32 kernel / 128 rows / shared keys, B H N at head dim
-// 128: 1 8 2048 193 / 174 / 145; 2 8 1024 102 / 92 / 81; 4 8 400 57 / 44 / 48; 2 12 700 117 / 67 / 94; 1 8 161 17.4 / 24.6 / 16.6; causal
-// 1 8 3438 297 / 284 / 223; 1 12 1500 142 / 128 / 109; 1 16 2048 220 / 175 / 168; 2 16 1500 258 / 156 / 206; at 96: 1 8 1024 43.7 / 82.7 /
-// 35.8; 8 8 200 29.5 / 25.8 / 25.7; 1 16 2048 317 / 163 / 216; causal 2 12 999 96 / 85 / 70; 4 12 600 78 / 55 / 61.
+// 128: 1 8 2048 178 / 174 / 145; 2 8 1024 95 / 92 / 81; 4 8 400 52 / 44 / 48; 2 12 700 107 / 67 / 94; 1 8 161 15.7 / 24.6 / 15.6; causal
+// 1 8 3438 271 / 284 / 223; 1 12 1500 133 / 128 / 109; 1 16 2048 196 / 175 / 168; 2 16 1500 236 / 156 / 206; at 96: 1 8 1024 39.7 / 82.7 /
+// 29.9; 8 8 200 26.3 / 25.8 / 25.7; 1 16 2048 288 / 163 / 216; causal 2 12 999 84 / 85 / 70; 4 12 600 67 / 55 / 61.
 static bool flash_f32_rows_pay(const FlashF32Params& p) {
     const double n_cus = p.n_cus > 0 ? p.n_cus : 256;
     const long long keys = p.seq_kv ? p.seq_kv : p.seq;
@@ -561,8 +551,8 @@ static bool flash_f32_rows_pay(const FlashF32Params& p) {
     return 1.41 * rows < share * (3.8 * full + (rest > n_cus ? 3.8 : (rest > 0 ? 2.2 : 0.0)));
 }
 
-// Keys from which the shared keys pay: with 128 a wave has one tile at most, and the f32 kernel is level (7.1 / 7.4 us; at head dim
-// 128 11.9 / 12.5, and with two tiles a wave at most nearly so: 17.4 / 16.5).
+// Keys from which the shared keys pay: with 128 a wave has one tile at most, and the f32 kernel is ahead (1 8 128 at head dim 64 6.6 / 7.3 us, 96
+// 8.9 / 9.3, 128 10.2 / 11.6, and with two tiles a wave at most nearly level there: 1 8 160 15.6 / 15.5, 224 16.2 / 15.6; at 64 1 8 161 9.5 / 9.3).
 // Unmasked up to head dim 32 it is level up to 256 (us, f32 kernel / shared keys, B H N: 1 8 256 6.9 / 6.8, 2 12 256 7.0 / 6.9,
 // 8 8 256 10.0 / 9.4) and keeps those calls, which then give the bits of the forward that keeps its row statistic; against
 // 128 rows a workgroup they pay there as well (1 8 160 10.5 / 6.7).

@@ -442,9 +442,9 @@ __global__ __launch_bounds__(256, DT <= 2 ? 2 : 1) void flash_fwd_f32_split_kern
 //
 // What bounds it: the vector unit, with two workgroups a CU up to head dim 64 and one above (a wave then has its SIMD to itself, Q in
 // the accumulation registers): at head dim 64 about 700 instructions a tile and wave, half of them splits of K
-// and V that a workgroup of 128 rows shares.  us, f32 kernel -> this, B H N head dim: causal 1 8 2048 64 55.0 -> 42.9, 2 12 999 64
-// 51.5 -> 39.3, 1 4 3664 32 60.2 -> 48.9, 1 8 3438 128 297 -> 223, 1 12 1500 96 120 -> 83, 2 4 333 68 19.5 -> 16.2; unmasked 1 8 1024 64
-// 28.5 -> 22.9, 1 8 512 64 16.6 -> 13.9, 1 8 1024 96 43.7 -> 35.8; 1 8 2048 64 90.2 -> 68.7 (from 128 rows a workgroup).  Eight waves that
+// and V that a workgroup of 128 rows shares.  us, f32 kernel -> this, B H N head dim: causal 1 8 2048 64 52.5 -> 42.6, 2 12 999 64
+// 46.0 -> 36.8, 1 4 3664 32 63.6 -> 45.9, 1 8 3438 128 271 -> 213, 1 12 1500 96 109 -> 79, 2 4 333 68 17.7 -> 15.5; unmasked 1 8 1024 64
+// 28.5 -> 23.2, 1 8 512 64 15.6 -> 13.1, 1 8 1024 96 39.7 -> 29.9; 1 8 2048 64 90.2 -> 68.7 (from 128 rows a workgroup).  Eight waves that
 // share them, one workgroup a CU: 1 8 2048 64 42.6 -> 42.8, 4096 128 -> 140, unmasked 1 4 1024 22.2 -> 20.2, not kept.  Relative error
 // against 64 bits at head dim 128, N = 2048 unmasked 5.8e-7 -> 2.0e-7.
 template <int DT, bool kExactD, bool kCausal>
