@@ -523,11 +523,14 @@ static bool flash_f32_split_pays(const FlashF32Params& p) {
 // head dim 64: 1 8 2048 94 / 69, causal 91 / 43; 8 8 256 17.0 / 14.5; 2 12 400 23 / 19; 1 12 1500 69 / 72; 5 12 300 20 / 25; 4 16 1024
 // 95 / 129, causal 63 / 85; causal 1 8 4096 173 / 128, 2 12 999 49 / 38, 4 16 512 29 / 32, 8 16 256 19 / 24; at 32: 8 16 300 24 / 21,
 // 4 16 1024 63 / 73, causal 1 8 4096 144 / 78, 2 16 2048 80 / 83.
-// Above head dim 64 one workgroup of either form fills a CU: a tile step of 128 rows takes 2.45 us (2.8 above 96), one of the
-// four waves' 3.6 (4.5), and a workgroup of them 4.5 (5.5) beside its steps; causal blocks of 128 rows go two to a workgroup
-// from one a CU on, those of 32 come near the chip's mean but for the longest.  us, f32 kernel / 128 rows / shared keys, B H N at head dim
-// 128: 1 8 2048 178 / 174 / 145; 2 8 1024 95 / 92 / 81; 4 8 400 52 / 44 / 48; 2 12 700 107 / 67 / 94; 1 8 161 15.7 / 24.6 / 15.6; causal
-// 1 8 3438 271 / 284 / 223; 1 12 1500 133 / 128 / 109; 1 16 2048 196 / 175 / 168; 2 16 1500 236 / 156 / 206; at 96: 1 8 1024 39.7 / 82.7 /
+// Above head dim 64 one workgroup of either form fills a CU.  Causal, a tile step of 128 rows takes 2.45 us (2.8 above 96), one of the
+// four waves' 3.6 (4.5), and a workgroup of them 4.5 (5.5) beside its steps; blocks of 128 rows go two to a workgroup
+// from one a CU on, those of 32 come near the chip's mean but for the longest.  Unmasked 2.45 (2.65) and 6.2 (6.5) a launch, against 2.85 (3.9), 5.6
+// a workgroup (6.8, and 8 between 96 and 128) and 1.2 (0.5): fitted to 110 drawn calls near the line and held against 70 others, of which the
+// slower form is taken by 2 to 5 % in three.  us, f32 kernel / 128 rows / shared keys, B H N at head dim 128: 1 8 2048 178 / 174 / 145; 2 8 1024
+// 95 / 92 / 81; 4 8 400 52 / 44 / 48; 2 12 700 107 / 67 / 94; 1 8 161 15.7 / 24.6 / 15.6; 128 rows / shared keys 3 16 248 28.2 / 30.1, 1 16 575 51.0 / 52.0, 1 32/8
+// 371 37.7 / 37.6, 1 12 1185 100 / 91; at 100 2 12 337 34.3 / 38.9, 1 8 1751 140 / 125; at 80 2 32/8 206 23.2 / 24.2, 2 16 308 30.1 / 29.4; at 68 3 8 1556
+// 238 / 213.  Causal 1 8 3438 271 / 284 / 223; 1 12 1500 133 / 128 / 109; 1 16 2048 196 / 175 / 168; 2 16 1500 236 / 156 / 206; unmasked at 96 1 8 1024 39.7 / 82.7 /
 // 29.9; 8 8 200 26.3 / 25.8 / 25.7; 1 16 2048 288 / 163 / 216; causal 2 12 999 84 / 85 / 70; 4 12 600 67 / 55 / 61.
 static bool flash_f32_rows_pay(const FlashF32Params& p) {
     const double n_cus = p.n_cus > 0 ? p.n_cus : 256;
@@ -535,11 +538,15 @@ static bool flash_f32_rows_pay(const FlashF32Params& p) {
     const double tiles = (double)((keys + 31) / 32), n_bh = (double)p.heads * p.batch, groups = n_bh * ((p.seq + 31) / 32);
     const double per_cu = n_bh * ((p.seq + 127) / 128) / n_cus, share = __builtin_ceil(tiles / 4);
     if (p.dim > 64) {
-        const double row_step = p.dim > 96 ? 2.8 : 2.45, key_step = p.dim > 96 ? 4.5 : 3.6, own = p.dim > 96 ? 5.5 : 4.5;
-        if (p.mask == kMaskCausal)
+        const bool high = p.dim > 96;
+        if (p.mask == kMaskCausal) {
+            const double row_step = high ? 2.8 : 2.45, key_step = high ? 4.5 : 3.6, own = high ? 5.5 : 4.5;
             return row_step * (per_cu > 1 ? __builtin_ceil(per_cu / 2) * (tiles + 4) : tiles) <
                    __builtin_fmax(key_step * share, key_step * groups * (tiles + 1) / (8 * n_cus) + own * groups / n_cus);
-        return row_step * __builtin_ceil(per_cu) * tiles + 2 < __builtin_ceil(groups / n_cus) * (key_step * share + own) - own;
+        }
+        const double each = high ? (p.dim == 128 ? 6.8 : 8.0) : 5.6;
+        return (high ? 2.65 : 2.45) * __builtin_ceil(per_cu) * tiles + (high ? 6.5 : 6.2) <
+               __builtin_ceil(groups / n_cus) * ((high ? 3.9 : 2.85) * share + each) + (high ? 0.5 : 1.2);
     }
     if (p.mask == kMaskCausal) {
         const double rows = __builtin_fmax(tiles, 1.1 * per_cu * (tiles + 4) / 2), mean = groups * (tiles + 1) / (8 * n_cus);
