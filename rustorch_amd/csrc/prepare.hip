@@ -303,12 +303,14 @@ hipError_t launch_decode_prepare(hipStream_t stream, const DecodePrepareParams& 
         pp.pair_magic = (1u << 20) / (uint32_t)(p.head_dim / 16) + 1u;
         auto launch = [&](auto rows_c, auto dmax_c) {
             constexpr int kRows = decltype(rows_c)::value, kDMax = decltype(dmax_c)::value;
-            // Token blocks up to a multiple of eight, so that every head's land on the XCD that has their table rows (those behind the
-            // last token end at once), where that adds a fifth at most.  us, as they are / so, 1 x 32 / 8 heads of 128: 550 tokens (9 blocks)
-            // 6.5 / 7.4, 1100 (18) 8.8 / 9.3, 1300 (21) 10.5 / 9.9, 2200 (35) 13.4 / 12.8, 2600 (41) 14.7 / 13.9, 3000 (47) 16.4 / 14.6.
+            // Token blocks up to a multiple of eight, so that every head's land on the XCD that has their table rows (those behind the last
+            // token end at once), where that adds a twelfth at most and rows stay in the caches.  us, as they are / so, four or more sets of buffers in turn, 32 / 8
+            // heads of 128: 1 x 4500 tokens (71 blocks) 27.2 / 25.9, 5300 (83) 33.5 / 30.7, 3500 (55) 20.4 / 20.2; but 1 x 2200 (35) 11.0 / 11.5, 2 x 2600
+            // (41) 28.4 / 31.3, 4 x 1300 (21) 28.9 / 32.1; past the caches 8 x 1300 46.7 / 52.3, 4 x 2711 (43) 48.4 / 51.8, 2 x 32 / 32 of 80, 2600 46.8 / 53.0, 2 x 5500
+            // (86) 49.4 / 50.0.
             int blocks = (p.seq + kRows - 1) / kRows;
             const int eights = (blocks + 7) / 8 * 8;
-            if (5 * (eights - blocks) <= blocks) blocks = eights;
+            if (!past && 12 * (eights - blocks) <= blocks) blocks = eights;
             const dim3 grid(blocks, p.n_heads + p.n_kv, p.batch), block(256);
             if (past) hipLaunchKernelGGL((prompt_prepare_kernel<kRows, kDMax, true>), grid, block, 0, stream, pp);
             else hipLaunchKernelGGL((prompt_prepare_kernel<kRows, kDMax, false>), grid, block, 0, stream, pp);
